@@ -367,53 +367,72 @@ __global__ __launch_bounds__(256) void k_paged_attn16(AttnKArgs a) {
     }
 }
 
-// Merge the key-slice partials of each (token, head): thread = 8 consecutive dims.
-__global__ __launch_bounds__(256) void k_attn_combine(const float* __restrict__ part_acc,
-                                                      const float* __restrict__ part_ml, int T, int H, int HD,
-                                                      int nsplit, float* out_f32, __half* out_a16, int Kb_out) {
-    const long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    const int c8 = HD / 8;
-    if (idx >= (long)T * H * c8) return;
-    const int c = (int)(idx % c8);
-    const long th = idx / c8;           // t * H + h
-    const int h = (int)(th % H);
-    const int t = (int)(th / H);
-    const float* ml = part_ml + th * nsplit * 2;
-    const float* pa = part_acc + th * nsplit * HD + c * 8;
+// Merge the key-slice partials of a (token, head): lane = 4 consecutive dims x one of the wave's slice groups, WPR waves
+// per (token, head).  With one thread walking all slices of its dims (the first form) a few long contexts -- 36 items in
+// 57 slices each -- made 9 workgroups of 57 dependent round trips: 30 us a layer; every slice has a lane group of its own
+// up to 16 (64 dims, 4 waves), and what is left of a walk is loads that do not wait for each other.
+template <int WPR>
+__global__ __launch_bounds__(256) void k_attn_combine(const float* __restrict__ part_acc, const float* __restrict__ part_ml, int rows, int H, int HD,
+                                                      int nsplit, int c_shift, float* out_f32, __half* out_a16, int Kb_out) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int th = (int)blockIdx.x * (4 / WPR) + (WPR == 1 ? wave : 0);   // t * H + h
+    const int part = WPR == 1 ? 0 : wave;
+    const bool live = th < rows;
+    const size_t row = live ? th : rows - 1;
+    const int C = 1 << c_shift, c = lane & (C - 1), grp = lane >> c_shift, G = 64 >> c_shift;
+    const float* ml = part_ml + row * nsplit * 2;
+    const float* pa = part_acc + row * nsplit * HD + 4 * c;
+    const bool has = 4 * c < HD;
     float M = -INFINITY;
-    for (int s = 0; s < nsplit; s++) M = fmaxf(M, ml[2 * s]);
-    float L = 0.f, o[8];
+    for (int s = lane; s < nsplit; s += 64) M = fmaxf(M, ml[2 * s]);
 #pragma unroll
-    for (int j = 0; j < 8; j++) o[j] = 0.f;
-    for (int s = 0; s < nsplit; s++) {
+    for (int o = 32; o > 0; o >>= 1) M = fmaxf(M, __shfl_xor(M, o, 64));
+    float L = 0.f;
+    f4_t o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+    for (int s = part * G + grp; s < nsplit; s += WPR * G) {
         const float w = expf(ml[2 * s] - M);   // empty slices carry max = -inf -> weight 0
         L = fmaf(ml[2 * s + 1], w, L);
-        const float4 a0 = *reinterpret_cast<const float4*>(pa + (size_t)s * HD);
-        const float4 a1 = *reinterpret_cast<const float4*>(pa + (size_t)s * HD + 4);
-        o[0] = fmaf(a0.x, w, o[0]); o[1] = fmaf(a0.y, w, o[1]); o[2] = fmaf(a0.z, w, o[2]); o[3] = fmaf(a0.w, w, o[3]);
-        o[4] = fmaf(a1.x, w, o[4]); o[5] = fmaf(a1.y, w, o[5]); o[6] = fmaf(a1.z, w, o[6]); o[7] = fmaf(a1.w, w, o[7]);
+        const f4_t a = has ? *reinterpret_cast<const f4_t*>(pa + (size_t)s * HD) : f4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int e = 0; e < 4; e++) o[e] = fmaf(a[e], w, o[e]);
     }
+    for (int d = C; d < 64; d <<= 1) {
+        L += __shfl_xor(L, d, 64);
+#pragma unroll
+        for (int e = 0; e < 4; e++) o[e] += __shfl_xor(o[e], d, 64);
+    }
+    if constexpr (WPR > 1) {
+        __shared__ f4_t s_o[WPR][32];
+        __shared__ float s_l[WPR];
+        if (grp == 0) s_o[part][c] = o;
+        if (lane == 0) s_l[part] = L;
+        __syncthreads();
+        if (part != 0) return;
+        o = s_o[0][c], L = s_l[0];
+#pragma unroll
+        for (int w = 1; w < WPR; w++) {
+            o += s_o[w][c];
+            L += s_l[w];
+        }
+    }
+    if (!live || grp != 0 || !has) return;
     const float inv = 1.0f / L;
-#pragma unroll
-    for (int j = 0; j < 8; j++) o[j] *= inv;
-    if (out_f32) {
-        float* dst = out_f32 + th * HD + c * 8;
-        *reinterpret_cast<float4*>(dst) = make_float4(o[0], o[1], o[2], o[3]);
-        *reinterpret_cast<float4*>(dst + 4) = make_float4(o[4], o[5], o[6], o[7]);
-    }
+    o *= inv;
+    if (out_f32) *reinterpret_cast<f4_t*>(out_f32 + row * HD + 4 * c) = o;
     if (out_a16) {
-        const int kk = h * HD + c * 8;
-        H8 hi, lo;
+        const int t = th / H, kk = (th % H) * HD + 4 * c;
+        alignas(8) __half hi[4], lo[4];
 #pragma unroll
-        for (int j = 0; j < 8; j++) {
-            const float xv = fminf(fmaxf(o[j], -65504.f), 65504.f);
-            hi.v[j] = __float2half_rn(xv);
-            lo.v[j] = __float2half_rn(xv - __half2float(hi.v[j]));
+        for (int e = 0; e < 4; e++) {
+            const float xv = fminf(fmaxf(o[e], -65504.f), 65504.f);
+            hi[e] = __float2half_rn(xv);
+            lo[e] = __float2half_rn(xv - __half2float(hi[e]));
         }
         const size_t tl = ((size_t)(t >> 4) * Kb_out + (kk >> 5)) * 2;
-        const size_t off = (size_t)((t & 15) + 16 * ((kk >> 3) & 3)) * 8;
-        *reinterpret_cast<H8*>(out_a16 + tl * TILE_HALVES + off) = hi;
-        *reinterpret_cast<H8*>(out_a16 + (tl + 1) * TILE_HALVES + off) = lo;
+        const size_t off = (size_t)((t & 15) + 16 * ((kk >> 3) & 3)) * 8 + (kk & 7);
+        *reinterpret_cast<uint2*>(out_a16 + tl * TILE_HALVES + off) = *reinterpret_cast<const uint2*>(hi);
+        *reinterpret_cast<uint2*>(out_a16 + (tl + 1) * TILE_HALVES + off) = *reinterpret_cast<const uint2*>(lo);
     }
 }
 
@@ -553,9 +572,13 @@ void launch_paged_attention(const AttnArgs& a) {
     }
     if (nsplit > 1 && !merge_waves) {
         ProfScope ps(PC_ATTN_COMBINE, (double)a.T * a.H * nsplit * (a.hd + 2) * 4.0, 0);
-        const long threads = (long)a.T * a.H * (a.hd / 8);
-        NVLLM_LAUNCH(k_attn_combine, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0,
-                           k.part_acc, k.part_ml, a.T, a.H, a.hd, nsplit, a.out_f32, a.out_a16, k.Kb_out);
+        const int rows = a.T * a.H;
+        int c_shift = 0;   // lanes that cover a row, four dims each
+        while ((4 << c_shift) < a.hd) c_shift++;
+        if (nsplit > 4 * (64 >> c_shift))
+            NVLLM_LAUNCH((k_attn_combine<4>), dim3(rows), dim3(256), 0, k.part_acc, k.part_ml, rows, a.H, a.hd, nsplit, c_shift, a.out_f32, a.out_a16, k.Kb_out);
+        else
+            NVLLM_LAUNCH((k_attn_combine<1>), dim3(cdiv(rows, 4)), dim3(256), 0, k.part_acc, k.part_ml, rows, a.H, a.hd, nsplit, c_shift, a.out_f32, a.out_a16, k.Kb_out);
     }
 }
 
