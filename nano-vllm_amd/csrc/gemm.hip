@@ -316,40 +316,4 @@ void gemm_release() {
     g_counters = nullptr;
 }
 
-// --------------------------------------------- raw fp32 weights (ops.h matmul)
-// One wave per output feature, eight tokens at a time; used only when matmul() is
-// handed a plain fp32 [N, K] device buffer instead of a load_model handle.
-__global__ __launch_bounds__(256) void k_matmul_f32w(float* __restrict__ out, const float* __restrict__ in,
-                                                     const float* __restrict__ w, int T, int K, int N) {
-    const int lane = threadIdx.x & 63;
-    const int n = blockIdx.x * 4 + (threadIdx.x >> 6);
-    const int t0 = blockIdx.y * 8;
-    if (n >= N) return;
-    float acc[8];
-#pragma unroll
-    for (int i = 0; i < 8; i++) acc[i] = 0.f;
-    const float* wr = w + (size_t)n * K;
-    for (int k = lane; k < K; k += 64) {
-        const float wv = wr[k];
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-            const int t = min(t0 + i, T - 1);
-            acc[i] = fmaf(in[(size_t)t * K + k], wv, acc[i]);
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < 8; i++) {
-        float v = acc[i];
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-        if (lane == 0 && t0 + i < T) out[(size_t)(t0 + i) * N + n] = v;
-    }
-}
-
-void launch_matmul_f32w(float* out, const float* in, const float* w, int T, int K, int N) {
-    if (T <= 0 || N <= 0) return;
-    ProfScope ps(PC_GEMM_OTHER, (double)N * K * 4.0 + (double)T * (K + N) * 4.0, 2.0 * T * (double)N * K);
-    NVLLM_LAUNCH(k_matmul_f32w, dim3(cdiv(N, 4), cdiv(T, 8)), dim3(256), 0, out, in, w, T, K, N);
-}
-
 }  // namespace nvllm

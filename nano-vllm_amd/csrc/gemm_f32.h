@@ -1,0 +1,76 @@
+// gemm_f32.h -- projections of models whose weights and activations are fp32 (row-major, as the files hold them).
+#pragma once
+
+#include "nvllm_internal.h"
+
+namespace nvllm {
+
+// What happens to a segment's complete sums y[t][n].
+enum class F32Out {
+    STORE,    // out[t][n] = y
+    ADD,      // out[t][n] += y (residual)
+    SILU,     // y * sigmoid(y)
+    RELU2,    // max(y, 0)^2
+    ROPE_Q,   // rotated -> out
+    ROPE_K,   // rotated -> key rows of the block pool
+    KV_V      // -> value rows of the block pool
+};
+struct F32Segment {
+    const float* W;      // [N][K]
+    const float* W2;     // second matrix of a gated pair: out = silu(y + bias) * (y2 + bias2) (null: none)
+    const float *bias, *bias2;   // of a pair, per feature (null: none)
+    int N;
+    F32Out kind;
+    float* out;          // [T][ldo]
+    int ldo;
+    int first;           // first feature tile of the launch (set by the launcher)
+    bool vec;            // 16-byte stores (set by the launcher)
+};
+constexpr int F32_SEGMENTS = 4;
+struct F32Gemm {
+    const float* in;               // [rows][K]
+    const int* in_rows = nullptr;  // row of `in` that token t reads (null: t)
+    const float* gain = nullptr;   // RMS norm of the input: in * gain / rms(in)
+    float eps = 0.f;
+    int K, T;
+    int n_segs = 0;
+    F32Segment seg[F32_SEGMENTS];
+    // rows sorted by expert, 16 of one expert at a time (moe.h): expert of a 16-row block (-1: none), floats between the
+    // experts' matrices, and what a row's results are scaled by (null: nothing)
+    const int* block_expert = nullptr;
+    long expert_stride = 0;
+    const float* row_weight = nullptr;
+    // ROPE_*, KV_V
+    const int* pos = nullptr;
+    const int* kv_row = nullptr;
+    const float2* rope = nullptr;
+    void* pool_k = nullptr;
+    void* pool_v = nullptr;
+    int hd = 0, KD = 0, kv_elem_bytes = 4, bs = 16;
+    long layer_off = 0;
+
+    F32Gemm(const float* in_, int T_, int K_) : in(in_), K(K_), T(T_) {}
+    F32Gemm& norm(const float* g, float e) {
+        gain = g;
+        eps = e;
+        return *this;
+    }
+    F32Gemm& add(const float* W, int N, float* out, F32Out kind = F32Out::STORE) {
+        seg[n_segs++] = F32Segment{W, nullptr, nullptr, nullptr, N, kind, out, N, 0, false};
+        return *this;
+    }
+    F32Gemm& add_pair(const float* gate, const float* up, int N, float* out, const float* bias_gate = nullptr, const float* bias_up = nullptr) {
+        seg[n_segs++] = F32Segment{gate, up, bias_gate, bias_up, N, F32Out::STORE, out, N, 0, false};
+        return *this;
+    }
+    F32Gemm& experts(const int* blocks, long stride, const float* weight) {
+        block_expert = blocks;
+        expert_stride = stride;
+        row_weight = weight;
+        return *this;
+    }
+};
+// One launch for all segments: all of them gated pairs, or none.
+void launch_gemm_f32(const F32Gemm& g, int prof_cls);
+
+}  // namespace nvllm

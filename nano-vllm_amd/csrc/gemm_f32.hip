@@ -1,0 +1,455 @@
+// gemm_f32.hip -- out[T, N] = act[T, K] x W[N, K]^T with everything in fp32, on v_mfma_f32_16x16x4_f32 (an exact fma
+// chain), and the element-wise work around a projection in the same launch: the RMS norm in front (x * gain enters the
+// product, 1/rms scales its sums -- a scalar per token commutes with the projection), and behind it SwiGLU of a gated
+// pair, the residual add, rotation and cache rows.
+//
+// A wave owns NB 16-row blocks of W (of both matrices of a pair) x TB 16-token blocks, or shares them with KS - 1 others
+// of its workgroup: these take the K-steps of 32 round-robin and meet in LDS, so nothing is cut across workgroups and a
+// launch needs no second one.  A workgroup's waves that do not share take neighbouring feature tiles.
+// Operands go from global memory into MFMA registers as they lie: lane (row x, group g) reads 4 consecutive k at
+// 4g (+16 for the step's second half), product i of a quad takes element i of every lane, and the same rule on both
+// sides makes the four products one 16-deep step.  No LDS staging: at 2 x 4 blocks a step of 32 multiplies (1,024
+// matrix-core cycles per SIMD) needs 6 KiB per wave, 24 bytes per cycle and CU, well below what L2 delivers.
+//
+// What bounds it: few tokens -- bytes of W, and below ~10 MB the launch itself; hundreds of tokens -- the fp32 matrix
+// rate (157 TFLOP/s).
+#include <algorithm>
+
+#include "gemm_common.h"
+#include "gemm_f32.h"
+
+namespace nvllm {
+
+constexpr int F32_STEP = 32;   // k per step: 128 bytes, a cache line, of every row
+constexpr int f32_waves(int KS) { return KS == 8 ? 8 : 4; }   // waves of a workgroup: feature tiles x slices of K
+
+// What follows a token's complete sums of features n .. n+3 (n % 4 == 0; `old`: what ADD adds to).
+template <bool PAIR>
+__device__ __forceinline__ void f32_finish(const F32Gemm& p, const F32Segment& sg, int t, int n, f4_t y, const f4_t u, const f4_t old) {
+    if constexpr (PAIR) {
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const int f = min(n + r, sg.N - 1);
+            y[r] = silu_mul(sg.bias ? y[r] + sg.bias[f] : y[r], sg.bias2 ? u[r] + sg.bias2[f] : u[r]);
+        }
+    } else {
+        switch (sg.kind) {
+            case F32Out::ADD:
+#pragma unroll
+                for (int r = 0; r < 4; r++) y[r] = __fadd_rn(old[r], y[r]);
+                break;
+            case F32Out::SILU:
+#pragma unroll
+                for (int r = 0; r < 4; r++) y[r] = silu_mul(y[r], 1.f);
+                break;
+            case F32Out::RELU2:
+#pragma unroll
+                for (int r = 0; r < 4; r++) y[r] = fmaxf(y[r], 0.f) * fmaxf(y[r], 0.f);
+                break;
+            case F32Out::ROPE_Q:
+            case F32Out::ROPE_K: {   // the two pairs of this quad turn (layers.c:118-141)
+                const float2* tab = p.rope + (size_t)p.pos[t] * (p.hd >> 1) + ((n % p.hd) >> 1);
+                const float2 c0 = tab[0], c1 = tab[1];
+                y = f4_t{__fsub_rn(__fmul_rn(y[0], c0.x), __fmul_rn(y[1], c0.y)), __fadd_rn(__fmul_rn(y[0], c0.y), __fmul_rn(y[1], c0.x)),
+                         __fsub_rn(__fmul_rn(y[2], c1.x), __fmul_rn(y[3], c1.y)), __fadd_rn(__fmul_rn(y[2], c1.y), __fmul_rn(y[3], c1.x))};
+                break;
+            }
+            default: break;
+        }
+        if (sg.kind == F32Out::ROPE_K || sg.kind == F32Out::KV_V) {
+            const int row = p.kv_row[t];
+            if (row < 0) return;
+            const bool is_k = sg.kind == F32Out::ROPE_K;
+            const float z[4] = {y[0], y[1], y[2], y[3]};
+            if (p.kv_elem_bytes == 4) {   // the reference's rows (memory.c:37-43)
+                kv_put4<float>(reinterpret_cast<float*>(is_k ? p.pool_k : p.pool_v) + p.layer_off + (size_t)row * p.KD + n, z);
+            } else {                      // fp16 pages in matrix-core operand order
+                __half* page = reinterpret_cast<__half*>(is_k ? p.pool_k : p.pool_v) + p.layer_off + kv16_page(row / p.bs, n / p.hd, p.KD / p.hd, p.hd);
+                if (is_k) kv_put4<__half>(page + kv16_k_off(row % p.bs, n % p.hd), z);
+                else kv_put4_strided<__half>(page + kv16_v_off(row % p.bs, n % p.hd), z);
+            }
+            return;
+        }
+    }
+    float* o = sg.out + (size_t)t * sg.ldo + n;
+    if (sg.vec) {
+        *reinterpret_cast<f4_t*>(o) = y;
+    } else {
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+            if (n + r < sg.N) o[r] = y[r];
+    }
+}
+__device__ __forceinline__ f4_t f32_old(const F32Segment& sg, int t, int n) {   // t < T; features past the last are those of the last
+    const float* o = sg.out + (size_t)t * sg.ldo;
+    if (sg.vec) return *reinterpret_cast<const f4_t*>(o + min(n, sg.N - 4));
+    f4_t v;
+#pragma unroll
+    for (int r = 0; r < 4; r++) v[r] = o[min(n + r, sg.N - 1)];
+    return v;
+}
+
+template <int NB, int TB, int KS, bool PAIR, bool NORM>
+__global__ __launch_bounds__(f32_waves(KS) * 64) void k_gemm_f32(F32Gemm p) {
+    constexpr int NT = PAIR ? 2 * NB : NB;   // weight blocks per step: all of the first matrix, then all of the second
+    constexpr int RING = NT * TB == 1 ? 4 : 2;
+    constexpr int GROUPS = f32_waves(KS) / KS;      // feature tiles of a workgroup
+    constexpr int ITEMS = NB * TB * 64;             // results of a group, four features of a token each
+    constexpr int FPT = (ITEMS + KS * 64 - 1) / (KS * 64);
+    __shared__ f4_t s_red[KS > 1 ? GROUPS * KS : 1][NT * TB][64];
+    __shared__ float s_ss[NORM && KS > 1 ? GROUPS * KS : 1][TB * 16];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int slice = wave % KS, grp = wave / KS, tid = slice * 64 + lane;   // (tid: within the group)
+    const int x = lane & 15, g = lane >> 4;
+    const int tile = (int)blockIdx.x * GROUPS + grp;
+    int s = 0;
+    while (s + 1 < p.n_segs && tile >= p.seg[s + 1].first) s++;
+    const F32Segment& sg = p.seg[s];
+    const int nb0 = (tile - sg.first) * NB, tb0 = (int)blockIdx.y * TB;
+    const int K = p.K, T = p.T, N = sg.N;
+    const float *W = sg.W, *W2 = sg.W2;
+    if (KS == 1 && nb0 * 16 >= N) return;   // (no barrier in this form)
+    if (p.block_expert) {   // (TB = 1: a workgroup's rows are of one expert)
+        const int e = __builtin_amdgcn_readfirstlane(p.block_expert[tb0]);
+        if (e < 0) return;   // fewer rows than the launch has room for
+        W += (size_t)e * p.expert_stride;
+        if (PAIR) W2 += (size_t)e * p.expert_stride;
+    }
+    const float* wp[NT];
+#pragma unroll
+    for (int i = 0; i < NB; i++) {
+        const size_t row = (size_t)min((nb0 + i) * 16 + x, N - 1) * K + 4 * g;   // rows past the last are read again and not stored
+        wp[i] = W + row;
+        if constexpr (PAIR) wp[NB + i] = W2 + row;
+    }
+    const float* ap[TB];
+#pragma unroll
+    for (int j = 0; j < TB; j++) {
+        const int t = min((tb0 + j) * 16 + x, T - 1);
+        ap[j] = p.in + (size_t)(p.in_rows ? p.in_rows[t] : t) * K + 4 * g;
+    }
+    const float* gp = NORM ? p.gain + 4 * g : nullptr;
+
+    f4_t w[RING][NT][2], a[RING][TB][2], gv[RING][NORM ? 2 : 1];
+    const f4_t zero = {0.f, 0.f, 0.f, 0.f};
+    auto load = [&](int r, int i) {
+        const int k = (slice + i * KS) * F32_STEP;
+        __builtin_amdgcn_sched_barrier(0);   // requests stay in the order of their use: waits count what is younger
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+#pragma unroll
+            for (int n = 0; n < NT; n++) w[r][n][h] = *reinterpret_cast<const f4_t*>(wp[n] + k + 16 * h);
+#pragma unroll
+            for (int j = 0; j < TB; j++) a[r][j][h] = *reinterpret_cast<const f4_t*>(ap[j] + k + 16 * h);
+            if constexpr (NORM) gv[r][h] = *reinterpret_cast<const f4_t*>(gp + k + 16 * h);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    // Sums are taken in three levels -- 16 products, a step's two halves into the wave's total, the waves -- which keeps
+    // their error that of short chains, and leaves four products in a row to wait for each other instead of all.
+    f4_t acc[NT][TB];
+#pragma unroll
+    for (int n = 0; n < NT; n++)
+#pragma unroll
+        for (int j = 0; j < TB; j++) acc[n][j] = zero;
+    float ss[TB];
+#pragma unroll
+    for (int j = 0; j < TB; j++) ss[j] = 0.f;
+    auto multiply = [&](int r) {
+        f4_t part[2][NT][TB];
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            f4_t v[TB];
+#pragma unroll
+            for (int j = 0; j < TB; j++) {
+                v[j] = a[r][j][h];
+                if constexpr (NORM) {
+                    float sq = v[j][0] * v[j][0];
+#pragma unroll
+                    for (int e = 1; e < 4; e++) sq = fmaf(v[j][e], v[j][e], sq);
+                    ss[j] += sq;
+#pragma unroll
+                    for (int e = 0; e < 4; e++) v[j][e] *= gv[r][h][e];
+                }
+            }
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+#pragma unroll
+                for (int n = 0; n < NT; n++)
+#pragma unroll
+                    for (int j = 0; j < TB; j++)
+                        part[h][n][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[r][n][h][e], v[j][e], e == 0 ? zero : part[h][n][j], 0, 0, 0);
+        }
+#pragma unroll
+        for (int n = 0; n < NT; n++)
+#pragma unroll
+            for (int j = 0; j < TB; j++) acc[n][j] += part[0][n][j] + part[1][n][j];
+    };
+    // Whole steps: the steady loop requests without a condition (where paths with and without requests meet, the compiler
+    // waits for all of them); what is left of it is at most RING conditional requests.
+    const int whole = K / F32_STEP;
+    const int mine = slice < whole && nb0 * 16 < N ? (whole - slice + KS - 1) / KS : 0;
+    if (mine < RING) {
+#pragma unroll
+        for (int r = 0; r + 1 < RING; r++)
+            if (r < mine) load(r, r);
+#pragma unroll
+        for (int r = 0; r + 1 < RING; r++)
+            if (r < mine) multiply(r);
+    } else {
+#pragma unroll
+        for (int r = 0; r < RING; r++) load(r, r);
+        int i0 = 0;
+        for (; i0 + 2 * RING <= mine; i0 += RING) {
+#pragma unroll
+            for (int r = 0; r < RING; r++) {
+                multiply(r);
+                load(r, i0 + r + RING);
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < RING; r++) {
+            if (i0 + r < mine) multiply(r);
+            if (i0 + r + RING < mine) load(r, i0 + r + RING);
+        }
+#pragma unroll
+        for (int r = 0; r < RING; r++)
+            if (i0 + r + RING < mine) multiply(r);
+    }
+    if (whole * F32_STEP < K && whole % KS == slice && nb0 * 16 < N) {   // the rest of K (K % 4 == 0: a lane's four are in or out together)
+        const int k = whole * F32_STEP;
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const bool in = k + 16 * h + 4 * g < K;
+#pragma unroll
+            for (int n = 0; n < NT; n++) w[0][n][h] = in ? *reinterpret_cast<const f4_t*>(wp[n] + k + 16 * h) : zero;
+#pragma unroll
+            for (int j = 0; j < TB; j++) a[0][j][h] = in ? *reinterpret_cast<const f4_t*>(ap[j] + k + 16 * h) : zero;
+            if constexpr (NORM) gv[0][h] = in ? *reinterpret_cast<const f4_t*>(gp + k + 16 * h) : zero;
+        }
+        multiply(0);
+    }
+    auto rinv_of = [&](float sum) { return __fdiv_rn(1.0f, sqrtf(__fadd_rn(__fdiv_rn(sum, (float)K), p.eps))); };
+    if constexpr (NORM) {
+#pragma unroll
+        for (int j = 0; j < TB; j++) {
+            ss[j] += __shfl_xor(ss[j], 16, 64);
+            ss[j] += __shfl_xor(ss[j], 32, 64);
+        }
+    }
+    auto finish = [&](int t, int n, f4_t y, f4_t u, float sum, f4_t old) {
+        if (t >= T || n >= N) return;
+        float scale = NORM ? rinv_of(sum) : 1.f;
+        if (p.row_weight) scale *= p.row_weight[t];
+        if (NORM || p.row_weight) {
+            y *= scale;
+            if constexpr (PAIR) u *= scale;
+        }
+        f32_finish<PAIR>(p, sg, t, n, y, u, old);
+    };
+    const bool adds = !PAIR && sg.kind == F32Out::ADD;
+    if constexpr (KS == 1) {   // a lane's sums are complete: features 4g .. 4g + 3 of token x of every block pair
+        f4_t old[NB][TB];
+#pragma unroll
+        for (int i = 0; i < NB; i++)
+#pragma unroll
+            for (int j = 0; j < TB; j++)
+                old[i][j] = adds ? f32_old(sg, min((tb0 + j) * 16 + x, T - 1), (nb0 + i) * 16 + 4 * g) : zero;
+#pragma unroll
+        for (int i = 0; i < NB; i++)
+#pragma unroll
+            for (int j = 0; j < TB; j++)
+                finish((tb0 + j) * 16 + x, (nb0 + i) * 16 + 4 * g, acc[i][j], PAIR ? acc[NT - NB + i][j] : zero, ss[j], old[i][j]);
+    } else {
+        // what the epilogue adds to is requested before the waves' sums meet
+        f4_t old[FPT];
+#pragma unroll
+        for (int q = 0; q < FPT; q++) {
+            const int e = min(tid + q * KS * 64, ITEMS - 1), l = e & 63, j = (e >> 6) % TB, i = (e >> 6) / TB;
+            old[q] = adds ? f32_old(sg, min((tb0 + j) * 16 + (l & 15), T - 1), (nb0 + i) * 16 + 4 * (l >> 4)) : zero;
+        }
+#pragma unroll
+        for (int n = 0; n < NT; n++)
+#pragma unroll
+            for (int j = 0; j < TB; j++) s_red[wave][n * TB + j][lane] = acc[n][j];
+        if constexpr (NORM) {
+#pragma unroll
+            for (int j = 0; j < TB; j++)
+                if (g == 0) s_ss[wave][j * 16 + x] = ss[j];
+        }
+        __syncthreads();
+        const int w0 = grp * KS;
+#pragma unroll
+        for (int q = 0; q < FPT; q++) {
+            const int e = tid + q * KS * 64;
+            if (e >= ITEMS) break;
+            const int l = e & 63, j = (e >> 6) % TB, i = (e >> 6) / TB;
+            f4_t y = s_red[w0][i * TB + j][l], u = zero;
+#pragma unroll
+            for (int v = 1; v < KS; v++) y += s_red[w0 + v][i * TB + j][l];
+            if constexpr (PAIR) {
+                u = s_red[w0][(NB + i) * TB + j][l];
+#pragma unroll
+                for (int v = 1; v < KS; v++) u += s_red[w0 + v][(NB + i) * TB + j][l];
+            }
+            float sum = 0.f;
+            if constexpr (NORM) {
+#pragma unroll
+                for (int v = 0; v < KS; v++) sum += s_ss[w0 + v][j * 16 + (l & 15)];
+            }
+            finish((tb0 + j) * 16 + (l & 15), (nb0 + i) * 16 + 4 * (l >> 4), y, u, sum, old[q]);
+        }
+    }
+}
+
+// Rows that are no multiples of 16 bytes (K % 4 != 0, or a caller's odd pointer): a wave sums four features of four tokens,
+// its lanes striding over k.
+template <bool PAIR>
+__global__ __launch_bounds__(256) void k_gemm_f32_any(F32Gemm p) {
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    int s = 0;
+    while (s + 1 < p.n_segs && (int)blockIdx.x >= p.seg[s + 1].first) s++;
+    const F32Segment& sg = p.seg[s];
+    const int n = (((int)blockIdx.x - sg.first) * 4 + wave) * 4;
+    int t0 = (int)blockIdx.y * 4;
+    const int K = p.K, T = p.T, N = sg.N;
+    if (n >= N) return;
+    for (; t0 < T; t0 += (int)gridDim.y * 4) {
+        const float *W = sg.W, *W2 = sg.W2;
+        if (p.block_expert) {
+            const int e = p.block_expert[t0 >> 4];
+            if (e < 0) continue;
+            W += (size_t)e * p.expert_stride;
+            if (PAIR) W2 += (size_t)e * p.expert_stride;
+        }
+        float acc[4][4] = {}, acc2[4][4] = {}, ss[4] = {};   // [token][feature]
+        const float* ap[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const int t = min(t0 + j, T - 1);
+            ap[j] = p.in + (size_t)(p.in_rows ? p.in_rows[t] : t) * K;
+        }
+        for (int k = lane; k < K; k += 64) {
+            float v[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                v[j] = ap[j][k];
+                if (p.gain) {
+                    ss[j] = fmaf(v[j], v[j], ss[j]);
+                    v[j] *= p.gain[k];
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const size_t at = (size_t)min(n + i, N - 1) * K + k;
+                const float w = W[at], w2 = PAIR ? W2[at] : 0.f;
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    acc[j][i] = fmaf(v[j], w, acc[j][i]);
+                    if (PAIR) acc2[j][i] = fmaf(v[j], w2, acc2[j][i]);
+                }
+            }
+        }
+        auto total = [](float v) {
+#pragma unroll
+            for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+            return v;
+        };
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            float scale = 1.f;
+            if (p.gain) scale = __fdiv_rn(1.0f, sqrtf(__fadd_rn(__fdiv_rn(total(ss[j]), (float)K), p.eps)));
+            if (p.row_weight) scale *= p.row_weight[min(t0 + j, T - 1)];
+            f4_t y, u = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                y[i] = total(acc[j][i]) * scale;
+                if (PAIR) u[i] = total(acc2[j][i]) * scale;
+            }
+            if (lane == 0 && t0 + j < T) f32_finish<PAIR>(p, sg, t0 + j, n, y, u, !PAIR && sg.kind == F32Out::ADD ? f32_old(sg, t0 + j, n) : u);
+        }
+    }
+}
+
+void launch_gemm_f32(const F32Gemm& g, int prof_cls) {
+    if (g.T <= 0 || g.n_segs == 0) return;
+    F32Gemm a = g;
+    const bool pair = a.seg[0].W2 != nullptr;
+    double weights = 0, outs = 0;
+    int blocks = 0;   // 16-row blocks of W (of each matrix of a pair)
+    auto aligned = [](const void* q) { return (reinterpret_cast<size_t>(q) & 15) == 0; };
+    bool rows16 = a.K % 4 == 0 && aligned(a.in) && aligned(a.gain);
+    for (int s = 0; s < a.n_segs; s++) {
+        F32Segment& q = a.seg[s];
+        if (pair != (q.W2 != nullptr) || q.N <= 0) NVLLM_FATAL("fp32 projection: segment %d of %d", s, a.n_segs);
+        rows16 = rows16 && aligned(q.W) && aligned(q.W2) && a.expert_stride % 4 == 0;
+        q.vec = q.N % 4 == 0 && q.ldo % 4 == 0 && aligned(q.out);
+        weights += (double)q.N * a.K * (pair ? 2 : 1);
+        outs += q.N;
+        blocks += cdiv(q.N, 16);
+    }
+    // Blocks per wave.  A launch takes about what its busiest CU has to fetch (64 bytes per block and k, at about 20 bytes
+    // per cycle of the mix of weights and activations) and to multiply (8 cycles per product and quad of k on four SIMDs):
+    // larger tiles fetch less per product, smaller ones reach more CUs.  K = 512 at 301 tokens: 2 x 2 blocks of a 512-wide
+    // output 8 us, 1 x 1 10 us; 2 x 4 of a 1,536-wide one 13.7 us against 17.0 in 2 x 2.
+    const int Tb = cdiv(a.T, 16), cus = rt().num_cus, steps = cdiv(a.K, F32_STEP);
+    static const int shapes[][2] = {{1, 1}, {1, 2}, {2, 2}, {2, 4}}, pair_shapes[][2] = {{1, 1}, {1, 2}, {1, 4}};
+    int NB = 1, TB = 1;
+    long tiles_all = (long)blocks * Tb;
+    if (!a.block_expert && rows16) {
+        double best = 0;
+        for (int i = 0; i < (pair ? 3 : 4); i++) {
+            const int nb = pair ? pair_shapes[i][0] : shapes[i][0], tb = pair ? pair_shapes[i][1] : shapes[i][1], nt = pair ? 2 * nb : nb;
+            const long tiles = (long)cdiv(blocks, nb) * cdiv(Tb, tb);
+            const double cost = (double)cdiv((int)std::min(tiles, 1L << 30), cus) * ((nt + tb) * 64.0 / 20.0 + nt * tb * 2.0);
+            if (i == 0 || cost < best) best = cost, NB = nb, TB = tb, tiles_all = tiles;
+        }
+    }
+    // slices of K (they meet in LDS): until every SIMD has two waves; a slice keeps a step at least
+    int KS = 1;
+    while (KS < (TB == 4 ? 4 : 8) && KS * 2 <= steps && tiles_all * KS < (a.block_expert ? 16L : 8L) * cus) KS *= 2;   // (a grid of experts is an upper bound)
+    int tiles = 0;
+    for (int s = 0; s < a.n_segs; s++) {
+        a.seg[s].first = tiles;
+        tiles += cdiv(cdiv(a.seg[s].N, 16), NB);
+    }
+    ProfScope ps(prof_cls, 4.0 * (weights + (double)a.T * (a.K + outs)), 2.0 * a.T * weights);
+    if (!rows16) {
+        const dim3 grid(tiles, std::min(cdiv(a.T, 4), 32768));
+        if (pair) NVLLM_LAUNCH(k_gemm_f32_any<true>, grid, dim3(256), 0, a);
+        else NVLLM_LAUNCH(k_gemm_f32_any<false>, grid, dim3(256), 0, a);
+        return;
+    }
+    const int waves = f32_waves(KS);
+    const dim3 grid(cdiv(tiles, waves / KS), cdiv(Tb, TB));
+#define NVLLM_GEMM_F32_KS(nb, tb, ks, pr)                                                                                \
+    do {                                                                                                                 \
+        if (a.gain) NVLLM_LAUNCH((k_gemm_f32<nb, tb, ks, pr, true>), grid, dim3(waves * 64), 0, a);                      \
+        else NVLLM_LAUNCH((k_gemm_f32<nb, tb, ks, pr, false>), grid, dim3(waves * 64), 0, a);                            \
+    } while (0)
+#define NVLLM_GEMM_F32(nb, tb, pr, eight)                                                                                \
+    do {                                                                                                                 \
+        if (KS == 1) NVLLM_GEMM_F32_KS(nb, tb, 1, pr);                                                                    \
+        else if (KS == 2) NVLLM_GEMM_F32_KS(nb, tb, 2, pr);                                                               \
+        else if (KS == 4 || !(eight)) NVLLM_GEMM_F32_KS(nb, tb, 4, pr);                                                   \
+        else NVLLM_GEMM_F32_KS(nb, tb, (eight) ? 8 : 4, pr);                                                              \
+    } while (0)
+    if (pair) {
+        if (TB == 1) NVLLM_GEMM_F32(1, 1, true, true);
+        else if (TB == 2) NVLLM_GEMM_F32(1, 2, true, true);
+        else NVLLM_GEMM_F32(1, 4, true, false);
+    } else if (TB == 1) {
+        NVLLM_GEMM_F32(1, 1, false, true);
+    } else if (TB == 2) {
+        if (NB == 1) NVLLM_GEMM_F32(1, 2, false, true);
+        else NVLLM_GEMM_F32(2, 2, false, true);
+    } else {
+        NVLLM_GEMM_F32(2, 4, false, false);
+    }
+#undef NVLLM_GEMM_F32
+#undef NVLLM_GEMM_F32_KS
+}
+
+}  // namespace nvllm

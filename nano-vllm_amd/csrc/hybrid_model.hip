@@ -18,6 +18,7 @@
 #include <cstring>
 
 #include "gemm_common.h"
+#include "gemm_f32.h"
 #include "lightning.h"
 #include "model_dir.h"
 #include "moe.h"
@@ -630,48 +631,46 @@ void HybridModel::forward_b16(const PassArgs& a, const StepArrays& st) {
 
 void HybridModel::forward_f32(const PassArgs& a, const StepArrays& st) {
     const int T = a.T, B = a.B;
-    size_t wide = D_, q_row = 0, z_ld = 0, ints = 0;
+    size_t mixer = 0, dense = 0, rows_up = 0, rows_down = 0, shared = 0, q_row = 0, z_ld = 0, ints = 0;
     for (const auto& l : layers_) {
         const MixerSizes& m = l.m;
         const FfSizes& f = l.f;
         const size_t H = m.heads;
-        wide = std::max({wide, H * m.vdim, (size_t)f.dense, (size_t)f.top * std::max(f.expert_ff, D_), (size_t)f.shared_ff});
-        if (m.lightning) wide = std::max(wide, H * m.dim);
-        else wide = std::max(wide, (size_t)m.channels());
+        mixer = std::max(mixer, std::max(H * m.vdim, m.lightning ? H * m.dim : (size_t)m.channels()));
+        dense = std::max({dense, (size_t)f.dense, (size_t)f.shared_ff});
+        if (f.shared_ff) shared = D_;
         q_row = std::max(q_row, H * m.dim);
         if (f.experts) {
             z_ld = std::max(z_ld, (size_t)f.experts + 1);
             ints = std::max(ints, route_ints(T, f.experts, f.top, 16));
+            const size_t cap = route_plan(nullptr, T, f.experts, f.top, 16).capacity;
+            rows_up = std::max(rows_up, cap * f.expert_ff);
+            rows_down = std::max(rows_down, cap * D_);
         }
     }
-    auto rows = [&](WsSlot slot, size_t n) { return (float*)ws_get(slot, (size_t)T * n * sizeof(float)); };
-    float *x = rows(WS_STREAMS, D_), *act = rows(WS_A16_X, D_), *b = rows(WS_F32_A, wide), *c = rows(WS_F32_B, wide), *d = rows(WS_F32_C, wide);
-    float *q = rows(WS_Q_ROWS, q_row), *z = rows(WS_MISC, z_ld);
+    auto floats = [&](WsSlot slot, size_t n) { return (float*)ws_get(slot, n * sizeof(float)); };
+    float *x = floats(WS_STREAMS, (size_t)T * D_), *b = floats(WS_F32_A, std::max((size_t)T * std::max(mixer, dense), rows_up));
+    float *c = floats(WS_F32_B, (size_t)T * std::max({mixer, shared, (size_t)D_})), *d = floats(WS_F32_C, std::max((size_t)T * mixer, rows_down));
+    float *q = floats(WS_Q_ROWS, (size_t)T * q_row), *z = floats(WS_MISC, (size_t)T * z_ld), *gate = floats(WS_A16_X, (size_t)T * mixer);
     int* route_mem = (int*)ws_get(WS_LATENT, ints * sizeof(int));
     launch_embed_streams(x, embed_, false, st.d_tokens, T, 1, D_, st.d_tok_src, a.d_argmax);
     for (size_t run = 0; run < source_.size(); run++) {
         const HybridLayer& w = layers_[source_[run]];
         const MixerSizes& m = w.m;
         const FfSizes& f = w.f;
-        const int H = m.heads;
-        launch_rmsnorm_f32(act, x, w.norm[0], D_, T, eps_);
+        const int H = m.heads, vn = H * m.vdim;
+        auto normed = [&](int part) { return F32Gemm(x, T, D_).norm(w.norm[part], eps_); };   // a projection of the normed residual
         if (m.lightning) {
-            const int qn = H * m.dim, vn = H * m.vdim;
-            launch_matmul_f32w(q, act, w.in32[0], T, D_, qn);
-            launch_matmul_f32w(b, act, w.in32[1], T, D_, qn);
-            launch_matmul_f32w(c, act, w.in32[2], T, D_, vn);
-            launch_silu(q, (long)T * qn);
-            launch_silu(b, (long)T * qn);
-            launch_silu(c, (long)T * vn);
+            const int qn = H * m.dim;
+            F32Gemm in = normed(0).add(w.in32[0], qn, q, F32Out::SILU).add(w.in32[1], qn, b, F32Out::SILU).add(w.in32[2], vn, c, F32Out::SILU);
+            launch_gemm_f32(in.add(w.in32[3], vn, gate), PC_GEMM_QKV);
             Lightning l = lightning(w, (int)run);
             l.q32 = q; l.k32 = b; l.v32 = c; l.out_f32 = d;
             launch_lightning(l, st);
             launch_rmsnorm_f32(d, d, w.head_norm, vn, T, eps_);
-            launch_matmul_f32w(b, act, w.in32[3], T, D_, vn);
-            launch_sigmoid_gate(d, d, b, (long)T * vn);
-            launch_matmul_f32w(b, d, w.o32, T, vn, D_);
+            launch_sigmoid_gate(d, d, gate, (long)T * vn);
         } else {
-            launch_matmul_f32w(c, act, w.in32[0], T, D_, m.channels());
+            launch_gemm_f32(normed(0).add(w.in32[0], m.channels(), c), PC_GEMM_QKV);
             const KvPages pool = pages(a.mgr, (int)run);
             ConvRope r = conv_rope(w, (int)run, st);
             r.raw = c; r.raw_ld = m.channels(); r.q_out = q;
@@ -679,41 +678,37 @@ void HybridModel::forward_f32(const PassArgs& a, const StepArrays& st) {
             WindowAttn t = attention(w, pool);
             t.q = q; t.out_f32 = d;
             launch_window_attention(t, st);
-            launch_matmul_f32w(b, d, w.o32, T, H * m.vdim, D_);
         }
-        launch_accum(x, b, (long)T * D_);
+        launch_gemm_f32(F32Gemm(d, T, vn).add(w.o32, D_, x, F32Out::ADD), PC_GEMM_WO);
         if (!f.any()) continue;
-        launch_rmsnorm_f32(act, x, w.norm[1], D_, T, eps_);
         if (f.dense) {
-            launch_matmul_f32w(b, act, w.up32, T, D_, f.dense);
-            launch_relu2(b, (long)T * f.dense);
-            launch_matmul_f32w(c, b, w.down32, T, f.dense, D_);
-            launch_accum(x, c, (long)T * D_);
+            launch_gemm_f32(normed(1).add(w.up32, f.dense, b, F32Out::RELU2), PC_GEMM_GATEUP);
+            launch_gemm_f32(F32Gemm(b, T, f.dense).add(w.down32, D_, x, F32Out::ADD), PC_GEMM_DOWN);
             continue;
         }
         const int ldz = f.experts + 1;
-        launch_matmul_f32w(z, act, w.router32, T, D_, ldz);
+        launch_gemm_f32(normed(1).add(w.router32, ldz, z), PC_GEMM_ROUTER);
         const RoutePlan plan = route_plan(route_mem, T, f.experts, f.top, 16);
         launch_route(plan, z, ldz);
-        launch_matmul_experts_f32(b, act, w.gate32, plan, true, D_, f.expert_ff);
-        launch_matmul_experts_f32(c, act, w.up32, plan, true, D_, f.expert_ff);
-        launch_swiglu(b, b, c, (long)T * f.top * f.expert_ff);
-        launch_matmul_experts_f32(d, b, w.down32, plan, false, f.expert_ff, D_);
+        const long expert = (long)f.expert_ff * D_;
+        F32Gemm up = F32Gemm(x, plan.capacity, D_).norm(w.norm[1], eps_).experts(plan.block_expert, expert, plan.weight);
+        up.in_rows = plan.source;
+        launch_gemm_f32(up.add_pair(w.gate32, w.up32, f.expert_ff, b), PC_GEMM_EXPERT_UP);
+        launch_gemm_f32(F32Gemm(b, plan.capacity, f.expert_ff).experts(plan.block_expert, expert, nullptr).add(w.down32, D_, d), PC_GEMM_EXPERT_DOWN);
         if (f.shared_ff) {
-            launch_matmul_f32w(b, act, w.shared_gate32, T, D_, f.shared_ff);
-            launch_matmul_f32w(c, act, w.shared_up32, T, D_, f.shared_ff);
-            launch_swiglu(b, b, c, (long)T * f.shared_ff);
-            launch_matmul_f32w(c, b, w.shared_down32, T, f.shared_ff, D_);
+            launch_gemm_f32(normed(1).add_pair(w.shared_gate32, w.shared_up32, f.shared_ff, b), PC_GEMM_SHARED_UP);
+            launch_gemm_f32(F32Gemm(b, T, f.shared_ff).add(w.shared_down32, D_, c), PC_GEMM_SHARED_DOWN);
         }
         MoeCombine mc{};
-        mc.x = x; mc.rows = d; mc.top = f.top; mc.shared = f.shared_ff ? c : nullptr; mc.z = z; mc.ldz = ldz; mc.z_col = f.experts; mc.ld = D_;
+        mc.x = x; mc.rows = d; mc.row_of = plan.row_of; mc.top = f.top; mc.shared = f.shared_ff ? c : nullptr; mc.z = z; mc.ldz = ldz;
+        mc.z_col = f.experts; mc.ld = D_;
         launch_moe_combine(mc, T);
     }
     if (B <= 0) return;
     wait_for_row_copies();
-    launch_rmsnorm_f32(act, x, final_norm_, D_, T, eps_);
-    launch_gather_rows_f32(b, act, st.d_out_idx, B, D_);
-    launch_matmul_f32w(a.d_logits, b, (const float*)embed_, B, D_, V_);
+    F32Gemm head = F32Gemm(x, B, D_).norm(final_norm_, eps_);
+    head.in_rows = st.d_out_idx;
+    launch_gemm_f32(head.add((const float*)embed_, V_, a.d_logits), PC_GEMM_HEAD);
     launch_argmax_ld(a.d_argmax, a.d_logits, B, V_, V_, a.argmax_host);
 }
 

@@ -4,6 +4,7 @@
 #include <vector>
 
 #include "gemm_common.h"
+#include "gemm_f32.h"
 #include "latent_attention.h"
 #include "lightning.h"
 #include "model_dir.h"
@@ -170,14 +171,14 @@ void nvllm_expert_ff(float* out, int* choice, float* score, const float* in, con
     if (score) device_memcpy(score, plan.score, pairs * 4, DEVICE_TO_DEVICE);
     if (!out) return;
     if (elem_bytes == 4) {
-        const Temp g(pairs * ff * 4), u(pairs * ff * 4), y(pairs * dim * 4);
-        launch_matmul_experts_f32(g.f(), in, gate, plan, true, dim, ff);
-        launch_matmul_experts_f32(u.f(), in, up, plan, true, dim, ff);
-        launch_swiglu(g.f(), g.f(), u.f(), (long)pairs * ff);
-        launch_matmul_experts_f32(y.f(), g.f(), down, plan, false, ff, dim);
+        const Temp g((size_t)plan.capacity * ff * 4), y((size_t)plan.capacity * dim * 4);
+        F32Gemm pair = F32Gemm(in, plan.capacity, dim).experts(plan.block_expert, (long)ff * dim, plan.weight);
+        pair.in_rows = plan.source;
+        launch_gemm_f32(pair.add_pair(gate, up, ff, g.f()), PC_GEMM_EXPERT_UP);
+        launch_gemm_f32(F32Gemm(g.f(), plan.capacity, ff).experts(plan.block_expert, (long)dim * ff, nullptr).add(down, dim, y.f()), PC_GEMM_EXPERT_DOWN);
         HIP_CHECK(hipMemsetAsync(out, 0, (size_t)num_tokens * dim * 4, rt().stream));
         MoeCombine c{};
-        c.x = out; c.rows = y.f(); c.top = top; c.ld = dim;
+        c.x = out; c.rows = y.f(); c.row_of = plan.row_of; c.top = top; c.ld = dim;
         launch_moe_combine(c, num_tokens);
         return;
     }

@@ -21,6 +21,7 @@
 #include <memory>
 
 #include "gemm_common.h"
+#include "gemm_f32.h"
 #include "latent_attention.h"
 #include "model_dir.h"
 
@@ -473,32 +474,29 @@ void LatentHyperModel::forward_f32(const PassArgs& a, const StepArrays& st) {
         const Mixer& m = w.m;
         const int H = m.heads;
         if (s.part == 1) {
-            launch_matmul_f32w(b, act, w.gate, T, D_, w.ff);
-            launch_matmul_f32w(c, act, w.up, T, D_, w.ff);
-            launch_swiglu_bias(b, b, c, w.bias_gate, w.bias_up, T, w.ff);
-            launch_matmul_f32w(c, b, w.down32, T, w.ff, D_);
+            launch_gemm_f32(F32Gemm(act, T, D_).add_pair(w.gate, w.up, w.ff, b, w.bias_gate, w.bias_up), PC_GEMM_GATEUP);
+            launch_gemm_f32(F32Gemm(b, T, w.ff).add(w.down32, D_, c), PC_GEMM_DOWN);
             step(c, w.bias_down, w.ls[1], s.record, s.next_w, s.next_b);
             continue;
         }
         const float2* rope = rotation_table(m.base, m.rot, st.max_pos + 1);
-        launch_matmul_f32w(b, act, w.dq, T, D_, m.q_rank);
-        launch_rmsnorm_f32(b, b, w.gain_q, m.q_rank, T, eps_);
-        launch_matmul_f32w(c, b, w.uq32, T, m.q_rank, H * (m.dim + m.rot));
+        launch_gemm_f32(F32Gemm(act, T, D_).add(w.dq, m.q_rank, b).add(w.dkv, m.rank + m.rot, raw), PC_GEMM_LATENT_IN);
+        launch_gemm_f32(F32Gemm(b, T, m.q_rank).norm(w.gain_q, eps_).add(w.uq32, H * (m.dim + m.rot), c), PC_GEMM_LATENT_Q);
         launch_latent_q_f32(q, c, w.uk32, rope, st.d_pos, T, H, m.dim, m.rot, m.rank);
-        launch_matmul_f32w(raw, act, w.dkv, T, D_, m.rank + m.rot);
         const LatentPool pl = pool(a.mgr, s.run);
         launch_latent_kv(pl, raw, m.rank + m.rot, m.rank, w.gain_kv, eps_, rope, st);
         LatentAttn at{};
         at.pool = pl; at.q = q; at.sink = w.sink; at.scale = m.scale; at.H = H; at.out_f32 = latents;
         launch_latent_attention(at, st);
         launch_latent_v_f32(b, latents, w.uv32, T, H, m.vdim, m.rank);
-        launch_matmul_f32w(c, b, w.o32, T, H * m.vdim, D_);
+        launch_gemm_f32(F32Gemm(b, T, H * m.vdim).add(w.o32, D_, c), PC_GEMM_WO);
         step(c, nullptr, w.ls[0], s.record, s.next_w, s.next_b);
     }
     if (B <= 0) return;
     wait_for_row_copies();
-    launch_gather_rows_f32(b, act, st.d_out_idx, B, D_);
-    launch_matmul_f32w(a.d_logits, b, (const float*)embed_, B, D_, V_);
+    F32Gemm head(act, B, D_);
+    head.in_rows = st.d_out_idx;
+    launch_gemm_f32(head.add((const float*)embed_, V_, a.d_logits), PC_GEMM_HEAD);
     launch_softcap(a.d_logits, softcap_, (long)B * V_);
     launch_argmax_ld(a.d_argmax, a.d_logits, B, V_, V_, a.argmax_host);
 }

@@ -33,6 +33,5 @@ void launch_lightning(const Lightning& a, const StepArrays& st);
 
 // out = x * sigmoid(g) (fp32 path: the gate on the normed heads)
 void launch_sigmoid_gate(float* out, const float* x, const float* g, long n);
-void launch_silu(float* x, long n);
 
 }  // namespace nvllm

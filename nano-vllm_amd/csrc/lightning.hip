@@ -552,14 +552,5 @@ void launch_sigmoid_gate(float* out, const float* x, const float* g, long n) {
     ProfScope ps(PC_ELEMWISE, (double)n * 12.0, 0);
     NVLLM_LAUNCH(k_sigmoid_gate, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, out, x, g, n);
 }
-__global__ __launch_bounds__(256) void k_silu(float* x, long n) {
-    const long i = (long)blockIdx.x * 256 + threadIdx.x;
-    if (i < n) x[i] = silu_mul(x[i], 1.f);
-}
-void launch_silu(float* x, long n) {
-    if (n <= 0) return;
-    ProfScope ps(PC_ELEMWISE, (double)n * 8.0, 0);
-    NVLLM_LAUNCH(k_silu, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, x, n);
-}
 
 }  // namespace nvllm

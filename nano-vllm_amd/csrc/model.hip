@@ -7,6 +7,7 @@
 #include <sys/stat.h>
 #include <vector>
 
+#include "gemm_f32.h"
 #include "model_dir.h"
 #include "nvllm_internal.h"
 #include "step_arrays.h"
@@ -322,8 +323,8 @@ static void load_model_f32(Weights* w, Config* p, FILE* f, bool shared) {
     printf("DEBUG: Embed[100]: %f\n", dbg100);
 }
 
-// The reference's layer loop (model.c:352-418) on fp32 weights, one operator launch per
-// reference call; leaves the logits of the output rows in d_logits.
+// The reference's layer loop (model.c:352-418) on fp32 weights, five launches a layer: the norms, rotation, cache write,
+// SwiGLU and residual adds ride in the projections (gemm_f32.hip).  Leaves the logits of the output rows in d_logits.
 static void forward_f32(const StepArrays& st, int T, int B, Config* p, RunState* s, Weights* w, const KvPoolView& pool,
                         const float2* rope, float* d_logits) {
     const int D = p->dim, F = p->hidden_dim, hd = p->head_dim, H = p->n_heads, KVH = p->n_kv_heads;
@@ -332,12 +333,12 @@ static void forward_f32(const StepArrays& st, int T, int B, Config* p, RunState*
     launch_gather_rows_f32(s->x, w->token_embedding_table, st.d_tokens, T, D);
     for (int l = 0; l < p->n_layers; l++) {
         const LayerWeights& lw = w->layers[l];
-        launch_rmsnorm_f32(s->xb, s->x, lw.rms_att_weight, D, T, eps);
-        launch_matmul_f32w(s->q, s->xb, lw.wq, T, D, QD);
-        launch_matmul_f32w(s->k, s->xb, lw.wk, T, D, KD);
-        launch_matmul_f32w(s->v, s->xb, lw.wv, T, D, KD);
-        launch_rope(s->q, s->k, st.d_pos, 0, rope, T, H, KVH, hd);
-        launch_kv_write(s->k, s->v, st.d_pos, 0, st.d_seq, st.d_tbl_off, st.d_tables, pool, l, st.write_limit, KVH, hd);
+        F32Gemm qkv = F32Gemm(s->x, T, D).norm(lw.rms_att_weight, eps);
+        qkv.add(lw.wq, QD, s->q, F32Out::ROPE_Q).add(lw.wk, KD, nullptr, F32Out::ROPE_K).add(lw.wv, KD, nullptr, F32Out::KV_V);
+        qkv.pos = st.d_pos; qkv.kv_row = st.d_kv_row; qkv.rope = rope;
+        qkv.pool_k = pool.k; qkv.pool_v = pool.v; qkv.kv_elem_bytes = pool.elem_bytes; qkv.bs = pool.block_size;
+        qkv.layer_off = (long)l * pool.layer_stride; qkv.hd = hd; qkv.KD = KD;
+        launch_gemm_f32(qkv, PC_GEMM_QKV);
         AttnArgs at{};
         at.q = s->q;
         at.out_f32 = s->xb2;
@@ -352,18 +353,13 @@ static void forward_f32(const StepArrays& st, int T, int B, Config* p, RunState*
         at.kv_rows = st.kv_rows;
         at.qk_pairs = st.qk_pairs;
         launch_paged_attention(at);
-        launch_matmul_f32w(s->xb, s->xb2, lw.wo, T, QD, D);
-        launch_accum(s->x, s->xb, (long)T * D);
-        launch_rmsnorm_f32(s->xb, s->x, lw.rms_ffn_weight, D, T, eps);
-        launch_matmul_f32w(s->hb, s->xb, lw.w_gate, T, D, F);
-        launch_matmul_f32w(s->hb2, s->xb, lw.w_up, T, D, F);
-        launch_swiglu(s->hb, s->hb, s->hb2, (long)T * F);
-        launch_matmul_f32w(s->xb, s->hb, lw.w_down, T, F, D);
-        launch_accum(s->x, s->xb, (long)T * D);
+        launch_gemm_f32(F32Gemm(s->xb2, T, QD).add(lw.wo, D, s->x, F32Out::ADD), PC_GEMM_WO);
+        launch_gemm_f32(F32Gemm(s->x, T, D).norm(lw.rms_ffn_weight, eps).add_pair(lw.w_gate, lw.w_up, F, s->hb), PC_GEMM_GATEUP);
+        launch_gemm_f32(F32Gemm(s->hb, T, F).add(lw.w_down, D, s->x, F32Out::ADD), PC_GEMM_DOWN);
     }
-    launch_rmsnorm_f32(s->x, s->x, w->rms_final_weight, D, T, eps);
-    launch_gather_rows_f32(s->xb, s->x, st.d_out_idx, B, D);
-    launch_matmul_f32w(d_logits, s->xb, w->lm_head, B, D, V);
+    F32Gemm head = F32Gemm(s->x, B, D).norm(w->rms_final_weight, eps);
+    head.in_rows = st.d_out_idx;
+    if (B > 0) launch_gemm_f32(head.add(w->lm_head, V, d_logits), PC_GEMM_HEAD);
 }
 
 }  // namespace nvllm

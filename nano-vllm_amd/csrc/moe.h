@@ -29,7 +29,7 @@ void launch_expert_rows(__half* dst, const float* x, const float* gain, const Ro
 // x += sum of the chosen experts' rows + sigmoid(z_shared) * shared;  then what the next sublayer needs of x
 struct MoeCombine {
     float* x;                  // [T][ld]
-    const float* rows;         // expert results [row][ld], rows by row_of (null: by token and choice, [T][top][ld])
+    const float* rows;         // expert results [row][ld], rows by row_of
     const int* row_of;
     int top;
     const float* shared;       // [T][ld] or null
@@ -41,9 +41,5 @@ struct MoeCombine {
     int ld;
 };
 void launch_moe_combine(const MoeCombine& m, int T);
-// fp32 path: out[i][n] = sum_k w[expert(i)][n][k] * scale(i) * in[row(i)][k], i = token * top + choice;
-// row(i) = i, or the token when by_token (then the input is scaled by its score)
-void launch_matmul_experts_f32(float* out, const float* in, const float* w, const RoutePlan& r, bool by_token, int K, int N);
-void launch_relu2(float* x, long n);
 
 }  // namespace nvllm

@@ -233,7 +233,7 @@ __global__ __launch_bounds__(256) void k_moe_combine(MoeCombine m, int top) {
 #pragma unroll
             for (int e = 0; e < VEC; e++) y.v[e] = 0.f;
             for (int j = 0; j < top; j++) {
-                const size_t row = m.row_of ? (size_t)m.row_of[(size_t)t * top + j] : (size_t)t * top + j;
+                const size_t row = (size_t)m.row_of[(size_t)t * top + j];
                 const Vec r = *reinterpret_cast<const Vec*>(m.rows + row * m.ld + n);
 #pragma unroll
                 for (int e = 0; e < VEC; e++) y.v[e] += r.v[e];
@@ -271,39 +271,6 @@ void launch_moe_combine(const MoeCombine& m, int T) {
     ProfScope ps(PC_MOE_COMBINE, (double)T * m.ld * (4.0 * m.top + (m.shared ? 4.0 : 0.0) + 8.0 + (m.out_b16 ? 2.0 : 0.0)), 0);
     if (m.ld % 4 == 0) NVLLM_LAUNCH((k_moe_combine<4>), dim3(T), dim3(256), 0, m, m.top);
     else NVLLM_LAUNCH((k_moe_combine<1>), dim3(T), dim3(256), 0, m, m.top);
-}
-
-// ------------------------------------------------------------------ fp32 path
-__global__ __launch_bounds__(256) void k_matmul_experts_f32(float* __restrict__ out, const float* __restrict__ in, const float* __restrict__ w,
-                                                            const int* __restrict__ choice, const float* __restrict__ score, int top, int by_token, int K, int N) {
-    const int i = blockIdx.x, n = blockIdx.y * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-    if (n >= N) return;
-    const float* x = in + (size_t)(by_token ? i / top : i) * K;
-    const float* wr = w + ((size_t)choice[i] * N + n) * K;
-    const float scale = by_token ? score[i] : 1.f;
-    float acc = 0.f;
-    for (int k = lane; k < K; k += 64) acc = fmaf(scale * x[k], wr[k], acc);
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o, 64);
-    if (lane == 0) out[(size_t)i * N + n] = acc;
-}
-void launch_matmul_experts_f32(float* out, const float* in, const float* w, const RoutePlan& r, bool by_token, int K, int N) {
-    const int pairs = r.T * r.top;
-    if (pairs <= 0) return;
-    ProfScope ps(PC_GEMM_OTHER, (double)std::min(r.E, pairs) * N * K * 4.0 + (double)pairs * (K + N) * 4.0, 2.0 * pairs * (double)N * K);
-    NVLLM_LAUNCH(k_matmul_experts_f32, dim3(pairs, cdiv(N, 4)), dim3(256), 0, out, in, w, r.choice, r.score, r.top, by_token ? 1 : 0, K, N);
-}
-__global__ __launch_bounds__(256) void k_relu2(float* x, long n) {
-    const long i = (long)blockIdx.x * 256 + threadIdx.x;
-    if (i < n) {
-        const float v = fmaxf(x[i], 0.f);
-        x[i] = v * v;
-    }
-}
-void launch_relu2(float* x, long n) {
-    if (n <= 0) return;
-    ProfScope ps(PC_ELEMWISE, (double)n * 8.0, 0);
-    NVLLM_LAUNCH(k_relu2, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, x, n);
 }
 
 }  // namespace nvllm

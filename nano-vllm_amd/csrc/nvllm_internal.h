@@ -385,7 +385,6 @@ struct ExpertRows {
 void launch_gemm_experts(const B16Weight& w, int experts, const __half* act, const ExpertRows& rows, const GemmEpilogue& epi, int prof_cls);
 
 void launch_pack_a16(__half* a16, const float* in, int T, int K);
-void launch_matmul_f32w(float* out, const float* in, const float* w, int T, int K, int N);
 
 void launch_rmsnorm_f32(float* o, const float* x, const float* gain, int D, int T, float eps);
 

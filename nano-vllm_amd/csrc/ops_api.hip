@@ -6,6 +6,7 @@
 #include <unordered_map>
 #include <vector>
 
+#include "gemm_f32.h"
 #include "latent_attention.h"
 #include "model_dir.h"
 #include "nvllm_internal.h"
@@ -253,7 +254,7 @@ void matmul(float* out, float* in, float* weight, int num_tokens, int in_dim, in
     ensure_init();
     const WeightEntry* w = find_weight(weight);
     if (!w) {  // a plain fp32 [out_dim, in_dim] device buffer
-        launch_matmul_f32w(out, in, weight, num_tokens, in_dim, out_dim);
+        if (out_dim > 0) launch_gemm_f32(F32Gemm(in, num_tokens, in_dim).add(weight, out_dim, out), PC_GEMM_OTHER);
         return;
     }
     if (w->rowmajor && !w->tiles) NVLLM_FATAL("matmul: the embedding table handle is not a projection weight");
