@@ -1,4 +1,5 @@
-// gemm_f32.h -- projections of models whose weights and activations are fp32 (row-major, as the files hold them).
+// gemm_f32.h -- projections whose activations are fp32 rows: of fp32 weights (row-major, as the files hold them), and of
+// fp16 weights in tile order for a few tokens.
 #pragma once
 
 #include "nvllm_internal.h"
@@ -16,9 +17,10 @@ enum class F32Out {
     KV_V      // -> value rows of the block pool
 };
 struct F32Segment {
-    const float* W;      // [N][K]
+    const float* W;      // [N][K]; fp16 weights: tiles, ...
     const float* W2;     // second matrix of a gated pair: out = silu(y + bias) * (y2 + bias2) (null: none)
     const float *bias, *bias2;   // of a pair, per feature (null: none)
+    long nb_stride;      // ... halves between their 16-row blocks
     int N;
     F32Out kind;
     float* out;          // [T][ldo]
@@ -40,6 +42,9 @@ struct F32Gemm {
     const int* block_expert = nullptr;
     long expert_stride = 0;
     const float* row_weight = nullptr;
+    // fp16 weights, one STORE segment: (maximum, its first index) of each 16 outputs of a token -> [block][amax_ld]
+    float2* amax_pairs = nullptr;
+    int amax_ld = 0;
     // ROPE_*, KV_V
     const int* pos = nullptr;
     const int* kv_row = nullptr;
@@ -56,11 +61,15 @@ struct F32Gemm {
         return *this;
     }
     F32Gemm& add(const float* W, int N, float* out, F32Out kind = F32Out::STORE) {
-        seg[n_segs++] = F32Segment{W, nullptr, nullptr, nullptr, N, kind, out, N, 0, false};
+        seg[n_segs++] = F32Segment{W, nullptr, nullptr, nullptr, 0, N, kind, out, N, 0, false};
+        return *this;
+    }
+    F32Gemm& add16(const __half* tiles, long nb_stride, int N, float* out, F32Out kind = F32Out::STORE, const __half* tiles2 = nullptr) {
+        seg[n_segs++] = F32Segment{(const float*)tiles, (const float*)tiles2, nullptr, nullptr, nb_stride, N, kind, out, N, 0, false};
         return *this;
     }
     F32Gemm& add_pair(const float* gate, const float* up, int N, float* out, const float* bias_gate = nullptr, const float* bias_up = nullptr) {
-        seg[n_segs++] = F32Segment{gate, up, bias_gate, bias_up, N, F32Out::STORE, out, N, 0, false};
+        seg[n_segs++] = F32Segment{gate, up, bias_gate, bias_up, 0, N, F32Out::STORE, out, N, 0, false};
         return *this;
     }
     F32Gemm& experts(const int* blocks, long stride, const float* weight) {
@@ -72,5 +81,10 @@ struct F32Gemm {
 };
 // One launch for all segments: all of them gated pairs, or none.
 void launch_gemm_f32(const F32Gemm& g, int prof_cls);
+
+// The same for fp16 weights in tile order (add16) and up to THIN_TOKENS tokens; K % 32 == 0.  Activations enter the matrix
+// cores as fp16 hi + lo, as in gemm.hip.
+constexpr int THIN_TOKENS = 8;   // (at most 16: one block of tokens)
+void launch_gemm_thin(const F32Gemm& g, int prof_cls);
 
 }  // namespace nvllm

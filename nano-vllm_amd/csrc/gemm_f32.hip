@@ -16,78 +16,12 @@
 #include <algorithm>
 
 #include "gemm_common.h"
-#include "gemm_f32.h"
+#include "gemm_f32_tail.h"
 
 namespace nvllm {
 
 constexpr int F32_STEP = 32;   // k per step: 128 bytes, a cache line, of every row
 constexpr int f32_waves(int KS) { return KS == 8 ? 8 : 4; }   // waves of a workgroup: feature tiles x slices of K
-
-// What follows a token's complete sums of features n .. n+3 (n % 4 == 0; `old`: what ADD adds to).
-template <bool PAIR>
-__device__ __forceinline__ void f32_finish(const F32Gemm& p, const F32Segment& sg, int t, int n, f4_t y, const f4_t u, const f4_t old) {
-    if constexpr (PAIR) {
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-            const int f = min(n + r, sg.N - 1);
-            y[r] = silu_mul(sg.bias ? y[r] + sg.bias[f] : y[r], sg.bias2 ? u[r] + sg.bias2[f] : u[r]);
-        }
-    } else {
-        switch (sg.kind) {
-            case F32Out::ADD:
-#pragma unroll
-                for (int r = 0; r < 4; r++) y[r] = __fadd_rn(old[r], y[r]);
-                break;
-            case F32Out::SILU:
-#pragma unroll
-                for (int r = 0; r < 4; r++) y[r] = silu_mul(y[r], 1.f);
-                break;
-            case F32Out::RELU2:
-#pragma unroll
-                for (int r = 0; r < 4; r++) y[r] = fmaxf(y[r], 0.f) * fmaxf(y[r], 0.f);
-                break;
-            case F32Out::ROPE_Q:
-            case F32Out::ROPE_K: {   // the two pairs of this quad turn (layers.c:118-141)
-                const float2* tab = p.rope + (size_t)p.pos[t] * (p.hd >> 1) + ((n % p.hd) >> 1);
-                const float2 c0 = tab[0], c1 = tab[1];
-                y = f4_t{__fsub_rn(__fmul_rn(y[0], c0.x), __fmul_rn(y[1], c0.y)), __fadd_rn(__fmul_rn(y[0], c0.y), __fmul_rn(y[1], c0.x)),
-                         __fsub_rn(__fmul_rn(y[2], c1.x), __fmul_rn(y[3], c1.y)), __fadd_rn(__fmul_rn(y[2], c1.y), __fmul_rn(y[3], c1.x))};
-                break;
-            }
-            default: break;
-        }
-        if (sg.kind == F32Out::ROPE_K || sg.kind == F32Out::KV_V) {
-            const int row = p.kv_row[t];
-            if (row < 0) return;
-            const bool is_k = sg.kind == F32Out::ROPE_K;
-            const float z[4] = {y[0], y[1], y[2], y[3]};
-            if (p.kv_elem_bytes == 4) {   // the reference's rows (memory.c:37-43)
-                kv_put4<float>(reinterpret_cast<float*>(is_k ? p.pool_k : p.pool_v) + p.layer_off + (size_t)row * p.KD + n, z);
-            } else {                      // fp16 pages in matrix-core operand order
-                __half* page = reinterpret_cast<__half*>(is_k ? p.pool_k : p.pool_v) + p.layer_off + kv16_page(row / p.bs, n / p.hd, p.KD / p.hd, p.hd);
-                if (is_k) kv_put4<__half>(page + kv16_k_off(row % p.bs, n % p.hd), z);
-                else kv_put4_strided<__half>(page + kv16_v_off(row % p.bs, n % p.hd), z);
-            }
-            return;
-        }
-    }
-    float* o = sg.out + (size_t)t * sg.ldo + n;
-    if (sg.vec) {
-        *reinterpret_cast<f4_t*>(o) = y;
-    } else {
-#pragma unroll
-        for (int r = 0; r < 4; r++)
-            if (n + r < sg.N) o[r] = y[r];
-    }
-}
-__device__ __forceinline__ f4_t f32_old(const F32Segment& sg, int t, int n) {   // t < T; features past the last are those of the last
-    const float* o = sg.out + (size_t)t * sg.ldo;
-    if (sg.vec) return *reinterpret_cast<const f4_t*>(o + min(n, sg.N - 4));
-    f4_t v;
-#pragma unroll
-    for (int r = 0; r < 4; r++) v[r] = o[min(n + r, sg.N - 1)];
-    return v;
-}
 
 template <int NB, int TB, int KS, bool PAIR, bool NORM>
 __global__ __launch_bounds__(f32_waves(KS) * 64) void k_gemm_f32(F32Gemm p) {
@@ -246,7 +180,7 @@ __global__ __launch_bounds__(f32_waves(KS) * 64) void k_gemm_f32(F32Gemm p) {
             y *= scale;
             if constexpr (PAIR) u *= scale;
         }
-        f32_finish<PAIR>(p, sg, t, n, y, u, old);
+        f32_finish<PAIR>(p, sg, t, n, y, u, old, PAIR ? zero : f32_turn(p, sg, t, n), PAIR ? -1 : f32_row(p, sg, t));
     };
     const bool adds = !PAIR && sg.kind == F32Out::ADD;
     if constexpr (KS == 1) {   // a lane's sums are complete: features 4g .. 4g + 3 of token x of every block pair
@@ -368,7 +302,8 @@ __global__ __launch_bounds__(256) void k_gemm_f32_any(F32Gemm p) {
                 y[i] = total(acc[j][i]) * scale;
                 if (PAIR) u[i] = total(acc2[j][i]) * scale;
             }
-            if (lane == 0 && t0 + j < T) f32_finish<PAIR>(p, sg, t0 + j, n, y, u, !PAIR && sg.kind == F32Out::ADD ? f32_old(sg, t0 + j, n) : u);
+            if (lane == 0 && t0 + j < T)
+                f32_finish<PAIR>(p, sg, t0 + j, n, y, u, !PAIR && sg.kind == F32Out::ADD ? f32_old(sg, t0 + j, n) : u, f32_turn(p, sg, t0 + j, n), f32_row(p, sg, t0 + j));
         }
     }
 }

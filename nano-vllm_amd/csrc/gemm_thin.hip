@@ -1,0 +1,217 @@
+// gemm_thin.hip -- projections of fp16 weights for up to 8 tokens: the layers of a model that serves one user or a few.
+//
+// The weights are all there is to read (2 bytes each, against 4 bytes per token and k of activations), so a launch is as
+// fast as its CUs can fetch: about 50 GB/s each from HBM, 128 CUs saturate it.  A workgroup therefore owns ONE 16-row block
+// (2,048 rows: 128 workgroups of 64 KiB), and its KS waves take the tiles of K round-robin, four tiles in flight each, and
+// meet in LDS: no K split across workgroups, whose close costs about 5 us.  Activations are plain fp32 rows, 32 bytes per
+// lane and tile (tile order would bring 16 rows where one is alive): the RMS norm in front (gain and sum of squares), the
+// split into fp16 hi + lo and the element-wise work behind the product happen here, and the next launch reads rows again.
+//
+// TinyLlama shape, one token, us per launch, 64-row tiles of gemm.hip (K cut over workgroups) and here: wo and w_down
+// together 18.2 and 15.5, gate/up 13.2 and 13.9, q/k/v 8.6 and 7.2; the pass 1,217 and 1,168.  At 9 tokens the two are
+// equal (1,558 and 1,575 a pass), from where the activations, read by every workgroup, weigh more: up to 8 tokens.
+// Eight rows to a workgroup instead of 16 (256 of them for wo and w_down) and six tiles in flight measured the same or
+// slower: it is the start of a launch, two dependent trips to memory, that is left.
+#include "gemm_f32_tail.h"
+#include "gemm_tile.h"
+
+namespace nvllm {
+
+// tiles in flight per wave, as many as 128 registers hold (16 waves per CU)
+constexpr int thin_ring(int NT, bool norm) { return NT == 1 ? 4 : NT == 2 ? (norm ? 3 : 4) : 2; }
+
+template <int NB, int KS, bool PAIR, bool NORM>
+__global__ __launch_bounds__(KS * 64) void k_gemm_thin(F32Gemm p) {
+    static_assert(!PAIR || NB == 1, "a pair is one block of either matrix");
+    static_assert(NB <= KS, "a wave finishes a block");
+    constexpr int NT = PAIR ? 2 : NB, RING = thin_ring(NT, NORM);
+    __shared__ f4_t s_red[KS][NT][64];
+    __shared__ float s_ss[KS][16];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int x = lane & 15, g = lane >> 4;
+    int s = 0;
+    while (s + 1 < p.n_segs && (int)blockIdx.x >= p.seg[s + 1].first) s++;
+    const F32Segment& sg = p.seg[s];
+    const int nb0 = ((int)blockIdx.x - sg.first) * NB;
+    const int K = p.K, T = p.T, N = sg.N, blocks = (N + 15) >> 4;
+    const h8_t* wp[NT];
+#pragma unroll
+    for (int n = 0; n < NT; n++) {
+        const float* W = PAIR && n == 1 ? sg.W2 : sg.W;
+        wp[n] = reinterpret_cast<const h8_t*>(reinterpret_cast<const __half*>(W) + (size_t)(PAIR ? nb0 : min(nb0 + n, blocks - 1)) * sg.nb_stride) + lane;
+    }
+    const int tx = min(x, T - 1);   // columns past the last token compute it again and are not stored
+    const float* ap = p.in + (size_t)(p.in_rows ? p.in_rows[tx] : tx) * K + 8 * g;
+    const float* gp = NORM ? p.gain + 8 * g : nullptr;
+    // what the epilogue needs beside the sums travels from the start
+    const int nb = nb0 + (PAIR ? 0 : wave), n0 = nb * 16 + 4 * g;   // of the block this wave finishes
+    f4_t turn = {0.f, 0.f, 0.f, 0.f};
+    int row = -1;
+    if (!PAIR && wave < NB) {
+        turn = f32_turn(p, sg, tx, n0);
+        row = f32_row(p, sg, tx);
+    }
+    h8_t w[RING][NT];
+    f4_t a[RING][2], gv[RING][NORM ? 2 : 1];
+    auto load = [&](int r, int i) {
+        const int kb = wave + i * KS;
+        __builtin_amdgcn_sched_barrier(0);   // requests stay in the order of their use: waits count what is younger
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            a[r][h] = *reinterpret_cast<const f4_t*>(ap + kb * 32 + 4 * h);
+            if constexpr (NORM) gv[r][h] = *reinterpret_cast<const f4_t*>(gp + kb * 32 + 4 * h);
+        }
+#pragma unroll
+        for (int n = 0; n < NT; n++) w[r][n] = NVLLM_WLOAD(wp[n] + (size_t)kb * 64);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    const f4_t zero = {0.f, 0.f, 0.f, 0.f};
+    f4_t hi[NT], lo[NT];
+#pragma unroll
+    for (int n = 0; n < NT; n++) hi[n] = lo[n] = zero;
+    float ss = 0.f;
+    auto multiply = [&](int r) {
+        h8_t vh, vl;
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            f4_t v = a[r][h];
+            if constexpr (NORM) {
+                float sq = v[0] * v[0];
+#pragma unroll
+                for (int e = 1; e < 4; e++) sq = fmaf(v[e], v[e], sq);
+                ss += sq;
+                v *= gv[r][h];
+            }
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const float c = fminf(fmaxf(v[e], -65504.f), 65504.f);
+                vh[4 * h + e] = (_Float16)c;
+                vl[4 * h + e] = (_Float16)(c - (float)vh[4 * h + e]);
+            }
+        }
+#pragma unroll
+        for (int n = 0; n < NT; n++) {
+            hi[n] = OpF16x2::mfma(w[r][n], vh, hi[n]);
+            lo[n] = OpF16x2::mfma(w[r][n], vl, lo[n]);
+        }
+    };
+    // (as in gemm_f32.hip: the steady loop requests without a condition)
+    const int Kb = K >> 5, mine = wave < Kb ? (Kb - wave + KS - 1) / KS : 0;
+    if (mine < RING) {
+#pragma unroll
+        for (int r = 0; r + 1 < RING; r++)
+            if (r < mine) load(r, r);
+#pragma unroll
+        for (int r = 0; r + 1 < RING; r++)
+            if (r < mine) multiply(r);
+    } else {
+#pragma unroll
+        for (int r = 0; r < RING; r++) load(r, r);
+        int i0 = 0;
+        for (; i0 + 2 * RING <= mine; i0 += RING) {
+#pragma unroll
+            for (int r = 0; r < RING; r++) {
+                multiply(r);
+                load(r, i0 + r + RING);
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < RING; r++) {
+            if (i0 + r < mine) multiply(r);
+            if (i0 + r + RING < mine) load(r, i0 + r + RING);
+        }
+#pragma unroll
+        for (int r = 0; r < RING; r++)
+            if (i0 + r + RING < mine) multiply(r);
+    }
+    const f4_t old = !PAIR && sg.kind == F32Out::ADD && wave < NB ? f32_old(sg, tx, n0) : zero;
+#pragma unroll
+    for (int n = 0; n < NT; n++) s_red[wave][n][lane] = hi[n] + lo[n];
+    if constexpr (NORM) {
+        ss += __shfl_xor(ss, 16, 64);
+        ss += __shfl_xor(ss, 32, 64);
+        if (g == 0) s_ss[wave][x] = ss;
+    }
+    __syncthreads();
+    if (wave >= NB || nb >= blocks) return;
+    f4_t y = s_red[0][PAIR ? 0 : wave][lane], u = zero;
+#pragma unroll
+    for (int v = 1; v < KS; v++) y += s_red[v][PAIR ? 0 : wave][lane];
+    if constexpr (PAIR) {
+        u = s_red[0][1][lane];
+#pragma unroll
+        for (int v = 1; v < KS; v++) u += s_red[v][1][lane];
+    }
+    if constexpr (NORM) {
+        float sum = 0.f;
+#pragma unroll
+        for (int v = 0; v < KS; v++) sum += s_ss[v][x];
+        const float rinv = __fdiv_rn(1.0f, sqrtf(__fadd_rn(__fdiv_rn(sum, (float)K), p.eps)));
+        y *= rinv;
+        if constexpr (PAIR) u *= rinv;
+    }
+    if (x < T && n0 < N) f32_finish<PAIR>(p, sg, x, n0, y, u, old, turn, row);
+    if (!PAIR && p.amax_pairs != nullptr) {
+        // the block's first maximum per token, by the reference's scan (sampler.c:86-97): strict >, so a NaN never wins --
+        // except at index 0, which nothing displaces: +inf there wins every comparison downstream
+        float bv = -INFINITY, bi = -1.0f;
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+            if (n0 + r < N && (y[r] > bv || (bi < 0.f && y[r] == bv))) {
+                bv = y[r];
+                bi = (float)(n0 + r);
+            }
+        if (n0 == 0 && y[0] != y[0]) {
+            bv = INFINITY;
+            bi = 0.f;
+        }
+#pragma unroll
+        for (int o = 16; o < 64; o <<= 1) {
+            const float ov = __shfl_xor(bv, o, 64), oi = __shfl_xor(bi, o, 64);
+            if (oi >= 0.f && (ov > bv || bi < 0.f || (ov == bv && oi < bi))) {
+                bv = ov;
+                bi = oi;
+            }
+        }
+        if (g == 0 && x < T) p.amax_pairs[(size_t)nb * p.amax_ld + x] = make_float2(bv, bi);
+    }
+}
+
+void launch_gemm_thin(const F32Gemm& g, int prof_cls) {
+    if (g.T <= 0 || g.n_segs == 0) return;
+    if (g.T > THIN_TOKENS || g.K % 32) NVLLM_FATAL("thin projection: %d tokens of %d values", g.T, g.K);
+    F32Gemm a = g;
+    const bool pair = a.seg[0].W2 != nullptr;
+    double weights = 0, outs = 0;
+    int blocks = 0;
+    for (int s = 0; s < a.n_segs; s++) {
+        F32Segment& q = a.seg[s];
+        if (pair != (q.W2 != nullptr)) NVLLM_FATAL("thin projection: pairs and single matrices in one launch");
+        q.vec = q.N % 4 == 0 && q.ldo % 4 == 0 && (reinterpret_cast<size_t>(q.out) & 15) == 0;
+        weights += (double)q.N * a.K * (pair ? 2 : 1);
+        outs += q.N;
+        blocks += cdiv(q.N, 16);
+    }
+    // One block per workgroup, and as many waves as keep a CU's fetch path busy: 16 where a CU has one workgroup, 8 where
+    // it has two.  Thousands of blocks (the classifier): four to a workgroup, which then reads the activations once for all.
+    const int cus = rt().num_cus, NB = !pair && blocks > 4 * cus ? 4 : 1;
+    int tiles = 0;
+    for (int s = 0; s < a.n_segs; s++) {
+        a.seg[s].first = tiles;
+        tiles += cdiv(cdiv(a.seg[s].N, 16), NB);
+    }
+    ProfScope ps(prof_cls, 2.0 * weights + 4.0 * a.T * (a.K + outs), 2.0 * a.T * weights);
+#define NVLLM_GEMM_THIN(nb, ks, pair_)                                                                             \
+    do {                                                                                                         \
+        if (a.gain) NVLLM_LAUNCH((k_gemm_thin<nb, ks, pair_, true>), dim3(tiles), dim3((ks) * 64), 0, a);  \
+        else NVLLM_LAUNCH((k_gemm_thin<nb, ks, pair_, false>), dim3(tiles), dim3((ks) * 64), 0, a);        \
+    } while (0)
+    if (NB == 4) NVLLM_GEMM_THIN(4, 8, false);
+    else if (pair) NVLLM_GEMM_THIN(1, 8, true);
+    else if (tiles <= cus) NVLLM_GEMM_THIN(1, 16, false);
+    else NVLLM_GEMM_THIN(1, 8, false);
+#undef NVLLM_GEMM_THIN
+}
+
+}  // namespace nvllm

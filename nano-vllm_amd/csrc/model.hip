@@ -323,6 +323,32 @@ static void load_model_f32(Weights* w, Config* p, FILE* f, bool shared) {
     printf("DEBUG: Embed[100]: %f\n", dbg100);
 }
 
+static AttnArgs attn_args(const StepArrays& st, int T, int H, int KVH, int hd, const KvPoolView& pool, int layer, const float* q) {
+    AttnArgs at{};
+    at.q = q;
+    at.pool = pool;
+    at.layer = layer;
+    at.tables = st.d_tables;
+    at.T = T; at.H = H; at.KVH = KVH; at.hd = hd;
+    at.max_pos = st.max_pos;
+    at.runs = st.d_runs;
+    at.n_runs = st.n_runs;
+    at.kv_positions = st.kv_positions;
+    at.kv_rows = st.kv_rows;
+    at.qk_pairs = st.qk_pairs;
+    return at;
+}
+
+// q, k, v of a layer from fp32 rows: the caller adds the three matrices (ROPE_Q, ROPE_K, KV_V)
+static F32Gemm rows_qkv(const float* x, const StepArrays& st, int T, int D, const float* gain, float eps, const KvPoolView& pool, int layer,
+                        const float2* rope, int hd, int KD) {
+    F32Gemm g = F32Gemm(x, T, D).norm(gain, eps);
+    g.pos = st.d_pos; g.kv_row = st.d_kv_row; g.rope = rope;
+    g.pool_k = pool.k; g.pool_v = pool.v; g.kv_elem_bytes = pool.elem_bytes; g.bs = pool.block_size;
+    g.layer_off = (long)layer * pool.layer_stride; g.hd = hd; g.KD = KD;
+    return g;
+}
+
 // The reference's layer loop (model.c:352-418) on fp32 weights, five launches a layer: the norms, rotation, cache write,
 // SwiGLU and residual adds ride in the projections (gemm_f32.hip).  Leaves the logits of the output rows in d_logits.
 static void forward_f32(const StepArrays& st, int T, int B, Config* p, RunState* s, Weights* w, const KvPoolView& pool,
@@ -333,25 +359,10 @@ static void forward_f32(const StepArrays& st, int T, int B, Config* p, RunState*
     launch_gather_rows_f32(s->x, w->token_embedding_table, st.d_tokens, T, D);
     for (int l = 0; l < p->n_layers; l++) {
         const LayerWeights& lw = w->layers[l];
-        F32Gemm qkv = F32Gemm(s->x, T, D).norm(lw.rms_att_weight, eps);
-        qkv.add(lw.wq, QD, s->q, F32Out::ROPE_Q).add(lw.wk, KD, nullptr, F32Out::ROPE_K).add(lw.wv, KD, nullptr, F32Out::KV_V);
-        qkv.pos = st.d_pos; qkv.kv_row = st.d_kv_row; qkv.rope = rope;
-        qkv.pool_k = pool.k; qkv.pool_v = pool.v; qkv.kv_elem_bytes = pool.elem_bytes; qkv.bs = pool.block_size;
-        qkv.layer_off = (long)l * pool.layer_stride; qkv.hd = hd; qkv.KD = KD;
-        launch_gemm_f32(qkv, PC_GEMM_QKV);
-        AttnArgs at{};
-        at.q = s->q;
+        F32Gemm qkv = rows_qkv(s->x, st, T, D, lw.rms_att_weight, eps, pool, l, rope, hd, KD);
+        launch_gemm_f32(qkv.add(lw.wq, QD, s->q, F32Out::ROPE_Q).add(lw.wk, KD, nullptr, F32Out::ROPE_K).add(lw.wv, KD, nullptr, F32Out::KV_V), PC_GEMM_QKV);
+        AttnArgs at = attn_args(st, T, H, KVH, hd, pool, l, s->q);
         at.out_f32 = s->xb2;
-        at.pool = pool;
-        at.layer = l;
-        at.tables = st.d_tables;
-        at.T = T; at.H = H; at.KVH = KVH; at.hd = hd;
-        at.max_pos = st.max_pos;
-        at.runs = st.d_runs;
-        at.n_runs = st.n_runs;
-        at.kv_positions = st.kv_positions;
-        at.kv_rows = st.kv_rows;
-        at.qk_pairs = st.qk_pairs;
         launch_paged_attention(at);
         launch_gemm_f32(F32Gemm(s->xb2, T, QD).add(lw.wo, D, s->x, F32Out::ADD), PC_GEMM_WO);
         launch_gemm_f32(F32Gemm(s->x, T, D).norm(lw.rms_ffn_weight, eps).add_pair(lw.w_gate, lw.w_up, F, s->hb), PC_GEMM_GATEUP);
@@ -360,6 +371,27 @@ static void forward_f32(const StepArrays& st, int T, int B, Config* p, RunState*
     F32Gemm head = F32Gemm(s->x, B, D).norm(w->rms_final_weight, eps);
     head.in_rows = st.d_out_idx;
     if (B > 0) launch_gemm_f32(head.add(w->lm_head, V, d_logits), PC_GEMM_HEAD);
+}
+
+// The layers of a step of up to THIN_TOKENS tokens on fp16 weights: activations are fp32 rows between the launches
+// (gemm_thin.hip).  s->x holds the embedded tokens.
+static void forward_thin(const ModelPriv& m, const StepArrays& st, int T, const Config* p, RunState* s, const KvPoolView& pool, const float2* rope) {
+    const int D = p->dim, F = p->hidden_dim, hd = p->head_dim, H = p->n_heads, KVH = p->n_kv_heads;
+    const int QD = H * hd, KD = KVH * hd;
+    const float eps = 1e-5f;
+    const long str_D = (long)(D / 32) * TILE_HALVES, str_QD = (long)(QD / 32) * TILE_HALVES, str_F = (long)(F / 32) * TILE_HALVES;
+    for (int l = 0; l < p->n_layers; l++) {
+        const LayerPriv& lp = m.layers[l];
+        F32Gemm qkv = rows_qkv(s->x, st, T, D, lp.rms_att, eps, pool, l, rope, hd, KD);
+        qkv.add16(lp.qkv, str_D, QD, s->q, F32Out::ROPE_Q).add16(lp.qkv + QD / 16 * str_D, str_D, KD, nullptr, F32Out::ROPE_K);
+        launch_gemm_thin(qkv.add16(lp.qkv + (QD + KD) / 16 * str_D, str_D, KD, nullptr, F32Out::KV_V), PC_GEMM_QKV);
+        AttnArgs at = attn_args(st, T, H, KVH, hd, pool, l, s->q);
+        at.out_f32 = s->xb2;
+        launch_paged_attention(at);
+        launch_gemm_thin(F32Gemm(s->xb2, T, QD).add16(lp.wo, str_QD, D, s->x, F32Out::ADD), PC_GEMM_WO);
+        launch_gemm_thin(F32Gemm(s->x, T, D).norm(lp.rms_ffn, eps).add16(lp.gateup, 2 * str_D, F, s->hb, F32Out::STORE, lp.gateup + str_D), PC_GEMM_GATEUP);
+        launch_gemm_thin(F32Gemm(s->hb, T, F).add16(lp.down, str_F, D, s->x, F32Out::ADD), PC_GEMM_DOWN);
+    }
 }
 
 }  // namespace nvllm
@@ -792,7 +824,9 @@ static long enqueue_pass(int* tokens, int num_tokens, int* pos_arr, int* seq_ids
         chained = launch_decode_chain(cs);
     }
 
-    for (int l = 0; l < p->n_layers && !chained; l++) {
+    const bool thin = T <= THIN_TOKENS && !partial && !chained && QD % 16 == 0;
+    if (thin) forward_thin(*m, st, T, p, s, pool, rope);
+    for (int l = 0; l < p->n_layers && !chained && !thin; l++) {
         const LayerPriv& lp = m->layers[l];
         // q,k,v = rmsnorm(x) . [wq;wk;wv]^T, RoPE, K/V rows into the pool      (model.c:361-377)
         WeightEntry wqkv{lp.qkv, QD + 2 * KD, D, D / 32, (long)(D / 32) * TILE_HALVES, nullptr};
@@ -806,19 +840,8 @@ static long enqueue_pass(int* tokens, int num_tokens, int* pos_arr, int* seq_ids
         e1.layer_off = (long)l * pool.layer_stride;
         launch_gemm(wqkv, lp.qkv, QD + 2 * KD, a16_x, T, e1, 0, PC_GEMM_QKV);
         // attention over the block table -> fp16 hi/lo tiles                     (model.c:380-383)
-        AttnArgs at{};
-        at.q = s->q;
+        AttnArgs at = attn_args(st, T, H, KVH, hd, pool, l, s->q);
         at.out_a16 = a16_att;
-        at.pool = pool;
-        at.layer = l;
-        at.tables = st.d_tables;
-        at.T = T; at.H = H; at.KVH = KVH; at.hd = hd;
-        at.max_pos = st.max_pos;
-        at.runs = st.d_runs;
-        at.n_runs = st.n_runs;
-        at.kv_positions = st.kv_positions;
-        at.kv_rows = st.kv_rows;
-        at.qk_pairs = st.qk_pairs;
         launch_paged_attention(at);
         // x += att . wo^T; a16_x = x * rms_ffn; ss_b                              (model.c:385-388)
         WeightEntry wwo{lp.wo, D, QD, QD / 32, (long)(QD / 32) * TILE_HALVES, nullptr};
@@ -866,8 +889,9 @@ static long enqueue_pass(int* tokens, int num_tokens, int* pos_arr, int* seq_ids
     if (B <= 0) return finish_pass(s, d_logits, d_argmax, 0, V, PassView{}, chained);   // nobody wants a row of this pass
     // logits only for the rows named by output_indices                            (model.c:396,411-418)
     wait_for_row_copies();   // the previous pass's rows have left the workspaces the classifier writes
-    bool identity = B == T;
-    for (int k = 0; identity && k < B; k++) identity = output_indices[k] == k;
+    const bool thin_head = B <= THIN_TOKENS && !partial;   // the classifier norms the residual rows itself
+    bool identity = B == T || thin_head;
+    for (int k = 0; identity && !thin_head && k < B; k++) identity = output_indices[k] == k;
     const __half* a16_head = a16_x;
     const float* ss_head = ss_a;
     if (!identity) {
@@ -897,8 +921,17 @@ static long enqueue_pass(int* tokens, int num_tokens, int* pos_arr, int* seq_ids
         host_written = direct_env && rt().logits_mode == NVLLM_LOGITS_ARGMAX && !chained;
         if (host_written) e5.amax_out_host = next_slot(B).host;
         e5.amax_ld = (B + 63) & ~63;
-        e5.amax_pairs = (float2*)ws_get(WS_AMAX_PAIRS, (size_t)cdiv(V, 32) * e5.amax_ld * sizeof(float2));
-        launch_gemm(wh, m->head, V, a16_head, B, e5, head_split, PC_GEMM_HEAD);
+        e5.amax_pairs = (float2*)ws_get(WS_AMAX_PAIRS, (size_t)cdiv(V, 16) * e5.amax_ld * sizeof(float2));
+        if (thin_head) {
+            F32Gemm head = F32Gemm(s->x, B, D).norm(m->rms_final, eps);
+            head.in_rows = st.d_out_idx;
+            head.amax_pairs = e5.amax_pairs;
+            head.amax_ld = e5.amax_ld;
+            launch_gemm_thin(head.add16(m->head, wh.nb_stride, V, d_logits), PC_GEMM_HEAD);
+            launch_argmax_tiles(d_argmax, e5.amax_pairs, cdiv(V, 16), B, e5.amax_ld, e5.amax_out_host);
+        } else {
+            launch_gemm(wh, m->head, V, a16_head, B, e5, head_split, PC_GEMM_HEAD);
+        }
     } else {
         // this rank's vocabulary rows; then either one (max, index) pair per row from every rank,
         // or the slices themselves when full rows are wanted
