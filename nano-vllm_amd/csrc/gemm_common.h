@@ -281,5 +281,7 @@ __device__ __forceinline__ void copy_tile_to_lds(const __half* lane_src, unsigne
 
 // gemm_prefill.hip: 128 x 128 output tiles through LDS, for batches of hundreds of tokens
 void launch_gemm_prefill(GemmArgs a);
+// gemm_wide_f16.hip: the same in tiles of 256 features; false: not for this launch
+bool launch_gemm_wide_f16(const GemmArgs& a);
 
 }  // namespace nvllm

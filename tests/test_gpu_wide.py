@@ -1,0 +1,78 @@
+"""The 256-feature tiles (csrc/gemm_wide.h) at every height, on widths and token counts that end inside a tile, and K that
+ends inside a turn of the ring: one projection at a time against the oracle, and whole passes with every epilogue.  The
+height is read from the environment once per process, hence a child process per height."""
+import os
+import subprocess
+import sys
+
+import numpy as np
+import pytest
+
+from nvllm_amd import synth
+from tests import dense_tile_child, util
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+TOKENS = (256, 300, 433)
+
+
+@pytest.fixture(scope="module")
+def wanted(oracle, tmp_path_factory):
+    path = str(tmp_path_factory.mktemp("wide") / "m.bin")
+    # K of 9, 10 and 25 steps; N of 288, 320, 800 and 1,003
+    synth.write_model(path, synth.ModelShape(dim=288, hidden_dim=800, n_layers=1, n_heads=6, n_kv_heads=6, vocab_size=1003, max_seq_len=512), seed=3)
+    return path, dense_tile_child.run(oracle, path, TOKENS)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("height", [4, 6, 9])
+def test_every_height_of_the_wide_tiles(wanted, tmp_path, height):
+    path, want = wanted
+    dst = str(tmp_path / "got.npz")
+    env = dict(os.environ, PYTHONPATH=ROOT + os.pathsep + os.environ.get("PYTHONPATH", ""))
+    env["NVLLM_GEMM_WIDE"] = str(height)
+    r = subprocess.run([sys.executable, os.path.join(ROOT, "tests", "dense_tile_child.py"), path, dst, ",".join(map(str, TOKENS))], env=env,
+                       capture_output=True, text=True, timeout=150)
+    assert r.returncode == 0, r.stderr[-2000:]
+    got = np.load(dst)
+    assert set(got.files) == set(want)
+    for key, w in want.items():
+        # fp16 weights are exact in both; the activation enters as hi + lo fp16 (~2^-22 relative)
+        np.testing.assert_allclose(got[key], w, rtol=0, atol=3e-6 * np.abs(w).max() + 1e-7, err_msg=key)
+
+
+PASSES = dict(n_new=3, collect_logits=True, chunk_size=280, temperature=0.0)
+CHILD = """
+import sys
+import numpy as np
+from nvllm_amd import capi, synth
+from tests import test_gpu_wide, util
+lib = capi.load_hip()
+lib.nvllm_set_kv_elem_bytes(int(sys.argv[3]))
+steps = util.run_engine(lib, sys.argv[1], test_gpu_wide.prompts(), **test_gpu_wide.PASSES)["steps"]
+np.savez(sys.argv[2], **{k + str(i): s[k] for i, s in enumerate(steps) for k in ("sampled", "logits")})
+"""
+
+
+def prompts():
+    return synth.make_requests(2, 300, 301, 700, seed=6)
+
+
+@pytest.fixture(scope="module")
+def passes(oracle, tmp_path_factory):
+    path = str(tmp_path_factory.mktemp("wide_passes") / "m.bin")
+    synth.write_model(path, synth.ModelShape(dim=256, hidden_dim=800, n_layers=2, n_heads=4, n_kv_heads=2, vocab_size=700, max_seq_len=512), seed=5)
+    return path, util.run_engine(oracle, path, prompts(), **PASSES)["steps"]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("height,kv_bytes", [(4, 4), (6, 2), (9, 4), (9, 2)])
+def test_passes_through_every_epilogue(passes, tmp_path, height, kv_bytes):
+    path, want = passes
+    dst = str(tmp_path / "got.npz")
+    env = dict(os.environ, PYTHONPATH=ROOT + os.pathsep + os.environ.get("PYTHONPATH", ""), NVLLM_GEMM_WIDE=str(height))
+    r = subprocess.run([sys.executable, "-c", CHILD, path, dst, str(kv_bytes)], env=env, capture_output=True, text=True, timeout=150)
+    assert r.returncode == 0, r.stderr[-2000:]
+    got = np.load(dst)
+    for i, o in enumerate(want):
+        np.testing.assert_array_equal(got[f"sampled{i}"], o["sampled"])
+        assert np.abs(got[f"logits{i}"] - o["logits"]).max() < (2e-4 if kv_bytes == 4 else 2e-3)   # the bars of the forward pass
