@@ -172,39 +172,54 @@ __device__ __forceinline__ void hyper_load_4(HyperIn<SMAX>& in, const GemmEpilog
     in.w = *reinterpret_cast<const f4_t*>(ep.norm_w + n);
     in.b = *reinterpret_cast<const f4_t*>(ep.norm_b + n);
 }
+// The connection's coefficients, read once: left in memory they would be read again after every store to x, which might
+// alias them (a chain of loads and stores per four features).
 template <int SMAX>
-__device__ __forceinline__ void hyper_update_4(const HyperIn<SMAX>& in, const GemmEpilogue& ep, int N, int t, int n, const float* y_in) {
+struct HyperMix {
+    float mix[SMAX][SMAX], out[SMAX], in[SMAX], alpha;   // (entries of absent streams repeat others and are not used)
+};
+template <int SMAX>
+__device__ __forceinline__ HyperMix<SMAX> hyper_mix(const GemmEpilogue& ep) {
+    auto uniform = [](float v) { return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, v))); };
+    const int S = ep.streams;
+    HyperMix<SMAX> m;
+#pragma unroll
+    for (int s = 0; s < SMAX; s++) {
+#pragma unroll
+        for (int to = 0; to < SMAX; to++) m.mix[s][to] = uniform(ep.hyper[min(s, S - 1) * S + min(to, S - 1)]);
+        m.out[s] = uniform(ep.hyper[S * S + min(s, S - 1)]);
+        m.in[s] = uniform(ep.hyper[S * S + S + min(s, S - 1)]);
+    }
+    m.alpha = uniform(ep.hyper[S * S + 2 * S]);
+    return m;
+}
+template <int SMAX>
+__device__ __forceinline__ void hyper_update_4(const HyperIn<SMAX>& in, const HyperMix<SMAX>& c, const GemmEpilogue& ep, int N, int t, int n, const float* y_in) {
     const int S = ep.streams;
     float y[4];
 #pragma unroll
     for (int r = 0; r < 4; r++) y[r] = (y_in[r] + in.bias[r]) * in.scale[r];
     float* xr = ep.x + (size_t)t * S * N + n;
-    const float* mix = ep.hyper;
-    const float* out = mix + S * S;
-    const float* weight = out + S;
-    const float alpha = weight[S];
     f4_t u = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int to = 0; to < SMAX; to++)
         if (to < S) {
-            const float o = out[to], ii = weight[to];
             f4_t v;
 #pragma unroll
-            for (int r = 0; r < 4; r++) v[r] = o * y[r];
+            for (int r = 0; r < 4; r++) v[r] = c.out[to] * y[r];
 #pragma unroll
             for (int s = 0; s < SMAX; s++)
                 if (s < S) {
-                    const float m = mix[s * S + to];
 #pragma unroll
-                    for (int r = 0; r < 4; r++) v[r] = fmaf(m, in.xs[s][r], v[r]);
+                    for (int r = 0; r < 4; r++) v[r] = fmaf(c.mix[s][to], in.xs[s][r], v[r]);
                 }
             *reinterpret_cast<f4_t*>(xr + (size_t)to * N) = v;
 #pragma unroll
-            for (int r = 0; r < 4; r++) u[r] = fmaf(ii, v[r], u[r]);
+            for (int r = 0; r < 4; r++) u[r] = fmaf(c.in[to], v[r], u[r]);
         }
     float z[4];
 #pragma unroll
-    for (int r = 0; r < 4; r++) z[r] = fmaf(tanhf(alpha * u[r]), in.w[r], in.b[r]);
+    for (int r = 0; r < 4; r++) z[r] = fmaf(tanhf(c.alpha * u[r]), in.w[r], in.b[r]);
     store_b16_4(ep.a16_out, ep.Kb_out, t, n, z);
 }
 constexpr int hyper_streams(int kind) { return kind == GemmEpilogue::HYPER_2 ? 2 : kind == GemmEpilogue::HYPER_4 ? 4 : 0; }   // 0: another epilogue

@@ -16,8 +16,7 @@
 //            group of four waves takes the odd K-steps, so every SIMD has two waves to
 //            alternate between LDS reads and MFMAs and a barrier covers two K-steps; the
 //            two groups add their accumulators through LDS before the epilogue.
-// (256-feature tiles have the better operand traffic per MFMA and measured slower at
-// prefill sizes: too few workgroups, and the last round of them runs nearly empty.)
+// Launches with enough tiles take the 256-feature ones of gemm_wide.h instead.
 //
 // Both operands are stored in matrix-core operand order, one 1-KiB tile per (16 rows,
 // 32 k), so a tile is copied by ONE wave instruction (64 lanes x 16 B, lane-linear in
@@ -95,6 +94,74 @@ __device__ __forceinline__ void wait_copies_but(int stages) {
     }
 }
 
+// RESID_*, HYPER_*: the operands of token block j + 1 travel while block j is finished.
+template <int NI, int NJ, int EPI>
+__device__ __forceinline__ void pf_residual(const GemmArgs& p, const f4_t (&v)[NI][NJ], int nb_first, int tbl_first, int tb0, const float* s_rinv, int lane,
+                                            int nb_lim) {
+    const GemmEpilogue& ep = p.e;
+    constexpr int HS = hyper_streams(EPI);
+    const int n_of = nb_first * 16 + 4 * (lane >> 4);
+    float4 xo[2][HS ? 1 : NI], gain[HS ? 1 : NI];
+    HyperIn<HS ? HS : 1> hyper[2][HS ? NI : 1];
+    auto load = [&](int set, int j) {
+        const int t = min((tb0 + tbl_first + j) * 16 + (lane & 15), p.T - 1);
+#pragma unroll
+        for (int i = 0; i < NI; i++) {
+            const int n = min(n_of + 16 * i, p.N - 4);
+            if constexpr (HS > 0) hyper_load_4<HS>(hyper[set][i], ep, p.N, t, n);
+            else xo[set][i] = *reinterpret_cast<const float4*>(ep.x + (size_t)t * p.N + n);
+        }
+    };
+    load(0, 0);
+    HyperMix<HS ? HS : 1> mix;
+    if constexpr (HS > 0) {
+        mix = hyper_mix<HS>(ep);
+    } else {
+#pragma unroll
+        for (int i = 0; i < NI; i++) gain[i] = *reinterpret_cast<const float4*>(ep.gain_next + min(n_of + 16 * i, p.N - 4));
+    }
+#pragma unroll
+    for (int j = 0; j < NJ; j++) {
+        if (j + 1 < NJ) load((j + 1) & 1, j + 1);
+        const int tl = (tbl_first + j) * 16 + (lane & 15), t = tb0 * 16 + tl;
+        const bool tok_live = t < p.T && tb0 + tbl_first + j < p.Tb;
+        const float rinv = ep.ss_in ? s_rinv[tl] : 1.0f;
+        float ssq[NI / 2];
+#pragma unroll
+        for (int h = 0; h < NI / 2; h++) ssq[h] = 0.f;
+#pragma unroll
+        for (int i = 0; i < NI; i++) {
+            const int n = n_of + 16 * i;
+            if (!tok_live || nb_first + i >= nb_lim) continue;
+            const float y[4] = {v[i][j][0] * rinv, v[i][j][1] * rinv, v[i][j][2] * rinv, v[i][j][3] * rinv};
+            if constexpr (HS > 0) {
+                hyper_update_4<HS>(hyper[j & 1][i], mix, ep, p.N, t, n, y);
+            } else if constexpr (EPI == GemmEpilogue::RESID_B16) {
+                ssq[i >> 1] += resid_b16_4(ep, p.N, t, n, xo[j & 1][i], gain[i], y);
+            } else {
+                const float4 x = xo[j & 1][i], g = gain[i];
+                // residual add as the reference's accum(): x = x + branch (layers.c:163-168)
+                const float xn[4] = {__fadd_rn(x.x, y[0]), __fadd_rn(x.y, y[1]), __fadd_rn(x.z, y[2]), __fadd_rn(x.w, y[3])};
+                *reinterpret_cast<float4*>(ep.x + (size_t)t * p.N + n) = make_float4(xn[0], xn[1], xn[2], xn[3]);
+                const float z[4] = {xn[0] * g.x, xn[1] * g.y, xn[2] * g.z, xn[3] * g.w};
+                store_a16_4(ep.a16_out, ep.Kb_out, t, n, z);
+                ssq[i >> 1] += xn[0] * xn[0] + xn[1] * xn[1] + xn[2] * xn[2] + xn[3] * xn[3];
+            }
+        }
+        if constexpr (epi_has_ss(EPI)) {
+            // per-token sum of x^2 over each 32-feature group = two row blocks (same lane) x four lane groups
+#pragma unroll
+            for (int h = 0; h < NI / 2; h++) {
+                float sq = ssq[h];
+                sq += __shfl_xor(sq, 16, 64);
+                sq += __shfl_xor(sq, 32, 64);
+                const int col = (nb_first + 2 * h) >> 1;
+                if (lane < 16 && tok_live && col < (p.N + 31) >> 5) ep.ss_out[(size_t)t * ((p.N + 31) >> 5) + col] = sq;
+            }
+        }
+    }
+}
+
 // The epilogues of gemm.hip applied to NI x NJ accumulator tiles of one wave.  v[i][j] of
 // lane l: token t = (tb0 + tbl_first + j)*16 + (l & 15), features n .. n+3 with
 // n = nb*16 + 4*(l >> 4), nb = nb_first + i.
@@ -102,6 +169,10 @@ template <int NI, int NJ, int EPI, typename KVT, typename OP = OpF16x2>
 __device__ __forceinline__ void pf_epilogue(const GemmArgs& p, const f4_t (&v)[NI][NJ], int nb_first, int tbl_first, int tb0,
                                             const float* s_rinv, int lane, int nb_lim) {
     const GemmEpilogue& ep = p.e;
+    if constexpr (EPI == GemmEpilogue::RESID_A16 || EPI == GemmEpilogue::RESID_B16 || hyper_streams(EPI) > 0) {
+        pf_residual<NI, NJ, EPI>(p, v, nb_first, tbl_first, tb0, s_rinv, lane, nb_lim);
+        return;
+    }
 #pragma unroll
     for (int j = 0; j < NJ; j++) {
         const int tbj = tb0 + tbl_first + j;
@@ -114,12 +185,6 @@ __device__ __forceinline__ void pf_epilogue(const GemmArgs& p, const f4_t (&v)[N
             pos = ep.pos[t];
             kv_row = ep.kv_row[t];
         }
-        constexpr int HS = hyper_streams(EPI);
-        HyperIn<HS ? HS : 1> hyper[HS ? NI : 1];   // the residual operands of all NI tiles of this token block travel together
-        if constexpr (HS > 0) {
-#pragma unroll
-            for (int i = 0; i < NI; i++) hyper_load_4<HS>(hyper[i], ep, p.N, min(t, p.T - 1), min((nb_first + i) * 16 + 4 * (lane >> 4), p.N - 4));
-        }
         float ssq[NI / 2];
 #pragma unroll
         for (int h = 0; h < NI / 2; h++) ssq[h] = 0.f;
@@ -129,9 +194,7 @@ __device__ __forceinline__ void pf_epilogue(const GemmArgs& p, const f4_t (&v)[N
             const int n = nb * 16 + 4 * (lane >> 4);
             const bool live = tok_live && nb < nb_lim;
             float y[4] = {v[i][j][0] * rinv, v[i][j][1] * rinv, v[i][j][2] * rinv, v[i][j][3] * rinv};
-            if constexpr (HS > 0) {
-                if (live) hyper_update_4<HS>(hyper[i], ep, p.N, t, n, y);
-            } else if constexpr (epi_is_point(EPI)) {
+            if constexpr (epi_is_point(EPI)) {
                 if (live) ssq[i >> 1] += epi_point<EPI>(ep, p.N, t, n, y);
             } else if (EPI == GemmEpilogue::F32) {
                 if constexpr (OP::PLANES == 1) {
@@ -172,22 +235,6 @@ __device__ __forceinline__ void pf_epilogue(const GemmArgs& p, const f4_t (&v)[N
                     if constexpr (OP::PLANES == 1) store_b16_4(ep.a16_out, ep.Kb_out, t, hid, z);
                     else store_a16_4(ep.a16_out, ep.Kb_out, t, hid, z);
                 }
-            } else if (EPI == GemmEpilogue::RESID_B16) {
-                if (live)
-                    ssq[i >> 1] += resid_b16_4(ep, p.N, t, n, *reinterpret_cast<const float4*>(ep.x + (size_t)t * p.N + n),
-                                               *reinterpret_cast<const float4*>(ep.gain_next + n), y);
-            } else if (EPI == GemmEpilogue::RESID_A16) {
-                if (live) {
-                    float* xr = ep.x + (size_t)t * p.N + n;
-                    const float4 xo = *reinterpret_cast<const float4*>(xr);
-                    const float4 g = *reinterpret_cast<const float4*>(ep.gain_next + n);
-                    // residual add as the reference's accum(): x = x + branch (layers.c:163-168)
-                    const float xn[4] = {__fadd_rn(xo.x, y[0]), __fadd_rn(xo.y, y[1]), __fadd_rn(xo.z, y[2]), __fadd_rn(xo.w, y[3])};
-                    *reinterpret_cast<float4*>(xr) = make_float4(xn[0], xn[1], xn[2], xn[3]);
-                    const float z[4] = {xn[0] * g.x, xn[1] * g.y, xn[2] * g.z, xn[3] * g.w};
-                    store_a16_4(ep.a16_out, ep.Kb_out, t, n, z);
-                    ssq[i >> 1] += xn[0] * xn[0] + xn[1] * xn[1] + xn[2] * xn[2] + xn[3] * xn[3];
-                }
             } else {  // ROPE_KV
                 if (live) {
                     if (n < ep.QD + ep.KD) {   // q or k: rotate the two pairs of this float4 (layers.c:118-141)
@@ -220,10 +267,8 @@ __device__ __forceinline__ void pf_epilogue(const GemmArgs& p, const f4_t (&v)[N
                 }
             }
         }
-        if (epi_has_ss(EPI)) {
-            // per-token sum of x^2 over each 32-feature group = two row blocks (same lane)
-            // x four lane groups
-            const int ss_cols = EPI == GemmEpilogue::LATENT_IN ? ep.latent_q >> 5 : (p.N + 31) >> 5;
+        if (epi_has_ss(EPI)) {   // LATENT_IN; as in pf_residual
+            const int ss_cols = ep.latent_q >> 5;
 #pragma unroll
             for (int h = 0; h < NI / 2; h++) {
                 float sq = ssq[h];
@@ -284,6 +329,33 @@ __device__ __forceinline__ bool pf_close_split(const GemmArgs& p, f4_t (&v)[NI][
     }
     if (threadIdx.x == 0) __hip_atomic_store(p.counters + tile_id, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     return true;
+}
+
+// 1/rms of the tile's tokens from the producer's sums of squares, while the first stages travel: neighbouring threads share
+// a token and every load of a thread is requested at once (two threads per token and one load after the other, in front of
+// the copies, cost 4 to 6 us a launch).
+template <int TOKENS, int THREADS>
+__device__ __forceinline__ void tile_rinv(const GemmArgs& p, int tb0, float* s_rinv) {
+    constexpr int PARTS = TOKENS * 8 <= THREADS ? 8 : TOKENS * 4 <= THREADS ? 4 : TOKENS * 2 <= THREADS ? 2 : 1;
+    const int tl = (int)threadIdx.x / PARTS, part = (int)threadIdx.x % PARTS;
+    const int t = min(tb0 * 16 + tl, p.T - 1), cols = p.e.ss_tiles;
+    const float* sp = p.e.ss_in + (size_t)(p.e.ss_gather ? p.e.ss_gather[t] : t) * cols;
+    float ss = 0.f;
+    if ((cols & 3) == 0) {
+        for (int j0 = 4 * part; j0 < cols; j0 += 64 * PARTS) {
+            f4_t v[16];
+#pragma unroll
+            for (int j = 0; j < 16; j++) v[j] = *reinterpret_cast<const f4_t*>(sp + min(j0 + 4 * PARTS * j, cols - 4));
+#pragma unroll
+            for (int j = 0; j < 16; j++)
+                if (j0 + 4 * PARTS * j < cols) ss += (v[j][0] + v[j][1]) + (v[j][2] + v[j][3]);
+        }
+    } else {
+        for (int j = part; j < cols; j += PARTS) ss += sp[j];
+    }
+#pragma unroll
+    for (int o = 1; o < PARTS; o <<= 1) ss += __shfl_xor(ss, o, 64);
+    if (part == 0 && tl < TOKENS) s_rinv[tl] = __fdiv_rn(1.0f, sqrtf(__fadd_rn(__fdiv_rn(ss, (float)p.e.d_in), p.e.eps)));
 }
 
 template <int FW, int KG, int EPI, typename KVT, int WR = 2, int TW = 4, typename OP = OpF16x2, bool GRP = false, bool EXP = false>
@@ -390,26 +462,10 @@ __global__ __launch_bounds__(128 * WR * KG, WR == 4 ? 4 : 2) void k_gemm_prefill
 #pragma unroll
         for (int j = 0; j < TW; j++) acc[i][j] = f4_t{0.f, 0.f, 0.f, 0.f};
 
-    // 1/rms of the tile's tokens from the producer's sums of squares (two threads per token);
-    // done before the first copy is issued, so that its barrier does not wait for copies
-    if (p.e.ss_in != nullptr) {
-        const int tl = threadIdx.x & 127, part = threadIdx.x >> 7;
-        float ss = 0.f;
-        if (part < 2) {
-            const int t = min(tb0 * 16 + tl, p.T - 1);
-            const int srow = p.e.ss_gather ? p.e.ss_gather[t] : t;
-            const float* sp = p.e.ss_in + (size_t)srow * p.e.ss_tiles;
-            for (int j = part; j < p.e.ss_tiles; j += 2) ss += sp[j];
-        }
-        // the two halves meet in the result array itself: the upper half writes, the lower adds
-        if (part == 1) s_rinv[tl] = ss;
-        __syncthreads();
-        if (part == 0) s_rinv[tl] = __fdiv_rn(1.0f, sqrtf(__fadd_rn(__fdiv_rn(ss + s_rinv[tl], (float)p.e.d_in), p.e.eps)));
-    }
-
     const int n_stages = (kb_hi - kb_lo + KG - 1) / KG;
     const int ahead = nbuf - 1;   // stages in flight beyond the one being multiplied
     for (int s0 = 0; s0 < ahead && s0 < n_stages; s0++) stage(s0, s0);
+    if (p.e.ss_in != nullptr) tile_rinv<16 * G::TB, 64 * G::WAVES>(p, tb0, s_rinv);   // (the barrier in front of the epilogue publishes it)
     NVLLM_STAMP(1, lane);
 
     // Steady state: stage s + ahead is a whole stage inside [kb_lo, kb_hi), so its copies need

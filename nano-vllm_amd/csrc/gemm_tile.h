@@ -329,7 +329,9 @@ __device__ __forceinline__ bool gemm_tile(const GemmArgs& p, const TileIdx ix, u
     }
     constexpr int HS = hyper_streams(EPI);
     HyperIn<HS ? HS : 1> pf_hyper[HS ? FPT : 1];
+    HyperMix<HS ? HS : 1> hyper_c;
     if constexpr (HS > 0) {
+        hyper_c = hyper_mix<HS>(ep);
 #pragma unroll
         for (int s = 0; s < FPT; s++) {
             const int w_ = min(tid + s * NW * 64, WITEMS - 1);
@@ -466,7 +468,7 @@ __device__ __forceinline__ bool gemm_tile(const GemmArgs& p, const TileIdx ix, u
             const float rinv = ep.ss_in ? s_rinv[tl] : 1.0f;
             float y[4] = {v[s][0] * rinv, v[s][1] * rinv, v[s][2] * rinv, v[s][3] * rinv};
             if constexpr (HS > 0) {
-                if (live) hyper_update_4<HS>(pf_hyper[s], ep, p.N, t, n, y);
+                if (live) hyper_update_4<HS>(pf_hyper[s], hyper_c, ep, p.N, t, n, y);
             } else if constexpr (epi_is_point(EPI)) {
                 if (live) ssq[s] += epi_point<EPI>(ep, p.N, t, n, y);
             } else if (EPI == GemmEpilogue::F32) {

@@ -13,7 +13,7 @@
 // registers by then.  TinyLlama-1.1B's gate/up of 1,548 tokens: 175 us in the smaller tiles, 140 here (512 TFLOP/s of
 // products, twice that in the matrix cores: hi + lo; large library products of this type reach 1,096).
 //
-// The epilogues are those of gemm_prefill_tile.h; the residual rows they add to are requested a token block ahead.
+// The epilogues are those of gemm_prefill_tile.h.
 #pragma once
 
 #include "gemm_prefill_tile.h"
@@ -42,78 +42,11 @@ __device__ __forceinline__ void wide_wait() {
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
-// RESID_*, HYPER_*: the operands of token block j + 1 travel while block j is finished.
-template <int TBN, int EPI>
-__device__ __forceinline__ void wide_residual(const GemmArgs& p, const f4_t (&v)[4][TBN], int nb_first, int tb0, const float* s_rinv, int lane, int nb_lim) {
-    const GemmEpilogue& ep = p.e;
-    constexpr int HS = hyper_streams(EPI);
-    const int n_of = nb_first * 16 + 4 * (lane >> 4);
-    float4 xo[2][HS ? 1 : 4], gain[HS ? 1 : 4];
-    HyperIn<HS ? HS : 1> hyper[2][HS ? 4 : 1];
-    auto load = [&](int set, int j) {
-        const int t = min((tb0 + j) * 16 + (lane & 15), p.T - 1);
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int n = min(n_of + 16 * i, p.N - 4);
-            if constexpr (HS > 0) hyper_load_4<HS>(hyper[set][i], ep, p.N, t, n);
-            else xo[set][i] = *reinterpret_cast<const float4*>(ep.x + (size_t)t * p.N + n);
-        }
-    };
-    if constexpr (HS == 0)
-#pragma unroll
-        for (int i = 0; i < 4; i++) gain[i] = *reinterpret_cast<const float4*>(ep.gain_next + min(n_of + 16 * i, p.N - 4));
-    load(0, 0);
-#pragma unroll
-    for (int j = 0; j < TBN; j++) {
-        if (j + 1 < TBN) load((j + 1) & 1, j + 1);
-        const int tl = j * 16 + (lane & 15), t = tb0 * 16 + tl;
-        const bool tok_live = t < p.T && tb0 + j < p.Tb;
-        const float rinv = ep.ss_in ? s_rinv[tl] : 1.0f;
-        float ssq[2] = {0.f, 0.f};
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int n = n_of + 16 * i;
-            const bool live = tok_live && nb_first + i < nb_lim;
-            const float y[4] = {v[i][j][0] * rinv, v[i][j][1] * rinv, v[i][j][2] * rinv, v[i][j][3] * rinv};
-            if (!live) continue;
-            if constexpr (HS > 0) {
-                hyper_update_4<HS>(hyper[j & 1][i], ep, p.N, t, n, y);
-            } else if constexpr (EPI == GemmEpilogue::RESID_B16) {
-                ssq[i >> 1] += resid_b16_4(ep, p.N, t, n, xo[j & 1][i], gain[i], y);
-            } else {
-                const float4 x = xo[j & 1][i], g = gain[i];
-                // residual add as the reference's accum(): x = x + branch (layers.c:163-168)
-                const float xn[4] = {__fadd_rn(x.x, y[0]), __fadd_rn(x.y, y[1]), __fadd_rn(x.z, y[2]), __fadd_rn(x.w, y[3])};
-                *reinterpret_cast<float4*>(ep.x + (size_t)t * p.N + n) = make_float4(xn[0], xn[1], xn[2], xn[3]);
-                const float z[4] = {xn[0] * g.x, xn[1] * g.y, xn[2] * g.z, xn[3] * g.w};
-                store_a16_4(ep.a16_out, ep.Kb_out, t, n, z);
-                ssq[i >> 1] += xn[0] * xn[0] + xn[1] * xn[1] + xn[2] * xn[2] + xn[3] * xn[3];
-            }
-        }
-        if constexpr (epi_has_ss(EPI)) {
-#pragma unroll
-            for (int h = 0; h < 2; h++) {
-                float sq = ssq[h];
-                sq += __shfl_xor(sq, 16, 64);
-                sq += __shfl_xor(sq, 32, 64);
-                const int col = (nb_first + 2 * h) >> 1;
-                if (lane < 16 && tok_live && col < (p.N + 31) >> 5) ep.ss_out[(size_t)t * ((p.N + 31) >> 5) + col] = sq;
-            }
-        }
-    }
-}
-
-template <int TBN, int EPI, typename KVT, typename OP, bool EXP>
+template <int TBN, int EPI, typename KVT, typename OP>
 __global__ __launch_bounds__(256, 1) void k_gemm_wide(GemmArgs p, int tiles_n, int tiles_t) {
     constexpr int PL = OP::PLANES;
     using G = WideGeom<TBN, PL>;
     constexpr int RING = G::RING, CPW = G::CPW;
-    if constexpr (EPI == GemmEpilogue::LATENT_Q) {
-        if ((int)blockIdx.x >= p.ride_from) {
-            latent_kv_ride(p.ride, ((int)blockIdx.x - p.ride_from) * 4 + (int)(threadIdx.x >> 6), threadIdx.x & 63);
-            return;
-        }
-    }
     extern __shared__ __attribute__((aligned(16))) unsigned char lds_wide[];
     float* s_rinv = reinterpret_cast<float*>(lds_wide);
     const h8_t* ring = reinterpret_cast<const h8_t*>(lds_wide + G::RINV_BYTES);
@@ -128,12 +61,6 @@ __global__ __launch_bounds__(256, 1) void k_gemm_wide(GemmArgs p, int tiles_n, i
         id = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + slot;
     }
     const int nb0 = id / tiles_t * G::FB, tb0 = id % tiles_t * TBN;
-    const __half* W = p.W;
-    if constexpr (EXP) {
-        const int e = __builtin_amdgcn_readfirstlane(p.block_expert[tb0]);
-        if (e < 0) return;   // fewer rows than the launch has room for
-        W += (size_t)e * p.expert_stride;
-    }
     // wave w copies tiles w, w + 4, ...: weight blocks, then the planes of each token block (past the last: the last again, the
     // same bytes to the same place, so that no branch parts the loop)
     const __half* src[CPW];
@@ -142,7 +69,7 @@ __global__ __launch_bounds__(256, 1) void k_gemm_wide(GemmArgs p, int tiles_n, i
     for (int u = 0; u < CPW; u++) {
         const int q = min(wave + 4 * u, G::TILES - 1);
         dst[u] = (unsigned)(size_t)(lds_void*)lds_wide + G::RINV_BYTES + q * 1024;
-        src[u] = q < G::FB ? W + (size_t)min(nb0 + q, p.NB - 1) * p.nb_stride
+        src[u] = q < G::FB ? p.W + (size_t)min(nb0 + q, p.NB - 1) * p.nb_stride
                            : p.A + ((size_t)min(tb0 + (q - G::FB) / PL, p.Tb - 1) * p.Kb * PL + (q - G::FB) % PL) * TILE_HALVES;
     }
     unsigned at_w = lane * 16, at_a = lane * 16;   // bytes from a source's start: its k-tile, this lane's piece
@@ -162,30 +89,7 @@ __global__ __launch_bounds__(256, 1) void k_gemm_wide(GemmArgs p, int tiles_n, i
         for (int u = 0; u < CPW; u++) copy(u, s * G::TILES * 1024);
         copied();
     }
-    // 1/rms of the tile's tokens from the producer's sums of squares, while the first stages travel: PARTS neighbouring
-    // threads per token, every load of a thread requested at once (one after the other they cost 5 us)
-    if (p.e.ss_in != nullptr) {
-        constexpr int PARTS = TBN <= 4 ? 4 : TBN <= 8 ? 2 : 1;
-        const int tl = (int)threadIdx.x / PARTS, part = (int)threadIdx.x % PARTS;
-        const int t = min(tb0 * 16 + tl, p.T - 1), cols = p.e.ss_tiles;
-        const float* sp = p.e.ss_in + (size_t)(p.e.ss_gather ? p.e.ss_gather[t] : t) * cols;
-        float ss = 0.f;
-        if ((cols & 3) == 0) {
-            for (int j0 = 4 * part; j0 < cols; j0 += 64 * PARTS) {
-                f4_t v[16];
-#pragma unroll
-                for (int j = 0; j < 16; j++) v[j] = *reinterpret_cast<const f4_t*>(sp + min(j0 + 4 * PARTS * j, cols - 4));
-#pragma unroll
-                for (int j = 0; j < 16; j++)
-                    if (j0 + 4 * PARTS * j < cols) ss += (v[j][0] + v[j][1]) + (v[j][2] + v[j][3]);
-            }
-        } else {
-            for (int j = part; j < cols; j += PARTS) ss += sp[j];
-        }
-#pragma unroll
-        for (int o = 1; o < PARTS; o <<= 1) ss += __shfl_xor(ss, o, 64);
-        if (part == 0 && tl < TBN * 16) s_rinv[tl] = __fdiv_rn(1.0f, sqrtf(__fadd_rn(__fdiv_rn(ss, (float)p.e.d_in), p.e.eps)));
-    }
+    if (p.e.ss_in != nullptr) tile_rinv<16 * TBN, 256>(p, tb0, s_rinv);
 
     f4_t acc[4][TBN];
 #pragma unroll
@@ -267,22 +171,18 @@ __global__ __launch_bounds__(256, 1) void k_gemm_wide(GemmArgs p, int tiles_n, i
     phase(wa, wb, no{}, no{});
 
     const int nb_first = nb0 + wave * 4;
-    if constexpr (EPI == GemmEpilogue::RESID_A16 || EPI == GemmEpilogue::RESID_B16 || hyper_streams(EPI) > 0)
-        wide_residual<TBN, EPI>(p, acc, nb_first, tb0, s_rinv, lane, p.NB);
-    else
-        pf_epilogue<4, TBN, EPI, KVT, OP>(p, acc, nb_first, 0, tb0, s_rinv, lane, p.NB);
+    pf_epilogue<4, TBN, EPI, KVT, OP>(p, acc, nb_first, 0, tb0, s_rinv, lane, p.NB);
 }
 
-template <int TBN, int EPI, typename KVT, typename OP, bool EXP = false>
+template <int TBN, int EPI, typename KVT, typename OP>
 void launch_wide(const GemmArgs& a, int tiles_n, int tiles_t) {
     using G = WideGeom<TBN, OP::PLANES>;
     static bool enabled = false;
     if (!enabled) {
-        HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_gemm_wide<TBN, EPI, KVT, OP, EXP>), hipFuncAttributeMaxDynamicSharedMemorySize, G::LDS));
+        HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_gemm_wide<TBN, EPI, KVT, OP>), hipFuncAttributeMaxDynamicSharedMemorySize, G::LDS));
         enabled = true;
     }
-    const int riders = EPI == GemmEpilogue::LATENT_Q && a.ride.base ? cdiv(a.ride.T, 4) : 0;
-    NVLLM_LAUNCH((k_gemm_wide<TBN, EPI, KVT, OP, EXP>), dim3(tiles_n * tiles_t + riders), dim3(256), G::LDS, a, tiles_n, tiles_t);
+    NVLLM_LAUNCH((k_gemm_wide<TBN, EPI, KVT, OP>), dim3(tiles_n * tiles_t), dim3(256), G::LDS, a, tiles_n, tiles_t);
 }
 
 inline int wide_env() {   // NVLLM_GEMM_WIDE: 0 = never these tiles, a number of token blocks = always that height
