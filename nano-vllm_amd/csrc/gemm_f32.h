@@ -84,7 +84,7 @@ void launch_gemm_f32(const F32Gemm& g, int prof_cls);
 
 // The same for fp16 weights in tile order (add16) and up to THIN_TOKENS tokens; K % 32 == 0.  Activations enter the matrix
 // cores as fp16 hi + lo, as in gemm.hip.
-constexpr int THIN_TOKENS = 8;   // (at most 16: one block of tokens)
+constexpr int THIN_TOKENS = 6;   // (at most 16: one block of tokens)
 void launch_gemm_thin(const F32Gemm& g, int prof_cls);
 
 }  // namespace nvllm

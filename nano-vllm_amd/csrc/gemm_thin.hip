@@ -1,4 +1,4 @@
-// gemm_thin.hip -- projections of fp16 weights for up to 8 tokens: the layers of a model that serves one user or a few.
+// gemm_thin.hip -- projections of fp16 weights for up to 6 tokens: the layers of a model that serves one user or a few.
 //
 // The weights are all there is to read (2 bytes each, against 4 bytes per token and k of activations), so a launch is as
 // fast as its CUs can fetch: about 50 GB/s each from HBM, 128 CUs saturate it.  A workgroup therefore owns ONE 16-row block
@@ -8,8 +8,9 @@
 // split into fp16 hi + lo and the element-wise work behind the product happen here, and the next launch reads rows again.
 //
 // TinyLlama shape, one token, us per launch, 64-row tiles of gemm.hip (K cut over workgroups) and here: wo and w_down
-// together 18.2 and 15.5, gate/up 13.2 and 13.9, q/k/v 8.6 and 7.2; the pass 1,217 and 1,168.  At 9 tokens the two are
-// equal (1,558 and 1,575 a pass), from where the activations, read by every workgroup, weigh more: up to 8 tokens.
+// together 18.2 and 15.5, gate/up 13.2 and 13.9, q/k/v 8.6 and 7.2; the pass 1,217 and 1,168.  The activations, read by every
+// workgroup, weigh more with every token: a pass of 4 tokens 1,134 and 1,104, of 6 1,136 and 1,126, of 7 1,137 and 1,142, of
+// 8 1,145 and 1,164.  So up to 6.
 // Eight rows to a workgroup instead of 16 (256 of them for wo and w_down) and six tiles in flight measured the same or
 // slower: it is the start of a launch, two dependent trips to memory, that is left.
 #include "gemm_f32_tail.h"

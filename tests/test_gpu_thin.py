@@ -9,7 +9,7 @@ from tests import util
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("n", [1, 7, 8, 9])
+@pytest.mark.parametrize("n", [1, 5, 6, 7])
 @pytest.mark.parametrize("kv_bytes", [4, 2])
 @pytest.mark.parametrize("shape", [
     dict(dim=96, hidden_dim=224, n_layers=2, n_heads=2, n_kv_heads=2, vocab_size=1003),        # 3 and 7 tiles of K
