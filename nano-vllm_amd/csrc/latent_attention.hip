@@ -68,48 +68,87 @@ void launch_latent_kv(const LatentPool& pool, const float* raw, int raw_ld, int 
 }
 
 // ------------------------------------------------------------------ attention, any size
-template <bool B16>
-__device__ __forceinline__ float latent_elem(const void* base, long r, int d, int row) {
-    if (B16) return bf16_to_f32(reinterpret_cast<const unsigned short*>(base)[latent_off(r, d, row)]);
-    return reinterpret_cast<const float*>(base)[(size_t)r * row + d];
+// accumulators of k_latent_attn_any: a set per group of threads, or one row that is wider than the workgroup
+__host__ __device__ inline int latent_any_acc(int rank_ld, int vec) { return rank_ld > 256 * vec ? rank_ld : 256 * vec; }
+template <bool B16, int VEC>
+__device__ __forceinline__ auto latent_elems(const void* base, long r, int d, int row) {
+    typedef float vec_t __attribute__((ext_vector_type(VEC)));
+    vec_t v;
+    if constexpr (B16) v[0] = bf16_to_f32(reinterpret_cast<const unsigned short*>(base)[latent_off(r, d, row)]);
+    else v = *reinterpret_cast<const vec_t*>(reinterpret_cast<const float*>(base) + (size_t)r * row + d);
+    return v;
 }
 
-template <bool B16>
+// A workgroup per (token, head), keys in blocks of 256; bound by the latency of a block's loads.  Sixteen lanes share a key's
+// row, four keys a group at once, and the threads beyond an output row's take other keys (VEC = 4: fp32 rows of whole
+// float4s; a key per thread, read value by value, took 59 us for 80 tokens x 16 heads and 200 keys of 256 + 32 values).
+template <bool B16, int VEC>
 __global__ __launch_bounds__(256) void k_latent_attn_any(const void* base, const void* q, const float* __restrict__ sink, float scale,
                                                          const int* __restrict__ pos, const int* __restrict__ seq,
                                                          const int* __restrict__ tbl_off, const int* __restrict__ tables, int block_size, int H,
                                                          int rank, int rank_ld, int row, float* out_f32, __half* out_b16, int Kb_out) {
-    extern __shared__ float lds_any[];   // q row [row], accumulators [rank_ld], weights [256], reductions [8]
+    typedef float vec_t __attribute__((ext_vector_type(VEC)));
+    extern __shared__ __attribute__((aligned(16))) float lds_any[];   // q row [row], accumulators [latent_any_acc()], weights [256], reductions [8], rows [256]
     float* sq = lds_any;
     float* acc = sq + row;
-    float* sp = acc + rank_ld;
+    const int acc_n = latent_any_acc(rank_ld, VEC);
+    float* sp = acc + acc_n;
     float* red = sp + 256;
+    int* srow = reinterpret_cast<int*>(red + 8);
     const int t = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     for (int d = tid; d < row; d += 256) {
         const size_t i = ((size_t)t * H + h) * row + d;
         sq[d] = B16 ? bf16_to_f32(reinterpret_cast<const unsigned short*>(q)[i]) : reinterpret_cast<const float*>(q)[i];
     }
-    for (int d = tid; d < rank_ld; d += 256) acc[d] = 0.f;
+    for (int d = tid; d < acc_n; d += 256) acc[d] = 0.f;
+    // columns: VEC neighbouring outputs; `groups` of threads share the keys of a block where a row has fewer columns than threads
+    const int cols = rank / VEC, per = min(cols, 256), groups = 256 / per, grp = tid / per, col0 = tid - grp * per;
+    const int sub = lane & 15, quarter = wave * 4 + (lane >> 4);
     const int p = pos[t];
     const int* table = tables + tbl_off[seq[t]];
     float m = -INFINITY, l = 0.f;   // the same in every thread
-    __syncthreads();
     for (int k0 = 0; k0 <= p; k0 += 256) {
-        const int key = k0 + tid;
-        float s = -INFINITY;
-        if (key <= p) {
-            const long r = (long)table[key / block_size] * block_size + key % block_size;
-            float dot = 0.f;
-            for (int d = 0; d < row; d++) dot = fmaf(sq[d], latent_elem<B16>(base, r, d, row), dot);
-            s = dot * scale;
+        const int n = min(256, p - k0 + 1);
+        if (tid < n) {
+            const int key = k0 + tid;
+            srow[tid] = table[key / block_size] * block_size + key % block_size;
         }
+        __syncthreads();   // (and the query, the first time)
+        for (int b = 0; b < n; b += 64) {
+            constexpr int U = 4;
+            float dot[U];
+            int at[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                dot[u] = 0.f;
+                at[u] = srow[min(b + 16 * u + quarter, n - 1)];
+            }
+            for (int d = sub * VEC; d < row; d += 16 * VEC) {
+                const vec_t qv = *reinterpret_cast<const vec_t*>(sq + d);
+                vec_t kv[U];
+#pragma unroll
+                for (int u = 0; u < U; u++) kv[u] = latent_elems<B16, VEC>(base, at[u], d, row);
+#pragma unroll
+                for (int u = 0; u < U; u++)
+#pragma unroll
+                    for (int e = 0; e < VEC; e++) dot[u] = fmaf(qv[e], kv[u][e], dot[u]);
+            }
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+#pragma unroll
+                for (int o = 8; o > 0; o >>= 1) dot[u] += __shfl_xor(dot[u], o, 64);
+                if (sub == u) sp[b + 16 * u + quarter] = dot[u];   // (past the n-th key: unused)
+            }
+        }
+        __syncthreads();
+        const float s = tid < n ? sp[tid] * scale : -INFINITY;
         float mx = s;
 #pragma unroll
         for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
         if (lane == 0) red[wave] = mx;
         __syncthreads();
         const float mn = fmaxf(m, fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3])));
-        const float e = key <= p ? expf(s - mn) : 0.f;
+        const float e = tid < n ? expf(s - mn) : 0.f;
         sp[tid] = e;
         float sum = e;
 #pragma unroll
@@ -119,22 +158,41 @@ __global__ __launch_bounds__(256) void k_latent_attn_any(const void* base, const
         const float alpha = m == -INFINITY ? 0.f : expf(m - mn);
         l = l * alpha + ((red[4] + red[5]) + (red[6] + red[7]));
         m = mn;
-        const int n = min(256, p - k0 + 1);
-        for (int d = tid; d < rank; d += 256) {
-            float a = acc[d] * alpha;
-            for (int k = 0; k < n; k++) {
-                const int kk = k0 + k;
-                const long r = (long)table[kk / block_size] * block_size + kk % block_size;
-                a = fmaf(sp[k], latent_elem<B16>(base, r, d, row), a);
+        if (grp < groups)
+            for (int c = col0; c < cols; c += per) {   // (one round unless the rows are very wide: then groups = 1)
+                float* mine = acc + ((size_t)grp * per + c) * VEC;
+                vec_t o;
+#pragma unroll
+                for (int i = 0; i < VEC; i++) o[i] = mine[i] * alpha;
+                constexpr int U = 8;   // keys in flight
+                for (int j = grp; j < n; j += U * groups) {
+                    vec_t v[U];
+                    float w[U];
+#pragma unroll
+                    for (int u = 0; u < U; u++) {
+                        const int k = j + u * groups;
+                        v[u] = latent_elems<B16, VEC>(base, srow[min(k, n - 1)], c * VEC, row);
+                        w[u] = k < n ? sp[k] : 0.f;
+                    }
+#pragma unroll
+                    for (int u = 0; u < U; u++)
+                        if (j + u * groups < n)
+#pragma unroll
+                            for (int i = 0; i < VEC; i++) o[i] = fmaf(w[u], v[u][i], o[i]);
+                }
+#pragma unroll
+                for (int i = 0; i < VEC; i++) mine[i] = o[i];
             }
-            acc[d] = a;
-        }
-        __syncthreads();   // weights and reductions are free again
+        __syncthreads();   // weights, rows and reductions are free again; the sums are there
     }
     const float top = fmaxf(m, sink[h]);
     const float f = expf(m - top), den = l * f + expf(sink[h] - top);
     for (int d = tid; d < rank_ld; d += 256) {
-        const float o = d < rank ? acc[d] * f / den : 0.f;
+        float o = 0.f;
+        if (d < rank) {
+            for (int i = 0; i < groups; i++) o += acc[i * per * VEC + d];
+            o = o * f / den;
+        }
         if (B16) {
             const int k = h * rank_ld + d;
             const __bf16 b = (__bf16)o;
@@ -143,6 +201,19 @@ __global__ __launch_bounds__(256) void k_latent_attn_any(const void* base, const
             out_f32[((size_t)t * H + h) * rank + d] = o;
         }
     }
+}
+template <bool B16, int VEC>
+static void launch_latent_any(const LatentAttn& a, const StepArrays& st) {
+    const LatentPool& P = a.pool;
+    const int row = P.row();
+    const size_t lds = ((size_t)row + latent_any_acc(P.rank_ld, VEC) + 256 + 8 + 256) * sizeof(float);
+    static bool enabled = false;
+    if (lds > 64 * 1024 && !enabled) {   // (up to 5 KiB more than the sizes the caller allows)
+        HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_latent_attn_any<B16, VEC>), hipFuncAttributeMaxDynamicSharedMemorySize, 72 * 1024));
+        enabled = true;
+    }
+    NVLLM_LAUNCH((k_latent_attn_any<B16, VEC>), dim3(st.T, a.H), dim3(256), lds, P.base, a.q, a.sink, a.scale, st.d_pos, st.d_seq, st.d_tbl_off, st.d_tables,
+                 P.block_size, a.H, P.rank, P.rank_ld, row, a.out_f32, a.out_b16, B16 ? a.H * P.rank_ld / 32 : 0);
 }
 
 // ------------------------------------------------------------------ attention, bf16 pages
@@ -516,13 +587,9 @@ void launch_latent_attention(const LatentAttn& a, const StepArrays& st) {
         const size_t lds = ((size_t)row + P.rank_ld + 256 + 8) * sizeof(float);
         if (lds > 64 * 1024) NVLLM_FATAL("latent attention: a cached row of %d values is not supported", row);
         ProfScope ps(PC_LATENT_ATTN, bytes, flops);
-        const dim3 grid(st.T, a.H);
-        if (P.elem_bytes == 2)
-            NVLLM_LAUNCH((k_latent_attn_any<true>), grid, dim3(256), lds, P.base, a.q, a.sink, a.scale, st.d_pos, st.d_seq, st.d_tbl_off, st.d_tables,
-                         P.block_size, a.H, P.rank, P.rank_ld, row, a.out_f32, a.out_b16, a.H * P.rank_ld / 32);
-        else
-            NVLLM_LAUNCH((k_latent_attn_any<false>), grid, dim3(256), lds, P.base, a.q, a.sink, a.scale, st.d_pos, st.d_seq, st.d_tbl_off, st.d_tables,
-                         P.block_size, a.H, P.rank, P.rank_ld, row, a.out_f32, a.out_b16, 0);
+        if (P.elem_bytes == 2) launch_latent_any<true, 1>(a, st);
+        else if (P.rank % 4 || row % 4) launch_latent_any<false, 1>(a, st);
+        else launch_latent_any<false, 4>(a, st);
         return;
     }
     LatentKArgs k{};
@@ -590,46 +657,83 @@ void launch_latent_attention(const LatentAttn& a, const StepArrays& st) {
 }
 
 // ------------------------------------------------------------------ fp32 head products
+// A workgroup takes a head, HEAD_T tokens and 64 columns (k_latent_q_f32) or 16 outputs (k_latent_v_f32), so that a weight is
+// read once for several tokens and a wave has a dozen loads in flight (a token a workgroup, one load after the other: 25 and
+// 29 us for 80 tokens x 16 heads of 64 x 256; the products themselves are 42 MFLOP each).
+constexpr int HEAD_T = 8;
 __global__ __launch_bounds__(256) void k_latent_q_f32(float* __restrict__ rows, const float* __restrict__ q, const float* __restrict__ uk,
-                                                      const float2* __restrict__ rope, const int* __restrict__ pos, int H, int dim, int rot, int rank) {
-    const int t = blockIdx.x, h = blockIdx.y;
-    const float* qh = q + ((size_t)t * H + h) * (dim + rot);
-    float* dst = rows + ((size_t)t * H + h) * (rank + rot);
-    for (int j = threadIdx.x; j < rank; j += 256) {
-        float s = 0.f;
-        for (int d = 0; d < dim; d++) s = fmaf(qh[d], uk[((size_t)h * dim + d) * rank + j], s);
-        dst[j] = s;
+                                                      const float2* __restrict__ rope, const int* __restrict__ pos, int T, int H, int dim, int rot, int rank) {
+    __shared__ float s_q[HEAD_T][64], s_part[4][HEAD_T][64];
+    const int t0 = blockIdx.x * HEAD_T, h = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, j = blockIdx.z * 64 + lane;
+    const int n = min(HEAD_T, T - t0);
+    auto row_of = [&](int u) { return q + ((size_t)(t0 + min(u, n - 1)) * H + h) * (dim + rot); };
+    float acc[HEAD_T] = {};
+    for (int d0 = 0; d0 < dim; d0 += 64) {   // a wave takes sixteen of each 64 dims
+        __syncthreads();
+        for (int i = tid; i < HEAD_T * 64; i += 256) s_q[i >> 6][i & 63] = d0 + (i & 63) < dim ? row_of(i >> 6)[d0 + (i & 63)] : 0.f;
+        float w[16];
+#pragma unroll
+        for (int i = 0; i < 16; i++) w[i] = uk[((size_t)h * dim + min(d0 + wave * 16 + i, dim - 1)) * rank + min(j, rank - 1)];
+#pragma unroll
+        for (int i = 0; i < 16; i++)
+            if (d0 + wave * 16 + i >= dim) w[i] = 0.f;
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < 16; i++)
+#pragma unroll
+            for (int u = 0; u < HEAD_T; u++) acc[u] = fmaf(s_q[u][wave * 16 + i], w[i], acc[u]);
     }
-    for (int i = threadIdx.x; i < rot / 2; i += 256) {
-        const float2 cs = rope[(size_t)pos[t] * (rot / 2) + i];
-        const float u = qh[dim + 2 * i], v = qh[dim + 2 * i + 1];
-        dst[rank + 2 * i] = u * cs.x - v * cs.y;
-        dst[rank + 2 * i + 1] = v * cs.x + u * cs.y;
-    }
+#pragma unroll
+    for (int u = 0; u < HEAD_T; u++) s_part[wave][u][lane] = acc[u];
+    __syncthreads();
+    for (int u = wave; u < n; u += 4)
+        if (j < rank) rows[((size_t)(t0 + u) * H + h) * (rank + rot) + j] = (s_part[0][u][lane] + s_part[1][u][lane]) + (s_part[2][u][lane] + s_part[3][u][lane]);
+    if (blockIdx.z) return;
+    for (int u = wave; u < n; u += 4)
+        for (int i = lane; i < rot / 2; i += 64) {
+            const float* qh = row_of(u);
+            float* dst = rows + ((size_t)(t0 + u) * H + h) * (rank + rot);
+            const float2 cs = rope[(size_t)pos[t0 + u] * (rot / 2) + i];
+            const float a = qh[dim + 2 * i], b = qh[dim + 2 * i + 1];
+            dst[rank + 2 * i] = a * cs.x - b * cs.y;
+            dst[rank + 2 * i + 1] = b * cs.x + a * cs.y;
+        }
 }
 void launch_latent_q_f32(float* rows, const float* q, const float* uk, const float2* rope, const int* pos, int T, int H, int dim, int rot, int rank) {
     if (T <= 0) return;
     ProfScope ps(PC_GEMM_ABSORB, (double)H * dim * rank * 4.0 + (double)T * H * (dim + rank + 2 * rot) * 4.0, 2.0 * T * (double)H * dim * rank);
-    NVLLM_LAUNCH(k_latent_q_f32, dim3(T, H), dim3(256), 0, rows, q, uk, rope, pos, H, dim, rot, rank);
+    NVLLM_LAUNCH(k_latent_q_f32, dim3(cdiv(T, HEAD_T), H, cdiv(rank, 64)), dim3(256), 0, rows, q, uk, rope, pos, T, H, dim, rot, rank);
 }
 
-__global__ __launch_bounds__(256) void k_latent_v_f32(float* __restrict__ out, const float* __restrict__ lat, const float* __restrict__ uv, int H, int vdim,
+__global__ __launch_bounds__(256) void k_latent_v_f32(float* __restrict__ out, const float* __restrict__ lat, const float* __restrict__ uv, int T, int H, int vdim,
                                                       int rank) {
-    const int t = blockIdx.x, h = blockIdx.y, lane = threadIdx.x & 63;
-    const float* lh = lat + ((size_t)t * H + h) * rank;
-    for (int v = threadIdx.x >> 6; v < vdim; v += 4) {   // a wave per output
-        const float* w = uv + ((size_t)h * vdim + v) * rank;
-        float s = 0.f;
-        for (int c = lane; c < rank; c += 64) s = fmaf(lh[c], w[c], s);
+    const int t0 = blockIdx.x * HEAD_T, h = blockIdx.y, lane = threadIdx.x & 63, v0 = blockIdx.z * 16 + (threadIdx.x >> 6) * 4;   // four outputs a wave
+    const int n = min(HEAD_T, T - t0);
+    float s[4][HEAD_T] = {};
+    for (int c = lane; c < rank; c += 64) {
+        float w[4], x[HEAD_T];
 #pragma unroll
-        for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
-        if (lane == 0) out[((size_t)t * H + h) * vdim + v] = s;
+        for (int i = 0; i < 4; i++) w[i] = uv[((size_t)h * vdim + min(v0 + i, vdim - 1)) * rank + c];
+#pragma unroll
+        for (int u = 0; u < HEAD_T; u++) x[u] = lat[((size_t)(t0 + min(u, n - 1)) * H + h) * rank + c];
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+#pragma unroll
+            for (int u = 0; u < HEAD_T; u++) s[i][u] = fmaf(x[u], w[i], s[i][u]);
     }
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int u = 0; u < HEAD_T; u++) {
+#pragma unroll
+            for (int o = 32; o > 0; o >>= 1) s[i][u] += __shfl_xor(s[i][u], o, 64);
+            if (lane == i * HEAD_T + u && u < n && v0 + i < vdim) out[((size_t)(t0 + u) * H + h) * vdim + v0 + i] = s[i][u];
+        }
 }
 void launch_latent_v_f32(float* out, const float* lat, const float* uv, int T, int H, int vdim, int rank) {
     if (T <= 0) return;
     ProfScope ps(PC_GEMM_VALUE, (double)H * vdim * rank * 4.0 + (double)T * H * (vdim + rank) * 4.0, 2.0 * T * (double)H * vdim * rank);
-    NVLLM_LAUNCH(k_latent_v_f32, dim3(T, H), dim3(256), 0, out, lat, uv, H, vdim, rank);
+    NVLLM_LAUNCH(k_latent_v_f32, dim3(cdiv(T, HEAD_T), H, cdiv(vdim, 16)), dim3(256), 0, out, lat, uv, T, H, vdim, rank);
 }
 
 // ------------------------------------------------------------------ converters

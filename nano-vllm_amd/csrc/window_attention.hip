@@ -37,6 +37,8 @@ size_t kv_pages_bytes(int elem_bytes, int block_size, int num_blocks, int G, int
     return ((size_t)num_blocks * block_size * G * (p.dim_ld + p.vdim_ld) * elem_bytes + 255) & ~(size_t)255;
 }
 
+// accumulators of k_window_attn_any: a set per group of threads, or one row that is wider than the workgroup
+__host__ __device__ inline int window_any_acc(int vdim_ld, int vec) { return vdim_ld > 256 * vec ? vdim_ld : 256 * vec; }
 __device__ __forceinline__ float b16_f32(unsigned short v) { return __builtin_bit_cast(float, (unsigned)v << 16); }
 __device__ __forceinline__ size_t key_off(long row, int g, int G, int d, int dim_ld) {
     return ((size_t)(row >> 4) * G + g) * (KV_PAGE * dim_ld) + (d >> 5) * 512 + ((row & 15) + 16 * ((d >> 3) & 3)) * 8 + (d & 7);
@@ -410,14 +412,20 @@ void launch_conv_rope(const ConvRope& c, const KvPages& pool, const StepArrays& 
 }
 
 // ------------------------------------------------------------------ attention, any size
-template <bool B16>
+// A workgroup per (token, head), keys in blocks of 256.  What bounds it is the latency of a block's loads: a key per thread,
+// read value by value, and a thread per output over all the block's keys were two chains of hundreds of loads (87 us for 80
+// tokens x 16 heads of 64 and 200 keys).  So sixteen lanes share a key's row, four keys a group at once, and the threads
+// beyond an output row's take other keys (VEC = 4: fp32 rows of whole float4s).
+template <bool B16, int VEC>
 __global__ __launch_bounds__(256) void k_window_attn_any(KvPages pool, const void* q, float scale, float cap, int size, int keep, const int* __restrict__ pos,
                                                          const int* __restrict__ seq, const int* __restrict__ tbl_off, const int* __restrict__ tables, int H,
                                                          float* out_f32, __half* out_b16, int Kb_out) {
-    extern __shared__ float lds_any[];   // query [dim_ld], accumulators [vdim_ld], weights [256], reductions [8], rows [256]
+    typedef float vec_t __attribute__((ext_vector_type(VEC)));
+    extern __shared__ __attribute__((aligned(16))) float lds_any[];   // query [dim_ld], accumulators [window_any_acc()], weights [256], reductions [8], rows [256]
     float* sq = lds_any;
     float* acc = sq + pool.dim_ld;
-    float* sp = acc + pool.vdim_ld;
+    const int acc_n = window_any_acc(pool.vdim_ld, VEC);
+    float* sp = acc + acc_n;
     float* red = sp + 256;
     int* srow = reinterpret_cast<int*>(red + 8);
     const int t = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = h / (H / pool.G);
@@ -425,25 +433,56 @@ __global__ __launch_bounds__(256) void k_window_attn_any(KvPages pool, const voi
         const size_t i = ((size_t)t * H + h) * pool.dim_ld + d;
         sq[d] = B16 ? b16_f32(reinterpret_cast<const unsigned short*>(q)[i]) : reinterpret_cast<const float*>(q)[i];
     }
-    for (int d = tid; d < pool.vdim_ld; d += 256) acc[d] = 0.f;
+    for (int d = tid; d < acc_n; d += 256) acc[d] = 0.f;
+    auto load = [&](const void* base, bool values, int row, int d) {
+        vec_t v;
+        if constexpr (B16) v[0] = b16_f32(reinterpret_cast<const unsigned short*>(base)[values ? value_off(row, g, pool.G, d, pool.vdim_ld) : key_off(row, g, pool.G, d, pool.dim_ld)]);
+        else v = *reinterpret_cast<const vec_t*>(reinterpret_cast<const float*>(base) + ((size_t)row * pool.G + g) * (values ? pool.vdim : pool.dim) + d);
+        return v;
+    };
+    // columns: VEC neighbouring outputs; `groups` of threads share the keys of a block where a row has fewer columns than threads
+    const int cols = pool.vdim / VEC, per = min(cols, 256), groups = 256 / per, grp = tid / per, col0 = tid - grp * per;
+    const int sub = lane & 15, quarter = wave * 4 + (lane >> 4);
     const int p = pos[t], lo = max(0, p - size + 1), first = min(keep, lo), n_keys = first + p - lo + 1;
     const int* table = tables + tbl_off[seq[t]];
     float m = -INFINITY, l = 0.f;   // the same in every thread
-    __syncthreads();
     for (int k0 = 0; k0 < n_keys; k0 += 256) {
-        const int k = k0 + tid;
-        float s = -INFINITY;
+        const int k = k0 + tid, n = min(256, n_keys - k0);
         if (k < n_keys) {
             const int key = k < first ? k : lo + k - first;
-            const int row = table[key / pool.block_size] * pool.block_size + key % pool.block_size;
-            srow[tid] = row;
-            float dot = 0.f;
-            for (int d = 0; d < pool.dim; d++) {
-                const float kv = B16 ? b16_f32(reinterpret_cast<const unsigned short*>(pool.keys)[key_off(row, g, pool.G, d, pool.dim_ld)])
-                                     : reinterpret_cast<const float*>(pool.keys)[((size_t)row * pool.G + g) * pool.dim + d];
-                dot = fmaf(sq[d], kv, dot);
+            srow[tid] = table[key / pool.block_size] * pool.block_size + key % pool.block_size;
+        }
+        __syncthreads();   // (and the query, the first time)
+        for (int b = 0; b < n; b += 64) {
+            constexpr int U = 4;
+            float dot[U];
+            int row[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                dot[u] = 0.f;
+                row[u] = srow[min(b + 16 * u + quarter, n - 1)];
             }
-            s = dot * scale;
+            for (int d = sub * VEC; d < pool.dim; d += 16 * VEC) {
+                const vec_t qv = *reinterpret_cast<const vec_t*>(sq + d);
+                vec_t kv[U];
+#pragma unroll
+                for (int u = 0; u < U; u++) kv[u] = load(pool.keys, false, row[u], d);
+#pragma unroll
+                for (int u = 0; u < U; u++)
+#pragma unroll
+                    for (int e = 0; e < VEC; e++) dot[u] = fmaf(qv[e], kv[u][e], dot[u]);
+            }
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+#pragma unroll
+                for (int o = 8; o > 0; o >>= 1) dot[u] += __shfl_xor(dot[u], o, 64);
+                if (sub == u) sp[b + 16 * u + quarter] = dot[u];   // (past the n-th key: unused)
+            }
+        }
+        __syncthreads();
+        float s = -INFINITY;
+        if (tid < n) {
+            s = sp[tid] * scale;
             if (cap > 0.f) s = cap * tanhf(s / cap);
         }
         float mx = s;
@@ -452,7 +491,7 @@ __global__ __launch_bounds__(256) void k_window_attn_any(KvPages pool, const voi
         if (lane == 0) red[wave] = mx;
         __syncthreads();
         const float mn = fmaxf(m, fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3])));
-        const float e = k < n_keys ? expf(s - mn) : 0.f;
+        const float e = tid < n ? expf(s - mn) : 0.f;
         sp[tid] = e;
         float sum = e;
 #pragma unroll
@@ -462,20 +501,39 @@ __global__ __launch_bounds__(256) void k_window_attn_any(KvPages pool, const voi
         const float alpha = m == -INFINITY ? 0.f : expf(m - mn);
         l = l * alpha + ((red[4] + red[5]) + (red[6] + red[7]));
         m = mn;
-        const int n = min(256, n_keys - k0);
-        for (int d = tid; d < pool.vdim; d += 256) {
-            float o = acc[d] * alpha;
-            for (int j = 0; j < n; j++) {
-                const float vv = B16 ? b16_f32(reinterpret_cast<const unsigned short*>(pool.values)[value_off(srow[j], g, pool.G, d, pool.vdim_ld)])
-                                     : reinterpret_cast<const float*>(pool.values)[((size_t)srow[j] * pool.G + g) * pool.vdim + d];
-                o = fmaf(sp[j], vv, o);
+        if (grp < groups)
+            for (int c = col0; c < cols; c += per) {   // (one round unless the values are very wide: then groups = 1)
+                float* mine = acc + ((size_t)grp * per + c) * VEC;
+                vec_t o;
+#pragma unroll
+                for (int i = 0; i < VEC; i++) o[i] = mine[i] * alpha;
+                constexpr int U = 4;   // keys in flight
+                for (int j = grp; j < n; j += U * groups) {
+                    vec_t v[U];
+                    float w[U];
+#pragma unroll
+                    for (int u = 0; u < U; u++) {
+                        const int at = j + u * groups;
+                        v[u] = load(pool.values, true, srow[min(at, n - 1)], c * VEC);
+                        w[u] = at < n ? sp[at] : 0.f;
+                    }
+#pragma unroll
+                    for (int u = 0; u < U; u++)
+                        if (j + u * groups < n)
+#pragma unroll
+                            for (int i = 0; i < VEC; i++) o[i] = fmaf(w[u], v[u][i], o[i]);
+                }
+#pragma unroll
+                for (int i = 0; i < VEC; i++) mine[i] = o[i];
             }
-            acc[d] = o;
-        }
-        __syncthreads();   // weights, rows and reductions are free again
+        __syncthreads();   // weights, rows and reductions are free again; the sums are there
     }
     for (int d = tid; d < pool.vdim_ld; d += 256) {
-        const float o = d < pool.vdim ? acc[d] / l : 0.f;
+        float o = 0.f;
+        if (d < pool.vdim) {
+            for (int i = 0; i < groups; i++) o += acc[i * per * VEC + d];
+            o /= l;
+        }
         if (B16) {
             const int k = h * pool.vdim_ld + d;
             reinterpret_cast<__bf16*>(out_b16)[((size_t)(t >> 4) * Kb_out + (k >> 5)) * TILE_HALVES + (size_t)((t & 15) + 16 * ((k >> 3) & 3)) * 8 + (k & 7)] = (__bf16)o;
@@ -483,6 +541,18 @@ __global__ __launch_bounds__(256) void k_window_attn_any(KvPages pool, const voi
             out_f32[((size_t)t * H + h) * pool.vdim + d] = o;
         }
     }
+}
+template <bool B16, int VEC>
+static void launch_window_any(const WindowAttn& w, const StepArrays& st, int Kb_out) {
+    const KvPages& pool = w.pool;
+    const size_t lds = ((size_t)pool.dim_ld + window_any_acc(pool.vdim_ld, VEC) + 256 + 8 + 256) * 4;
+    static bool enabled = false;
+    if (lds > 64 * 1024 && !enabled) {   // (up to 4 KiB more than the sizes the caller allows)
+        HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_window_attn_any<B16, VEC>), hipFuncAttributeMaxDynamicSharedMemorySize, 72 * 1024));
+        enabled = true;
+    }
+    NVLLM_LAUNCH((k_window_attn_any<B16, VEC>), dim3(st.T, w.H), dim3(256), lds, pool, w.q, w.scale, w.cap, w.size, w.keep_first, st.d_pos, st.d_seq, st.d_tbl_off,
+                 st.d_tables, w.H, w.out_f32, w.out_b16, Kb_out);
 }
 
 // ------------------------------------------------------------------ attention, bf16 pages
@@ -835,13 +905,9 @@ void launch_window_attention(const WindowAttn& w, const StepArrays& st) {
         const size_t lds = ((size_t)pool.dim_ld + pool.vdim_ld + 256 + 8 + 256) * 4;
         if (lds > 64 * 1024) NVLLM_FATAL("attention heads of %d and %d values are too wide", pool.dim, pool.vdim);
         ProfScope ps(PC_WINDOW_ATTN, 0, 0);
-        const dim3 grid(st.T, w.H);
-        if (pool.elem_bytes == 4)
-            NVLLM_LAUNCH((k_window_attn_any<false>), grid, dim3(256), lds, pool, w.q, w.scale, w.cap, w.size, w.keep_first, st.d_pos, st.d_seq, st.d_tbl_off, st.d_tables, w.H,
-                         w.out_f32, w.out_b16, Kb_out);
-        else
-            NVLLM_LAUNCH((k_window_attn_any<true>), grid, dim3(256), lds, pool, w.q, w.scale, w.cap, w.size, w.keep_first, st.d_pos, st.d_seq, st.d_tbl_off, st.d_tables, w.H,
-                         w.out_f32, w.out_b16, Kb_out);
+        if (pool.elem_bytes != 4) launch_window_any<true, 1>(w, st, Kb_out);
+        else if (pool.dim % 4 || pool.vdim % 4) launch_window_any<false, 1>(w, st, Kb_out);
+        else launch_window_any<false, 4>(w, st, Kb_out);
         return;
     }
     WindowKArgs a{};
