@@ -81,7 +81,7 @@ __device__ __forceinline__ auto latent_elems(const void* base, long r, int d, in
 
 // A workgroup per (token, head), keys in blocks of 256; bound by the latency of a block's loads.  Sixteen lanes share a key's
 // row, four keys a group at once, and the threads beyond an output row's take other keys (VEC = 4: fp32 rows of whole
-// float4s; a key per thread, read value by value, took 59 us for 80 tokens x 16 heads and 200 keys of 256 + 32 values).
+// float4s).  80 tokens x 16 heads, 200 keys of 256 + 32 values: 60 us with a key per thread, read value by value, 23 so.
 template <bool B16, int VEC>
 __global__ __launch_bounds__(256) void k_latent_attn_any(const void* base, const void* q, const float* __restrict__ sink, float scale,
                                                          const int* __restrict__ pos, const int* __restrict__ seq,
@@ -658,8 +658,9 @@ void launch_latent_attention(const LatentAttn& a, const StepArrays& st) {
 
 // ------------------------------------------------------------------ fp32 head products
 // A workgroup takes a head, HEAD_T tokens and 64 columns (k_latent_q_f32) or 16 outputs (k_latent_v_f32), so that a weight is
-// read once for several tokens and a wave has a dozen loads in flight (a token a workgroup, one load after the other: 25 and
-// 29 us for 80 tokens x 16 heads of 64 x 256; the products themselves are 42 MFLOP each).
+// read once for several tokens and a wave has a dozen loads in flight: 6 and 13 us for 80 tokens x 16 heads of 64 x 256 (a
+// token a workgroup, one load after the other: 25 and 29; the products themselves are 42 MFLOP each).  k_latent_v_f32 with
+// float4 loads and a sum over lanes of half the steps measured 26.
 constexpr int HEAD_T = 8;
 __global__ __launch_bounds__(256) void k_latent_q_f32(float* __restrict__ rows, const float* __restrict__ q, const float* __restrict__ uk,
                                                       const float2* __restrict__ rope, const int* __restrict__ pos, int T, int H, int dim, int rot, int rank) {

@@ -459,10 +459,11 @@ __global__ __launch_bounds__(256) void k_lightning_step(Lightning a, const int4*
 
 // fp32 portions whose state fits the workgroup's registers (a thread: four value columns x NR dims): the state is read and
 // written once per portion instead of once per token, and BATCH tokens' rows and partial results pass through LDS together.
-// Streaming the state took 1.9 us a token (142 us for a portion of 77 tokens x 16 heads of 64 x 64).
+// What is left is a batch's chain: rows to LDS, eight tokens of products, the sum over lanes and waves.  A portion of 77
+// tokens x 16 heads of 64 x 64: 142 us with the state streamed, 53 with a token's rows fetched when it comes, 33 so.
 template <int NR>
 __global__ __launch_bounds__(256) void k_lightning_portion(Lightning a, const int4* __restrict__ spans) {
-    constexpr int BATCH = 8;
+    constexpr int BATCH = 8, ITEMS = 5;
     extern __shared__ __attribute__((aligned(16))) float lds_s[];   // q, k [BATCH][dim], v [BATCH][vdim], partial results [BATCH][4][vdim]
     float* s_q = lds_s;
     float* s_k = s_q + BATCH * a.dim;
@@ -479,37 +480,57 @@ __global__ __launch_bounds__(256) void k_lightning_portion(Lightning a, const in
         S[r] = f4_t{0.f, 0.f, 0.f, 0.f};
         if (span.z > 0) S[r] = *reinterpret_cast<const f4_t*>(st + (size_t)(row0 + rows * r) * a.vdim + col);   // (a sequence's first token: from zero)
     }
+    // the float4s of a batch's rows that this thread brings: q, k and v of a token lie behind one another, as in LDS
+    const int token4 = (2 * a.dim + a.vdim) / 4;
+    const float* src[ITEMS];
+    int tok[ITEMS], ld[ITEMS], dst[ITEMS];
+#pragma unroll
+    for (int i = 0; i < ITEMS; i++) {
+        const int item = min(tid + 256 * i, BATCH * token4 - 1), d = (item % token4) * 4;
+        tok[i] = item / token4;
+        const bool is_v = d >= 2 * a.dim, is_k = d >= a.dim;
+        const int at = is_v ? d - 2 * a.dim : is_k ? d - a.dim : d;
+        ld[i] = a.H * (is_v ? a.vdim : a.dim);
+        src[i] = (is_v ? a.v32 + h * a.vdim : (is_k ? a.k32 : a.q32) + h * a.dim) + at;
+        dst[i] = is_v ? 2 * BATCH * a.dim + tok[i] * a.vdim + at : (is_k ? BATCH * a.dim : 0) + tok[i] * a.dim + at;
+    }
+    f4_t in[ITEMS];
+    auto fetch = [&](int i0) {
+#pragma unroll
+        for (int i = 0; i < ITEMS; i++) in[i] = *reinterpret_cast<const f4_t*>(src[i] + (size_t)(span.x + min(i0 + tok[i], span.y - 1)) * ld[i]);
+    };
+    fetch(0);
     for (int i0 = 0; i0 < span.y; i0 += BATCH) {
         const int n = min(BATCH, span.y - i0), t0 = span.x + i0;
-        for (int i = tid; i < n * a.dim; i += 256) {
-            const int u = i / a.dim, d = i - u * a.dim;
-            const size_t at = ((size_t)(t0 + u) * a.H + h) * a.dim + d;
-            s_q[i] = a.q32[at];
-            s_k[i] = a.k32[at];
-        }
-        for (int i = tid; i < n * a.vdim; i += 256) {
-            const int u = i / a.vdim, v = i - u * a.vdim;
-            s_v[i] = a.v32[((size_t)(t0 + u) * a.H + h) * a.vdim + v];
-        }
+        // rows of zeros behind the last token: with a decay of one they change nothing, so the tokens' loop has no branch
+#pragma unroll
+        for (int i = 0; i < ITEMS; i++) *reinterpret_cast<f4_t*>(lds_s + dst[i]) = tok[i] < n ? in[i] : f4_t{0.f, 0.f, 0.f, 0.f};
         __syncthreads();
-        for (int u = 0; u < n; u++) {
+        fetch(i0 + BATCH);   // (behind the last batch: the last token again)
+        f4_t part[BATCH];
+#pragma unroll
+        for (int u = 0; u < BATCH; u++) {
             const f4_t v = *reinterpret_cast<const f4_t*>(s_v + u * a.vdim + col);
-            const bool fresh = span.z + i0 + u == 0;
-            f4_t part = {0.f, 0.f, 0.f, 0.f};
+            const float keep = u < n ? decay : 1.f;
+            part[u] = f4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int r = 0; r < NR; r++) {
                 const float kd = s_k[u * a.dim + row0 + rows * r], qd = s_q[u * a.dim + row0 + rows * r];
 #pragma unroll
                 for (int e = 0; e < 4; e++) {
-                    S[r][e] = fmaf(kd, v[e], fresh ? 0.f : decay * S[r][e]);
-                    part[e] = fmaf(qd, S[r][e], part[e]);
+                    S[r][e] = fmaf(kd, v[e], keep * S[r][e]);
+                    part[u][e] = fmaf(qd, S[r][e], part[u][e]);
                 }
             }
-            for (int o = per; o < 64; o <<= 1)
-#pragma unroll
-                for (int e = 0; e < 4; e++) part[e] += __shfl_xor(part[e], o, 64);
-            if (lane < per) *reinterpret_cast<f4_t*>(s_part + (u * 4 + wave) * a.vdim + col) = part;
         }
+        for (int o = per; o < 64; o <<= 1)
+#pragma unroll
+            for (int u = 0; u < BATCH; u++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) part[u][e] += __shfl_xor(part[u][e], o, 64);
+        if (lane < per)
+#pragma unroll
+            for (int u = 0; u < BATCH; u++) *reinterpret_cast<f4_t*>(s_part + (u * 4 + wave) * a.vdim + col) = part[u];
         __syncthreads();
         for (int i = tid; i < n * a.vdim; i += 256) {
             const int u = i / a.vdim, v = i - u * a.vdim;
@@ -527,7 +548,7 @@ static bool launch_portion(const Lightning& a, const int4* spans, const dim3& gr
     if (a.vdim % 4 || per < 8 || per > 64 || (per & (per - 1)) || a.dim % (256 / per)) return false;
     const int nr = a.dim / (256 / per);
     const size_t lds = (size_t)8 * (2 * a.dim + 5 * a.vdim) * sizeof(float);
-    if (lds > 64 * 1024) return false;
+    if (lds > 64 * 1024 || 8 * (2 * a.dim + a.vdim) > 5 * 256 * 4) return false;
     if (nr == 4) NVLLM_LAUNCH((k_lightning_portion<4>), grid, dim3(256), lds, a, spans);
     else if (nr == 8) NVLLM_LAUNCH((k_lightning_portion<8>), grid, dim3(256), lds, a, spans);
     else if (nr == 16) NVLLM_LAUNCH((k_lightning_portion<16>), grid, dim3(256), lds, a, spans);

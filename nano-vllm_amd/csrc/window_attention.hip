@@ -123,11 +123,22 @@ __global__ __launch_bounds__(256) void k_conv_rope(ConvKArgs a) {
         }
 #pragma unroll
         for (int e = 0; e < VEC; e++) y[e] = 0.f;
-        for (int j = 0; j <= keep; j++) {
-            const Vec u = input(off - keep + j, ch);
-            const float* w = a.c.taps + (size_t)j * a.channels + ch;
+        constexpr int U = VEC == 1 ? 4 : 1;   // taps requested together (one after the other a token of three taps took 12.8 us)
+        for (int j0 = 0; j0 <= keep; j0 += U) {
+            Vec u[U];
+            float wf[U][VEC];
 #pragma unroll
-            for (int e = 0; e < VEC; e++) y[e] = fmaf(w[e], (float)u.v[e], y[e]);
+            for (int i = 0; i < U; i++) {
+                const int j = min(j0 + i, keep);
+                u[i] = input(off - keep + j, ch);
+#pragma unroll
+                for (int e = 0; e < VEC; e++) wf[i][e] = a.c.taps[(size_t)j * a.channels + ch + e];
+            }
+#pragma unroll
+            for (int i = 0; i < U; i++)
+                if (j0 + i <= keep)
+#pragma unroll
+                    for (int e = 0; e < VEC; e++) y[e] = fmaf(wf[i][e], (float)u[i].v[e], y[e]);
         }
     };
     auto store = [&](int t, int d, const float* y) {
@@ -413,8 +424,8 @@ void launch_conv_rope(const ConvRope& c, const KvPages& pool, const StepArrays& 
 
 // ------------------------------------------------------------------ attention, any size
 // A workgroup per (token, head), keys in blocks of 256.  What bounds it is the latency of a block's loads: a key per thread,
-// read value by value, and a thread per output over all the block's keys were two chains of hundreds of loads (87 us for 80
-// tokens x 16 heads of 64 and 200 keys).  So sixteen lanes share a key's row, four keys a group at once, and the threads
+// read value by value, and a thread per output over all the block's keys were two chains of hundreds of loads (90 us for 80
+// tokens x 16 heads of 64 and 200 keys, 13 so).  So sixteen lanes share a key's row, four keys a group at once, and the threads
 // beyond an output row's take other keys (VEC = 4: fp32 rows of whole float4s).
 template <bool B16, int VEC>
 __global__ __launch_bounds__(256) void k_window_attn_any(KvPages pool, const void* q, float scale, float cap, int size, int keep, const int* __restrict__ pos,
