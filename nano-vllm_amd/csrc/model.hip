@@ -211,13 +211,15 @@ static PassSlot& next_slot(int B) {
     return slot;
 }
 
-// `host_written`: the pass's last kernel has stored the indices into next_slot(B).host itself.
-static long finish_pass(RunState* s, float* d_logits, int* d_argmax, int B, int V, PassView view, bool chained = false,
+// `host_written`: the pass's last kernel has stored the indices into next_slot(B).host itself.  `waits`: the caller waits for
+// the pass before it sends another, so its rows follow its kernels on the same stream: the switch to the copies' stream and
+// the event between them cost a pass 10 us.
+static long finish_pass(RunState* s, float* d_logits, int* d_argmax, int B, int V, PassView view, bool waits, bool chained = false,
                         bool host_written = false) {
     PassSlot& slot = next_slot(B);
     const long ticket = g_next_ticket++;
     hipStream_t stream = rt().stream;
-    if (rt().logits_mode == NVLLM_LOGITS_HOST) {
+    if (rt().logits_mode == NVLLM_LOGITS_HOST && !waits) {
         if (!rt().copy_stream) HIP_CHECK(hipStreamCreateWithFlags(&rt().copy_stream, hipStreamNonBlocking));
         if (!g_kernels_done) HIP_CHECK(hipEventCreateWithFlags(&g_kernels_done, hipEventDisableTiming));
         HIP_CHECK(hipEventRecord(g_kernels_done, stream));
@@ -232,7 +234,7 @@ static long finish_pass(RunState* s, float* d_logits, int* d_argmax, int B, int 
     if (rt().logits_mode == NVLLM_LOGITS_HOST && B > 0)
         HIP_CHECK(hipMemcpyAsync(s->logits, d_logits, (size_t)B * V * sizeof(float), hipMemcpyDeviceToHost, stream));
     HIP_CHECK(hipEventRecord(slot.ev, stream));
-    if (rt().logits_mode == NVLLM_LOGITS_HOST) g_rows_copied = slot.ev;
+    if (rt().logits_mode == NVLLM_LOGITS_HOST && !waits) g_rows_copied = slot.ev;
     slot.ticket = ticket;
     view.argmax = slot.host;
     view.outputs = B;
@@ -732,7 +734,7 @@ void transformer(int* tokens, int num_tokens, int pos, Config* p, RunState* s, W
 // the pass enqueued just before this one, taken on the GPU (the host need not have seen it yet).
 static long enqueue_pass(int* tokens, int num_tokens, int* pos_arr, int* seq_ids, int* output_indices,
                          int num_outputs, Config* p, RunState* s, Weights* w, BlockTable** block_tables,
-                         const int* token_src) {
+                         const int* token_src, bool waits) {
     ensure_init();
     if (!g_paged_mode) {  // model.c:374-377
         printf("Error: Continuous batching requires paged mode.\n");
@@ -745,12 +747,12 @@ static long enqueue_pass(int* tokens, int num_tokens, int* pos_arr, int* seq_ids
     if (T > p->max_seq_len || B > p->max_seq_len) NVLLM_FATAL("batch of %d tokens exceeds the workspace (%d)", T, p->max_seq_len);
     if (m->dir) {
         if (tp().active) NVLLM_FATAL("model folders are not split over tensor-parallel ranks");
-        const bool to_host = rt().logits_mode == NVLLM_LOGITS_ARGMAX && B > 0;
+        const bool to_host = B > 0;   // the arg-max kernel stores into the pass's page-locked array too
         PassArgs a{tokens, pos_arr, seq_ids, output_indices, token_src, T, B, block_tables, &g_kv_manager,
                    (float*)ws_get(WS_LOGITS, (size_t)B * p->vocab_size * sizeof(float)),
                    (int*)ws_get(WS_ARGMAX, (size_t)(p->max_seq_len + 64) * sizeof(int)), to_host ? next_slot(B).host : nullptr};
         m->dir->forward(a);
-        return finish_pass(s, a.d_logits, a.d_argmax, B, p->vocab_size, PassView{}, false, to_host);
+        return finish_pass(s, a.d_logits, a.d_argmax, B, p->vocab_size, PassView{}, waits, false, to_host);
     }
     // H, KVH, F, QD, KD: what THIS process computes (its tensor-parallel slice; the whole model when world == 1)
     const int D = p->dim, F = m->sh.hidden, hd = p->head_dim, H = m->sh.n_heads, KVH = m->sh.n_kv_heads;
@@ -784,8 +786,8 @@ static long enqueue_pass(int* tokens, int num_tokens, int* pos_arr, int* seq_ids
         if (st.d_tok_src) launch_patch_tokens(st.d_tokens, st.d_tok_src, d_argmax, T);
         wait_for_row_copies();
         forward_f32(st, T, B, p, s, w, pool, rope, d_logits);
-        launch_argmax(d_argmax, d_logits, B, V);
-        return finish_pass(s, d_logits, d_argmax, B, V, PassView{});
+        if (B > 0) launch_argmax_ld(d_argmax, d_logits, B, V, V, next_slot(B).host);
+        return finish_pass(s, d_logits, d_argmax, B, V, PassView{}, waits, false, true);
     }
 
     // One launch for all layers (chain.hip) when the step fits it: a decode-sized batch on an fp16 page pool,
@@ -886,7 +888,7 @@ static long enqueue_pass(int* tokens, int num_tokens, int* pos_arr, int* seq_ids
             }
         }
     }
-    if (B <= 0) return finish_pass(s, d_logits, d_argmax, 0, V, PassView{}, chained);   // nobody wants a row of this pass
+    if (B <= 0) return finish_pass(s, d_logits, d_argmax, 0, V, PassView{}, waits, chained);   // nobody wants a row of this pass
     // logits only for the rows named by output_indices                            (model.c:396,411-418)
     wait_for_row_copies();   // the previous pass's rows have left the workspaces the classifier writes
     const bool thin_head = B <= THIN_TOKENS && !partial;   // the classifier norms the residual rows itself
@@ -916,9 +918,9 @@ static long enqueue_pass(int* tokens, int num_tokens, int* pos_arr, int* seq_ids
         // the classifier's tiles also report their (maximum, index) pairs: the greedy token comes from
         // a merge of those instead of a second pass over the logits
         e5.amax_out = d_argmax;
-        // only token ids leave the GPU: the kernel that picks them also stores them into the pass's page-locked array
+        // the kernel that picks the token ids also stores them into the pass's page-locked array
         static const int direct_env = getenv("NVLLM_ARGMAX_DIRECT") ? atoi(getenv("NVLLM_ARGMAX_DIRECT")) : 1;
-        host_written = direct_env && rt().logits_mode == NVLLM_LOGITS_ARGMAX && !chained;
+        host_written = direct_env && !chained;
         if (host_written) e5.amax_out_host = next_slot(B).host;
         e5.amax_ld = (B + 63) & ~63;
         e5.amax_pairs = (float2*)ws_get(WS_AMAX_PAIRS, (size_t)cdiv(V, 16) * e5.amax_ld * sizeof(float2));
@@ -959,13 +961,13 @@ static long enqueue_pass(int* tokens, int num_tokens, int* pos_arr, int* seq_ids
         }
     }
 
-    return finish_pass(s, d_logits, d_argmax, B, V, view, chained, host_written);
+    return finish_pass(s, d_logits, d_argmax, B, V, view, waits, chained, host_written);
 }
 
 void transformer_batch(int* tokens, int num_tokens, int* pos_arr, int* seq_ids, int* output_indices,
                        int num_outputs, Config* p, RunState* s, Weights* w, BlockTable** block_tables) {
     const long ticket = enqueue_pass(tokens, num_tokens, pos_arr, seq_ids, output_indices, num_outputs, p, s, w,
-                                     block_tables, nullptr);
+                                     block_tables, nullptr, true);
     if (ticket < 0) return;
     collect_pass(ticket, nullptr);
     HIP_CHECK(hipStreamSynchronize(rt().stream));  // the call is synchronous, like the CPU reference
@@ -976,7 +978,7 @@ long nvllm_forward_enqueue(int* tokens, int num_tokens, int* pos_arr, int* seq_i
                            const int* token_src, Config* p, RunState* s, Weights* w, BlockTable** block_tables) {
     // (with host logits rows, every pass in flight needs a RunState of its own: its rows land in s->logits)
     if (num_tokens <= 0 || num_outputs < 0 || !tokens || !pos_arr || !seq_ids || !p || !s || !w || !block_tables) return -1;
-    return enqueue_pass(tokens, num_tokens, pos_arr, seq_ids, output_indices, num_outputs, p, s, w, block_tables, token_src);
+    return enqueue_pass(tokens, num_tokens, pos_arr, seq_ids, output_indices, num_outputs, p, s, w, block_tables, token_src, false);
 }
 
 int nvllm_forward_collect(long ticket, int* argmax_out, int cap) {
