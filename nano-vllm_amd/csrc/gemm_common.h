@@ -298,5 +298,6 @@ __device__ __forceinline__ void copy_tile_to_lds(const __half* lane_src, unsigne
 void launch_gemm_prefill(GemmArgs a);
 // gemm_wide_f16.hip: the same in tiles of 256 features; false: not for this launch
 bool launch_gemm_wide_f16(const GemmArgs& a);
+bool launch_gemm_wide_b16(const GemmArgs& a);   // gemm_wide_b16.hip: bf16 models
 
 }  // namespace nvllm

@@ -27,7 +27,7 @@ struct WideGeom {
     static constexpr int FB = 16;                          // 16-row blocks of W per tile, four per wave
     static constexpr int TILES = FB + PL * TBN;            // 1-KiB tiles per stage
     static constexpr int CPW = (TILES + 3) / 4;            // copies per wave and stage (the last tile is copied by several waves when there are fewer)
-    static constexpr int RING = TILES <= 24 ? 6 : TILES <= 30 ? 5 : 4;
+    static constexpr int RING = TILES <= 22 ? 7 : TILES <= 24 ? 6 : TILES <= 30 ? 5 : 4;
     static constexpr int RINV_BYTES = 1024;                // 1/rms of up to 256 tokens in front of the ring
     static constexpr int LDS = RINV_BYTES + RING * TILES * 1024;
     static_assert(LDS <= 160 * 1024, "the ring must fit the CU's LDS");

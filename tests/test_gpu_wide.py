@@ -1,6 +1,6 @@
 """The 256-feature tiles (csrc/gemm_wide.h) at every height, on widths and token counts that end inside a tile, and K that
 ends inside a turn of the ring: one projection at a time against the oracle, and whole passes with every epilogue.  The
-height is read from the environment once per process, hence a child process per height."""
+height is read from the environment once per process, hence a child process per height.  In bf16 too."""
 import os
 import subprocess
 import sys
@@ -9,7 +9,7 @@ import numpy as np
 import pytest
 
 from nvllm_amd import synth
-from tests import dense_tile_child, util
+from tests import dense_tile_child, hybrid_oracle, hybrid_util, util
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 TOKENS = (256, 300, 433)
@@ -76,3 +76,41 @@ def test_passes_through_every_epilogue(passes, tmp_path, height, kv_bytes):
     for i, o in enumerate(want):
         np.testing.assert_array_equal(got[f"sampled{i}"], o["sampled"])
         assert np.abs(got[f"logits{i}"] - o["logits"]).max() < (2e-4 if kv_bytes == 4 else 2e-3)   # the bars of the forward pass
+
+
+BF16_CHILD = """
+import sys
+import numpy as np
+from nvllm_amd import capi
+from tests import hybrid_util, test_gpu_wide
+eng = hybrid_util.engine(capi.load_hip(), sys.argv[1], False, tokens=704)
+got = hybrid_util.feed_all(eng, [[(0, 300), (1, 257)], [(0, 133)]], test_gpu_wide.bf16_sequences())
+eng.close()
+np.savez(sys.argv[2], **{str(q): rows for q, rows in got.items()})
+"""
+
+
+def bf16_sequences():
+    return {0: hybrid_util.tokens(433, 203, 1), 1: hybrid_util.tokens(257, 203, 2)}
+
+
+@pytest.fixture(scope="module")
+def bf16_passes(tmp_path_factory):
+    # K of 9 and 13 steps; dense, gated and row projections whose widths end inside a tile of 256 features
+    cfg = synth.hybrid_config(288, 203, [(hybrid_util.A(6, 2, 48, 64, size=150, keep_first=3, taps=3, rot=16), hybrid_util.E(64, 4, 2, 416)),
+                                         (hybrid_util.L(3, 64, 64), 800)])
+    path, cfg, w = hybrid_util.model(tmp_path_factory.mktemp("wide_bf16"), "wide", cfg=cfg)
+    return path, {q: hybrid_oracle.forward(cfg, w, seq) for q, seq in bf16_sequences().items()}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("height", [4, 6, 8, 10])
+def test_bf16_passes(bf16_passes, tmp_path, height):
+    path, want = bf16_passes
+    dst = str(tmp_path / "got.npz")
+    env = dict(os.environ, PYTHONPATH=ROOT + os.pathsep + os.environ.get("PYTHONPATH", ""), NVLLM_GEMM_WIDE=str(height))
+    r = subprocess.run([sys.executable, "-c", BF16_CHILD, path, dst], env=env, capture_output=True, text=True, timeout=150)
+    assert r.returncode == 0, r.stderr[-2000:]
+    got = np.load(dst)
+    for q, o in want.items():
+        assert hybrid_util.error(got[str(q)], o) < hybrid_util.limit(False), q   # the bar of the design's whole passes
