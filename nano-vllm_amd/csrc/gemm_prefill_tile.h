@@ -49,10 +49,9 @@ namespace nvllm {
 
 namespace {
 
-// FW = 16-row weight blocks per wave (4 or 8), KG = wave groups that split the K-steps, WR = rows of
-// the wave grid (WR x 2 waves per group: 2 -> 128-feature tiles; 4 -> 256-feature tiles compiles but measured
-// slower on this model's shapes and is not instantiated), TW = 16-token
-// blocks per wave (4, 3 or 2: the tile's height is chosen per launch so that its rounds of workgroups fill)
+// FW = 16-row weight blocks per wave, KG = wave groups that split the K-steps, WR = rows of the wave grid (WR x 2 waves per
+// group; 2: 128-feature tiles), TW = 16-token blocks per wave (4, 3 or 2: the tile's height is chosen per launch so that its
+// rounds of workgroups fill)
 template <int FW, int KG, int WR = 2, int TW = 4, int PL = 2>
 struct PfGeom {
     static constexpr int FB = WR * FW;                 // weight blocks per workgroup tile

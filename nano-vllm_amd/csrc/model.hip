@@ -118,8 +118,8 @@ struct PassSlot {
     PassView view;
 };
 static PassSlot g_pass[PASS_RING];
-// Logits rows to the host (8 MB per 64-row pass at a 32,000-word vocabulary): the copies of a pass run on a
-// stream of their own, behind an event that follows the pass's kernels, so that the next pass's layers do
+// Logits rows to the host (8 MB per 64-row pass at a 32,000-word vocabulary): the copies of a pass enqueued ahead run on
+// a stream of their own, behind an event that follows the pass's kernels, so that the next pass's layers do
 // not queue behind 0.16 ms of PCIe traffic.  What the copies read (the logits and index workspaces) is
 // overwritten by the next pass's classifier, which therefore waits for `g_rows_copied` first.
 static hipEvent_t g_kernels_done = nullptr;
