@@ -330,31 +330,64 @@ __device__ __forceinline__ bool pf_close_split(const GemmArgs& p, f4_t (&v)[NI][
     return true;
 }
 
-// 1/rms of the tile's tokens from the producer's sums of squares, while the first stages travel: neighbouring threads share
-// a token and every load of a thread is requested at once (two threads per token and one load after the other, in front of
-// the copies, cost 4 to 6 us a launch).
+// 1/rms of the tile's tokens from the producer's sums of squares, while the first stages travel (in front of the copies and one
+// load after the other it cost 4 to 6 us a launch): four neighbouring threads share a token's loads, all requested at once, and
+// each adds all of them, the even columns in one chain and the odd ones in another.  That order is kept whatever the tile: the
+// last bit of 1/rms decides how bf16 activations round, so another order gives a model other outputs.
+template <int Q>
+__device__ __forceinline__ float of_quad(float v) {   // the value of thread Q of each four
+    const int i = __builtin_bit_cast(int, v);
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(i, i, Q * 0x55, 0xf, 0xf, false));
+}
 template <int TOKENS, int THREADS>
 __device__ __forceinline__ void tile_rinv(const GemmArgs& p, int tb0, float* s_rinv) {
-    constexpr int PARTS = TOKENS * 8 <= THREADS ? 8 : TOKENS * 4 <= THREADS ? 4 : TOKENS * 2 <= THREADS ? 2 : 1;
-    const int tl = (int)threadIdx.x / PARTS, part = (int)threadIdx.x % PARTS;
-    const int t = min(tb0 * 16 + tl, p.T - 1), cols = p.e.ss_tiles;
-    const float* sp = p.e.ss_in + (size_t)(p.e.ss_gather ? p.e.ss_gather[t] : t) * cols;
-    float ss = 0.f;
+    constexpr int ROUNDS = (TOKENS * 4 + THREADS - 1) / THREADS;   // tokens of a thread
+    const int part = (int)threadIdx.x & 3, first = (int)threadIdx.x >> 2, cols = p.e.ss_tiles;
+    const float* sp[ROUNDS];
+    float even[ROUNDS], odd[ROUNDS];
+#pragma unroll
+    for (int r = 0; r < ROUNDS; r++) {
+        const int t = min(tb0 * 16 + first + r * (THREADS / 4), p.T - 1);
+        sp[r] = p.e.ss_in + (size_t)(p.e.ss_gather ? p.e.ss_gather[t] : t) * cols;
+        even[r] = odd[r] = 0.f;
+    }
     if ((cols & 3) == 0) {
-        for (int j0 = 4 * part; j0 < cols; j0 += 64 * PARTS) {
-            f4_t v[16];
+        for (int j0 = 0; j0 < cols; j0 += 64) {
+            f4_t v[ROUNDS][4];
 #pragma unroll
-            for (int j = 0; j < 16; j++) v[j] = *reinterpret_cast<const f4_t*>(sp + min(j0 + 4 * PARTS * j, cols - 4));
+            for (int r = 0; r < ROUNDS; r++)
 #pragma unroll
-            for (int j = 0; j < 16; j++)
-                if (j0 + 4 * PARTS * j < cols) ss += (v[j][0] + v[j][1]) + (v[j][2] + v[j][3]);
+                for (int i = 0; i < 4; i++) v[r][i] = *reinterpret_cast<const f4_t*>(sp[r] + min(j0 + 16 * i + 4 * part, cols - 4));
+#pragma unroll
+            for (int r = 0; r < ROUNDS; r++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    if (j0 + 16 * i + 4 * part >= cols) v[r][i] = f4_t{0.f, 0.f, 0.f, 0.f};
+                    auto add = [&](auto q) {
+                        even[r] += of_quad<decltype(q)::value>(v[r][i][0]);
+                        odd[r] += of_quad<decltype(q)::value>(v[r][i][1]);
+                        even[r] += of_quad<decltype(q)::value>(v[r][i][2]);
+                        odd[r] += of_quad<decltype(q)::value>(v[r][i][3]);
+                    };
+                    add(std::integral_constant<int, 0>{});
+                    add(std::integral_constant<int, 1>{});
+                    add(std::integral_constant<int, 2>{});
+                    add(std::integral_constant<int, 3>{});
+                }
         }
     } else {
-        for (int j = part; j < cols; j += PARTS) ss += sp[j];
+#pragma unroll
+        for (int r = 0; r < ROUNDS; r++)
+            for (int j = 0; j < cols; j += 2) {
+                even[r] += sp[r][j];
+                if (j + 1 < cols) odd[r] += sp[r][j + 1];
+            }
     }
 #pragma unroll
-    for (int o = 1; o < PARTS; o <<= 1) ss += __shfl_xor(ss, o, 64);
-    if (part == 0 && tl < TOKENS) s_rinv[tl] = __fdiv_rn(1.0f, sqrtf(__fadd_rn(__fdiv_rn(ss, (float)p.e.d_in), p.e.eps)));
+    for (int r = 0; r < ROUNDS; r++) {
+        const int tl = first + r * (THREADS / 4);
+        if (part == 0 && tl < TOKENS) s_rinv[tl] = __fdiv_rn(1.0f, sqrtf(__fadd_rn(__fdiv_rn(even[r] + odd[r], (float)p.e.d_in), p.e.eps)));
+    }
 }
 
 template <int FW, int KG, int EPI, typename KVT, int WR = 2, int TW = 4, typename OP = OpF16x2, bool GRP = false, bool EXP = false>
@@ -596,7 +629,7 @@ __global__ __launch_bounds__(128 * WR * KG, WR == 4 ? 4 : 2) void k_gemm_prefill
         wb = wb + 1 == nbuf ? 0 : wb + 1;
     }
     NVLLM_STAMP(3, acc[FW - 1][TW - 1][0]);
-    __syncthreads();   // the ring is free; s_rinv (written by a quarter of the threads) is visible
+    __syncthreads();   // the ring is free; s_rinv is visible
     NVLLM_STAMP(4, lane);
 
     if (KG == 1) {
