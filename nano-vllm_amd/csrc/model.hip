@@ -782,7 +782,7 @@ static long enqueue_pass(int* tokens, int num_tokens, int* pos_arr, int* seq_ids
     float* d_logits = (float*)ws_get(WS_LOGITS, (size_t)B * V * sizeof(float));
     // the arg-max indices live in a buffer that never moves (the next pass may read them as its tokens)
     int* d_argmax = (int*)ws_get(WS_ARGMAX, (size_t)(p->max_seq_len + 64) * sizeof(int));
-    if (m->f32) {   // fp32 weights: the reference's operator sequence
+    if (m->f32) {
         if (st.d_tok_src) launch_patch_tokens(st.d_tokens, st.d_tok_src, d_argmax, T);
         wait_for_row_copies();
         forward_f32(st, T, B, p, s, w, pool, rope, d_logits);
@@ -826,7 +826,9 @@ static long enqueue_pass(int* tokens, int num_tokens, int* pos_arr, int* seq_ids
         chained = launch_decode_chain(cs);
     }
 
-    const bool thin = T <= THIN_TOKENS && !partial && !chained && QD % 16 == 0;
+    // the few-token layers leave fp32 rows only, which the classifier of few rows reads (below); a caller that wants more rows
+    // than there are tokens (indices repeat) takes the tiles for both
+    const bool thin = T <= THIN_TOKENS && B <= THIN_TOKENS && !partial && !chained;
     if (thin) forward_thin(*m, st, T, p, s, pool, rope);
     for (int l = 0; l < p->n_layers && !chained && !thin; l++) {
         const LayerPriv& lp = m->layers[l];

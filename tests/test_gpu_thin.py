@@ -1,9 +1,12 @@
 """Passes on either side of the line between the few-token projections and the tiles of 16 and more: a batch of n one-token
-rows at widths whose K ends inside a wave's ring, a vocabulary that ends inside a row block, both pool formats."""
+rows at widths whose K ends inside a wave's ring, a vocabulary that ends inside a row block, both pool formats; and passes
+whose layers and whose classifier lie on different sides of it."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
-from nvllm_amd import synth
+from nvllm_amd import capi, synth
 from tests import util
 
 pytestmark = pytest.mark.gpu
@@ -34,3 +37,51 @@ def test_few_rows(hip, oracle, tmp_path, n, kv_bytes, shape):
         np.testing.assert_array_equal(g["sampled"], o["sampled"])
         # the bars of the forward pass: exact pool rows, fp16 pool rows
         assert np.abs(g["logits"] - o["logits"]).max() < (2e-4 if kv_bytes == 4 else 2e-3)
+
+
+def batch(lib, path, kv_bytes, history, tokens, out):
+    """Logits rows (and the library's token ids) of one pass of one sequence behind `history`."""
+    w, cfg, st = capi.Weights(), capi.Config(), capi.RunState()
+    lib.load_model(C.byref(w), C.byref(cfg), path.encode())
+    lib.malloc_run_state(C.byref(st), C.byref(cfg))
+    if lib.kind == "hip":
+        before = lib.nvllm_get_kv_elem_bytes()
+        lib.nvllm_set_kv_elem_bytes(kv_bytes)
+    mgr = capi.KVCacheManager.in_dll(lib.dll, "g_kv_manager")
+    lib.init_kv_cache_manager(C.byref(mgr), 16, 4, cfg.n_layers, cfg.n_kv_heads, cfg.head_dim)
+    arr = (C.c_int * 4)(*[lib.alloc_block(C.byref(mgr)) for _ in range(4)])
+    table = capi.BlockTable(C.cast(arr, capi.c_int_p), 4)
+    tables = (C.POINTER(capi.BlockTable) * 1)(C.pointer(table))
+    for part, at, rows in ((history, 0, [0]), (tokens, len(history), out)):
+        n = len(part)
+        lib.transformer_batch(capi.ints(part), n, capi.ints(range(at, at + n)), capi.ints([0] * n), capi.ints(rows), len(rows), C.byref(cfg), C.byref(st),
+                              C.byref(w), tables)
+    V = cfg.vocab_size
+    logits = np.ctypeslib.as_array(C.cast(st.logits, capi.c_float_p), shape=(len(out), V)).copy()
+    ids = None
+    if lib.kind == "hip":
+        n = C.c_int()
+        ids = list(lib.nvllm_last_argmax(C.byref(n))[:len(out)])
+        assert n.value == len(out)
+        lib.nvllm_set_kv_elem_bytes(before)
+    lib.free_kv_cache_manager(C.byref(mgr))
+    lib.free_run_state(C.byref(st))
+    if lib.kind == "hip":
+        lib.nvllm_free_model(C.byref(w))
+    return logits, ids
+
+
+@pytest.mark.parametrize("kv_bytes", [4, 2])
+@pytest.mark.parametrize("tokens,rows", [(1, 7), (1, 17), (3, 8), (6, 7), (6, 17), (6, 6), (3, 0), (9, 5), (17, 1), (20, 6)])
+def test_output_rows_that_repeat(hip, oracle, tmp_models, tokens, rows, kv_bytes):
+    """Few tokens and more output rows than that (eight samples of a prompt's last token), many tokens and a few rows of them
+    out of order, and nobody's row."""
+    path, shape = tmp_models("tiny")
+    rng = np.random.default_rng(100 * tokens + rows)
+    out = [int(i) for i in rng.integers(0, tokens, rows)]
+    ids = rng.integers(3, shape.vocab_size, 11 + tokens).tolist()
+    want, _ = batch(oracle, path, 4, ids[:11], ids[11:], out)
+    got, picked = batch(hip, path, kv_bytes, ids[:11], ids[11:], out)
+    assert picked == want.argmax(1).tolist() if rows else picked == []
+    if rows:
+        assert np.abs(got - want).max() < (2e-4 if kv_bytes == 4 else 2e-3)   # the bars of the forward pass
