@@ -2,7 +2,7 @@
 // fp16 weights in tile order for a few tokens.
 #pragma once
 
-#include "nvllm_internal.h"
+#include "moe.h"
 
 namespace nvllm {
 
@@ -42,6 +42,7 @@ struct F32Gemm {
     const int* block_expert = nullptr;
     long expert_stride = 0;
     const float* row_weight = nullptr;
+    int live, touched = 1;   // for the figures of a profile: rows that are some token's, matrices they can be of
     // fp16 weights, one STORE segment: (maximum, its first index) of each 16 outputs of a token -> [block][amax_ld]
     float2* amax_pairs = nullptr;
     int amax_ld = 0;
@@ -54,7 +55,7 @@ struct F32Gemm {
     int hd = 0, KD = 0, kv_elem_bytes = 4, bs = 16;
     long layer_off = 0;
 
-    F32Gemm(const float* in_, int T_, int K_) : in(in_), K(K_), T(T_) {}
+    F32Gemm(const float* in_, int T_, int K_) : in(in_), K(K_), T(T_), live(T_) {}
     F32Gemm& norm(const float* g, float e) {
         gain = g;
         eps = e;
@@ -72,10 +73,12 @@ struct F32Gemm {
         seg[n_segs++] = F32Segment{gate, up, bias_gate, bias_up, 0, N, F32Out::STORE, out, N, 0, false};
         return *this;
     }
-    F32Gemm& experts(const int* blocks, long stride, const float* weight) {
-        block_expert = blocks;
+    F32Gemm& experts(const RoutePlan& r, long stride, const float* weight) {
+        block_expert = r.block_expert;
         expert_stride = stride;
         row_weight = weight;
+        live = r.T * r.top;
+        touched = r.E < live ? r.E : live;
         return *this;
     }
 };

@@ -350,7 +350,7 @@ void launch_gemm_f32(const F32Gemm& g, int prof_cls) {
         a.seg[s].first = tiles;
         tiles += cdiv(cdiv(a.seg[s].N, 16), NB);
     }
-    ProfScope ps(prof_cls, 4.0 * (weights + (double)a.T * (a.K + outs)), 2.0 * a.T * weights);
+    ProfScope ps(prof_cls, 4.0 * (weights * a.touched + (double)a.live * (a.K + outs)), 2.0 * a.live * weights);
     if (!rows16) {
         const dim3 grid(tiles, std::min(cdiv(a.T, 4), 32768));
         if (pair) NVLLM_LAUNCH(k_gemm_f32_any<true>, grid, dim3(256), 0, a);

@@ -691,10 +691,10 @@ void HybridModel::forward_f32(const PassArgs& a, const StepArrays& st) {
         const RoutePlan plan = route_plan(route_mem, T, f.experts, f.top, 16);
         launch_route(plan, z, ldz);
         const long expert = (long)f.expert_ff * D_;
-        F32Gemm up = F32Gemm(x, plan.capacity, D_).norm(w.norm[1], eps_).experts(plan.block_expert, expert, plan.weight);
+        F32Gemm up = F32Gemm(x, plan.capacity, D_).norm(w.norm[1], eps_).experts(plan, expert, plan.weight);
         up.in_rows = plan.source;
         launch_gemm_f32(up.add_pair(w.gate32, w.up32, f.expert_ff, b), PC_GEMM_EXPERT_UP);
-        launch_gemm_f32(F32Gemm(b, plan.capacity, f.expert_ff).experts(plan.block_expert, expert, nullptr).add(w.down32, D_, d), PC_GEMM_EXPERT_DOWN);
+        launch_gemm_f32(F32Gemm(b, plan.capacity, f.expert_ff).experts(plan, expert, nullptr).add(w.down32, D_, d), PC_GEMM_EXPERT_DOWN);
         if (f.shared_ff) {
             launch_gemm_f32(normed(1).add_pair(w.shared_gate32, w.shared_up32, f.shared_ff, b), PC_GEMM_SHARED_UP);
             launch_gemm_f32(F32Gemm(b, T, f.shared_ff).add(w.shared_down32, D_, c), PC_GEMM_SHARED_DOWN);

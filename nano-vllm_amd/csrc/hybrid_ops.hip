@@ -172,10 +172,10 @@ void nvllm_expert_ff(float* out, int* choice, float* score, const float* in, con
     if (!out) return;
     if (elem_bytes == 4) {
         const Temp g((size_t)plan.capacity * ff * 4), y((size_t)plan.capacity * dim * 4);
-        F32Gemm pair = F32Gemm(in, plan.capacity, dim).experts(plan.block_expert, (long)ff * dim, plan.weight);
+        F32Gemm pair = F32Gemm(in, plan.capacity, dim).experts(plan, (long)ff * dim, plan.weight);
         pair.in_rows = plan.source;
         launch_gemm_f32(pair.add_pair(gate, up, ff, g.f()), PC_GEMM_EXPERT_UP);
-        launch_gemm_f32(F32Gemm(g.f(), plan.capacity, ff).experts(plan.block_expert, (long)dim * ff, nullptr).add(down, dim, y.f()), PC_GEMM_EXPERT_DOWN);
+        launch_gemm_f32(F32Gemm(g.f(), plan.capacity, ff).experts(plan, (long)dim * ff, nullptr).add(down, dim, y.f()), PC_GEMM_EXPERT_DOWN);
         HIP_CHECK(hipMemsetAsync(out, 0, (size_t)num_tokens * dim * 4, rt().stream));
         MoeCombine c{};
         c.x = out; c.rows = y.f(); c.row_of = plan.row_of; c.top = top; c.ld = dim;
