@@ -211,9 +211,16 @@ static PassSlot& next_slot(int B) {
     return slot;
 }
 
+// Whether the kernel that picks a pass's token ids also stores them into its page-locked array (NVLLM_ARGMAX_DIRECT=0: a copy
+// operation brings them, which costs the stream 10 us between two passes).
+static bool argmax_direct() {
+    static const bool on = !getenv("NVLLM_ARGMAX_DIRECT") || atoi(getenv("NVLLM_ARGMAX_DIRECT"));
+    return on;
+}
+
 // `host_written`: the pass's last kernel has stored the indices into next_slot(B).host itself.  `waits`: the caller waits for
-// the pass before it sends another, so its rows follow its kernels on the same stream: the switch to the copies' stream and
-// the event between them cost a pass 10 us.
+// the pass before it sends another, so its rows follow its kernels on the same stream, without the switch to the copies'
+// stream and the event between them.
 static long finish_pass(RunState* s, float* d_logits, int* d_argmax, int B, int V, PassView view, bool waits, bool chained = false,
                         bool host_written = false) {
     PassSlot& slot = next_slot(B);
@@ -747,7 +754,7 @@ static long enqueue_pass(int* tokens, int num_tokens, int* pos_arr, int* seq_ids
     if (T > p->max_seq_len || B > p->max_seq_len) NVLLM_FATAL("batch of %d tokens exceeds the workspace (%d)", T, p->max_seq_len);
     if (m->dir) {
         if (tp().active) NVLLM_FATAL("model folders are not split over tensor-parallel ranks");
-        const bool to_host = B > 0;   // the arg-max kernel stores into the pass's page-locked array too
+        const bool to_host = B > 0 && argmax_direct();
         PassArgs a{tokens, pos_arr, seq_ids, output_indices, token_src, T, B, block_tables, &g_kv_manager,
                    (float*)ws_get(WS_LOGITS, (size_t)B * p->vocab_size * sizeof(float)),
                    (int*)ws_get(WS_ARGMAX, (size_t)(p->max_seq_len + 64) * sizeof(int)), to_host ? next_slot(B).host : nullptr};
@@ -786,8 +793,8 @@ static long enqueue_pass(int* tokens, int num_tokens, int* pos_arr, int* seq_ids
         if (st.d_tok_src) launch_patch_tokens(st.d_tokens, st.d_tok_src, d_argmax, T);
         wait_for_row_copies();
         forward_f32(st, T, B, p, s, w, pool, rope, d_logits);
-        if (B > 0) launch_argmax_ld(d_argmax, d_logits, B, V, V, next_slot(B).host);
-        return finish_pass(s, d_logits, d_argmax, B, V, PassView{}, waits, false, true);
+        if (B > 0) launch_argmax_ld(d_argmax, d_logits, B, V, V, argmax_direct() ? next_slot(B).host : nullptr);
+        return finish_pass(s, d_logits, d_argmax, B, V, PassView{}, waits, false, argmax_direct());
     }
 
     // One launch for all layers (chain.hip) when the step fits it: a decode-sized batch on an fp16 page pool,
@@ -920,9 +927,7 @@ static long enqueue_pass(int* tokens, int num_tokens, int* pos_arr, int* seq_ids
         // the classifier's tiles also report their (maximum, index) pairs: the greedy token comes from
         // a merge of those instead of a second pass over the logits
         e5.amax_out = d_argmax;
-        // the kernel that picks the token ids also stores them into the pass's page-locked array
-        static const int direct_env = getenv("NVLLM_ARGMAX_DIRECT") ? atoi(getenv("NVLLM_ARGMAX_DIRECT")) : 1;
-        host_written = direct_env && !chained;
+        host_written = argmax_direct() && !chained;
         if (host_written) e5.amax_out_host = next_slot(B).host;
         e5.amax_ld = (B + 63) & ~63;
         e5.amax_pairs = (float2*)ws_get(WS_AMAX_PAIRS, (size_t)cdiv(V, 16) * e5.amax_ld * sizeof(float2));
