@@ -35,3 +35,23 @@ def test_rows_beyond_the_sixteen_byte_grid_of_a_caller(hip):
         hip.free(p)
     x64, w64 = x.astype(np.float64), w.astype(np.float64)
     assert (np.abs(got - x64 @ w64.T) <= (K + 2) * 2.0 ** -24 * (np.abs(x64) @ np.abs(w64).T)).all()
+
+
+@pytest.mark.parametrize("T,K,N", [(3, 288, 768), (2, 512, 16500), (20, 512, 512), (40, 288, 3000), (300, 512, 768), (300, 288, 3000), (16, 1376, 512)])
+def test_no_further_from_64_bits_than_64_chains(hip, T, K, N):
+    """One block and several, K in eight and in four slices: the error of sums in 64 chains that meet in a tree, or near it."""
+    rng = np.random.default_rng(T + K)
+    x, w = rng.standard_normal((T, K)).astype(np.float32), (rng.standard_normal((N, K)) * K ** -0.5).astype(np.float32)
+    got = util.op_matmul(hip, x, w)
+    at = rng.integers(0, T, 16384), rng.integers(0, N, 16384)
+    a, b = x[at[0]].astype(np.float64), w[at[1]].astype(np.float64)
+    want = (a * b).sum(1)
+    chains = np.zeros((16384, 64), np.float32)
+    for k in range(0, K, 64):   # (a product of two fp32 numbers is exact in 64 bits)
+        n = min(64, K - k)
+        chains[:, :n] = a[:, k:k + n] * b[:, k:k + n] + chains[:, :n]
+    while chains.shape[1] > 1:
+        half = chains.shape[1] // 2
+        chains = chains[:, :half] + chains[:, half:]
+    # roundings counted: chains of eight with sums over each step come to 1.06 of it at K = 288, less above; chains of 16 to 1.17 at 512
+    assert np.linalg.norm(got[at] - want) < 1.1 * np.linalg.norm(chains[:, 0] - want)
