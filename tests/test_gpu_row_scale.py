@@ -56,7 +56,8 @@ def logits(lib, path, tokens):
     out = np.ctypeslib.as_array(C.cast(st.logits, capi.c_float_p), shape=(tokens, tokens)).copy()
     lib.free_kv_cache_manager(C.byref(mgr))
     lib.free_run_state(C.byref(st))
-    lib.nvllm_free_model(C.byref(w))
+    if lib.kind == "hip":
+        lib.nvllm_free_model(C.byref(w))
     return out
 
 

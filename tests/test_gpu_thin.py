@@ -32,7 +32,7 @@ def test_few_rows(hip, oracle, tmp_path, n, kv_bytes, shape):
     finally:
         hip.nvllm_set_kv_elem_bytes(before)
     np.testing.assert_array_equal(got["trace"], want["trace"])
-    assert min(len(st["tokens"]) for st in got["steps"]) <= 8
+    assert n in {len(st["tokens"]) for st in got["steps"]}   # a pass of just that many tokens
     for g, o in zip(got["steps"], want["steps"]):
         np.testing.assert_array_equal(g["sampled"], o["sampled"])
         # the bars of the forward pass: exact pool rows, fp16 pool rows

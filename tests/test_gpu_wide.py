@@ -1,6 +1,7 @@
 """The 256-feature tiles (csrc/gemm_wide.h) at every height, on widths and token counts that end inside a tile, and K that
 ends inside a turn of the ring: one projection at a time against the oracle, and whole passes with every epilogue.  The
-height is read from the environment once per process, hence a child process per height.  In bf16 too."""
+height is read from the environment once per process, hence a child process per height.  In bf16 too, and by the launchers'
+own rules."""
 import os
 import subprocess
 import sys
@@ -9,7 +10,7 @@ import numpy as np
 import pytest
 
 from nvllm_amd import synth
-from tests import dense_tile_child, hybrid_oracle, hybrid_util, util
+from tests import dense_tile_child, hybrid_oracle, hybrid_util, latent_oracle, latent_util, test_gpu_row_scale, util
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 TOKENS = (256, 300, 433)
@@ -114,3 +115,52 @@ def test_bf16_passes(bf16_passes, tmp_path, height):
     got = np.load(dst)
     for q, o in want.items():
         assert hybrid_util.error(got[str(q)], o) < hybrid_util.limit(False), q   # the bar of the design's whole passes
+
+
+RULE_CHILD = """
+import sys
+import numpy as np
+from nvllm_amd import capi
+from tests import hybrid_util, test_gpu_row_scale, test_gpu_wide
+lib = capi.load_hip()
+if sys.argv[3] == "f16":
+    lib.init_ops()
+    rows = test_gpu_row_scale.logits(lib, sys.argv[1], test_gpu_wide.RULE_TOKENS)
+else:
+    eng = hybrid_util.engine(lib, sys.argv[1], False, tokens=704)
+    rows = hybrid_util.feed_all(eng, [[(0, test_gpu_wide.RULE_TOKENS)]], {0: test_gpu_wide.rule_tokens()})[0]
+    eng.close()
+np.save(sys.argv[2], rows)
+"""
+RULE_TOKENS = 700
+
+
+def rule_tokens():
+    return np.arange(RULE_TOKENS, dtype=np.int32)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["f16", "bf16"])
+def test_the_launchers_own_rules(oracle, tmp_path, kind):
+    """Gated pairs of 2,816 x 1,024 at 700 tokens: 242 tiles of 256 x 64 for 256 CUs, K of 32 steps, which both rules take.  The
+    smaller tiles add the same products in the same order: the same bits."""
+    path = str(tmp_path / "model")
+    if kind == "f16":
+        synth.write_model(path, synth.ModelShape(dim=1024, hidden_dim=2816, n_layers=1, n_heads=16, n_kv_heads=4, vocab_size=RULE_TOKENS, max_seq_len=704), seed=4)
+        want = test_gpu_row_scale.logits(oracle, path, RULE_TOKENS)
+    else:
+        cfg = synth.latent_config(1024, RULE_TOKENS, [(synth.latent_mixer(4, 32, 16, 32, 64, 64), 2816)])
+        want = latent_oracle.forward(cfg, latent_util.model(tmp_path, "rule", cfg=cfg)[2], rule_tokens())
+        path = str(tmp_path / "rule_3")
+    got = []
+    for env in ({}, {"NVLLM_GEMM_WIDE": "0"}):
+        dst = str(tmp_path / f"got{len(got)}.npy")
+        r = subprocess.run([sys.executable, "-c", RULE_CHILD, path, dst, kind], capture_output=True, text=True, timeout=150,
+                           env=dict(os.environ, PYTHONPATH=ROOT + os.pathsep + os.environ.get("PYTHONPATH", ""), **env))
+        assert r.returncode == 0, r.stderr[-2000:]
+        got.append(np.load(dst))
+    np.testing.assert_array_equal(got[0], got[1])
+    if kind == "f16":
+        assert np.abs(got[0] - want).max() < 2e-4   # the bar of the forward pass
+    else:
+        assert hybrid_util.error(got[0], want) < hybrid_util.limit(False)
