@@ -224,8 +224,8 @@ int launch_gemm(const WeightEntry& w, const __half* tiles, int N, const __half* 
     // LDS-shared 128 x 128 tiles of gemm_prefill.hip.
     static const int pf_min_t = getenv("NVLLM_GEMM_PREFILL_T") ? atoi(getenv("NVLLM_GEMM_PREFILL_T")) : 256;
     // ... and already for a wide decode batch (about 128 rows) when the projection is wide enough that its
-    // 128 x 128 tiles occupy most of the chip without a K split (the 7B gate/up projection at batch 128:
-    // 172 tiles, 78 us against 104 us for the streaming kernel in two 64-token groups).
+    // 128 x 128 tiles occupy most of the chip without a K split (the 7B gate/up projection at batch 128: 172 tiles, 104 us
+    // for the streaming kernel in two 64-token groups, 69 in the eight-wave tiles, 67 in those of gemm_wide.h).
     // A projection half that wide (7B q/k/v: 96 tiles) takes it with K cut in two: 192 workgroups, and
     // the tile's second half arrives through a 64 KiB slab (70 -> about 45 us).
     const int tiles128 = cdiv(a.NB, 8);

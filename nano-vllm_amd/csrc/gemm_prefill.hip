@@ -56,8 +56,8 @@ void launch_gemm_prefill(GemmArgs a) {
     // against 1,496 = 1.95 rounds of 3/4 the height, 150 -> 147 us; a projection half as wide
     // 88 -> 74 us).  Projections whose 128-token tiles would not even give every CU one
     // workgroup (wo, w_down: 208) take 64-token tiles, two workgroups per CU with three buffers
-    // (35 -> 32 and 80 -> 77 us against the eight-wave form, which wide decode batches keep:
-    // there every weight tile must still be read only once).
+    // (35 -> 32 and 80 -> 77 us against the eight-wave form, which wide decode batches keep where gemm_wide.h's
+    // tiles do not fill the chip: there every weight tile must still be read only once).
     const int tiles4 = tiles_n * cdiv(a.Tb, 8);
     const bool wide_decode = a.Tb <= 8 || want_split > 1;
     int shape = wide_decode && tiles4 * want_split <= cus ? 2 : 3;

@@ -391,7 +391,7 @@ __device__ __forceinline__ void tile_rinv(const GemmArgs& p, int tb0, float* s_r
 }
 
 template <int FW, int KG, int EPI, typename KVT, int WR = 2, int TW = 4, typename OP = OpF16x2, bool GRP = false, bool EXP = false>
-__global__ __launch_bounds__(128 * WR * KG, WR == 4 ? 4 : 2) void k_gemm_prefill(GemmArgs p, int tiles_n, int tiles_t, int nbuf, int split_from) {
+__global__ __launch_bounds__(128 * WR * KG, 2) void k_gemm_prefill(GemmArgs p, int tiles_n, int tiles_t, int nbuf, int split_from) {
     constexpr int PL = OP::PLANES;
     using G = PfGeom<FW, KG, WR, TW, PL>;
 #ifdef NVLLM_PF_ABLATE

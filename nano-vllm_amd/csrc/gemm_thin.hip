@@ -10,7 +10,8 @@
 // TinyLlama shape, one token, us per launch, 64-row tiles of gemm.hip (K cut over workgroups) and here: wo and w_down
 // together 18.2 and 15.5, gate/up 13.2 and 13.9, q/k/v 8.6 and 7.2; the pass 1,217 and 1,168.  The activations, read by every
 // workgroup, weigh more with every token: a pass of 4 tokens 1,134 and 1,104, of 6 1,136 and 1,126, of 7 1,137 and 1,142, of
-// 8 1,145 and 1,164.  So up to 6.
+// 8 1,145 and 1,164.  So up to 6; passes of 6 and (tiles) 7 tokens at other widths: stories42M 303 and 352, four layers of
+// Llama-2-7B 522 and 551.
 // Eight rows to a workgroup instead of 16 (256 of them for wo and w_down) and six tiles in flight measured the same or
 // slower: it is the start of a launch, two dependent trips to memory, that is left.
 #include "gemm_f32_tail.h"

@@ -6,7 +6,8 @@
 //     (16 + PL TBN) KiB into the CU and 4 (4 + PL TBN) KiB out of LDS per 64 PL TBN matrix-core cycles
 // (PL activation planes), e.g. fp16 hi + lo at 96 tokens 28 KiB and 64 KiB per 768 cycles, where the tiles of 128 x 96 in
 // gemm_prefill_tile.h (2 x 2 waves) take 40 and 112 for the same products.  One wave per SIMD then has the register file to
-// itself: accumulators for up to nine token blocks, and operands that are replaced as they are used, so that the LDS reads
+// itself: accumulators for up to nine token blocks with hi + lo planes of
+// activations (ten with one bf16 plane), and operands that are replaced as they are used, so that the LDS reads
 // of step s + 1 and the copies of step s + RING - 1 are issued between the products of step s.  Copies go global -> LDS
 // directly (one 1-KiB tile per wave instruction, both operands are stored in operand order) through a ring of RING stages
 // with counted waits; one barrier a step publishes step s + 1 and frees the buffer of step s - 1, whose operands are in

@@ -32,7 +32,9 @@ bool launch_gemm_wide_f16(const GemmArgs& a) {
     // One workgroup per CU has nothing to run beside it, so where the tiles leave a third of the CUs empty the smaller ones of
     // gemm_prefill.hip win.  TinyLlama-1.1B, those against these: gate/up at 256 tokens (176 tiles) 43 -> 35 us, at 520 (176)
     // 74 -> 60, at 1,200 (396 of 512) 136 -> 119, at 3,000 310 -> 265; q/k/v at 1,200 tokens (190 tiles) 47 -> 43, but at 640
-    // (100) 34 -> 39; w_down at 2,048 (256) 114 -> 97, at 1,380 (176) 87 -> 86, at 1,000 (128) 73 -> 81.
+    // (100) 34 -> 39; w_down at 2,048 (256) 114 -> 97, at 1,380 (176) 87 -> 86, at 1,000 (128) 73 -> 81.  Decode batches of
+    // Llama-2-7B, against the eight-wave tiles: gate/up (172 tiles) at 112, 120 and 128 rows 67.1, 68.3, 68.8 -> 64.5, 66.4, 67.1,
+    // the classifier (250) 79.4, 80.3, 83.7 -> 79.8, 81.1, 81.0.
     const int tiles_t = cdiv(a.Tb, best), tiles = tiles_n * tiles_t;
     if (wide_env() < 0 && 100 * tiles < 65 * cus * cdiv(tiles, cus)) return false;
     const bool kv16 = a.e.kind == GemmEpilogue::ROPE_KV && a.e.kv_elem_bytes == 2;
