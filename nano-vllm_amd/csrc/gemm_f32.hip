@@ -77,11 +77,11 @@ __global__ __launch_bounds__(KS * 64, f32_occupancy((PAIR ? 2 : 1) * NB * TB, NO
         }
         __builtin_amdgcn_sched_barrier(0);
     };
-    // Short chains keep the error that of pairwise sums.  One block by eight waves keeps the eight products of a step apart, each in
-    // a chain of its own over the wave's steps: 64 chains of K / 64, no addition between products.  Larger tiles have no
+    // Short chains keep the error that of pairwise sums.  One block by eight waves keeps the eight products of a step apart, each
+    // in a chain of its own over the wave's steps: 64 chains of K / 64, no addition between products.  Larger tiles have no
     // registers for that, four waves too few chains: they sum chains of eight (two products of four k) over every step, a tile's
-    // behind the next one's first products.  Against 64 bits, K = 288 / 512 / 1,024, in units of 1e-8: 64 chains 7.8 / 8.6 / 10, chains of eight 8.2 / 8.7 / 9.5;
-    // chains of 16 were 9.9 / 10 / 10.5, chains of four 7.9 / 8.4 / 9.2 but 7 % of a pass of 301 tokens.
+    // behind the next one's first products.  Error against 64 bits in 1e-8, K = 288 / 512 / 1,024: 64 chains 7.8 / 8.6 / 10, chains
+    // of eight 8.2 / 8.7 / 9.5, of 16 9.9 / 10 / 10.5; chains of four 7.9 / 8.4 / 9.2, but a pass of 301 tokens takes 7 % longer.
     constexpr int TILES = NT * TB;
     constexpr bool APART = TILES == 1 && KS == 8;
     f4_t acc[NT][TB], chain[APART ? 1 : 2][APART ? 8 : 4];
