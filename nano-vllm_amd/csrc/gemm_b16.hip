@@ -104,7 +104,7 @@ void launch_kind(GemmArgs a, int prof_cls, double bytes, double flops) {
         {
             ProfScope ps(prof_cls, bytes, flops);
             a.e.amax_pairs = nullptr;   // the dense-tile kernel does not emit pairs: the rows are scanned afterwards
-            if (GRP || !launch_gemm_wide_b16(a)) launch_dense<EPI, GRP>(a);   // (its own rule is there)
+            if (GRP || !(launch_gemm_waves_b16(a) || launch_gemm_wide_b16(a))) launch_dense<EPI, GRP>(a);   // (their own rules are there)
         }
         if (EPI == GemmEpilogue::F32 && a.e.amax_out) launch_argmax_ld(a.e.amax_out, a.e.out, a.T, a.N, a.e.ldo, a.e.amax_out_host);
         return;

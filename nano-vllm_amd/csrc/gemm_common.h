@@ -299,5 +299,8 @@ void launch_gemm_prefill(GemmArgs a);
 // gemm_wide_f16.hip: the same in tiles of 256 features; false: not for this launch
 bool launch_gemm_wide_f16(const GemmArgs& a);
 bool launch_gemm_wide_b16(const GemmArgs& a);   // gemm_wide_b16.hip: bf16 models
+// gemm_waves_f16.hip, gemm_waves_b16.hip: one round of tiles with K dealt to the waves; false: not for this launch
+bool launch_gemm_waves_f16(const GemmArgs& a);
+bool launch_gemm_waves_b16(const GemmArgs& a);
 
 }  // namespace nvllm

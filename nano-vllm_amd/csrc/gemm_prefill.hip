@@ -47,7 +47,7 @@ void launch_gemm_prefill(GemmArgs a) {
     const bool kv16 = a.e.kind == GemmEpilogue::ROPE_KV && a.e.kv_elem_bytes == 2;
     int want_split = a.ksplit > 1 ? a.ksplit : 1;
     if (ksplit_env > 1) want_split = ksplit_env;
-    if (want_split == 1 && !shape_env && !tw_env && launch_gemm_wide_f16(a)) return;   // (its own rule is there)
+    if (want_split == 1 && !shape_env && !tw_env && (launch_gemm_waves_f16(a) || launch_gemm_wide_f16(a))) return;   // (their own rules are there)
     const int tiles_n = cdiv(a.NB, 8);
     // 128-feature tiles, 128, 96 or 64 tokens high.  A launch runs in rounds of co-resident
     // workgroups (three per CU with two ring buffers) and a partly filled last round costs

@@ -683,6 +683,11 @@ __global__ __launch_bounds__(128 * WR * KG, 2) void k_gemm_prefill(GemmArgs p, i
     }
 }
 
+inline int wide_env() {   // NVLLM_GEMM_WIDE: 0 = never the tiles of gemm_wide.h, a number of token blocks = always that height
+    static const int v = getenv("NVLLM_GEMM_WIDE") ? atoi(getenv("NVLLM_GEMM_WIDE")) : -1;
+    return v;
+}
+
 }  // namespace
 
 }  // namespace nvllm

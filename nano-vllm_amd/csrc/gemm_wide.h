@@ -186,10 +186,6 @@ void launch_wide(const GemmArgs& a, int tiles_n, int tiles_t) {
     NVLLM_LAUNCH((k_gemm_wide<TBN, EPI, KVT, OP>), dim3(tiles_n * tiles_t), dim3(256), G::LDS, a, tiles_n, tiles_t);
 }
 
-inline int wide_env() {   // NVLLM_GEMM_WIDE: 0 = never these tiles, a number of token blocks = always that height
-    static const int v = getenv("NVLLM_GEMM_WIDE") ? atoi(getenv("NVLLM_GEMM_WIDE")) : -1;
-    return v;
-}
 // Microseconds a launch takes in tiles of TBN token blocks: rounds of one workgroup per CU, each a start and an end beside its
 // Kb steps.  Fitted to fp16 launches of 64 and 176 steps on a full chip (a round of 4, 6 and 9 blocks: 36, 45 and 60 us; 92,
 // 120 and 140 us).
