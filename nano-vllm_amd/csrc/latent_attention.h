@@ -47,7 +47,8 @@ struct LatentAttn {
     __half* out_b16;       // bf16 pool: activation tiles of [T, H * rank_ld]
 };
 constexpr int LATENT_RUN = 32;   // stage_step(attn_ct, multi_first): tokens per run at most
-void launch_latent_attention(const LatentAttn& a, const StepArrays& st);
+// only_alone: nothing but the tokens that are their sequence's only one
+void launch_latent_attention(const LatentAttn& a, const StepArrays& st, bool only_alone = false);
 
 // fp32 models: q [T][H * (dim + rot)] -> rows [T][H][rank + rot] (W_uk [H * dim, rank] absorbed, rotated part turned)
 void launch_latent_q_f32(float* rows, const float* q, const float* uk, const float2* rope, const int* pos, int T, int H, int dim, int rot, int rank);

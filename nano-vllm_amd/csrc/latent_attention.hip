@@ -572,7 +572,7 @@ static void launch_latent_rc(const LatentKArgs& k, long units, int columns) {
     else launch_latent_c<RC, NT, 2, 2, (RC > 10)>(k, units);
 }
 
-void launch_latent_attention(const LatentAttn& a, const StepArrays& st) {
+void launch_latent_attention(const LatentAttn& a, const StepArrays& st, bool only_alone) {
     if (st.T <= 0) return;
     const LatentPool& P = a.pool;
     const int row = P.row(), chunks = row / 32, vt = cdiv(P.rank_ld, 64);   // value tiles per wave
@@ -583,7 +583,7 @@ void launch_latent_attention(const LatentAttn& a, const StepArrays& st) {
     const bool tiled = P.elem_bytes == 2 && ((chunks <= 4 && vt <= 1) || (chunks <= 6 && vt <= 2) || (chunks <= 10 && vt <= 4) || (chunks <= 18 && vt <= 8));
     int pages_per_block = P.block_size / LATENT_PAGE, page_shift = 0;
     while ((1 << page_shift) < pages_per_block) page_shift++;
-    if (!tiled || (1 << page_shift) != pages_per_block) {
+    if (!tiled || (1 << page_shift) != pages_per_block) {   // (all tokens, whoever was asked for)
         const size_t lds = ((size_t)row + P.rank_ld + 256 + 8) * sizeof(float);
         if (lds > 64 * 1024) NVLLM_FATAL("latent attention: a cached row of %d values is not supported", row);
         ProfScope ps(PC_LATENT_ATTN, bytes, flops);
@@ -650,6 +650,11 @@ void launch_latent_attention(const LatentAttn& a, const StepArrays& st) {
                          P.rank_ld, a.out_b16, k.Kb_out);
         }
     };
+    if (only_alone) {
+        launch(st.d_runs + 4 * (st.n_runs - st.n_alone), st.n_alone, 1, bytes_of((double)st.kv_rows_alone, st.n_alone),
+               2.0 * (double)st.kv_rows_alone * a.H * (row + P.rank_ld));
+        return;
+    }
     const double single_bytes = bytes_of((double)st.kv_rows_single, n_single);
     const double single_flops = 2.0 * (double)st.kv_rows_single * a.H * (row + P.rank_ld);
     launch(st.d_runs, st.n_multi, st.max_run, bytes - single_bytes, flops - single_flops);

@@ -23,6 +23,7 @@
 #include "gemm_common.h"
 #include "gemm_f32.h"
 #include "latent_attention.h"
+#include "latent_prompt.h"
 #include "model_dir.h"
 
 namespace nvllm {
@@ -40,6 +41,7 @@ struct LayerWeightsDir {
     int ff = 0;   // 0: the layer has no feed-forward
     // bf16
     B16Weight in, uq, uk, uv, o, gateup, down;
+    B16Weight uk_rows;   // W_uk as it is, [H * dim, rank]: keys of prompt portions (uk: for queries, head by head transposed)
     // fp32 (row-major, unpadded)
     float *dq = nullptr, *dkv = nullptr, *uq32 = nullptr, *uk32 = nullptr, *uv32 = nullptr, *o32 = nullptr, *gate = nullptr, *up = nullptr, *down32 = nullptr;
     // both: fp32 vectors, zero-padded in the bf16 form
@@ -76,7 +78,7 @@ private:
     LatentPool pool(const KVCacheManager* mgr, int run) const;
     size_t pool_bytes(int block_size, int num_blocks, int runs) const;   // of the first `runs` cache slices
     void load_layer(const ModelDir& dir, int i, const Json& cfg);
-    void forward_b16(const PassArgs& a, const StepArrays& st);
+    void forward_b16(const PassArgs& a, const StepArrays& st, const LatentPromptPlan& plan);
     void forward_f32(const PassArgs& a, const StepArrays& st);
 };
 
@@ -179,6 +181,9 @@ void LatentHyperModel::load_layer(const ModelDir& dir, int i, const Json& cfg) {
             for (int c = 0; c < m.rank; c++) o[(size_t)c * m.dim] = s[c];
         }
     w.uk = tile(dst, H * Cp, m.dim, H);
+    dst.assign((size_t)H * dimp * m.rank, 0);
+    for (int h = 0; h < H; h++) rows_to(h * dimp, h * m.dim, m.dim, m.rank);
+    w.uk_rows = tile(dst, H * dimp, m.rank);
     // W_uv head by head: [vdim, rank] per head
     read(M + "uv", H * m.vdim, m.rank);
     dst.assign((size_t)H * vp * m.rank, 0);
@@ -330,13 +335,15 @@ void LatentHyperModel::forward(const PassArgs& a) {
         NVLLM_FATAL("transformer_batch: the block pool was not made for this model (nvllm_init_model_kv)");
     for (int t = 0; t < a.T; t++)
         if (a.pos[t] < 0 || a.tokens[t] < 0 || a.tokens[t] >= V_) NVLLM_FATAL("transformer_batch: token %d (id %d, position %d) is out of range", t, a.tokens[t], a.pos[t]);
-    const StepArrays st = stage_step(a.tokens, a.pos, a.seq_ids, a.T, a.output_indices, a.B, a.tables, nullptr, 0, a.mgr->block_size, LATENT_RUN, a.token_src, true);
+    const LatentPromptPlan plan = f32_ ? LatentPromptPlan() : latent_prompt_plan(a.pos, a.seq_ids, a.T, a.tables, a.mgr->block_size);
+    const StepArrays st = stage_step(a.tokens, a.pos, a.seq_ids, a.T, a.output_indices, a.B, a.tables, nullptr, 0, a.mgr->block_size, LATENT_RUN, a.token_src, true,
+                                     false, 0, &plan.ints);
     if (st.table_short) NVLLM_FATAL("transformer_batch: a position lies beyond its sequence's block table (allocate the block first)");
     if (f32_) forward_f32(a, st);
-    else forward_b16(a, st);
+    else forward_b16(a, st, plan);
 }
 
-void LatentHyperModel::forward_b16(const PassArgs& a, const StepArrays& st) {
+void LatentHyperModel::forward_b16(const PassArgs& a, const StepArrays& st, const LatentPromptPlan& plan) {
     const int T = a.T, B = a.B;
     // workspaces of the widest layer
     int raw_ld = 0, q_row = 0, q_plain = 0, lat = 0, val = 0, ffp = 0, qlat = 0;
@@ -401,7 +408,7 @@ void LatentHyperModel::forward_b16(const PassArgs& a, const StepArrays& st) {
             continue;
         }
         const float2* rope = rotation_table(m.base, m.rot, st.max_pos + 1);
-        const int Qp = pad32(m.q_rank), Cp = pad32(m.rank), Rp = pad32(m.rot), dimp = pad32(m.dim);
+        const int Qp = pad32(m.q_rank), Cp = pad32(m.rank), Rp = pad32(m.rot), dimp = pad32(m.dim), vp = pad32(m.vdim);
         GemmEpilogue e1;
         e1.kind = GemmEpilogue::LATENT_IN;
         e1.latent_q = Qp; e1.gain_next = w.gain_q; e1.a16_out = qt; e1.ss_out = ss;
@@ -415,18 +422,35 @@ void LatentHyperModel::forward_b16(const PassArgs& a, const StepArrays& st) {
         e2.q_plain = m.heads * dimp; e2.rot_ld = Rp; e2.rot_dim = m.rot; e2.rope = rope; e2.pos = st.d_pos;
         e2.a16_out = hid; e2.q_rows = q; e2.q_heads = m.heads; e2.q_row = Cp + Rp; e2.head_ld = Cp;
         launch_gemm_b16(w.uq, qt, T, e2, PC_GEMM_LATENT_Q, &ride);
-        GemmEpilogue e3;
-        e3.kind = GemmEpilogue::ROWS_B16;
-        e3.q_rows = q; e3.q_heads = m.heads; e3.q_row = Cp + Rp; e3.head_ld = Cp;
-        launch_gemm_b16(w.uk, hid, T, e3, PC_GEMM_ABSORB);
-        LatentAttn at{};
-        at.pool = pl; at.q = q; at.sink = w.sink; at.scale = m.scale; at.H = m.heads; at.out_b16 = latents;
-        launch_latent_attention(at, st);
-        GemmEpilogue e4;
-        e4.kind = GemmEpilogue::TILE_B16;
-        e4.a16_out = hid;
-        launch_gemm_b16(w.uv, latents, T, e4, PC_GEMM_VALUE);
-        residual(w.o, hid, s, nullptr, PC_GEMM_WO);
+        // attention over the latents, of tokens [t0, t0 + n) (whole 16-token blocks): W_uk into the queries, W_uv behind
+        auto over_latents = [&](int t0, int n, __half* out, bool only_alone) {
+            GemmEpilogue e3;
+            e3.kind = GemmEpilogue::ROWS_B16;
+            e3.q_rows = q + (size_t)t0 * m.heads * (Cp + Rp); e3.q_heads = m.heads; e3.q_row = Cp + Rp; e3.head_ld = Cp;
+            launch_gemm_b16(w.uk, hid + b16_halves(t0, m.heads * dimp), n, e3, PC_GEMM_ABSORB);
+            LatentAttn at{};
+            at.pool = pl; at.q = q; at.sink = w.sink; at.scale = m.scale; at.H = m.heads; at.out_b16 = latents;
+            launch_latent_attention(at, st, only_alone);
+            GemmEpilogue e4;
+            e4.kind = GemmEpilogue::TILE_B16;
+            e4.a16_out = out + b16_halves(t0, m.heads * vp);
+            launch_gemm_b16(w.uv, latents + b16_halves(t0, m.heads * Cp), n, e4, PC_GEMM_VALUE);
+        };
+        if (!latent_prompt_pays(plan, pl, m.heads, dimp, vp)) {
+            over_latents(0, T, hid, false);
+            residual(w.o, hid, s, nullptr, PC_GEMM_WO);
+            continue;
+        }
+        // prompt portions: keys and values formed from the latents.  Their rows are written last: the blocks of the tokens beside them
+        // may hold some of theirs.
+        __half* values = (__half*)ws_get(WS_VALUES, b16_halves(T, val) * sizeof(__half));
+        if (plan.alone_to > plan.alone_from) over_latents(16 * plan.alone_from, std::min(T, 16 * plan.alone_to) - 16 * plan.alone_from, values, true);
+        LatentPrompt pr{};
+        pr.pool = pl; pr.q_tiles = hid; pr.q_rows = (const __half*)q; pr.sink = w.sink; pr.scale = m.scale; pr.H = m.heads;
+        pr.dim_ld = dimp; pr.vdim_ld = vp; pr.uk = w.uk_rows.tiles; pr.uv = w.uv.tiles; pr.out = values;
+        pr.items = st.d_extra; pr.pages = st.d_extra + 4 * plan.n_items;
+        launch_latent_prompt(pr, plan);
+        residual(w.o, values, s, nullptr, PC_GEMM_WO);
     }
     if (B <= 0) return;
     wait_for_row_copies();

@@ -1,0 +1,39 @@
+// latent_prompt.h -- latent attention of prompt portions with keys and values of each head expanded from the cached latents.
+#pragma once
+
+#include <vector>
+
+#include "latent_attention.h"
+
+namespace nvllm {
+
+// What a pass's portions of several tokens need, made on the host: the pool pages that hold their sequences' positions up to
+// the portion's last, in pairs, and items of up to LATENT_PROMPT_TOKENS tokens, those that see most first.
+constexpr int LATENT_PROMPT_TOKENS = 64;
+struct LatentPromptPlan {
+    std::vector<int> ints;   // [n_items][4] (first token, count, position of the first, first pair), then [n_pairs][2] page ids; a multiple of four
+    int n_items = 0, n_pairs = 0;
+    int most_pairs = 0;      // of one portion
+    int tokens = 0;          // tokens of the portions
+    long pairs_qk = 0;       // (token, position) pairs
+    // the 16-token blocks that hold the tokens which are their sequence's only ones (none: from == to)
+    int alone_from = 0, alone_to = 0;
+};
+LatentPromptPlan latent_prompt_plan(const int* pos, const int* seq_ids, int T, BlockTable** tables, int block_size);
+
+struct LatentPrompt {
+    LatentPool pool;
+    const __half* q_tiles;   // unrotated queries, activation tiles of [T, H * dim_ld]
+    const __half* q_rows;    // [T][H][pool.row()]: the rotated parts at pool.rank_ld
+    const float* sink;
+    float scale;
+    int H, dim_ld, vdim_ld;
+    const __half *uk, *uv;   // tiles of [H * dim_ld, rank_ld] and [H * vdim_ld, rank_ld]
+    __half* out;             // activation tiles of [T, H * vdim_ld]
+    const int *items, *pages;   // device copies of the plan
+};
+// Whether this is the way to go for the pass's portions.
+bool latent_prompt_pays(const LatentPromptPlan& plan, const LatentPool& pool, int H, int dim_ld, int vdim_ld);
+void launch_latent_prompt(const LatentPrompt& a, const LatentPromptPlan& plan);
+
+}  // namespace nvllm

@@ -1,0 +1,409 @@
+// latent_prompt.hip -- latent attention of prompt portions (latent_prompt.h).
+//
+// A token that attends over latents as they lie multiplies rank + rot values per key and head and adds up rank of them; with
+// keys W_uk c and values W_uv c formed first it is dim + rot and vdim (64 + 64 and 64 instead of 512 + 64 and 512), and
+// the queries need no product with W_uk, the results none with W_uv.  Forming them costs rank * (dim + vdim) products per
+// position and head, shared by all tokens of the portion: it pays from about seventy tokens on.
+//
+// k_latent_expand   a wave owns 32 features of [all heads' keys; all heads' values], whose weights (32 x rank) stay in its
+//                   registers, and multiplies page after page: two pages of 16 positions travel to LDS by direct copies, one pair
+//                   ahead, for the eight waves of the workgroup.  Keys are formed as W x latent (a lane holds four dims of a position),
+//                   values as latent x W^T (four positions of a dim), which are the orders the attention's operands lie in.
+// k_latent_prompt   64 tokens x one head; the four waves have 16 tokens each and walk the keys in blocks of 64 that
+//                   travel to LDS one block ahead.  Scores, maxima and sums are fp32; the weights of two pages are the next
+//                   product's operand as they lie in the score registers.
+// Bounds: the expansion its 32 KiB per pair into and 4 KiB per wave out of a CU; attention the issue of about 110 vector
+// instructions per 64 keys and 16 tokens beside 24 products.
+#include "latent_prompt.h"
+
+#include <algorithm>
+#include <array>
+
+#include "attn_tile.h"
+#include "gemm_common.h"
+
+namespace nvllm {
+
+namespace {
+
+typedef const __attribute__((address_space(4))) int* const_int_p;   // read-only for the whole launch: scalar loads
+
+__device__ __forceinline__ void prompt_barrier() {   // this wave's LDS accesses are done, then everybody meets
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+__device__ __forceinline__ void copies_landed() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
+struct ExpandArgs {
+    const __half* base;   // the pool
+    const int* pages;     // [n_pairs][2]
+    int n_pairs, per;     // pairs, and pairs of a workgroup
+    int chunks, row_tiles;   // tiles of a page: of its latent, in all
+    int H, dc, vt;        // tiles of 32 dims of a head's key; of 16 dims of its value
+    const __half *uk, *uv;
+    __half* kv;           // [pair][head][2 dc key tiles by page, vt value tiles]
+};
+
+// KC: tiles of a latent that a wave has registers for
+template <int KC>
+__global__ __launch_bounds__(512, 2) void k_latent_expand(ExpandArgs a) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds_expand[];   // [2][2][chunks] tiles
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int x = lane & 15, g = lane >> 4;
+    const int nc = a.chunks;
+    const int unit = (int)blockIdx.x * 8 + wave, key_units = a.H * a.dc, units = key_units + a.H * (a.vt / 2);
+    const bool is_key = unit < key_units, live = unit < units;
+    const int mine = min(unit, units - 1), block = (is_key ? mine : mine - key_units) * 2;   // this wave's first row block of its matrix
+    const int pair0 = (int)blockIdx.y * a.per, pair1 = min(a.n_pairs, pair0 + a.per);
+    const const_int_p pages = (const_int_p)(uintptr_t)a.pages;
+    const unsigned lds0 = (unsigned)(size_t)(lds_void*)lds_expand;
+    auto issue = [&](int pair, int buf) {   // waves 0-3 bring the first page's tiles, 4-7 the second's
+        const int half = wave >> 2;
+        const __half* src = a.base + (size_t)pages[2 * pair + half] * a.row_tiles * TILE_HALVES + lane * 8;
+        for (int c = wave & 3; c < nc; c += 4)
+            copy_tile_to_lds(src + (size_t)c * TILE_HALVES, __builtin_amdgcn_readfirstlane(lds0 + (unsigned)((buf * 2 + half) * nc + c) * 1024u));
+    };
+    issue(pair0, 0);
+    h8_t w[2][KC];
+    {
+        const __half* W = (is_key ? a.uk : a.uv) + (size_t)block * nc * TILE_HALVES + lane * 8;
+#pragma unroll
+        for (int f = 0; f < 2; f++)
+#pragma unroll
+            for (int k = 0; k < KC; k++) w[f][k] = *reinterpret_cast<const h8_t*>(W + ((size_t)f * nc + min(k, nc - 1)) * TILE_HALVES);
+    }
+    const size_t head_halves = (size_t)(2 * a.dc + a.vt) * TILE_HALVES;
+    for (int pair = pair0; pair < pair1; pair++) {
+        const int buf = (pair - pair0) & 1;
+        copies_landed();
+        prompt_barrier();
+        if (pair + 1 < pair1) issue(pair + 1, buf ^ 1);
+        const h8_t* lat = reinterpret_cast<const h8_t*>(lds_expand) + (size_t)buf * 2 * nc * 64 + lane;
+        f4_t acc[2][2] = {};   // [row block][page]
+        if (is_key) {
+#pragma unroll
+            for (int k = 0; k < KC; k++)
+                if (k < nc) {
+#pragma unroll
+                    for (int page = 0; page < 2; page++) {
+                        const h8_t c = lat[(page * nc + k) * 64];
+#pragma unroll
+                        for (int f = 0; f < 2; f++) acc[f][page] = OpBf16::mfma(w[f][k], c, acc[f][page]);
+                    }
+                }
+            if (!live) continue;
+            const int head = mine / a.dc, c = mine - head * a.dc;
+            __half* out = a.kv + ((size_t)pair * a.H + head) * head_halves;
+#pragma unroll
+            for (int f = 0; f < 2; f++)
+#pragma unroll
+                for (int page = 0; page < 2; page++) {   // dims 16 f + 4 g .. + 3 of position x
+                    const float y[4] = {acc[f][page][0], acc[f][page][1], acc[f][page][2], acc[f][page][3]};
+                    *reinterpret_cast<b4_t*>(out + (size_t)(page * a.dc + c) * TILE_HALVES + (x + 16 * (2 * f + (g >> 1))) * 8 + 4 * (g & 1)) = to_b4(y);
+                }
+        } else {
+#pragma unroll
+            for (int k = 0; k < KC; k++)
+                if (k < nc) {
+#pragma unroll
+                    for (int page = 0; page < 2; page++) {
+                        const h8_t c = lat[(page * nc + k) * 64];
+#pragma unroll
+                        for (int f = 0; f < 2; f++) acc[f][page] = OpBf16::mfma(c, w[f][k], acc[f][page]);
+                    }
+                }
+            if (!live) continue;
+            const int head = block / a.vt, n = block - head * a.vt;
+            __half* out = a.kv + ((size_t)pair * a.H + head) * head_halves + (size_t)(2 * a.dc + n) * TILE_HALVES;
+#pragma unroll
+            for (int f = 0; f < 2; f++) {   // positions 4 g .. + 3 of both pages, dim 16 (n + f) + x
+                alignas(16) b4_t both[2];
+#pragma unroll
+                for (int page = 0; page < 2; page++) {
+                    const float y[4] = {acc[f][page][0], acc[f][page][1], acc[f][page][2], acc[f][page][3]};
+                    both[page] = to_b4(y);
+                }
+                *reinterpret_cast<u4_t*>(out + (size_t)f * TILE_HALVES + lane * 8) = *reinterpret_cast<const u4_t*>(both);
+            }
+        }
+    }
+}
+
+struct PromptArgs {
+    const __half* base;
+    const int *items, *pages;
+    const __half *q_tiles, *q_rows, *kv;
+    const float* sink;
+    float scale;
+    int H;
+    int q_kb;                 // tiles of a token block of q_tiles
+    int row, rank_ld;
+    __half* out;
+    int Kb_out;
+};
+
+// DC, RC: chunks of 32 dims of a head's key, unrotated and rotated; VT: tiles of 16 dims of its value
+template <int DC, int RC, int VT, int RING>
+__global__ __launch_bounds__(256, 2) void k_latent_prompt(PromptArgs a) {
+    constexpr int TILES = 4 * DC + 4 * RC + 2 * VT;   // of a block of 64 keys: keys by page, rotated parts by page, values by pair
+    constexpr int COPIES = DC + RC + VT / 2;          // of a wave
+    extern __shared__ __attribute__((aligned(16))) __half lds_prompt[];   // [RING][TILES] tiles
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int x = lane & 15, g = lane >> 4;
+    // heads fastest: a head's items meet behind one L2 wherever the number of heads is a multiple of the eight XCDs
+    const int h = (int)(blockIdx.x % (unsigned)a.H), item = (int)(blockIdx.x / (unsigned)a.H);
+    const const_int_p it = (const_int_p)(uintptr_t)(a.items + 4 * item), pages = (const_int_p)(uintptr_t)a.pages;
+    const int t0 = it[0], ntok = it[1], p0 = it[2], pair0 = it[3];
+    const int last = p0 + ntok - 1, n_blocks = (last >> 6) + 1, last_pair = last >> 5;
+    const int tok = 16 * wave + x, t = t0 + min(tok, ntok - 1);
+    const int sees = tok < ntok ? p0 + tok : -1;                                  // last position of this lane's column
+    const int wave_sees = 16 * wave < ntok ? min(p0 + 16 * wave + 15, last) : -1;   // ... of the wave's last column
+    constexpr size_t HEAD = (size_t)(2 * DC + VT) * TILE_HALVES;
+    const unsigned lds0 = (unsigned)(size_t)(lds_void*)lds_prompt;
+    // wave w brings page w of a block: its key tiles, its rotated part, and every second value tile of its pair
+    auto pair_of = [&](int b) { return pair0 + min(2 * b + (wave >> 1), last_pair); };   // (past the last: the last again, masked)
+    auto issue = [&](int page_id, int b, int buf) {
+        const unsigned dst = lds0 + (unsigned)(buf * TILES) * 1024u;
+        const __half* own = a.kv + ((size_t)pair_of(b) * a.H + h) * HEAD + lane * 8;
+        const __half* rot = a.base + ((size_t)page_id * 16 * a.row + (size_t)a.rank_ld * 16) + lane * 8;
+#pragma unroll
+        for (int c = 0; c < DC; c++)
+            copy_tile_to_lds(own + (size_t)((wave & 1) * DC + c) * TILE_HALVES, __builtin_amdgcn_readfirstlane(dst + (unsigned)(wave * DC + c) * 1024u));
+#pragma unroll
+        for (int c = 0; c < RC; c++)
+            copy_tile_to_lds(rot + (size_t)c * TILE_HALVES, __builtin_amdgcn_readfirstlane(dst + (unsigned)(4 * DC + wave * RC + c) * 1024u));
+#pragma unroll
+        for (int n = 0; n < VT / 2; n++)
+            copy_tile_to_lds(own + (size_t)(2 * DC + 2 * n + (wave & 1)) * TILE_HALVES,
+                             __builtin_amdgcn_readfirstlane(dst + (unsigned)(4 * DC + 4 * RC + (wave >> 1) * VT + 2 * n + (wave & 1)) * 1024u));
+    };
+    auto page_of = [&](int b) { return pages[2 * pair_of(b) + (wave & 1)]; };
+    // queries as the second operand: column x, dims 32 c + 8 g .. + 7
+    b8_t q[DC + RC];
+#pragma unroll
+    for (int c = 0; c < DC; c++)
+        q[c] = *reinterpret_cast<const b8_t*>(a.q_tiles + ((size_t)(t >> 4) * a.q_kb + h * DC + c) * TILE_HALVES + ((t & 15) + 16 * g) * 8);
+#pragma unroll
+    for (int c = 0; c < RC; c++) q[DC + c] = *reinterpret_cast<const b8_t*>(a.q_rows + ((size_t)t * a.H + h) * a.row + a.rank_ld + 32 * c + 8 * g);
+#pragma unroll
+    for (int i = 0; i < RING - 1; i++)
+        if (i < n_blocks) issue(page_of(i), i, i);
+    int next_page = page_of(RING - 1), buf = 0;
+#pragma unroll
+    for (int c = 0; c < DC + RC; c++) asm volatile("" : "+v"(q[c]));   // here, not in the loop, whose only loads are the copies
+    f4_t acc[VT];
+#pragma unroll
+    for (int n = 0; n < VT; n++) acc[n] = f4_t{0.f, 0.f, 0.f, 0.f};
+    float m = -INFINITY, lsum = 0.f;
+    const float sl2 = a.scale * 1.44269504088896340736f;   // scores in the log2 domain
+    for (int b = 0; b < n_blocks; b++) {
+        if (b + RING - 1 <= n_blocks) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((RING - 2) * COPIES) : "memory");   // all later blocks are on their way
+        else copies_landed();
+        prompt_barrier();   // everybody's copies of block b; block b - 1 has been consumed
+        const b8_t* blk = reinterpret_cast<const b8_t*>(lds_prompt) + (size_t)buf * TILES * 64 + lane;
+        if (b + RING - 1 < n_blocks) {
+            issue(next_page, b + RING - 1, buf == 0 ? RING - 1 : buf - 1);
+            next_page = page_of(b + RING);
+        }
+        buf = buf + 1 == RING ? 0 : buf + 1;
+        if (64 * b > wave_sees) continue;
+        f4_t s[4];
+#pragma unroll
+        for (int page = 0; page < 4; page++) {
+            s[page] = f4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int c = 0; c < DC; c++) s[page] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(blk[(page * DC + c) * 64], q[c], s[page], 0, 0, 0);
+#pragma unroll
+            for (int c = 0; c < RC; c++) s[page] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(blk[(4 * DC + page * RC + c) * 64], q[DC + c], s[page], 0, 0, 0);
+        }
+        // lane (column x): keys 64 b + 16 page + 4 g + r
+        if (64 * b + 63 > p0 + 16 * wave || 16 * wave + 15 >= ntok) {   // some column does not see all of them
+            const int from = 64 * b + 4 * g;
+#pragma unroll
+            for (int page = 0; page < 4; page++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) s[page][r] = from + 16 * page + r <= sees ? s[page][r] * sl2 : -INFINITY;
+        } else {
+#pragma unroll
+            for (int page = 0; page < 4; page++) s[page] *= sl2;
+        }
+        float mx = -INFINITY;
+#pragma unroll
+        for (int page = 0; page < 4; page++) mx = fmaxf(mx, fmaxf(fmaxf(s[page][0], s[page][1]), fmaxf(s[page][2], s[page][3])));
+        mx = rows_max(mx);
+        if (__any(mx > m)) {   // some column's maximum rises
+            const float mn = fmaxf(m, mx), alpha = mn == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m - mn);
+            lsum *= alpha;
+#pragma unroll
+            for (int n = 0; n < VT; n++) acc[n] *= alpha;
+            m = mn;
+        }
+        const float msafe = fmaxf(m, -1.0e30f);   // nothing visible: exp2(-inf - finite) = 0, no NaN
+        b8_t p[2];
+#pragma unroll
+        for (int pair = 0; pair < 2; pair++) {
+            typedef float f8_t __attribute__((ext_vector_type(8)));
+            f8_t e;
+#pragma unroll
+            for (int r = 0; r < 8; r++) {
+                e[r] = __builtin_amdgcn_exp2f(s[2 * pair + (r >> 2)][r & 3] - msafe);
+                lsum += e[r];
+            }
+            p[pair] = __builtin_convertvector(e, b8_t);
+        }
+#pragma unroll
+        for (int pair = 0; pair < 2; pair++)
+#pragma unroll
+            for (int n = 0; n < VT; n++)
+                acc[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(blk[(4 * DC + 4 * RC + pair * VT + n) * 64], p[pair], acc[n], 0, 0, 0);
+    }
+    lsum += __shfl_xor(lsum, 16, 64);
+    lsum += __shfl_xor(lsum, 32, 64);
+    if (tok >= ntok) return;
+    const float sk = a.sink[h] * 1.44269504088896340736f, top = fmaxf(m, sk);
+    const float w = __builtin_amdgcn_exp2f(m - top), f = w / fmaf(lsum, w, __builtin_amdgcn_exp2f(sk - top));
+#pragma unroll
+    for (int n = 0; n < VT; n++) {
+        const float o[4] = {acc[n][0] * f, acc[n][1] * f, acc[n][2] * f, acc[n][3] * f};
+        store_b16_4(a.out, a.Kb_out, t, h * VT * 16 + 16 * n + 4 * g, o);
+    }
+}
+
+template <int DC, int RC, int VT>
+void launch_prompt(const PromptArgs& k, int workgroups) {
+    constexpr int TILES = 4 * DC + 4 * RC + 2 * VT, RING = TILES <= 26 ? 3 : 2;   // (two workgroups a CU)
+    constexpr int lds = RING * TILES * 1024;
+    static bool enabled = false;
+    if (lds > 64 * 1024 && !enabled) {
+        HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_latent_prompt<DC, RC, VT, RING>), hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+        enabled = true;
+    }
+    NVLLM_LAUNCH((k_latent_prompt<DC, RC, VT, RING>), dim3(workgroups), dim3(256), lds, k);
+}
+template <int KC>
+void launch_expand(const ExpandArgs& e, dim3 grid) {
+    const int lds = 4 * e.chunks * 1024;
+    static bool enabled = false;
+    if (!enabled) {
+        HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_latent_expand<KC>), hipFuncAttributeMaxDynamicSharedMemorySize, 4 * KC * 1024));
+        enabled = true;
+    }
+    NVLLM_LAUNCH((k_latent_expand<KC>), grid, dim3(512), lds, e);
+}
+
+}  // namespace
+
+LatentPromptPlan latent_prompt_plan(const int* pos, const int* seq_ids, int T, BlockTable** tables, int block_size) {
+    LatentPromptPlan p;
+    std::vector<int> pages;
+    std::vector<std::array<int, 4>> items;
+    int alone_last = -1;
+    const int per_block = block_size / LATENT_PAGE;
+    for (int t = 0, n; t < T; t += n) {
+        n = 1;
+        while (t + n < T && seq_ids[t + n] == seq_ids[t] && pos[t + n] == pos[t + n - 1] + 1) n++;
+        if (n == 1) {
+            if (alone_last < 0) p.alone_from = t / 16;
+            alone_last = t;
+            continue;
+        }
+        const BlockTable* table = tables[seq_ids[t]];
+        const int last = pos[t + n - 1], first_pair = (int)pages.size() / 2;
+        for (int q = 0; q < 2 * (last / 32 + 1); q++) {
+            const int page = std::min(q, last / LATENT_PAGE), block = std::min(page / per_block, table->num_blocks - 1);   // (a short table ends the pass later)
+            pages.push_back(block < 0 ? 0 : table->block_indices[block] * per_block + page % per_block);
+        }
+        for (int i = 0; i < n; i += LATENT_PROMPT_TOKENS) items.push_back({t + i, std::min(LATENT_PROMPT_TOKENS, n - i), pos[t] + i, first_pair});
+        p.most_pairs = std::max(p.most_pairs, (int)pages.size() / 2 - first_pair);
+        p.tokens += n;
+        p.pairs_qk += (long)n * pos[t] + (long)n * (n + 1) / 2;
+    }
+    if (alone_last >= 0) p.alone_to = alone_last / 16 + 1;
+    std::stable_sort(items.begin(), items.end(), [](const auto& a, const auto& b) { return a[2] + a[1] > b[2] + b[1]; });
+    for (const auto& i : items) p.ints.insert(p.ints.end(), i.begin(), i.end());
+    p.n_items = (int)items.size();
+    p.n_pairs = (int)pages.size() / 2;
+    p.ints.insert(p.ints.end(), pages.begin(), pages.end());
+    while (p.ints.size() % 4) p.ints.push_back(0);
+    return p;
+}
+
+bool latent_prompt_pays(const LatentPromptPlan& plan, const LatentPool& P, int H, int dim_ld, int vdim_ld) {
+    static const int env = getenv("NVLLM_LATENT_EXPAND") ? atoi(getenv("NVLLM_LATENT_EXPAND")) : -1;   // 0: never, 1: wherever it can be done
+    auto one_of = [](int v, int a, int b, int c) { return v == a || v == b || v == c; };
+    const bool fits = P.elem_bytes == 2 && P.rank_ld <= 512 && one_of(dim_ld, 32, 64, 128) && one_of(P.rot_ld, 32, 64, 64) && one_of(vdim_ld, 32, 64, 128);
+    const double positions = 32.0 * plan.n_pairs;
+    if (env == 0 || plan.n_items == 0 || !fits || positions * H * (dim_ld + vdim_ld) * 2.0 > 512e6) return false;
+    if (env > 0) return true;
+    // us a layer, fitted to portions of 17 to 256 tokens at 0, 512 and 1,700 cached positions, alone and beside five single tokens,
+    // of 32 heads with 512 latent values and 16 with 256: two launches less, unless single tokens beside the portions want
+    // theirs as before; the walk of 64 keys after 64 keys, which few items do not hide; forming keys and values; and the products
+    // saved per pair of token and position.  96 tokens behind 512, 32 heads: 107 us a layer -> 91, beside five tokens 126 -> 118;
+    // 64 behind 1,700 93 -> 92; 17 behind 1,700 83 -> 89, not taken.  Passes of few columns (less than a thousand) gain the launches alone.
+    if ((long)plan.tokens * H < 1024) return false;
+    const double forming = 0.35 * plan.most_pairs / 2 + positions * H * (dim_ld + vdim_ld) * P.rank_ld / 4e8;
+    const double launches = plan.alone_to > plan.alone_from ? 0.0 : 8.0;
+    const double saved = plan.pairs_qk * (double)H * (P.row() + P.rank_ld - dim_ld - P.rot_ld - vdim_ld) / 2e8;
+    return forming < launches + saved;
+}
+
+void launch_latent_prompt(const LatentPrompt& a, const LatentPromptPlan& plan) {
+    if (plan.n_items <= 0) return;
+    const LatentPool& P = a.pool;
+    __half* kv = (__half*)ws_get(WS_EXPANDED, (size_t)plan.n_pairs * a.H * 32 * (a.dim_ld + a.vdim_ld) * sizeof(__half));
+    const double positions = 32.0 * plan.n_pairs, width = (double)a.H * (a.dim_ld + a.vdim_ld);
+    {
+        ExpandArgs e{};
+        e.base = (const __half*)P.base;
+        e.pages = a.pages;
+        e.n_pairs = plan.n_pairs;
+        e.chunks = P.rank_ld / 32;
+        e.row_tiles = P.row() / 32;
+        e.H = a.H;
+        e.dc = a.dim_ld / 32;
+        e.vt = a.vdim_ld / 16;
+        e.uk = a.uk;
+        e.uv = a.uv;
+        e.kv = kv;
+        const int cols = cdiv(a.H * (e.dc + e.vt / 2), 8);
+        // as many workgroups as CUs, of four pairs at least (a wave's weights are as many bytes as two pairs)
+        e.per = std::max(4, cdiv(plan.n_pairs, std::max(1, rt().num_cus / cols)));
+        ProfScope ps(PC_LATENT_EXPAND, width * P.rank_ld * 2.0 + positions * P.rank_ld * 2.0 + positions * width * 2.0, 2.0 * positions * width * P.rank_ld);
+        const dim3 grid(cols, cdiv(plan.n_pairs, e.per));
+        if (e.chunks <= 8) launch_expand<8>(e, grid);
+        else launch_expand<16>(e, grid);
+    }
+    PromptArgs k{};
+    k.base = (const __half*)P.base;
+    k.items = a.items;
+    k.pages = a.pages;
+    k.q_tiles = a.q_tiles;
+    k.q_rows = a.q_rows;
+    k.kv = kv;
+    k.sink = a.sink;
+    k.scale = a.scale;
+    k.H = a.H;
+    k.q_kb = a.H * a.dim_ld / 32;
+    k.row = P.row();
+    k.rank_ld = P.rank_ld;
+    k.out = a.out;
+    k.Kb_out = a.H * a.vdim_ld / 32;
+    ProfScope ps(PC_LATENT_ATTN, positions * (width + P.rot_ld) * 2.0 + (double)plan.tokens * a.H * (a.dim_ld + P.rot_ld + a.vdim_ld) * 2.0,
+                 2.0 * (double)plan.pairs_qk * a.H * (a.dim_ld + P.rot_ld + a.vdim_ld));
+    auto values = [&](auto dc, auto rc) {
+        constexpr int DC = decltype(dc)::value, RC = decltype(rc)::value;
+        if (a.vdim_ld == 32) launch_prompt<DC, RC, 2>(k, plan.n_items * a.H);
+        else if (a.vdim_ld == 64) launch_prompt<DC, RC, 4>(k, plan.n_items * a.H);
+        else launch_prompt<DC, RC, 8>(k, plan.n_items * a.H);
+    };
+    auto rotated = [&](auto dc) {
+        if (P.rot_ld == 32) values(dc, std::integral_constant<int, 1>{});
+        else values(dc, std::integral_constant<int, 2>{});
+    };
+    if (a.dim_ld == 32) rotated(std::integral_constant<int, 1>{});
+    else if (a.dim_ld == 64) rotated(std::integral_constant<int, 2>{});
+    else rotated(std::integral_constant<int, 4>{});
+}
+
+}  // namespace nvllm

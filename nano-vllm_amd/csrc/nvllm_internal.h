@@ -135,6 +135,8 @@ enum WsSlot {
     WS_KV_RAW,      // latent attention: a batch's latents and rotated key parts before norm and rotation
     WS_Q_ROWS,      // ... its absorbed queries
     WS_LATENT,      // ... its attended latents
+    WS_EXPANDED,    // ... keys and values of prompt portions, formed from the cached latents
+    WS_VALUES,      // ... and the attended values beside them
     WS_STATES,      // linear attention: the states a batch's chunks start from
     WS_A16_SORTED,  // mixture of experts: a batch's rows sorted by expert
     WS_F32_A,       // fp32 models: activations between operators
@@ -180,6 +182,7 @@ enum ProfClass {
     PC_LATENT_ATTN,      // attention over latents: prompt portions ...
     PC_LATENT_ATTN_TOK,  // ... and single tokens
     PC_LATENT_COMBINE,
+    PC_LATENT_EXPAND,    // ... keys and values of prompt portions
     PC_HYPER,            // hyper-connection update and norm as a launch of its own
     PC_CONV_ROPE,        // short convolution over time, rotation, cache write
     PC_WINDOW_ATTN,      // windowed attention: prompt portions ...

@@ -51,7 +51,8 @@ KvPoolView pool_view(const KVCacheManager* mgr, int n_kv_heads, int head_dim) {
 // pinned region and upload it with a single copy.
 StepArrays stage_step(const int* tokens, const int* pos_arr, const int* seq_ids, int T,
                       const int* output_indices, int B, BlockTable** tables, const BlockTable* single,
-                      int pos0, int block_size, int attn_ct, const int* token_src, bool multi_first, bool spans, int chunk_len) {
+                      int pos0, int block_size, int attn_ct, const int* token_src, bool multi_first, bool spans, int chunk_len,
+                      const std::vector<int>* extra) {
     StepArrays s{};
     s.T = T;
     s.B = B;
@@ -111,19 +112,25 @@ StepArrays stage_step(const int* tokens, const int* pos_arr, const int* seq_ids,
             t += n;
         }
         if (multi_first) {
-            std::vector<int> singles;
+            std::vector<int> singles, alone;
             size_t keep = 0;
             for (size_t i = 0; i < runs.size(); i += 4) {
                 if (runs[i + 1] == 1) {
-                    singles.insert(singles.end(), runs.begin() + (long)i, runs.begin() + (long)i + 4);
+                    const int t = runs[i];
+                    const bool tail = t > 0 && seq_of(t - 1) == seq_of(t) && pos_of(t - 1) + 1 == pos_of(t);   // of a longer portion
+                    std::vector<int>& to = tail ? singles : alone;
+                    to.insert(to.end(), runs.begin() + (long)i, runs.begin() + (long)i + 4);
                     s.kv_rows_single += runs[i + 2] + 1;
+                    if (!tail) s.kv_rows_alone += runs[i + 2] + 1;
                 } else {
                     std::copy(runs.begin() + (long)i, runs.begin() + (long)i + 4, runs.begin() + (long)keep);
                     keep += 4;
                 }
             }
             std::copy(singles.begin(), singles.end(), runs.begin() + (long)keep);
+            std::copy(alone.begin(), alone.end(), runs.begin() + (long)(keep + singles.size()));
             s.n_multi = (int)(keep / 4);
+            s.n_alone = (int)(alone.size() / 4);
         }
     }
     if (attn_ct > 0) {
@@ -189,7 +196,8 @@ StepArrays stage_step(const int* tokens, const int* pos_arr, const int* seq_ids,
         }
     }
     const size_t n_ints = (size_t)(tokens ? T : 0) + (token_src ? T : 0) + (pos_arr ? T : 0) + (seq_ids ? T : 0) + kv_row.size() +
-                          (output_indices ? B : 0) + n_seqs + total_tbl + runs.size() + span.size() + span_of.size() + chunks.size() + first_chunk.size() + 64;
+                          (output_indices ? B : 0) + n_seqs + total_tbl + runs.size() + span.size() + span_of.size() + chunks.size() + first_chunk.size() +
+                          (extra ? extra->size() : 0) + 64;
     int* host = pinned_ints(n_ints);
     int* dev = (int*)ws_get(WS_STEP, n_ints * sizeof(int));
     size_t o = 0;
@@ -226,6 +234,7 @@ StepArrays stage_step(const int* tokens, const int* pos_arr, const int* seq_ids,
     }
     o = (o + 3) & ~(size_t)3;  // int4 alignment
     s.d_runs = runs.empty() ? nullptr : put(runs.data(), runs.size());
+    s.d_extra = extra && !extra->empty() ? put(extra->data(), extra->size()) : nullptr;   // (a multiple of four)
     s.d_spans = span.empty() ? nullptr : put(span.data(), span.size());
     s.d_chunks = chunks.empty() ? nullptr : put(chunks.data(), chunks.size());   // (pairs, behind quadruples)
     s.d_first_chunk = first_chunk.empty() ? nullptr : put(first_chunk.data(), first_chunk.size());

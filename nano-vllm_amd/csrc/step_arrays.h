@@ -28,7 +28,8 @@ struct StepArrays {
     long qk_pairs;           // sum over tokens of the positions they see
     int max_run;             // tokens of the longest run
     int n_multi;             // with `multi_first`: the first n_multi runs have several tokens, the others one each
-    long kv_rows_single;     // ... positions those others see
+    int n_alone;             // ... the last n_alone of which are their sequence's only token
+    long kv_rows_single, kv_rows_alone;   // ... positions those others see
     int runs_in_tb[4];       // runs that touch each of the first four 16-token blocks
     bool one_token_per_seq;  // no sequence contributes more than one token (a pure decode step)
     // with `spans`: every sequence's portion of the batch as a whole (models whose layers carry a state from token to token)
@@ -42,6 +43,7 @@ struct StepArrays {
     int* d_chunks;           // [n_chunks][2] (span, its chunk)
     int* d_first_chunk;      // [n_spans_multi]
     std::vector<int> host_spans;
+    int* d_extra;            // with `extra`: the caller's own numbers, 16-byte aligned
     // Kernel timing, when a token sees at most `limit` positions: rows of K/V that the portions of several tokens (of one
     // token) see, each counted once, and (token, position) pairs of the former.
     long multi_rows(long limit) const { return count(0, n_spans_multi, limit, false); }
@@ -69,7 +71,7 @@ private:
 StepArrays stage_step(const int* tokens, const int* pos_arr, const int* seq_ids, int T,
                       const int* output_indices, int B, BlockTable** tables, const BlockTable* single,
                       int pos0, int block_size, int attn_ct = 0, const int* token_src = nullptr, bool multi_first = false,
-                      bool spans = false, int chunk_len = 0);
+                      bool spans = false, int chunk_len = 0, const std::vector<int>* extra = nullptr);
 
 KvPoolView pool_view(const KVCacheManager* mgr, int n_kv_heads, int head_dim);
 
