@@ -180,7 +180,7 @@ void launch_gemm_experts(const B16Weight& w, int experts, const __half* act, con
     if (rows.capacity <= 0) return;
     ensure_init();
     const bool dense = rows.pad >= 64;
-    if (w.K % 32 || w.N % 32 || experts < 1 || rows.capacity % rows.pad || !(rows.pad == 16 || rows.pad == 32 || rows.pad == 64 || rows.pad == 128))
+    if (w.K % 32 || w.N % 32 || experts < 1 || rows.capacity % rows.pad || (rows.wide && rows.source) || !(rows.wide || rows.pad == 16 || rows.pad == 32 || rows.pad == 64 || rows.pad == 128))
         NVLLM_FATAL("expert projection: [%d, %d] on %d rows in groups of %d is not supported", w.N, w.K, rows.capacity, rows.pad);
     GemmArgs a{};
     a.W = w.tiles;
@@ -200,6 +200,13 @@ void launch_gemm_experts(const B16Weight& w, int experts, const __half* act, con
     const double touched = std::min(experts, rows.live);   // matrices read
     const double bytes = touched * w.N * w.K * 2.0 + (double)rows.live * w.K * 2.0 + (double)rows.live * w.N * (epi.kind == GemmEpilogue::F32 ? 4.0 : 1.0);
     const double flops = 2.0 * rows.live * (double)w.N * w.K;
+    if (rows.wide) {
+        if (epi.kind == GemmEpilogue::SWIGLU_A16 && w.N % 64) NVLLM_FATAL("expert projection: a hidden width of %d is not padded to 32", w.N / 2);
+        if (epi.kind == GemmEpilogue::SWIGLU_A16) a.e.Kb_out = w.N / 64;
+        ProfScope ps(prof_cls, bytes, flops);
+        if (!launch_experts_wide_b16(a, rows.pad)) NVLLM_FATAL("expert projection: no tiles for groups of %d rows", rows.pad);
+        return;
+    }
     if (epi.kind == GemmEpilogue::SWIGLU_A16) {
         if (w.N % 64) NVLLM_FATAL("expert projection: a hidden width of %d is not padded to 32", w.N / 2);
         a.e.Kb_out = w.N / 64;

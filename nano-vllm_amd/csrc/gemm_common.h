@@ -163,14 +163,22 @@ struct HyperIn {
     f4_t xs[SMAX], scale, bias, w, b;
 };
 template <int SMAX>
-__device__ __forceinline__ void hyper_load_4(HyperIn<SMAX>& in, const GemmEpilogue& ep, int N, int t, int n) {
+__device__ __forceinline__ void hyper_load_x(f4_t (&xs)[SMAX], const GemmEpilogue& ep, int N, int t, int n) {
     const float* xr = ep.x + (size_t)t * ep.streams * N + n;
 #pragma unroll
-    for (int s = 0; s < SMAX; s++) in.xs[s] = *reinterpret_cast<const f4_t*>(xr + (size_t)min(s, ep.streams - 1) * N);
+    for (int s = 0; s < SMAX; s++) xs[s] = *reinterpret_cast<const f4_t*>(xr + (size_t)min(s, ep.streams - 1) * N);
+}
+template <int SMAX>
+__device__ __forceinline__ void hyper_load_vectors(HyperIn<SMAX>& in, const GemmEpilogue& ep, int n) {
     in.scale = *reinterpret_cast<const f4_t*>(ep.hyper_scale + n);
     in.bias = ep.bias ? *reinterpret_cast<const f4_t*>(ep.bias + n) : f4_t{0.f, 0.f, 0.f, 0.f};
     in.w = *reinterpret_cast<const f4_t*>(ep.norm_w + n);
     in.b = *reinterpret_cast<const f4_t*>(ep.norm_b + n);
+}
+template <int SMAX>
+__device__ __forceinline__ void hyper_load_4(HyperIn<SMAX>& in, const GemmEpilogue& ep, int N, int t, int n) {
+    hyper_load_x<SMAX>(in.xs, ep, N, t, n);
+    hyper_load_vectors<SMAX>(in, ep, n);
 }
 // The connection's coefficients, read once: left in memory they would be read again after every store to x, which might
 // alias them (a chain of loads and stores per four features).
@@ -233,6 +241,23 @@ __device__ __forceinline__ float resid_b16_4(const GemmEpilogue& ep, int N, int 
     return xn[0] * xn[0] + xn[1] * xn[1] + xn[2] * xn[2] + xn[3] * xn[3];
 }
 
+// LATENT_Q: one token's features n .. n+3, the rotated ones by the angles `turn` of their two pairs.
+__device__ __forceinline__ void latent_q_4(const GemmEpilogue& ep, int t, int n, const float* y, const float2 (&turn)[2]) {
+    if (n < ep.q_plain) {
+        store_b16_4(ep.a16_out, ep.Kb_out, t, n, y);
+        return;
+    }
+    const int m = n - ep.q_plain, h = m / ep.rot_ld, d = m - h * ep.rot_ld;
+    float z[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int e = 0; e < 4; e += 2)
+        if (d + e < ep.rot_dim) {   // (features past rot_dim are padding)
+            z[e] = y[e] * turn[e >> 1].x - y[e + 1] * turn[e >> 1].y;
+            z[e + 1] = y[e + 1] * turn[e >> 1].x + y[e] * turn[e >> 1].y;
+        }
+    *reinterpret_cast<b4_t*>(ep.q_rows + ((size_t)t * ep.q_heads + h) * ep.q_row + ep.head_ld + d) = to_b4(z);
+}
+
 // One token's features n .. n+3 through a point epilogue other than HYPER_*; returns their share of the sum of squares.
 template <int EPI>
 __device__ __forceinline__ float epi_point(const GemmEpilogue& ep, int N, int t, int n, const float* y) {
@@ -261,21 +286,14 @@ __device__ __forceinline__ float epi_point(const GemmEpilogue& ep, int N, int t,
         }
         *reinterpret_cast<f4_t*>(ep.out + (size_t)t * ep.ldo + (n - ep.latent_q)) = f4_t{y[0], y[1], y[2], y[3]};
     } else if constexpr (EPI == GemmEpilogue::LATENT_Q) {
-        if (n < ep.q_plain) {
-            store_b16_4(ep.a16_out, ep.Kb_out, t, n, y);
-        } else {
-            const int m = n - ep.q_plain, h = m / ep.rot_ld, d = m - h * ep.rot_ld;
-            float z[4] = {0.f, 0.f, 0.f, 0.f};
+        float2 turn[2] = {};
+        if (n >= ep.q_plain) {
+            const int d = (n - ep.q_plain) % ep.rot_ld, last = (ep.rot_dim >> 1) - 1;
             const float2* tab = ep.rope + (size_t)ep.pos[t] * (ep.rot_dim >> 1);
-#pragma unroll
-            for (int e = 0; e < 4; e += 2)
-                if (d + e < ep.rot_dim) {   // (features past rot_dim are padding)
-                    const float2 cs = tab[(d + e) >> 1];
-                    z[e] = y[e] * cs.x - y[e + 1] * cs.y;
-                    z[e + 1] = y[e + 1] * cs.x + y[e] * cs.y;
-                }
-            *reinterpret_cast<b4_t*>(ep.q_rows + ((size_t)t * ep.q_heads + h) * ep.q_row + ep.head_ld + d) = to_b4(z);
+            turn[0] = tab[min(d >> 1, last)];
+            turn[1] = tab[min((d >> 1) + 1, last)];
         }
+        latent_q_4(ep, t, n, y, turn);
     }
     return 0.f;
 }
@@ -299,6 +317,7 @@ void launch_gemm_prefill(GemmArgs a);
 // gemm_wide_f16.hip: the same in tiles of 256 features; false: not for this launch
 bool launch_gemm_wide_f16(const GemmArgs& a);
 bool launch_gemm_wide_b16(const GemmArgs& a);   // gemm_wide_b16.hip: bf16 models
+bool launch_experts_wide_b16(const GemmArgs& a, int pad);   // ... rows sorted by expert, in groups of expert_rows_wide()
 // gemm_waves_f16.hip, gemm_waves_b16.hip: one round of tiles with K dealt to the waves; false: not for this launch
 bool launch_gemm_waves_f16(const GemmArgs& a);
 bool launch_gemm_waves_b16(const GemmArgs& a);

@@ -93,73 +93,122 @@ __device__ __forceinline__ void wait_copies_but(int stages) {
     }
 }
 
-// RESID_*, HYPER_*: the operands of token block j + 1 travel while block j is finished.
-template <int NI, int NJ, int EPI>
-__device__ __forceinline__ void pf_residual(const GemmArgs& p, const f4_t (&v)[NI][NJ], int nb_first, int tbl_first, int tb0, const float* s_rinv, int lane,
-                                            int nb_lim) {
-    const GemmEpilogue& ep = p.e;
-    constexpr int HS = hyper_streams(EPI);
-    const int n_of = nb_first * 16 + 4 * (lane >> 4);
-    float4 xo[2][HS ? 1 : NI], gain[HS ? 1 : NI];
-    HyperIn<HS ? HS : 1> hyper[2][HS ? NI : 1];
-    auto load = [&](int set, int j) {
-        const int t = min((tb0 + tbl_first + j) * 16 + (lane & 15), p.T - 1);
+// RESID_*, HYPER_*: what a wave adds its NI x NJ tiles to.  begin() requests the first SETS token blocks' operands, finish() those of
+// block j + SETS as soon as block j is done; in between the sums may still be on their way.
+template <int NI, int NJ, int EPI, int SETS>
+struct PfResidual {
+    static constexpr int HS = hyper_streams(EPI), AHEAD = SETS < NJ ? SETS : NJ;
+    float4 xo[AHEAD][HS ? 1 : NI], gain[HS ? 1 : NI];
+    f4_t xs[HS ? AHEAD : 1][HS ? NI : 1][HS ? HS : 1];
+    HyperIn<HS ? HS : 1> vectors[HS ? NI : 1];
+    HyperMix<HS ? HS : 1> mix;
+
+    __device__ __forceinline__ void load(const GemmArgs& p, int set, int t, int n_of) {
+        const GemmEpilogue& ep = p.e;
+        t = min(t, p.T - 1);
 #pragma unroll
         for (int i = 0; i < NI; i++) {
             const int n = min(n_of + 16 * i, p.N - 4);
-            if constexpr (HS > 0) hyper_load_4<HS>(hyper[set][i], ep, p.N, t, n);
+            if constexpr (HS > 0) hyper_load_x<HS>(xs[set][i], ep, p.N, t, n);
             else xo[set][i] = *reinterpret_cast<const float4*>(ep.x + (size_t)t * p.N + n);
         }
-    };
-    load(0, 0);
-    HyperMix<HS ? HS : 1> mix;
-    if constexpr (HS > 0) {
-        mix = hyper_mix<HS>(ep);
-    } else {
-#pragma unroll
-        for (int i = 0; i < NI; i++) gain[i] = *reinterpret_cast<const float4*>(ep.gain_next + min(n_of + 16 * i, p.N - 4));
     }
+    __device__ __forceinline__ void begin(const GemmArgs& p, int nb_first, int tb_first, int lane) {
+        const GemmEpilogue& ep = p.e;
+        const int n_of = nb_first * 16 + 4 * (lane >> 4);
 #pragma unroll
-    for (int j = 0; j < NJ; j++) {
-        if (j + 1 < NJ) load((j + 1) & 1, j + 1);
-        const int tl = (tbl_first + j) * 16 + (lane & 15), t = tb0 * 16 + tl;
-        const bool tok_live = t < p.T && tb0 + tbl_first + j < p.Tb;
-        const float rinv = ep.ss_in ? s_rinv[tl] : 1.0f;
-        float ssq[NI / 2];
-#pragma unroll
-        for (int h = 0; h < NI / 2; h++) ssq[h] = 0.f;
+        for (int j = 0; j < AHEAD; j++) load(p, j, (tb_first + j) * 16 + (lane & 15), n_of);
 #pragma unroll
         for (int i = 0; i < NI; i++) {
-            const int n = n_of + 16 * i;
-            if (!tok_live || nb_first + i >= nb_lim) continue;
-            const float y[4] = {v[i][j][0] * rinv, v[i][j][1] * rinv, v[i][j][2] * rinv, v[i][j][3] * rinv};
-            if constexpr (HS > 0) {
-                hyper_update_4<HS>(hyper[j & 1][i], mix, ep, p.N, t, n, y);
-            } else if constexpr (EPI == GemmEpilogue::RESID_B16) {
-                ssq[i >> 1] += resid_b16_4(ep, p.N, t, n, xo[j & 1][i], gain[i], y);
-            } else {
-                const float4 x = xo[j & 1][i], g = gain[i];
-                // residual add as the reference's accum(): x = x + branch (layers.c:163-168)
-                const float xn[4] = {__fadd_rn(x.x, y[0]), __fadd_rn(x.y, y[1]), __fadd_rn(x.z, y[2]), __fadd_rn(x.w, y[3])};
-                *reinterpret_cast<float4*>(ep.x + (size_t)t * p.N + n) = make_float4(xn[0], xn[1], xn[2], xn[3]);
-                const float z[4] = {xn[0] * g.x, xn[1] * g.y, xn[2] * g.z, xn[3] * g.w};
-                store_a16_4(ep.a16_out, ep.Kb_out, t, n, z);
-                ssq[i >> 1] += xn[0] * xn[0] + xn[1] * xn[1] + xn[2] * xn[2] + xn[3] * xn[3];
-            }
+            const int n = min(n_of + 16 * i, p.N - 4);
+            if constexpr (HS > 0) hyper_load_vectors<HS>(vectors[i], ep, n);
+            else gain[i] = *reinterpret_cast<const float4*>(ep.gain_next + n);
         }
-        if constexpr (epi_has_ss(EPI)) {
-            // per-token sum of x^2 over each 32-feature group = two row blocks (same lane) x four lane groups
+        if constexpr (HS > 0) mix = hyper_mix<HS>(ep);
+    }
+    __device__ __forceinline__ void finish(const GemmArgs& p, const f4_t (&v)[NI][NJ], int nb_first, int tbl_first, int tb0, const float* s_rinv, int lane,
+                                           int nb_lim) {
+        const GemmEpilogue& ep = p.e;
+        const int n_of = nb_first * 16 + 4 * (lane >> 4);
 #pragma unroll
-            for (int h = 0; h < NI / 2; h++) {
-                float sq = ssq[h];
-                sq += __shfl_xor(sq, 16, 64);
-                sq += __shfl_xor(sq, 32, 64);
-                const int col = (nb_first + 2 * h) >> 1;
-                if (lane < 16 && tok_live && col < (p.N + 31) >> 5) ep.ss_out[(size_t)t * ((p.N + 31) >> 5) + col] = sq;
+        for (int j = 0; j < NJ; j++) {
+            const int set = j % AHEAD;
+            const int tl = (tbl_first + j) * 16 + (lane & 15), t = tb0 * 16 + tl;
+            const bool tok_live = t < p.T && tb0 + tbl_first + j < p.Tb;
+            const float rinv = ep.ss_in ? s_rinv[tl] : 1.0f;
+            float ssq[NI / 2];
+#pragma unroll
+            for (int h = 0; h < NI / 2; h++) ssq[h] = 0.f;
+#pragma unroll
+            for (int i = 0; i < NI; i++) {
+                const int n = n_of + 16 * i;
+                if (!tok_live || nb_first + i >= nb_lim) continue;
+                const float y[4] = {v[i][j][0] * rinv, v[i][j][1] * rinv, v[i][j][2] * rinv, v[i][j][3] * rinv};
+                if constexpr (HS > 0) {
+                    HyperIn<HS>& in = vectors[i];
+#pragma unroll
+                    for (int s = 0; s < HS; s++) in.xs[s] = xs[set][i][s];
+                    hyper_update_4<HS>(in, mix, ep, p.N, t, n, y);
+                } else if constexpr (EPI == GemmEpilogue::RESID_B16) {
+                    ssq[i >> 1] += resid_b16_4(ep, p.N, t, n, xo[set][i], gain[i], y);
+                } else {
+                    const float4 x = xo[set][i], g = gain[i];
+                    // residual add as the reference's accum(): x = x + branch (layers.c:163-168)
+                    const float xn[4] = {__fadd_rn(x.x, y[0]), __fadd_rn(x.y, y[1]), __fadd_rn(x.z, y[2]), __fadd_rn(x.w, y[3])};
+                    *reinterpret_cast<float4*>(ep.x + (size_t)t * p.N + n) = make_float4(xn[0], xn[1], xn[2], xn[3]);
+                    const float z[4] = {xn[0] * g.x, xn[1] * g.y, xn[2] * g.z, xn[3] * g.w};
+                    store_a16_4(ep.a16_out, ep.Kb_out, t, n, z);
+                    ssq[i >> 1] += xn[0] * xn[0] + xn[1] * xn[1] + xn[2] * xn[2] + xn[3] * xn[3];
+                }
+            }
+            if (j + AHEAD < NJ) load(p, set, t + AHEAD * 16, n_of);
+            if constexpr (epi_has_ss(EPI)) {
+                // per-token sum of x^2 over each 32-feature group = two row blocks (same lane) x four lane groups
+#pragma unroll
+                for (int h = 0; h < NI / 2; h++) {
+                    float sq = ssq[h];
+                    sq += __shfl_xor(sq, 16, 64);
+                    sq += __shfl_xor(sq, 32, 64);
+                    const int col = (nb_first + 2 * h) >> 1;
+                    if (lane < 16 && tok_live && col < (p.N + 31) >> 5) ep.ss_out[(size_t)t * ((p.N + 31) >> 5) + col] = sq;
+                }
             }
         }
     }
-}
+};
+constexpr bool epi_is_residual(int kind) { return kind == GemmEpilogue::RESID_A16 || kind == GemmEpilogue::RESID_B16 || hyper_streams(kind) > 0; }
+
+// ROPE_KV, LATENT_Q: a wave's angles, requested a token block ahead of their use and before anything is stored (a store might change
+// them for all the compiler knows, and a chain of position, angle and store for each of sixteen results costs 10 us).
+template <int NI, int NJ, int EPI>
+struct PfTurn {
+    int pos[NJ];
+    float2 turn[2][NI][2];
+    __device__ __forceinline__ void load(const GemmArgs& p, int j, int nb_first, int lane) {
+        const GemmEpilogue& ep = p.e;
+#pragma unroll
+        for (int i = 0; i < NI; i++) {
+            const int n = (nb_first + i) * 16 + 4 * (lane >> 4);
+            int d, dims;   // of a head
+            if constexpr (EPI == GemmEpilogue::ROPE_KV) {
+                d = (n < ep.QD ? n : n - ep.QD) % ep.hd;   // (values do not turn: theirs are read and not used)
+                dims = ep.hd;
+            } else {
+                d = max(n - ep.q_plain, 0) % ep.rot_ld;
+                dims = ep.rot_dim;
+            }
+            const float2* tab = ep.rope + (size_t)pos[j] * (dims >> 1);
+            const int last = (dims >> 1) - 1;
+            turn[j & 1][i][0] = tab[min(d >> 1, last)];
+            turn[j & 1][i][1] = tab[min((d >> 1) + 1, last)];
+        }
+    }
+    __device__ __forceinline__ void begin(const GemmArgs& p, int nb_first, int tb_first, int lane) {
+#pragma unroll
+        for (int j = 0; j < NJ; j++) pos[j] = p.e.pos[min((tb_first + j) * 16 + (lane & 15), p.T - 1)];
+        load(p, 0, nb_first, lane);
+    }
+};
 
 // The epilogues of gemm.hip applied to NI x NJ accumulator tiles of one wave.  v[i][j] of
 // lane l: token t = (tb0 + tbl_first + j)*16 + (l & 15), features n .. n+3 with
@@ -168,22 +217,30 @@ template <int NI, int NJ, int EPI, typename KVT, typename OP = OpF16x2>
 __device__ __forceinline__ void pf_epilogue(const GemmArgs& p, const f4_t (&v)[NI][NJ], int nb_first, int tbl_first, int tb0,
                                             const float* s_rinv, int lane, int nb_lim) {
     const GemmEpilogue& ep = p.e;
-    if constexpr (EPI == GemmEpilogue::RESID_A16 || EPI == GemmEpilogue::RESID_B16 || hyper_streams(EPI) > 0) {
-        pf_residual<NI, NJ, EPI>(p, v, nb_first, tbl_first, tb0, s_rinv, lane, nb_lim);
+    if constexpr (epi_is_residual(EPI)) {
+        PfResidual<NI, NJ, EPI, 2> r;
+        r.begin(p, nb_first, tb0 + tbl_first, lane);
+        r.finish(p, v, nb_first, tbl_first, tb0, s_rinv, lane, nb_lim);
         return;
+    }
+    constexpr bool TURNS = EPI == GemmEpilogue::ROPE_KV || EPI == GemmEpilogue::LATENT_Q;
+    PfTurn<NI, NJ, EPI> turns;
+    int kv_rows[NJ];
+    if constexpr (TURNS) turns.begin(p, nb_first, tb0 + tbl_first, lane);
+    if constexpr (EPI == GemmEpilogue::ROPE_KV) {
+#pragma unroll
+        for (int j = 0; j < NJ; j++) kv_rows[j] = ep.kv_row[min((tb0 + tbl_first + j) * 16 + (lane & 15), p.T - 1)];
     }
 #pragma unroll
     for (int j = 0; j < NJ; j++) {
+        if constexpr (TURNS)
+            if (j + 1 < NJ) turns.load(p, j + 1, nb_first, lane);
         const int tbj = tb0 + tbl_first + j;
         const int tl = (tbl_first + j) * 16 + (lane & 15);
         const int t = tb0 * 16 + tl;
         const bool tok_live = t < p.T && tbj < p.Tb;
         const float rinv = ep.ss_in ? s_rinv[tl] : 1.0f;
-        int pos = 0, kv_row = -1;
-        if (EPI == GemmEpilogue::ROPE_KV && tok_live) {
-            pos = ep.pos[t];
-            kv_row = ep.kv_row[t];
-        }
+        const int kv_row = EPI == GemmEpilogue::ROPE_KV ? kv_rows[j] : -1;
         float ssq[NI / 2];
 #pragma unroll
         for (int h = 0; h < NI / 2; h++) ssq[h] = 0.f;
@@ -194,7 +251,11 @@ __device__ __forceinline__ void pf_epilogue(const GemmArgs& p, const f4_t (&v)[N
             const bool live = tok_live && nb < nb_lim;
             float y[4] = {v[i][j][0] * rinv, v[i][j][1] * rinv, v[i][j][2] * rinv, v[i][j][3] * rinv};
             if constexpr (epi_is_point(EPI)) {
-                if (live) ssq[i >> 1] += epi_point<EPI>(ep, p.N, t, n, y);
+                if constexpr (EPI == GemmEpilogue::LATENT_Q) {
+                    if (live) latent_q_4(ep, t, n, y, turns.turn[j & 1][i]);
+                } else {
+                    if (live) ssq[i >> 1] += epi_point<EPI>(ep, p.N, t, n, y);
+                }
             } else if (EPI == GemmEpilogue::F32) {
                 if constexpr (OP::PLANES == 1) {
                     if (ep.softcap > 0.f)
@@ -237,9 +298,7 @@ __device__ __forceinline__ void pf_epilogue(const GemmArgs& p, const f4_t (&v)[N
             } else {  // ROPE_KV
                 if (live) {
                     if (n < ep.QD + ep.KD) {   // q or k: rotate the two pairs of this float4 (layers.c:118-141)
-                        const int d = (n < ep.QD ? n : n - ep.QD) % ep.hd;
-                        const float2* tab = ep.rope + (size_t)pos * (ep.hd >> 1) + (d >> 1);
-                        const float2 c0 = tab[0], c1 = tab[1];
+                        const float2 c0 = turns.turn[j & 1][i][0], c1 = turns.turn[j & 1][i][1];
                         const float a0 = y[0], b0 = y[1], a1 = y[2], b1 = y[3];
                         y[0] = __fsub_rn(__fmul_rn(a0, c0.x), __fmul_rn(b0, c0.y));
                         y[1] = __fadd_rn(__fmul_rn(a0, c0.y), __fmul_rn(b0, c0.x));
@@ -681,6 +740,18 @@ __global__ __launch_bounds__(128 * WR * KG, 2) void k_gemm_prefill(GemmArgs p, i
         if (split && !pf_close_split<FW, 2, 128 * WR * KG>(p, fin, id - split_from, slice)) return;
         pf_epilogue<FW, 2, EPI, KVT, OP>(p, fin, nb0 + wr * FW, wc * 4 + kg * 2, tb0, s_rinv, lane, nb_lim);
     }
+}
+
+// Workgroups that ride on a launch of `tiles` workgroups of which a CU holds one: those for which a CU is free, each wave with
+// several tokens, or a wave per token where few are (they then run when tiles are done).  A wave's tokens follow each other at about
+// 2.5 us: 208 tiles and 258 riders of 1,029 tokens took 28 us (22 since the angles are requested early), with 48 riders as long as without any
+inline int rider_groups(const GemmArgs& a, int tiles, int waves) {
+    if (a.e.kind != GemmEpilogue::LATENT_Q || !a.ride.base) return 0;
+    const int all = cdiv(a.ride.T, waves), spare = rt().num_cus - tiles;
+    return spare >= 24 ? std::min(all, spare) : all;
+}
+__device__ __forceinline__ void ride_along(const GemmArgs& p, int waves, int wave, int lane) {
+    for (int t = ((int)blockIdx.x - p.ride_from) * waves + wave; t < p.ride.T; t += ((int)gridDim.x - p.ride_from) * waves) latent_kv_ride(p.ride, t, lane);
 }
 
 inline int wide_env() {   // NVLLM_GEMM_WIDE: 0 = never the tiles of gemm_wide.h, a number of token blocks = always that height

@@ -37,7 +37,7 @@ __global__ __launch_bounds__(256, 1) void k_gemm_waves(GemmArgs p, int tiles_n, 
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     if constexpr (EPI == GemmEpilogue::LATENT_Q) {
         if ((int)blockIdx.x >= p.ride_from) {
-            latent_kv_ride(p.ride, ((int)blockIdx.x - p.ride_from) * 4 + wave, lane);
+            ride_along(p, 4, wave, lane);
             return;
         }
     }
@@ -123,6 +123,9 @@ __global__ __launch_bounds__(256, 1) void k_gemm_waves(GemmArgs p, int tiles_n, 
     if constexpr (RING > 3)
         if (i + 2 < mine) step(std::integral_constant<int, 2>{}, no{});
 
+    // what the residual epilogues add to travels while the sums meet (all of it: the steps' registers are free)
+    PfResidual<2, TBN, EPI, TBN> residual;
+    if constexpr (epi_is_residual(EPI)) residual.begin(p, nb0 + 2 * wave, tb0, lane);
     // the waves' sums meet: first the even row block of each wave's two, then the odd one
     f4_t sum[2][TBN];
 #pragma unroll
@@ -141,7 +144,8 @@ __global__ __launch_bounds__(256, 1) void k_gemm_waves(GemmArgs p, int tiles_n, 
             sum[h][j] = (z[0] + z[1]) + (z[2] + z[3]);
         }
     }
-    pf_epilogue<2, TBN, EPI, KVT, OP>(p, sum, nb0 + 2 * wave, 0, tb0, s_rinv, lane, p.NB);
+    if constexpr (epi_is_residual(EPI)) residual.finish(p, sum, nb0 + 2 * wave, 0, tb0, s_rinv, lane, p.NB);
+    else pf_epilogue<2, TBN, EPI, KVT, OP>(p, sum, nb0 + 2 * wave, 0, tb0, s_rinv, lane, p.NB);
 }
 
 template <int TBN, int EPI, typename KVT, typename OP>
@@ -154,10 +158,12 @@ void launch_waves(GemmArgs a, int tiles_n, int tiles_t) {
         enabled = true;
     }
     a.ride_from = tiles_n * tiles_t;
-    const int riders = EPI == GemmEpilogue::LATENT_Q && a.ride.base ? cdiv(a.ride.T, 4) : 0;
-    NVLLM_LAUNCH((k_gemm_waves<TBN, EPI, KVT, OP>), dim3(tiles_n * tiles_t + riders), dim3(256), LDS, a, tiles_n, tiles_t);
+    NVLLM_LAUNCH((k_gemm_waves<TBN, EPI, KVT, OP>), dim3(tiles_n * tiles_t + rider_groups(a, tiles_n * tiles_t, 4)), dim3(256), LDS, a, tiles_n, tiles_t);
 }
 
+// Seven blocks of two planes leave registers for two steps in flight, and lose: prompts of TinyLlama-1.1B, 1,547 tokens, w_down in such
+// tiles 7,890 us a pass, in those of gemm_wide.h 7,790 (six blocks at 1,500 tokens 6,710 and 7,100).
+constexpr int waves_tallest(int planes) { return planes == 1 ? 7 : 6; }
 template <int EPI, typename KVT, typename OP>
 void launch_waves_height(const GemmArgs& a, int tbn) {
     const int tiles_n = cdiv(a.NB, WAVES_FB), tiles_t = cdiv(a.Tb, tbn);
@@ -168,19 +174,19 @@ void launch_waves_height(const GemmArgs& a, int tbn) {
         case 4: launch_waves<4, EPI, KVT, OP>(a, tiles_n, tiles_t); break;
         case 5: launch_waves<5, EPI, KVT, OP>(a, tiles_n, tiles_t); break;
         case 6: launch_waves<6, EPI, KVT, OP>(a, tiles_n, tiles_t); break;
-        default: launch_waves<7, EPI, KVT, OP>(a, tiles_n, tiles_t); break;
+        default:
+            if constexpr (waves_tallest(OP::PLANES) == 7) launch_waves<7, EPI, KVT, OP>(a, tiles_n, tiles_t);
     }
 }
 
-constexpr int WAVES_TALLEST = 7;
 // The lowest height whose tiles are one round of the chip; 0: none is.  (A second round costs as much as the first, a lower
 // tile than needed only bytes.)
-inline int waves_height(const GemmArgs& a) {
+inline int waves_height(const GemmArgs& a, int tallest) {
     static const int env = getenv("NVLLM_GEMM_WAVES") ? atoi(getenv("NVLLM_GEMM_WAVES")) : -1;   // 0: never; token blocks: always that height
-    if (env >= 0 || wide_env() > 0) return wide_env() > 0 ? 0 : std::min(env, WAVES_TALLEST);
+    if (env >= 0 || wide_env() > 0) return wide_env() > 0 ? 0 : std::min(env, tallest);
     const int tiles_n = cdiv(a.NB, WAVES_FB), room = rt().num_cus / tiles_n;   // token tiles that fit beside each other
-    const int tbn = room ? cdiv(a.Tb, room) : WAVES_TALLEST + 1;
-    return tbn <= WAVES_TALLEST ? tbn : 0;
+    const int tbn = room ? cdiv(a.Tb, room) : tallest + 1;
+    return tbn <= tallest ? tbn : 0;
 }
 
 }  // namespace

@@ -8,7 +8,7 @@ namespace nvllm {
 // 16.6 -> 10.6, 17.4 -> 11.9, 19.3 -> 16.8, 22.2 -> 18.9, 23.8 -> 21.9, 25.0 -> 23.9; 1,024 features x 1,024 k at 512 and 2,000
 // tokens (1 and 4) 11.1 -> 7.9, 13.7 -> 13.5; 5,632 x 2,048 at 400 (5) 27.8 -> 20.1.
 bool launch_gemm_waves_b16(const GemmArgs& a) {
-    const int tbn = waves_height(a);
+    const int tbn = waves_height(a, waves_tallest(1));
     if (!tbn) return false;
     switch (a.e.kind) {
         case GemmEpilogue::F32: launch_waves_height<GemmEpilogue::F32, float, OpBf16>(a, tbn); break;

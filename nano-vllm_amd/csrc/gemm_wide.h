@@ -23,12 +23,14 @@ namespace nvllm {
 
 namespace {
 
-template <int TBN, int PL>
+// WT: 1, four waves with all the tokens; 2, eight waves, two groups of four with half the tokens each
+template <int TBN, int PL, int WT>
 struct WideGeom {
     static constexpr int FB = 16;                          // 16-row blocks of W per tile, four per wave
     static constexpr int TILES = FB + PL * TBN;            // 1-KiB tiles per stage
-    static constexpr int CPW = (TILES + 3) / 4;            // copies per wave and stage (the last tile is copied by several waves when there are fewer)
-    static constexpr int RING = TILES <= 22 ? 7 : TILES <= 24 ? 6 : TILES <= 30 ? 5 : 4;
+    static constexpr int WAVES = 4 * WT;
+    static constexpr int CPW = (TILES + WAVES - 1) / WAVES;   // copies per wave and stage (the last tile is copied by several waves when there are fewer)
+    static constexpr int RING = TILES <= 22 ? 7 : TILES <= 24 ? 6 : TILES <= 30 ? 5 : TILES <= 39 ? 4 : 3;
     static constexpr int RINV_BYTES = 1024;                // 1/rms of up to 256 tokens in front of the ring
     static constexpr int LDS = RINV_BYTES + RING * TILES * 1024;
     static_assert(LDS <= 160 * 1024, "the ring must fit the CU's LDS");
@@ -43,17 +45,26 @@ __device__ __forceinline__ void wide_wait() {
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
-template <int TBN, int EPI, typename KVT, typename OP>
-__global__ __launch_bounds__(256, 1) void k_gemm_wide(GemmArgs p, int tiles_n, int tiles_t) {
+// EXP: rows sorted by expert, every tile's of one (ExpertRows)
+template <int TBN, int WT, int EPI, typename KVT, typename OP, bool EXP = false>
+__global__ __launch_bounds__(256 * WT, 1) void k_gemm_wide(GemmArgs p, int tiles_n, int tiles_t) {
     constexpr int PL = OP::PLANES;
-    using G = WideGeom<TBN, PL>;
-    constexpr int RING = G::RING, CPW = G::CPW;
+    using G = WideGeom<TBN, PL, WT>;
+    constexpr int RING = G::RING, CPW = G::CPW, WAVES = G::WAVES, TBW = TBN / WT;   // TBW: token blocks of a wave
+    static_assert(TBN % WT == 0);
     extern __shared__ __attribute__((aligned(16))) unsigned char lds_wide[];
     float* s_rinv = reinterpret_cast<float*>(lds_wide);
     const h8_t* ring = reinterpret_cast<const h8_t*>(lds_wide + G::RINV_BYTES);
 
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wf = wave & 3, wt = wave >> 2;   // this wave's features and tokens inside the tile
+    if constexpr (EPI == GemmEpilogue::LATENT_Q) {
+        if ((int)blockIdx.x >= p.ride_from) {
+            ride_along(p, WAVES, wave, lane);
+            return;
+        }
+    }
     // every XCD a contiguous range of tiles, token tiles fastest: what runs together behind one L2 shares weights
     const int total = tiles_n * tiles_t;
     int id;
@@ -62,20 +73,26 @@ __global__ __launch_bounds__(256, 1) void k_gemm_wide(GemmArgs p, int tiles_n, i
         id = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + slot;
     }
     const int nb0 = id / tiles_t * G::FB, tb0 = id % tiles_t * TBN;
-    // wave w copies tiles w, w + 4, ...: weight blocks, then the planes of each token block (past the last: the last again, the
+    const __half* W = p.W;
+    if constexpr (EXP) {
+        const int e = __builtin_amdgcn_readfirstlane(p.block_expert[tb0]);
+        if (e < 0) return;   // fewer rows than the launch has room for
+        W += (size_t)e * p.expert_stride;
+    }
+    // wave w copies tiles w, w + WAVES, ...: weight blocks, then the planes of each token block (past the last: the last again, the
     // same bytes to the same place, so that no branch parts the loop)
     const __half* src[CPW];
     unsigned dst[CPW];
 #pragma unroll
     for (int u = 0; u < CPW; u++) {
-        const int q = min(wave + 4 * u, G::TILES - 1);
+        const int q = min(wave + WAVES * u, G::TILES - 1);
         dst[u] = (unsigned)(size_t)(lds_void*)lds_wide + G::RINV_BYTES + q * 1024;
-        src[u] = q < G::FB ? p.W + (size_t)min(nb0 + q, p.NB - 1) * p.nb_stride
+        src[u] = q < G::FB ? W + (size_t)min(nb0 + q, p.NB - 1) * p.nb_stride
                            : p.A + ((size_t)min(tb0 + (q - G::FB) / PL, p.Tb - 1) * p.Kb * PL + (q - G::FB) % PL) * TILE_HALVES;
     }
     unsigned at_w = lane * 16, at_a = lane * 16;   // bytes from a source's start: its k-tile, this lane's piece
-    auto copy = [&](int u, unsigned buf) {   // (whether a copy brings weights or activations depends on u alone: FB is a multiple of 4)
-        wide_copy(src[u], 4 * u < G::FB ? at_w : at_a, dst[u], buf);
+    auto copy = [&](int u, unsigned buf) {   // (whether a copy brings weights or activations depends on u alone: FB is a multiple of WAVES)
+        wide_copy(src[u], WAVES * u < G::FB ? at_w : at_a, dst[u], buf);
     };
     auto copied = [&]() {   // a stage's copies are out
         at_w += 1024;
@@ -90,16 +107,16 @@ __global__ __launch_bounds__(256, 1) void k_gemm_wide(GemmArgs p, int tiles_n, i
         for (int u = 0; u < CPW; u++) copy(u, s * G::TILES * 1024);
         copied();
     }
-    if (p.e.ss_in != nullptr) tile_rinv<16 * TBN, 256>(p, tb0, s_rinv);
+    if (p.e.ss_in != nullptr) tile_rinv<16 * TBN, 64 * WAVES>(p, tb0, s_rinv);
 
-    f4_t acc[4][TBN];
+    f4_t acc[4][TBW];
 #pragma unroll
     for (int i = 0; i < 4; i++)
 #pragma unroll
-        for (int j = 0; j < TBN; j++) acc[i][j] = f4_t{0.f, 0.f, 0.f, 0.f};
-    h8_t wa[4], wb[4], af[PL * TBN];   // weights of this stage and the next, in turn; activations: a block's are replaced as soon as it is done
-    const h8_t* mine = ring + (size_t)wave * 4 * 64 + lane;
-    const h8_t* acts = ring + (size_t)G::FB * 64 + lane;
+        for (int j = 0; j < TBW; j++) acc[i][j] = f4_t{0.f, 0.f, 0.f, 0.f};
+    h8_t wa[4], wb[4], af[PL * TBW];   // weights of this stage and the next, in turn; activations: a block's are replaced as soon as it is done
+    const h8_t* mine = ring + (size_t)wf * 4 * 64 + lane;
+    const h8_t* acts = ring + (size_t)(G::FB + wt * PL * TBW) * 64 + lane;
     int rb = 0;   // buffer of stage s
     // The products of a stage; between them the reads of the next one's operands and, with COPY, the copies of stage
     // s + RING - 1 into the buffer of stage s - 1.
@@ -112,7 +129,7 @@ __global__ __launch_bounds__(256, 1) void k_gemm_wide(GemmArgs p, int tiles_n, i
         // A wave issues an instruction every four cycles and a product takes sixteen: up to three others fit behind one, and
         // more of them in a row leave the matrix cores idle.  So one read or one copy behind a product, in places of their own.
 #pragma unroll
-        for (int j = 0; j < TBN; j++) {
+        for (int j = 0; j < TBW; j++) {
 #pragma unroll
             for (int m = 0; m < GROUP; m++) {
                 const int i = m & 3, pl = m >> 2;
@@ -120,12 +137,12 @@ __global__ __launch_bounds__(256, 1) void k_gemm_wide(GemmArgs p, int tiles_n, i
                 if (READ && i == 3) af[PL * j + pl] = next_a[(PL * j + pl) * 64];
                 if (READ && m == 1 && j < 4) wn[j] = next_w[j * 64];
                 if (COPY && m == GROUP - 2 && j < CPW) copy(j, to);
-                if (COPY && m == 0 && TBN + j < CPW) copy(TBN + j, to);
-                if (COPY && m == 2 && PL == 2 && 2 * TBN + j < CPW) copy(2 * TBN + j, to);
+                if (COPY && m == 0 && TBW + j < CPW) copy(TBW + j, to);
+                if (COPY && m == 2 && PL == 2 && 2 * TBW + j < CPW) copy(2 * TBW + j, to);
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
-        static_assert(CPW <= (PL == 2 ? 3 : 2) * TBN && TBN >= 4, "a place for every copy and every read");
+        static_assert(CPW <= (PL == 2 ? 3 : 2) * TBW && TBW >= 4, "a place for every copy and every read");
         if (COPY) copied();
         rb = nx;
     };
@@ -140,7 +157,7 @@ __global__ __launch_bounds__(256, 1) void k_gemm_wide(GemmArgs p, int tiles_n, i
 #pragma unroll
     for (int f = 0; f < 4; f++) wa[f] = mine[f * 64];
 #pragma unroll
-    for (int f = 0; f < PL * TBN; f++) af[f] = acts[f * 64];
+    for (int f = 0; f < PL * TBW; f++) af[f] = acts[f * 64];
     int s = 0;
     using yes = std::true_type;
     using no = std::false_type;
@@ -171,19 +188,19 @@ __global__ __launch_bounds__(256, 1) void k_gemm_wide(GemmArgs p, int tiles_n, i
     }
     phase(wa, wb, no{}, no{});
 
-    const int nb_first = nb0 + wave * 4;
-    pf_epilogue<4, TBN, EPI, KVT, OP>(p, acc, nb_first, 0, tb0, s_rinv, lane, p.NB);
+    pf_epilogue<4, TBW, EPI, KVT, OP>(p, acc, nb0 + wf * 4, wt * TBW, tb0, s_rinv, lane, p.NB);
 }
 
-template <int TBN, int EPI, typename KVT, typename OP>
-void launch_wide(const GemmArgs& a, int tiles_n, int tiles_t) {
-    using G = WideGeom<TBN, OP::PLANES>;
+template <int TBN, int EPI, typename KVT, typename OP, int WT = 1, bool EXP = false>
+void launch_wide(GemmArgs a, int tiles_n, int tiles_t) {
+    using G = WideGeom<TBN, OP::PLANES, WT>;
     static bool enabled = false;
     if (!enabled) {
-        HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_gemm_wide<TBN, EPI, KVT, OP>), hipFuncAttributeMaxDynamicSharedMemorySize, G::LDS));
+        HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_gemm_wide<TBN, WT, EPI, KVT, OP, EXP>), hipFuncAttributeMaxDynamicSharedMemorySize, G::LDS));
         enabled = true;
     }
-    NVLLM_LAUNCH((k_gemm_wide<TBN, EPI, KVT, OP>), dim3(tiles_n * tiles_t), dim3(256), G::LDS, a, tiles_n, tiles_t);
+    a.ride_from = tiles_n * tiles_t;
+    NVLLM_LAUNCH((k_gemm_wide<TBN, WT, EPI, KVT, OP, EXP>), dim3(tiles_n * tiles_t + rider_groups(a, tiles_n * tiles_t, G::WAVES)), dim3(64 * G::WAVES), G::LDS, a, tiles_n, tiles_t);
 }
 
 // Microseconds a launch takes in tiles of TBN token blocks: rounds of one workgroup per CU, each a start and an end beside its

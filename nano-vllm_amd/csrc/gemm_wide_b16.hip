@@ -1,10 +1,29 @@
 // gemm_wide_b16.hip -- launches of the 256-feature tiles (gemm_wide.h) for bf16 models: the wide projections whose epilogue
 // only writes (gated pairs, tiles, rows).
+#include <cmath>
+
 #include "gemm_wide.h"
 
 namespace nvllm {
 
 namespace {
+
+template <int EPI, bool EXP>
+bool launch_wide_height(const GemmArgs& a, int tbn, int tiles_n, int tiles_t) {
+    switch (tbn) {
+        case 4: launch_wide<4, EPI, float, OpBf16, 1, EXP>(a, tiles_n, tiles_t); break;
+        case 5: launch_wide<5, EPI, float, OpBf16, 1, EXP>(a, tiles_n, tiles_t); break;
+        case 6: launch_wide<6, EPI, float, OpBf16, 1, EXP>(a, tiles_n, tiles_t); break;
+        case 8: launch_wide<8, EPI, float, OpBf16, 2, EXP>(a, tiles_n, tiles_t); break;
+        case 10: launch_wide<10, EPI, float, OpBf16, 2, EXP>(a, tiles_n, tiles_t); break;
+        case 12: launch_wide<12, EPI, float, OpBf16, 2, EXP>(a, tiles_n, tiles_t); break;
+        case 14: launch_wide<14, EPI, float, OpBf16, 2, EXP>(a, tiles_n, tiles_t); break;
+        case 16: launch_wide<16, EPI, float, OpBf16, 2, EXP>(a, tiles_n, tiles_t); break;
+        default: return false;
+    }
+    return true;
+}
+constexpr int WIDE_HEIGHTS[] = {4, 5, 6, 8, 10, 12, 14, 16};   // token blocks
 
 template <int EPI>
 bool launch_wide_b16(const GemmArgs& a) {
@@ -16,18 +35,15 @@ bool launch_wide_b16(const GemmArgs& a) {
     // at 700 (220 of 160) 50 -> 46; of 2,816 at 700 (242 of 64) 30.4 -> 29, at 1,029 (242 of 96) 38 -> 34, at 1,600 (220 of
     // 160) 55 -> 45.  154 tiles of 64 measured the same, two rounds (484 of 96) 66 -> 69; heights of 13 and 16 blocks, whose
     // sums do not fit 256 registers, 65 -> 69 where they make one round of two.
+    // Eight waves, two to a SIMD, from eight blocks on: one's requests go out behind the other's products.
     const int cus = rt().num_cus, tiles_n = cdiv(a.NB, 16);
-    int tbn = 4;
-    while (tbn < 10 && tiles_n * cdiv(a.Tb, tbn) > cus) tbn += 2;
+    int tbn = 0;
+    for (int h : WIDE_HEIGHTS)
+        if (!tbn && tiles_n * cdiv(a.Tb, h) <= cus) tbn = h;
     if (wide_env() > 0) tbn = wide_env();
-    const int tiles_t = cdiv(a.Tb, tbn), tiles = tiles_n * tiles_t;
-    if (wide_env() < 0 && (tiles > cus || 100 * tiles < 85 * cus)) return false;
-    if (tbn == 4) launch_wide<4, EPI, float, OpBf16>(a, tiles_n, tiles_t);
-    else if (tbn == 6) launch_wide<6, EPI, float, OpBf16>(a, tiles_n, tiles_t);
-    else if (tbn == 8) launch_wide<8, EPI, float, OpBf16>(a, tiles_n, tiles_t);
-    else if (tbn == 10) launch_wide<10, EPI, float, OpBf16>(a, tiles_n, tiles_t);
-    else return false;
-    return true;
+    const int tiles_t = tbn ? cdiv(a.Tb, tbn) : 0, tiles = tiles_n * tiles_t;
+    if (wide_env() < 0 && (!tbn || 100 * tiles < 80 * cus)) return false;
+    return launch_wide_height<EPI, false>(a, tbn, tiles_n, tiles_t);
 }
 
 }  // namespace
@@ -37,8 +53,25 @@ bool launch_gemm_wide_b16(const GemmArgs& a) {
         case GemmEpilogue::SWIGLU_A16: return launch_wide_b16<GemmEpilogue::SWIGLU_A16>(a);
         case GemmEpilogue::TILE_B16: return launch_wide_b16<GemmEpilogue::TILE_B16>(a);
         case GemmEpilogue::ROWS_B16: return launch_wide_b16<GemmEpilogue::ROWS_B16>(a);
+        case GemmEpilogue::LATENT_Q: return launch_wide_b16<GemmEpilogue::LATENT_Q>(a);
         default: return false;
     }
+}
+
+// Rows sorted by expert: groups as tall as hold the rows an expert gets from a batch of that many, with the chance that one of
+// sixteen gets more at a few in a hundred (a second group then); 0: not for these sizes.
+int expert_rows_wide(int rows, int experts, int N, int K) {
+    const double per = (double)rows / experts;
+    const int cus = rt().num_cus, tiles = cdiv(N, 256) * experts;
+    if (wide_env() == 0 || K < 1024 || per < 40 || tiles > cus || 100 * tiles < 40 * cus) return 0;
+    for (int h : WIDE_HEIGHTS)
+        if (16 * h >= per + 2.5 * std::sqrt(per)) return 16 * h;
+    return 0;
+}
+bool launch_experts_wide_b16(const GemmArgs& a, int pad) {
+    const int tbn = pad / 16, tiles_n = cdiv(a.NB, 16), tiles_t = a.Tb / tbn;
+    if (a.e.kind == GemmEpilogue::SWIGLU_A16) return launch_wide_height<GemmEpilogue::SWIGLU_A16, true>(a, tbn, tiles_n, tiles_t);
+    return a.e.kind == GemmEpilogue::F32 && launch_wide_height<GemmEpilogue::F32, true>(a, tbn, tiles_n, tiles_t);
 }
 
 }  // namespace nvllm

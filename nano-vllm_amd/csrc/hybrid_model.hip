@@ -503,7 +503,7 @@ void HybridModel::forward_b16(const PassArgs& a, const StepArrays& st) {
         hid = std::max(hid, b16_halves(T, (int)(H * vp)));
         hid = std::max(hid, b16_halves(T, pad32(f.dense)));
         if (f.experts) {
-            const int pad = route_pad(T, f.experts, f.top);
+            const int pad = expert_groups(T, f.experts, f.top, l.experts_up, l.experts_down).pad;
             const size_t w = route_ints(T, f.experts, f.top, pad);
             const int cap = route_plan(nullptr, T, f.experts, f.top, pad).capacity;
             hid = std::max(hid, b16_halves(cap, pad32(f.expert_ff)));
@@ -580,9 +580,10 @@ void HybridModel::forward_b16(const PassArgs& a, const StepArrays& st) {
             GemmEpilogue ez = normed(GemmEpilogue::F32);
             ez.out = z; ez.ldo = ldz;
             launch_gemm_b16(w.router, act, T, ez, PC_GEMM_ROUTER);
-            const RoutePlan plan = route_plan(route_mem, T, f.experts, f.top, route_pad(T, f.experts, f.top));
+            const ExpertGroups groups = expert_groups(T, f.experts, f.top, w.experts_up, w.experts_down);
+            const RoutePlan plan = route_plan(route_mem, T, f.experts, f.top, groups.pad);
             launch_route(plan, z, ldz);
-            ExpertRows er{plan.block_expert, plan.source, plan.capacity, plan.pad, T * f.top};
+            ExpertRows er{plan.block_expert, plan.source, plan.capacity, plan.pad, T * f.top, groups.wide};
             GemmEpilogue eu = normed(GemmEpilogue::SWIGLU_A16);
             eu.ss_gather = plan.source; eu.row_weight = plan.weight; eu.a16_out = wide;
             if (plan.pad >= 64) {   // many rows per expert: sorted once (a gathering tile copy touches a cache line per 16 bytes)

@@ -17,7 +17,13 @@ struct RoutePlan {
     int* choice;           // [T][top] expert
     float* score;          // [T][top]
 };
-int route_pad(int T, int E, int top);               // group size that suits a batch
+int route_pad(int T, int E, int top);   // group size that suits a batch in tiles of 128 features or less
+// The group size that suits a batch's products with [up] and [down] stacked by expert (bf16); wide: expert_rows_wide()'s.
+struct ExpertGroups {
+    int pad;
+    bool wide;
+};
+ExpertGroups expert_groups(int T, int E, int top, const B16Weight& up, const B16Weight& down);
 size_t route_ints(int T, int E, int top, int pad);  // 4-byte words route_plan() lays out
 RoutePlan route_plan(int* mem, int T, int E, int top, int pad);
 // z: [T][ldz] router logits in columns 0 .. E-1; the `top` largest (the first of equals) are chosen

@@ -381,9 +381,12 @@ struct ExpertRows {
     const int* block_expert;   // [capacity / 16] expert of each 16-row block, -1: no rows (the same within a group)
     const int* source;         // row -> row of the activations, null: rows are the activations' own
     int capacity;              // rows, a multiple of pad: an upper bound known to the host
-    int pad;                   // 16, 32, 64 or 128
+    int pad;                   // 16, 32, 64 or 128; expert_rows_wide()
     int live;                  // expected number of rows (bytes and flops of the kernel timing)
+    bool wide = false;         // pad is expert_rows_wide()'s (the rows are the activations' own)
 };
+// gemm_wide_b16.hip: the group size with which `rows` rows of all experts meet [N][K] matrices in tiles of 256 features; 0: they do not
+int expert_rows_wide(int rows, int experts, int N, int K);
 // w: [experts][N][K] stacked, N a multiple of 32.  Kinds SWIGLU_A16 and F32.
 void launch_gemm_experts(const B16Weight& w, int experts, const __half* act, const ExpertRows& rows, const GemmEpilogue& epi, int prof_cls);
 
