@@ -254,6 +254,13 @@ int launch_gemm(const WeightEntry& w, const __half* tiles, int N, const __half* 
         if (epi.kind == GemmEpilogue::F32 && epi.amax_out) launch_argmax_ld(epi.amax_out, epi.out, T, N, epi.ldo, epi.amax_out_host);
         return a.ksplit;
     }
+    if (force_ksplit <= 0 && !wsp && !(epi.kind == GemmEpilogue::F32 && epi.amax_out) && gemm_leaves_streaming(a.NB, a.Kb, a.Tb, 2, rt().num_cus)) {
+        a.ksplit = 1;
+        a.kb_per_split = a.Kb;
+        ProfScope ps(prof_cls, bytes, 2.0 * T * (double)N * w.K);
+        if (launch_gemm_waves_f16(a) || launch_gemm_wide_f16(a)) return 1;
+        ps.drop();
+    }
     const GemmPlan pl = gemm_plan(N, w.K, T, epi.kind, force_ksplit, max_counters, wsp ? wsp->slab_bytes : 0);
     const int TB = pl.TB, nbw = pl.nbw, tiles_n = pl.tiles_n, tiles_t = pl.tiles_t;
     int ks = pl.ks;

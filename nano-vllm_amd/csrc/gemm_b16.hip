@@ -109,6 +109,13 @@ void launch_kind(GemmArgs a, int prof_cls, double bytes, double flops) {
         if (EPI == GemmEpilogue::F32 && a.e.amax_out) launch_argmax_ld(a.e.amax_out, a.e.out, a.T, a.N, a.e.ldo, a.e.amax_out_host);
         return;
     }
+    if (!GRP && !narrow && !(EPI == GemmEpilogue::F32 && a.e.amax_out) && gemm_leaves_streaming(a.NB, a.Kb, a.Tb, 1, rt().num_cus)) {
+        a.ksplit = 1;
+        a.kb_per_split = a.Kb;
+        ProfScope ps(prof_cls, bytes, flops);
+        if (launch_gemm_waves_b16(a) || launch_gemm_wide_b16(a)) return;
+        ps.drop();
+    }
     // a block-diagonal product has a short K and no K split; its plan is that of one group times the groups
     const int groups = GRP ? a.NB / a.group_nb : 1;
     GemmPlan pl = gemm_plan(GRP ? a.group_nb * 16 * groups : a.N, a.Kb * 32, a.T, EPI, GRP || narrow || (EPI == GemmEpilogue::F32 && a.e.amax_out) ? 1 : 0, 1 << 16, 0);

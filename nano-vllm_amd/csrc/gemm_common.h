@@ -320,6 +320,17 @@ bool launch_gemm_wide_b16(const GemmArgs& a);   // gemm_wide_b16.hip: bf16 model
 bool launch_experts_wide_b16(const GemmArgs& a, int pad);   // ... rows sorted by expert, in groups of expert_rows_wide()
 // gemm_waves_f16.hip, gemm_waves_b16.hip: one round of tiles with K dealt to the waves; false: not for this launch
 bool launch_gemm_waves_f16(const GemmArgs& a);
+// Whether 65 to 255 tokens are better off in the launchers of hundreds (if these have tiles for them) than in groups of 64 that
+// stream the weights: where the groups' workgroups are more than the CUs, and past 128 tokens, where narrow projections of a short K
+// leave the 16-token groups for a K split across workgroups, if tiles of 16 tokens fit the chip.  fp16, us there and here: 11,264 x 2,048 k at
+// 80, 128, 160 tokens 29.4 -> 20.8, 28.6 -> 25.0, 46 -> 27; 5,632 x 2,048 at 160 27.3 -> 17.2; 2,048 x 2,048 at 160, 255
+// 12.7 -> 10.6, 13.3 -> 11.7; 1,024 x 1,024 8.9 -> 7.0; 512 x 512 8.0 -> 5.4; longer K: 2,048 x 5,632 at 160 23.0 -> 28.1, not taken.
+// bf16: 24.2 -> 18.9, 26.0 -> 20.3; 21.6 -> 15.4; 11.1 -> 10.5, 11.3 -> 9.8; 8.5 -> 6.2; 2,560 x 2,048 at 160 11.5 -> 12.5, not taken.
+inline bool gemm_leaves_streaming(int NB, int Kb, int Tb, int planes, int cus) {
+    if (Tb <= 4) return false;
+    if (cdiv(NB, 4) * cdiv(Tb, 4) > cus) return true;
+    return Tb > 8 && Kb <= 64 && cdiv(NB, 8) * Tb <= cus && (planes == 2 || NB <= 128);
+}
 bool launch_gemm_waves_b16(const GemmArgs& a);
 
 }  // namespace nvllm

@@ -220,6 +220,7 @@ struct ProfSuppress {
 struct ProfScope {  // names the class of, and attaches timing events to, the ONE launch made inside it
     ProfScope(int cls, double bytes, double flops);
     ~ProfScope();
+    void drop();   // nothing was launched inside after all
     int slot;
 };
 

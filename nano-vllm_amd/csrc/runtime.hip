@@ -166,6 +166,14 @@ ProfScope::ProfScope(int cls, double bytes, double flops) : slot(-1) {
     g_cur_start = r.a;   // consumed by the launch inside this scope (one launch per scope)
     g_cur_stop = r.b;
 }
+void ProfScope::drop() {
+    if (slot < 0) return;
+    g_prof_free.push_back(g_prof_pending.back().a);
+    g_prof_free.push_back(g_prof_pending.back().b);
+    g_prof_pending.pop_back();
+    slot = -1;
+    g_cur_start = g_cur_stop = nullptr;
+}
 ProfScope::~ProfScope() {
     if (slot < 0) return;
     g_cur_start = g_cur_stop = nullptr;

@@ -115,3 +115,35 @@ def test_bf16_passes(folders, tmp_path, kind, height):
     got = np.load(dst)
     for q, o in want.items():
         assert hybrid_util.error(got[str(q)], o) < hybrid_util.limit(False), q   # the bar of the designs' whole passes
+
+
+# Passes of 65 to 255 tokens: gated pairs so wide that groups of 64 tokens are more workgroups than CUs, and narrow
+# projections past 128 tokens (csrc/gemm_common.h, gemm_leaves_streaming)
+@pytest.mark.gpu
+@pytest.mark.parametrize("kv_bytes", [4, 2])
+def test_between_decode_and_prompts_fp16(hip, oracle, tmp_path, kv_bytes):
+    path = str(tmp_path / "m.bin")
+    synth.write_model(path, synth.ModelShape(dim=256, hidden_dim=5632, n_layers=2, n_heads=4, n_kv_heads=2, vocab_size=700, max_seq_len=512), seed=7)
+    for chunk in (65, 129, 193, 255):
+        kw = dict(n_new=2, collect_logits=True, chunk_size=chunk, temperature=0.0)
+        want = util.run_engine(oracle, path, synth.make_requests(1, 255, 256, 700, seed=chunk), **kw)["steps"]
+        hip.nvllm_set_kv_elem_bytes(kv_bytes)
+        try:
+            got = util.run_engine(hip, path, synth.make_requests(1, 255, 256, 700, seed=chunk), **kw)["steps"]
+        finally:
+            hip.nvllm_set_kv_elem_bytes(4)
+        for g, o in zip(got, want):
+            np.testing.assert_array_equal(g["sampled"], o["sampled"])
+            assert np.abs(g["logits"] - o["logits"]).max() < (2e-4 if kv_bytes == 4 else 2e-3)   # the bars of the forward pass
+
+
+@pytest.mark.gpu
+def test_between_decode_and_prompts_bf16(hip, tmp_path):
+    cfg = synth.latent_config(256, 203, [(synth.latent_mixer(4, 32, 32, 32, 64, 96), 5632)] * 2, streams=2)
+    path, cfg, w = latent_util.model(tmp_path, "between", cfg=cfg)
+    seq = hybrid_util.tokens(700, 203, 3)
+    want = latent_oracle.forward(cfg, w, seq)
+    eng = latent_util.engine(hip, path, False, tokens=704)
+    got = latent_util.feed_all(eng, [[(0, n)] for n in (65, 255, 129, 193, 58)], {0: seq})[0]
+    eng.close()
+    assert latent_util.error(got, want) < latent_util.limit(False)
