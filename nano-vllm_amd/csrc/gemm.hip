@@ -100,12 +100,13 @@ constexpr int MAX_COUNTERS = 1 << 16;
 // token block); sizes beyond the 64 KiB default are enabled once.
 template <int NBW, int TB, int NW, int EPI, typename KVT, int RW = NVLLM_RW>
 static void launch_k(const GemmArgs& a, dim3 grid) {
-    constexpr int shmem = gemm_tile_lds<NBW, TB, NW>();
-    static_assert(shmem <= 160 * 1024, "partial tiles must fit the CU's LDS");
+    constexpr int least = gemm_tile_lds<NBW, TB, NW>(), most = EPI == GemmEpilogue::F32 && TB > 1 ? std::max(least, GEMM_LDS_ALONE) : least;
+    const int shmem = EPI == GemmEpilogue::F32 ? gemm_tile_lds<NBW, TB, NW>(a.e) : least;
+    static_assert(most <= 160 * 1024, "partial tiles must fit the CU's LDS");
     static bool enabled = false;
-    if (shmem > 64 * 1024 && !enabled) {
+    if (most > 64 * 1024 && !enabled) {
         HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_gemm<NBW, TB, NW, EPI, KVT, RW>),
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, shmem));
+                                      hipFuncAttributeMaxDynamicSharedMemorySize, most));
         enabled = true;
     }
     NVLLM_LAUNCH((k_gemm<NBW, TB, NW, EPI, KVT, RW>), grid, dim3(NW * 64), shmem, a);
@@ -252,6 +253,7 @@ int launch_gemm(const WeightEntry& w, const __half* tiles, int N, const __half* 
             launch_gemm_prefill(a);
         }
         if (epi.kind == GemmEpilogue::F32 && epi.amax_out) launch_argmax_ld(epi.amax_out, epi.out, T, N, epi.ldo, epi.amax_out_host);
+        if (epi.kind == GemmEpilogue::F32 && epi.out_host) copy_rows_to_host(epi.out_host, epi.out, (size_t)T * epi.ldo);
         return a.ksplit;
     }
     if (force_ksplit <= 0 && !wsp && !(epi.kind == GemmEpilogue::F32 && epi.amax_out) && gemm_leaves_streaming(a.NB, a.Kb, a.Tb, 2, rt().num_cus)) {

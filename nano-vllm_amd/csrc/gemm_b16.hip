@@ -28,12 +28,13 @@ __global__ __launch_bounds__(WAVES * 64) void k_gemm_b16(GemmArgs p) {
 
 template <int NBW, int TB, int WAVES, int EPI, bool GRP, bool EXP = false>
 void launch_stream(const GemmArgs& a, dim3 grid) {
-    constexpr int shmem = gemm_tile_lds<NBW, TB, WAVES>();
-    static_assert(shmem <= 160 * 1024, "partial tiles must fit the CU's LDS");
+    constexpr int least = gemm_tile_lds<NBW, TB, WAVES>(), most = EPI == GemmEpilogue::F32 && TB > 1 ? std::max(least, GEMM_LDS_ALONE) : least;
+    const int shmem = EPI == GemmEpilogue::F32 ? gemm_tile_lds<NBW, TB, WAVES>(a.e) : least;
+    static_assert(most <= 160 * 1024, "partial tiles must fit the CU's LDS");
     static bool enabled = false;
-    if (shmem > 64 * 1024 && !enabled) {
+    if (most > 64 * 1024 && !enabled) {
         HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_gemm_b16<NBW, TB, WAVES, EPI, GRP, EXP>),
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, shmem));
+                                      hipFuncAttributeMaxDynamicSharedMemorySize, most));
         enabled = true;
     }
     NVLLM_LAUNCH((k_gemm_b16<NBW, TB, WAVES, EPI, GRP, EXP>), grid, dim3(WAVES * 64), shmem, a);
@@ -107,6 +108,7 @@ void launch_kind(GemmArgs a, int prof_cls, double bytes, double flops) {
             if (GRP || !(launch_gemm_waves_b16(a) || launch_gemm_wide_b16(a))) launch_dense<EPI, GRP>(a);   // (their own rules are there)
         }
         if (EPI == GemmEpilogue::F32 && a.e.amax_out) launch_argmax_ld(a.e.amax_out, a.e.out, a.T, a.N, a.e.ldo, a.e.amax_out_host);
+        if (EPI == GemmEpilogue::F32 && a.e.out_host) copy_rows_to_host(a.e.out_host, a.e.out, (size_t)a.T * a.e.ldo);
         return;
     }
     if (!GRP && !narrow && !(EPI == GemmEpilogue::F32 && a.e.amax_out) && gemm_leaves_streaming(a.NB, a.Kb, a.Tb, 1, rt().num_cus)) {

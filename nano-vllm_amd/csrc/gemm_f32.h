@@ -43,6 +43,8 @@ struct F32Gemm {
     long expert_stride = 0;
     const float* row_weight = nullptr;
     int live, touched = 1;   // for the figures of a profile: rows that are some token's, matrices they can be of
+    // one STORE segment: its rows also go to this page-locked host array, laid out like its `out` (null: no)
+    float* out_host = nullptr;
     // fp16 weights, one STORE segment: (maximum, its first index) of each 16 outputs of a token -> [block][amax_ld]
     float2* amax_pairs = nullptr;
     int amax_ld = 0;

@@ -60,13 +60,15 @@ __device__ __forceinline__ void f32_finish(const F32Gemm& p, const F32Segment& s
             return;
         }
     }
-    float* o = sg.out + (size_t)t * sg.ldo + n;
-    if (sg.vec) {
-        *reinterpret_cast<f4_t*>(o) = y;
-    } else {
+    for (float* rows = sg.out; rows; rows = rows == sg.out ? p.out_host : nullptr) {
+        float* o = rows + (size_t)t * sg.ldo + n;
+        if (sg.vec) {
+            *reinterpret_cast<f4_t*>(o) = y;
+        } else {
 #pragma unroll
-        for (int r = 0; r < 4; r++)
-            if (n + r < sg.N) o[r] = y[r];
+            for (int r = 0; r < 4; r++)
+                if (n + r < sg.N) o[r] = y[r];
+        }
     }
 }
 __device__ __forceinline__ f4_t f32_old(const F32Segment& sg, int t, int n) {   // t < T; features past the last are those of the last

@@ -12,6 +12,8 @@
 // angles and the integer arrays of the step are read-only during the launch and stay on plain loads.
 #pragma once
 
+#include <algorithm>
+
 #include "gemm_common.h"
 
 namespace nvllm {
@@ -37,6 +39,16 @@ struct TileIdx {
 template <int NBW, int TB, int NW>
 constexpr int gemm_tile_lds() {
     return NW * NBW * TB * 64 * 16 + (TB * 16 + NW * 64 + 2 * TB * 16) * 4 + 16;
+}
+
+// Bytes of LDS a launch of F32 takes when its rows go to the host: with two workgroups per CU all tiles of a 32,000-word classifier
+// are resident and done at once, and PCIe would idle until then; one per CU, and the first half's rows cross beside the second's
+// products (64 rows of TinyLlama: the pass 6 us shorter than with a copy behind it, and 20 like this).  Up to 16 rows the weights take as long as PCIe: left alone.
+constexpr int GEMM_LDS_ALONE = 84 * 1024;
+template <int NBW, int TB, int NW>
+inline int gemm_tile_lds(const GemmEpilogue& e) {
+    constexpr int need = gemm_tile_lds<NBW, TB, NW>();
+    return TB > 1 && e.out_host && need < GEMM_LDS_ALONE ? GEMM_LDS_ALONE : need;
 }
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t gemm_rsrc(const void* base, unsigned bytes) {
@@ -478,13 +490,17 @@ __device__ __forceinline__ bool gemm_tile(const GemmArgs& p, const TileIdx ix, u
                         for (int r = 0; r < 4; r++) y[r] = ep.softcap * tanhf(y[r] / ep.softcap);
                 }
                 if (live) {
-                    float* o = ep.out + (size_t)t * ep.ldo + n;
-                    if (n + 3 < p.N && (ep.ldo & 3) == 0) {
-                        *reinterpret_cast<float4*>(o) = make_float4(y[0], y[1], y[2], y[3]);
-                    } else {
+                    // logits rows go to the host from here: 64-byte pieces cross PCIe as fast as a copy's (64 rows of 32,000:
+                    // 157 us, a copy kernel 151), beside the products instead of after them and after a launch's gap
+                    for (float* rows = ep.out; rows; rows = rows == ep.out ? ep.out_host : nullptr) {
+                        float* o = rows + (size_t)t * ep.ldo + n;
+                        if (n + 3 < p.N && (ep.ldo & 3) == 0) {
+                            *reinterpret_cast<float4*>(o) = make_float4(y[0], y[1], y[2], y[3]);
+                        } else {
 #pragma unroll
-                        for (int r = 0; r < 4; r++)
-                            if (n + r < p.N) o[r] = y[r];
+                            for (int r = 0; r < 4; r++)
+                                if (n + r < p.N) o[r] = y[r];
+                        }
                     }
                 }
                 if (ep.amax_pairs != nullptr) {

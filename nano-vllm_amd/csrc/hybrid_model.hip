@@ -625,6 +625,7 @@ void HybridModel::forward_b16(const PassArgs& a, const StepArrays& st) {
     e.out = a.d_logits; e.ldo = V_;
     e.amax_out = a.d_argmax;
     e.amax_out_host = a.argmax_host;
+    e.out_host = a.logits_host;
     e.amax_ld = (B + 63) & ~63;
     e.amax_pairs = (float2*)ws_get(WS_AMAX_PAIRS, (size_t)cdiv(V_, 32) * e.amax_ld * sizeof(float2));
     launch_gemm_b16(head_, rows_out, B, e, PC_GEMM_HEAD);
@@ -709,6 +710,7 @@ void HybridModel::forward_f32(const PassArgs& a, const StepArrays& st) {
     wait_for_row_copies();
     F32Gemm head = F32Gemm(x, B, D_).norm(final_norm_, eps_);
     head.in_rows = st.d_out_idx;
+    head.out_host = a.logits_host;
     launch_gemm_f32(head.add((const float*)embed_, V_, a.d_logits), PC_GEMM_HEAD);
     launch_argmax_ld(a.d_argmax, a.d_logits, B, V_, V_, a.argmax_host);
 }

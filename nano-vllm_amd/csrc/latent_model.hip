@@ -467,6 +467,7 @@ void LatentHyperModel::forward_b16(const PassArgs& a, const StepArrays& st, cons
     e.out = a.d_logits; e.ldo = V_; e.softcap = softcap_;
     e.amax_out = a.d_argmax;
     e.amax_out_host = a.argmax_host;
+    e.out_host = a.logits_host;
     e.amax_ld = (B + 63) & ~63;
     e.amax_pairs = (float2*)ws_get(WS_AMAX_PAIRS, (size_t)cdiv(V_, 32) * e.amax_ld * sizeof(float2));
     launch_gemm_b16(head_, rows, B, e, PC_GEMM_HEAD);
@@ -522,6 +523,7 @@ void LatentHyperModel::forward_f32(const PassArgs& a, const StepArrays& st) {
     head.in_rows = st.d_out_idx;
     launch_gemm_f32(head.add((const float*)embed_, V_, a.d_logits), PC_GEMM_HEAD);
     launch_softcap(a.d_logits, softcap_, (long)B * V_);
+    if (a.logits_host) copy_rows_to_host(a.logits_host, a.d_logits, (size_t)B * V_);
     launch_argmax_ld(a.d_argmax, a.d_logits, B, V_, V_, a.argmax_host);
 }
 

@@ -18,6 +18,7 @@ extern "C" {
 extern int g_paged_mode;
 extern KVCacheManager g_kv_manager;
 void* nvllm_internal_pinned_alloc(size_t bytes);
+bool nvllm_internal_pinned_holds(const void* ptr, size_t bytes);
 }
 
 namespace nvllm {
@@ -218,11 +219,19 @@ static bool argmax_direct() {
     return on;
 }
 
+// Where the classifier itself stores a pass's logits rows for the host (null: finish_pass() copies them).  The caller must be waiting
+// for the pass -- rows of a pass sent ahead cross PCIe beside the next pass's kernels --, and the rows lie in malloc_run_state's array.
+// A pass of 64 rows of 32,000 values gets 20 us shorter (classifier 38, copy 147 before), of 32 rows 20 (15 and 73), of one 12: the copy's launch.
+static float* direct_rows(const RunState* s, int B, int V, bool waits) {
+    if (rt().logits_mode != NVLLM_LOGITS_HOST || !waits || B <= 0 || !argmax_direct() || ((size_t)s->logits & 15)) return nullptr;
+    return nvllm_internal_pinned_holds(s->logits, (size_t)B * V * sizeof(float)) ? s->logits : nullptr;
+}
+
 // `host_written`: the pass's last kernel has stored the indices into next_slot(B).host itself.  `waits`: the caller waits for
 // the pass before it sends another, so its rows follow its kernels on the same stream, without the switch to the copies'
-// stream and the event between them.
+// stream and the event between them.  `rows_written`: direct_rows() was given to the classifier.
 static long finish_pass(RunState* s, float* d_logits, int* d_argmax, int B, int V, PassView view, bool waits, bool chained = false,
-                        bool host_written = false) {
+                        bool host_written = false, bool rows_written = false) {
     PassSlot& slot = next_slot(B);
     const long ticket = g_next_ticket++;
     hipStream_t stream = rt().stream;
@@ -238,7 +247,7 @@ static long finish_pass(RunState* s, float* d_logits, int* d_argmax, int B, int 
     if (!host_written && (B > 0 || chained))
         HIP_CHECK(hipMemcpyAsync(slot.host, d_argmax, (size_t)(B + (chained ? 1 : 0)) * sizeof(int), hipMemcpyDeviceToHost, stream));
     slot.chained = chained;
-    if (rt().logits_mode == NVLLM_LOGITS_HOST && B > 0)
+    if (rt().logits_mode == NVLLM_LOGITS_HOST && B > 0 && !rows_written)
         HIP_CHECK(hipMemcpyAsync(s->logits, d_logits, (size_t)B * V * sizeof(float), hipMemcpyDeviceToHost, stream));
     HIP_CHECK(hipEventRecord(slot.ev, stream));
     if (rt().logits_mode == NVLLM_LOGITS_HOST && !waits) g_rows_copied = slot.ev;
@@ -361,7 +370,7 @@ static F32Gemm rows_qkv(const float* x, const StepArrays& st, int T, int D, cons
 // The reference's layer loop (model.c:352-418) on fp32 weights, five launches a layer: the norms, rotation, cache write,
 // SwiGLU and residual adds ride in the projections (gemm_f32.hip).  Leaves the logits of the output rows in d_logits.
 static void forward_f32(const StepArrays& st, int T, int B, Config* p, RunState* s, Weights* w, const KvPoolView& pool,
-                        const float2* rope, float* d_logits) {
+                        const float2* rope, float* d_logits, float* logits_host) {
     const int D = p->dim, F = p->hidden_dim, hd = p->head_dim, H = p->n_heads, KVH = p->n_kv_heads;
     const int QD = H * hd, KD = KVH * hd, V = p->vocab_size;
     const float eps = 1e-5f;
@@ -379,6 +388,7 @@ static void forward_f32(const StepArrays& st, int T, int B, Config* p, RunState*
     }
     F32Gemm head = F32Gemm(s->x, B, D).norm(w->rms_final_weight, eps);
     head.in_rows = st.d_out_idx;
+    head.out_host = logits_host;
     if (B > 0) launch_gemm_f32(head.add(w->lm_head, V, d_logits), PC_GEMM_HEAD);
 }
 
@@ -757,9 +767,10 @@ static long enqueue_pass(int* tokens, int num_tokens, int* pos_arr, int* seq_ids
         const bool to_host = B > 0 && argmax_direct();
         PassArgs a{tokens, pos_arr, seq_ids, output_indices, token_src, T, B, block_tables, &g_kv_manager,
                    (float*)ws_get(WS_LOGITS, (size_t)B * p->vocab_size * sizeof(float)),
-                   (int*)ws_get(WS_ARGMAX, (size_t)(p->max_seq_len + 64) * sizeof(int)), to_host ? next_slot(B).host : nullptr};
+                   (int*)ws_get(WS_ARGMAX, (size_t)(p->max_seq_len + 64) * sizeof(int)), to_host ? next_slot(B).host : nullptr,
+                   direct_rows(s, B, p->vocab_size, waits)};
         m->dir->forward(a);
-        return finish_pass(s, a.d_logits, a.d_argmax, B, p->vocab_size, PassView{}, waits, false, to_host);
+        return finish_pass(s, a.d_logits, a.d_argmax, B, p->vocab_size, PassView{}, waits, false, to_host, a.logits_host != nullptr);
     }
     // H, KVH, F, QD, KD: what THIS process computes (its tensor-parallel slice; the whole model when world == 1)
     const int D = p->dim, F = m->sh.hidden, hd = p->head_dim, H = m->sh.n_heads, KVH = m->sh.n_kv_heads;
@@ -792,9 +803,10 @@ static long enqueue_pass(int* tokens, int num_tokens, int* pos_arr, int* seq_ids
     if (m->f32) {
         if (st.d_tok_src) launch_patch_tokens(st.d_tokens, st.d_tok_src, d_argmax, T);
         wait_for_row_copies();
-        forward_f32(st, T, B, p, s, w, pool, rope, d_logits);
+        float* rows = direct_rows(s, B, V, waits);
+        forward_f32(st, T, B, p, s, w, pool, rope, d_logits, rows);
         if (B > 0) launch_argmax_ld(d_argmax, d_logits, B, V, V, argmax_direct() ? next_slot(B).host : nullptr);
-        return finish_pass(s, d_logits, d_argmax, B, V, PassView{}, waits, false, argmax_direct());
+        return finish_pass(s, d_logits, d_argmax, B, V, PassView{}, waits, false, argmax_direct(), rows != nullptr);
     }
 
     // One launch for all layers (chain.hip) when the step fits it: a decode-sized batch on an fp16 page pool,
@@ -917,6 +929,7 @@ static long enqueue_pass(int* tokens, int num_tokens, int* pos_arr, int* seq_ids
     e5.ss_in = ss_head; e5.ss_tiles = ssn; e5.d_in = D; e5.eps = eps;
     PassView view;
     bool host_written = false;
+    float* rows_host = partial || chained ? nullptr : direct_rows(s, B, V, waits);
     // no K split for the classifier (tens of thousands of rows fill the chip); from 112 output rows the
     // launcher may take the dense-tile kernel instead (0 = its own choice)
     const int head_split = B >= 112 ? 0 : 1;
@@ -924,6 +937,7 @@ static long enqueue_pass(int* tokens, int num_tokens, int* pos_arr, int* seq_ids
         WeightEntry wh{m->head, V, D, D / 32, (long)(D / 32) * TILE_HALVES, nullptr};
         e5.out = d_logits;
         e5.ldo = V;
+        e5.out_host = rows_host;
         // the classifier's tiles also report their (maximum, index) pairs: the greedy token comes from
         // a merge of those instead of a second pass over the logits
         e5.amax_out = d_argmax;
@@ -936,6 +950,7 @@ static long enqueue_pass(int* tokens, int num_tokens, int* pos_arr, int* seq_ids
             head.in_rows = st.d_out_idx;
             head.amax_pairs = e5.amax_pairs;
             head.amax_ld = e5.amax_ld;
+            head.out_host = rows_host;
             launch_gemm_thin(head.add16(m->head, wh.nb_stride, V, d_logits), PC_GEMM_HEAD);
             launch_argmax_tiles(d_argmax, e5.amax_pairs, cdiv(V, 16), B, e5.amax_ld, e5.amax_out_host);
         } else {
@@ -968,7 +983,7 @@ static long enqueue_pass(int* tokens, int num_tokens, int* pos_arr, int* seq_ids
         }
     }
 
-    return finish_pass(s, d_logits, d_argmax, B, V, view, waits, chained, host_written);
+    return finish_pass(s, d_logits, d_argmax, B, V, view, waits, chained, host_written, rows_host != nullptr);
 }
 
 void transformer_batch(int* tokens, int num_tokens, int* pos_arr, int* seq_ids, int* output_indices,

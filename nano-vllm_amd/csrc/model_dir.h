@@ -59,6 +59,7 @@ struct PassArgs {
     float* d_logits;              // [B, vocab] in HBM: to be filled
     int* d_argmax;                // [B] in HBM: to be filled; holds the previous pass's indices on entry
     int* argmax_host;             // optional: the indices also go to this page-locked array
+    float* logits_host;           // optional: the rows also go to this one
 };
 
 // A design loaded from a folder.  One subclass per design; everything a subclass needs from the rest of

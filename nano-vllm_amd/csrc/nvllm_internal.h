@@ -250,6 +250,9 @@ struct GemmEpilogue {
     // F32: out[t, ldo]
     float* out = nullptr;
     int ldo = 0;
+    // F32, optional: the rows also go to this page-locked host array, laid out like `out` (launchers of kernels that cannot store
+    // there copy them)
+    float* out_host = nullptr;
     // F32, optional: also the first index of each row's maximum over all N outputs (the sampler's greedy
     // rule, reference sampler.c:86-97) -> amax_out[t].  Every tile leaves one (maximum, index) pair per
     // token in amax_pairs[tile][amax_ld] (room for cdiv(N, 32) tiles), a small launch merges them.
@@ -501,6 +504,7 @@ void launch_argmax(int* out, const float* logits, int B, int V);
 // gathered vocabulary slices [rank][row][Vl] into logits rows [row][V]
 void launch_argmax_pairs(float2* pairs, const float* logits, int B, int n_valid, int ld, int index_base);
 void launch_argmax_merge(int* out, const float2* pairs, int W, int B);
+void copy_rows_to_host(float* dst, const float* src, size_t n);   // enqueued; dst page-locked
 void launch_argmax_ld(int* out, const float* logits, int B, int V, int ld, int* out_host = nullptr);   // rows `ld` floats apart; out_host: also to that page-locked host array
 void launch_argmax_tiles(int* out, const float2* pairs, int n_tiles, int B, int ld, int* out_host = nullptr);
 void launch_logits_unshard(float* full, const float* parts, int W, int B, int Vl, int V);

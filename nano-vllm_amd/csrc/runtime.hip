@@ -230,6 +230,8 @@ void ensure_init() {
     g_rt.inited = true;
 }
 
+void copy_rows_to_host(float* dst, const float* src, size_t n) { HIP_CHECK(hipMemcpyAsync(dst, src, n * sizeof(float), hipMemcpyDeviceToHost, rt().stream)); }
+
 }  // namespace nvllm
 
 using namespace nvllm;
@@ -291,16 +293,26 @@ void nvllm_prof_get(int cls, long long* launches, double* total_ms, double* byte
 // ---- include/backend.h ---------------------------------------------------------
 // Page-locked buffers handed out by malloc_run_state are remembered here so that
 // device_free() can release them with the right call.
-static std::vector<void*>& pinned_list() {
-    static std::vector<void*> v;
+struct Pinned {
+    void* at;
+    size_t bytes;
+};
+static std::vector<Pinned>& pinned_list() {
+    static std::vector<Pinned> v;
     return v;
 }
 void* nvllm_internal_pinned_alloc(size_t bytes) {
     ensure_init();
     void* p = nullptr;
     HIP_CHECK(hipHostMalloc(&p, bytes, hipHostMallocDefault));
-    pinned_list().push_back(p);
+    pinned_list().push_back({p, bytes});
     return p;
+}
+bool nvllm_internal_pinned_holds(const void* ptr, size_t bytes) {
+    const size_t at = (size_t)ptr;
+    for (const Pinned& p : pinned_list())
+        if (at >= (size_t)p.at && at - (size_t)p.at <= p.bytes && bytes <= p.bytes - (at - (size_t)p.at)) return true;
+    return false;
 }
 
 int device_malloc(void** ptr, size_t size) {
@@ -321,7 +333,7 @@ void device_free(void* ptr) {
     sync_streams();
     auto& pl = pinned_list();
     for (size_t i = 0; i < pl.size(); i++)
-        if (pl[i] == ptr) {
+        if (pl[i].at == ptr) {
             pl.erase(pl.begin() + (long)i);
             HIP_CHECK(hipHostFree(ptr));
             return;
