@@ -5,6 +5,7 @@
 #include "gemm_prefill_tile.h"
 #include "gemm_tile.h"
 #include "latent_kv.h"
+#include "moe_route.h"
 
 namespace nvllm {
 
@@ -24,6 +25,76 @@ __global__ __launch_bounds__(WAVES * 64) void k_gemm_b16(GemmArgs p) {
     h8_t w[RW][NBW];
     const TileIdx ix{(int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z, EPI == GemmEpilogue::LATENT_Q ? p.ride_from : (int)gridDim.x};
     gemm_tile<NBW, TB, WAVES, RW, RA, EPI, float, false, 0, OpBf16, GRP, EXP>(p, ix, lds_dyn, w, [](int) {}, (int)threadIdx.x);
+}
+
+// The same with a mixture's router (SWIGLU_A16) or its choices (F32) in the workgroups from ride_from on (moe.h).  Each is a launch of
+// 6.4 to 8 us that keeps one to four CUs busy; the products they ride on leave 80 and 128 of them idle.
+struct MoeRide {
+    GemmArgs router;
+    int router_tiles;
+    RoutePlan plan;
+    const float* z;
+    int ldz;
+};
+constexpr int ROUTER_NB = 2;   // 16-row blocks of the router and ...
+template <int NBW, int TB, int EPI>
+__global__ __launch_bounds__(NW * 64) void k_gemm_b16_moe(GemmArgs p, MoeRide r) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds_dyn[];
+    if ((int)blockIdx.x >= p.ride_from) {
+        if (blockIdx.y != 0 || blockIdx.z != 0) return;
+        if constexpr (EPI == GemmEpilogue::SWIGLU_A16) {   // ... 16 tokens each
+            const int i = (int)blockIdx.x - p.ride_from;
+            const TileIdx ix{i % r.router_tiles, 0, i / r.router_tiles, r.router_tiles};
+            h8_t w[RW][ROUTER_NB];
+            gemm_tile<ROUTER_NB, 1, NW, RW, RA, GemmEpilogue::F32, float, false, 0, OpBf16, false, false>(r.router, ix, lds_dyn, w, [](int) {}, (int)threadIdx.x);
+        } else {
+            route_sort<true, NW * 64>(r.plan, r.z, r.ldz, reinterpret_cast<int*>(lds_dyn));
+        }
+        return;
+    }
+    h8_t w[RW][NBW];
+    const TileIdx ix{(int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z, p.ride_from};
+    gemm_tile<NBW, TB, NW, RW, RA, EPI, float, false, 0, OpBf16, false, false>(p, ix, lds_dyn, w, [](int) {}, (int)threadIdx.x);
+}
+template <int NBW, int TB, int EPI>
+void launch_stream_moe(const GemmArgs& a, const MoeRide& r, int riders, const GemmPlan& pl) {
+    constexpr int shmem = gemm_tile_lds<NBW, TB, NW>();
+    static bool enabled = false;
+    if (shmem > 64 * 1024 && !enabled) {
+        HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_gemm_b16_moe<NBW, TB, EPI>), hipFuncAttributeMaxDynamicSharedMemorySize, shmem));
+        enabled = true;
+    }
+    NVLLM_LAUNCH((k_gemm_b16_moe<NBW, TB, EPI>), dim3(pl.tiles_n + riders, pl.ks, pl.tiles_t), dim3(NW * 64), shmem, a, r);
+}
+// false: this plan has no such form
+template <int EPI>
+bool launch_moe_plan(const GemmArgs& a, const GemmPlan& pl, const MoeRider& m, const GemmArgs& router) {
+    MoeRide r{};
+    int riders = 1, least = 0;   // bytes of LDS the rider needs
+    if (EPI == GemmEpilogue::SWIGLU_A16) {
+        r.router = router;
+        r.router_tiles = cdiv(router.NB, ROUTER_NB);
+        riders = r.router_tiles * router.Tb;
+        least = gemm_tile_lds<ROUTER_NB, 1, NW>();
+        if (riders > 4 * rt().num_cus) return false;
+    } else {
+        r.plan = m.plan; r.z = m.z; r.ldz = m.ldz;
+        if (m.plan.T > ROUTE_ONE) return false;
+        least = (int)route_sort_lds(m.plan.T, m.plan.E, m.plan.top);
+    }
+    if (pl.nw != NW && pl.nw != 0) return false;
+    auto go = [&](auto nbw, auto tb) {
+        constexpr int NBW = decltype(nbw)::value, TB = decltype(tb)::value;
+        if (least > gemm_tile_lds<NBW, TB, NW>()) return false;
+        launch_stream_moe<NBW, TB, EPI>(a, r, riders, pl);
+        return true;
+    };
+    using std::integral_constant;
+    if constexpr (EPI == GemmEpilogue::SWIGLU_A16)
+        if (pl.nbw == 6) return go(integral_constant<int, 6>{}, integral_constant<int, 2>{});
+    if (pl.nbw == 2) return pl.TB == 1 ? go(integral_constant<int, 2>{}, integral_constant<int, 1>{}) : go(integral_constant<int, 2>{}, integral_constant<int, 2>{});
+    if (pl.TB == 1) return go(integral_constant<int, 4>{}, integral_constant<int, 1>{});
+    return pl.TB == 2 ? go(integral_constant<int, 4>{}, integral_constant<int, 2>{}) : go(integral_constant<int, 4>{}, integral_constant<int, 4>{});
 }
 
 template <int NBW, int TB, int WAVES, int EPI, bool GRP, bool EXP = false>
@@ -96,8 +167,9 @@ void launch_dense(GemmArgs a) {
     else launch_dense_tw<EPI, GRP, 4>(a, tiles_n, tiles_t, nbuf);
 }
 
+// What is launched without its rider has the caller launch that: false.
 template <int EPI, bool GRP>
-void launch_kind(GemmArgs a, int prof_cls, double bytes, double flops) {
+bool launch_kind(GemmArgs a, int prof_cls, double bytes, double flops, const MoeRider* moe = nullptr, const GemmArgs* router = nullptr) {
     static const int pf_min_t = getenv("NVLLM_GEMM_PREFILL_T") ? atoi(getenv("NVLLM_GEMM_PREFILL_T")) : 256;
     // few features: the chip fills with token groups of 16 or 32, not with dense tiles
     const bool narrow = !GRP && EPI == GemmEpilogue::F32 && !a.e.amax_out && a.NB <= 8 && a.Tb <= 4 * rt().num_cus;
@@ -109,13 +181,13 @@ void launch_kind(GemmArgs a, int prof_cls, double bytes, double flops) {
         }
         if (EPI == GemmEpilogue::F32 && a.e.amax_out) launch_argmax_ld(a.e.amax_out, a.e.out, a.T, a.N, a.e.ldo, a.e.amax_out_host);
         if (EPI == GemmEpilogue::F32 && a.e.out_host) copy_rows_to_host(a.e.out_host, a.e.out, (size_t)a.T * a.e.ldo);
-        return;
+        return false;
     }
     if (!GRP && !narrow && !(EPI == GemmEpilogue::F32 && a.e.amax_out) && gemm_leaves_streaming(a.NB, a.Kb, a.Tb, 1, rt().num_cus)) {
         a.ksplit = 1;
         a.kb_per_split = a.Kb;
         ProfScope ps(prof_cls, bytes, flops);
-        if (launch_gemm_waves_b16(a) || launch_gemm_wide_b16(a)) return;
+        if (launch_gemm_waves_b16(a) || launch_gemm_wide_b16(a)) return false;
         ps.drop();
     }
     // a block-diagonal product has a short K and no K split; its plan is that of one group times the groups
@@ -145,15 +217,19 @@ void launch_kind(GemmArgs a, int prof_cls, double bytes, double flops) {
     a.kb_per_split = pl.kb_per_split;
     const long wgs = (long)pl.tiles_n * pl.ks * pl.tiles_t;
     if (pl.ks > 1) a.slab = (float*)ws_get(WS_SLAB, (size_t)wgs * (pl.nbw / 2) * 2 * pl.TB * 64 * 16);
-    a.close_sc1 = pl.ks > 1 && wgs <= rt().num_cus;
+    a.close_sc1 = pl.ks > 1 && wgs + (moe ? 1 : 0) <= rt().num_cus;
+    bool rode = false;
     {
         ProfScope ps(prof_cls, bytes, flops);
-        launch_stream_plan<EPI, GRP>(a, pl);
+        if constexpr (!GRP && (EPI == GemmEpilogue::SWIGLU_A16 || EPI == GemmEpilogue::F32))
+            rode = moe && launch_moe_plan<EPI>(a, pl, *moe, router ? *router : a);
+        if (!rode) launch_stream_plan<EPI, GRP>(a, pl);
     }
     if (EPI == GemmEpilogue::F32 && a.e.amax_out) {
         if (!a.e.amax_pairs || a.e.amax_ld < a.T) NVLLM_FATAL("fused arg-max needs a pair buffer of at least %d rows per tile", a.T);
         launch_argmax_tiles(a.e.amax_out, a.e.amax_pairs, cdiv(a.NB, pl.nbw), a.T, a.e.amax_ld, a.e.amax_out_host);
     }
+    return rode;
 }
 
 template <int EPI>
@@ -227,8 +303,8 @@ void launch_gemm_experts(const B16Weight& w, int experts, const __half* act, con
     }
 }
 
-void launch_gemm_b16(const B16Weight& w, const __half* act, int T, const GemmEpilogue& epi, int prof_cls, const LatentKvRider* ride) {
-    if (T <= 0) return;
+bool launch_gemm_b16(const B16Weight& w, const __half* act, int T, const GemmEpilogue& epi, int prof_cls, const LatentKvRider* ride, const MoeRider* moe) {
+    if (T <= 0) return false;
     ensure_init();
     if (w.K % 32) NVLLM_FATAL("bf16 projection: the input width %d is not padded to 32", w.K);
     const bool grp = w.groups > 1;
@@ -282,8 +358,21 @@ void launch_gemm_b16(const B16Weight& w, const __half* act, int T, const GemmEpi
     const double bytes = (double)w.N * w.K * 2.0 + (double)T * w.K * w.groups * 2.0 + out_bytes;
     const double flops = 2.0 * T * (double)w.N * w.K;
     switch (epi.kind) {
-        case GemmEpilogue::F32: launch_kind<GemmEpilogue::F32, false>(a, prof_cls, bytes, flops); break;
-        case GemmEpilogue::SWIGLU_A16: launch_kind<GemmEpilogue::SWIGLU_A16, false>(a, prof_cls, bytes, flops); break;
+        case GemmEpilogue::F32: return launch_kind<GemmEpilogue::F32, false>(a, prof_cls, bytes, flops, moe);
+        case GemmEpilogue::SWIGLU_A16: {
+            GemmArgs router = a;
+            if (moe) {
+                const B16Weight& r = *moe->router;
+                if (r.K != w.K || r.groups != 1) NVLLM_FATAL("router of %d inputs beside a projection of %d", r.K, w.K);
+                router.W = r.tiles;
+                router.NB = cdiv(r.N, 16);
+                router.N = r.N;
+                router.ksplit = 1;
+                router.kb_per_split = router.Kb;
+                router.e = moe->router_epi;
+            }
+            return launch_kind<GemmEpilogue::SWIGLU_A16, false>(a, prof_cls, bytes, flops, moe, &router);
+        }
         case GemmEpilogue::TILE_B16:
             if (grp) launch_kind<GemmEpilogue::TILE_B16, true>(a, prof_cls, bytes, flops);
             else launch_kind<GemmEpilogue::TILE_B16, false>(a, prof_cls, bytes, flops);
@@ -299,6 +388,7 @@ void launch_gemm_b16(const B16Weight& w, const __half* act, int T, const GemmEpi
         case GemmEpilogue::HYPER_4: launch_kind<GemmEpilogue::HYPER_4, false>(a, prof_cls, bytes, flops); break;
         default: NVLLM_FATAL("this epilogue belongs to fp16 models");
     }
+    return false;
 }
 
 }  // namespace nvllm

@@ -579,10 +579,17 @@ void HybridModel::forward_b16(const PassArgs& a, const StepArrays& st) {
             const int ldz = pad32(f.experts + 1);
             GemmEpilogue ez = normed(GemmEpilogue::F32);
             ez.out = z; ez.ldo = ldz;
-            launch_gemm_b16(w.router, act, T, ez, PC_GEMM_ROUTER);
             const ExpertGroups groups = expert_groups(T, f.experts, f.top, w.experts_up, w.experts_down);
             const RoutePlan plan = route_plan(route_mem, T, f.experts, f.top, groups.pad);
-            launch_route(plan, z, ldz);
+            // the shared expert first: router and choice ride on its products where there are few tokens (64: 14 us a layer)
+            MoeRider rider;
+            rider.router = &w.router; rider.router_epi = ez; rider.plan = plan; rider.z = z; rider.ldz = ldz;
+            GemmEpilogue su = normed(GemmEpilogue::SWIGLU_A16), sd;
+            su.a16_out = hid_shared;
+            sd.kind = GemmEpilogue::F32;
+            sd.out = y_shared; sd.ldo = Dp_;
+            if (!f.shared_ff || !launch_gemm_b16(w.shared_up, act, T, su, PC_GEMM_SHARED_UP, nullptr, &rider)) launch_gemm_b16(w.router, act, T, ez, PC_GEMM_ROUTER);
+            if (!f.shared_ff || !launch_gemm_b16(w.shared_down, hid_shared, T, sd, PC_GEMM_SHARED_DOWN, nullptr, &rider)) launch_route(plan, z, ldz);
             ExpertRows er{plan.block_expert, plan.source, plan.capacity, plan.pad, T * f.top, groups.wide};
             GemmEpilogue eu = normed(GemmEpilogue::SWIGLU_A16);
             eu.ss_gather = plan.source; eu.row_weight = plan.weight; eu.a16_out = wide;
@@ -596,15 +603,6 @@ void HybridModel::forward_b16(const PassArgs& a, const StepArrays& st) {
             ed.kind = GemmEpilogue::F32;
             ed.out = y_experts; ed.ldo = Dp_;
             launch_gemm_experts(w.experts_down, f.experts, wide, er, ed, PC_GEMM_EXPERT_DOWN);
-            if (f.shared_ff) {
-                GemmEpilogue su = normed(GemmEpilogue::SWIGLU_A16);
-                su.a16_out = hid_shared;
-                launch_gemm_b16(w.shared_up, act, T, su, PC_GEMM_SHARED_UP);
-                GemmEpilogue sd;
-                sd.kind = GemmEpilogue::F32;
-                sd.out = y_shared; sd.ldo = Dp_;
-                launch_gemm_b16(w.shared_down, hid_shared, T, sd, PC_GEMM_SHARED_DOWN);
-            }
             MoeCombine c{};
             c.x = x; c.rows = y_experts; c.row_of = plan.row_of; c.top = f.top; c.shared = f.shared_ff ? y_shared : nullptr;
             c.z = z; c.ldz = ldz; c.z_col = f.experts; c.gain = next_gain(run, 1); c.out_b16 = act; c.ss = ss; c.ld = Dp_;

@@ -29,6 +29,16 @@ RoutePlan route_plan(int* mem, int T, int E, int top, int pad);
 // z: [T][ldz] router logits in columns 0 .. E-1; the `top` largest (the first of equals) are chosen
 void launch_route(const RoutePlan& r, const float* z, int ldz);
 
+// Work that needs a fraction of the chip, beside the shared expert's products on the CUs those leave idle: the router beside the first,
+// the choice beside the second (launch_gemm_b16).
+struct MoeRider {
+    const B16Weight* router = nullptr;   // SWIGLU_A16 launches: its activations are the launch's
+    GemmEpilogue router_epi;             // F32
+    RoutePlan plan{};                    // F32 launches
+    const float* z = nullptr;
+    int ldz = 0;
+};
+
 // the rows x * gain of a batch in the plan's order, as activation tiles (x [T][ld])
 void launch_expert_rows(__half* dst, const float* x, const float* gain, const RoutePlan& r, int ld);
 

@@ -3,13 +3,12 @@
 
 #include <algorithm>
 
-#include "attn_tile.h"
 #include "gemm_common.h"
+#include "moe_route.h"
 
 namespace nvllm {
 
 namespace {
-constexpr int ROUTE_ONE = 256;      // up to here one workgroup routes and sorts
 constexpr int MAX_EXPERTS = 4096;
 }
 
@@ -46,142 +45,15 @@ RoutePlan route_plan(int* mem, int T, int E, int top, int pad) {
     return r;
 }
 
-// Maximum over a wave, in every lane, on the vector unit alone (many waves of one CU would queue for the LDS crossbar):
-// rotations within rows of 16 lanes, then the rows.
-template <int N>
-__device__ __forceinline__ float row_rotate(float x) {
-    const int v = __builtin_bit_cast(int, x);
-    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(v, v, 0x120 + N, 0xf, 0xf, false));
-}
-__device__ __forceinline__ float wave_max(float x) {
-    x = fmaxf(x, row_rotate<8>(x));
-    x = fmaxf(x, row_rotate<4>(x));
-    x = fmaxf(x, row_rotate<2>(x));
-    x = fmaxf(x, row_rotate<1>(x));
-    return rows_max(x);
-}
-
-// One wave chooses for one token: `top` times the best of what comes after the previous choice in the order
-// (score descending, index ascending).
-__device__ __forceinline__ void route_token(const RoutePlan& r, const float* __restrict__ z, int t, int lane) {
-    float last = INFINITY;
-    int last_e = -1;
-    for (int j = 0; j < r.top; j++) {
-        float best = -INFINITY;
-        int best_e = 0x7fffffff;
-        for (int e = lane; e < r.E; e += 64) {
-            const float v = z[e];
-            const bool open = v < last || (v == last && e > last_e);
-            if (open && v > best) {
-                best = v;
-                best_e = e;
-            }
-        }
-        const float top = wave_max(best);
-        int first = best == top ? best_e : 0x7fffffff;
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) first = min(first, __shfl_xor(first, o, 64));
-        best = top;
-        best_e = first;
-        if (best_e >= r.E) best_e = 0;   // (no number compares: NaN logits)
-        last = best;
-        last_e = best_e;
-        if (lane == 0) {
-            r.choice[(size_t)t * r.top + j] = best_e;
-            r.score[(size_t)t * r.top + j] = 1.f / (1.f + expf(-best));
-        }
-    }
-}
 __global__ __launch_bounds__(256) void k_route(RoutePlan r, const float* __restrict__ z, int ldz) {
     const int t = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (t < r.T) route_token(r, z + (size_t)t * ldz, t, threadIdx.x & 63);
 }
 
-// One workgroup: counts, segment starts, then every choice takes a row of its expert's segment (in any order: a row's
-// result does not depend on its place).
 template <bool CHOOSE>
 __global__ __launch_bounds__(1024) void k_route_sort(RoutePlan r, const float* __restrict__ z, int ldz) {
-    extern __shared__ int lds_r[];   // counts [E], next free row [E], segment start [E + 1], CHOOSE: choices and scores [T * top]
-    int* count = lds_r;
-    int* cursor = count + r.E;
-    int* start = cursor + r.E;
-    const int tid = threadIdx.x, lane = tid & 63, pairs = r.T * r.top;
-    int *choice = CHOOSE ? start + r.E + 1 : r.choice, *out_choice = r.choice;
-    float* out_score = r.score;
-    float* score = CHOOSE ? reinterpret_cast<float*>(choice + pairs) : r.score;
-    for (int e = tid; e < r.E; e += 1024) count[e] = 0;
-    if (CHOOSE) {
-        r.choice = choice;   // (route_token fills the LDS copies)
-        r.score = score;
-        if (r.E <= 64) {   // a logit per lane, four tokens at a time
-            for (int t0 = tid >> 6; t0 < r.T; t0 += 64) {
-                float v[4];
-#pragma unroll
-                for (int u = 0; u < 4; u++) v[u] = lane < r.E ? z[(size_t)min(t0 + 16 * u, r.T - 1) * ldz + lane] : -INFINITY;
-                for (int j = 0; j < r.top; j++) {
-                    float best[4];
-#pragma unroll
-                    for (int u = 0; u < 4; u++) best[u] = wave_max(v[u]);
-#pragma unroll
-                    for (int u = 0; u < 4; u++) {
-                        const int t = t0 + 16 * u;
-                        const unsigned long long at = __ballot(v[u] == best[u] && lane < r.E);
-                        const int e = at ? __ffsll(at) - 1 : 0;   // (no number compares: NaN logits)
-                        if (lane == e) v[u] = -INFINITY;
-                        if (lane == 0 && t < r.T) {
-                            choice[t * r.top + j] = e;
-                            score[t * r.top + j] = 1.f / (1.f + expf(-best[u]));
-                        }
-                    }
-                }
-            }
-        } else {
-            for (int t = tid >> 6; t < r.T; t += 16) route_token(r, z + (size_t)t * ldz, t, lane);
-        }
-    }
-    __syncthreads();
-    for (int i = tid; i < pairs; i += 1024) atomicAdd(count + choice[i], 1);
-    __syncthreads();
-    if (tid < 64) {   // the first wave sums the padded counts
-        int base = 0;
-        for (int e0 = 0; e0 < r.E; e0 += 64) {
-            const int e = e0 + tid, n = e < r.E ? (count[e] + r.pad - 1) / r.pad * r.pad : 0;
-            int sum = n;
-#pragma unroll
-            for (int o = 1; o < 64; o <<= 1) {
-                const int v = __shfl_up(sum, o, 64);
-                if (tid >= o) sum += v;
-            }
-            if (e < r.E) start[e] = cursor[e] = base + sum - n;
-            base += __shfl(sum, 63, 64);
-        }
-        if (tid == 0) start[r.E] = base;
-    }
-    __syncthreads();   // the last one: from here on everybody only writes results (a barrier would wait for the stores)
-    const int used = start[r.E];
-    for (int b = used / 16 + tid; b < r.capacity / 16; b += 1024) r.block_expert[b] = -1;
-    for (int i = used + tid; i < r.capacity; i += 1024) {   // (a tile may look up rows behind its own: they name a token too)
-        r.source[i] = 0;
-        r.weight[i] = 0.f;
-    }
-    for (int e = tid >> 4; e < r.E; e += 64) {   // 16 threads per expert: its blocks, and the padding of its segment
-        const int lo = start[e], hi = start[e + 1], n = count[e];
-        for (int b = lo / 16 + (tid & 15); b < hi / 16; b += 16) r.block_expert[b] = e;
-        for (int i = lo + n + (tid & 15); i < hi; i += 16) {
-            r.source[i] = 0;
-            r.weight[i] = 0.f;
-        }
-    }
-    for (int i = tid; i < pairs; i += 1024) {
-        const int row = atomicAdd(cursor + choice[i], 1);
-        r.source[row] = i / r.top;
-        r.weight[row] = score[i];
-        r.row_of[i] = row;
-        if (CHOOSE) {
-            out_choice[i] = choice[i];
-            out_score[i] = score[i];
-        }
-    }
+    extern __shared__ int lds_r[];
+    route_sort<CHOOSE, 1024>(r, z, ldz, lds_r);
 }
 
 void launch_route(const RoutePlan& r, const float* z, int ldz) {
@@ -189,7 +61,7 @@ void launch_route(const RoutePlan& r, const float* z, int ldz) {
     if (r.E < 1 || r.E > MAX_EXPERTS || r.top < 1 || r.top > r.E) NVLLM_FATAL("routing: %d of %d experts per token", r.top, r.E);
     const size_t lds = ((size_t)3 * r.E + 1) * sizeof(int);
     const double bytes = (double)r.T * (r.E * 4.0 + r.top * 20.0);
-    const size_t lds_one = lds + (size_t)r.T * r.top * 8;
+    const size_t lds_one = route_sort_lds(r.T, r.E, r.top);
     if (r.T <= ROUTE_ONE && lds_one <= 64 * 1024) {
         ProfScope ps(PC_ROUTE, bytes, 0);
         NVLLM_LAUNCH((k_route_sort<true>), dim3(1), dim3(1024), lds_one, r, z, ldz);

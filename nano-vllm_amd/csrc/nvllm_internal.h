@@ -379,7 +379,10 @@ struct B16Weight {
 };
 static inline size_t b16_halves(int tokens, int K) { return (size_t)cdiv(tokens, 16) * cdiv(K, 32) * TILE_HALVES; }
 struct LatentKvRider;   // gemm_common.h: cache rows written by extra workgroups of a LATENT_Q launch
-void launch_gemm_b16(const B16Weight& w, const __half* act, int T, const GemmEpilogue& epi, int prof_cls, const LatentKvRider* ride = nullptr);
+struct MoeRider;        // moe.h: a router beside a SWIGLU_A16 launch, or its choices and their sorting beside an F32 one
+// `moe`: true is returned if it rode along (few tokens), false if the caller has to launch it
+bool launch_gemm_b16(const B16Weight& w, const __half* act, int T, const GemmEpilogue& epi, int prof_cls, const LatentKvRider* ride = nullptr,
+                     const MoeRider* moe = nullptr);
 // Rows sorted by expert (moe.h): every group of `pad` rows meets the matrix of ONE expert.
 struct ExpertRows {
     const int* block_expert;   // [capacity / 16] expert of each 16-row block, -1: no rows (the same within a group)

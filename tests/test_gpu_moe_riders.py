@@ -1,0 +1,23 @@
+"""Passes of few tokens, whose router and choice of experts ride on the shared expert's products: at the edges of a token block, of the
+chosen tile heights and of the passes that launch them apart; routers of one and of several feature tiles."""
+import numpy as np
+import pytest
+
+from nvllm_amd import synth
+from tests import hybrid_oracle as O
+from tests import hybrid_util as U
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("experts,shared", [(5, 40), (40, 96), (70, 64)])
+def test_passes_of_few_tokens(hip, tmp_path, experts, shared):
+    window = synth.window_mixer(4, 2, 16, 16, size=48, keep_first=4)
+    cfg = synth.hybrid_config(128, 211, [(window, synth.expert_mlp(48, experts, 2, shared)), (window, synth.expert_mlp(48, experts, 2, shared))])
+    path, cfg, weights = U.model(tmp_path, "riders", seed=experts, cfg=cfg)
+    eng = U.engine(hip, path, False, slots=1)
+    for n in (1, 16, 17, 64, 65, 255, 256):
+        seq = U.tokens(n, 211, n)
+        got = U.feed_all(eng, [[(0, n)]], {0: seq})[0]
+        assert U.error(got, O.forward(cfg, weights, seq)) < U.limit(False), n
+    eng.close()
