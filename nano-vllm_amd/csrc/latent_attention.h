@@ -45,10 +45,13 @@ struct LatentAttn {
     int H;
     float* out_f32;        // fp32 pool: [T][H][rank]
     __half* out_b16;       // bf16 pool: activation tiles of [T, H * rank_ld]
+    const B16Weight* uv = nullptr;   // optional, bf16 pool: W_uv, a group of vdim_ld rows per head, and ...
+    __half* values = nullptr;        // ... activation tiles of [T, H * vdim_ld] for its products
 };
 constexpr int LATENT_RUN = 32;   // stage_step(attn_ct, multi_first): tokens per run at most
-// only_alone: nothing but the tokens that are their sequence's only one
-void launch_latent_attention(const LatentAttn& a, const StepArrays& st, bool only_alone = false);
+// only_alone: nothing but the tokens that are their sequence's only one.  True: the results went through W_uv into `values` (out_b16 is
+// not written); false: the caller multiplies out_b16
+bool launch_latent_attention(const LatentAttn& a, const StepArrays& st, bool only_alone = false);
 
 // fp32 models: q [T][H * (dim + rot)] -> rows [T][H][rank + rot] (W_uk [H * dim, rank] absorbed, rotated part turned)
 void launch_latent_q_f32(float* rows, const float* q, const float* uk, const float2* rope, const int* pos, int T, int H, int dim, int rot, int rank);

@@ -548,6 +548,107 @@ __global__ __launch_bounds__(128) void k_latent_combine(const float* __restrict_
     }
 }
 
+// The same for TW tokens and one head, and the product with the head's W_uv (vt blocks of 16 features, a wave each) in the same
+// launch: the merged rows go to LDS as bf16 and from there into the product.  A wave merges a token, lanes holding the slices' maxima and
+// four neighbouring values; the weights are requested first.  Bound by what a CU takes in: 4 KiB per token and pair of slices, and W_uv.
+// 64 tokens, 32 heads, 4 slices of 512 values: merge 5.8 us + product 4.6 before, 7.1 so; five tokens in 9 slices 6.0 + 5.1 before, 6.8.
+constexpr int VALUE_SLOTS = 128, VALUE_KC = 16, VALUE_WAVES = 8;   // tiles of a latent that a wave has registers for
+struct LatentValueArgs {
+    const float *part_acc, *part_ml, *sink;
+    const int4* runs;
+    int slots, run_ld, H, nsplit, rank_ld, vt;
+    const __half* uv;   // [H * vt][rank_ld / 32] tiles
+    __half* out;
+    int Kb_out;
+};
+template <int TW, int U>   // U: slices requested at once
+__global__ __launch_bounds__(VALUE_WAVES * 64) void k_latent_value(LatentValueArgs a) {
+    constexpr int LD = VALUE_KC * 32 + 8;   // halves of a row: 16 rows' pieces of 16 bytes meet every bank once
+    constexpr int D = VALUE_KC * 32 / 256;  // pieces of four values a lane has
+    __shared__ __attribute__((aligned(16))) __bf16 rows[16][LD];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int x = lane & 15, g = lane >> 4;
+    const int h = (int)blockIdx.x, slot0 = (int)blockIdx.y * TW, nc = a.rank_ld / 32;
+    float m, l;   // lane s: slice s (at most 64)
+    f4_t v[U][D];
+    // (a slot past the last is merged again and not stored)
+    auto place = [&](int i) { return (size_t)min(slot0 + i, a.slots - 1) * a.H + h; };
+    auto request_ml = [&](int i) {
+        const float2 ml = *reinterpret_cast<const float2*>(a.part_ml + (place(i) * a.nsplit + min(lane, a.nsplit - 1)) * 2);
+        m = ml.x;
+        l = ml.y;
+    };
+    auto request = [&](int i, int s0) {
+        const float* acc = a.part_acc + place(i) * a.nsplit * a.rank_ld;
+#pragma unroll
+        for (int u = 0; u < U; u++)
+#pragma unroll
+            for (int d = 0; d < D; d++)
+                v[u][d] = *reinterpret_cast<const f4_t*>(acc + (size_t)min(s0 + u, a.nsplit - 1) * a.rank_ld + min(4 * (lane + 64 * d), a.rank_ld - 4));
+    };
+    // requests are answered in order: the first token's slices, then the weights, which are needed last
+    const float sk = a.sink[h] * 1.44269504088896340736f;
+    request_ml(wave);
+    request(wave, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    h8_t w[VALUE_KC];
+    {
+        const __half* W = a.uv + (size_t)(h * a.vt + min(wave, a.vt - 1)) * nc * TILE_HALVES + lane * 8;
+        if (wave < a.vt) {
+#pragma unroll
+            for (int k = 0; k < VALUE_KC; k++) w[k] = *reinterpret_cast<const h8_t*>(W + (size_t)min(k, nc - 1) * TILE_HALVES);
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = wave; i < TW; i += VALUE_WAVES) {
+        if (i != wave) {
+            request_ml(i);
+            request(i, 0);
+        }
+        if (lane >= a.nsplit) {
+            m = -INFINITY;
+            l = 0.f;
+        }
+        float top = fmaxf(m, sk);
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) top = fmaxf(top, __shfl_xor(top, o, 64));
+        float f = __builtin_amdgcn_exp2f(m - top), den = l * f;   // a slice without pages: exp2(-inf) = 0, its sums are zeros
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) den += __shfl_xor(den, o, 64);
+        f *= 1.0f / (den + __builtin_amdgcn_exp2f(sk - top));
+        f4_t o[D] = {};
+        for (int s0 = 0; s0 < a.nsplit; s0 += U) {
+            if (s0) request(i, s0);
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const float fs = s0 + u < a.nsplit ? __shfl(f, s0 + u, 64) : 0.f;
+#pragma unroll
+                for (int d = 0; d < D; d++)
+#pragma unroll
+                    for (int r = 0; r < 4; r++) o[d][r] = s0 + u < a.nsplit ? fmaf(v[u][d][r], fs, o[d][r]) : o[d][r];
+            }
+        }
+#pragma unroll
+        for (int d = 0; d < D; d++) {
+            const float z[4] = {o[d][0], o[d][1], o[d][2], o[d][3]};
+            if (4 * (lane + 64 * d) < a.rank_ld) *reinterpret_cast<b4_t*>(&rows[i][4 * (lane + 64 * d)]) = to_b4(z);
+        }
+    }
+    __syncthreads();
+    if (wave >= a.vt) return;
+    f4_t y[2] = {};   // (two chains)
+#pragma unroll
+    for (int k = 0; k < VALUE_KC; k++)
+        if (k < nc) y[k & 1] = OpBf16::mfma(w[k], *reinterpret_cast<const h8_t*>(&rows[TW == 16 ? x : x & (TW - 1)][32 * k + 8 * g]), y[k & 1]);
+    const int slot = slot0 + x;
+    if (x >= TW || slot >= a.slots) return;
+    const int4 run = a.runs[slot / a.run_ld];
+    if (slot % a.run_ld >= run.y) return;
+    const float z[4] = {y[0][0] + y[1][0], y[0][1] + y[1][1], y[0][2] + y[1][2], y[0][3] + y[1][3]};
+    store_b16_4(a.out, a.Kb_out, run.x + slot % a.run_ld, (h * a.vt + wave) * 16 + 4 * g, z);
+}
+
 template <int RC, int NT, int C, int WC, bool EXACT_ONLY = false>
 static void launch_latent_c(const LatentKArgs& k, long units) {
     const size_t lds = latent_attn_lds(k.chunks, C * WC);
@@ -572,8 +673,8 @@ static void launch_latent_rc(const LatentKArgs& k, long units, int columns) {
     else launch_latent_c<RC, NT, 2, 2, (RC > 10)>(k, units);
 }
 
-void launch_latent_attention(const LatentAttn& a, const StepArrays& st, bool only_alone) {
-    if (st.T <= 0) return;
+bool launch_latent_attention(const LatentAttn& a, const StepArrays& st, bool only_alone) {
+    if (st.T <= 0) return false;
     const LatentPool& P = a.pool;
     const int row = P.row(), chunks = row / 32, vt = cdiv(P.rank_ld, 64);   // value tiles per wave
     // algorithmic work: every sequence's rows read once; per (token, key, head) the two products
@@ -590,7 +691,7 @@ void launch_latent_attention(const LatentAttn& a, const StepArrays& st, bool onl
         if (P.elem_bytes == 2) launch_latent_any<true, 1>(a, st);
         else if (P.rank % 4 || row % 4) launch_latent_any<false, 1>(a, st);
         else launch_latent_any<false, 4>(a, st);
-        return;
+        return false;
     }
     LatentKArgs k{};
     k.base = (const __half*)P.base;
@@ -606,59 +707,82 @@ void launch_latent_attention(const LatentAttn& a, const StepArrays& st, bool onl
     k.out = a.out_b16;
     k.Kb_out = a.H * P.rank_ld / 32;
     // prompt portions and single tokens want differently shaped items: a launch each when the batch has both
-    const int n_single = st.n_runs - st.n_multi;
-    auto launch = [&](const int* runs, int n_runs, int max_run, double bytes, double flops) {
-        if (n_runs <= 0) return;
+    struct Shape {
+        const int4* runs;
+        int n_runs, max_run, W, ct, nsplit;
+        long items;
+        double bytes, flops;
+    };
+    auto shape = [&](const int* runs, int n_runs, int max_run, double bytes, double flops) {
+        Shape s{(const int4*)runs, n_runs, max_run, 0, 1, 1, 0, bytes, flops};
+        if (n_runs <= 0) return s;
         // columns per item: 64, or 32 or 16 when no item would fill more
         // (64 columns of the widest class fit the register file only when the row is exactly that class's)
         const bool wide = chunks > 10 || vt > 4, exact = chunks == 18 && vt * 64 == P.rank_ld;
-        const int W = a.H * max_run <= 16 ? 16 : a.H * max_run <= 32 || (wide && !exact) ? 32 : 64;
+        s.W = a.H * max_run <= 16 ? 16 : a.H * max_run <= 32 || (wide && !exact) ? 32 : 64;
         // up to 16 tokens per item (so that a column group is one head's neighbouring tokens), more only when there are few heads
-        int ct = 1;
-        while (ct < 16 && ct < max_run) ct *= 2;
-        k.runs = (const int4*)runs;
-        k.run_ld = max_run;
-        k.HG = a.H < W / ct ? a.H : W / ct;
-        k.NG = cdiv(a.H, k.HG);
-        k.CT = W / k.HG;
-        k.n_sub = cdiv(max_run, k.CT);
+        while (s.ct < 16 && s.ct < max_run) s.ct *= 2;
+        const int HG = a.H < s.W / s.ct ? a.H : s.W / s.ct;
         // slices of pages until every CU has a workgroup, eight pages per slice at least
-        const long items = (long)n_runs * k.n_sub * k.NG;
+        s.items = (long)n_runs * cdiv(max_run, s.W / HG) * cdiv(a.H, HG);
         const int npages = st.max_pos / LATENT_PAGE + 1;
-        int nsplit = (int)((rt().num_cus + items / 2) / items);
-        if (nsplit > cdiv(npages, 8)) nsplit = cdiv(npages, 8);
-        if (nsplit > 64) nsplit = 64;
-        if (nsplit < 1) nsplit = 1;
-        k.nsplit = nsplit;
-        const size_t rows = (size_t)n_runs * max_run * a.H * nsplit;
-        if (nsplit > 1) {
+        s.nsplit = (int)((rt().num_cus + s.items / 2) / s.items);
+        s.nsplit = std::max(1, std::min(std::min(s.nsplit, cdiv(npages, 8)), 64));
+        return s;
+    };
+    auto launch = [&](const Shape& s, bool through_uv) {
+        if (s.n_runs <= 0) return;
+        k.runs = s.runs;
+        k.run_ld = s.max_run;
+        k.HG = a.H < s.W / s.ct ? a.H : s.W / s.ct;
+        k.NG = cdiv(a.H, k.HG);
+        k.CT = s.W / k.HG;
+        k.n_sub = cdiv(s.max_run, k.CT);
+        k.nsplit = s.nsplit;
+        const size_t rows = (size_t)s.n_runs * s.max_run * a.H * s.nsplit;
+        if (s.nsplit > 1) {
             float* part = (float*)ws_get(WS_ATT_PART, rows * (P.rank_ld + 2) * sizeof(float));
             k.part_acc = part;
             k.part_ml = part + rows * P.rank_ld;
         }
         {
-            ProfScope ps(max_run == 1 ? PC_LATENT_ATTN_TOK : PC_LATENT_ATTN, bytes, flops);
-            const long units = items * nsplit;
-            if (chunks <= 4 && vt <= 1) launch_latent_rc<4, 1>(k, units, W);
-            else if (chunks <= 6 && vt <= 2) launch_latent_rc<6, 2>(k, units, W);
-            else if (chunks <= 10 && vt <= 4) launch_latent_rc<10, 4>(k, units, W);
-            else launch_latent_rc<18, 8>(k, units, W);
+            ProfScope ps(s.max_run == 1 ? PC_LATENT_ATTN_TOK : PC_LATENT_ATTN, s.bytes, s.flops);
+            const long units = s.items * s.nsplit;
+            if (chunks <= 4 && vt <= 1) launch_latent_rc<4, 1>(k, units, s.W);
+            else if (chunks <= 6 && vt <= 2) launch_latent_rc<6, 2>(k, units, s.W);
+            else if (chunks <= 10 && vt <= 4) launch_latent_rc<10, 4>(k, units, s.W);
+            else launch_latent_rc<18, 8>(k, units, s.W);
         }
-        if (nsplit > 1) {
-            ProfScope ps(PC_LATENT_COMBINE, (double)rows * (P.rank_ld + 2) * 4.0, 0);
-            NVLLM_LAUNCH(k_latent_combine, dim3((unsigned)n_runs * max_run * a.H), dim3(128), 0, k.part_acc, k.part_ml, a.sink, k.runs, max_run, a.H, nsplit,
-                         P.rank_ld, a.out_b16, k.Kb_out);
+        if (s.nsplit <= 1) return;
+        const int slots = s.n_runs * s.max_run;
+        ProfScope ps(PC_LATENT_COMBINE, (double)rows * (P.rank_ld + 2) * 4.0, through_uv ? 2.0 * slots * (double)a.uv->N * P.rank_ld : 0);
+        if (through_uv) {
+            LatentValueArgs v{k.part_acc, k.part_ml, a.sink, k.runs, slots, s.max_run, a.H, s.nsplit, P.rank_ld, a.uv->N / a.H / 16, a.uv->tiles, a.values, a.uv->N / 32};
+            const int tw = (long)cdiv(slots, 8) * a.H <= rt().num_cus ? 8 : 16;   // eight tokens a workgroup where that leaves one for every CU
+            const dim3 grid(a.H, cdiv(slots, tw)), block(VALUE_WAVES * 64);
+            if (tw == 8 && s.nsplit <= 4) NVLLM_LAUNCH((k_latent_value<8, 4>), grid, block, 0, v);
+            else if (tw == 8) NVLLM_LAUNCH((k_latent_value<8, 8>), grid, block, 0, v);
+            else NVLLM_LAUNCH((k_latent_value<16, 4>), grid, block, 0, v);
+        } else {
+            NVLLM_LAUNCH(k_latent_combine, dim3((unsigned)slots * a.H), dim3(128), 0, k.part_acc, k.part_ml, a.sink, k.runs, s.max_run, a.H, s.nsplit, P.rank_ld, a.out_b16,
+                         k.Kb_out);
         }
     };
-    if (only_alone) {
-        launch(st.d_runs + 4 * (st.n_runs - st.n_alone), st.n_alone, 1, bytes_of((double)st.kv_rows_alone, st.n_alone),
-               2.0 * (double)st.kv_rows_alone * a.H * (row + P.rank_ld));
-        return;
-    }
+    const int n_single = st.n_runs - st.n_multi;
     const double single_bytes = bytes_of((double)st.kv_rows_single, n_single);
     const double single_flops = 2.0 * (double)st.kv_rows_single * a.H * (row + P.rank_ld);
-    launch(st.d_runs, st.n_multi, st.max_run, bytes - single_bytes, flops - single_flops);
-    launch(st.d_runs + 4 * st.n_multi, n_single, 1, single_bytes, single_flops);
+    const Shape parts[2] = {
+        only_alone ? shape(nullptr, 0, 1, 0, 0) : shape(st.d_runs, st.n_multi, st.max_run, bytes - single_bytes, flops - single_flops),
+        only_alone ? shape(st.d_runs + 4 * (st.n_runs - st.n_alone), st.n_alone, 1, bytes_of((double)st.kv_rows_alone, st.n_alone),
+                           2.0 * (double)st.kv_rows_alone * a.H * (row + P.rank_ld))
+                   : shape(st.d_runs + 4 * st.n_multi, n_single, 1, single_bytes, single_flops)};
+    // merged and multiplied in one launch: every part in slices, few enough tokens that reading W_uv for each sixteen of them costs
+    // less than a launch, rows and heads that the kernel has registers for
+    bool through_uv = a.uv && a.uv->groups == a.H && a.uv->N % (16 * a.H) == 0 && a.uv->N / a.H / 16 <= VALUE_WAVES && P.rank_ld <= VALUE_KC * 32 && a.uv->K == P.rank_ld && a.uv->N % 32 == 0;
+    for (const Shape& s : parts)
+        if (s.n_runs > 0 && (s.nsplit <= 1 || s.n_runs * s.max_run > VALUE_SLOTS)) through_uv = false;
+    for (const Shape& s : parts) launch(s, through_uv);
+    return through_uv;
 }
 
 // ------------------------------------------------------------------ fp32 head products

@@ -430,7 +430,8 @@ void LatentHyperModel::forward_b16(const PassArgs& a, const StepArrays& st, cons
             launch_gemm_b16(w.uk, hid + b16_halves(t0, m.heads * dimp), n, e3, PC_GEMM_ABSORB);
             LatentAttn at{};
             at.pool = pl; at.q = q; at.sink = w.sink; at.scale = m.scale; at.H = m.heads; at.out_b16 = latents;
-            launch_latent_attention(at, st, only_alone);
+            at.uv = &w.uv; at.values = out;
+            if (launch_latent_attention(at, st, only_alone)) return;
             GemmEpilogue e4;
             e4.kind = GemmEpilogue::TILE_B16;
             e4.a16_out = out + b16_halves(t0, m.heads * vp);
