@@ -480,6 +480,7 @@ int attn_tokens_per_item(int H, int KVH) {
     return 16 / gt;
 }
 
+constexpr int MERGE_PAGES = 20;
 void launch_paged_attention(const AttnArgs& a) {
     if (a.T <= 0) return;
     const int CT = attn_tokens_per_item(a.H, a.KVH), GT = 16 / CT;
@@ -507,10 +508,24 @@ void launch_paged_attention(const AttnArgs& a) {
     const int min_pages = wg_items ? 8 : 2;   // pages per slice worth a slice
     if (nsplit > (pages + min_pages - 1) / min_pages) nsplit = (pages + min_pages - 1) / min_pages;
     if (nsplit < 1) nsplit = 1;
+    // ... and only where the walk that slices take off an item costs more than the merge's launch; more so where the slices are more than
+    // one round of the chip, two of which never pay.  A pass of TinyLlama-1.1B, one row with 150, 300, 500, 700 cached: sliced 1,052, 1,050,
+    // 1,048, 1,058 us, whole 1,005, 1,020, 1,044, 1,079; twelve 1,165, 1,166, 1,167, 1,185 and 1,131, 1,137, 1,169, 1,195; 30 with 1,050:
+    // 1,357 and 1,372.  Of more than a round: 18 rows with 480, 800: 1,255, 1,273 and 1,230, 1,277; 25 with 400, 640, 1,000: 1,288, 1,315,
+    // 1,348 and 1,251, 1,287, 1,340; 40 with 500, 1,050, 2,000, 3,000: 1,443, 1,530, 1,659, 1,809 and 1,381, 1,472, 1,628, 1,790
+    if (wg_items && env_units <= 0) {
+        const bool rounds = base_items * nsplit > target;
+        const long walk = (long)pages * std::max(a.hd, 64) / 64;
+        if ((rounds && nsplit == 2) || walk * (nsplit - 1) <= (rounds && nsplit <= 4 ? 32 : 20) * nsplit) nsplit = 1;
+    }
     // fp32 rows, 2..8 slices per item: the slices of an item share a workgroup (4 or 8 waves) and merge in LDS
     // instead of going through memory and k_attn_combine (NVLLM_ATTN_MERGE=0 keeps the two launches)
     static const int env_merge = getenv("NVLLM_ATTN_MERGE") ? atoi(getenv("NVLLM_ATTN_MERGE")) : 1;
+    // ... and so do more of them where eight waves have few pages each (the page that more slices would take off a wave costs less
+    // than the merge's launch) and there are more than a few items: stories42M, a prompt of 301 tokens 615 -> 589 us, of 310 on fp16 weights
+    // 428 -> 397; with 32 pages rows lose (3 rows at 700 cached: 317 -> 346), eight items gain nothing
     int merge_waves = 0;
+    if (!wg_items && env_merge && nsplit > 8 && pages <= MERGE_PAGES && base_items >= 16) nsplit = 8;
     if (!wg_items && env_merge && nsplit > 1 && nsplit <= 8) {
         merge_waves = nsplit <= 4 ? 4 : 8;
         nsplit = merge_waves;

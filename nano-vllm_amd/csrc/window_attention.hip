@@ -904,6 +904,7 @@ static void launch_win_cap(const WindowKArgs& a, int grid) {
     else launch_win_exact<KC, VT, C, SINGLE, 2>(a, grid);
 }
 
+constexpr int WINDOW_PAIRS = 6;
 void launch_window_attention(const WindowAttn& w, const StepArrays& st) {
     if (st.n_runs <= 0) return;
     const KvPages& pool = w.pool;
@@ -966,8 +967,9 @@ void launch_window_attention(const WindowAttn& w, const StepArrays& st) {
         a.NHG = cdiv(rep, 16);
         const int items = n_single * a.G * a.NHG, waves = window_waves(cls == 0 ? 4 : cls == 1 ? 8 : 16, true);
         const long longest = std::min<long>(st.max_pos + 1, seen_cap + 32);
-        // slices until every CU has a workgroup, each wave of a slice with at least one pair of pages
-        a.nsplit = (int)std::max<long>(1, std::min<long>(rt().num_cus / items, longest / 32 / waves));
+        // slices until every CU has a workgroup, each wave of a slice with at least one pair of pages; none where a wave has few
+        // pairs, which take less time than the merge's launch (window of 528 keys, 22 layers: one row 1,306 -> 1,279 us a pass, six 1,584 -> 1,550)
+        a.nsplit = longest <= 32L * WINDOW_PAIRS * waves ? 1 : (int)std::max<long>(1, std::min<long>(rt().num_cus / items, longest / 32 / waves));
         if (a.nsplit > 1) {
             const size_t slices = (size_t)n_single * w.H * a.nsplit;
             a.part_acc = (float*)ws_get(WS_ATT_PART, slices * (16 * vt + 2) * sizeof(float));
