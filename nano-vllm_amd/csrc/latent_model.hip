@@ -41,7 +41,8 @@ struct LayerWeightsDir {
     int ff = 0;   // 0: the layer has no feed-forward
     // bf16
     B16Weight in, uq, uk, uv, o, gateup, down;
-    B16Weight uk_rows;   // W_uk as it is, [H * dim, rank]: keys of prompt portions (uk: for queries, head by head transposed)
+    bool expands = false;   // prompt portions may form keys and values (latent_prompt.h) ...
+    B16Weight uk_rows;      // ... with W_uk as it is, [H * dim, rank] (uk: for queries, head by head transposed)
     // fp32 (row-major, unpadded)
     float *dq = nullptr, *dkv = nullptr, *uq32 = nullptr, *uk32 = nullptr, *uv32 = nullptr, *o32 = nullptr, *gate = nullptr, *up = nullptr, *down32 = nullptr;
     // both: fp32 vectors, zero-padded in the bf16 form
@@ -81,6 +82,20 @@ private:
     void forward_b16(const PassArgs& a, const StepArrays& st, const LatentPromptPlan& plan);
     void forward_f32(const PassArgs& a, const StepArrays& st);
 };
+
+// Whether fp16 holds the products of a row of weights with RMS-normed rows times `gain`, which are sqrt(n) |row x gain| at most: none
+// overflows, and usual ones (a twentieth to a thousandth of that) keep more bits than in bf16.  Else the layer attends over latents.
+static bool fp16_holds(const uint16_t* row, const std::vector<float>& gain) {
+    double sq = 0.0;
+    for (size_t i = 0; i < gain.size(); i++) {
+        const uint32_t bits = (uint32_t)row[i] << 16;
+        float v;
+        memcpy(&v, &bits, 4);
+        sq += (double)v * v * gain[i] * gain[i];
+    }
+    const double most = std::sqrt(sq * (double)gain.size());
+    return most == 0.0 || (most >= 0x1p-10 && most <= 60000.0);
+}
 
 void LatentHyperModel::load_layer(const ModelDir& dir, int i, const Json& cfg) {
     const std::string at = "layers[" + std::to_string(i) + "]", L = "l" + std::to_string(i) + ".", M = L + "mix.", P = L + "mlp.";
@@ -163,8 +178,14 @@ void LatentHyperModel::load_layer(const ModelDir& dir, int i, const Json& cfg) {
     rows_to(Qp, 0, m.rank, D_);
     rows_to(Qp + Cp, m.rank, m.rot, D_);
     w.in = tile(dst, Qp + Cp + Rp, D_);
+    std::vector<float> gain_q(m.q_rank), gain_kv(m.rank);
+    dir.read_f32(M + "dq.norm", {m.q_rank}, gain_q.data());
+    dir.read_f32(M + "dkv.norm", {m.rank}, gain_kv.data());
+    w.expands = latent_prompt_fits(Cp, Rp, dimp, vp);
+    auto check = [&](int r, const std::vector<float>& gain) { w.expands = w.expands && fp16_holds(src.data() + (size_t)r * gain.size(), gain); };
     // W_uq: every head's unrotated rows, then every head's rotated rows
     read(M + "uq", H * QD, m.q_rank);
+    for (int r = 0; r < H * m.dim; r++) check(r / m.dim * QD + r % m.dim, gain_q);
     dst.assign((size_t)H * (dimp + Rp) * m.q_rank, 0);
     for (int h = 0; h < H; h++) {
         rows_to(h * dimp, h * QD, m.dim, m.q_rank);
@@ -181,11 +202,13 @@ void LatentHyperModel::load_layer(const ModelDir& dir, int i, const Json& cfg) {
             for (int c = 0; c < m.rank; c++) o[(size_t)c * m.dim] = s[c];
         }
     w.uk = tile(dst, H * Cp, m.dim, H);
+    for (int r = 0; r < H * m.dim; r++) check(r, gain_kv);
     dst.assign((size_t)H * dimp * m.rank, 0);
     for (int h = 0; h < H; h++) rows_to(h * dimp, h * m.dim, m.dim, m.rank);
-    w.uk_rows = tile(dst, H * dimp, m.rank);
     // W_uv head by head: [vdim, rank] per head
     read(M + "uv", H * m.vdim, m.rank);
+    for (int r = 0; r < H * m.vdim; r++) check(r, gain_kv);
+    if (w.expands) w.uk_rows = tile(dst, H * dimp, m.rank);
     dst.assign((size_t)H * vp * m.rank, 0);
     for (int h = 0; h < H; h++) rows_to(h * vp, h * m.vdim, m.vdim, m.rank);
     w.uv = tile(dst, H * vp, m.rank, H);
@@ -437,7 +460,7 @@ void LatentHyperModel::forward_b16(const PassArgs& a, const StepArrays& st, cons
             e4.a16_out = out + b16_halves(t0, m.heads * vp);
             launch_gemm_b16(w.uv, latents + b16_halves(t0, m.heads * Cp), n, e4, PC_GEMM_VALUE);
         };
-        if (!latent_prompt_pays(plan, pl, m.heads, dimp, vp)) {
+        if (!w.expands || !latent_prompt_pays(plan, pl, m.heads, dimp, vp)) {
             over_latents(0, T, hid, false);
             residual(w.o, hid, s, nullptr, PC_GEMM_WO);
             continue;

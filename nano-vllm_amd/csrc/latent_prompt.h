@@ -21,9 +21,10 @@ struct LatentPromptPlan {
 };
 LatentPromptPlan latent_prompt_plan(const int* pos, const int* seq_ids, int T, BlockTable** tables, int block_size);
 
+// Keys, values and unrotated queries are held in fp16: the caller sees to it that they fit (latent_model.hip, fp16_holds).
 struct LatentPrompt {
     LatentPool pool;
-    const __half* q_tiles;   // unrotated queries, activation tiles of [T, H * dim_ld]
+    const __half* q_tiles;   // unrotated queries, bf16 activation tiles of [T, H * dim_ld]
     const __half* q_rows;    // [T][H][pool.row()]: the rotated parts at pool.rank_ld
     const float* sink;
     float scale;
@@ -32,6 +33,8 @@ struct LatentPrompt {
     __half* out;             // activation tiles of [T, H * vdim_ld]
     const int *items, *pages;   // device copies of the plan
 };
+// Whether there are kernels for rows and heads of these widths.
+bool latent_prompt_fits(int rank_ld, int rot_ld, int dim_ld, int vdim_ld);
 // Whether this is the way to go for the pass's portions.
 bool latent_prompt_pays(const LatentPromptPlan& plan, const LatentPool& pool, int H, int dim_ld, int vdim_ld);
 void launch_latent_prompt(const LatentPrompt& a, const LatentPromptPlan& plan);
