@@ -79,6 +79,9 @@ private:
     LatentPool pool(const KVCacheManager* mgr, int run) const;
     size_t pool_bytes(int block_size, int num_blocks, int runs) const;   // of the first `runs` cache slices
     void load_layer(const ModelDir& dir, int i, const Json& cfg);
+    static bool expands(const LayerWeightsDir& w, const LatentPromptPlan& plan) {
+        return w.expands && latent_prompt_pays(plan, w.m.heads, pad32(w.m.rank), pad32(w.m.dim), pad32(w.m.vdim));
+    }
     void forward_b16(const PassArgs& a, const StepArrays& st, const LatentPromptPlan& plan);
     void forward_f32(const PassArgs& a, const StepArrays& st);
 };
@@ -358,10 +361,16 @@ void LatentHyperModel::forward(const PassArgs& a) {
         NVLLM_FATAL("transformer_batch: the block pool was not made for this model (nvllm_init_model_kv)");
     for (int t = 0; t < a.T; t++)
         if (a.pos[t] < 0 || a.tokens[t] < 0 || a.tokens[t] >= V_) NVLLM_FATAL("transformer_batch: token %d (id %d, position %d) is out of range", t, a.tokens[t], a.pos[t]);
-    const LatentPromptPlan plan = f32_ ? LatentPromptPlan() : latent_prompt_plan(a.pos, a.seq_ids, a.T, a.tables, a.mgr->block_size);
+    // prompt portions that form keys and values: their pages are listed only where some layer takes that way and the staging has room
+    LatentPromptPlan plan;
+    std::vector<int> listed;
+    if (!f32_) plan = latent_prompt_plan(a.pos, a.seq_ids, a.T);
+    if (std::none_of(layers_.begin(), layers_.end(), [&](const LayerWeightsDir& w) { return expands(w, plan); })) plan = LatentPromptPlan();
+    if (plan.n_items) listed = latent_prompt_ints(plan, a.pos, a.seq_ids, a.T, a.tables, a.mgr->block_size);
     const StepArrays st = stage_step(a.tokens, a.pos, a.seq_ids, a.T, a.output_indices, a.B, a.tables, nullptr, 0, a.mgr->block_size, LATENT_RUN, a.token_src, true,
-                                     false, 0, &plan.ints);
+                                     false, 0, &listed);
     if (st.table_short) NVLLM_FATAL("transformer_batch: a position lies beyond its sequence's block table (allocate the block first)");
+    if (!st.d_extra) plan = LatentPromptPlan();
     if (f32_) forward_f32(a, st);
     else forward_b16(a, st, plan);
 }
@@ -460,7 +469,7 @@ void LatentHyperModel::forward_b16(const PassArgs& a, const StepArrays& st, cons
             e4.a16_out = out + b16_halves(t0, m.heads * vp);
             launch_gemm_b16(w.uv, latents + b16_halves(t0, m.heads * Cp), n, e4, PC_GEMM_VALUE);
         };
-        if (!w.expands || !latent_prompt_pays(plan, pl, m.heads, dimp, vp)) {
+        if (!expands(w, plan)) {
             over_latents(0, T, hid, false);
             residual(w.o, hid, s, nullptr, PC_GEMM_WO);
             continue;

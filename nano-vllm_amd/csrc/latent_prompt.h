@@ -7,19 +7,20 @@
 
 namespace nvllm {
 
-// What a pass's portions of several tokens need, made on the host: the pool pages that hold their sequences' positions up to
-// the portion's last, in pairs, and items of up to LATENT_PROMPT_TOKENS tokens, those that see most first.
+// A pass's portions of several tokens, on the host, in items of up to LATENT_PROMPT_TOKENS tokens.
 constexpr int LATENT_PROMPT_TOKENS = 64;
 struct LatentPromptPlan {
-    std::vector<int> ints;   // [n_items][4] (first token, count, position of the first, first pair), then [n_pairs][2] page ids; a multiple of four
-    int n_items = 0, n_pairs = 0;
+    int n_items = 0, n_pairs = 0;   // pairs: of pool pages with the positions up to a portion's last
     int most_pairs = 0;      // of one portion
     int tokens = 0;          // tokens of the portions
     long pairs_qk = 0;       // (token, position) pairs
     // the 16-token blocks that hold the tokens which are their sequence's only ones (none: from == to)
     int alone_from = 0, alone_to = 0;
 };
-LatentPromptPlan latent_prompt_plan(const int* pos, const int* seq_ids, int T, BlockTable** tables, int block_size);
+LatentPromptPlan latent_prompt_plan(const int* pos, const int* seq_ids, int T);
+// What the kernels read: [n_items][4] (first token, count, position of the first, first pair), those that see most first, then
+// [n_pairs][2] page ids; a multiple of four.
+std::vector<int> latent_prompt_ints(const LatentPromptPlan& plan, const int* pos, const int* seq_ids, int T, BlockTable** tables, int block_size);
 
 // Keys, values and unrotated queries are held in fp16: the caller sees to it that they fit (latent_model.hip, fp16_holds).
 struct LatentPrompt {
@@ -36,7 +37,7 @@ struct LatentPrompt {
 // Whether there are kernels for rows and heads of these widths.
 bool latent_prompt_fits(int rank_ld, int rot_ld, int dim_ld, int vdim_ld);
 // Whether this is the way to go for the pass's portions.
-bool latent_prompt_pays(const LatentPromptPlan& plan, const LatentPool& pool, int H, int dim_ld, int vdim_ld);
+bool latent_prompt_pays(const LatentPromptPlan& plan, int H, int rank_ld, int dim_ld, int vdim_ld);
 void launch_latent_prompt(const LatentPrompt& a, const LatentPromptPlan& plan);
 
 }  // namespace nvllm

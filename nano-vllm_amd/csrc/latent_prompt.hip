@@ -21,6 +21,7 @@
 
 #include <algorithm>
 #include <array>
+#include <climits>
 
 #include "attn_tile.h"
 #include "gemm_common.h"
@@ -297,20 +298,44 @@ void launch_expand(const ExpandArgs& e, dim3 grid) {
 
 }  // namespace
 
-LatentPromptPlan latent_prompt_plan(const int* pos, const int* seq_ids, int T, BlockTable** tables, int block_size) {
+static int portion_at(const int* pos, const int* seq_ids, int T, int t) {   // tokens of the portion that begins with token t
+    int n = 1;
+    while (t + n < T && seq_ids[t + n] == seq_ids[t] && pos[t + n] == pos[t + n - 1] + 1) n++;
+    return n;
+}
+
+LatentPromptPlan latent_prompt_plan(const int* pos, const int* seq_ids, int T) {
     LatentPromptPlan p;
-    std::vector<int> pages;
-    std::vector<std::array<int, 4>> items;
     int alone_last = -1;
-    const int per_block = block_size / LATENT_PAGE;
+    long n_pairs = 0;
     for (int t = 0, n; t < T; t += n) {
-        n = 1;
-        while (t + n < T && seq_ids[t + n] == seq_ids[t] && pos[t + n] == pos[t + n - 1] + 1) n++;
+        n = portion_at(pos, seq_ids, T, t);
         if (n == 1) {
             if (alone_last < 0) p.alone_from = t / 16;
             alone_last = t;
             continue;
         }
+        const int pairs = pos[t + n - 1] / 32 + 1;
+        n_pairs += pairs;
+        p.most_pairs = std::max(p.most_pairs, pairs);
+        p.n_items += cdiv(n, LATENT_PROMPT_TOKENS);
+        p.tokens += n;
+        p.pairs_qk += (long)n * pos[t] + (long)n * (n + 1) / 2;
+    }
+    if (alone_last >= 0) p.alone_to = alone_last / 16 + 1;
+    p.n_pairs = (int)n_pairs;
+    if (n_pairs > INT_MAX / 32) p.n_items = 0;   // (no pool is as large)
+    return p;
+}
+
+std::vector<int> latent_prompt_ints(const LatentPromptPlan& plan, const int* pos, const int* seq_ids, int T, BlockTable** tables, int block_size) {
+    std::vector<std::array<int, 4>> items;
+    std::vector<int> pages, ints;
+    const int per_block = block_size / LATENT_PAGE;
+    pages.reserve(2 * (size_t)plan.n_pairs);
+    for (int t = 0, n; t < T; t += n) {
+        n = portion_at(pos, seq_ids, T, t);
+        if (n == 1) continue;
         const BlockTable* table = tables[seq_ids[t]];
         const int last = pos[t + n - 1], first_pair = (int)pages.size() / 2;
         for (int q = 0; q < 2 * (last / 32 + 1); q++) {
@@ -318,18 +343,12 @@ LatentPromptPlan latent_prompt_plan(const int* pos, const int* seq_ids, int T, B
             pages.push_back(block < 0 ? 0 : table->block_indices[block] * per_block + page % per_block);
         }
         for (int i = 0; i < n; i += LATENT_PROMPT_TOKENS) items.push_back({t + i, std::min(LATENT_PROMPT_TOKENS, n - i), pos[t] + i, first_pair});
-        p.most_pairs = std::max(p.most_pairs, (int)pages.size() / 2 - first_pair);
-        p.tokens += n;
-        p.pairs_qk += (long)n * pos[t] + (long)n * (n + 1) / 2;
     }
-    if (alone_last >= 0) p.alone_to = alone_last / 16 + 1;
     std::stable_sort(items.begin(), items.end(), [](const auto& a, const auto& b) { return a[2] + a[1] > b[2] + b[1]; });
-    for (const auto& i : items) p.ints.insert(p.ints.end(), i.begin(), i.end());
-    p.n_items = (int)items.size();
-    p.n_pairs = (int)pages.size() / 2;
-    p.ints.insert(p.ints.end(), pages.begin(), pages.end());
-    while (p.ints.size() % 4) p.ints.push_back(0);
-    return p;
+    for (const auto& i : items) ints.insert(ints.end(), i.begin(), i.end());
+    ints.insert(ints.end(), pages.begin(), pages.end());
+    while (ints.size() % 4) ints.push_back(0);
+    return ints;
 }
 
 bool latent_prompt_fits(int rank_ld, int rot_ld, int dim_ld, int vdim_ld) {
@@ -337,7 +356,7 @@ bool latent_prompt_fits(int rank_ld, int rot_ld, int dim_ld, int vdim_ld) {
     return rank_ld <= 512 && one_of(dim_ld, 32, 64, 128) && (rot_ld == 32 || rot_ld == 64) && one_of(vdim_ld, 32, 64, 128);
 }
 
-bool latent_prompt_pays(const LatentPromptPlan& plan, const LatentPool& P, int H, int dim_ld, int vdim_ld) {
+bool latent_prompt_pays(const LatentPromptPlan& plan, int H, int rank_ld, int dim_ld, int vdim_ld) {
     static const int env = getenv("NVLLM_LATENT_EXPAND") ? atoi(getenv("NVLLM_LATENT_EXPAND")) : -1;   // 0: never, 1: wherever it can be done
     const double positions = 32.0 * plan.n_pairs;
     if (env == 0 || plan.n_items == 0 || positions * H * (dim_ld + vdim_ld) * 2.0 > 512e6) return false;
@@ -348,9 +367,9 @@ bool latent_prompt_pays(const LatentPromptPlan& plan, const LatentPool& P, int H
     // saved per pair of token and position.  96 tokens behind 512, 32 heads: 107 us a layer -> 91, beside five tokens 126 -> 118;
     // 64 behind 1,700 93 -> 92; 17 behind 1,700 83 -> 89, not taken.  Passes of few columns (less than a thousand) gain the launches alone.
     if ((long)plan.tokens * H < 1024) return false;
-    const double forming = 0.35 * plan.most_pairs / 2 + positions * H * (dim_ld + vdim_ld) * P.rank_ld / 4e8;
+    const double forming = 0.35 * plan.most_pairs / 2 + positions * H * (dim_ld + vdim_ld) * rank_ld / 4e8;
     const double launches = plan.alone_to > plan.alone_from ? 0.0 : 8.0;
-    const double saved = plan.pairs_qk * (double)H * (P.row() + P.rank_ld - dim_ld - P.rot_ld - vdim_ld) / 2e8;
+    const double saved = plan.pairs_qk * (double)H * (2 * rank_ld - dim_ld - vdim_ld) / 2e8;
     return forming < launches + saved;
 }
 

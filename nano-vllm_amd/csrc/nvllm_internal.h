@@ -148,6 +148,7 @@ void* ws_get(WsSlot slot, size_t bytes);
 
 // Pinned host staging for the integer arrays of one call.
 int* pinned_ints(size_t n);   // ring allocation, for callers that fill it themselves
+size_t staging_ints();        // the most of one call
 
 // RoPE angle table for (theta, head_dim), covering positions [0, min_positions):
 // float2 {cos, sin} per (position, pair), computed on the host with the same libm

@@ -195,9 +195,10 @@ StepArrays stage_step(const int* tokens, const int* pos_arr, const int* seq_ids,
             kv_row[t] = t < s.write_limit ? bt->block_indices[p / block_size] * block_size + p % block_size : -1;
         }
     }
-    const size_t n_ints = (size_t)(tokens ? T : 0) + (token_src ? T : 0) + (pos_arr ? T : 0) + (seq_ids ? T : 0) + kv_row.size() +
-                          (output_indices ? B : 0) + n_seqs + total_tbl + runs.size() + span.size() + span_of.size() + chunks.size() + first_chunk.size() +
-                          (extra ? extra->size() : 0) + 64;
+    size_t n_ints = (size_t)(tokens ? T : 0) + (token_src ? T : 0) + (pos_arr ? T : 0) + (seq_ids ? T : 0) + kv_row.size() +
+                          (output_indices ? B : 0) + n_seqs + total_tbl + runs.size() + span.size() + span_of.size() + chunks.size() + first_chunk.size() + 64;
+    if (extra && n_ints + extra->size() > staging_ints()) extra = nullptr;   // (the caller can do without)
+    if (extra) n_ints += extra->size();
     int* host = pinned_ints(n_ints);
     int* dev = (int*)ws_get(WS_STEP, n_ints * sizeof(int));
     size_t o = 0;

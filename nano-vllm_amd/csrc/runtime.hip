@@ -64,6 +64,7 @@ static void stage_next_region() {
     g_stage_fill = 0;
 }
 
+size_t staging_ints() { return STAGE_INTS; }
 int* pinned_ints(size_t n) {
     ensure_init();
     if (n > STAGE_INTS) NVLLM_FATAL("staging request of %zu ints exceeds the ring region", n);

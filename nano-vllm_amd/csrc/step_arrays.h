@@ -43,7 +43,7 @@ struct StepArrays {
     int* d_chunks;           // [n_chunks][2] (span, its chunk)
     int* d_first_chunk;      // [n_spans_multi]
     std::vector<int> host_spans;
-    int* d_extra;            // with `extra`: the caller's own numbers, 16-byte aligned
+    int* d_extra;            // with `extra`: the caller's own numbers, 16-byte aligned; null: none, or no room in the staging
     // Kernel timing, when a token sees at most `limit` positions: rows of K/V that the portions of several tokens (of one
     // token) see, each counted once, and (token, position) pairs of the former.
     long multi_rows(long limit) const { return count(0, n_spans_multi, limit, false); }
