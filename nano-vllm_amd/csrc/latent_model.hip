@@ -469,7 +469,8 @@ void LatentHyperModel::forward_b16(const PassArgs& a, const StepArrays& st, cons
             e4.a16_out = out + b16_halves(t0, m.heads * vp);
             launch_gemm_b16(w.uv, latents + b16_halves(t0, m.heads * Cp), n, e4, PC_GEMM_VALUE);
         };
-        if (!expands(w, plan)) {
+        __half* formed = expands(w, plan) ? latent_prompt_scratch(plan, m.heads, dimp, vp) : nullptr;
+        if (!formed) {
             over_latents(0, T, hid, false);
             residual(w.o, hid, s, nullptr, PC_GEMM_WO);
             continue;
@@ -480,7 +481,7 @@ void LatentHyperModel::forward_b16(const PassArgs& a, const StepArrays& st, cons
         if (plan.alone_to > plan.alone_from) over_latents(16 * plan.alone_from, std::min(T, 16 * plan.alone_to) - 16 * plan.alone_from, values, true);
         LatentPrompt pr{};
         pr.pool = pl; pr.q_tiles = hid; pr.q_rows = (const __half*)q; pr.sink = w.sink; pr.scale = m.scale; pr.H = m.heads;
-        pr.dim_ld = dimp; pr.vdim_ld = vp; pr.uk = w.uk_rows.tiles; pr.uv = w.uv.tiles; pr.out = values;
+        pr.dim_ld = dimp; pr.vdim_ld = vp; pr.uk = w.uk_rows.tiles; pr.uv = w.uv.tiles; pr.kv = formed; pr.out = values;
         pr.items = st.d_extra; pr.pages = st.d_extra + 4 * plan.n_items;
         launch_latent_prompt(pr, plan);
         residual(w.o, values, s, nullptr, PC_GEMM_WO);

@@ -31,6 +31,7 @@ struct LatentPrompt {
     float scale;
     int H, dim_ld, vdim_ld;
     const __half *uk, *uv;   // tiles of [H * dim_ld, rank_ld] and [H * vdim_ld, rank_ld]
+    __half* kv;              // latent_prompt_scratch()
     __half* out;             // activation tiles of [T, H * vdim_ld]
     const int *items, *pages;   // device copies of the plan
 };
@@ -38,6 +39,8 @@ struct LatentPrompt {
 bool latent_prompt_fits(int rank_ld, int rot_ld, int dim_ld, int vdim_ld);
 // Whether this is the way to go for the pass's portions.
 bool latent_prompt_pays(const LatentPromptPlan& plan, int H, int rank_ld, int dim_ld, int vdim_ld);
+// Memory for the portions' keys and values; null: none (the portions attend over latents).
+__half* latent_prompt_scratch(const LatentPromptPlan& plan, int H, int dim_ld, int vdim_ld);
 void launch_latent_prompt(const LatentPrompt& a, const LatentPromptPlan& plan);
 
 }  // namespace nvllm

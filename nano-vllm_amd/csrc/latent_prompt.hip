@@ -356,10 +356,11 @@ bool latent_prompt_fits(int rank_ld, int rot_ld, int dim_ld, int vdim_ld) {
     return rank_ld <= 512 && one_of(dim_ld, 32, 64, 128) && (rot_ld == 32 || rot_ld == 64) && one_of(vdim_ld, 32, 64, 128);
 }
 
+constexpr double EXPAND_BYTES = 512e6;   // of keys and values at most
 bool latent_prompt_pays(const LatentPromptPlan& plan, int H, int rank_ld, int dim_ld, int vdim_ld) {
     static const int env = getenv("NVLLM_LATENT_EXPAND") ? atoi(getenv("NVLLM_LATENT_EXPAND")) : -1;   // 0: never, 1: wherever it can be done
     const double positions = 32.0 * plan.n_pairs;
-    if (env == 0 || plan.n_items == 0 || positions * H * (dim_ld + vdim_ld) * 2.0 > 512e6) return false;
+    if (env == 0 || plan.n_items == 0 || positions * H * (dim_ld + vdim_ld) * 2.0 > EXPAND_BYTES) return false;
     if (env > 0) return true;
     // us a layer, fitted to portions of 17 to 256 tokens at 0, 512 and 1,700 cached positions, alone and beside five single tokens,
     // of 32 heads with 512 latent values and 16 with 256: two launches less, unless single tokens beside the portions want
@@ -373,10 +374,15 @@ bool latent_prompt_pays(const LatentPromptPlan& plan, int H, int rank_ld, int di
     return forming < launches + saved;
 }
 
+__half* latent_prompt_scratch(const LatentPromptPlan& plan, int H, int dim_ld, int vdim_ld) {
+    static const double most = getenv("NVLLM_LATENT_EXPAND_BYTES") ? atof(getenv("NVLLM_LATENT_EXPAND_BYTES")) : EXPAND_BYTES;
+    const size_t bytes = (size_t)plan.n_pairs * H * 32 * (dim_ld + vdim_ld) * sizeof(__half);
+    return (double)bytes <= most ? (__half*)ws_try(WS_EXPANDED, bytes) : nullptr;
+}
+
 void launch_latent_prompt(const LatentPrompt& a, const LatentPromptPlan& plan) {
     if (plan.n_items <= 0) return;
     const LatentPool& P = a.pool;
-    __half* kv = (__half*)ws_get(WS_EXPANDED, (size_t)plan.n_pairs * a.H * 32 * (a.dim_ld + a.vdim_ld) * sizeof(__half));
     const double positions = 32.0 * plan.n_pairs, width = (double)a.H * (a.dim_ld + a.vdim_ld);
     {
         ExpandArgs e{};
@@ -390,7 +396,7 @@ void launch_latent_prompt(const LatentPrompt& a, const LatentPromptPlan& plan) {
         e.vt = a.vdim_ld / 16;
         e.uk = a.uk;
         e.uv = a.uv;
-        e.kv = kv;
+        e.kv = a.kv;
         const int cols = cdiv(a.H * (e.dc + e.vt / 2), 8);
         // as many workgroups as CUs, of four pairs at least (a wave's weights are as many bytes as two pairs)
         e.per = std::max(4, cdiv(plan.n_pairs, std::max(1, rt().num_cus / cols)));
@@ -405,7 +411,7 @@ void launch_latent_prompt(const LatentPrompt& a, const LatentPromptPlan& plan) {
     k.pages = a.pages;
     k.q_tiles = a.q_tiles;
     k.q_rows = a.q_rows;
-    k.kv = kv;
+    k.kv = a.kv;
     k.sink = a.sink;
     k.scale = a.scale;
     k.H = a.H;

@@ -145,6 +145,7 @@ enum WsSlot {
     WS_COUNT
 };
 void* ws_get(WsSlot slot, size_t bytes);
+void* ws_try(WsSlot slot, size_t bytes);   // null: no memory
 
 // Pinned host staging for the integer arrays of one call.
 int* pinned_ints(size_t n);   // ring allocation, for callers that fill it themselves

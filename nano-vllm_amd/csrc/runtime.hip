@@ -27,7 +27,7 @@ void sync_streams() {
     if (g_rt.copy_stream) HIP_CHECK(hipStreamSynchronize(g_rt.copy_stream));
 }
 
-void* ws_get(WsSlot slot, size_t bytes) {
+void* ws_try(WsSlot slot, size_t bytes) {
     ensure_init();
     WsBuf& b = g_ws[slot];
     if (bytes > b.bytes) {
@@ -35,12 +35,24 @@ void* ws_get(WsSlot slot, size_t bytes) {
             sync_streams();
             HIP_CHECK(hipFree(b.p));
         }
+        b = WsBuf{};
         size_t want = bytes + bytes / 4;  // head-room: shapes creep up during prefill
         want = (want + 255) & ~(size_t)255;
-        HIP_CHECK(hipMalloc(&b.p, want));
+        const hipError_t e = hipMalloc(&b.p, want);
+        if (e == hipErrorOutOfMemory) {
+            (void)hipGetLastError();
+            b.p = nullptr;
+            return nullptr;
+        }
+        HIP_CHECK(e);
         b.bytes = want;
     }
     return b.p;
+}
+void* ws_get(WsSlot slot, size_t bytes) {
+    void* p = ws_try(slot, bytes);
+    if (!p && bytes) HIP_CHECK(hipErrorOutOfMemory);
+    return p;
 }
 
 // ------------------------------------------------------- pinned staging ring
