@@ -356,7 +356,47 @@ void LatentHyperModel::init_kv(KVCacheManager* mgr, int block_size, int num_bloc
     init_block_pool(mgr, block_size, num_blocks, pool_bytes(block_size, num_blocks, (int)runs_.size()));
 }
 
-void LatentHyperModel::forward(const PassArgs& a) {
+// The pass with its tokens in another order: portions of several tokens first, then the single ones, whose products with W_uk and W_uv
+// then are those of a few neighbouring blocks wherever the scheduler put them.  Nothing hangs on the order of a pass's tokens.
+namespace {
+struct PortionsFirst {
+    std::vector<int> ints;   // tokens, positions, ids, [token_src], output rows
+    // false: they lie like that, or output rows name no token
+    bool arrange(PassArgs& a) {
+        const int T = a.T;
+        std::vector<int> order, alone;
+        bool behind = true;   // no single token before a portion
+        for (int t = 0, n; t < T; t += n) {
+            n = latent_portion(a.pos, a.seq_ids, T, t);
+            behind = behind && (n == 1 || alone.empty());
+            for (int i = 0; i < n; i++) (n == 1 ? alone : order).push_back(t + i);
+        }
+        for (int b = 0; b < a.B; b++)
+            if (a.output_indices[b] < 0 || a.output_indices[b] >= T) return false;
+        if (behind) return false;
+        order.insert(order.end(), alone.begin(), alone.end());
+        std::vector<int> to(T);
+        for (int i = 0; i < T; i++) to[order[i]] = i;
+        ints.resize((size_t)4 * T + a.B);
+        int* at = ints.data();
+        auto moved = [&](const int*& p) {
+            for (int i = 0; i < T; i++) at[i] = p[order[i]];
+            p = at;
+            at += T;
+        };
+        moved(a.tokens);
+        moved(a.pos);
+        moved(a.seq_ids);
+        if (a.token_src) moved(a.token_src);
+        for (int b = 0; b < a.B; b++) at[b] = to[a.output_indices[b]];
+        a.output_indices = at;
+        return true;
+    }
+};
+}  // namespace
+
+void LatentHyperModel::forward(const PassArgs& given) {
+    PassArgs a = given;
     if (block_pool_bytes(a.mgr) != pool_bytes(a.mgr->block_size, a.mgr->num_blocks, (int)runs_.size()))
         NVLLM_FATAL("transformer_batch: the block pool was not made for this model (nvllm_init_model_kv)");
     for (int t = 0; t < a.T; t++)
@@ -364,8 +404,10 @@ void LatentHyperModel::forward(const PassArgs& a) {
     // prompt portions that form keys and values: their pages are listed only where some layer takes that way and the staging has room
     LatentPromptPlan plan;
     std::vector<int> listed;
+    PortionsFirst order;
     if (!f32_) plan = latent_prompt_plan(a.pos, a.seq_ids, a.T);
     if (std::none_of(layers_.begin(), layers_.end(), [&](const LayerWeightsDir& w) { return expands(w, plan); })) plan = LatentPromptPlan();
+    if (plan.n_items && order.arrange(a)) plan = latent_prompt_plan(a.pos, a.seq_ids, a.T);   // (portions that now lie side by side may be one)
     if (plan.n_items) listed = latent_prompt_ints(plan, a.pos, a.seq_ids, a.T, a.tables, a.mgr->block_size);
     const StepArrays st = stage_step(a.tokens, a.pos, a.seq_ids, a.T, a.output_indices, a.B, a.tables, nullptr, 0, a.mgr->block_size, LATENT_RUN, a.token_src, true,
                                      false, 0, &listed);

@@ -17,6 +17,7 @@ struct LatentPromptPlan {
     // the 16-token blocks that hold the tokens which are their sequence's only ones (none: from == to)
     int alone_from = 0, alone_to = 0;
 };
+int latent_portion(const int* pos, const int* seq_ids, int T, int t);   // tokens of the portion that begins with token t
 LatentPromptPlan latent_prompt_plan(const int* pos, const int* seq_ids, int T);
 // What the kernels read: [n_items][4] (first token, count, position of the first, first pair), those that see most first, then
 // [n_pairs][2] page ids; a multiple of four.

@@ -298,7 +298,7 @@ void launch_expand(const ExpandArgs& e, dim3 grid) {
 
 }  // namespace
 
-static int portion_at(const int* pos, const int* seq_ids, int T, int t) {   // tokens of the portion that begins with token t
+int latent_portion(const int* pos, const int* seq_ids, int T, int t) {
     int n = 1;
     while (t + n < T && seq_ids[t + n] == seq_ids[t] && pos[t + n] == pos[t + n - 1] + 1) n++;
     return n;
@@ -309,7 +309,7 @@ LatentPromptPlan latent_prompt_plan(const int* pos, const int* seq_ids, int T) {
     int alone_last = -1;
     long n_pairs = 0;
     for (int t = 0, n; t < T; t += n) {
-        n = portion_at(pos, seq_ids, T, t);
+        n = latent_portion(pos, seq_ids, T, t);
         if (n == 1) {
             if (alone_last < 0) p.alone_from = t / 16;
             alone_last = t;
@@ -334,7 +334,7 @@ std::vector<int> latent_prompt_ints(const LatentPromptPlan& plan, const int* pos
     const int per_block = block_size / LATENT_PAGE;
     pages.reserve(2 * (size_t)plan.n_pairs);
     for (int t = 0, n; t < T; t += n) {
-        n = portion_at(pos, seq_ids, T, t);
+        n = latent_portion(pos, seq_ids, T, t);
         if (n == 1) continue;
         const BlockTable* table = tables[seq_ids[t]];
         const int last = pos[t + n - 1], first_pair = (int)pages.size() / 2;
