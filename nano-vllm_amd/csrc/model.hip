@@ -222,8 +222,13 @@ static bool argmax_direct() {
 // Where the classifier itself stores a pass's logits rows for the host (null: finish_pass() copies them).  The caller must be waiting
 // for the pass -- rows of a pass sent ahead cross PCIe beside the next pass's kernels --, and the rows lie in malloc_run_state's array.
 // A pass of 64 rows of 32,000 values gets 20 us shorter (classifier 38, copy 147 before), of 32 rows 20 (15 and 73), of one 12: the copy's launch.
+// Rows of a length that is no multiple of four are stored value by value, which PCIe takes more slowly.  Copied -> stored, us a pass of
+// four layers, 32,001 to 32,003 words: one row 270 -> 255 (fp16), 228 -> 216 (fp32), 295 -> 280 (bf16); 32 rows 375 -> 367, 327 -> 323,
+// 360 -> 359; 64 rows 479 -> 476, 438 -> 461, 467 -> 473.  So up to 32 of them.
+constexpr int DIRECT_ODD_ROWS = 32;
 static float* direct_rows(const RunState* s, int B, int V, bool waits) {
     if (rt().logits_mode != NVLLM_LOGITS_HOST || !waits || B <= 0 || !argmax_direct() || ((size_t)s->logits & 15)) return nullptr;
+    if (V % 4 && B > DIRECT_ODD_ROWS) return nullptr;
     return nvllm_internal_pinned_holds(s->logits, (size_t)B * V * sizeof(float)) ? s->logits : nullptr;
 }
 
