@@ -1,6 +1,8 @@
 // gemm_wide_b16.hip -- launches of the 256-feature tiles (gemm_wide.h) for bf16 models: the wide projections whose epilogue
 // only writes (gated pairs, tiles, rows).
+#include <algorithm>
 #include <cmath>
+#include <iterator>
 
 #include "gemm_wide.h"
 
@@ -62,6 +64,7 @@ bool launch_gemm_wide_b16(const GemmArgs& a) {
 // sixteen gets more at a few in a hundred (a second group then); 0: not for these sizes.
 int expert_rows_wide(int rows, int experts, int N, int K) {
     const double per = (double)rows / experts;
+    if (wide_env() > 0) return K < 256 || std::find(std::begin(WIDE_HEIGHTS), std::end(WIDE_HEIGHTS), wide_env()) == std::end(WIDE_HEIGHTS) ? 0 : 16 * wide_env();
     const int cus = rt().num_cus, tiles = cdiv(N, 256) * experts;
     if (wide_env() == 0 || K < 1024 || per < 40 || tiles > cus || 100 * tiles < 40 * cus) return 0;
     for (int h : WIDE_HEIGHTS)

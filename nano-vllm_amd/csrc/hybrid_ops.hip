@@ -162,7 +162,12 @@ void nvllm_expert_ff(float* out, int* choice, float* score, const float* in, con
                      int experts, int top, int elem_bytes, int num_tokens) {
     ensure_init();
     if (num_tokens <= 0) return;
-    const int pad = elem_bytes == 4 ? 16 : route_pad(num_tokens, experts, top);
+    const int Dp = pad32(dim), Fp = pad32(ff);
+    B16Weight wu, wd;
+    wu.N = 2 * Fp; wu.K = Dp;
+    wd.N = Dp; wd.K = Fp;
+    const ExpertGroups groups = elem_bytes == 4 ? ExpertGroups{16, false} : expert_groups(num_tokens, experts, top, wu, wd);
+    const int pad = groups.pad;
     const Temp mem(route_ints(num_tokens, experts, top, pad) * 4);
     const RoutePlan plan = route_plan((int*)mem.p, num_tokens, experts, top, pad);
     launch_route(plan, z, experts);
@@ -182,7 +187,6 @@ void nvllm_expert_ff(float* out, int* choice, float* score, const float* in, con
         launch_moe_combine(c, num_tokens);
         return;
     }
-    const int Dp = pad32(dim), Fp = pad32(ff);
     const long up_nb = (long)(Dp / 32) * TILE_HALVES, down_nb = (long)(Fp / 32) * TILE_HALVES;
     const Temp act(b16_halves(num_tokens, Dp) * 2), w_up((size_t)experts * (2 * Fp / 16) * up_nb * 2), w_down((size_t)experts * (Dp / 16) * down_nb * 2),
         hid(b16_halves(plan.capacity, Fp) * 2), y((size_t)plan.capacity * Dp * 4), y_sum((size_t)num_tokens * Dp * 4);
@@ -199,14 +203,22 @@ void nvllm_expert_ff(float* out, int* choice, float* score, const float* in, con
         rows_b16(stage.h(), down + (size_t)e * dim * ff, dim, ff, ff, ff);
         launch_tile_weights(w_down.h() + (size_t)e * (Dp / 16) * down_nb, stage.h(), dim, ff, down_nb);
     }
-    B16Weight wu, wd;
-    wu.tiles = w_up.h(); wu.N = 2 * Fp; wu.K = Dp;
-    wd.tiles = w_down.h(); wd.N = Dp; wd.K = Fp;
-    ExpertRows er{plan.block_expert, plan.source, plan.capacity, plan.pad, num_tokens * top};
+    wu.tiles = w_up.h();
+    wd.tiles = w_down.h();
+    ExpertRows er{plan.block_expert, plan.source, plan.capacity, plan.pad, num_tokens * top, groups.wide};
+    const Temp sorted(groups.wide ? b16_halves(plan.capacity, Dp) * 2 : 1), padded(groups.wide ? (size_t)num_tokens * Dp * 4 : 1), ones((size_t)Dp * 4);
+    if (groups.wide) {   // rows in the plan's order, as the models lay them out
+        const std::vector<float> one(Dp, 1.f);
+        device_memcpy(ones.p, one.data(), one.size() * 4, HOST_TO_DEVICE);
+        HIP_CHECK(hipMemsetAsync(padded.p, 0, (size_t)num_tokens * Dp * 4, rt().stream));
+        HIP_CHECK(hipMemcpy2DAsync(padded.p, (size_t)Dp * 4, in, (size_t)dim * 4, (size_t)dim * 4, num_tokens, hipMemcpyDeviceToDevice, rt().stream));
+        launch_expert_rows(sorted.h(), padded.f(), ones.f(), plan, Dp);
+        er.source = nullptr;
+    }
     GemmEpilogue eu;
     eu.kind = GemmEpilogue::SWIGLU_A16;
     eu.row_weight = plan.weight; eu.a16_out = hid.h();
-    launch_gemm_experts(wu, experts, act.h(), er, eu, PC_GEMM_EXPERT_UP);
+    launch_gemm_experts(wu, experts, groups.wide ? sorted.h() : act.h(), er, eu, PC_GEMM_EXPERT_UP);
     er.source = nullptr;
     GemmEpilogue ed;
     ed.kind = GemmEpilogue::F32;
