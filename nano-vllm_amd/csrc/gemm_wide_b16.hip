@@ -61,12 +61,19 @@ bool launch_gemm_wide_b16(const GemmArgs& a) {
 }
 
 // Rows sorted by expert: groups as tall as hold the rows an expert gets from a batch of that many, with the chance that one of
-// sixteen gets more at a few in a hundred (a second group then); 0: not for these sizes.
-int expert_rows_wide(int rows, int experts, int N, int K) {
+// sixteen gets more at a few in a hundred (a second group then); 0: not for these sizes.  One round of the chip, and one that pays
+// beside groups of 64 rows (from 96 rows an expert on: 128) in 128-feature tiles.  Passes of four layers of sixteen experts, two a token,
+// 330 to 1,600 tokens, those groups -> these, by the share of the CUs that have a tile of the first and of the second product: 62 and 44,
+// 62 and 50, 62 and 62, 69 and 50, 94 and 50 % always faster (780 -> 735, 820 -> 776, 993 -> 888, 843 -> 788, 933 -> 891 us at 330 tokens; 1,122 -> 1,036 ..
+// 1,370 -> 1,201 at 1,029); 56 and 50, 56 and 56 at 50 rows an expert 766 -> 793, 825 -> 855, at 64 829 -> 819, 962 -> 909; 50 and 44 at 64 rows
+// 718 -> 754, at 100 852 -> 826, at 200 the same; eight experts of 41 and 41 at 82 rows 996 -> 1,032, at 128 1,148 -> 1,114.
+int expert_rows_wide(int rows, int experts, const B16Weight& up, const B16Weight& down) {
     const double per = (double)rows / experts;
-    if (wide_env() > 0) return K < 256 || std::find(std::begin(WIDE_HEIGHTS), std::end(WIDE_HEIGHTS), wide_env()) == std::end(WIDE_HEIGHTS) ? 0 : 16 * wide_env();
-    const int cus = rt().num_cus, tiles = cdiv(N, 256) * experts;
-    if (wide_env() == 0 || K < 1024 || per < 40 || tiles > cus || 100 * tiles < 40 * cus) return 0;
+    auto height = [](int h) { return std::find(std::begin(WIDE_HEIGHTS), std::end(WIDE_HEIGHTS), h) != std::end(WIDE_HEIGHTS); };
+    if (wide_env() > 0) return up.K >= 256 && down.K >= 256 && height(wide_env()) ? 16 * wide_env() : 0;
+    const int cus = rt().num_cus, tiles_up = cdiv(up.N, 256) * experts, tiles_down = cdiv(down.N, 256) * experts;
+    if (wide_env() == 0 || up.K < 1024 || down.K < 1024 || std::max(tiles_up, tiles_down) > cus || 100 * std::min(tiles_up, tiles_down) < 40 * cus) return 0;
+    if (per < (100 * tiles_up >= 60 * cus ? 40 : 100 * tiles_up >= 55 * cus ? 60 : 96)) return 0;
     for (int h : WIDE_HEIGHTS)
         if (16 * h >= per + 2.5 * std::sqrt(per)) return 16 * h;
     return 0;

@@ -20,9 +20,8 @@ int route_pad(int T, int E, int top) {
 // 16 experts of 2 x 1,408 x 2,048, two per token, 1,029 tokens: groups of 128 rows, which every other expert's overflow, took 74 us
 // and 44 for the two products; of 160 56 and 41.
 ExpertGroups expert_groups(int T, int E, int top, const B16Weight& up, const B16Weight& down) {
-    const int wide = expert_rows_wide(T * top, E, up.N, up.K);
-    if (wide && expert_rows_wide(T * top, E, down.N, down.K)) return {wide, true};
-    return {route_pad(T, E, top), false};
+    const int wide = expert_rows_wide(T * top, E, up, down);
+    return {wide ? wide : route_pad(T, E, top), wide != 0};
 }
 static int route_capacity(int T, int E, int top, int pad) {
     const long rows = (long)T * top, groups = std::min(rows, rows / pad + E);   // full groups, and one partly filled per expert

@@ -394,8 +394,8 @@ struct ExpertRows {
     int live;                  // expected number of rows (bytes and flops of the kernel timing)
     bool wide = false;         // pad is expert_rows_wide()'s (the rows are the activations' own)
 };
-// gemm_wide_b16.hip: the group size with which `rows` rows of all experts meet [N][K] matrices in tiles of 256 features; 0: they do not
-int expert_rows_wide(int rows, int experts, int N, int K);
+// gemm_wide_b16.hip: the group size with which `rows` rows of all experts meet both products' matrices in tiles of 256 features; 0: they do not
+int expert_rows_wide(int rows, int experts, const B16Weight& up, const B16Weight& down);
 // w: [experts][N][K] stacked, N a multiple of 32.  Kinds SWIGLU_A16 and F32.
 void launch_gemm_experts(const B16Weight& w, int experts, const __half* act, const ExpertRows& rows, const GemmEpilogue& epi, int prof_cls);
 
