@@ -32,19 +32,19 @@ bool launch_wide_b16(const GemmArgs& a) {
     // 8: more steps than the deepest ring.  Below 32 steps a launch is mostly start and end, which the smaller tiles overlap.
     if (a.Kb < (wide_env() < 0 ? 32 : 8) || wide_env() == 0) return false;
     // With one plane of activations a step multiplies for as long as it copies, and the tiles of gemm_b16.hip, three to a CU,
-    // come close.  So only launches that are one round here: the lowest height that fits them into the CUs, and 85 of 100 CUs
-    // with a tile.  2,048 x 2,048 k, those against these: gated pairs of 5,632 at 400 tokens (220 tiles of 96) 35.9 -> 34.1 us,
-    // at 700 (220 of 160) 50 -> 46; of 2,816 at 700 (242 of 64) 30.4 -> 29, at 1,029 (242 of 96) 38 -> 34, at 1,600 (220 of
-    // 160) 55 -> 45.  154 tiles of 64 measured the same, two rounds (484 of 96) 66 -> 69; heights of 13 and 16 blocks, whose
-    // sums do not fit 256 registers, 65 -> 69 where they make one round of two.
-    // Eight waves, two to a SIMD, from eight blocks on: one's requests go out behind the other's products.
+    // come close.  So only launches that are one round here, at the lowest height that fits them into the CUs, and fill most of it: two
+    // rounds (484 tiles of 96) 66 -> 69 us.  2,048 k, those against these, twelve layers' weights in turn: four blocks with a tile on 81 % of the
+    // CUs 27.1 -> 28.4 (4,864 features, 700 tokens), 27.1 -> 28.2 (3,328, 1,024), 28.2 -> 28.6 (6,656, 512), on 95 % 30.4 -> 29 (5,632, 700); five
+    // on 81 % 27.8 -> 24.7 (6,656, 640); six 36.3 -> 32.1 (4,864, 1,024), 38.4 -> 35.2 (13,312, 380), on 86 % 35.9 -> 34.1 (11,264, 400).  Eight waves,
+    // two to a SIMD, from eight blocks on: one's requests go out behind the other's products; on 81 % 33.9 -> 29.4 (6,656, 1,024), and ten to
+    // sixteen 45.4 -> 35.8, 48.2 -> 41.7, 51.9 -> 47.8, 66.3 -> 50.8 (6,656; 1,280, 1,536, 1,792, 2,000).
     const int cus = rt().num_cus, tiles_n = cdiv(a.NB, 16);
     int tbn = 0;
     for (int h : WIDE_HEIGHTS)
         if (!tbn && tiles_n * cdiv(a.Tb, h) <= cus) tbn = h;
     if (wide_env() > 0) tbn = wide_env();
     const int tiles_t = tbn ? cdiv(a.Tb, tbn) : 0, tiles = tiles_n * tiles_t;
-    if (wide_env() < 0 && (!tbn || 100 * tiles < 80 * cus)) return false;
+    if (wide_env() < 0 && (!tbn || 100 * tiles < (tbn == 4 ? 85 : 80) * cus)) return false;
     return launch_wide_height<EPI, false>(a, tbn, tiles_n, tiles_t);
 }
 
