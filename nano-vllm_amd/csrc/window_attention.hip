@@ -904,7 +904,12 @@ static void launch_win_cap(const WindowKArgs& a, int grid) {
     else launch_win_exact<KC, VT, C, SINGLE, 2>(a, grid);
 }
 
-constexpr int WINDOW_PAIRS = 6;
+// Keys up to which a token's window stays whole: the merge of slices is a launch of its own.  Passes of twelve layers, 1, 6, 16 and 30
+// rows, sliced -> whole: heads of 64 values at 1,500 keys 562 -> 526, 586 -> 544, 609 -> 580, 646 -> 626 us; of 128 at 900 565 -> 543, 587 -> 562,
+// 636 -> 633, 669 -> 651, at 1,200 564 -> 555, 585 -> 576, 644 -> 683, 689 -> 689; of 256 at 520 574 -> 554, 595 -> 571, 623 -> 603, 639 -> 640, at 700
+// 576 -> 573, 590 -> 594, 631 -> 630, 660 -> 692; of 192, in the form for other widths, at 300 601 -> 590, 618 -> 613, 637 -> 643, 647 -> 654, at 400
+// 599 -> 634, 604 -> 645, 649 -> 686, 675 -> 736 (160: at 400 the same; 224: as 192).
+static int window_whole(int cls, bool exact) { return cls == 0 ? 1536 : cls == 1 ? 960 : exact ? 576 : 320; }
 void launch_window_attention(const WindowAttn& w, const StepArrays& st) {
     if (st.n_runs <= 0) return;
     const KvPages& pool = w.pool;
@@ -967,9 +972,9 @@ void launch_window_attention(const WindowAttn& w, const StepArrays& st) {
         a.NHG = cdiv(rep, 16);
         const int items = n_single * a.G * a.NHG, waves = window_waves(cls == 0 ? 4 : cls == 1 ? 8 : 16, true);
         const long longest = std::min<long>(st.max_pos + 1, seen_cap + 32);
-        // slices until every CU has a workgroup, each wave of a slice with at least one pair of pages; none where a wave has few
-        // pairs, which take less time than the merge's launch (window of 528 keys, 22 layers: one row 1,306 -> 1,279 us a pass, six 1,584 -> 1,550)
-        a.nsplit = longest <= 32L * WINDOW_PAIRS * waves ? 1 : (int)std::max<long>(1, std::min<long>(rt().num_cus / items, longest / 32 / waves));
+        // slices until every CU has a workgroup, each wave of a slice with at least one pair of pages
+        const int whole = window_whole(cls, kc == 8 && vt == 16);
+        a.nsplit = longest <= whole ? 1 : (int)std::max<long>(1, std::min<long>(rt().num_cus / items, longest / 32 / waves));
         if (a.nsplit > 1) {
             const size_t slices = (size_t)n_single * w.H * a.nsplit;
             a.part_acc = (float*)ws_get(WS_ATT_PART, slices * (16 * vt + 2) * sizeof(float));
