@@ -63,7 +63,7 @@ struct GemmArgs {
     float* slab;      // [tile][slice][round][item] float4
     unsigned* counters;
     int close_sc1;    // K split: the closing workgroup loads the partials past the vector cache instead of invalidating it
-                      // (launches of at most one workgroup per CU over a hipMalloc slab)
+                      // (hipMalloc slab; launches of at most one tile per CU, where it was measured: riders are not counted)
     GemmEpilogue e;
     LatentKvRider ride;
     int ride_from;    // first workgroup (grid x) of the riders

@@ -408,9 +408,11 @@ __device__ __forceinline__ bool gemm_tile(const GemmArgs& p, const TileIdx ix, u
         __syncthreads();
         if (*s_ticket != (unsigned)p.ksplit - 1) return false;     // not the last slice of this tile
         // The partials were stored write-through, every storing wave drained, and this workgroup's add came
-        // last (its returned value says so, read behind the barrier above).  With one workgroup per CU the
-        // partials may then be loaded past the vector cache (sc1) with no invalidate; otherwise an agent
-        // acquire comes first.
+        // last (its returned value says so, read behind the barrier above).  They may then be loaded past the
+        // vector cache (sc1) with no invalidate: such a load misses that cache whoever shares the CU, and no
+        // cache holds an older copy, because a line of the slab is stored once and read once in a launch, here,
+        // and launches begin with clean caches.  Tiles and riders beside this one load no line of its partials.
+        // Otherwise an agent acquire comes first.
         const bool past_l1 = p.close_sc1;
         if (!past_l1) {
             if (tid == 0) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");

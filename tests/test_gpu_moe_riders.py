@@ -21,3 +21,19 @@ def test_passes_of_few_tokens(hip, tmp_path, experts, shared):
         got = U.feed_all(eng, [[(0, n)]], {0: seq})[0]
         assert U.error(got, O.forward(cfg, weights, seq)) < U.limit(False), n
     eng.close()
+
+
+# K splits of both products; of the second, with 96-feature tiles of the first from 33 tokens on
+@pytest.mark.parametrize("width,experts,shared", [(1024, 20, 96), (512, 70, 2816), (256, 30, 2816)])
+def test_riders_beside_k_splits(hip, tmp_path, width, experts, shared):
+    """The same bits twice: riders share the launch, and the CUs, with tiles whose partial sums meet through memory."""
+    window = synth.window_mixer(4, 2, 16, 16, size=48, keep_first=4)
+    cfg = synth.hybrid_config(width, 211, [(window, synth.expert_mlp(48, experts, 2, shared))] * 2)
+    path, cfg, weights = U.model(tmp_path, "splits", seed=experts, cfg=cfg)
+    eng = U.engine(hip, path, False, slots=1)
+    for n in (1, 16, 40, 64, 65, 128, 200):
+        seq = U.tokens(n, 211, n)
+        got = U.feed_all(eng, [[(0, n)]], {0: seq})[0]
+        np.testing.assert_array_equal(U.feed_all(eng, [[(0, n)]], {0: seq})[0], got)
+        assert U.error(got, O.forward(cfg, weights, seq)) < U.limit(False), n
+    eng.close()
