@@ -599,8 +599,8 @@ void LatentHyperModel::forward_f32(const PassArgs& a, const StepArrays& st) {
     head.in_rows = st.d_out_idx;
     launch_gemm_f32(head.add((const float*)embed_, V_, a.d_logits), PC_GEMM_HEAD);
     launch_softcap(a.d_logits, softcap_, (long)B * V_);
-    if (a.logits_host) copy_rows_to_host(a.logits_host, a.d_logits, (size_t)B * V_);
     launch_argmax_ld(a.d_argmax, a.d_logits, B, V_, V_, a.argmax_host);
+    if (a.logits_host) copy_rows_to_host(a.logits_host, a.d_logits, (size_t)B * V_);   // (last: a launch behind a copy waits for more than the copy)
 }
 
 }  // namespace
