@@ -512,7 +512,9 @@ void launch_paged_attention(const AttnArgs& a) {
     // one round of the chip, two of which never pay.  A pass of TinyLlama-1.1B, one row with 150, 300, 500, 700 cached: sliced 1,052, 1,050,
     // 1,048, 1,058 us, whole 1,005, 1,020, 1,044, 1,079; twelve 1,165, 1,166, 1,167, 1,185 and 1,131, 1,137, 1,169, 1,195; 30 with 1,050:
     // 1,357 and 1,372.  Of more than a round: 18 rows with 480, 800: 1,255, 1,273 and 1,230, 1,277; 25 with 400, 640, 1,000: 1,288, 1,315,
-    // 1,348 and 1,251, 1,287, 1,340; 40 with 500, 1,050, 2,000, 3,000: 1,443, 1,530, 1,659, 1,809 and 1,381, 1,472, 1,628, 1,790
+    // 1,348 and 1,251, 1,287, 1,340; 40 with 500, 1,050, 2,000, 3,000: 1,443, 1,530, 1,659, 1,809 and 1,381, 1,472, 1,628, 1,790.  Other heads,
+    // ten layers, sliced and whole: of 128 values (16 on 4) 1, 12, 40 rows with 150 538, 611, 789 and 522, 603, 752, 25 and 40 with 300 707, 804 and
+    // 681, 774; of 32 (64 on 8) 1 and 12 with 300 507, 583 and 489, 561; what the rule leaves in slices, 1 row with 300 of 128 and 500 of 32, is even
     if (wg_items && env_units <= 0) {
         const bool rounds = base_items * nsplit > target;
         const long walk = (long)pages * std::max(a.hd, 64) / 64;

@@ -5,7 +5,7 @@
 // wave + 4, ...: operands go from global memory straight into the registers that feed the matrix cores (both are stored
 // in operand order), nothing is shared through LDS and no barrier stands in the loop.  A byte still enters the CU once,
 // because no two waves want the same one.  One wave per SIMD has 512 registers: up to 224 hold the sums, the rest two to
-// four K-steps in flight, 80 to 156 KiB per CU.  The waves' sums meet in LDS once, at the end; wave w finishes row
+// four K-steps, 144 to 216 KiB per CU, of which 80 to 144 are on their way while a step is multiplied.  The waves' sums meet in LDS once, at the end; wave w finishes row
 // blocks 2 w and 2 w + 1 of the tile.
 //
 // What bounds it: the bytes into a CU, (8 + PL TBN) KiB a step (PL activation planes).  2,048 features x 5,632 k at 1,029

@@ -6,7 +6,8 @@ namespace nvllm {
 // Every launch that is one round takes them.  us, tiles of gemm_b16.hip and here, 2,048 features: K = 5,632 at 256, 512, 900, 1,029,
 // 1,400, 1,600 tokens (heights of 1, 2, 4, 5, 6, 7 blocks) 39 -> 28, 40 -> 29, 42 -> 34, 48 -> 38, 53 -> 42, 54 -> 45; K = 2,048
 // 16.6 -> 10.6, 17.4 -> 11.9, 19.3 -> 16.8, 22.2 -> 18.9, 23.8 -> 21.9, 25.0 -> 23.9; 1,024 features x 1,024 k at 512 and 2,000
-// tokens (1 and 4) 11.1 -> 7.9, 13.7 -> 13.5; 5,632 x 2,048 at 400 (5) 27.8 -> 20.1.
+// tokens (1 and 4) 11.1 -> 7.9, 13.7 -> 13.5; 5,632 x 2,048 at 400 (5) 27.8 -> 20.1; few tiles of a long K too: 256 and 512 features x 8,192 k at
+// 256 tokens (32 and 64 tiles) 54.3 -> 25.8, 52.7 -> 24.9, 512 x 4,096 31.3 -> 14.5.
 bool launch_gemm_waves_b16(const GemmArgs& a) {
     const int tbn = waves_height(a, waves_tallest(1));
     if (!tbn) return false;
