@@ -27,25 +27,29 @@ bool launch_wide_height(const GemmArgs& a, int tbn, int tiles_n, int tiles_t) {
 }
 constexpr int WIDE_HEIGHTS[] = {4, 5, 6, 8, 10, 12, 14, 16};   // token blocks
 
+// Height in token blocks of the tiles that a launch takes, 0: none of these.
+// With one plane of activations a step multiplies for as long as it copies, and the tiles of gemm_b16.hip, three to a CU,
+// come close.  So only launches that are one round here, at the lowest height that fits them into the CUs, and fill most of it: two
+// rounds (484 tiles of 96) 66 -> 69 us.  2,048 k, those against these, layers' weights in turn: four blocks with a tile on 81 % of the CUs
+// 27.1 -> 28.4 (4,864 features, 700 tokens), 27.1 -> 28.2 (3,328, 1,024), 28.2 -> 28.6 (6,656, 512), on 95 % 30.4 -> 29 (5,632, 700); five on
+// 81 % 27.8 -> 24.7 (6,656, 640), on 96 % 36.3 -> 32.1 (4,864, 1,024); six on 81 % 38.4 -> 35.2 (13,312, 380).  Eight waves, two to a SIMD, from
+// eight blocks on: one's requests go out behind the other's products; eight to sixteen on 81 % 33.9 -> 29.4, 45.4 -> 35.8, 48.2 -> 41.7,
+// 51.9 -> 47.8 (6,656; 1,024, 1,280, 1,536, 1,792), 73.9 -> 53.4 (13,312, 1,024).
+int wide_height(int NB, int Kb, int Tb) {
+    // 8: more steps than the deepest ring.  Below 32 steps a launch is mostly start and end, which the smaller tiles overlap.
+    if (Kb < (wide_env() < 0 ? 32 : 8) || wide_env() == 0) return 0;
+    if (wide_env() > 0) return wide_env();
+    const int cus = rt().num_cus, tiles_n = cdiv(NB, 16);
+    for (int h : WIDE_HEIGHTS) {
+        const int tiles = tiles_n * cdiv(Tb, h);
+        if (tiles <= cus) return 100 * tiles < (h == 4 ? 85 : 80) * cus ? 0 : h;
+    }
+    return 0;
+}
 template <int EPI>
 bool launch_wide_b16(const GemmArgs& a) {
-    // 8: more steps than the deepest ring.  Below 32 steps a launch is mostly start and end, which the smaller tiles overlap.
-    if (a.Kb < (wide_env() < 0 ? 32 : 8) || wide_env() == 0) return false;
-    // With one plane of activations a step multiplies for as long as it copies, and the tiles of gemm_b16.hip, three to a CU,
-    // come close.  So only launches that are one round here, at the lowest height that fits them into the CUs, and fill most of it: two
-    // rounds (484 tiles of 96) 66 -> 69 us.  2,048 k, those against these, twelve layers' weights in turn: four blocks with a tile on 81 % of the
-    // CUs 27.1 -> 28.4 (4,864 features, 700 tokens), 27.1 -> 28.2 (3,328, 1,024), 28.2 -> 28.6 (6,656, 512), on 95 % 30.4 -> 29 (5,632, 700); five
-    // on 81 % 27.8 -> 24.7 (6,656, 640); six 36.3 -> 32.1 (4,864, 1,024), 38.4 -> 35.2 (13,312, 380), on 86 % 35.9 -> 34.1 (11,264, 400).  Eight waves,
-    // two to a SIMD, from eight blocks on: one's requests go out behind the other's products; on 81 % 33.9 -> 29.4 (6,656, 1,024), and ten to
-    // sixteen 45.4 -> 35.8, 48.2 -> 41.7, 51.9 -> 47.8, 66.3 -> 50.8 (6,656; 1,280, 1,536, 1,792, 2,000).
-    const int cus = rt().num_cus, tiles_n = cdiv(a.NB, 16);
-    int tbn = 0;
-    for (int h : WIDE_HEIGHTS)
-        if (!tbn && tiles_n * cdiv(a.Tb, h) <= cus) tbn = h;
-    if (wide_env() > 0) tbn = wide_env();
-    const int tiles_t = tbn ? cdiv(a.Tb, tbn) : 0, tiles = tiles_n * tiles_t;
-    if (wide_env() < 0 && (!tbn || 100 * tiles < (tbn == 4 ? 85 : 80) * cus)) return false;
-    return launch_wide_height<EPI, false>(a, tbn, tiles_n, tiles_t);
+    const int tbn = wide_height(a.NB, a.Kb, a.Tb);
+    return tbn && launch_wide_height<EPI, false>(a, tbn, cdiv(a.NB, 16), cdiv(a.Tb, tbn));
 }
 
 }  // namespace
@@ -85,3 +89,16 @@ bool launch_experts_wide_b16(const GemmArgs& a, int pad) {
 }
 
 }  // namespace nvllm
+
+// the rules above, for tests
+extern "C" int nvllm_internal_wide_height(int N, int K, int T) {
+    nvllm::ensure_init();
+    return nvllm::wide_height(nvllm::cdiv(N, 16), nvllm::cdiv(K, 32), nvllm::cdiv(T, 16));
+}
+extern "C" int nvllm_internal_expert_rows_wide(int rows, int experts, int up_n, int up_k, int down_n, int down_k) {
+    nvllm::ensure_init();
+    nvllm::B16Weight up, down;
+    up.N = up_n; up.K = up_k;
+    down.N = down_n; down.K = down_k;
+    return nvllm::expert_rows_wide(rows, experts, up, down);
+}

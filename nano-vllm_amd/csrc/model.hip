@@ -1276,4 +1276,7 @@ int sample(Sampler* s, float* logits) {
     return pick_from_row(s, pl, 0);
 }
 
+// whether the classifier itself stores `num_outputs` rows of a pass that is waited for, for tests
+int nvllm_internal_rows_stored(const RunState* s, int num_outputs, int vocab) { return direct_rows(s, num_outputs, vocab, true) != nullptr; }
+
 }  // extern "C"

@@ -8,7 +8,6 @@ import sys
 import numpy as np
 import pytest
 
-from nvllm_amd import synth
 from tests import hybrid_oracle as O
 from tests.test_gpu_latent_ops import rng, rounded
 from tests.test_gpu_waves import ROOT
@@ -78,45 +77,14 @@ def test_every_height(wants, tmp_path, height):
         assert np.abs(got["y%d" % i] - want).max() < 1e-2 * np.abs(want).max(), SHAPES[i]   # the bar of test_gpu_hybrid_ops.py
 
 
-TIMED_CHILD = """
-import ctypes as C
-import sys
-from nvllm_amd import capi
-from tests import hybrid_util as U
-hip = capi.load_hip()
-best = 1e9
-eng = U.engine(hip, sys.argv[1], False, slots=14, tokens=14 * 512)
-for slot in range(14):
-    hip.nvllm_prof_reset()
-    hip.nvllm_prof_enable(1)
-    eng.feed(slot, U.tokens(512, 203, slot), [511])
-    eng.feed_run()
-    hip.nvllm_prof_enable(0)
-    us = 0.0
-    for c in range(hip.nvllm_prof_num_classes()):
-        n, ms, by, fl = C.c_longlong(), C.c_double(), C.c_double(), C.c_double()
-        hip.nvllm_prof_get(c, C.byref(n), C.byref(ms), C.byref(by), C.byref(fl))
-        if hip.nvllm_prof_name(c) in (b"gemm_expert_up", b"gemm_expert_down"):
-            us += 1e3 * ms.value
-    best = min(best, us)
-eng.close()
-print("US", best)
-"""
-
-
+# sixteen (eight) experts of 2 x ff x width, rows of a batch of T tokens with two choices: those that measured slower in these tiles stay out
 @pytest.mark.gpu
-def test_half_filled_launches_are_left_alone(tmp_path):
-    """64 rows an expert, 128 and 112 tiles of 256 features."""
-    mixer = synth.window_mixer(4, 2, 16, 16, size=64, keep_first=4)
-    path = str(tmp_path / "half")
-    synth.write_model_dir(path, synth.hybrid_config(1792, 203, [(mixer, synth.expert_mlp(1024, 16, 2, 32))]), seed=3)
-
-    def us(**env):
-        base = {k: v for k, v in os.environ.items() if k != "NVLLM_GEMM_WIDE"}
-        r = subprocess.run([sys.executable, "-c", TIMED_CHILD, path], capture_output=True, text=True, timeout=100,
-                           env=dict(base, PYTHONPATH=ROOT + os.pathsep + base.get("PYTHONPATH", ""), **env))
-        assert r.returncode == 0, r.stderr[-2000:]
-        return float(r.stdout.split("US")[1])
-
-    # 57 us in these tiles, 51 in groups of 64 rows; launches differ by two or three percent from process to process
-    assert us() < 1.06 * us(NVLLM_GEMM_WIDE="0")
+@pytest.mark.skipif("NVLLM_GEMM_WIDE" in os.environ, reason="the environment forces a height")
+@pytest.mark.parametrize("width,ff,experts,T,height", [
+    (1792, 1024, 16, 512, 0), (1792, 1024, 16, 640, 0), (1792, 1024, 16, 800, 8), (1664, 832, 16, 800, 0),      # 50 and 44 % of 256 CUs; K of 832
+    (2048, 1152, 16, 400, 0), (2304, 1152, 16, 400, 0), (2048, 1152, 16, 512, 6), (2304, 1152, 16, 512, 6),     # 56 %
+    (3328, 1664, 8, 330, 0), (3328, 1664, 8, 512, 10),                                                          # 41 %
+    (1792, 1280, 16, 330, 4), (2048, 1280, 16, 330, 4), (2560, 1280, 16, 400, 5), (2048, 1408, 16, 1029, 10),   # 62, 62, 62, 69 %
+    (1536, 1280, 16, 800, 0), (2048, 1408, 16, 300, 0), (2048, 1408, 16, 2000, 0)])                             # 37 % of the second; few rows; many
+def test_which_batches_take_them(hip, width, ff, experts, T, height):
+    assert hip.dll.nvllm_internal_expert_rows_wide(2 * T, experts, 2 * ff, width, width, ff) == 16 * height

@@ -1,48 +1,17 @@
-"""Which launches take the 256-feature tiles of bf16 models (csrc/gemm_wide_b16.hip): not those that are slower in them."""
+"""Which launches take the 256-feature tiles of bf16 models (csrc/gemm_wide_b16.hip), and at which height: the sizes whose times stand
+beside the rules, and their neighbours.  (256 CUs.)"""
 import os
-import subprocess
-import sys
 
 import pytest
 
-from nvllm_amd import synth
-from tests.test_gpu_waves import ROOT
-
-CHILD = """
-import ctypes as C
-import sys
-from nvllm_amd import capi
-from tests import latent_util as U
-hip = capi.load_hip()
-eng = U.engine(hip, sys.argv[1], False, slots=14, tokens=14 * 704)
-for slot in range(14):
-    if slot == 2:
-        hip.nvllm_prof_reset()
-        hip.nvllm_prof_enable(1)
-    eng.feed(slot, U.tokens(700, 203, slot), [699])
-    eng.feed_run()
-hip.nvllm_prof_enable(0)
-for c in range(hip.nvllm_prof_num_classes()):
-    n, ms, by, fl = C.c_longlong(), C.c_double(), C.c_double(), C.c_double()
-    hip.nvllm_prof_get(c, C.byref(n), C.byref(ms), C.byref(by), C.byref(fl))
-    if hip.nvllm_prof_name(c) == b"gemm_gateup":
-        print("US", 1e3 * ms.value / n.value)
-eng.close()
-"""
+pytestmark = [pytest.mark.gpu, pytest.mark.skipif("NVLLM_GEMM_WIDE" in os.environ, reason="the environment forces a height")]
 
 
-@pytest.mark.gpu
-def test_tiles_of_four_blocks_on_four_fifths_of_the_chip(tmp_path):
-    """Gated pairs of 4,864 x 2,048 at 700 tokens, 19 x 11 tiles; ten layers, whose weights do not wait in a cache."""
-    path = str(tmp_path / "rule")
-    synth.write_model_dir(path, synth.latent_config(2048, 203, [(synth.latent_mixer(2, 64, 32, 64, 64, 64), 2432)] * 10, streams=1), seed=3)
-
-    def us(**env):
-        base = {k: v for k, v in os.environ.items() if k != "NVLLM_GEMM_WIDE"}
-        r = subprocess.run([sys.executable, "-c", CHILD, path], capture_output=True, text=True, timeout=100,
-                           env=dict(base, PYTHONPATH=ROOT + os.pathsep + base.get("PYTHONPATH", ""), **env))
-        assert r.returncode == 0, r.stderr[-2000:]
-        return float(r.stdout.split("US")[1].split()[0])
-
-    # the mean of 120 launches: 28.4 us in these tiles, 27.1 in those of 128 features, within a percent from process to process
-    assert us() < 1.025 * us(NVLLM_GEMM_WIDE="0")
+@pytest.mark.parametrize("N,K,T,height", [
+    (4864, 2048, 700, 0), (3328, 2048, 1024, 0), (6656, 2048, 512, 0),       # four blocks on 209, 208, 208 CUs
+    (5632, 2048, 700, 4), (6656, 2048, 528, 4),                              # ... on 242 and 234
+    (6656, 2048, 640, 5), (4864, 2048, 1024, 5), (13312, 2048, 380, 6),      # 208, 247, 208
+    (6656, 2048, 1024, 8), (6656, 2048, 1280, 10), (6656, 2048, 1536, 12), (6656, 2048, 1792, 14), (13312, 2048, 1024, 16),   # 208
+    (11264, 2048, 1029, 14), (6656, 992, 1024, 0), (13312, 2048, 1152, 0)])  # a pass of prompts; a short K; more than a round at any height
+def test_heights(hip, N, K, T, height):
+    assert hip.dll.nvllm_internal_wide_height(N, K, T) == height
