@@ -24,8 +24,9 @@
 // reference; only the summation order differs.  Key slices of one column leave
 // (acc, max, sum) partials that k_attn_combine merges.
 //
-// fp16 pool (pages in operand order), k_paged_attn16: see the comment above it.
+// fp16 pool (pages in operand order), k_paged_attn16: see the comment above it; prompts' portions: prompt_attention.hip.
 #include "attn_tile.h"
+#include "prompt_attention.h"
 
 namespace nvllm {
 
@@ -480,6 +481,18 @@ int attn_tokens_per_item(int H, int KVH) {
     return 16 / gt;
 }
 
+LongRuns attn_long_runs(const KvPoolView& pool, int H, int KVH, int hd) {
+    static const int env = getenv("NVLLM_ATTN_LONG") ? atoi(getenv("NVLLM_ATTN_LONG")) : -1;   // 0: none; else the fewest items
+    if (pool.elem_bytes != 2 || hd < 32 || hd % 32 != 0 || env == 0) return {};
+    const int ct = attn_tokens_per_item(H, KVH), ng = H / (16 / ct);
+    // From nine sixteenths of a workgroup for each CU on: with fewer a workgroup's walk, 0.7 (1.1) us per 64 keys of heads of 64 (128), is longer
+    // than the four times as many items that split theirs over four waves take.  us a layer, k_paged_attn16 and prompts, 32 heads on 4 of 64
+    // (16 on 4 of 128): three portions of 512 behind 512 60.4 and 27.6 (64.6 and 30.0), first portions 35.3 and 15.5 (43.2 and 18.7); one of
+    // 512 22.6 and 16.7 (128 items: 23.4 and 23.3), behind 1,500 38.5 and 28.6 (37.8 and 40.2); one of 256 there, 128 items, 21.5 and 25.0; three of
+    // 200, 300 items (152), 43.5 and 30.3 (51.0 and 35.6).  Portions of less than half a run's tokens stay as they were
+    return {4 * ct, 2 * ct, cdiv(env > 0 ? env : rt().num_cus * 9 / 16, ng), std::max(1, rt().num_cus / ng)};
+}
+
 constexpr int MERGE_PAGES = 20;
 void launch_paged_attention(const AttnArgs& a) {
     if (a.T <= 0) return;
@@ -493,7 +506,7 @@ void launch_paged_attention(const AttnArgs& a) {
     if (a.tables && ((16 << bs_shift) != a.pool.block_size || (a.pool.elem_bytes == 2 && bs_shift != 0)))
         NVLLM_FATAL("paged attention supports block sizes 16, 32, 64 ... for fp32 rows and 16 for fp16 pages, got %d", a.pool.block_size);
     if (a.pool.elem_bytes == 2 && !a.tables) NVLLM_FATAL("an fp16 KV pool is always paged");
-    const long base_items = (long)a.n_runs * NG;
+    const long base_items = (long)std::max(a.n_runs, 1) * NG;
     const int pages = (a.max_pos + 16) / 16;
     // Work items are cut into key slices until the chip is full.  fp32 rows: a unit is
     // a wave (the kernel is bound by its own instruction stream: 2 waves per SIMD).
@@ -532,9 +545,10 @@ void launch_paged_attention(const AttnArgs& a) {
         merge_waves = nsplit <= 4 ? 4 : 8;
         nsplit = merge_waves;
     }
-    const long waves = base_items * nsplit;
+    const long waves = (long)a.n_runs * NG * nsplit;
     // a wave per item: at least eight items per CU and at most 16 pages each
     static const int env_solo = getenv("NVLLM_ATTN_SOLO") ? atoi(getenv("NVLLM_ATTN_SOLO")) : -1;
+    if (a.n_long > 0) nsplit = 1;   // (one launch, which the portions fill)
     bool solo = wg_items && nsplit == 1 && pages <= 16 && waves >= (long)rt().num_cus * 8;
     if (env_solo >= 0) solo = wg_items && env_solo > 0;
 
@@ -576,6 +590,10 @@ void launch_paged_attention(const AttnArgs& a) {
         // algorithmic work: keys and values of every sequence read once per kv head; two products per (token, position) pair
         const double kvb = (double)(a.kv_rows ? a.kv_rows : a.kv_positions) * 2.0 * a.KVH * a.hd * a.pool.elem_bytes;
         ProfScope ps(PC_ATTN, kvb + (double)a.T * a.H * a.hd * 8.0, 4.0 * (a.qk_pairs ? (double)a.qk_pairs : (double)a.kv_positions * CT) * a.H * a.hd);
+        if (a.n_long > 0) {
+            launch_prompt_attn16({k, (const int4*)a.long_runs, a.n_long}, a.hd);
+            return;
+        }
         switch (a.hd) {
             case 16: launch_hd<16>(k, waves, a.pool.elem_bytes, solo, once, merge_waves); break;
             case 32: launch_hd<32>(k, waves, a.pool.elem_bytes, solo, once, merge_waves); break;

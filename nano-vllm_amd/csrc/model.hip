@@ -356,6 +356,8 @@ static AttnArgs attn_args(const StepArrays& st, int T, int H, int KVH, int hd, c
     at.max_pos = st.max_pos;
     at.runs = st.d_runs;
     at.n_runs = st.n_runs;
+    at.long_runs = st.d_long;
+    at.n_long = st.n_long;
     at.kv_positions = st.kv_positions;
     at.kv_rows = st.kv_rows;
     at.qk_pairs = st.qk_pairs;
@@ -788,7 +790,8 @@ static long enqueue_pass(int* tokens, int num_tokens, int* pos_arr, int* seq_ids
     const float eps = 1e-5f;  // model.c:361,388,396
 
     StepArrays st = stage_step(tokens, pos_arr, seq_ids, T, output_indices, B, block_tables, nullptr, 0,
-                               g_kv_manager.block_size, attn_tokens_per_item(H, KVH), token_src);
+                               g_kv_manager.block_size, attn_tokens_per_item(H, KVH), token_src, false, false, 0, nullptr,
+                               chain_enabled() && T <= 64 ? LongRuns{} : attn_long_runs(pool_view(&g_kv_manager, KVH, hd), H, KVH, hd));
     // The reference prints "Block table too small" once per layer and then attends over block ids
     // read past the table (attention.c:159-162, 285); here the pass ends before any kernel reads them.
     if (st.table_short) NVLLM_FATAL("transformer_batch: a position lies beyond its sequence's block table (allocate the block first, main.c:320-335)");

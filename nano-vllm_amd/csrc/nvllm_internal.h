@@ -451,12 +451,21 @@ struct AttnArgs {
     int max_pos;           // largest position in the batch (host knowledge, for split sizing)
     const int* runs;       // device int4 (first token, count, last position, table offset): runs of consecutive
     int n_runs;            //   positions of one sequence, at most attn_tokens_per_item() tokens each
+    const int* long_runs;  // the same of portions' tokens that are in no run above, at most attn_long_runs().tokens each
+    int n_long;
     long kv_positions;     // sum over runs of (last position + 1): rows of K/V each kv head reads
     long kv_rows;          // kernel timing: rows of K/V of the batch's sequences, each counted once (0: kv_positions) ...
     long qk_pairs;         // ... and (token, position) pairs
 };
 void launch_paged_attention(const AttnArgs& a);
 int attn_tokens_per_item(int H, int KVH);
+struct LongRuns {          // portions for the kernel of prompts (prompt_attention.hip)
+    int tokens = 0;        // of a run at most; 0: no portion
+    int min_tokens = 0;    // of a portion at least
+    int min_runs = 0;      // of a batch at least, else it has none
+    int round = 1;         // whose items are one for every CU
+};
+LongRuns attn_long_runs(const KvPoolView& pool, int H, int KVH, int hd);
 
 // ---- hyper.hip: hyper-connections with the Dynamic Tanh norm, as launches of their own
 // One hyper-connection step on x [T][streams][ld] (all pointers device; width <= ld, the rest is padding):

@@ -2,6 +2,7 @@
 // launchers: argument checking, host->HBM staging of the integer arrays and block
 // tables, and the host-side KV block allocator.
 #include <algorithm>
+#include <array>
 #include <cstring>
 #include <unordered_map>
 #include <vector>
@@ -52,7 +53,7 @@ KvPoolView pool_view(const KVCacheManager* mgr, int n_kv_heads, int head_dim) {
 StepArrays stage_step(const int* tokens, const int* pos_arr, const int* seq_ids, int T,
                       const int* output_indices, int B, BlockTable** tables, const BlockTable* single,
                       int pos0, int block_size, int attn_ct, const int* token_src, bool multi_first, bool spans, int chunk_len,
-                      const std::vector<int>* extra) {
+                      const std::vector<int>* extra, LongRuns attn_long) {
     StepArrays s{};
     s.T = T;
     s.B = B;
@@ -92,25 +93,51 @@ StepArrays stage_step(const int* tokens, const int* pos_arr, const int* seq_ids,
     for (int i = 1; i < n_seqs; i++) tbl_off[i] = tbl_off[i - 1] + need[i - 1];
     // attention work items: (first token, token count, last position, offset of the
     // sequence's block table) -- everything a wave needs in one 16-byte load
-    std::vector<int> runs;
+    std::vector<int> runs, long_runs;
     s.kv_positions = 0;
     if (attn_ct > 0) {
         auto pos_of = [&](int t) { return pos_arr ? pos_arr[t] : pos0 + t; };
         auto seq_of = [&](int t) { return seq_ids ? seq_ids[t] : 0; };
-        for (int t = 0; t < T;) {
+        auto portion = [&](int t, int most) {   // tokens of one sequence at consecutive positions from t on
             int n = 1;
-            while (t + n < T && n < attn_ct && seq_of(t + n) == seq_of(t) && pos_of(t + n) == pos_of(t + n - 1) + 1) n++;
-            runs.push_back(t);
-            runs.push_back(n);
-            runs.push_back(pos_of(t + n - 1));
-            runs.push_back(tbl_off[seq_of(t)]);
+            while (t + n < T && n < most && seq_of(t + n) == seq_of(t) && pos_of(t + n) == pos_of(t + n - 1) + 1) n++;
+            return n;
+        };
+        auto is_long = [&](int n) { return attn_long.tokens > 0 && n >= attn_long.min_tokens; };
+        if (attn_long.tokens > 0) {
+            int n_long = 0;
+            for (int t = 0, n; t < T; t += n) {
+                n = portion(t, T);
+                if (is_long(n)) n_long += (n + attn_long.tokens - 1) / attn_long.tokens;
+            }
+            if (n_long < attn_long.min_runs) attn_long = {};
+        }
+        auto add = [&](std::vector<int>& to, int t, int n) {
+            to.insert(to.end(), {t, n, pos_of(t + n - 1), tbl_off[seq_of(t)]});
             s.kv_positions += pos_of(t + n - 1) + 1;
             for (int i = 0; i < n; i++) s.qk_pairs += pos_of(t + i) + 1;
             if (n > s.max_run) s.max_run = n;
             for (int tb = t >> 4; tb <= (t + n - 1) >> 4; tb++)
                 if (tb < 4) s.runs_in_tb[tb]++;
+        };
+        for (int t = 0; t < T;) {
+            const int whole = attn_long.tokens > 0 ? portion(t, T) : 0;
+            if (is_long(whole)) {
+                for (int i = 0; i < whole; i += attn_long.tokens) add(long_runs, t + i, std::min(attn_long.tokens, whole - i));
+                t += whole;
+                continue;
+            }
+            const int n = portion(t, attn_ct);
+            add(runs, t, n);
             t += n;
         }
+        // longest walks first, and every second round of the chip backwards: all are resident at once, so a CU's time is its items' sum
+        std::vector<std::array<int, 4>> order(long_runs.size() / 4);
+        for (size_t i = 0; i < order.size(); i++) std::copy_n(long_runs.begin() + 4 * (long)i, 4, order[i].begin());
+        std::stable_sort(order.begin(), order.end(), [](const auto& a, const auto& b) { return a[2] > b[2]; });
+        for (size_t i = (size_t)attn_long.round; i < order.size(); i += 2 * (size_t)attn_long.round)
+            std::reverse(order.begin() + (long)i, order.begin() + (long)std::min(order.size(), i + (size_t)attn_long.round));
+        for (size_t i = 0; i < order.size(); i++) std::copy_n(order[i].begin(), 4, long_runs.begin() + 4 * (long)i);
         if (multi_first) {
             std::vector<int> singles, alone;
             size_t keep = 0;
@@ -152,6 +179,7 @@ StepArrays stage_step(const int* tokens, const int* pos_arr, const int* seq_ids,
         }
     }
     s.n_runs = (int)runs.size() / 4;
+    s.n_long = (int)long_runs.size() / 4;
     std::vector<int> span, span_of;
     if (spans) {
         auto pos_of = [&](int t) { return pos_arr ? pos_arr[t] : pos0 + t; };
@@ -196,7 +224,7 @@ StepArrays stage_step(const int* tokens, const int* pos_arr, const int* seq_ids,
         }
     }
     size_t n_ints = (size_t)(tokens ? T : 0) + (token_src ? T : 0) + (pos_arr ? T : 0) + (seq_ids ? T : 0) + kv_row.size() +
-                          (output_indices ? B : 0) + n_seqs + total_tbl + runs.size() + span.size() + span_of.size() + chunks.size() + first_chunk.size() + 64;
+                          (output_indices ? B : 0) + n_seqs + total_tbl + runs.size() + long_runs.size() + span.size() + span_of.size() + chunks.size() + first_chunk.size() + 64;
     if (extra && n_ints + extra->size() > staging_ints()) extra = nullptr;   // (the caller can do without)
     if (extra) n_ints += extra->size();
     int* host = pinned_ints(n_ints);
@@ -235,6 +263,7 @@ StepArrays stage_step(const int* tokens, const int* pos_arr, const int* seq_ids,
     }
     o = (o + 3) & ~(size_t)3;  // int4 alignment
     s.d_runs = runs.empty() ? nullptr : put(runs.data(), runs.size());
+    s.d_long = long_runs.empty() ? nullptr : put(long_runs.data(), long_runs.size());
     s.d_extra = extra && !extra->empty() ? put(extra->data(), extra->size()) : nullptr;   // (a multiple of four)
     s.d_spans = span.empty() ? nullptr : put(span.data(), span.size());
     s.d_chunks = chunks.empty() ? nullptr : put(chunks.data(), chunks.size());   // (pairs, behind quadruples)
@@ -458,6 +487,8 @@ void multi_head_attention(float* out, float* q, float* key_cache, float* value_c
     a.max_pos = s.max_pos;
     a.runs = s.d_runs;
     a.n_runs = s.n_runs;
+    a.long_runs = s.d_long;
+    a.n_long = s.n_long;
     a.kv_positions = s.kv_positions;
     launch_paged_attention(a);
 }
@@ -470,7 +501,8 @@ void paged_attention(float* out, float* q, KVCacheManager* mgr, BlockTable* bloc
     ensure_init();
     if (num_tokens <= 0) return;
     StepArrays s = stage_step(nullptr, nullptr, nullptr, num_tokens, nullptr, 0, nullptr, block_table, pos,
-                              mgr->block_size, attn_tokens_per_item(n_heads, n_kv_heads));
+                              mgr->block_size, attn_tokens_per_item(n_heads, n_kv_heads), nullptr, false, false, 0, nullptr,
+                              attn_long_runs(pool_view(mgr, n_kv_heads, head_dim), n_heads, n_kv_heads, head_dim));
     // the reference reads block ids past the table here (attention.c:285 has no bounds check);
     // on the GPU that would be a wild read of the pool, so it ends the process instead
     if (s.table_short) NVLLM_FATAL("paged attention: a position lies beyond its sequence's block table");
@@ -487,6 +519,8 @@ void paged_attention(float* out, float* q, KVCacheManager* mgr, BlockTable* bloc
     a.max_pos = s.max_pos;
     a.runs = s.d_runs;
     a.n_runs = s.n_runs;
+    a.long_runs = s.d_long;
+    a.n_long = s.n_long;
     a.kv_positions = s.kv_positions;
     launch_paged_attention(a);
 }
@@ -499,7 +533,8 @@ void paged_attention_batch(float* out, float* q, KVCacheManager* mgr, BlockTable
     ensure_init();
     if (num_tokens <= 0) return;
     StepArrays s = stage_step(nullptr, pos_arr, seq_ids, num_tokens, nullptr, 0, block_tables, nullptr, 0,
-                              mgr->block_size, attn_tokens_per_item(n_heads, n_kv_heads));
+                              mgr->block_size, attn_tokens_per_item(n_heads, n_kv_heads), nullptr, false, false, 0, nullptr,
+                              attn_long_runs(pool_view(mgr, n_kv_heads, head_dim), n_heads, n_kv_heads, head_dim));
     // the reference reads block ids past the table here (attention.c:285 has no bounds check);
     // on the GPU that would be a wild read of the pool, so it ends the process instead
     if (s.table_short) NVLLM_FATAL("paged attention: a position lies beyond its sequence's block table");
@@ -516,6 +551,8 @@ void paged_attention_batch(float* out, float* q, KVCacheManager* mgr, BlockTable
     a.max_pos = s.max_pos;
     a.runs = s.d_runs;
     a.n_runs = s.n_runs;
+    a.long_runs = s.d_long;
+    a.n_long = s.n_long;
     a.kv_positions = s.kv_positions;
     launch_paged_attention(a);
 }

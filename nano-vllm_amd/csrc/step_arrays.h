@@ -23,6 +23,8 @@ struct StepArrays {
     int* d_kv_row;    // [T] pool row (block * block_size + slot) where the token's K/V go, -1: not stored
     int* d_runs;      // [n_runs][4] (first token, count, last position, table offset): attention work items
     int n_runs;
+    int* d_long;      // [n_long][4] the same of portions that take the kernel of prompts (attn_long); their tokens are in no run of d_runs
+    int n_long;
     long kv_positions;
     long kv_rows;            // sum over the batch's sequences of the positions their last token sees
     long qk_pairs;           // sum over tokens of the positions they see
@@ -67,11 +69,13 @@ private:
 // `tables` (indexed by seq id) or `single` (one table, positions pos0 + t) may be
 // null for operators that do not touch the pool.  attn_ct > 0 also cuts the batch into
 // attention work items: runs of at most attn_ct tokens of one sequence at
-// consecutive positions.  multi_first: runs of several tokens come before those of one.
+// consecutive positions.  multi_first: runs of several tokens come before those of one.  attn_long:
+// portions that the kernel of prompts takes are cut into longer runs, listed apart.
 StepArrays stage_step(const int* tokens, const int* pos_arr, const int* seq_ids, int T,
                       const int* output_indices, int B, BlockTable** tables, const BlockTable* single,
                       int pos0, int block_size, int attn_ct = 0, const int* token_src = nullptr, bool multi_first = false,
-                      bool spans = false, int chunk_len = 0, const std::vector<int>* extra = nullptr);
+                      bool spans = false, int chunk_len = 0, const std::vector<int>* extra = nullptr,
+                      LongRuns attn_long = {});
 
 KvPoolView pool_view(const KVCacheManager* mgr, int n_kv_heads, int head_dim);
 
