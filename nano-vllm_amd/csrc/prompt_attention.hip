@@ -10,6 +10,9 @@
 // the matrix cores for the planes).  Bound: issue of about 95 vector instructions, 16 of them exponentials, beside 32 products per 32 keys
 // and 32 columns; the depth of the ring and a fourth workgroup a CU change nothing.  Of the way there: 37 as first written; references that
 // rise at every new maximum, and maxima over all lanes for it, cost 5; walks of three workgroups of a CU that are all long or all short 4 (stage_step).
+// Error against 64 bits (2-norm of the results, queries of size 1, 4 and 30; k_paged_attn16 in brackets, 1e-7): heads of 64 1.42, 3.48, 7.80 (1.47, 3.61,
+// 8.01), of 32 1.34, 3.10, 6.26 (1.46, 3.59, 7.55), of 128 1.55, 3.54, 7.51 (1.52, 3.94, 8.30); with all products of a score in one chain and one set of
+// sums 1.60, 3.87, 8.70 at 64.
 #include "prompt_attention.h"
 
 #include "gemm_common.h"
@@ -114,11 +117,15 @@ __device__ __forceinline__ void prompt_item(const PromptAttnArgs& p, unsigned wi
     for (int j = 0; j < 2; j++)
 #pragma unroll
         for (int c = 0; c < HD / 32; c++) asm volatile("" : "+v"(qh[j][c]), "+v"(ql[j][c]));   // here, not in the loop, whose only loads are the copies
-    pf4_t acc[2][NC];
+    // results; those of the weights' lo plane apart where registers allow, which halves the roundings to the size of the sums
+    constexpr int SUMS = HD < 128 ? 2 : 1;
+    pf4_t acc[SUMS][2][NC];
 #pragma unroll
-    for (int j = 0; j < 2; j++)
+    for (int k = 0; k < SUMS; k++)
 #pragma unroll
-        for (int n = 0; n < NC; n++) acc[j][n] = pf4_t{0.f, 0.f, 0.f, 0.f};
+        for (int j = 0; j < 2; j++)
+#pragma unroll
+            for (int n = 0; n < NC; n++) acc[k][j][n] = pf4_t{0.f, 0.f, 0.f, 0.f};
     float m[2] = {-INFINITY, -INFINITY}, nm[2] = {0.f, 0.f}, lsum[2] = {0.f, 0.f};   // reference (a maximum of products), minus that as an exponent, sum
     float limit[2] = {-INFINITY, -INFINITY};
     const float sl2 = a.scale * 1.44269504088896340736f;
@@ -155,20 +162,30 @@ __device__ __forceinline__ void prompt_item(const PromptAttnArgs& p, unsigned wi
         pf4_t s[2][2];   // [column group][page]
 #pragma unroll
         for (int j = 0; j < 2; j++) s[j][0] = s[j][1] = pf4_t{0.f, 0.f, 0.f, 0.f};
+        ph8_t k[HD / 32][2];
 #pragma unroll
-        for (int c = 0; c < HD / 32; c++) {
-            ph8_t k[2];
+        for (int c = 0; c < HD / 32; c++)
 #pragma unroll
-            for (int page = 0; page < 2; page++) k[page] = pair(lane * 8 + page * W::PAGE + 1024 * c, 512);
+            for (int page = 0; page < 2; page++) k[c][page] = pair(lane * 8 + page * W::PAGE + 1024 * c, 512);
+        pf4_t s2[2][2];   // wide heads: a second chain
 #pragma unroll
-            for (int page = 0; page < 2; page++)
+        for (int j = 0; j < 2; j++) s2[j][0] = s2[j][1] = pf4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                for (int j = 0; j < 2; j++) s[j][page] = __builtin_amdgcn_mfma_f32_16x16x32_f16(k[page], ql[j][c], s[j][page], 0, 0, 0);
+        for (int plane = 0; plane < 2; plane++)   // the small products first, so that they are not rounded to the size of the others
 #pragma unroll
-            for (int page = 0; page < 2; page++)
+            for (int c = 0; c < HD / 32; c++)
 #pragma unroll
-                for (int j = 0; j < 2; j++) s[j][page] = __builtin_amdgcn_mfma_f32_16x16x32_f16(k[page], qh[j][c], s[j][page], 0, 0, 0);
-        }
+                for (int page = 0; page < 2; page++)
+#pragma unroll
+                    for (int j = 0; j < 2; j++) {
+                        pf4_t& sum = HD > 64 && (c & 1) ? s2[j][page] : s[j][page];
+                        sum = __builtin_amdgcn_mfma_f32_16x16x32_f16(k[c][page], plane ? qh[j][c] : ql[j][c], sum, 0, 0, 0);
+                    }
+        if constexpr (HD > 64)
+#pragma unroll
+            for (int j = 0; j < 2; j++)
+#pragma unroll
+                for (int page = 0; page < 2; page++) s[j][page] += s2[j][page];
         if (from + 31 > first_sees) {   // some column does not see all of them
 #pragma unroll
             for (int j = 0; j < 2; j++)
@@ -196,7 +213,9 @@ __device__ __forceinline__ void prompt_item(const PromptAttnArgs& p, unsigned wi
                     const float alpha = __builtin_amdgcn_exp2f((m[j] - mn) * sl2);
                     lsum[j] *= alpha;
 #pragma unroll
-                    for (int n = 0; n < NC; n++) acc[j][n] *= alpha;
+                    for (int k = 0; k < SUMS; k++)
+#pragma unroll
+                        for (int n = 0; n < NC; n++) acc[k][j][n] *= alpha;
                     m[j] = mn;
                     nm[j] = -mn * sl2;
                     limit[j] = mn + LAZY / sl2;
@@ -229,23 +248,28 @@ __device__ __forceinline__ void prompt_item(const PromptAttnArgs& p, unsigned wi
 #pragma unroll
             for (int i = 0; i < 2; i++)
 #pragma unroll
-                for (int j = 0; j < 2; j++) acc[j][n + i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(val[i], ph[j], acc[j][n + i], 0, 0, 0);
+                for (int j = 0; j < 2; j++) acc[0][j][n + i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(val[i], ph[j], acc[0][j][n + i], 0, 0, 0);
 #pragma unroll
             for (int i = 0; i < 2; i++)
 #pragma unroll
-                for (int j = 0; j < 2; j++) acc[j][n + i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(val[i], pl[j], acc[j][n + i], 0, 0, 0);
+                for (int j = 0; j < 2; j++) acc[SUMS - 1][j][n + i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(val[i], pl[j], acc[SUMS - 1][j][n + i], 0, 0, 0);
         }
     }
     // the two waves of 32 columns: each leaves the other's 16 and finishes its own (group j = part)
 #pragma unroll
     for (int j = 0; j < 2; j++) lsum[j] = rows_sum(lsum[j]);
+    if constexpr (SUMS == 2)
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+#pragma unroll
+            for (int n = 0; n < NC; n++) acc[0][j][n] += acc[1][j][n];
     __syncthreads();
     auto area = [&](int w) { return lds + w * (NC * 1024 + 128); };
     {
         unsigned char* mine = area(wave);
         const bool second = part == 0;   // group that this wave leaves
 #pragma unroll
-        for (int n = 0; n < NC; n++) reinterpret_cast<pf4_t*>(mine)[n * 64 + lane] = second ? acc[1][n] : acc[0][n];
+        for (int n = 0; n < NC; n++) reinterpret_cast<pf4_t*>(mine)[n * 64 + lane] = second ? acc[0][1][n] : acc[0][0][n];
         if (g == 0) reinterpret_cast<pf2_t*>(mine + NC * 1024)[x] = second ? pf2_t{m[1], lsum[1]} : pf2_t{m[0], lsum[0]};
     }
     __syncthreads();
@@ -259,7 +283,7 @@ __device__ __forceinline__ void prompt_item(const PromptAttnArgs& p, unsigned wi
     pf4_t o[NC];
 #pragma unroll
     for (int n = 0; n < NC; n++) {
-        const pf4_t mine = part ? acc[1][n] : acc[0][n], his = reinterpret_cast<const pf4_t*>(other)[n * 64 + lane];
+        const pf4_t mine = part ? acc[0][1][n] : acc[0][0][n], his = reinterpret_cast<const pf4_t*>(other)[n * 64 + lane];
 #pragma unroll
         for (int e = 0; e < 4; e++) o[n][e] = fmaf(his[e], f1, mine[e] * f0) * inv;
         if (store && a.out_f32) *reinterpret_cast<pf4_t*>(a.out_f32 + ((size_t)t * a.H + head) * HD + 16 * n + 4 * g) = o[n];
