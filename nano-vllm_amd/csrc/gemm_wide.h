@@ -17,6 +17,8 @@
 // The epilogues are those of gemm_prefill_tile.h.
 #pragma once
 
+#include <climits>
+
 #include "gemm_prefill_tile.h"
 
 namespace nvllm {
@@ -47,7 +49,7 @@ __device__ __forceinline__ void wide_wait() {
 
 // EXP: rows sorted by expert, every tile's of one (ExpertRows)
 template <int TBN, int WT, int EPI, typename KVT, typename OP, bool EXP = false>
-__global__ __launch_bounds__(256 * WT, 1) void k_gemm_wide(GemmArgs p, int tiles_n, int tiles_t) {
+__global__ __launch_bounds__(256 * WT, 1) void k_gemm_wide(GemmArgs p, int tiles_n, int tiles_t, int panel) {
     constexpr int PL = OP::PLANES;
     using G = WideGeom<TBN, PL, WT>;
     constexpr int RING = G::RING, CPW = G::CPW, WAVES = G::WAVES, TBW = TBN / WT;   // TBW: token blocks of a wave
@@ -65,14 +67,16 @@ __global__ __launch_bounds__(256 * WT, 1) void k_gemm_wide(GemmArgs p, int tiles
             return;
         }
     }
-    // every XCD a contiguous range of tiles, token tiles fastest: what runs together behind one L2 shares weights
+    // every XCD a contiguous range of tiles, panel after panel: what runs together behind one L2 shares weights and activations
     const int total = tiles_n * tiles_t;
     int id;
     {
         const int xcd = (int)blockIdx.x & 7, slot = (int)blockIdx.x >> 3, q = total >> 3, r = total & 7;
         id = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + slot;
     }
-    const int nb0 = id / tiles_t * G::FB, tb0 = id % tiles_t * TBN;
+    // a panel: `panel` feature tiles, whose token tiles follow each other, of each all its features
+    const int first = id / (panel * tiles_t) * panel, width = min(panel, tiles_n - first), at = id - first * tiles_t;
+    const int nb0 = (first + at % width) * G::FB, tb0 = at / width * TBN;
     const __half* W = p.W;
     if constexpr (EXP) {
         const int e = __builtin_amdgcn_readfirstlane(p.block_expert[tb0]);
@@ -191,6 +195,22 @@ __global__ __launch_bounds__(256 * WT, 1) void k_gemm_wide(GemmArgs p, int tiles
     pf_epilogue<4, TBW, EPI, KVT, OP>(p, acc, nb0 + wf * 4, wt * TBW, tb0, s_rinv, lane, p.NB);
 }
 
+// Feature tiles of a panel: those with which the tiles that an XCD works on at a time, a contiguous range of its CUs' number, bring the
+// fewest bytes into its L2 (`w` KiB a feature tile and step, `a` a token tile).  One, which is token tiles fastest, has all activations enter every
+// L2: TinyLlama-1.1B's w_down and wo, 200 tiles of 64 tokens, 55.9 us on average, in panels of four 53.9; its gate/up 123.8 and 122.4; with one plane of
+// activations no difference.
+inline int wide_panel(int tiles_n, int tiles_t, int w, int a) {
+    const int range = std::min(cdiv(tiles_n * tiles_t, 8), rt().num_cus / 8);
+    int best = 1;
+    long least = LONG_MAX;
+    for (int panel = 1; panel <= std::min(tiles_n, range); panel++) {
+        const int tokens = std::min(tiles_t, cdiv(range, panel));
+        const long bytes = (long)cdiv(range, tokens) * w + (long)tokens * a;
+        if (bytes < least) least = bytes, best = panel;
+    }
+    return best;
+}
+
 template <int TBN, int EPI, typename KVT, typename OP, int WT = 1, bool EXP = false>
 void launch_wide(GemmArgs a, int tiles_n, int tiles_t) {
     using G = WideGeom<TBN, OP::PLANES, WT>;
@@ -200,7 +220,8 @@ void launch_wide(GemmArgs a, int tiles_n, int tiles_t) {
         enabled = true;
     }
     a.ride_from = tiles_n * tiles_t;
-    NVLLM_LAUNCH((k_gemm_wide<TBN, WT, EPI, KVT, OP, EXP>), dim3(tiles_n * tiles_t + rider_groups(a, tiles_n * tiles_t, G::WAVES)), dim3(64 * G::WAVES), G::LDS, a, tiles_n, tiles_t);
+    NVLLM_LAUNCH((k_gemm_wide<TBN, WT, EPI, KVT, OP, EXP>), dim3(tiles_n * tiles_t + rider_groups(a, tiles_n * tiles_t, G::WAVES)), dim3(64 * G::WAVES), G::LDS, a, tiles_n, tiles_t,
+                 OP::PLANES == 1 ? 1 : wide_panel(tiles_n, tiles_t, G::FB, OP::PLANES * TBN));
 }
 
 // Microseconds a launch takes in tiles of TBN token blocks: rounds of one workgroup per CU, each a start and an end beside its
