@@ -493,6 +493,21 @@ LongRuns attn_long_runs(const KvPoolView& pool, int H, int KVH, int hd) {
     return {4 * ct, 2 * ct, cdiv(env > 0 ? env : rt().num_cus * 9 / 16, ng), std::max(1, rt().num_cus / ng)};
 }
 
+// Do single tokens over fp32 rows take the kernel of row_attention.hip?  One or two heads on a key/value head, no more than two workgroups a
+// CU, and keys that are two trips of a workgroup or, where the items fill the CUs, up to 1,024.  us a layer, k_paged_attn (with its merge's launch
+// where slices leave parts) and rows: 8 heads of 64 (two trips: 512 keys), 1 row of 220 and 500 9.0 and 5.3, 10.0 and 7.9, of 1,000 10.0 and 12.6;
+// 16 rows 9.6 and 6.4, 12.6 and 9.2, 17.9 and 17.4; 32 rows (256 items) of 120, 220, 500, 1,000 7.6 and 6.4, 11.2 and 7.4, 16.7 and 13.2, 26.0 and 22.8; 64
+// 9.9 and 7.9 .. 43.5 and 40.7.  6 of 48, 120 and 240 keys 6.3 and 5.3, 8.6 and 5.5.  16 of 128, 1 and 8 rows of 100 7.6 and 5.4, 8.4 and 6.0, of 1,000
+// 11.7 and 22.9; 32 on 16 of 64, 100 and 300 6.4 and 5.6, 10.8 and 8.5.  More items: 64 of 32, 32 rows of 100 13.1 and 20.4
+static bool rows_alone(const AttnArgs& a, int pages) {
+    static const int env = getenv("NVLLM_ATTN_ROWS") ? atoi(getenv("NVLLM_ATTN_ROWS")) : -1;   // 0: none; else up to that many pages
+    const int group = a.H / a.KVH, cus = rt().num_cus;
+    const long items = (long)a.n_runs * a.KVH;
+    if (a.pool.elem_bytes != 4 || !a.tables || a.n_runs != a.T || (group != 1 && group != 2)) return false;
+    if (env >= 0) return pages <= env;
+    return items <= 2L * cus && pages <= (items >= cus ? 64 : 2 * row_attn_keys(a.hd) / 16);
+}
+
 constexpr int MERGE_PAGES = 20;
 void launch_paged_attention(const AttnArgs& a) {
     if (a.T <= 0) return;
@@ -519,6 +534,7 @@ void launch_paged_attention(const AttnArgs& a) {
     const int target = env_units > 0 ? env_units : (wg_items ? rt().num_cus : 2048);
     int nsplit = (int)((target + base_items / 2) / base_items);
     const int min_pages = wg_items ? 8 : 2;   // pages per slice worth a slice
+    const bool rows = rows_alone(a, pages);
     if (nsplit > (pages + min_pages - 1) / min_pages) nsplit = (pages + min_pages - 1) / min_pages;
     if (nsplit < 1) nsplit = 1;
     // ... and only where the walk that slices take off an item costs more than the merge's launch; more so where the slices are more than
@@ -540,6 +556,7 @@ void launch_paged_attention(const AttnArgs& a) {
     // than the merge's launch) and there are more than a few items: stories42M, a prompt of 301 tokens 615 -> 589 us, of 310 on fp16 weights
     // 428 -> 397; with 32 pages rows lose (3 rows at 700 cached: 317 -> 346), eight items gain nothing
     int merge_waves = 0;
+    if (rows) nsplit = 1;
     if (!wg_items && env_merge && nsplit > 8 && pages <= MERGE_PAGES && base_items >= 16) nsplit = 8;
     if (!wg_items && env_merge && nsplit > 1 && nsplit <= 8) {
         merge_waves = nsplit <= 4 ? 4 : 8;
@@ -592,6 +609,10 @@ void launch_paged_attention(const AttnArgs& a) {
         ProfScope ps(PC_ATTN, kvb + (double)a.T * a.H * a.hd * 8.0, 4.0 * (a.qk_pairs ? (double)a.qk_pairs : (double)a.kv_positions * CT) * a.H * a.hd);
         if (a.n_long > 0) {
             launch_prompt_attn16({k, (const int4*)a.long_runs, a.n_long}, a.hd);
+            return;
+        }
+        if (rows) {
+            launch_row_attn(k, a.hd);
             return;
         }
         switch (a.hd) {

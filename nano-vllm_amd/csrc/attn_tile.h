@@ -41,6 +41,11 @@ struct AttnKArgs {
     int bs_shift;     // fp32 rows: log2(block_size / 16) -- a block holds 2^bs_shift pages of 16 positions
 };
 
+// row_attention.hip: items of one token each over fp32 rows, k.group 1 or 2, all keys of an item in one workgroup
+void launch_row_attn(const AttnKArgs& k, int hd);
+constexpr int row_attn_lanes(int hd) { return hd <= 32 ? 8 : hd <= 64 ? 16 : 32; }        // of a key
+constexpr int row_attn_keys(int hd) { return 64 / row_attn_lanes(hd) * 8 * 8; }            // a workgroup requests together
+
 __device__ __forceinline__ ah4_t as_ah4(au2_t v) { return __builtin_bit_cast(ah4_t, v); }
 
 // Maximum / sum over the four 16-lane rows of a wave (lanes l, l^16, l^32, l^48), the result in all four:
