@@ -495,9 +495,9 @@ LongRuns attn_long_runs(const KvPoolView& pool, int H, int KVH, int hd) {
 
 // Do single tokens over fp32 rows take the kernel of row_attention.hip?  One or two heads on a key/value head, no more than two workgroups a
 // CU, and keys that are two trips of a workgroup or, where the items fill the CUs, up to 1,024.  us a layer, k_paged_attn (with its merge's launch
-// where slices leave parts) and rows: 8 heads of 64 (two trips: 512 keys), 1 row of 220 and 500 9.0 and 5.3, 10.0 and 7.9, of 1,000 10.0 and 12.6;
-// 16 rows 9.6 and 6.4, 12.6 and 9.2, 17.9 and 17.4; 32 rows (256 items) of 120, 220, 500, 1,000 7.6 and 6.4, 11.2 and 7.4, 16.7 and 13.2, 26.0 and 22.8; 64
-// 9.9 and 7.9 .. 43.5 and 40.7.  6 of 48, 120 and 240 keys 6.3 and 5.3, 8.6 and 5.5.  16 of 128, 1 and 8 rows of 100 7.6 and 5.4, 8.4 and 6.0, of 1,000
+// where slices leave parts) and rows: 8 heads of 64 (two trips: 512 keys), 1 row of 220 and 500 9.0 and 4.5, 10.0 and 6.3, of 1,000, four trips, 10.0 and 12.6;
+// 16 rows 9.6 and 5.7, 12.6 and 8.2, 17.9 and 17.4; 32 rows (256 items) of 120, 220, 500, 1,000 7.6 and 6.3, 11.2 and 7.4, 16.7 and 12.8, 26.0 and 22.4; 64
+// 9.9 and 7.9 .. 43.5 and 40.7.  6 of 48, 120 and 240 keys 6.3 and 4.6, 8.6 and 5.0.  16 of 128, 1 and 8 rows of 100 7.6 and 5.4, 8.4 and 6.0, of 1,000
 // 11.7 and 22.9; 32 on 16 of 64, 100 and 300 6.4 and 5.6, 10.8 and 8.5.  More items: 64 of 32, 32 rows of 100 13.1 and 20.4
 static bool rows_alone(const AttnArgs& a, int pages) {
     static const int env = getenv("NVLLM_ATTN_ROWS") ? atoi(getenv("NVLLM_ATTN_ROWS")) : -1;   // 0: none; else up to that many pages

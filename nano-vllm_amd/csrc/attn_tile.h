@@ -11,6 +11,8 @@
 // chain request them (start()) before the projection that produces q has finished.
 #pragma once
 
+#include <type_traits>
+
 #include "nvllm_internal.h"
 
 namespace nvllm {
@@ -58,6 +60,57 @@ __device__ __forceinline__ float rows_max(float x) {
     const unsigned v = __builtin_bit_cast(unsigned, m);
     const auto b = __builtin_amdgcn_permlane16_swap(v, v, false, false);
     return fmaxf(__builtin_bit_cast(float, (unsigned)b[0]), __builtin_bit_cast(float, (unsigned)b[1]));
+}
+
+// What kernels with a key per group of LPK lanes share (row_attention.hip, window_attention.hip): eight keys at a time, of which lane x of
+// a group ends up with number x & 7, so that caps and exponentials are formed once.
+template <int CTRL>
+__device__ __forceinline__ float lane_moved(float x) {
+    const int v = __builtin_bit_cast(int, x);
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(v, v, CTRL, 0xf, 0xf, false));
+}
+template <int LPK>
+__device__ __forceinline__ float eight_sums(const float (&dot)[8], int x) {   // sums over a group's lanes, number x & 7 in lane x
+    float a[4], b[2];
+#pragma unroll
+    for (int i = 0; i < 4; i++) a[i] = (x & 1 ? dot[2 * i + 1] : dot[2 * i]) + lane_moved<0xB1>(x & 1 ? dot[2 * i] : dot[2 * i + 1]);   // (from lane x ^ 1)
+#pragma unroll
+    for (int i = 0; i < 2; i++) b[i] = (x & 2 ? a[2 * i + 1] : a[2 * i]) + lane_moved<0x4E>(x & 2 ? a[2 * i] : a[2 * i + 1]);           // (x ^ 2)
+    const float keep = x & 4 ? b[1] : b[0], give = x & 4 ? b[0] : b[1];
+    if constexpr (LPK == 8) return keep + __shfl_xor(give, 4, 64);
+    float s = keep + lane_moved<0x124>(give);   // a row of 16 turned by four: the other half's, of either eight
+    s += lane_moved<0x128>(s);                  // ... by eight
+    if constexpr (LPK == 32) s += __shfl_xor(s, 16, 64);
+    return s;
+}
+template <int LPK>
+__device__ __forceinline__ float eight_max(float s) {   // over the eight keys, in all lanes of a group
+    s = fmaxf(s, lane_moved<0xB1>(s));
+    s = fmaxf(s, lane_moved<0x4E>(s));
+    return fmaxf(s, LPK == 8 ? __shfl_xor(s, 4, 64) : lane_moved<0x124>(s));   // (lanes x and x + 8 of a row hold the same)
+}
+template <int LPK, int U>
+__device__ __forceinline__ float of_eight(float p, int lane) {   // number U's, in all lanes of a group
+    if constexpr (LPK == 8) return __shfl(p, (lane & ~7) + U, 64);
+    return lane_moved<0x150 + U>(p);
+}
+// o += p[u] v[u]
+template <int LPK>
+__device__ __forceinline__ void add_eight(af4_t& o, float p, const af4_t (&v)[8], int lane) {
+    auto add = [&](auto u) {
+        constexpr int U = decltype(u)::value;
+        const float w = of_eight<LPK, U>(p, lane);
+#pragma unroll
+        for (int e = 0; e < 4; e++) o[e] = fmaf(w, v[U][e], o[e]);
+    };
+    add(std::integral_constant<int, 0>{});
+    add(std::integral_constant<int, 1>{});
+    add(std::integral_constant<int, 2>{});
+    add(std::integral_constant<int, 3>{});
+    add(std::integral_constant<int, 4>{});
+    add(std::integral_constant<int, 5>{});
+    add(std::integral_constant<int, 6>{});
+    add(std::integral_constant<int, 7>{});
 }
 
 // LDS an item's four waves need to merge: (max, sum) per wave and column, accumulators per wave

@@ -3,9 +3,9 @@
 // k_paged_attn multiplies 16 (token, head) columns at a time in v_mfma_f32_16x16x4_f32, of which such a token fills one or two: 1,024
 // matrix-core cycles a page for what the vector unit does in 250, and a page's 16 keys are one dependent chain.  Here a workgroup has a
 // (token, key/value head), LPK lanes a key, four dims each; its waves deal the keys among themselves 64 / LPK at a time and request
-// AHEAD such groups together, so a context of a few hundred tokens is one trip to memory.  Every group of lanes keeps a maximum, a sum
-// and results of its own: nothing crosses lanes but the sum of a score; groups and waves meet once at the end.
-// stories42M, 32 rows of 220 cached positions: 11.2 -> 7.4 us a layer; stories15M, one row of 240: 8.6 -> 5.5 (rows_alone() has both sides).  Bound: the
+// AHEAD such groups together, so a context of a few hundred tokens is one trip to memory.  Every group of lanes keeps a maximum, sums
+// and results of its own: nothing but scores crosses its lanes; groups and waves meet once at the end.
+// stories42M, 32 rows of 220 cached positions: 11.2 -> 7.4 us a layer; stories15M, one row of 240: 8.6 -> 5.0 (rows_alone() has both sides).  Bound: the
 // chain of run, table, rows and the merge, of about a microsecond a step.  fp32 throughout, fused multiply-adds, scale after the dot product, expf.
 #include "attn_tile.h"
 
@@ -13,32 +13,9 @@ namespace nvllm {
 
 namespace {
 
-typedef float rf4_t __attribute__((ext_vector_type(4)));
 typedef const __attribute__((address_space(4))) int* const_int_p;   // read-only for the whole launch: scalar loads
 
 constexpr int ROW_WAVES = 8;
-
-// sum over groups of LPK neighbouring lanes, in all of them
-template <int N>
-__device__ __forceinline__ float row_rotated(float x) {
-    const int v = __builtin_bit_cast(int, x);
-    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(v, v, 0x120 + N, 0xf, 0xf, false));
-}
-template <int LPK>
-__device__ __forceinline__ float lanes_sum(float x) {
-    if constexpr (LPK == 8) {   // (rotations of eight: two rows of eight lanes hold different keys)
-        x += __shfl_xor(x, 4, 64);
-        x += __shfl_xor(x, 2, 64);
-        x += __shfl_xor(x, 1, 64);
-    } else {
-        x += row_rotated<8>(x);
-        x += row_rotated<4>(x);
-        x += row_rotated<2>(x);
-        x += row_rotated<1>(x);
-        if constexpr (LPK == 32) x += __shfl_xor(x, 16, 64);
-    }
-    return x;
-}
 
 template <int HD, int G>
 __global__ __launch_bounds__(64 * ROW_WAVES) void k_row_attn(AttnKArgs a) {
@@ -55,56 +32,55 @@ __global__ __launch_bounds__(64 * ROW_WAVES) void k_row_attn(AttnKArgs a) {
     const int sh = a.bs_shift, groups = last / KEYS + 1;   // groups of keys; the last may go past the token
     const float* pk = reinterpret_cast<const float*>(a.pool_k) + a.layer_off + (size_t)kvh * HD + d;
     const float* pv = reinterpret_cast<const float*>(a.pool_v) + a.layer_off + (size_t)kvh * HD + d;
-    rf4_t q[G], o[G];
+    af4_t q[G], o[G];
     float m[G], l[G];
 #pragma unroll
     for (int h = 0; h < G; h++) {
-        q[h] = *reinterpret_cast<const rf4_t*>(a.q + ((size_t)t * a.H + kvh * G + h) * HD + d);
-        o[h] = rf4_t{0.f, 0.f, 0.f, 0.f};
+        q[h] = *reinterpret_cast<const af4_t*>(a.q + ((size_t)t * a.H + kvh * G + h) * HD + d);
+        o[h] = af4_t{0.f, 0.f, 0.f, 0.f};
         m[h] = -INFINITY, l[h] = 0.f;
     }
     for (int g0 = wave; g0 < groups; g0 += ROW_WAVES * AHEAD) {
-        rf4_t k[AHEAD], v[AHEAD];
-        int key[AHEAD];
+        af4_t k[AHEAD], v[AHEAD];
 #pragma unroll
         for (int u = 0; u < AHEAD; u++) {   // (groups past the last: the last again, not counted)
             const int grp = min(g0 + ROW_WAVES * u, groups - 1), page = grp * KEYS >> 4;
             const long row0 = ((long)table[page >> sh] << (4 + sh)) + ((page & ((1 << sh) - 1)) << 4) + ((grp * KEYS) & 15);
-            key[u] = g0 + ROW_WAVES * u < groups ? grp * KEYS + kg : last + 1;
             const int over = max(grp * KEYS + kg - last, 0);   // keys past the token: its own row again (written, finite)
             const long at = (row0 + kg - over) * a.rowstride;
-            k[u] = *reinterpret_cast<const rf4_t*>(pk + at);
-            v[u] = *reinterpret_cast<const rf4_t*>(pv + at);
+            k[u] = *reinterpret_cast<const af4_t*>(pk + at);
+            v[u] = *reinterpret_cast<const af4_t*>(pv + at);
         }
 #pragma unroll
         for (int h = 0; h < G; h++) {
-            if (!live) q[h] = rf4_t{0.f, 0.f, 0.f, 0.f};
-            float s[AHEAD], top = m[h];
+            if (!live) q[h] = af4_t{0.f, 0.f, 0.f, 0.f};
+            float dot[AHEAD];
 #pragma unroll
             for (int u = 0; u < AHEAD; u++) {
-                float dot = q[h][0] * k[u][0];
+                dot[u] = q[h][0] * k[u][0];
 #pragma unroll
-                for (int e = 1; e < 4; e++) dot = fmaf(q[h][e], k[u][e], dot);
-                s[u] = key[u] <= last ? lanes_sum<LPK>(dot) * a.scale : -INFINITY;
-                top = fmaxf(top, s[u]);
+                for (int e = 1; e < 4; e++) dot[u] = fmaf(q[h][e], k[u][e], dot[u]);
             }
-            const float base = fmaxf(top, -3.0e38f);   // (a group of lanes that has seen no key: exp(-inf - finite) = 0)
-            const float alpha = expf(m[h] - base);
-            l[h] *= alpha;
+            float s = eight_sums<LPK>(dot, x) * a.scale;   // of key number x & 7
+            const int grp = g0 + ROW_WAVES * (x & 7);
+            if (grp * KEYS + kg > last) s = -INFINITY;
+            const float top = fmaxf(m[h], eight_max<LPK>(s)), base = fmaxf(top, -3.0e38f);   // (a group of lanes that has seen no key: exp(-inf - finite) = 0)
+            const float alpha = expf(m[h] - base), p = expf(s - base);
+            l[h] = fmaf(l[h], alpha, p);
             o[h] *= alpha;
             m[h] = top;
-#pragma unroll
-            for (int u = 0; u < AHEAD; u++) {
-                const float p = expf(s[u] - base);
-                l[h] += p;
-#pragma unroll
-                for (int e = 0; e < 4; e++) o[h][e] = fmaf(p, v[u][e], o[h][e]);
-            }
+            add_eight<LPK>(o[h], p, v, lane);
         }
+    }
+#pragma unroll
+    for (int h = 0; h < G; h++) {   // (lanes x and x + 8 hold the same)
+        l[h] += lane_moved<0xB1>(l[h]);
+        l[h] += lane_moved<0x4E>(l[h]);
+        l[h] += LPK == 8 ? __shfl_xor(l[h], 4, 64) : lane_moved<0x124>(l[h]);
     }
     // the groups of lanes of all waves meet
     __shared__ float s_m[G][ROW_WAVES * KEYS], s_l[G][ROW_WAVES * KEYS];
-    __shared__ rf4_t s_o[G][ROW_WAVES * KEYS][LPK];
+    __shared__ af4_t s_o[G][ROW_WAVES * KEYS][LPK];
 #pragma unroll
     for (int h = 0; h < G; h++) {
         if (x == 0) s_m[h][wave * KEYS + kg] = m[h], s_l[h][wave * KEYS + kg] = l[h];
@@ -118,12 +94,12 @@ __global__ __launch_bounds__(64 * ROW_WAVES) void k_row_attn(AttnKArgs a) {
 #pragma unroll
     for (int i = 0; i < ROW_WAVES * KEYS; i++) M = fmaxf(M, s_m[h][i]);
     float L = 0.f;
-    rf4_t sum = {0.f, 0.f, 0.f, 0.f};
+    af4_t sum = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int i = 0; i < ROW_WAVES; i++) {
         const float f = expf(s_m[h][i * KEYS + kg] - M);   // parts without keys carry -inf: weight 0
         L = fmaf(s_l[h][i * KEYS + kg], f, L);
-        const rf4_t part = s_o[h][i * KEYS + kg][x];
+        const af4_t part = s_o[h][i * KEYS + kg][x];
 #pragma unroll
         for (int e = 0; e < 4; e++) sum[e] = fmaf(part[e], f, sum[e]);
     }
@@ -136,7 +112,7 @@ __global__ __launch_bounds__(64 * ROW_WAVES) void k_row_attn(AttnKArgs a) {
     if (kg != 0 || !live) return;
     sum *= 1.0f / L;
     const int head = kvh * G + h;
-    if (a.out_f32) *reinterpret_cast<rf4_t*>(a.out_f32 + ((size_t)t * a.H + head) * HD + d) = sum;
+    if (a.out_f32) *reinterpret_cast<af4_t*>(a.out_f32 + ((size_t)t * a.H + head) * HD + d) = sum;
     if (a.out_a16) {
         const int kk = head * HD + d;
         alignas(8) __half hi[4], lo[4];

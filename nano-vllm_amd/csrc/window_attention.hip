@@ -13,7 +13,7 @@
 // exp(score - cap), no running maximum and no rescaling (exp(-2 * 32) is far inside the range of fp32 and bf16).
 // Scores, caps, maxima and sums are fp32.
 //
-// k_window_attn_any (fp32 rows, and heads too wide for the kernel above): one workgroup per (token, head).
+// k_window_rows (fp32 rows of whole float4s), k_window_attn_any (what is left): one workgroup per (token, head).
 #include "window_attention.h"
 
 #include "attn_tile.h"
@@ -420,6 +420,124 @@ void launch_conv_rope(const ConvRope& c, const KvPages& pool, const StepArrays& 
     if (pool.elem_bytes == 4) NVLLM_LAUNCH((k_conv_rope<float, 1>), grid, dim3(256), 0, a);
     else if (wide) NVLLM_LAUNCH((k_conv_rope<__bf16, 8>), grid, dim3(256), 0, a);
     else NVLLM_LAUNCH((k_conv_rope<__bf16, 1>), grid, dim3(256), 0, a);
+}
+
+// ------------------------------------------------------------------ attention, fp32 rows of whole float4s
+// The scheme of row_attention.hip for a window and kept first tokens: a workgroup per (token, head), LPK lanes a key (four dims each, up to
+// 4 LPK), the waves deal the keys among themselves 64 / LPK at a time and request AHEAD such groups together; every group of lanes keeps a
+// maximum, a sum and results of its own, and they meet once at the end.  What bounds it is the chain position and sequence, table, block,
+// rows, merge.  80 tokens x 16 heads of 64, up to 200 keys: 13.6 us in k_window_attn_any (keys' rows, scores, maxima and weights one after the other
+// through LDS), 9.4 here (12.0 with the cap and the exponential formed by every lane of a key).
+template <int LPK, int WAVES, bool CAP>
+__global__ __launch_bounds__(64 * WAVES) void k_window_rows(KvPages pool, const float* __restrict__ q, float scale, float cap, int size, int keep,
+                                                            const int* __restrict__ pos, const int* __restrict__ seq, const int* __restrict__ tbl_off,
+                                                            const int* __restrict__ tables, int H, float* __restrict__ out, int shift) {   // shift: log2 of the block size, -1: it is no power of two
+    typedef const __attribute__((address_space(4))) int* scalar_int_p;   // read-only for the whole launch
+    constexpr int KEYS = 64 / LPK, AHEAD = 8;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), x = lane & (LPK - 1), kg = lane / LPK;
+    const int t = blockIdx.x, h = blockIdx.y, g = h / (H / pool.G), dim = pool.dim, vdim = pool.vdim;
+    const int p = ((scalar_int_p)(uintptr_t)pos)[t], first_block = ((scalar_int_p)(uintptr_t)tbl_off)[((scalar_int_p)(uintptr_t)seq)[t]];
+    const int* table = tables + first_block;
+    const int lo = max(0, p - size + 1), first = min(keep, lo), n_keys = first + p - lo + 1;
+    const bool has = 4 * x < dim, has_v = 4 * x < vdim;
+    const int d = has ? 4 * x : 0, dv = has_v ? 4 * x : 0;
+    const f4_t zero = {0.f, 0.f, 0.f, 0.f};
+    f4_t qv = *reinterpret_cast<const f4_t*>(q + ((size_t)t * H + h) * dim + d), o = zero;
+    if (!has) qv = zero;
+    float m = -INFINITY, l = 0.f;
+    for (int k0 = wave * KEYS + kg; k0 - kg < n_keys; k0 += KEYS * WAVES * AHEAD) {   // (the condition is the wave's)
+        int row[AHEAD];
+#pragma unroll
+        for (int u = 0; u < AHEAD; u++) {   // (past the last key: the last again, not counted)
+            const int i = min(k0 + KEYS * WAVES * u, n_keys - 1), key = i < first ? i : lo + i - first;
+            row[u] = shift >= 0 ? (table[key >> shift] << shift) + (key & ((1 << shift) - 1)) : table[key / pool.block_size] * pool.block_size + key % pool.block_size;
+        }
+        f4_t k[AHEAD], v[AHEAD];
+#pragma unroll
+        for (int u = 0; u < AHEAD; u++) {
+            const size_t at = (size_t)row[u] * pool.G + g;
+            k[u] = *reinterpret_cast<const f4_t*>((const float*)pool.keys + at * dim + d);
+            v[u] = *reinterpret_cast<const f4_t*>((const float*)pool.values + at * vdim + dv);
+        }
+        float dot[AHEAD];
+#pragma unroll
+        for (int u = 0; u < AHEAD; u++) {
+            dot[u] = qv[0] * k[u][0];
+#pragma unroll
+            for (int e = 1; e < 4; e++) dot[u] = fmaf(qv[e], k[u][e], dot[u]);
+        }
+        float s = eight_sums<LPK>(dot, x) * scale;   // of key number x & 7
+        if constexpr (CAP) s = cap * tanhf(s / cap);
+        if (k0 + KEYS * WAVES * (x & 7) >= n_keys) s = -INFINITY;
+        const float top = fmaxf(m, eight_max<LPK>(s)), base = fmaxf(top, -3.0e38f);   // (a group of lanes that has seen no key: exp(-inf - finite) = 0)
+        const float alpha = expf(m - base), w = expf(s - base);
+        l = fmaf(l, alpha, w);
+        o *= alpha;
+        m = top;
+        add_eight<LPK>(o, w, v, lane);
+    }
+    l += lane_moved<0xB1>(l);   // (lanes x and x + 8 hold the same)
+    l += lane_moved<0x4E>(l);
+    l += lane_moved<0x124>(l);
+    __shared__ float s_m[WAVES * KEYS], s_l[WAVES * KEYS];
+    __shared__ f4_t s_o[WAVES * KEYS][LPK];
+    if (x == 0) s_m[wave * KEYS + kg] = m, s_l[wave * KEYS + kg] = l;
+    s_o[wave * KEYS + kg][x] = o;
+    __syncthreads();
+    if (wave > 0) return;
+    float M = -INFINITY, L = 0.f;
+#pragma unroll
+    for (int i = 0; i < WAVES * KEYS; i++) M = fmaxf(M, s_m[i]);
+    f4_t sum = zero;
+#pragma unroll
+    for (int i = 0; i < WAVES; i++) {
+        const float f = expf(s_m[i * KEYS + kg] - M);   // parts without keys carry -inf: weight 0
+        L = fmaf(s_l[i * KEYS + kg], f, L);
+        const f4_t part = s_o[i * KEYS + kg][x];
+#pragma unroll
+        for (int e = 0; e < 4; e++) sum[e] = fmaf(part[e], f, sum[e]);
+    }
+#pragma unroll
+    for (int w = LPK; w < 64; w <<= 1) {
+        L += __shfl_xor(L, w, 64);
+#pragma unroll
+        for (int e = 0; e < 4; e++) sum[e] += __shfl_xor(sum[e], w, 64);
+    }
+    if (kg == 0 && has_v) *reinterpret_cast<f4_t*>(out + ((size_t)t * H + h) * vdim + dv) = sum * (1.0f / L);
+}
+// false: not for these heads
+static bool launch_window_rows(const WindowAttn& w, const StepArrays& st) {
+    const KvPages& pool = w.pool;
+    const int widest = std::max(pool.dim, pool.vdim);
+    if (pool.elem_bytes != 4 || pool.dim % 4 || pool.vdim % 4 || widest > 128) return false;
+    // us a layer, k_window_attn_any and these, 16 heads of 64 (128), a window of 512 and 16 kept: 1 row of 40 and 300 cached 5.2 and 4.6, 13.0 and 7.9 (5.9
+    // and 4.7, 17.2 and 11.0), 32 rows of 600 26.3 and 18.4 (38.4 and 29.6), prompts of 100, 200, 400 9.7 and 8.6, 23.1 and 19.8, 50.5 and 44.3 (11.1 and
+    // 11.2, 29.6 and 28.4, 66.6 and 70.4: wide heads of many tokens stay there)
+    if (widest > 64 && (long)st.T * w.H > 16L * rt().num_cus) return false;
+    const long keys = std::min((long)st.max_pos + 1, (long)w.size + w.keep_first);
+    // eight waves where four would walk more than two trips and the workgroups are not many
+    const bool many = widest <= 64 ? keys > 256 : keys > 128, eight = many && (long)st.T * w.H <= 4L * rt().num_cus;
+    int shift = 0;
+    while ((1 << shift) < pool.block_size) shift++;
+    if ((1 << shift) != pool.block_size) shift = -1;
+    auto go = [&](auto lpk, auto waves) {
+        constexpr int LPK = decltype(lpk)::value, WAVES = decltype(waves)::value;
+        const dim3 grid(st.T, w.H), block(64 * WAVES);
+        if (w.cap > 0.f)
+            NVLLM_LAUNCH((k_window_rows<LPK, WAVES, true>), grid, block, 0, pool, (const float*)w.q, w.scale, w.cap, w.size, w.keep_first, st.d_pos, st.d_seq, st.d_tbl_off,
+                         st.d_tables, w.H, w.out_f32, shift);
+        else
+            NVLLM_LAUNCH((k_window_rows<LPK, WAVES, false>), grid, block, 0, pool, (const float*)w.q, w.scale, w.cap, w.size, w.keep_first, st.d_pos, st.d_seq, st.d_tbl_off,
+                         st.d_tables, w.H, w.out_f32, shift);
+    };
+    using std::integral_constant;
+    auto by_waves = [&](auto lpk) {
+        if (eight) go(lpk, integral_constant<int, 8>{});
+        else go(lpk, integral_constant<int, 4>{});
+    };
+    if (widest <= 64) by_waves(integral_constant<int, 16>{});
+    else by_waves(integral_constant<int, 32>{});
+    return true;
 }
 
 // ------------------------------------------------------------------ attention, any size
@@ -922,6 +1040,7 @@ void launch_window_attention(const WindowAttn& w, const StepArrays& st) {
         const size_t lds = ((size_t)pool.dim_ld + pool.vdim_ld + 256 + 8 + 256) * 4;
         if (lds > 64 * 1024) NVLLM_FATAL("attention heads of %d and %d values are too wide", pool.dim, pool.vdim);
         ProfScope ps(PC_WINDOW_ATTN, 0, 0);
+        if (launch_window_rows(w, st)) return;
         if (pool.elem_bytes != 4) launch_window_any<true, 1>(w, st, Kb_out);
         else if (pool.dim % 4 || pool.vdim % 4) launch_window_any<false, 1>(w, st, Kb_out);
         else launch_window_any<false, 4>(w, st, Kb_out);
