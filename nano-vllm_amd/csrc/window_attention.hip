@@ -204,6 +204,100 @@ __global__ __launch_bounds__(256) void k_conv_rope(ConvKArgs a) {
     }
 }
 
+// The same for fp32 rows and KEEP + 1 taps, a channel (and its rotation partner) per thread: all that a thread needs -- its inputs, for a portion's
+// first token also those of the tokens that still see the state, and the ones that renew it; taps and angles -- is requested together, behind
+// the look-up of the portion.  80 tokens of a prompt and rows, 1,536 channels, four taps: 10.1 us in k_conv_rope, which takes the first
+// tokens and the rows of the state one after the other, 4.9 here.
+template <int KEEP>
+__global__ __launch_bounds__(256) void k_conv_rope_f32(ConvKArgs a) {
+    const int item = blockIdx.y * 256 + threadIdx.x, t_mine = blockIdx.x;
+    if (item >= a.items) return;
+    const int4 span = a.spans[a.span_of[t_mine]];   // (first token, count, first position, sequence)
+    const int off_mine = t_mine - span.x;
+    if (off_mine > 0 && off_mine < KEEP) return;    // (the first token's)
+    const int n_mine = off_mine == 0 ? min(span.y, KEEP) : 1;
+    int part, head, at, i = item;
+    if (i < a.c.H * a.items_q) {
+        part = 0;
+        head = i / a.items_q;
+        at = i - head * a.items_q;
+    } else if ((i -= a.c.H * a.items_q) < a.pool.G * a.items_k) {
+        part = 1;
+        head = i / a.items_k;
+        at = i - head * a.items_k;
+    } else {
+        i -= a.pool.G * a.items_k;
+        part = 2;
+        head = i / a.items_v;
+        at = i - head * a.items_v;
+    }
+    const int half = part == 2 ? 0 : a.c.rot >> 1;
+    const bool turns = at < half;
+    const int d0 = turns ? at : 2 * half + (at - half), dim = part == 2 ? a.pool.vdim : a.pool.dim;
+    const int ch = (part == 0 ? 0 : part == 1 ? a.QD : a.QD + a.KD) + head * dim + d0, partner = turns ? half : 0;
+    const float* raw = reinterpret_cast<const float*>(a.c.raw) + (size_t)span.x * a.c.raw_ld + ch;
+    float* state = reinterpret_cast<float*>(a.c.state) + (size_t)span.w * KEEP * a.channels + ch;
+    constexpr int N = 2 * KEEP;   // inputs of tokens off_mine - KEEP .. (the last KEEP - 1 for a portion's first token only)
+    float in[N], inz[N], tail[KEEP], tailz[KEEP], w[KEEP + 1], wz[KEEP + 1];
+    float2 turn[KEEP];
+    int rows[KEEP];
+    // the projected value at place `off` of this portion: from the state where negative, zero before the sequence
+    auto input = [&](int off, float& v, float& z) {
+        const bool old = off < 0, none = old && span.z + off < 0;
+        const float* src = old && !none ? state + (size_t)(KEEP + off) * a.channels : raw + (size_t)max(off, 0) * a.c.raw_ld;
+        v = src[0];
+        z = src[partner];
+        if (none) v = z = 0.f;
+    };
+#pragma unroll
+    for (int j = 0; j < N; j++)
+        if (j <= KEEP || off_mine == 0) input(min(off_mine - KEEP + j, span.y - 1), in[j], inz[j]);
+    if (off_mine == 0) {
+#pragma unroll
+        for (int r = 0; r < KEEP; r++) input(span.y - KEEP + r, tail[r], tailz[r]);
+    }
+#pragma unroll
+    for (int j = 0; j <= KEEP; j++) {
+        w[j] = a.c.taps[(size_t)j * a.channels + ch];
+        wz[j] = a.c.taps[(size_t)j * a.channels + ch + partner];
+    }
+#pragma unroll
+    for (int k = 0; k < KEEP; k++) {
+        const int off = off_mine + min(k, n_mine - 1);
+        turn[k] = turns ? a.c.rope[(size_t)(span.z + off) * half + d0] : make_float2(1.f, 0.f);
+        rows[k] = a.kv_row[span.x + off];
+    }
+#pragma unroll
+    for (int k = 0; k < KEEP; k++) {
+        float y = 0.f, z = 0.f;
+#pragma unroll
+        for (int j = 0; j <= KEEP; j++) {
+            y = fmaf(w[j], in[k + j], y);
+            z = fmaf(wz[j], inz[k + j], z);
+        }
+        const float u = y, v = z;
+        if (turns) {
+            y = u * turn[k].x - v * turn[k].y;
+            z = v * turn[k].x + u * turn[k].y;
+        }
+        float* dst = nullptr;
+        if (k >= n_mine) dst = nullptr;
+        else if (part == 0) dst = reinterpret_cast<float*>(a.c.q_out) + ((size_t)(t_mine + k) * a.c.H + head) * a.pool.dim_ld + d0;
+        else if (rows[k] >= 0) dst = reinterpret_cast<float*>(part == 1 ? a.pool.keys : a.pool.values) + ((size_t)rows[k] * a.pool.G + head) * dim + d0;
+        if (dst) {
+            dst[0] = y;
+            if (turns) dst[half] = z;
+        }
+    }
+    if (off_mine == 0) {   // (everything of the old state that this thread needs has been read)
+#pragma unroll
+        for (int r = 0; r < KEEP; r++) {
+            state[(size_t)r * a.channels] = tail[r];
+            if (turns) state[(size_t)r * a.channels + half] = tailz[r];
+        }
+    }
+}
+
 // The same for bf16 rows of 16-byte pieces and KEEP + 1 taps: a thread walks TOK neighbouring tokens with the taps and the
 // last KEEP inputs in registers (what the tokens need is requested up front), and on to the end of those that see the state
 // of a portion that starts among them.
@@ -414,6 +508,15 @@ void launch_conv_rope(const ConvRope& c, const KvPages& pool, const StepArrays& 
             case 3: launch_walk<2>(a, st.T); break;
             case 4: launch_walk<3>(a, st.T); break;
             default: launch_walk<4>(a, st.T); break;
+        }
+        return;
+    }
+    if (pool.elem_bytes == 4 && c.taps && c.n_taps >= 2 && c.n_taps <= 5) {
+        switch (c.n_taps) {
+            case 2: NVLLM_LAUNCH(k_conv_rope_f32<1>, grid, dim3(256), 0, a); break;
+            case 3: NVLLM_LAUNCH(k_conv_rope_f32<2>, grid, dim3(256), 0, a); break;
+            case 4: NVLLM_LAUNCH(k_conv_rope_f32<3>, grid, dim3(256), 0, a); break;
+            default: NVLLM_LAUNCH(k_conv_rope_f32<4>, grid, dim3(256), 0, a); break;
         }
         return;
     }
