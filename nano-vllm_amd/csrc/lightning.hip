@@ -460,7 +460,8 @@ __global__ __launch_bounds__(256) void k_lightning_step(Lightning a, const int4*
 // fp32 portions whose state fits the workgroup's registers (a thread: four value columns x NR dims): the state is read and
 // written once per portion instead of once per token, and BATCH tokens' rows and partial results pass through LDS together.
 // What is left is a batch's chain: rows to LDS, eight tokens of products, the sum over lanes and waves.  A portion of 77
-// tokens x 16 heads of 64 x 64: 142 us with the state streamed, 53 with a token's rows fetched when it comes, 33 so.
+// tokens x 16 heads of 64 x 64: 142 us with the state streamed, 53 with a token's rows fetched when it comes, 33 with dims dealt in turn and sums
+// through the LDS crossbar, 22.7 with a thread's dims side by side (one read of q and k for four) and sums of two values per row swap.
 template <int NR>
 __global__ __launch_bounds__(256) void k_lightning_portion(Lightning a, const int4* __restrict__ spans) {
     constexpr int BATCH = 8, ITEMS = 5;
@@ -472,13 +473,13 @@ __global__ __launch_bounds__(256) void k_lightning_portion(Lightning a, const in
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, h = blockIdx.x;
     const int4 span = spans[blockIdx.y];
     const float decay = a.decay[h * (CH + 1) + 1];
-    const int per = a.vdim / 4, rows = 256 / per, row0 = tid / per, col = (tid - row0 * per) * 4;   // per: 8, 16, 32 or 64; dims row0 + rows r
+    const int per = a.vdim / 4, row0 = tid / per * NR, col = tid % per * 4;   // per: 8, 16, 32 or 64; dims row0 .. row0 + NR - 1
     float* st = a.state + ((size_t)span.w * a.H + h) * a.dim * a.vdim;
     f4_t S[NR];
 #pragma unroll
     for (int r = 0; r < NR; r++) {
         S[r] = f4_t{0.f, 0.f, 0.f, 0.f};
-        if (span.z > 0) S[r] = *reinterpret_cast<const f4_t*>(st + (size_t)(row0 + rows * r) * a.vdim + col);   // (a sequence's first token: from zero)
+        if (span.z > 0) S[r] = *reinterpret_cast<const f4_t*>(st + (size_t)(row0 + r) * a.vdim + col);   // (a sequence's first token: from zero)
     }
     // the float4s of a batch's rows that this thread brings: q, k and v of a token lie behind one another, as in LDS
     const int token4 = (2 * a.dim + a.vdim) / 4;
@@ -514,23 +515,51 @@ __global__ __launch_bounds__(256) void k_lightning_portion(Lightning a, const in
             const float keep = u < n ? decay : 1.f;
             part[u] = f4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int r = 0; r < NR; r++) {
-                const float kd = s_k[u * a.dim + row0 + rows * r], qd = s_q[u * a.dim + row0 + rows * r];
+            for (int r0 = 0; r0 < NR; r0 += 4) {
+                const f4_t kd = *reinterpret_cast<const f4_t*>(s_k + u * a.dim + row0 + r0), qd = *reinterpret_cast<const f4_t*>(s_q + u * a.dim + row0 + r0);
+#pragma unroll
+                for (int r = 0; r < 4; r++)
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        S[r0 + r][e] = fmaf(kd[r], v[e], keep * S[r0 + r][e]);
+                        part[u][e] = fmaf(qd[r], S[r0 + r][e], part[u][e]);
+                    }
+            }
+            if (NR == 16) __builtin_amdgcn_sched_barrier(0);   // (all tokens' rows at once would not fit the registers)
+        }
+        if (per == 16) {
+            // the wave's four rows of lanes: two values a row swap, whose sum is the one's total in one half and the other's in the other
+            f4_t two[BATCH / 2];
+#pragma unroll
+            for (int u = 0; u < BATCH / 2; u++)
 #pragma unroll
                 for (int e = 0; e < 4; e++) {
-                    S[r][e] = fmaf(kd, v[e], keep * S[r][e]);
-                    part[u][e] = fmaf(qd, S[r][e], part[u][e]);
+                    const float a0 = part[2 * u][e], a1 = part[2 * u + 1][e];
+                    const auto x = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, a0), __builtin_bit_cast(unsigned, a1), false, false);
+                    two[u][e] = __builtin_bit_cast(float, (unsigned)x[0]) + __builtin_bit_cast(float, (unsigned)x[1]);
                 }
+            const int g = lane >> 4;
+#pragma unroll
+            for (int u = 0; u < BATCH / 2; u += 2) {
+                f4_t sum;
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const float a0 = two[u][e], a1 = two[u + 1][e];
+                    const auto x = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, a0), __builtin_bit_cast(unsigned, a1), false, false);
+                    sum[e] = __builtin_bit_cast(float, (unsigned)x[0]) + __builtin_bit_cast(float, (unsigned)x[1]);
+                }
+                *reinterpret_cast<f4_t*>(s_part + ((2 * u + 2 * (g & 1) + (g >> 1)) * 4 + wave) * a.vdim + col) = sum;   // row g: token 2 u + 0, 2, 1, 3
             }
+        } else {
+            for (int o = per; o < 64; o <<= 1)
+#pragma unroll
+                for (int u = 0; u < BATCH; u++)
+#pragma unroll
+                    for (int e = 0; e < 4; e++) part[u][e] += __shfl_xor(part[u][e], o, 64);
+            if (lane < per)
+#pragma unroll
+                for (int u = 0; u < BATCH; u++) *reinterpret_cast<f4_t*>(s_part + (u * 4 + wave) * a.vdim + col) = part[u];
         }
-        for (int o = per; o < 64; o <<= 1)
-#pragma unroll
-            for (int u = 0; u < BATCH; u++)
-#pragma unroll
-                for (int e = 0; e < 4; e++) part[u][e] += __shfl_xor(part[u][e], o, 64);
-        if (lane < per)
-#pragma unroll
-            for (int u = 0; u < BATCH; u++) *reinterpret_cast<f4_t*>(s_part + (u * 4 + wave) * a.vdim + col) = part[u];
         __syncthreads();
         for (int i = tid; i < n * a.vdim; i += 256) {
             const int u = i / a.vdim, v = i - u * a.vdim;
@@ -540,7 +569,7 @@ __global__ __launch_bounds__(256) void k_lightning_portion(Lightning a, const in
         // (the next batch's rows are free: everybody is past the barrier above; its partial results wait for the barrier behind the rows)
     }
 #pragma unroll
-    for (int r = 0; r < NR; r++) *reinterpret_cast<f4_t*>(st + (size_t)(row0 + rows * r) * a.vdim + col) = S[r];
+    for (int r = 0; r < NR; r++) *reinterpret_cast<f4_t*>(st + (size_t)(row0 + r) * a.vdim + col) = S[r];
 }
 // false: not for these heads
 static bool launch_portion(const Lightning& a, const int4* spans, const dim3& grid) {
