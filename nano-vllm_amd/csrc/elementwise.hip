@@ -202,9 +202,12 @@ void launch_gather_rows_f32(float* dst, const float* src, const int* idx, int B,
 // ------------------------------------------------------------------ RMSNorm
 // ops.h rms_norm (reference layers.c:23-38).  One workgroup per row; arithmetic per
 // element as layers.c:32-35: r = 1/sqrtf(ss/D + eps), out = (x * r) * g.  (Inside the
-// forward pass RMSNorm is folded into the projections, see gemm.hip.)
+// forward pass RMSNorm is folded into the projections, see gemm.hip.)  GATE: times the sigmoid of a gate of the same shape (the fp32 path
+// of linear attention; as a launch of its own the gate took 4.7 us for 80 rows of 1,024, here nothing).
+__device__ __forceinline__ float gate_sigmoid(float z) { return __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(z * -1.44269504088896340736f)); }
+template <bool GATE>
 __global__ __launch_bounds__(256) void k_rmsnorm(float* out, const float* x, const float* __restrict__ gain, int D,
-                                                 float eps) {
+                                                 float eps, const float* __restrict__ gate) {
     __shared__ float red[17];
     const float* xr = x + (size_t)blockIdx.x * D;
     float ss = 0.f;
@@ -223,13 +226,20 @@ __global__ __launch_bounds__(256) void k_rmsnorm(float* out, const float* x, con
         y.y = __fmul_rn(__fmul_rn(v.y, rinv), g.y);
         y.z = __fmul_rn(__fmul_rn(v.z, rinv), g.z);
         y.w = __fmul_rn(__fmul_rn(v.w, rinv), g.w);
+        if constexpr (GATE) {
+            const float4 z = *reinterpret_cast<const float4*>(gate + (size_t)blockIdx.x * D + i);
+            y.x *= gate_sigmoid(z.x);
+            y.y *= gate_sigmoid(z.y);
+            y.z *= gate_sigmoid(z.z);
+            y.w *= gate_sigmoid(z.w);
+        }
         *reinterpret_cast<float4*>(o + i) = y;
     }
 }
 
 // generic width (not a multiple of 4): scalar loops, fp32 output only
 __global__ __launch_bounds__(256) void k_rmsnorm_any(float* out, const float* x,
-                                                     const float* __restrict__ gain, int D, float eps) {
+                                                     const float* __restrict__ gain, int D, float eps, const float* __restrict__ gate) {
     __shared__ float red[17];
     const float* xr = x + (size_t)blockIdx.x * D;
     float* o = out + (size_t)blockIdx.x * D;
@@ -237,16 +247,19 @@ __global__ __launch_bounds__(256) void k_rmsnorm_any(float* out, const float* x,
     for (int i = threadIdx.x; i < D; i += blockDim.x) ss += xr[i] * xr[i];
     ss = block_sum(ss, red);
     const float rinv = __fdiv_rn(1.0f, sqrtf(__fadd_rn(__fdiv_rn(ss, (float)D), eps)));
-    for (int i = threadIdx.x; i < D; i += blockDim.x) o[i] = __fmul_rn(__fmul_rn(xr[i], rinv), gain[i]);
+    for (int i = threadIdx.x; i < D; i += blockDim.x) {
+        const float y = __fmul_rn(__fmul_rn(xr[i], rinv), gain[i]);
+        o[i] = gate ? y * gate_sigmoid(gate[(size_t)blockIdx.x * D + i]) : y;
+    }
 }
 
-void launch_rmsnorm_f32(float* o, const float* x, const float* gain, int D, int T, float eps) {
+void launch_rmsnorm_f32(float* o, const float* x, const float* gain, int D, int T, float eps, const float* gate) {
     if (T <= 0) return;
-    ProfScope ps(PC_RMSNORM, (double)T * D * 8.0, 0);
-    if (D % 4 == 0 && ((uintptr_t)o % 16 == 0) && ((uintptr_t)x % 16 == 0) && ((uintptr_t)gain % 16 == 0))
-        NVLLM_LAUNCH(k_rmsnorm, dim3(T), dim3(256), 0, o, x, gain, D, eps);
-    else
-        NVLLM_LAUNCH(k_rmsnorm_any, dim3(T), dim3(256), 0, o, x, gain, D, eps);
+    ProfScope ps(PC_RMSNORM, (double)T * D * (gate ? 12.0 : 8.0), 0);
+    const bool quads = D % 4 == 0 && ((uintptr_t)o % 16 == 0) && ((uintptr_t)x % 16 == 0) && ((uintptr_t)gain % 16 == 0) && ((uintptr_t)gate % 16 == 0);
+    if (quads && gate) NVLLM_LAUNCH(k_rmsnorm<true>, dim3(T), dim3(256), 0, o, x, gain, D, eps, gate);
+    else if (quads) NVLLM_LAUNCH(k_rmsnorm<false>, dim3(T), dim3(256), 0, o, x, gain, D, eps, gate);
+    else NVLLM_LAUNCH(k_rmsnorm_any, dim3(T), dim3(256), 0, o, x, gain, D, eps, gate);
 }
 
 // -------------------------------------------------------------- pack to a16

@@ -667,8 +667,7 @@ void HybridModel::forward_f32(const PassArgs& a, const StepArrays& st) {
             Lightning l = lightning(w, (int)run);
             l.q32 = q; l.k32 = b; l.v32 = c; l.out_f32 = d;
             launch_lightning(l, st);
-            launch_rmsnorm_f32(d, d, w.head_norm, vn, T, eps_);
-            launch_sigmoid_gate(d, d, gate, (long)T * vn);
+            launch_rmsnorm_f32(d, d, w.head_norm, vn, T, eps_, gate);
         } else {
             launch_gemm_f32(normed(0).add(w.in32[0], m.channels(), c), PC_GEMM_QKV);
             const KvPages pool = pages(a.mgr, (int)run);

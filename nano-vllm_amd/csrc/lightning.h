@@ -31,7 +31,4 @@ struct Lightning {
 static inline size_t lightning_state_floats(int H, int dim, int vdim) { return (size_t)H * dim * vdim; }   // of one slot
 void launch_lightning(const Lightning& a, const StepArrays& st);
 
-// out = x * sigmoid(g) (fp32 path: the gate on the normed heads)
-void launch_sigmoid_gate(float* out, const float* x, const float* g, long n);
-
 }  // namespace nvllm

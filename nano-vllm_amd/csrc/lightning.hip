@@ -672,15 +672,4 @@ void launch_lightning(const Lightning& a, const StepArrays& st) {
     else NVLLM_LAUNCH((k_lightning_step<false, 1>), grid, dim3(256), lds, a, spans);
 }
 
-// ------------------------------------------------------------------ element-wise steps of the fp32 path
-__global__ __launch_bounds__(256) void k_sigmoid_gate(float* out, const float* x, const float* __restrict__ g, long n) {
-    const long i = (long)blockIdx.x * 256 + threadIdx.x;
-    if (i < n) out[i] = x[i] * sigmoid_f(g[i]);
-}
-void launch_sigmoid_gate(float* out, const float* x, const float* g, long n) {
-    if (n <= 0) return;
-    ProfScope ps(PC_ELEMWISE, (double)n * 12.0, 0);
-    NVLLM_LAUNCH(k_sigmoid_gate, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, out, x, g, n);
-}
-
 }  // namespace nvllm

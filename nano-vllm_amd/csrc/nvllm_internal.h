@@ -401,7 +401,8 @@ void launch_gemm_experts(const B16Weight& w, int experts, const __half* act, con
 
 void launch_pack_a16(__half* a16, const float* in, int T, int K);
 
-void launch_rmsnorm_f32(float* o, const float* x, const float* gain, int D, int T, float eps);
+// gate [T][D]: times its sigmoid (null: no)
+void launch_rmsnorm_f32(float* o, const float* x, const float* gain, int D, int T, float eps, const float* gate = nullptr);
 
 struct KvPoolView {
     void* k;
