@@ -170,7 +170,15 @@ void launch_dense(GemmArgs a) {
 
 // What is launched without its rider has the caller launch that: false.
 template <int EPI, bool GRP>
-bool launch_kind(GemmArgs a, int prof_cls, double bytes, double flops, const MoeRider* moe = nullptr, const GemmArgs* router = nullptr) {
+bool launch_kind(GemmArgs a, int prof_cls, double bytes, double flops, MoeRider* moe = nullptr, const GemmArgs* router = nullptr) {
+    bool rode = false;
+    if (moe && EPI == GemmEpilogue::SWIGLU_A16) a.route = RouteRider{router->W, router->NB, router->e.out, router->e.ldo, moe->plan};
+    if (moe && EPI == GemmEpilogue::F32 && moe->chosen) a.route.plan = moe->plan;
+    auto tiles = [&]() {   // (their own rules are there)
+        const bool taken = launch_gemm_waves_b16(a, &rode) || launch_gemm_wide_b16(a, &rode);
+        if (rode && EPI == GemmEpilogue::SWIGLU_A16) moe->chosen = true;
+        return taken;
+    };
     static const int pf_min_t = getenv("NVLLM_GEMM_PREFILL_T") ? atoi(getenv("NVLLM_GEMM_PREFILL_T")) : 256;
     // few features: the chip fills with token groups of 16 or 32, not with dense tiles
     const bool narrow = !GRP && EPI == GemmEpilogue::F32 && !a.e.amax_out && a.NB <= 8 && a.Tb <= 4 * rt().num_cus;
@@ -178,17 +186,17 @@ bool launch_kind(GemmArgs a, int prof_cls, double bytes, double flops, const Moe
         {
             ProfScope ps(prof_cls, bytes, flops);
             a.e.amax_pairs = nullptr;   // the dense-tile kernel does not emit pairs: the rows are scanned afterwards
-            if (GRP || !(launch_gemm_waves_b16(a) || launch_gemm_wide_b16(a))) launch_dense<EPI, GRP>(a);   // (their own rules are there)
+            if (GRP || !tiles()) launch_dense<EPI, GRP>(a);
         }
         if (EPI == GemmEpilogue::F32 && a.e.amax_out) launch_argmax_ld(a.e.amax_out, a.e.out, a.T, a.N, a.e.ldo, a.e.amax_out_host);
         if (EPI == GemmEpilogue::F32 && a.e.out_host) copy_rows_to_host(a.e.out_host, a.e.out, (size_t)a.T * a.e.ldo);
-        return false;
+        return rode;
     }
     if (!GRP && !narrow && !(EPI == GemmEpilogue::F32 && a.e.amax_out) && gemm_leaves_streaming(a.NB, a.Kb, a.Tb, 1, rt().num_cus)) {
         a.ksplit = 1;
         a.kb_per_split = a.Kb;
         ProfScope ps(prof_cls, bytes, flops);
-        if (launch_gemm_waves_b16(a) || launch_gemm_wide_b16(a)) return false;
+        if (tiles()) return rode;
         ps.drop();
     }
     // a block-diagonal product has a short K and no K split; its plan is that of one group times the groups
@@ -219,7 +227,6 @@ bool launch_kind(GemmArgs a, int prof_cls, double bytes, double flops, const Moe
     const long wgs = (long)pl.tiles_n * pl.ks * pl.tiles_t;
     if (pl.ks > 1) a.slab = (float*)ws_get(WS_SLAB, (size_t)wgs * (pl.nbw / 2) * 2 * pl.TB * 64 * 16);
     a.close_sc1 = pl.ks > 1 && wgs <= rt().num_cus;   // (tiles: riders touch no partials)
-    bool rode = false;
     {
         ProfScope ps(prof_cls, bytes, flops);
         if constexpr (!GRP && (EPI == GemmEpilogue::SWIGLU_A16 || EPI == GemmEpilogue::F32))
@@ -304,7 +311,7 @@ void launch_gemm_experts(const B16Weight& w, int experts, const __half* act, con
     }
 }
 
-bool launch_gemm_b16(const B16Weight& w, const __half* act, int T, const GemmEpilogue& epi, int prof_cls, const LatentKvRider* ride, const MoeRider* moe) {
+bool launch_gemm_b16(const B16Weight& w, const __half* act, int T, const GemmEpilogue& epi, int prof_cls, const LatentKvRider* ride, MoeRider* moe) {
     if (T <= 0) return false;
     ensure_init();
     if (w.K % 32) NVLLM_FATAL("bf16 projection: the input width %d is not padded to 32", w.K);

@@ -2,6 +2,7 @@
 // element-wise pieces of their epilogues (see gemm.hip for what each epilogue does).
 #pragma once
 
+#include "moe.h"
 #include "nvllm_internal.h"
 
 namespace nvllm {
@@ -44,6 +45,15 @@ struct LatentKvRider {
     int raw_ld, rot_at, T, rank, rot, rank_ld, rot_ld;
 };
 
+// The router of a mixture with its choices, or their sorting, beside tiles of hundreds of tokens (moe_ride.h).
+struct RouteRider {
+    const __half* W;   // the router: tiles [NB][Kb]
+    int NB;
+    float* z;       // [T][ldz], whole blocks of a row
+    int ldz;
+    RoutePlan plan;    // T 0: nobody rides
+};
+
 struct GemmArgs {
     const __half* W;
     long nb_stride;   // halves between 16-row blocks
@@ -66,6 +76,7 @@ struct GemmArgs {
                       // (hipMalloc slab; launches of at most one tile per CU, where it was measured: riders are not counted)
     GemmEpilogue e;
     LatentKvRider ride;
+    RouteRider route;
     int ride_from;    // first workgroup (grid x) of the riders
 #ifdef NVLLM_STAMPS
     unsigned long long* stamps;   // diagnostic builds only: [workgroup][8] constant-rate clock readings
@@ -316,7 +327,7 @@ __device__ __forceinline__ void copy_tile_to_lds(const __half* lane_src, unsigne
 void launch_gemm_prefill(GemmArgs a);
 // gemm_wide_f16.hip: the same in tiles of 256 features; false: not for this launch
 bool launch_gemm_wide_f16(const GemmArgs& a);
-bool launch_gemm_wide_b16(const GemmArgs& a);   // gemm_wide_b16.hip: bf16 models
+bool launch_gemm_wide_b16(const GemmArgs& a, bool* rode);   // gemm_wide_b16.hip: bf16 models; rode: with a.route
 bool launch_experts_wide_b16(const GemmArgs& a, int pad);   // ... rows sorted by expert, in groups of expert_rows_wide()
 // gemm_waves_f16.hip, gemm_waves_b16.hip: one round of tiles with K dealt to the waves; false: not for this launch
 bool launch_gemm_waves_f16(const GemmArgs& a);
@@ -331,6 +342,6 @@ inline bool gemm_leaves_streaming(int NB, int Kb, int Tb, int planes, int cus) {
     if (cdiv(NB, 4) * cdiv(Tb, 4) > cus) return true;
     return Tb > 8 && Kb <= 64 && cdiv(NB, 8) * Tb <= cus && (planes == 2 || NB <= 128);
 }
-bool launch_gemm_waves_b16(const GemmArgs& a);
+bool launch_gemm_waves_b16(const GemmArgs& a, bool* rode);
 
 }  // namespace nvllm

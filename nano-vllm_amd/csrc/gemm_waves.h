@@ -16,6 +16,7 @@
 #pragma once
 
 #include "gemm_prefill_tile.h"
+#include "moe_ride.h"
 
 namespace nvllm {
 
@@ -25,6 +26,12 @@ constexpr int WAVES_FB = 8;   // 16-row blocks of W per tile
 // K-steps in flight per wave: what 512 registers hold beside the sums
 constexpr int waves_ring(int planes, int TBN) {
     return planes == 1 ? (TBN <= 3 ? 4 : 3) : (TBN <= 2 ? 4 : TBN <= 5 ? 3 : 2);
+}
+
+// A router beside the gated pairs, its sorting beside plain rows (moe_ride.h).  Not the router beside seven blocks: they fill the
+// registers, and the compiler waits in their loop for loads of the other branch.
+constexpr bool waves_carry_route(int TBN, int EPI, int planes) {
+    return planes == 1 && (EPI == GemmEpilogue::F32 || (EPI == GemmEpilogue::SWIGLU_A16 && TBN <= 6));
 }
 
 template <int TBN, int EPI, typename KVT, typename OP>
@@ -38,6 +45,13 @@ __global__ __launch_bounds__(256, 1) void k_gemm_waves(GemmArgs p, int tiles_n, 
     if constexpr (EPI == GemmEpilogue::LATENT_Q) {
         if ((int)blockIdx.x >= p.ride_from) {
             ride_along(p, 4, wave, lane);
+            return;
+        }
+    }
+    if constexpr (waves_carry_route(TBN, EPI, PL)) {
+        if ((int)blockIdx.x >= p.ride_from) {
+            if constexpr (EPI == GemmEpilogue::SWIGLU_A16) router_ride<4>(p, wave, lane, lds_waves);
+            else route_sort<false, 256>(p.route.plan, nullptr, 0, reinterpret_cast<int*>(lds_waves));
             return;
         }
     }
@@ -149,8 +163,8 @@ __global__ __launch_bounds__(256, 1) void k_gemm_waves(GemmArgs p, int tiles_n, 
 }
 
 template <int TBN, int EPI, typename KVT, typename OP>
-void launch_waves(GemmArgs a, int tiles_n, int tiles_t) {
-    constexpr int LDS = 1024 + 16 * TBN * 1024;
+bool launch_waves(GemmArgs a, int tiles_n, int tiles_t) {   // whether a.route rode
+    constexpr int NEED = 1024 + 16 * TBN * 1024, LDS = EPI == GemmEpilogue::SWIGLU_A16 && waves_carry_route(TBN, EPI, OP::PLANES) ? std::max(NEED, router_ride_lds(4)) : NEED;
     static_assert(LDS <= 160 * 1024, "the waves' sums must fit the CU's LDS");
     static bool enabled = false;
     if (!enabled) {
@@ -158,24 +172,28 @@ void launch_waves(GemmArgs a, int tiles_n, int tiles_t) {
         enabled = true;
     }
     a.ride_from = tiles_n * tiles_t;
-    NVLLM_LAUNCH((k_gemm_waves<TBN, EPI, KVT, OP>), dim3(tiles_n * tiles_t + rider_groups(a, tiles_n * tiles_t, 4)), dim3(256), LDS, a, tiles_n, tiles_t);
+    const int route = waves_carry_route(TBN, EPI, OP::PLANES) ? route_groups(a, a.ride_from) : 0;
+    static_assert((3 * 1024 + 1) * 4 <= LDS);   // (the sorting)
+    NVLLM_LAUNCH((k_gemm_waves<TBN, EPI, KVT, OP>), dim3(a.ride_from + rider_groups(a, a.ride_from, 4) + route), dim3(256), LDS, a, tiles_n, tiles_t);
+    return route > 0;
 }
 
 // Seven blocks of two planes leave registers for two steps in flight, and lose: prompts of TinyLlama-1.1B, 1,547 tokens, w_down in such
 // tiles 7,890 us a pass, in those of gemm_wide.h 7,790 (six blocks at 1,500 tokens 6,710 and 7,100).
 constexpr int waves_tallest(int planes) { return planes == 1 ? 7 : 6; }
 template <int EPI, typename KVT, typename OP>
-void launch_waves_height(const GemmArgs& a, int tbn) {
+bool launch_waves_height(const GemmArgs& a, int tbn) {
     const int tiles_n = cdiv(a.NB, WAVES_FB), tiles_t = cdiv(a.Tb, tbn);
     switch (tbn) {
-        case 1: launch_waves<1, EPI, KVT, OP>(a, tiles_n, tiles_t); break;
-        case 2: launch_waves<2, EPI, KVT, OP>(a, tiles_n, tiles_t); break;
-        case 3: launch_waves<3, EPI, KVT, OP>(a, tiles_n, tiles_t); break;
-        case 4: launch_waves<4, EPI, KVT, OP>(a, tiles_n, tiles_t); break;
-        case 5: launch_waves<5, EPI, KVT, OP>(a, tiles_n, tiles_t); break;
-        case 6: launch_waves<6, EPI, KVT, OP>(a, tiles_n, tiles_t); break;
+        case 1: return launch_waves<1, EPI, KVT, OP>(a, tiles_n, tiles_t);
+        case 2: return launch_waves<2, EPI, KVT, OP>(a, tiles_n, tiles_t);
+        case 3: return launch_waves<3, EPI, KVT, OP>(a, tiles_n, tiles_t);
+        case 4: return launch_waves<4, EPI, KVT, OP>(a, tiles_n, tiles_t);
+        case 5: return launch_waves<5, EPI, KVT, OP>(a, tiles_n, tiles_t);
+        case 6: return launch_waves<6, EPI, KVT, OP>(a, tiles_n, tiles_t);
         default:
-            if constexpr (waves_tallest(OP::PLANES) == 7) launch_waves<7, EPI, KVT, OP>(a, tiles_n, tiles_t);
+            if constexpr (waves_tallest(OP::PLANES) == 7) return launch_waves<7, EPI, KVT, OP>(a, tiles_n, tiles_t);
+            return false;
     }
 }
 

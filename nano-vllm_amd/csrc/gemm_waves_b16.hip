@@ -8,12 +8,12 @@ namespace nvllm {
 // 16.6 -> 10.6, 17.4 -> 11.9, 19.3 -> 16.8, 22.2 -> 18.9, 23.8 -> 21.9, 25.0 -> 23.9; 1,024 features x 1,024 k at 512 and 2,000
 // tokens (1 and 4) 11.1 -> 7.9, 13.7 -> 13.5; 5,632 x 2,048 at 400 (5) 27.8 -> 20.1; few tiles of a long K too: 256 and 512 features x 8,192 k at
 // 256 tokens (32 and 64 tiles) 54.3 -> 25.8, 52.7 -> 24.9, 512 x 4,096 31.3 -> 14.5.
-bool launch_gemm_waves_b16(const GemmArgs& a) {
+bool launch_gemm_waves_b16(const GemmArgs& a, bool* rode) {
     const int tbn = waves_height(a, waves_tallest(1));
     if (!tbn) return false;
     switch (a.e.kind) {
-        case GemmEpilogue::F32: launch_waves_height<GemmEpilogue::F32, float, OpBf16>(a, tbn); break;
-        case GemmEpilogue::SWIGLU_A16: launch_waves_height<GemmEpilogue::SWIGLU_A16, float, OpBf16>(a, tbn); break;
+        case GemmEpilogue::F32: *rode = launch_waves_height<GemmEpilogue::F32, float, OpBf16>(a, tbn); break;
+        case GemmEpilogue::SWIGLU_A16: *rode = launch_waves_height<GemmEpilogue::SWIGLU_A16, float, OpBf16>(a, tbn); break;
         case GemmEpilogue::TILE_B16: launch_waves_height<GemmEpilogue::TILE_B16, float, OpBf16>(a, tbn); break;
         case GemmEpilogue::ROWS_B16: launch_waves_height<GemmEpilogue::ROWS_B16, float, OpBf16>(a, tbn); break;
         case GemmEpilogue::LATENT_IN: launch_waves_height<GemmEpilogue::LATENT_IN, float, OpBf16>(a, tbn); break;

@@ -20,6 +20,7 @@
 #include <climits>
 
 #include "gemm_prefill_tile.h"
+#include "moe_ride.h"
 
 namespace nvllm {
 
@@ -64,6 +65,12 @@ __global__ __launch_bounds__(256 * WT, 1) void k_gemm_wide(GemmArgs p, int tiles
     if constexpr (EPI == GemmEpilogue::LATENT_Q) {
         if ((int)blockIdx.x >= p.ride_from) {
             ride_along(p, WAVES, wave, lane);
+            return;
+        }
+    }
+    if constexpr (EPI == GemmEpilogue::SWIGLU_A16 && PL == 1 && !EXP) {
+        if ((int)blockIdx.x >= p.ride_from) {
+            router_ride<WAVES>(p, wave, lane, lds_wide);
             return;
         }
     }
@@ -212,16 +219,20 @@ inline int wide_panel(int tiles_n, int tiles_t, int w, int a) {
 }
 
 template <int TBN, int EPI, typename KVT, typename OP, int WT = 1, bool EXP = false>
-void launch_wide(GemmArgs a, int tiles_n, int tiles_t) {
+bool launch_wide(GemmArgs a, int tiles_n, int tiles_t) {   // whether a.route rode
     using G = WideGeom<TBN, OP::PLANES, WT>;
+    constexpr bool CARRIES = EPI == GemmEpilogue::SWIGLU_A16 && OP::PLANES == 1 && !EXP;   // a router (moe_ride.h)
     static bool enabled = false;
     if (!enabled) {
         HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_gemm_wide<TBN, WT, EPI, KVT, OP, EXP>), hipFuncAttributeMaxDynamicSharedMemorySize, G::LDS));
         enabled = true;
     }
     a.ride_from = tiles_n * tiles_t;
-    NVLLM_LAUNCH((k_gemm_wide<TBN, WT, EPI, KVT, OP, EXP>), dim3(tiles_n * tiles_t + rider_groups(a, tiles_n * tiles_t, G::WAVES)), dim3(64 * G::WAVES), G::LDS, a, tiles_n, tiles_t,
+    const int route = CARRIES ? route_groups(a, a.ride_from) : 0;
+    static_assert(!CARRIES || router_ride_lds(G::WAVES) <= G::LDS);
+    NVLLM_LAUNCH((k_gemm_wide<TBN, WT, EPI, KVT, OP, EXP>), dim3(a.ride_from + rider_groups(a, a.ride_from, G::WAVES) + route), dim3(64 * G::WAVES), G::LDS, a, tiles_n, tiles_t,
                  OP::PLANES == 1 ? 1 : wide_panel(tiles_n, tiles_t, G::FB, OP::PLANES * TBN));
+    return route > 0;
 }
 
 // Microseconds a launch takes in tiles of TBN token blocks: rounds of one workgroup per CU, each a start and an end beside its

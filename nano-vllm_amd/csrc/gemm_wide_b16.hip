@@ -11,18 +11,20 @@ namespace nvllm {
 namespace {
 
 template <int EPI, bool EXP>
-bool launch_wide_height(const GemmArgs& a, int tbn, int tiles_n, int tiles_t) {
+bool launch_wide_height(const GemmArgs& a, int tbn, int tiles_n, int tiles_t, bool* rode = nullptr) {
+    bool ride;
     switch (tbn) {
-        case 4: launch_wide<4, EPI, float, OpBf16, 1, EXP>(a, tiles_n, tiles_t); break;
-        case 5: launch_wide<5, EPI, float, OpBf16, 1, EXP>(a, tiles_n, tiles_t); break;
-        case 6: launch_wide<6, EPI, float, OpBf16, 1, EXP>(a, tiles_n, tiles_t); break;
-        case 8: launch_wide<8, EPI, float, OpBf16, 2, EXP>(a, tiles_n, tiles_t); break;
-        case 10: launch_wide<10, EPI, float, OpBf16, 2, EXP>(a, tiles_n, tiles_t); break;
-        case 12: launch_wide<12, EPI, float, OpBf16, 2, EXP>(a, tiles_n, tiles_t); break;
-        case 14: launch_wide<14, EPI, float, OpBf16, 2, EXP>(a, tiles_n, tiles_t); break;
-        case 16: launch_wide<16, EPI, float, OpBf16, 2, EXP>(a, tiles_n, tiles_t); break;
+        case 4: ride = launch_wide<4, EPI, float, OpBf16, 1, EXP>(a, tiles_n, tiles_t); break;
+        case 5: ride = launch_wide<5, EPI, float, OpBf16, 1, EXP>(a, tiles_n, tiles_t); break;
+        case 6: ride = launch_wide<6, EPI, float, OpBf16, 1, EXP>(a, tiles_n, tiles_t); break;
+        case 8: ride = launch_wide<8, EPI, float, OpBf16, 2, EXP>(a, tiles_n, tiles_t); break;
+        case 10: ride = launch_wide<10, EPI, float, OpBf16, 2, EXP>(a, tiles_n, tiles_t); break;
+        case 12: ride = launch_wide<12, EPI, float, OpBf16, 2, EXP>(a, tiles_n, tiles_t); break;
+        case 14: ride = launch_wide<14, EPI, float, OpBf16, 2, EXP>(a, tiles_n, tiles_t); break;
+        case 16: ride = launch_wide<16, EPI, float, OpBf16, 2, EXP>(a, tiles_n, tiles_t); break;
         default: return false;
     }
+    if (rode) *rode = ride;
     return true;
 }
 constexpr int WIDE_HEIGHTS[] = {4, 5, 6, 8, 10, 12, 14, 16};   // token blocks
@@ -47,16 +49,16 @@ int wide_height(int NB, int Kb, int Tb) {
     return 0;
 }
 template <int EPI>
-bool launch_wide_b16(const GemmArgs& a) {
+bool launch_wide_b16(const GemmArgs& a, bool* rode = nullptr) {
     const int tbn = wide_height(a.NB, a.Kb, a.Tb);
-    return tbn && launch_wide_height<EPI, false>(a, tbn, cdiv(a.NB, 16), cdiv(a.Tb, tbn));
+    return tbn && launch_wide_height<EPI, false>(a, tbn, cdiv(a.NB, 16), cdiv(a.Tb, tbn), rode);
 }
 
 }  // namespace
 
-bool launch_gemm_wide_b16(const GemmArgs& a) {
+bool launch_gemm_wide_b16(const GemmArgs& a, bool* rode) {
     switch (a.e.kind) {
-        case GemmEpilogue::SWIGLU_A16: return launch_wide_b16<GemmEpilogue::SWIGLU_A16>(a);
+        case GemmEpilogue::SWIGLU_A16: return launch_wide_b16<GemmEpilogue::SWIGLU_A16>(a, rode);
         case GemmEpilogue::TILE_B16: return launch_wide_b16<GemmEpilogue::TILE_B16>(a);
         case GemmEpilogue::ROWS_B16: return launch_wide_b16<GemmEpilogue::ROWS_B16>(a);
         case GemmEpilogue::LATENT_Q: return launch_wide_b16<GemmEpilogue::LATENT_Q>(a);

@@ -589,7 +589,7 @@ void HybridModel::forward_b16(const PassArgs& a, const StepArrays& st) {
             sd.kind = GemmEpilogue::F32;
             sd.out = y_shared; sd.ldo = Dp_;
             if (!f.shared_ff || !launch_gemm_b16(w.shared_up, act, T, su, PC_GEMM_SHARED_UP, nullptr, &rider)) launch_gemm_b16(w.router, act, T, ez, PC_GEMM_ROUTER);
-            if (!f.shared_ff || !launch_gemm_b16(w.shared_down, hid_shared, T, sd, PC_GEMM_SHARED_DOWN, nullptr, &rider)) launch_route(plan, z, ldz);
+            if (!f.shared_ff || !launch_gemm_b16(w.shared_down, hid_shared, T, sd, PC_GEMM_SHARED_DOWN, nullptr, &rider)) launch_route(plan, z, ldz, rider.chosen);
             ExpertRows er{plan.block_expert, plan.source, plan.capacity, plan.pad, T * f.top, groups.wide};
             GemmEpilogue eu = normed(GemmEpilogue::SWIGLU_A16);
             eu.ss_gather = plan.source; eu.row_weight = plan.weight; eu.a16_out = wide;

@@ -27,16 +27,17 @@ ExpertGroups expert_groups(int T, int E, int top, const B16Weight& up, const B16
 size_t route_ints(int T, int E, int top, int pad);  // 4-byte words route_plan() lays out
 RoutePlan route_plan(int* mem, int T, int E, int top, int pad);
 // z: [T][ldz] router logits in columns 0 .. E-1; the `top` largest (the first of equals) are chosen
-void launch_route(const RoutePlan& r, const float* z, int ldz);
+void launch_route(const RoutePlan& r, const float* z, int ldz, bool chosen = false);   // chosen: sorting is left
 
 // Work that needs a fraction of the chip, beside the shared expert's products on the CUs those leave idle: the router beside the first,
-// the choice beside the second (launch_gemm_b16).
+// the choice beside the second (launch_gemm_b16); with hundreds of tokens the choice with the router, the sorting alone beside the second.
 struct MoeRider {
     const B16Weight* router = nullptr;   // SWIGLU_A16 launches: its activations are the launch's
     GemmEpilogue router_epi;             // F32
     RoutePlan plan{};                    // F32 launches
     const float* z = nullptr;
     int ldz = 0;
+    bool chosen = false;                 // (set by the SWIGLU_A16 launch)
 };
 
 // the rows x * gain of a batch in the plan's order, as activation tiles (x [T][ld])

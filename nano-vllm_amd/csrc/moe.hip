@@ -55,18 +55,18 @@ __global__ __launch_bounds__(1024) void k_route_sort(RoutePlan r, const float* _
     route_sort<CHOOSE, 1024>(r, z, ldz, lds_r);
 }
 
-void launch_route(const RoutePlan& r, const float* z, int ldz) {
+void launch_route(const RoutePlan& r, const float* z, int ldz, bool chosen) {
     if (r.T <= 0) return;
     if (r.E < 1 || r.E > MAX_EXPERTS || r.top < 1 || r.top > r.E) NVLLM_FATAL("routing: %d of %d experts per token", r.top, r.E);
     const size_t lds = ((size_t)3 * r.E + 1) * sizeof(int);
     const double bytes = (double)r.T * (r.E * 4.0 + r.top * 20.0);
     const size_t lds_one = route_sort_lds(r.T, r.E, r.top);
-    if (r.T <= ROUTE_ONE && lds_one <= 64 * 1024) {
+    if (!chosen && r.T <= ROUTE_ONE && lds_one <= 64 * 1024) {
         ProfScope ps(PC_ROUTE, bytes, 0);
         NVLLM_LAUNCH((k_route_sort<true>), dim3(1), dim3(1024), lds_one, r, z, ldz);
         return;
     }
-    {
+    if (!chosen) {
         ProfScope ps(PC_ROUTE, bytes, 0);
         NVLLM_LAUNCH(k_route, dim3(cdiv(r.T, 4)), dim3(256), 0, r, z, ldz);
     }

@@ -53,6 +53,22 @@ __device__ __forceinline__ void route_token(const RoutePlan& r, const float* __r
         }
     }
 }
+// The same for four tokens of up to 64 experts, a logit per lane (lanes past the last expert: -INFINITY).  put(token, place, expert, score) in lane 0.
+template <class Put>
+__device__ __forceinline__ void choose_four(float (&v)[4], int E, int top, int lane, Put&& put) {
+    for (int j = 0; j < top; j++) {
+        float best[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) best[u] = wave_max(v[u]);
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const unsigned long long at = __ballot(v[u] == best[u] && lane < E);
+            const int e = at ? __ffsll(at) - 1 : 0;   // (no number compares: NaN logits)
+            if (lane == e) v[u] = -INFINITY;
+            if (lane == 0) put(u, j, e, 1.f / (1.f + expf(-best[u])));
+        }
+    }
+}
 // One workgroup: counts, segment starts, then every choice takes a row of its expert's segment (in any order: a row's
 // result does not depend on its place).
 // lds_r: counts [E], next free row [E], segment start [E + 1], CHOOSE: choices and scores [T * top].
@@ -75,22 +91,13 @@ __device__ __forceinline__ void route_sort(RoutePlan r, const float* __restrict_
                 float v[4];
 #pragma unroll
                 for (int u = 0; u < 4; u++) v[u] = lane < r.E ? z[(size_t)min(t0 + WAVES * u, r.T - 1) * ldz + lane] : -INFINITY;
-                for (int j = 0; j < r.top; j++) {
-                    float best[4];
-#pragma unroll
-                    for (int u = 0; u < 4; u++) best[u] = wave_max(v[u]);
-#pragma unroll
-                    for (int u = 0; u < 4; u++) {
-                        const int t = t0 + WAVES * u;
-                        const unsigned long long at = __ballot(v[u] == best[u] && lane < r.E);
-                        const int e = at ? __ffsll(at) - 1 : 0;   // (no number compares: NaN logits)
-                        if (lane == e) v[u] = -INFINITY;
-                        if (lane == 0 && t < r.T) {
-                            choice[t * r.top + j] = e;
-                            score[t * r.top + j] = 1.f / (1.f + expf(-best[u]));
-                        }
+                choose_four(v, r.E, r.top, lane, [&](int u, int j, int e, float sc) {
+                    const int t = t0 + WAVES * u;
+                    if (t < r.T) {
+                        choice[t * r.top + j] = e;
+                        score[t * r.top + j] = sc;
                     }
-                }
+                });
             }
         } else {
             for (int t = tid >> 6; t < r.T; t += WAVES) route_token(r, z + (size_t)t * ldz, t, lane);

@@ -384,7 +384,7 @@ struct LatentKvRider;   // gemm_common.h: cache rows written by extra workgroups
 struct MoeRider;        // moe.h: a router beside a SWIGLU_A16 launch, or its choices and their sorting beside an F32 one
 // `moe`: true is returned if it rode along (few tokens), false if the caller has to launch it
 bool launch_gemm_b16(const B16Weight& w, const __half* act, int T, const GemmEpilogue& epi, int prof_cls, const LatentKvRider* ride = nullptr,
-                     const MoeRider* moe = nullptr);
+                     MoeRider* moe = nullptr);
 // Rows sorted by expert (moe.h): every group of `pad` rows meets the matrix of ONE expert.
 struct ExpertRows {
     const int* block_expert;   // [capacity / 16] expert of each 16-row block, -1: no rows (the same within a group)

@@ -23,6 +23,21 @@ def test_passes_of_few_tokens(hip, tmp_path, experts, shared):
     eng.close()
 
 
+# routers of one row block, of two and of four, and one wider than rides; 256 tokens and more take tiles whose idle CUs carry them
+@pytest.mark.parametrize("experts,top", [(5, 2), (31, 3), (63, 4), (64, 2)])
+def test_prompts(hip, tmp_path, experts, top):
+    window = synth.window_mixer(4, 2, 16, 16, size=48, keep_first=4)
+    cfg = synth.hybrid_config(288, 211, [(window, synth.expert_mlp(48, experts, top, 96))] * 2)
+    path, cfg, weights = U.model(tmp_path, "prompts", seed=experts, cfg=cfg)
+    eng = U.engine(hip, path, False, slots=1)
+    for n in (256, 257, 511, 1100):
+        seq = U.tokens(n, 211, n)
+        got = U.feed_all(eng, [[(0, n)]], {0: seq})[0]
+        np.testing.assert_array_equal(U.feed_all(eng, [[(0, n)]], {0: seq})[0], got)
+        assert U.error(got, O.forward(cfg, weights, seq)) < U.limit(False), n
+    eng.close()
+
+
 # K splits of both products; of the second, with 96-feature tiles of the first from 33 tokens on
 @pytest.mark.parametrize("width,experts,shared", [(1024, 20, 96), (512, 70, 2816), (256, 30, 2816)])
 def test_riders_beside_k_splits(hip, tmp_path, width, experts, shared):
