@@ -21,7 +21,7 @@ namespace nvllm {
 
 constexpr int F32_STEP = 32;   // k per step: 128 bytes, a cache line, of every row
 // waves per SIMD the registers are dealt for: two workgroups of eight waves share a CU where the tiles allow it
-constexpr int f32_occupancy(int tiles, bool norm) { return tiles == 8 ? 2 : tiles == 4 && norm ? 3 : 4; }
+constexpr int f32_occupancy(int tiles, bool norm) { return tiles >= 6 ? 2 : tiles == 4 && norm ? 3 : 4; }
 
 template <int NB, int TB, int KS, bool PAIR, bool NORM>
 __global__ __launch_bounds__(KS * 64, f32_occupancy((PAIR ? 2 : 1) * NB * TB, NORM)) void k_gemm_f32(F32Gemm p) {
@@ -29,8 +29,9 @@ __global__ __launch_bounds__(KS * 64, f32_occupancy((PAIR ? 2 : 1) * NB * TB, NO
     constexpr int RING = NT * TB == 1 ? (NORM ? 3 : 4) : 2;
     constexpr int ITEMS = NB * TB * 64;   // results, four features of a token each
     constexpr int FPT = (ITEMS + KS * 64 - 1) / (KS * 64);
-    __shared__ f4_t s_red[KS][NT * TB][64];
-    __shared__ float s_ss[NORM ? KS : 1][TB * 16];
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds_f32[];
+    f4_t(*s_red)[NT * TB][64] = reinterpret_cast<f4_t(*)[NT * TB][64]>(lds_f32);                     // [wave]
+    float(*s_ss)[TB * 16] = reinterpret_cast<float(*)[TB * 16]>(lds_f32 + KS * NT * TB * 1024);   // NORM: [wave]
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int x = lane & 15, g = lane >> 4;
@@ -84,6 +85,7 @@ __global__ __launch_bounds__(KS * 64, f32_occupancy((PAIR ? 2 : 1) * NB * TB, NO
     // of eight 8.2 / 8.7 / 9.5, of 16 9.9 / 10 / 10.5; chains of four 7.9 / 8.4 / 9.2, but a pass of 301 tokens takes 7 % longer.
     constexpr int TILES = NT * TB;
     constexpr bool APART = TILES == 1 && KS == 8;
+    static_assert(TILES == 1 || TILES % 2 == 0, "two sets of chains in turn, from one step's last tile to the next one's first");
     f4_t acc[NT][TB], chain[APART ? 1 : 2][APART ? 8 : 4];
 #pragma unroll
     for (int n = 0; n < NT; n++)
@@ -252,6 +254,17 @@ __global__ __launch_bounds__(KS * 64, f32_occupancy((PAIR ? 2 : 1) * NB * TB, NO
     }
 }
 
+template <int NB, int TB, int KS, bool PAIR, bool NORM>
+void launch_f32(const F32Gemm& a, dim3 grid) {
+    constexpr int LDS = KS * ((PAIR ? 2 : 1) * NB * TB * 1024 + (NORM ? TB * 64 : 0));
+    static bool enabled = false;
+    if (LDS > 64 * 1024 && !enabled) {
+        HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_gemm_f32<NB, TB, KS, PAIR, NORM>), hipFuncAttributeMaxDynamicSharedMemorySize, LDS));
+        enabled = true;
+    }
+    NVLLM_LAUNCH((k_gemm_f32<NB, TB, KS, PAIR, NORM>), grid, dim3(KS * 64), LDS, a);
+}
+
 // Rows that are no multiples of 16 bytes (K % 4 != 0, or a caller's odd pointer): a wave sums four features of four tokens,
 // its lanes striding over k.
 template <bool PAIR>
@@ -343,27 +356,33 @@ void launch_gemm_f32(const F32Gemm& g, int prof_cls) {
     // Blocks per wave.  A launch takes about what its busiest CU has to fetch (64 bytes per block and k, at about 20 bytes
     // per cycle of the mix of weights and activations) and to multiply (8 cycles per product and quad of k on four SIMDs):
     // larger tiles fetch less per product, smaller ones reach more CUs.  K = 512 at 301 tokens: 2 x 2 blocks of a 512-wide
-    // output 8 us, 1 x 1 10 us; 2 x 4 of a 1,536-wide one 13.6 us against 17.0 in 2 x 2.
+    // output 8 us, 1 x 1 10 us; 2 x 4 of a 1,536-wide one 13.6 us against 17.0 in 2 x 2.  Three token blocks where two and four fill
+    // their last round worse: 2,816 features x 1,024 k at 80 tokens (176 tiles of 2 x 3; 440 of 1 x 2) 19.9 -> 15.5, 1,024 x 1,024 at
+    // 300 15.9 -> 14.4, 864 x 288 at 301 11.6 -> 7.9; pairs 2 x 768 x 288 at 200 10.9 -> 7.9, 2 x 2,816 x 1,024 at 170 38.0 -> 32.3.  (1 x 3 of a
+    // plain one fetches as much per CU as 2 x 2: 13.6 -> 13.1 at best.)  With a short K in one round only: a second one has too few steps to hide its
+    // start (K = 288, pairs of 768 at 690 tokens 18.1 -> 20.3, 864 features at 600 11.0 -> 12.7).
     const int Tb = cdiv(a.T, 16), cus = rt().num_cus;
-    static const int shapes[][2] = {{1, 1}, {1, 2}, {2, 2}, {2, 4}}, pair_shapes[][2] = {{1, 1}, {1, 2}, {1, 4}};
+    static const int shapes[][2] = {{1, 1}, {1, 2}, {2, 2}, {2, 3}, {2, 4}}, pair_shapes[][2] = {{1, 1}, {1, 2}, {1, 3}, {1, 4}};
     int NB = 1, TB = 1;
     long tiles_all = (long)blocks * Tb;
     if (!a.block_expert && rows16) {
         double best = 0;
-        for (int i = 0; i < (pair ? 3 : 4); i++) {
+        for (int i = 0; i < (pair ? 4 : 5); i++) {
             const int nb = pair ? pair_shapes[i][0] : shapes[i][0], tb = pair ? pair_shapes[i][1] : shapes[i][1], nt = pair ? 2 * nb : nb;
             const long tiles = (long)cdiv(blocks, nb) * cdiv(Tb, tb);
+            if (tb == 3 && tiles > cus && a.K < 512) continue;
             const double cost = (double)cdiv((int)std::min(tiles, 1L << 30), cus) * ((nt + tb) * 64.0 / 20.0 + nt * tb * 2.0);
             if (i == 0 || cost < best) best = cost, NB = nb, TB = tb, tiles_all = tiles;
         }
     }
     // Thousands of tiles (a classifier): two row blocks share a workgroup's start and its activations, 32,000 x 1,024 for one
-    // token 31.4 -> 28.1 us.  Slices of K: eight until every SIMD has two waves.
+    // token 31.4 -> 28.1 us.  Slices of K: eight until every SIMD has two waves; of the large tiles in one round only, and of 2 x 4 blocks
+    // where eight waves request all of K at once (1,536 features x 512 at 301 tokens 12.3 -> 11.7; 1,024 x 2,816 at 400 34.0 -> 36.0).
     if (!pair && NB == 1 && TB == 1 && !a.block_expert && tiles_all >= 4L * cus) {
         NB = 2;
         tiles_all = (long)cdiv(blocks, 2) * Tb;
     }
-    const int KS = TB < 4 && tiles_all * 4 < (a.block_expert ? 16L : 8L) * cus ? 8 : 4;   // (a grid of experts is an upper bound)
+    const int KS = TB > 2 ? (tiles_all <= cus && (TB == 3 || a.K <= 512) ? 8 : 4) : tiles_all * 4 < (a.block_expert ? 16L : 8L) * cus ? 8 : 4;   // (a grid of experts is an upper bound)
     int tiles = 0;
     for (int s = 0; s < a.n_segs; s++) {
         a.seg[s].first = tiles;
@@ -379,8 +398,8 @@ void launch_gemm_f32(const F32Gemm& g, int prof_cls) {
     const dim3 grid(tiles, cdiv(Tb, TB));
 #define NVLLM_GEMM_F32(nb, tb, ks, pr)                                                                    \
     do {                                                                                                  \
-        if (a.gain) NVLLM_LAUNCH((k_gemm_f32<nb, tb, ks, pr, true>), grid, dim3((ks) * 64), 0, a);        \
-        else NVLLM_LAUNCH((k_gemm_f32<nb, tb, ks, pr, false>), grid, dim3((ks) * 64), 0, a);              \
+        if (a.gain) launch_f32<nb, tb, ks, pr, true>(a, grid);                                            \
+        else launch_f32<nb, tb, ks, pr, false>(a, grid);                                                  \
     } while (0)
 #define NVLLM_GEMM_F32_4_8(nb, tb, pr)                                                                    \
     do {                                                                                                  \
@@ -390,15 +409,18 @@ void launch_gemm_f32(const F32Gemm& g, int prof_cls) {
     if (pair) {
         if (TB == 1) NVLLM_GEMM_F32_4_8(1, 1, true);
         else if (TB == 2) NVLLM_GEMM_F32_4_8(1, 2, true);
-        else NVLLM_GEMM_F32(1, 4, 4, true);
+        else if (TB == 3) NVLLM_GEMM_F32_4_8(1, 3, true);
+        else NVLLM_GEMM_F32_4_8(1, 4, true);
     } else if (TB == 1) {
         if (NB == 1) NVLLM_GEMM_F32_4_8(1, 1, false);
         else NVLLM_GEMM_F32_4_8(2, 1, false);
     } else if (TB == 2) {
         if (NB == 1) NVLLM_GEMM_F32_4_8(1, 2, false);
         else NVLLM_GEMM_F32_4_8(2, 2, false);
+    } else if (TB == 3) {
+        NVLLM_GEMM_F32_4_8(2, 3, false);
     } else {
-        NVLLM_GEMM_F32(2, 4, 4, false);
+        NVLLM_GEMM_F32_4_8(2, 4, false);
     }
 #undef NVLLM_GEMM_F32_4_8
 #undef NVLLM_GEMM_F32

@@ -2,6 +2,9 @@
 import numpy as np
 import pytest
 
+from nvllm_amd import synth
+from tests import hybrid_oracle as O
+from tests import hybrid_util as U
 from tests import util
 
 pytestmark = pytest.mark.gpu
@@ -55,3 +58,22 @@ def test_no_further_from_64_bits_than_64_chains(hip, T, K, N):
         chains = chains[:, :half] + chains[:, half:]
     # roundings counted: chains of eight with sums over each step come to 1.06 of it at K = 288, less above; chains of 16 to 1.17 at 512
     assert np.linalg.norm(got[at] - want) < 1.1 * np.linalg.norm(chains[:, 0] - want)
+
+
+# three token blocks by two row blocks, in one round by eight waves and in several by four, and four token blocks by eight waves; ends of tiles
+# and a K that is no multiple of a step or of the waves' share
+@pytest.mark.parametrize("T,K,N", [(80, 1024, 2816), (289, 516, 500), (170, 1028, 2816), (200, 512, 1536), (193, 260, 1530), (230, 1024, 5632), (301, 512, 1536)])
+def test_three_and_four_token_blocks(hip, T, K, N):
+    test_matmul_on_fp32_weights(hip, T, K, N)
+    test_no_further_from_64_bits_than_64_chains(hip, T, K, N)
+
+
+@pytest.mark.parametrize("width,hidden,n", [(288, 768, 200), (512, 1376, 161)])
+def test_pairs_of_three_token_blocks(hip, tmp_path, width, hidden, n):
+    window = synth.window_mixer(4, 2, 16, 16, size=48, keep_first=4)
+    cfg = synth.hybrid_config(width, 211, [(window, synth.expert_mlp(48, 4, 2, hidden))])
+    path, cfg, weights = U.model(tmp_path, "pairs", seed=n, cfg=cfg)
+    eng = U.engine(hip, path, True, slots=1)
+    seq = U.tokens(n, 211, n)
+    assert U.error(U.feed_all(eng, [[(0, n)]], {0: seq})[0], O.forward(cfg, weights, seq)) < U.limit(True)
+    eng.close()
