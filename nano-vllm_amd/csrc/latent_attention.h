@@ -37,6 +37,7 @@ struct LatentKvRider;
 LatentKvRider latent_kv_rider(const LatentPool& pool, const float* raw, int raw_ld, int rot_at, const float* gain, float eps, const float2* rope,
                               const StepArrays& st);
 
+struct LatentExpandRider;   // latent_prompt.h
 struct LatentAttn {
     LatentPool pool;
     const void* q;         // [T][H][pool.row()], element type as the pool's
@@ -47,6 +48,7 @@ struct LatentAttn {
     __half* out_b16;       // bf16 pool: activation tiles of [T, H * rank_ld]
     const B16Weight* uv = nullptr;   // optional, bf16 pool: W_uv, a group of vdim_ld rows per head, and ...
     __half* values = nullptr;        // ... activation tiles of [T, H * vdim_ld] for its products
+    LatentExpandRider* expand = nullptr;   // optional, with only_alone
 };
 constexpr int LATENT_RUN = 32;   // stage_step(attn_ct, multi_first): tokens per run at most
 // only_alone: nothing but the tokens that are their sequence's only one.  True: the results went through W_uv into `values` (out_b16 is

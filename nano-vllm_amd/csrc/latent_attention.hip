@@ -18,6 +18,7 @@
 // k_latent_attn_any (fp32 rows, and bf16 rows wider than the kernel above has registers for): one workgroup per
 // (token, head), fp32 arithmetic on the vector units.
 #include "latent_attention.h"
+#include "latent_expand.h"
 
 #include "attn_tile.h"
 #include "gemm_common.h"
@@ -257,9 +258,17 @@ typedef const __attribute__((address_space(4))) int* const_int_p;   // read-only
 // RC: row chunks of 32 held as query fragments; NT: 16-dim value tiles per wave; C: column groups of 16 per wave; WC: waves
 // side by side over the columns (4 * WC waves: wave = page of the block + 4 * column part).
 // EXACT: the row has exactly RC chunks and 4 * NT value tiles.
-template <int RC, int NT, int C, int WC, bool EXACT>
-__global__ __launch_bounds__(256 * WC, WC) void k_latent_attn(LatentKArgs a) {
+// KC: beside the forming of a prompt's keys and values (latent_expand.h), in the workgroups from e_from on; 0: alone.  Neither wants what
+// the other writes, and the tokens that come alone beside a prompt keep few CUs busy.
+template <int RC, int NT, int C, int WC, bool EXACT, int KC = 0>
+__global__ __launch_bounds__(256 * WC, WC) void k_latent_attn(LatentKArgs a, ExpandArgs e, int e_from, int e_cols) {
     extern __shared__ __attribute__((aligned(16))) unsigned char lds_latent[];
+    if constexpr (KC > 0) {
+        if ((int)blockIdx.x >= e_from) {
+            latent_expand<KC>(e, ((int)blockIdx.x - e_from) % e_cols, ((int)blockIdx.x - e_from) / e_cols, lds_latent);
+            return;
+        }
+    }
     const int nc = EXACT ? RC : a.chunks;
     const int n_tiles = EXACT ? 4 * NT : a.n_tiles;
     __half* pages = reinterpret_cast<__half*>(lds_latent);                          // [2][4][nc][512]
@@ -663,14 +672,37 @@ static void launch_latent_c(const LatentKArgs& k, long units) {
         }
         ready = true;
     }
-    if (exact) NVLLM_LAUNCH((k_latent_attn<RC, NT, C, WC, true>), dim3((unsigned)units), dim3(256 * WC), lds, k);
-    else if constexpr (!EXACT_ONLY) NVLLM_LAUNCH((k_latent_attn<RC, NT, C, WC, false>), dim3((unsigned)units), dim3(256 * WC), lds, k);
+    if (exact) NVLLM_LAUNCH((k_latent_attn<RC, NT, C, WC, true>), dim3((unsigned)units), dim3(256 * WC), lds, k, ExpandArgs{}, 0, 1);
+    else if constexpr (!EXACT_ONLY) NVLLM_LAUNCH((k_latent_attn<RC, NT, C, WC, false>), dim3((unsigned)units), dim3(256 * WC), lds, k, ExpandArgs{}, 0, 1);
 }
 template <int RC, int NT>
 static void launch_latent_rc(const LatentKArgs& k, long units, int columns) {
     if (columns == 16) launch_latent_c<RC, NT, 1, 1>(k, units);
     else if (columns == 32) launch_latent_c<RC, NT, 1, 2>(k, units);
     else launch_latent_c<RC, NT, 2, 2, (RC > 10)>(k, units);
+}
+
+template <int RC, int NT, bool EXACT, int KC>
+static void launch_attn_expand(const LatentKArgs& k, const ExpandArgs& e, int units) {
+    static bool ready = false;
+    if (!ready) {
+        const size_t most = std::max(latent_attn_lds(RC, 2), (size_t)4 * KC * 1024);
+        HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_latent_attn<RC, NT, 1, 2, EXACT, KC>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)most));
+        ready = true;
+    }
+    const int cols = expand_cols(e);
+    const dim3 grid(units + cols * cdiv(e.n_pairs, e.per));
+    NVLLM_LAUNCH((k_latent_attn<RC, NT, 1, 2, EXACT, KC>), grid, dim3(512), std::max(latent_attn_lds(k.chunks, 2), expand_lds(e)), k, e, units, cols);
+}
+// Items of 32 columns (eight waves, as the forming has) on a quarter of the CUs at most, the forming on the others: five tokens at 1,050
+// beside 1,024 behind 1,024 positions, 32 heads of 512: 45 workgroups of 10.8 us and 256 of 14.4 one after the other, together 16.8 (253).
+static bool attn_with_expand(const LatentKArgs& k, const LatentAttn& a, long units, int columns) {
+    if (!a.expand || columns != 32 || units * 4 > rt().num_cus) return false;
+    const ExpandArgs e = latent_expand_args(*a.expand->prompt, *a.expand->plan, rt().num_cus - (int)units);
+    if (k.chunks == 18 && k.n_tiles == 32) launch_attn_expand<18, 8, true, 16>(k, e, (int)units);
+    else if (k.chunks <= 10 && k.n_tiles <= 16 && e.chunks <= 8) launch_attn_expand<10, 4, false, 8>(k, e, (int)units);
+    else return false;
+    return a.expand->rode = true;
 }
 
 bool launch_latent_attention(const LatentAttn& a, const StepArrays& st, bool only_alone) {
@@ -748,7 +780,8 @@ bool launch_latent_attention(const LatentAttn& a, const StepArrays& st, bool onl
         {
             ProfScope ps(s.max_run == 1 ? PC_LATENT_ATTN_TOK : PC_LATENT_ATTN, s.bytes, s.flops);
             const long units = s.items * s.nsplit;
-            if (chunks <= 4 && vt <= 1) launch_latent_rc<4, 1>(k, units, s.W);
+            if (attn_with_expand(k, a, units, s.W)) {}
+            else if (chunks <= 4 && vt <= 1) launch_latent_rc<4, 1>(k, units, s.W);
             else if (chunks <= 6 && vt <= 2) launch_latent_rc<6, 2>(k, units, s.W);
             else if (chunks <= 10 && vt <= 4) launch_latent_rc<10, 4>(k, units, s.W);
             else launch_latent_rc<18, 8>(k, units, s.W);

@@ -497,14 +497,14 @@ void LatentHyperModel::forward_b16(const PassArgs& a, const StepArrays& st, cons
         e2.a16_out = hid; e2.q_rows = q; e2.q_heads = m.heads; e2.q_row = Cp + Rp; e2.head_ld = Cp;
         launch_gemm_b16(w.uq, qt, T, e2, PC_GEMM_LATENT_Q, &ride);
         // attention over the latents, of tokens [t0, t0 + n) (whole 16-token blocks): W_uk into the queries, W_uv behind
-        auto over_latents = [&](int t0, int n, __half* out, bool only_alone) {
+        auto over_latents = [&](int t0, int n, __half* out, bool only_alone, LatentExpandRider* expand = nullptr) {
             GemmEpilogue e3;
             e3.kind = GemmEpilogue::ROWS_B16;
             e3.q_rows = q + (size_t)t0 * m.heads * (Cp + Rp); e3.q_heads = m.heads; e3.q_row = Cp + Rp; e3.head_ld = Cp;
             launch_gemm_b16(w.uk, hid + b16_halves(t0, m.heads * dimp), n, e3, PC_GEMM_ABSORB);
             LatentAttn at{};
             at.pool = pl; at.q = q; at.sink = w.sink; at.scale = m.scale; at.H = m.heads; at.out_b16 = latents;
-            at.uv = &w.uv; at.values = out;
+            at.uv = &w.uv; at.values = out; at.expand = expand;
             if (launch_latent_attention(at, st, only_alone)) return;
             GemmEpilogue e4;
             e4.kind = GemmEpilogue::TILE_B16;
@@ -520,12 +520,13 @@ void LatentHyperModel::forward_b16(const PassArgs& a, const StepArrays& st, cons
         // prompt portions: keys and values formed from the latents.  Their rows are written last: the blocks of the tokens beside them
         // may hold some of theirs.
         __half* values = (__half*)ws_get(WS_VALUES, b16_halves(T, val) * sizeof(__half));
-        if (plan.alone_to > plan.alone_from) over_latents(16 * plan.alone_from, std::min(T, 16 * plan.alone_to) - 16 * plan.alone_from, values, true);
         LatentPrompt pr{};
         pr.pool = pl; pr.q_tiles = hid; pr.q_rows = (const __half*)q; pr.sink = w.sink; pr.scale = m.scale; pr.H = m.heads;
         pr.dim_ld = dimp; pr.vdim_ld = vp; pr.uk = w.uk_rows.tiles; pr.uv = w.uv.tiles; pr.kv = formed; pr.out = values;
         pr.items = st.d_extra; pr.pages = st.d_extra + 4 * plan.n_items;
-        launch_latent_prompt(pr, plan);
+        LatentExpandRider expand{&pr, &plan};
+        if (plan.alone_to > plan.alone_from) over_latents(16 * plan.alone_from, std::min(T, 16 * plan.alone_to) - 16 * plan.alone_from, values, true, &expand);
+        launch_latent_prompt(pr, plan, expand.rode);
         residual(w.o, values, s, nullptr, PC_GEMM_WO);
     }
     if (B <= 0) return;

@@ -36,12 +36,30 @@ struct LatentPrompt {
     __half* out;             // activation tiles of [T, H * vdim_ld]
     const int *items, *pages;   // device copies of the plan
 };
+struct ExpandArgs {
+    const __half* base;   // the pool
+    const int* pages;     // [n_pairs][2]
+    int n_pairs, per;     // pairs, and pairs of a workgroup
+    int chunks, row_tiles;   // tiles of a page: of its latent, in all
+    int H, dc, vt;        // tiles of 32 dims of a head's key; of 16 dims of its value
+    const __half *uk, *uv;
+    __half* kv;           // [pair][head][2 dc key tiles by page, vt value tiles]
+};
+// split for `wgs` workgroups, four pairs each at least (a wave's weights are as many bytes as two pairs)
+ExpandArgs latent_expand_args(const LatentPrompt& a, const LatentPromptPlan& plan, int wgs);
 // Whether there are kernels for rows and heads of these widths.
 bool latent_prompt_fits(int rank_ld, int rot_ld, int dim_ld, int vdim_ld);
 // Whether this is the way to go for the pass's portions.
 bool latent_prompt_pays(const LatentPromptPlan& plan, int H, int rank_ld, int dim_ld, int vdim_ld);
 // Memory for the portions' keys and values; null: none (the portions attend over latents).
 __half* latent_prompt_scratch(const LatentPromptPlan& plan, int H, int dim_ld, int vdim_ld);
-void launch_latent_prompt(const LatentPrompt& a, const LatentPromptPlan& plan);
+// The same beside the attention of the tokens that come alone, if that leaves enough of the chip.
+struct LatentExpandRider {
+    const LatentPrompt* prompt;
+    const LatentPromptPlan* plan;
+    bool rode = false;
+};
+// formed: the keys and values are there (LatentAttn::expand rode)
+void launch_latent_prompt(const LatentPrompt& a, const LatentPromptPlan& plan, bool formed);
 
 }  // namespace nvllm

@@ -23,114 +23,11 @@
 #include <array>
 #include <climits>
 
-#include "attn_tile.h"
-#include "gemm_common.h"
+#include "latent_expand.h"
 
 namespace nvllm {
 
 namespace {
-
-typedef _Float16 h4_t __attribute__((ext_vector_type(4)));
-typedef float f8_t __attribute__((ext_vector_type(8)));
-typedef const __attribute__((address_space(4))) int* const_int_p;   // read-only for the whole launch: scalar loads
-
-__device__ __forceinline__ void prompt_barrier() {   // this wave's LDS accesses are done, then everybody meets
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-}
-__device__ __forceinline__ void copies_landed() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
-
-struct ExpandArgs {
-    const __half* base;   // the pool
-    const int* pages;     // [n_pairs][2]
-    int n_pairs, per;     // pairs, and pairs of a workgroup
-    int chunks, row_tiles;   // tiles of a page: of its latent, in all
-    int H, dc, vt;        // tiles of 32 dims of a head's key; of 16 dims of its value
-    const __half *uk, *uv;
-    __half* kv;           // [pair][head][2 dc key tiles by page, vt value tiles]
-};
-
-// KC: tiles of a latent that a wave has registers for
-template <int KC>
-__global__ __launch_bounds__(512, 2) void k_latent_expand(ExpandArgs a) {
-    extern __shared__ __attribute__((aligned(16))) unsigned char lds_expand[];   // [2][2][chunks] tiles
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int x = lane & 15, g = lane >> 4;
-    const int nc = a.chunks;
-    const int unit = (int)blockIdx.x * 8 + wave, key_units = a.H * a.dc, units = key_units + a.H * (a.vt / 2);
-    const bool is_key = unit < key_units, live = unit < units;
-    const int mine = min(unit, units - 1), block = (is_key ? mine : mine - key_units) * 2;   // this wave's first row block of its matrix
-    const int pair0 = (int)blockIdx.y * a.per, pair1 = min(a.n_pairs, pair0 + a.per);
-    const const_int_p pages = (const_int_p)(uintptr_t)a.pages;
-    const unsigned lds0 = (unsigned)(size_t)(lds_void*)lds_expand;
-    auto issue = [&](int pair, int buf) {   // waves 0-3 bring the first page's tiles, 4-7 the second's
-        const int half = wave >> 2;
-        const __half* src = a.base + (size_t)pages[2 * pair + half] * a.row_tiles * TILE_HALVES + lane * 8;
-        for (int c = wave & 3; c < nc; c += 4)
-            copy_tile_to_lds(src + (size_t)c * TILE_HALVES, __builtin_amdgcn_readfirstlane(lds0 + (unsigned)((buf * 2 + half) * nc + c) * 1024u));
-    };
-    issue(pair0, 0);
-    h8_t w[2][KC];
-    {
-        const __half* W = (is_key ? a.uk : a.uv) + (size_t)block * nc * TILE_HALVES + lane * 8;
-#pragma unroll
-        for (int f = 0; f < 2; f++)
-#pragma unroll
-            for (int k = 0; k < KC; k++) w[f][k] = *reinterpret_cast<const h8_t*>(W + ((size_t)f * nc + min(k, nc - 1)) * TILE_HALVES);
-    }
-    const size_t head_halves = (size_t)(2 * a.dc + a.vt) * TILE_HALVES;
-    for (int pair = pair0; pair < pair1; pair++) {
-        const int buf = (pair - pair0) & 1;
-        copies_landed();
-        prompt_barrier();
-        if (pair + 1 < pair1) issue(pair + 1, buf ^ 1);
-        const h8_t* lat = reinterpret_cast<const h8_t*>(lds_expand) + (size_t)buf * 2 * nc * 64 + lane;
-        f4_t acc[2][2] = {};   // [row block][page]
-        if (is_key) {
-#pragma unroll
-            for (int k = 0; k < KC; k++)
-                if (k < nc) {
-#pragma unroll
-                    for (int page = 0; page < 2; page++) {
-                        const h8_t c = lat[(page * nc + k) * 64];
-#pragma unroll
-                        for (int f = 0; f < 2; f++) acc[f][page] = OpBf16::mfma(w[f][k], c, acc[f][page]);
-                    }
-                }
-            if (!live) continue;
-            const int head = mine / a.dc, c = mine - head * a.dc;
-            __half* out = a.kv + ((size_t)pair * a.H + head) * head_halves;
-#pragma unroll
-            for (int f = 0; f < 2; f++)
-#pragma unroll
-                for (int page = 0; page < 2; page++)   // dims 16 f + 4 g .. + 3 of position x
-                    *reinterpret_cast<h4_t*>(out + (size_t)(page * a.dc + c) * TILE_HALVES + (x + 16 * (2 * f + (g >> 1))) * 8 + 4 * (g & 1)) =
-                        __builtin_convertvector(acc[f][page], h4_t);
-        } else {
-#pragma unroll
-            for (int k = 0; k < KC; k++)
-                if (k < nc) {
-#pragma unroll
-                    for (int page = 0; page < 2; page++) {
-                        const h8_t c = lat[(page * nc + k) * 64];
-#pragma unroll
-                        for (int f = 0; f < 2; f++) acc[f][page] = OpBf16::mfma(c, w[f][k], acc[f][page]);
-                    }
-                }
-            if (!live) continue;
-            const int head = block / a.vt, n = block - head * a.vt;
-            __half* out = a.kv + ((size_t)pair * a.H + head) * head_halves + (size_t)(2 * a.dc + n) * TILE_HALVES;
-#pragma unroll
-            for (int f = 0; f < 2; f++) {   // positions 4 g .. + 3 of both pages, dim 16 (n + f) + x
-                alignas(16) h4_t both[2];
-#pragma unroll
-                for (int page = 0; page < 2; page++) both[page] = __builtin_convertvector(acc[f][page], h4_t);
-                *reinterpret_cast<u4_t*>(out + (size_t)f * TILE_HALVES + lane * 8) = *reinterpret_cast<const u4_t*>(both);
-            }
-        }
-    }
-}
 
 struct PromptArgs {
     const __half* base;
@@ -286,8 +183,13 @@ void launch_prompt(const PromptArgs& k, int workgroups) {
     NVLLM_LAUNCH((k_latent_prompt<DC, RC, VT, RING>), dim3(workgroups), dim3(256), lds, k);
 }
 template <int KC>
+__global__ __launch_bounds__(512, 2) void k_latent_expand(ExpandArgs a) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds_expand[];
+    latent_expand<KC>(a, (int)blockIdx.x, (int)blockIdx.y, lds_expand);
+}
+template <int KC>
 void launch_expand(const ExpandArgs& e, dim3 grid) {
-    const int lds = 4 * e.chunks * 1024;
+    const int lds = (int)expand_lds(e);
     static bool enabled = false;
     if (!enabled) {
         HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_latent_expand<KC>), hipFuncAttributeMaxDynamicSharedMemorySize, 4 * KC * 1024));
@@ -380,28 +282,32 @@ __half* latent_prompt_scratch(const LatentPromptPlan& plan, int H, int dim_ld, i
     return (double)bytes <= most ? (__half*)ws_try(WS_EXPANDED, bytes) : nullptr;
 }
 
-void launch_latent_prompt(const LatentPrompt& a, const LatentPromptPlan& plan) {
+ExpandArgs latent_expand_args(const LatentPrompt& a, const LatentPromptPlan& plan, int wgs) {
+    const LatentPool& P = a.pool;
+    ExpandArgs e{};
+    e.base = (const __half*)P.base;
+    e.pages = a.pages;
+    e.n_pairs = plan.n_pairs;
+    e.chunks = P.rank_ld / 32;
+    e.row_tiles = P.row() / 32;
+    e.H = a.H;
+    e.dc = a.dim_ld / 32;
+    e.vt = a.vdim_ld / 16;
+    e.uk = a.uk;
+    e.uv = a.uv;
+    e.kv = a.kv;
+    e.per = std::max(4, cdiv(plan.n_pairs, std::max(1, wgs / expand_cols(e))));
+    return e;
+}
+
+void launch_latent_prompt(const LatentPrompt& a, const LatentPromptPlan& plan, bool formed) {
     if (plan.n_items <= 0) return;
     const LatentPool& P = a.pool;
     const double positions = 32.0 * plan.n_pairs, width = (double)a.H * (a.dim_ld + a.vdim_ld);
-    {
-        ExpandArgs e{};
-        e.base = (const __half*)P.base;
-        e.pages = a.pages;
-        e.n_pairs = plan.n_pairs;
-        e.chunks = P.rank_ld / 32;
-        e.row_tiles = P.row() / 32;
-        e.H = a.H;
-        e.dc = a.dim_ld / 32;
-        e.vt = a.vdim_ld / 16;
-        e.uk = a.uk;
-        e.uv = a.uv;
-        e.kv = a.kv;
-        const int cols = cdiv(a.H * (e.dc + e.vt / 2), 8);
-        // as many workgroups as CUs, of four pairs at least (a wave's weights are as many bytes as two pairs)
-        e.per = std::max(4, cdiv(plan.n_pairs, std::max(1, rt().num_cus / cols)));
+    if (!formed) {
+        const ExpandArgs e = latent_expand_args(a, plan, rt().num_cus);
         ProfScope ps(PC_LATENT_EXPAND, width * P.rank_ld * 2.0 + positions * P.rank_ld * 2.0 + positions * width * 2.0, 2.0 * positions * width * P.rank_ld);
-        const dim3 grid(cols, cdiv(plan.n_pairs, e.per));
+        const dim3 grid(expand_cols(e), cdiv(plan.n_pairs, e.per));
         if (e.chunks <= 8) launch_expand<8>(e, grid);
         else launch_expand<16>(e, grid);
     }

@@ -71,3 +71,20 @@ def test_portions_agree_with_attention_over_latents(tmp_path, name):
     # Both ways round as often, keys instead of absorbed queries and values instead of attended latents: the same error, in which
     # runs of a few hundred rows scatter by a tenth (0.86 to 1.12 over 36 models).
     assert error[1] < 1.25 * error[0] and error[1] < U.limit(False) / 2, error
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("heads,rank", [(32, 512), (24, 256), (17, 100), (32, 480), (16, 512)])
+def test_forming_beside_tokens_that_come_alone(hip, tmp_path, heads, rank):
+    """Items of 32 columns (17 to 32 heads) of the widest row and of one with up to eight tiles share a launch with the forming of keys and values; others
+    do not.  One, three and twenty such tokens (few and many workgroups) beside long portions."""
+    cfg = synth.latent_config(64, 130, [(M(heads, 64, 64, 64, rank, 32), 40)] * 2, streams=2)
+    path, cfg, w = U.model(tmp_path, "beside", seed=heads, cfg=cfg)
+    n = 22
+    seqs = {q: U.tokens(600 if q < 2 else 40, 130, 70 + q) for q in range(n)}
+    plan = [[(q, 30) for q in range(2, n)], [(0, 200), (5, 1)], [(3, 1), (0, 200), (1, 300), (4, 1), (6, 1)], [(q, 1) for q in range(2, 12)] + [(0, 190)] + [(q, 1) for q in range(12, n)]]
+    eng = U.engine(hip, path, False, slots=n)
+    got = U.feed_all(eng, plan, seqs)
+    eng.close()
+    for q, rows in got.items():
+        assert U.error(rows, O.forward(cfg, w, seqs[q][:len(rows)])) < U.limit(False), q
