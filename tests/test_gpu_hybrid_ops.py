@@ -221,6 +221,21 @@ def test_windowed_attention_of_a_ragged_batch(hip, H, G, dim, vdim, bs, elem):
     pool.close()
 
 
+# fp32 rows: keys that are a multiple of a workgroup's trip (128), one less and one more; lanes of a key with one piece and with all, blocks that are no power of two
+@pytest.mark.parametrize("H,G,dim,vdim,bs", [(4, 2, 64, 64, 48), (3, 3, 128, 100, 16), (2, 1, 4, 8, 16), (4, 4, 36, 64, 32)])
+def test_windows_of_whole_trips(hip, H, G, dim, vdim, bs):
+    lengths = [127, 128, 129, 255, 256, 257, 384, 385]
+    pool, kv = filled(hip, G, dim, vdim, 4, bs, lengths, dim + H)
+    seq, pos = list(range(len(lengths))), [n - 1 for n in lengths]
+    q = rng(8).standard_normal((len(pos), H, dim)).astype(np.float32)
+    for size, keep, cap in ((1000, 0, 30.0), (128, 0, 0.0), (127, 1, 30.0), (120, 9, 0.0)):
+        got = pool.attend(seq, pos, q, 2.5 * dim ** -0.5, cap, size, keep)
+        want = reference(kv, q, pos, seq, 2.5 * dim ** -0.5, cap, size, keep)
+        worst = np.abs(got - want).max() / np.abs(want).max()
+        assert worst < 3e-5, (size, keep, cap, worst)   # (the bound of the ragged batch)
+    pool.close()
+
+
 # batches large enough for items of two and four column groups: one head per group and several, exact sizes and not
 @pytest.mark.parametrize("H,G,dim,vdim,tokens", [(32, 32, 64, 64, 2048), (32, 8, 64, 64, 2048), (32, 8, 40, 48, 2048), (32, 32, 64, 64, 1024), (24, 8, 64, 64, 1536), (24, 8, 48, 40, 1536),
                                                  (32, 32, 128, 128, 1024), (32, 16, 80, 112, 1024), (6, 2, 192, 160, 600)])
