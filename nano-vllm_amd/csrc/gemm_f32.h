@@ -48,6 +48,11 @@ struct F32Gemm {
     // fp16 weights, one STORE segment: (maximum, its first index) of each 16 outputs of a token -> [block][amax_ld]
     float2* amax_pairs = nullptr;
     int amax_ld = 0;
+    // a mixture's choices and their sorting in one more workgroup, of pairs behind a norm (route.T 0: none)
+    RoutePlan route{};
+    const float* z = nullptr;   // router logits [T][ldz]
+    int ldz = 0;
+    int route_from;             // that workgroup (grid x, set by the launcher)
     // ROPE_*, KV_V
     const int* pos = nullptr;
     const int* kv_row = nullptr;
@@ -75,6 +80,12 @@ struct F32Gemm {
         seg[n_segs++] = F32Segment{gate, up, bias_gate, bias_up, 0, N, F32Out::STORE, out, N, 0, false};
         return *this;
     }
+    F32Gemm& choose(const RoutePlan& r, const float* logits, int ld) {
+        route = r;
+        z = logits;
+        ldz = ld;
+        return *this;
+    }
     F32Gemm& experts(const RoutePlan& r, long stride, const float* weight) {
         block_expert = r.block_expert;
         expert_stride = stride;
@@ -84,8 +95,8 @@ struct F32Gemm {
         return *this;
     }
 };
-// One launch for all segments: all of them gated pairs, or none.
-void launch_gemm_f32(const F32Gemm& g, int prof_cls);
+// One launch for all segments: all of them gated pairs, or none.  Whether g.route rode.
+bool launch_gemm_f32(const F32Gemm& g, int prof_cls);
 
 // The same for fp16 weights in tile order (add16) and up to THIN_TOKENS tokens; K % 32 == 0.  Activations enter the matrix
 // cores as fp16 hi + lo, as in gemm.hip.

@@ -688,16 +688,14 @@ void HybridModel::forward_f32(const PassArgs& a, const StepArrays& st) {
         const int ldz = f.experts + 1;
         launch_gemm_f32(normed(1).add(w.router32, ldz, z), PC_GEMM_ROUTER);
         const RoutePlan plan = route_plan(route_mem, T, f.experts, f.top, 16);
-        launch_route(plan, z, ldz);
+        // the shared expert first: the choice rides on its first product where there are few tokens
+        if (!f.shared_ff || !launch_gemm_f32(normed(1).add_pair(w.shared_gate32, w.shared_up32, f.shared_ff, b).choose(plan, z, ldz), PC_GEMM_SHARED_UP)) launch_route(plan, z, ldz);
+        if (f.shared_ff) launch_gemm_f32(F32Gemm(b, T, f.shared_ff).add(w.shared_down32, D_, c), PC_GEMM_SHARED_DOWN);
         const long expert = (long)f.expert_ff * D_;
         F32Gemm up = F32Gemm(x, plan.capacity, D_).norm(w.norm[1], eps_).experts(plan, expert, plan.weight);
         up.in_rows = plan.source;
         launch_gemm_f32(up.add_pair(w.gate32, w.up32, f.expert_ff, b), PC_GEMM_EXPERT_UP);
         launch_gemm_f32(F32Gemm(b, plan.capacity, f.expert_ff).experts(plan, expert, nullptr).add(w.down32, D_, d), PC_GEMM_EXPERT_DOWN);
-        if (f.shared_ff) {
-            launch_gemm_f32(normed(1).add_pair(w.shared_gate32, w.shared_up32, f.shared_ff, b), PC_GEMM_SHARED_UP);
-            launch_gemm_f32(F32Gemm(b, T, f.shared_ff).add(w.shared_down32, D_, c), PC_GEMM_SHARED_DOWN);
-        }
         MoeCombine mc{};
         mc.x = x; mc.rows = d; mc.row_of = plan.row_of; mc.top = f.top; mc.shared = f.shared_ff ? c : nullptr; mc.z = z; mc.ldz = ldz;
         mc.z_col = f.experts; mc.ld = D_;
