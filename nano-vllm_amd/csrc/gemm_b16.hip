@@ -172,7 +172,7 @@ void launch_dense(GemmArgs a) {
 template <int EPI, bool GRP>
 bool launch_kind(GemmArgs a, int prof_cls, double bytes, double flops, MoeRider* moe = nullptr, const GemmArgs* router = nullptr) {
     bool rode = false;
-    if (moe && EPI == GemmEpilogue::SWIGLU_A16) a.route = RouteRider{router->W, router->NB, router->e.out, router->e.ldo, moe->plan};
+    if (moe && EPI == GemmEpilogue::SWIGLU_A16) a.route = RouteRider{router->W, router->NB, router->e.out, router->e.ldo, router_parts(a.Tb, router->NB), moe->plan};
     if (moe && EPI == GemmEpilogue::F32 && moe->chosen) a.route.plan = moe->plan;
     auto tiles = [&]() {   // (their own rules are there)
         const bool taken = launch_gemm_waves_b16(a, &rode) || launch_gemm_wide_b16(a, &rode);
@@ -181,7 +181,7 @@ bool launch_kind(GemmArgs a, int prof_cls, double bytes, double flops, MoeRider*
     };
     static const int pf_min_t = getenv("NVLLM_GEMM_PREFILL_T") ? atoi(getenv("NVLLM_GEMM_PREFILL_T")) : 256;
     // few features: the chip fills with token groups of 16 or 32, not with dense tiles
-    const bool narrow = !GRP && EPI == GemmEpilogue::F32 && !a.e.amax_out && a.NB <= 8 && a.Tb <= 4 * rt().num_cus;
+    const bool narrow = !GRP && EPI == GemmEpilogue::F32 && !a.e.amax_out && narrow_token_blocks(a.Tb, a.NB);
     if (a.T >= pf_min_t && !narrow) {
         {
             ProfScope ps(prof_cls, bytes, flops);
@@ -205,7 +205,7 @@ bool launch_kind(GemmArgs a, int prof_cls, double bytes, double flops, MoeRider*
     if (narrow) {
         pl.nw = NW;
         pl.nbw = 2;
-        pl.TB = a.Tb * cdiv(a.NB, 2) <= rt().num_cus ? 1 : 2;
+        pl.TB = narrow_token_blocks(a.Tb, a.NB);
         pl.tiles_n = cdiv(a.NB, 2);
         pl.tiles_t = cdiv(a.Tb, pl.TB);
     }

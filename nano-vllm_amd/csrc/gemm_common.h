@@ -51,8 +51,16 @@ struct RouteRider {
     int NB;
     float* z;       // [T][ldz], whole blocks of a row
     int ldz;
+    int ss_parts;   // router_parts()
     RoutePlan plan;    // T 0: nobody rides
 };
+// Few bf16 features over whole K (gemm_b16.hip): token groups of 16, or of 32 where those are more than the CUs; 0: not in such groups.
+inline int narrow_token_blocks(int Tb, int NB) { return NB > 8 || Tb > 4 * rt().num_cus ? 0 : Tb * cdiv(NB, 2) <= rt().num_cus ? 1 : 2; }
+// Parts in which a router's launch of its own sums a token's squares (gemm_tile of eight waves).
+inline int router_parts(int Tb, int NB) {
+    const int tb = narrow_token_blocks(Tb, NB);
+    return tb ? 32 / tb : 0;
+}
 
 struct GemmArgs {
     const __half* W;

@@ -164,7 +164,7 @@ __global__ __launch_bounds__(256, 1) void k_gemm_waves(GemmArgs p, int tiles_n, 
 
 template <int TBN, int EPI, typename KVT, typename OP>
 bool launch_waves(GemmArgs a, int tiles_n, int tiles_t) {   // whether a.route rode
-    constexpr int NEED = 1024 + 16 * TBN * 1024, LDS = EPI == GemmEpilogue::SWIGLU_A16 && waves_carry_route(TBN, EPI, OP::PLANES) ? std::max(NEED, router_ride_lds(4)) : NEED;
+    constexpr int NEED = 1024 + 16 * TBN * 1024, LDS = EPI == GemmEpilogue::SWIGLU_A16 && waves_carry_route(TBN, EPI, OP::PLANES) ? std::max(NEED, ROUTER_RIDE_LDS) : NEED;
     static_assert(LDS <= 160 * 1024, "the waves' sums must fit the CU's LDS");
     static bool enabled = false;
     if (!enabled) {
@@ -173,8 +173,8 @@ bool launch_waves(GemmArgs a, int tiles_n, int tiles_t) {   // whether a.route r
     }
     a.ride_from = tiles_n * tiles_t;
     const int route = waves_carry_route(TBN, EPI, OP::PLANES) ? route_groups(a, a.ride_from) : 0;
-    static_assert((3 * 1024 + 1) * 4 <= LDS);   // (the sorting)
-    NVLLM_LAUNCH((k_gemm_waves<TBN, EPI, KVT, OP>), dim3(a.ride_from + rider_groups(a, a.ride_from, 4) + route), dim3(256), LDS, a, tiles_n, tiles_t);
+    static_assert((3 * 1024 + 1) * 4 <= NEED);   // (the sorting)
+    NVLLM_LAUNCH((k_gemm_waves<TBN, EPI, KVT, OP>), dim3(a.ride_from + rider_groups(a, a.ride_from, 4) + route), dim3(256), route > 0 ? LDS : NEED, a, tiles_n, tiles_t);
     return route > 0;
 }
 

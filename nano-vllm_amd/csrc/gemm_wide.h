@@ -229,7 +229,7 @@ bool launch_wide(GemmArgs a, int tiles_n, int tiles_t) {   // whether a.route ro
     }
     a.ride_from = tiles_n * tiles_t;
     const int route = CARRIES ? route_groups(a, a.ride_from) : 0;
-    static_assert(!CARRIES || router_ride_lds(G::WAVES) <= G::LDS);
+    static_assert(!CARRIES || ROUTER_RIDE_LDS <= G::LDS);
     NVLLM_LAUNCH((k_gemm_wide<TBN, WT, EPI, KVT, OP, EXP>), dim3(a.ride_from + rider_groups(a, a.ride_from, G::WAVES) + route), dim3(64 * G::WAVES), G::LDS, a, tiles_n, tiles_t,
                  OP::PLANES == 1 ? 1 : wide_panel(tiles_n, tiles_t, G::FB, OP::PLANES * TBN));
     return route > 0;

@@ -11,21 +11,28 @@ namespace {
 
 constexpr int ROUTER_LD = 68, ROUTER_NB = 4;   // floats between a token's logits in LDS; row blocks of the widest router
 constexpr int ROUTER_TB = 4;                   // token blocks at a time
-constexpr int router_ride_lds(int waves) { return ROUTER_TB * (2 * waves * 1024 + 16 * ROUTER_LD * 4); }
+constexpr int ROUTER_CHAINS = 8;               // sums of a logit's K: as many as the router's own launch has waves
+constexpr int ROUTER_RIDE_LDS = ROUTER_TB * (2 * ROUTER_CHAINS * 1024 + 16 * ROUTER_LD * 4);
 
 // Logits and choices of the activations (and their norm) that the tiles multiply: a workgroup's token blocks, ROUTER_TB at a time, in pairs of the
-// router's row blocks, K dealt to the waves as in gemm_waves.h, even and odd steps summed apart.  What bounds it: the bytes into its CU (a token block per wave and
-// all of K, where every wave reads the whole router, held the launch up: 33.8 us without riders, 44.6; so 34.4).
+// router's row blocks, K dealt to the waves as in gemm_waves.h.  Sums in the order of the router's own launch (gemm_tile of eight waves), so that a
+// mixture gives the same bits whether it rides or not -- a last bit moves the choice of a near tie: every eighth step is a chain of its own (even and odd
+// steps of four waves), chains are added one after the other, and squares are summed in that launch's parts (RouteRider::ss_parts).
+// What bounds it: the bytes into its CU (a token block per wave and all of K, where every wave reads the whole router, held the launch up: 33.8 us
+// without riders, 44.6; so 34.8 with chains and squares summed in pairs, 35.5 in this order).
 // Simivik-1.2B, prompts of 200, 256, 400, 700, 1,029, 1,500 tokens (router 8.7, choice and sorting 8 to 17 us a layer apart, 0.3 to 2 so):
 // 3,008 -> 2,903, 3,427 -> 3,157, 3,519 -> 3,326, 4,130 -> 3,969, 4,912 -> 4,756, 5,774 -> 5,641 us a pass.
 template <int WAVES>
 __device__ __forceinline__ void router_ride(const GemmArgs& p, int wave, int lane, unsigned char* lds) {
     constexpr int RB = ROUTER_TB, RING = 4, MINE = (RB + WAVES - 1) / WAVES;   // MINE: token blocks that a wave finishes
+    constexpr int CH = ROUTER_CHAINS / WAVES;                                   // chains of a wave
+    static_assert(CH * WAVES == ROUTER_CHAINS && RING % CH == 0);
     const RouteRider& r = p.route;
     const int group = (int)blockIdx.x - p.ride_from, groups = (int)gridDim.x - p.ride_from, part = lane >> 4, cols = p.e.ss_tiles;
-    f4_t* sums = reinterpret_cast<f4_t*>(lds);   // [RB][2][giving wave][64]
-    float* rows = reinterpret_cast<float*>(lds + RB * 2 * WAVES * 1024);   // [RB][16][ROUTER_LD]
+    f4_t* sums = reinterpret_cast<f4_t*>(lds);   // [RB][2][chain][64]
+    float* rows = reinterpret_cast<float*>(lds + RB * 2 * ROUTER_CHAINS * 1024);   // [RB][16][ROUTER_LD]
     const int steps = wave < p.Kb ? (p.Kb - wave + WAVES - 1) / WAVES : 0;
+    const bool parts32 = r.ss_parts == 32;   // (else 16)
     for (int tb0 = group * RB; tb0 < p.Tb; tb0 += groups * RB) {
         float rinv[MINE];
 #pragma unroll
@@ -33,20 +40,24 @@ __device__ __forceinline__ void router_ride(const GemmArgs& p, int wave, int lan
             rinv[m] = 1.f;
             if (!p.e.ss_in) continue;
             const float* sp = p.e.ss_in + (size_t)min((tb0 + wave + m * WAVES) * 16 + (lane & 15), p.T - 1) * cols;
-            float even = 0.f, odd = 0.f;
+            float of[8] = {};   // squares' part 4 u + (lane's row)
             for (int j0 = 0; j0 < cols; j0 += 64) {   // (all of a lane's requested together)
                 float v[16];
 #pragma unroll
                 for (int k = 0; k < 16; k++) v[k] = sp[min(j0 + 4 * k + part, cols - 1)];
 #pragma unroll
-                for (int k = 0; k < 16; k += 2) {
-                    even += j0 + 4 * k + part < cols ? v[k] : 0.f;
-                    odd += j0 + 4 * k + 4 + part < cols ? v[k + 1] : 0.f;
+                for (int k = 0; k < 16; k++) {
+                    if (j0 + 4 * k + part >= cols) v[k] = 0.f;
+                    if (k & 4 && parts32) of[4 + (k & 3)] += v[k];
+                    else of[k & 3] += v[k];
                 }
             }
-            float sum = even + odd;
-            sum += __shfl_xor(sum, 16, 64);
-            sum += __shfl_xor(sum, 32, 64);
+            float sum = 0.f;
+#pragma unroll
+            for (int q = 0; q < 32; q++) {
+                const float v = __shfl(of[q >> 2], (lane & 15) + 16 * (q & 3), 64);
+                if (q < 16 || parts32) sum += v;
+            }
             rinv[m] = __fdiv_rn(1.0f, sqrtf(__fadd_rn(__fdiv_rn(sum, (float)p.e.d_in), p.e.eps)));
         }
         for (int f0 = 0; f0 < r.NB; f0 += 2) {
@@ -57,7 +68,7 @@ __device__ __forceinline__ void router_ride(const GemmArgs& p, int wave, int lan
 #pragma unroll
             for (int j = 0; j < RB; j++) of[j] = min(j, p.Tb - 1 - tb0) * p.Kb * 64;
             h8_t a[RING][RB], w[RING][2];
-            f4_t acc[2][RB][2];
+            f4_t acc[CH][RB][2];   // of this wave's chains: wave, wave + 4
             auto load = [&](int s, int i) {   // step i of this wave's into slot s (past the last: the last again, not multiplied)
                 const int at = (wave + min(i, max(steps - 1, 0)) * WAVES) * 64;
                 const bool any = wave < p.Kb;
@@ -70,10 +81,12 @@ __device__ __forceinline__ void router_ride(const GemmArgs& p, int wave, int lan
 #pragma unroll
                 for (int j = 0; j < RB; j++)
 #pragma unroll
-                    for (int f = 0; f < 2; f++) acc[s & 1][j][f] = OpBf16::mfma(w[s][f], a[s][j], acc[s & 1][j][f]);
+                    for (int f = 0; f < 2; f++) acc[s % CH][j][f] = OpBf16::mfma(w[s][f], a[s][j], acc[s % CH][j][f]);
             };
 #pragma unroll
-            for (int j = 0; j < RB; j++) acc[0][j][0] = acc[0][j][1] = acc[1][j][0] = acc[1][j][1] = f4_t{0.f, 0.f, 0.f, 0.f};
+            for (int c = 0; c < CH; c++)
+#pragma unroll
+                for (int j = 0; j < RB; j++) acc[c][j][0] = acc[c][j][1] = f4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int s = 0; s < RING; s++) load(s, s);
             int i = 0;
@@ -89,9 +102,11 @@ __device__ __forceinline__ void router_ride(const GemmArgs& p, int wave, int lan
                 if (i + s < steps) step(s);
             __syncthreads();   // (the sums of the pair before have been read)
 #pragma unroll
-            for (int j = 0; j < RB; j++)
+            for (int c = 0; c < CH; c++)
 #pragma unroll
-                for (int f = 0; f < 2; f++) sums[((j * 2 + f) * WAVES + wave) * 64 + lane] = acc[0][j][f] + acc[1][j][f];
+                for (int j = 0; j < RB; j++)
+#pragma unroll
+                    for (int f = 0; f < 2; f++) sums[((j * 2 + f) * ROUTER_CHAINS + wave + WAVES * c) * 64 + lane] = acc[c][j][f];
             __syncthreads();
 #pragma unroll
             for (int m = 0; m < MINE; m++) {
@@ -99,15 +114,14 @@ __device__ __forceinline__ void router_ride(const GemmArgs& p, int wave, int lan
                 if (j >= RB) continue;
 #pragma unroll
                 for (int f = 0; f < 2; f++) {
-                    f4_t sum[WAVES];
+                    f4_t chain[ROUTER_CHAINS];
 #pragma unroll
-                    for (int u = 0; u < WAVES; u++) sum[u] = sums[((j * 2 + f) * WAVES + u) * 64 + lane];
+                    for (int u = 0; u < ROUTER_CHAINS; u++) chain[u] = sums[((j * 2 + f) * ROUTER_CHAINS + u) * 64 + lane];
+                    f4_t sum = chain[0];
 #pragma unroll
-                    for (int o = 1; o < WAVES; o *= 2)
-#pragma unroll
-                        for (int u = 0; u < WAVES; u += 2 * o) sum[u] += sum[u + o];
+                    for (int u = 1; u < ROUTER_CHAINS; u++) sum += chain[u];
                     const int n = (f0 + f) * 16 + 4 * part;
-                    const float4 y = make_float4(sum[0][0] * rinv[m], sum[0][1] * rinv[m], sum[0][2] * rinv[m], sum[0][3] * rinv[m]);
+                    const float4 y = make_float4(sum[0] * rinv[m], sum[1] * rinv[m], sum[2] * rinv[m], sum[3] * rinv[m]);
                     if (f0 + f < r.NB) {
                         *reinterpret_cast<float4*>(rows + (j * 16 + (lane & 15)) * ROUTER_LD + n) = y;
                         if (t < p.T) *reinterpret_cast<float4*>(r.z + (size_t)t * r.ldz + n) = y;
@@ -145,7 +159,7 @@ inline int route_groups(const GemmArgs& a, int tiles) {
     const int spare = rt().num_cus - tiles;
     if (r.T == 0 || spare <= 0) return 0;
     if (a.e.kind == GemmEpilogue::F32) return (long)r.T * r.top <= 4096 && r.E <= 1024 ? 1 : 0;
-    if (a.e.kind != GemmEpilogue::SWIGLU_A16 || a.route.NB > ROUTER_NB || r.E > 64) return 0;
+    if (a.e.kind != GemmEpilogue::SWIGLU_A16 || a.route.NB > ROUTER_NB || r.E > 64 || !router_parts(a.Tb, a.route.NB)) return 0;
     const int groups = std::min(cdiv(a.Tb, ROUTER_TB), spare);
     return cdiv(a.Tb, groups * ROUTER_TB) * cdiv(a.route.NB, 2) <= 2 ? groups : 0;
 }

@@ -1,13 +1,19 @@
 """Passes of few tokens, whose router and choice of experts ride on the shared expert's products: at the edges of a token block, of the
 chosen tile heights and of the passes that launch them apart; routers of one and of several feature tiles."""
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 
 from nvllm_amd import synth
 from tests import hybrid_oracle as O
 from tests import hybrid_util as U
+from tests.test_gpu_latent_order import flops_of
 
 pytestmark = pytest.mark.gpu
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
 @pytest.mark.parametrize("experts,shared", [(5, 40), (40, 96), (70, 64)])
@@ -67,3 +73,59 @@ def test_riders_beside_k_splits(hip, tmp_path, width, experts, shared):
         np.testing.assert_array_equal(U.feed_all(eng, [[(0, n)]], {0: seq})[0], got)
         assert U.error(got, O.forward(cfg, weights, seq)) < U.limit(False), n
     eng.close()
+
+
+def passes(hip, path, tokens):
+    """Logits of a prompt per count, and the launches of a router and of a choice apart in them."""
+    eng = U.engine(hip, path, False, slots=1, tokens=2208)
+    out = {}
+    hip.nvllm_prof_reset()
+    hip.nvllm_prof_enable(1)
+    try:
+        for n in tokens:
+            out[str(n)] = U.feed_all(eng, [[(0, n)]], {0: U.tokens(n, 211, n)})[0]
+    finally:
+        hip.nvllm_prof_enable(0)
+    out["apart"] = np.array([flops_of(hip, c)[0] for c in ("gemm_router", "route")])
+    hip.nvllm_prof_reset()
+    eng.close()
+    return out
+
+
+CHILD = """
+import sys
+import numpy as np
+from nvllm_amd import capi
+from tests import test_gpu_moe_riders
+np.savez(sys.argv[2], **test_gpu_moe_riders.passes(capi.load_hip(), sys.argv[1], [int(n) for n in sys.argv[3:]]))
+"""
+
+
+# Tiles: the launchers' own; K dealt to four waves (one height of 22 x 11 tiles, which leave fewer CUs than there are groups of token blocks, so
+# that a rider has two); 256 features by four waves (19 x 13) and by eight (35 x 7), the same.  Squares in 9, 35 and 65 sums, two of them past the parts
+# (32; 16 of 2,100 tokens with four row blocks).  200 tokens: the first product in tiles, the second streaming
+@pytest.mark.parametrize("env,width,shared,experts,top,tokens", [
+    ({}, 288, 96, 31, 3, (256, 257, 1100)), ({}, 288, 96, 63, 4, (511, 2100)), ({}, 1100, 96, 15, 2, (300,)), ({}, 2080, 64, 63, 2, (256, 2100)), ({}, 288, 2816, 16, 2, (200,)),
+    ({"NVLLM_GEMM_WAVES": "6"}, 288, 1408, 16, 2, (1029,)), ({"NVLLM_GEMM_WAVES": "2"}, 1100, 416, 40, 2, (433,)),
+    ({"NVLLM_GEMM_WIDE": "4"}, 288, 2400, 31, 2, (800,)), ({"NVLLM_GEMM_WIDE": "8"}, 288, 4480, 5, 2, (800,)), ({"NVLLM_GEMM_WIDE": "12"}, 1100, 416, 63, 2, (433,))])
+def test_the_same_choices_as_apart(hip, tmp_path, env, width, shared, experts, top, tokens):
+    """A shared expert whose second matrix is zero against none at all: only who forms logits and choices differs, and no bit may."""
+    window = synth.window_mixer(4, 2, 16, 16, size=48, keep_first=4)
+    got = []
+    for ff in (shared, None):
+        cfg = synth.hybrid_config(width, 211, [(window, synth.expert_mlp(48, experts, top, ff))] * 2)
+        if ff:
+            path, _, weights = U.model(tmp_path, "rides", seed=experts, cfg=cfg, edit=lambda name, v: 0 * v if name.endswith("shared.down") else None)
+        else:
+            path, _, _ = U.model(tmp_path, "apart", seed=experts, cfg=cfg, edit=lambda name, v: weights[name])
+        if env:
+            dst = str(tmp_path / ("got%d.npz" % len(got)))
+            r = subprocess.run([sys.executable, "-c", CHILD, path, dst, *map(str, tokens)], capture_output=True, text=True, timeout=110,
+                               env=dict(os.environ, PYTHONPATH=ROOT + os.pathsep + os.environ.get("PYTHONPATH", ""), **env))
+            assert r.returncode == 0, r.stderr[-2000:]
+            got.append(np.load(dst))
+        else:
+            got.append(passes(hip, path, tokens))
+    assert got[0]["apart"][0] == 0 and got[1]["apart"][0] == 2 * len(tokens)
+    for n in tokens:
+        np.testing.assert_array_equal(got[0][str(n)], got[1][str(n)], err_msg=str(n))
