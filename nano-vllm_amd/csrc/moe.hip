@@ -31,7 +31,9 @@ size_t route_ints(int T, int E, int top, int pad) {
     const size_t cap = (size_t)route_capacity(T, E, top, pad);
     return cap / 16 + 2 * cap + 3 * (size_t)T * top + 64;
 }
+// (the sizes are checked here, for plans whose choices ride in a projection's launch too)
 RoutePlan route_plan(int* mem, int T, int E, int top, int pad) {
+    if (E < 1 || E > MAX_EXPERTS || top < 1 || top > E) NVLLM_FATAL("routing: %d of %d experts per token", top, E);
     RoutePlan r{};
     r.T = T; r.E = E; r.top = top; r.pad = pad;
     r.capacity = route_capacity(T, E, top, pad);
@@ -57,7 +59,6 @@ __global__ __launch_bounds__(1024) void k_route_sort(RoutePlan r, const float* _
 
 void launch_route(const RoutePlan& r, const float* z, int ldz, bool chosen) {
     if (r.T <= 0) return;
-    if (r.E < 1 || r.E > MAX_EXPERTS || r.top < 1 || r.top > r.E) NVLLM_FATAL("routing: %d of %d experts per token", r.top, r.E);
     const size_t lds = ((size_t)3 * r.E + 1) * sizeof(int);
     const double bytes = (double)r.T * (r.E * 4.0 + r.top * 20.0);
     const size_t lds_one = route_sort_lds(r.T, r.E, r.top);

@@ -129,3 +129,17 @@ def test_the_same_choices_as_apart(hip, tmp_path, env, width, shared, experts, t
     assert got[0]["apart"][0] == 0 and got[1]["apart"][0] == 2 * len(tokens)
     for n in tokens:
         np.testing.assert_array_equal(got[0][str(n)], got[1][str(n)], err_msg=str(n))
+
+
+@pytest.mark.parametrize("f32,shared", [(True, 8), (True, None), (False, 8)])
+def test_more_experts_than_the_limit_are_refused(tmp_path, monkeypatch, f32, shared):
+    """4,096 experts, whoever chooses among them: refused before the pass launches anything."""
+    cfg = synth.hybrid_config(32, 64, [(synth.window_mixer(1, 1, 8, 8, size=16, keep_first=1), synth.expert_mlp(4, 4097, 2, shared))])
+    monkeypatch.setattr(synth, "_tensor_values", lambda shape, kind, rng, routed: rng.standard_normal(shape))
+    path, _, _ = U.model(tmp_path, "many", cfg=cfg)
+    code = ("import sys\nfrom nvllm_amd import capi\nfrom tests import hybrid_util as U\neng = U.engine(capi.load_hip(), sys.argv[1], %r, slots=1, tokens=64)\n"
+            "eng.feed(0, [1, 2, 3], range(3))\neng.feed_run()\nprint('survived')\n" % f32)
+    r = subprocess.run([sys.executable, "-c", code, path], capture_output=True, text=True, timeout=110,
+                       env=dict(os.environ, PYTHONPATH=ROOT + os.pathsep + os.environ.get("PYTHONPATH", "")))
+    assert r.returncode != 0 and "survived" not in r.stdout
+    assert "2 of 4097 experts" in r.stderr, r.stderr[-500:]
