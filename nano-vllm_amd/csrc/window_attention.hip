@@ -612,7 +612,7 @@ __global__ __launch_bounds__(64 * WAVES) void k_window_rows(KvPages pool, const 
 static bool launch_window_rows(const WindowAttn& w, const StepArrays& st) {
     const KvPages& pool = w.pool;
     const int widest = std::max(pool.dim, pool.vdim);
-    if (pool.elem_bytes != 4 || pool.dim % 4 || pool.vdim % 4 || widest > 128) return false;
+    if (pool.elem_bytes != 4 || pool.dim % 4 || pool.vdim % 4 || widest > 128 || ((uintptr_t)w.q | (uintptr_t)w.out_f32) % 16) return false;   // (a caller's rows of 16-byte pieces)
     // us a layer, k_window_attn_any and these, 16 heads of 64 (128), a window of 512 and 16 kept: 1 row of 40 and 300 cached 5.2 and 4.6, 13.0 and 7.9 (5.9
     // and 4.7, 17.2 and 11.0), 32 rows of 600 26.3 and 18.4 (38.4 and 29.6), prompts of 100, 200, 400 9.7 and 8.6, 23.1 and 19.8, 50.5 and 44.3 (11.1 and
     // 11.2, 29.6 and 28.4, 66.6 and 70.4: wide heads of many tokens stay there)

@@ -51,10 +51,12 @@ class WindowPool:
         raw = np.concatenate([np.zeros((n, self.dim * self.G)), keys.reshape(n, -1), values.reshape(n, -1)], 1)
         self.conv([seq] * n, list(range(n)), raw, self.G)
 
-    def attend(self, seq_ids, pos, q, scale, cap, size, keep):
+    def attend(self, seq_ids, pos, q, scale, cap, size, keep, off=(0, 0)):
+        """off: floats in front of the results and of the queries."""
         (T, H), d = q.shape[:2], Dev(self.hip)
-        out = d.empty(T * H * self.vdim)
-        self.hip.nvllm_window_attention(out, d(q), C.byref(self.mgr), self.ptrs(), capi.ints(seq_ids), capi.ints(pos), scale, cap, size, keep, H, self.G,
+        out = d.empty(T * H * self.vdim + off[0]) + 4 * off[0]
+        q = d(np.concatenate([np.zeros(off[1], np.float32), np.ravel(q)])) + 4 * off[1]
+        self.hip.nvllm_window_attention(out, q, C.byref(self.mgr), self.ptrs(), capi.ints(seq_ids), capi.ints(pos), scale, cap, size, keep, H, self.G,
                                         self.dim, self.vdim, self.elem, T)
         res = self.hip.to_host(out, (T, H, self.vdim))
         d.close()
@@ -233,6 +235,9 @@ def test_windows_of_whole_trips(hip, H, G, dim, vdim, bs):
         want = reference(kv, q, pos, seq, 2.5 * dim ** -0.5, cap, size, keep)
         worst = np.abs(got - want).max() / np.abs(want).max()
         assert worst < 3e-5, (size, keep, cap, worst)   # (the bound of the ragged batch)
+    for off in ((0, 1), (2, 0), (3, 3)):   # rows that no 16-byte piece may be read from or written to
+        again = pool.attend(seq, pos, q, 2.5 * dim ** -0.5, cap, size, keep, off)
+        assert np.abs(again - want).max() < 3e-5 * np.abs(want).max(), off
     pool.close()
 
 
