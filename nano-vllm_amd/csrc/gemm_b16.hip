@@ -80,7 +80,8 @@ bool launch_moe_plan(const GemmArgs& a, const GemmPlan& pl, const MoeRider& m, c
         if (riders > 4 * rt().num_cus) return false;
     } else {
         r.plan = m.plan; r.z = m.z; r.ldz = m.ldz;
-        if (m.plan.T > ROUTE_ONE) return false;
+        const double bytes = (double)a.N * a.Kb * 64.0 + (double)a.T * a.Kb * 64.0 + (double)a.T * a.N * 4.0;
+        if (!route_rides(m.plan, NW, 5.0 + bytes / 3.0e6)) return false;
         least = (int)route_sort_lds(m.plan.T, m.plan.E, m.plan.top);
     }
     if (pl.nw != NW && pl.nw != 0) return false;

@@ -373,8 +373,8 @@ bool launch_gemm_f32(const F32Gemm& g, int prof_cls) {
     static const int shapes[][2] = {{1, 1}, {1, 2}, {2, 2}, {2, 3}, {2, 4}}, pair_shapes[][2] = {{1, 1}, {1, 2}, {1, 3}, {1, 4}};
     int NB = 1, TB = 1;
     long tiles_all = (long)blocks * Tb;
+    double best = 0;   // cycles per k
     if (!a.block_expert && rows16) {
-        double best = 0;
         for (int i = 0; i < (pair ? 4 : 5); i++) {
             const int nb = pair ? pair_shapes[i][0] : shapes[i][0], tb = pair ? pair_shapes[i][1] : shapes[i][1], nt = pair ? 2 * nb : nb;
             const long tiles = (long)cdiv(blocks, nb) * cdiv(Tb, tb);
@@ -403,10 +403,9 @@ bool launch_gemm_f32(const F32Gemm& g, int prof_cls) {
         else NVLLM_LAUNCH(k_gemm_f32_any<false>, grid, dim3(256), 0, a);
         return false;
     }
-    // Choices of few tokens and their sorting, by one workgroup more: 80 tokens over 16 experts 9.4 us in a launch of their own, beside 440 tiles that
-    // take 16.0 without it 1.0.
+    // Choices of few tokens and their sorting, by one workgroup more (route_rides)
     a.route_from = tiles;
-    const bool rides = a.route.T > 0 && pair && a.gain && a.route.T <= ROUTE_ONE && route_sort_lds(a.route.T, a.route.E, a.route.top) <= 64 * 1024;
+    const bool rides = a.route.T > 0 && pair && a.gain && route_rides(a.route, KS, 3.0 + best * a.K / 2600.0) && route_sort_lds(a.route.T, a.route.E, a.route.top) <= 64 * 1024;
     const dim3 grid(tiles + rides, cdiv(Tb, TB));
 #define NVLLM_GEMM_F32(nb, tb, ks, pr)                                                                    \
     do {                                                                                                  \

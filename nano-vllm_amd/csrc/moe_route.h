@@ -152,4 +152,19 @@ __device__ __forceinline__ void route_sort(RoutePlan r, const float* __restrict_
 static inline size_t route_sort_lds(int T, int E, int top) { return ((size_t)3 * E + 1) * sizeof(int) + (size_t)T * top * 8; }
 constexpr int ROUTE_ONE = 256;      // tokens up to which one workgroup chooses and sorts
 
+// us that a workgroup takes to choose and sort: a step of a wave picks the best of what is left for four tokens (one, past 64 experts).
+// 256 tokens, 4, 8 and 16 waves: 8 of 64 experts 114, 69, 54; 2 of 128 140, 66, 34; 8 of 512 952, 537, 316; 8 of 2,048 3,449, -, 1,150.
+static inline double route_us(int T, int E, int top, int waves) {
+    const double step = E > 64 ? 0.9 + 0.18 * E / 64 : waves <= 4 ? 0.9 : waves <= 8 ? 1.03 : 1.7;
+    return 2.0 + step * top * (double)((E > 64 ? T + waves - 1 : (T + 4 * waves - 1) / 4) / waves);
+}
+// Whether that rides in a workgroup of `waves` waves beside tiles of `tiles_us`: where it then ends no later than a launch of its own would,
+// which costs another microsecond and has 16 waves.  fp32 pairs of 2,816 features over 1,024 k, both ways (tiles alone): 80 tokens, 2 of 16 experts 28 and 36 us (28); 128, 2
+// of 64 28 and 39 (29); 8 of 64, 96 tokens 40 and 53 (26), 192 86 and 80 (36); 2 of 128, 48 tokens 16 and 25 (16), 64 34 and 29, 256 140 and 82
+// (44); 8 of 512, 256 tokens 952 and 365.  bf16, 1,024 features over 2,816 k: 2 of 16, 64 tokens 11 and 16 (10); 8 of 64, 128 36 and 39 (9); 2 of 65,
+// 64 tokens 19 and 22 (10), 128 34 and 29; 8 of 512, 16 tokens 36 and 30 (8).
+static inline bool route_rides(const RoutePlan& r, int waves, double tiles_us) {
+    return r.T <= ROUTE_ONE && route_us(r.T, r.E, r.top, waves) <= tiles_us + 1.0 + route_us(r.T, r.E, r.top, 16);
+}
+
 }  // namespace nvllm

@@ -143,3 +143,28 @@ def test_more_experts_than_the_limit_are_refused(tmp_path, monkeypatch, f32, sha
                        env=dict(os.environ, PYTHONPATH=ROOT + os.pathsep + os.environ.get("PYTHONPATH", "")))
     assert r.returncode != 0 and "survived" not in r.stdout
     assert "2 of 4097 experts" in r.stderr, r.stderr[-500:]
+
+
+@pytest.mark.parametrize("f32", [True, False], ids=["fp32", "bf16"])
+@pytest.mark.parametrize("experts,top,rides,apart", [(16, 2, (8, 64, 80), ()), (64, 8, (16,), (192,)), (128, 2, (16,), (96, 128)), (128, 8, (), (64, 128))])
+def test_long_choices_are_launched_apart(hip, tmp_path, f32, experts, top, rides, apart):
+    """One workgroup beside a product's tiles chooses only where it is about as soon done as a launch of its own (route_rides); who chooses shows in no bit."""
+    if not f32:
+        rides, apart = [n for n in rides if n <= 128], [n for n in apart if n <= 128]   # (more tokens take tiles, which carry other riders)
+    window = synth.window_mixer(4, 2, 16, 16, size=48, keep_first=4)
+    cfg = synth.hybrid_config(128, 211, [(window, synth.expert_mlp(16, experts, top, 256))])
+    path, cfg, weights = U.model(tmp_path, "long", seed=experts, cfg=cfg)
+    eng = U.engine(hip, path, f32, slots=1)
+    try:
+        for n in sorted([*rides, *apart]):
+            seq = U.tokens(n, 211, n)
+            hip.nvllm_prof_reset()
+            hip.nvllm_prof_enable(1)
+            got = U.feed_all(eng, [[(0, n)]], {0: seq})[0]
+            hip.nvllm_prof_enable(0)
+            assert flops_of(hip, "route")[0] == (n in apart), n
+            assert U.error(got, O.forward(cfg, weights, seq)) < U.limit(f32), n
+    finally:
+        hip.nvllm_prof_enable(0)
+        hip.nvllm_prof_reset()
+        eng.close()
