@@ -36,6 +36,7 @@ struct MoeRide {
     RoutePlan plan;
     const float* z;
     int ldz;
+    bool chosen;   // (beside the product before: sorting is left)
 };
 constexpr int ROUTER_NB = 2;   // 16-row blocks of the router and ...
 template <int NBW, int TB, int EPI>
@@ -48,6 +49,8 @@ __global__ __launch_bounds__(NW * 64) void k_gemm_b16_moe(GemmArgs p, MoeRide r)
             const TileIdx ix{i % r.router_tiles, 0, i / r.router_tiles, r.router_tiles};
             h8_t w[RW][ROUTER_NB];
             gemm_tile<ROUTER_NB, 1, NW, RW, RA, GemmEpilogue::F32, float, false, 0, OpBf16, false, false>(r.router, ix, lds_dyn, w, [](int) {}, (int)threadIdx.x);
+        } else if (r.chosen) {
+            route_sort<false, NW * 64>(r.plan, nullptr, 0, reinterpret_cast<int*>(lds_dyn));
         } else {
             route_sort<true, NW * 64>(r.plan, r.z, r.ldz, reinterpret_cast<int*>(lds_dyn));
         }
@@ -79,9 +82,9 @@ bool launch_moe_plan(const GemmArgs& a, const GemmPlan& pl, const MoeRider& m, c
         least = gemm_tile_lds<ROUTER_NB, 1, NW>();
         if (riders > 4 * rt().num_cus) return false;
     } else {
-        r.plan = m.plan; r.z = m.z; r.ldz = m.ldz;
+        r.plan = m.plan; r.z = m.z; r.ldz = m.ldz; r.chosen = m.chosen;
         const double bytes = (double)a.N * a.Kb * 64.0 + (double)a.T * a.Kb * 64.0 + (double)a.T * a.N * 4.0;
-        if (!route_rides(m.plan, NW, 5.0 + bytes / 3.0e6)) return false;
+        if (!(m.chosen ? m.plan.T <= ROUTE_ONE : route_rides(m.plan, NW, 5.0 + bytes / 3.0e6))) return false;
         least = (int)route_sort_lds(m.plan.T, m.plan.E, m.plan.top);
     }
     if (pl.nw != NW && pl.nw != 0) return false;
