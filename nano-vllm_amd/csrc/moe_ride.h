@@ -152,16 +152,23 @@ __device__ __forceinline__ void router_ride(const GemmArgs& p, int wave, int lan
     __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0): else the compiler waits inside the tiles' loop for what flies here
 }
 
-// Riders beside `tiles` workgroups, of which a CU holds one: on free CUs only, and only what is done before the tiles are: up to
-// two passes of the router over a workgroup's blocks, up to 4,096 choices to sort (256 threads; the launch of its own has 1,024).
+// Riders beside `tiles` workgroups, of which a CU holds one: on free CUs only, and only what is done about when the tiles are: up to two passes of the
+// router over a workgroup's blocks, of which a wave chooses for 16 tokens, and up to 4,096 choices to sort (256 threads; the launch of its own has 1,024).
+// us: a pass over the blocks, a step of four tokens' choices, the tiles at 900 TFLOP/s; and what the launches of router, choice and sorting take that are
+// saved.  Both ways, those launches and both products (Kb 64, 5,632 features, 31 and 32, 9): 2 of 16 experts, 400 and 1,029 tokens 31 and 50, 57 and 68;
+// 4 of 31 at 32 400, 1,029 (two trips of a rider), 1,500 33 and 41, 65 and 56, 54 and 63; 8 of 63 256, 700, 1,500 55 and 91, 71 and 68, 99 and 103; at 32
+// 46 and 85, 63 and 53, 80 and 76; of 1,536 features at 9 39 and 73, 50 and 35, 61 and 50.
 inline int route_groups(const GemmArgs& a, int tiles) {
     const RoutePlan& r = a.route.plan;
     const int spare = rt().num_cus - tiles;
     if (r.T == 0 || spare <= 0) return 0;
     if (a.e.kind == GemmEpilogue::F32) return (long)r.T * r.top <= 4096 && r.E <= 1024 ? 1 : 0;
     if (a.e.kind != GemmEpilogue::SWIGLU_A16 || a.route.NB > ROUTER_NB || r.E > 64 || !router_parts(a.Tb, a.route.NB)) return 0;
-    const int groups = std::min(cdiv(a.Tb, ROUTER_TB), spare);
-    return cdiv(a.Tb, groups * ROUTER_TB) * cdiv(a.route.NB, 2) <= 2 ? groups : 0;
+    const int groups = std::min(cdiv(a.Tb, ROUTER_TB), spare), trips = cdiv(a.Tb, groups * ROUTER_TB), passes = cdiv(a.route.NB, 2);
+    if (trips * passes > 2) return 0;
+    const double rider = 2.0 + trips * (passes * (2.0 + 0.065 * a.Kb) + 4.0 * r.top * 0.87), tiled = 5.0 + 1024.0 * r.T * a.Kb * a.NB / 9.0e8;
+    const double saved = 7.5 + 0.06 * a.Kb + (r.T <= ROUTE_ONE ? 1.0 + route_us(r.T, r.E, r.top, 16) : 3.0 + 0.5 * r.top);
+    return rider <= tiled + saved ? groups : 0;
 }
 
 }  // namespace
