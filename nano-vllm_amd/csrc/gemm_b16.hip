@@ -178,6 +178,13 @@ bool launch_kind(GemmArgs a, int prof_cls, double bytes, double flops, MoeRider*
     bool rode = false;
     if (moe && EPI == GemmEpilogue::SWIGLU_A16) a.route = RouteRider{router->W, router->NB, router->e.out, router->e.ldo, router_parts(a.Tb, router->NB), moe->plan};
     if (moe && EPI == GemmEpilogue::F32 && moe->chosen) a.route.plan = moe->plan;
+    auto count = [&](ProfScope& ps) {   // what rode
+        if (!rode) return;
+        if (EPI == GemmEpilogue::SWIGLU_A16)
+            ps.add((double)router->N * router->Kb * 64.0 + (double)a.T * router->N * 4.0 + (moe->chosen ? choice_bytes(moe->plan) : 0.0), 2.0 * a.T * (double)router->N * router->Kb * 32.0);
+        else
+            ps.add(moe->chosen ? sort_bytes(moe->plan) : choice_bytes(moe->plan), 0);
+    };
     auto tiles = [&]() {   // (their own rules are there)
         const bool taken = launch_gemm_waves_b16(a, &rode) || launch_gemm_wide_b16(a, &rode);
         if (rode && EPI == GemmEpilogue::SWIGLU_A16) moe->chosen = true;
@@ -191,6 +198,7 @@ bool launch_kind(GemmArgs a, int prof_cls, double bytes, double flops, MoeRider*
             ProfScope ps(prof_cls, bytes, flops);
             a.e.amax_pairs = nullptr;   // the dense-tile kernel does not emit pairs: the rows are scanned afterwards
             if (GRP || !tiles()) launch_dense<EPI, GRP>(a);
+            count(ps);
         }
         if (EPI == GemmEpilogue::F32 && a.e.amax_out) launch_argmax_ld(a.e.amax_out, a.e.out, a.T, a.N, a.e.ldo, a.e.amax_out_host);
         if (EPI == GemmEpilogue::F32 && a.e.out_host) copy_rows_to_host(a.e.out_host, a.e.out, (size_t)a.T * a.e.ldo);
@@ -200,7 +208,10 @@ bool launch_kind(GemmArgs a, int prof_cls, double bytes, double flops, MoeRider*
         a.ksplit = 1;
         a.kb_per_split = a.Kb;
         ProfScope ps(prof_cls, bytes, flops);
-        if (tiles()) return rode;
+        if (tiles()) {
+            count(ps);
+            return rode;
+        }
         ps.drop();
     }
     // a block-diagonal product has a short K and no K split; its plan is that of one group times the groups
@@ -236,6 +247,7 @@ bool launch_kind(GemmArgs a, int prof_cls, double bytes, double flops, MoeRider*
         if constexpr (!GRP && (EPI == GemmEpilogue::SWIGLU_A16 || EPI == GemmEpilogue::F32))
             rode = moe && launch_moe_plan<EPI>(a, pl, *moe, router ? *router : a);
         if (!rode) launch_stream_plan<EPI, GRP>(a, pl);
+        count(ps);
     }
     if (EPI == GemmEpilogue::F32 && a.e.amax_out) {
         if (!a.e.amax_pairs || a.e.amax_ld < a.T) NVLLM_FATAL("fused arg-max needs a pair buffer of at least %d rows per tile", a.T);

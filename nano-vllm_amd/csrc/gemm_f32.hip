@@ -406,6 +406,7 @@ bool launch_gemm_f32(const F32Gemm& g, int prof_cls) {
     // Choices of few tokens and their sorting, by one workgroup more (route_rides)
     a.route_from = tiles;
     const bool rides = a.route.T > 0 && pair && a.gain && route_rides(a.route, KS, 3.0 + best * a.K / 2600.0) && route_sort_lds(a.route.T, a.route.E, a.route.top) <= 64 * 1024;
+    if (rides) ps.add(choice_bytes(a.route), 0);
     const dim3 grid(tiles + rides, cdiv(Tb, TB));
 #define NVLLM_GEMM_F32(nb, tb, ks, pr)                                                                    \
     do {                                                                                                  \

@@ -696,12 +696,15 @@ static void launch_attn_expand(const LatentKArgs& k, const ExpandArgs& e, int un
 }
 // Items of 32 columns (eight waves, as the forming has) on a quarter of the CUs at most, the forming on the others: five tokens at 1,050
 // beside 1,024 behind 1,024 positions, 32 heads of 512: 45 workgroups of 10.8 us and 256 of 14.4 one after the other, together 16.8 (253).
-static bool attn_with_expand(const LatentKArgs& k, const LatentAttn& a, long units, int columns) {
+static bool attn_with_expand(const LatentKArgs& k, const LatentAttn& a, long units, int columns, ProfScope& ps) {
     if (!a.expand || columns != 32 || units * 4 > rt().num_cus) return false;
     const ExpandArgs e = latent_expand_args(*a.expand->prompt, *a.expand->plan, rt().num_cus - (int)units);
     if (k.chunks == 18 && k.n_tiles == 32) launch_attn_expand<18, 8, true, 16>(k, e, (int)units);
     else if (k.chunks <= 10 && k.n_tiles <= 16 && e.chunks <= 8) launch_attn_expand<10, 4, false, 8>(k, e, (int)units);
     else return false;
+    double bytes, flops;
+    latent_expand_work(*a.expand->prompt, *a.expand->plan, &bytes, &flops);
+    ps.add(bytes, flops);
     return a.expand->rode = true;
 }
 
@@ -780,7 +783,7 @@ bool launch_latent_attention(const LatentAttn& a, const StepArrays& st, bool onl
         {
             ProfScope ps(s.max_run == 1 ? PC_LATENT_ATTN_TOK : PC_LATENT_ATTN, s.bytes, s.flops);
             const long units = s.items * s.nsplit;
-            if (attn_with_expand(k, a, units, s.W)) {}
+            if (attn_with_expand(k, a, units, s.W, ps)) {}
             else if (chunks <= 4 && vt <= 1) launch_latent_rc<4, 1>(k, units, s.W);
             else if (chunks <= 6 && vt <= 2) launch_latent_rc<6, 2>(k, units, s.W);
             else if (chunks <= 10 && vt <= 4) launch_latent_rc<10, 4>(k, units, s.W);

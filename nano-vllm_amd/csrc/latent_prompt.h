@@ -47,6 +47,8 @@ struct ExpandArgs {
 };
 // split for `wgs` workgroups, four pairs each at least (a wave's weights are as many bytes as two pairs)
 ExpandArgs latent_expand_args(const LatentPrompt& a, const LatentPromptPlan& plan, int wgs);
+// ... and its work, for kernel timing
+void latent_expand_work(const LatentPrompt& a, const LatentPromptPlan& plan, double* bytes, double* flops);
 // Whether there are kernels for rows and heads of these widths.
 bool latent_prompt_fits(int rank_ld, int rot_ld, int dim_ld, int vdim_ld);
 // Whether this is the way to go for the pass's portions.

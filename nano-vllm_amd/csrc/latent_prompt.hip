@@ -300,13 +300,21 @@ ExpandArgs latent_expand_args(const LatentPrompt& a, const LatentPromptPlan& pla
     return e;
 }
 
+void latent_expand_work(const LatentPrompt& a, const LatentPromptPlan& plan, double* bytes, double* flops) {
+    const double positions = 32.0 * plan.n_pairs, width = (double)a.H * (a.dim_ld + a.vdim_ld), rank = a.pool.rank_ld;
+    *bytes = width * rank * 2.0 + positions * rank * 2.0 + positions * width * 2.0;
+    *flops = 2.0 * positions * width * rank;
+}
+
 void launch_latent_prompt(const LatentPrompt& a, const LatentPromptPlan& plan, bool formed) {
     if (plan.n_items <= 0) return;
     const LatentPool& P = a.pool;
     const double positions = 32.0 * plan.n_pairs, width = (double)a.H * (a.dim_ld + a.vdim_ld);
     if (!formed) {
         const ExpandArgs e = latent_expand_args(a, plan, rt().num_cus);
-        ProfScope ps(PC_LATENT_EXPAND, width * P.rank_ld * 2.0 + positions * P.rank_ld * 2.0 + positions * width * 2.0, 2.0 * positions * width * P.rank_ld);
+        double bytes, flops;
+        latent_expand_work(a, plan, &bytes, &flops);
+        ProfScope ps(PC_LATENT_EXPAND, bytes, flops);
         const dim3 grid(expand_cols(e), cdiv(plan.n_pairs, e.per));
         if (e.chunks <= 8) launch_expand<8>(e, grid);
         else launch_expand<16>(e, grid);

@@ -29,6 +29,10 @@ RoutePlan route_plan(int* mem, int T, int E, int top, int pad);
 // z: [T][ldz] router logits in columns 0 .. E-1; the `top` largest (the first of equals) are chosen
 void launch_route(const RoutePlan& r, const float* z, int ldz, bool chosen = false);   // chosen: sorting is left
 
+// bytes for kernel timing: of the choice, and of the sorting as a launch of its own
+inline double choice_bytes(const RoutePlan& r) { return (double)r.T * (r.E * 4.0 + r.top * 20.0); }
+inline double sort_bytes(const RoutePlan& r) { return (double)r.T * r.top * 28.0; }
+
 // Work that needs a fraction of the chip, beside the shared expert's products on the CUs those leave idle: the router beside the first,
 // the choice beside the second (launch_gemm_b16); with hundreds of tokens the choice with the router, the sorting alone beside the second.
 struct MoeRider {

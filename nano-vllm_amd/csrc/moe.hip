@@ -60,18 +60,17 @@ __global__ __launch_bounds__(1024) void k_route_sort(RoutePlan r, const float* _
 void launch_route(const RoutePlan& r, const float* z, int ldz, bool chosen) {
     if (r.T <= 0) return;
     const size_t lds = ((size_t)3 * r.E + 1) * sizeof(int);
-    const double bytes = (double)r.T * (r.E * 4.0 + r.top * 20.0);
     const size_t lds_one = route_sort_lds(r.T, r.E, r.top);
     if (!chosen && r.T <= ROUTE_ONE && lds_one <= 64 * 1024) {
-        ProfScope ps(PC_ROUTE, bytes, 0);
+        ProfScope ps(PC_ROUTE, choice_bytes(r), 0);
         NVLLM_LAUNCH((k_route_sort<true>), dim3(1), dim3(1024), lds_one, r, z, ldz);
         return;
     }
     if (!chosen) {
-        ProfScope ps(PC_ROUTE, bytes, 0);
+        ProfScope ps(PC_ROUTE, choice_bytes(r), 0);
         NVLLM_LAUNCH(k_route, dim3(cdiv(r.T, 4)), dim3(256), 0, r, z, ldz);
     }
-    ProfScope ps(PC_ROUTE, (double)r.T * r.top * 28.0, 0);
+    ProfScope ps(PC_ROUTE, sort_bytes(r), 0);
     NVLLM_LAUNCH((k_route_sort<false>), dim3(1), dim3(1024), lds, r, z, ldz);
 }
 

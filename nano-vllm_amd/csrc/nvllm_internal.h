@@ -223,6 +223,7 @@ struct ProfScope {  // names the class of, and attaches timing events to, the ON
     ProfScope(int cls, double bytes, double flops);
     ~ProfScope();
     void drop();   // nothing was launched inside after all
+    void add(double bytes, double flops);   // of work that rides in the launch
     int slot;
 };
 

@@ -187,6 +187,11 @@ void ProfScope::drop() {
     slot = -1;
     g_cur_start = g_cur_stop = nullptr;
 }
+void ProfScope::add(double bytes, double flops) {
+    if (slot < 0) return;
+    g_prof_pending[slot].bytes += bytes;
+    g_prof_pending[slot].flops += flops;
+}
 ProfScope::~ProfScope() {
     if (slot < 0) return;
     g_cur_start = g_cur_stop = nullptr;
