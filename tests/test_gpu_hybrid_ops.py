@@ -317,7 +317,9 @@ def test_capped_scores_far_outside_the_cap(hip, elem):
 
 # ------------------------------------------------------------------ linear attention with decay
 @BOTH
-@pytest.mark.parametrize("H,dim,vdim", [(2, 32, 32), (3, 20, 26), (2, 64, 64), (1, 96, 48), (2, 128, 128), (1, 40, 200), (1, 256, 70), (2, 300, 16), (1, 130, 33)])
+@pytest.mark.parametrize("H,dim,vdim", [(2, 32, 32), (3, 20, 26), (2, 64, 64), (1, 96, 48), (2, 128, 128), (1, 40, 200), (1, 256, 70), (2, 300, 16), (1, 130, 33),
+                                        # fp32 portions in registers: four, eight and sixteen dims a thread by 8, 16, 32 and 64 value columns
+                                        (2, 128, 32), (1, 256, 32), (2, 128, 64), (1, 256, 64), (1, 64, 128), (1, 32, 256), (1, 64, 256)])
 def test_linear_attention(hip, H, dim, vdim, elem):
     """Portions of many sizes beside single tokens; results and the 32-bit state against the plain recurrence; slots used before."""
     r = rng(dim * vdim)

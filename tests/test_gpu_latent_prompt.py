@@ -12,6 +12,7 @@ import pytest
 from nvllm_amd import synth
 from tests import latent_oracle as O
 from tests import latent_util as U
+from tests.test_gpu_latent_order import flops_of
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 M = synth.latent_mixer
@@ -74,17 +75,24 @@ def test_portions_agree_with_attention_over_latents(tmp_path, name):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("heads,rank", [(32, 512), (24, 256), (17, 100), (32, 480), (16, 512)])
-def test_forming_beside_tokens_that_come_alone(hip, tmp_path, heads, rank):
+@pytest.mark.parametrize("heads,rank,length,formings", [(32, 512, 600, 4), (24, 256, 600, 4), (17, 100, 1300, 2), (32, 480, 600, 8), (16, 512, 600, 8)])
+def test_forming_beside_tokens_that_come_alone(hip, tmp_path, heads, rank, length, formings):
     """Items of 32 columns (17 to 32 heads) of the widest row and of one with up to eight tiles share a launch with the forming of keys and values; others
-    do not.  One, three and twenty such tokens (few and many workgroups) beside long portions."""
+    do not.  One, three and twenty such tokens (few and, for the last pass's portion, too many workgroups) beside long portions."""
     cfg = synth.latent_config(64, 130, [(M(heads, 64, 64, 64, rank, 32), 40)] * 2, streams=2)
     path, cfg, w = U.model(tmp_path, "beside", seed=heads, cfg=cfg)
     n = 22
-    seqs = {q: U.tokens(600 if q < 2 else 40, 130, 70 + q) for q in range(n)}
-    plan = [[(q, 30) for q in range(2, n)], [(0, 200), (5, 1)], [(3, 1), (0, 200), (1, 300), (4, 1), (6, 1)], [(q, 1) for q in range(2, 12)] + [(0, 190)] + [(q, 1) for q in range(12, n)]]
-    eng = U.engine(hip, path, False, slots=n)
-    got = U.feed_all(eng, plan, seqs)
+    seqs = {q: U.tokens(length + 190 if q == 0 else length if q == 1 else 40, 130, 70 + q) for q in range(n)}
+    plan = [[(q, 30) for q in range(2, n)], [(0, length), (5, 1)], [(3, 1), (1, length), (4, 1), (6, 1)], [(q, 1) for q in range(2, 12)] + [(0, 190)] + [(q, 1) for q in range(12, n)]]
+    eng = U.engine(hip, path, False, slots=n, tokens=4096)
+    hip.nvllm_prof_reset()
+    hip.nvllm_prof_enable(1)
+    try:
+        got = U.feed_all(eng, plan, seqs)
+    finally:
+        hip.nvllm_prof_enable(0)
+    assert flops_of(hip, "latent_expand")[0] == formings   # launches of its own, two layers a pass: the first has no single tokens
+    hip.nvllm_prof_reset()
     eng.close()
     for q, rows in got.items():
         assert U.error(rows, O.forward(cfg, w, seqs[q][:len(rows)])) < U.limit(False), q

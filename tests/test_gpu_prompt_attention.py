@@ -2,11 +2,17 @@
 
 Portions begin and end inside runs, blocks of 64 keys and halves of them; single tokens and short ends ride in the same launch.
 """
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 
-from tests import util
+from nvllm_amd import synth
+from tests import test_gpu_wide, util
 
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 pytestmark = pytest.mark.gpu
 
 
@@ -48,3 +54,25 @@ def test_portions(hip, hd, heads, kv_heads, scale):
             # scores, weights and sums carry a few units in the last place, scores of some hundreds that many times more
             np.testing.assert_allclose(got[at:at + n, h * hd:(h + 1) * hd], w, atol=4e-6 * max(1.0, scale), rtol=0, err_msg="portion %d head %d" % (i, h))
         at += n
+
+
+@pytest.mark.parametrize("hd,heads,kv_heads", [(32, 8, 8), (32, 8, 1), (64, 6, 3), (96, 4, 4), (96, 4, 1), (128, 4, 4), (128, 4, 2)])
+def test_passes_store_activation_tiles(oracle, tmp_path, hd, heads, kv_heads):
+    """Whole passes, whose next projection reads the results as tiles of two planes: against the oracle, and against the attention of 16 columns (the
+    environment, read once per process, lets one item be enough, or none)."""
+    path = str(tmp_path / "m.bin")
+    synth.write_model(path, synth.ModelShape(dim=hd * heads, hidden_dim=416, n_layers=2, n_heads=heads, n_kv_heads=kv_heads, vocab_size=700, max_seq_len=512), seed=hd)
+    want = util.run_engine(oracle, path, test_gpu_wide.prompts(), **test_gpu_wide.PASSES)["steps"]
+    got = []
+    for items in ("1", "0"):
+        dst = str(tmp_path / ("got%s.npz" % items))
+        r = subprocess.run([sys.executable, "-c", test_gpu_wide.CHILD, path, dst, "2"], capture_output=True, text=True, timeout=110,
+                           env=dict(os.environ, PYTHONPATH=ROOT + os.pathsep + os.environ.get("PYTHONPATH", ""), NVLLM_ATTN_LONG=items))
+        assert r.returncode == 0, r.stderr[-2000:]
+        got.append(np.load(dst))
+    apart = 0.0
+    for i, o in enumerate(want):
+        np.testing.assert_array_equal(got[0][f"sampled{i}"], o["sampled"])
+        assert np.abs(got[0][f"logits{i}"] - o["logits"]).max() < 2e-3   # the bar of the forward pass over an fp16 pool
+        apart = max(apart, float(np.abs(got[0][f"logits{i}"] - got[1][f"logits{i}"]).max()))
+    assert 0 < apart < 2e-4   # (other sums, so some bit differs; the bar of the pass over an fp32 pool)
