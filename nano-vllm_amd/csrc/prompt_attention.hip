@@ -6,13 +6,14 @@
 // a wave 32 of them against half of each block of 64 keys, in v_mfma_f32_16x16x32_f16 (two 16-dim pieces of a page's keys, or
 // two pages' values, are one operand as they lie).  Blocks travel to LDS by direct copies, RING - 1 ahead, once per workgroup.  A lane
 // keeps its column's sums and results (values are the first operand), so in most blocks nothing crosses lanes; the two waves
-// of a column group meet once at the end.  Three portions of 512 tokens behind 512, 32 heads on 4 of 64: 62 -> 27.6 us a layer, 9.7 GFLOP (twice that in
+// of a column group meet once at the end.  Three portions of 512 tokens behind 512, 32 heads on 4 of 64: 61.3 -> 28.1 us a layer, 9.7 GFLOP (twice that in
 // the matrix cores for the planes).  Bound: issue of about 95 vector instructions, 16 of them exponentials, beside 32 products per 32 keys
 // and 32 columns; the depth of the ring and a fourth workgroup a CU change nothing.  Of the way there: 37 as first written; references that
 // rise at every new maximum, and maxima over all lanes for it, cost 5; walks of three workgroups of a CU that are all long or all short 4 (stage_step).
-// Error against 64 bits (2-norm of the results, queries of size 1, 4 and 30; k_paged_attn16 in brackets, 1e-7): heads of 64 1.42, 3.48, 7.80 (1.47, 3.61,
-// 8.01), of 32 1.34, 3.10, 6.26 (1.46, 3.59, 7.55), of 128 1.55, 3.54, 7.51 (1.52, 3.94, 8.30); with all products of a score in one chain and one set of
-// sums 1.60, 3.87, 8.70 at 64.
+// Error against 64 bits (2-norm of the results, queries of size 1, 4 and 30; k_paged_attn16 in brackets, 1e-7): heads of 64 1.43, 3.48, 7.73 (1.47, 3.61,
+// 8.01), of 32 1.35, 3.09, 6.29 (1.46, 3.58, 7.50), of 96 1.50, 3.43, 7.42 (1.56, 3.71, 8.07), of 128 1.39, 3.41, 7.56 (1.53, 3.93, 8.31); with both planes of a
+// block's weights in one chain of sums 1.54 at 128 (which took 30.1 us for 16 heads where it now takes 31.6), with all products of a score in one chain
+// too 1.60, 3.87, 8.70 at 64.
 #include "prompt_attention.h"
 
 #include "gemm_common.h"
@@ -117,7 +118,8 @@ __device__ __forceinline__ void prompt_item(const PromptAttnArgs& p, unsigned wi
     for (int j = 0; j < 2; j++)
 #pragma unroll
         for (int c = 0; c < HD / 32; c++) asm volatile("" : "+v"(qh[j][c]), "+v"(ql[j][c]));   // here, not in the loop, whose only loads are the copies
-    // results; those of the weights' lo plane apart where registers allow, which halves the roundings to the size of the sums
+    // results; those of the weights' lo plane apart where registers allow, else a block's of both planes added to the sums as one: either way one
+    // rounding to the size of the sums per 32 keys
     constexpr int SUMS = HD < 128 ? 2 : 1;
     pf4_t acc[SUMS][2][NC];
 #pragma unroll
@@ -245,14 +247,30 @@ __device__ __forceinline__ void prompt_item(const PromptAttnArgs& p, unsigned wi
             ph8_t val[2];
 #pragma unroll
             for (int i = 0; i < 2; i++) val[i] = pair(v_at[n + i], W::PAGE);
+            if constexpr (SUMS == 2) {
 #pragma unroll
-            for (int i = 0; i < 2; i++)
+                for (int i = 0; i < 2; i++)
 #pragma unroll
-                for (int j = 0; j < 2; j++) acc[0][j][n + i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(val[i], ph[j], acc[0][j][n + i], 0, 0, 0);
+                    for (int j = 0; j < 2; j++) acc[0][j][n + i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(val[i], ph[j], acc[0][j][n + i], 0, 0, 0);
 #pragma unroll
-            for (int i = 0; i < 2; i++)
+                for (int i = 0; i < 2; i++)
 #pragma unroll
-                for (int j = 0; j < 2; j++) acc[SUMS - 1][j][n + i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(val[i], pl[j], acc[SUMS - 1][j][n + i], 0, 0, 0);
+                    for (int j = 0; j < 2; j++) acc[1][j][n + i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(val[i], pl[j], acc[1][j][n + i], 0, 0, 0);
+            } else {
+                pf4_t block[2][2];
+#pragma unroll
+                for (int i = 0; i < 2; i++)
+#pragma unroll
+                    for (int j = 0; j < 2; j++) block[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(val[i], pl[j], pf4_t{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+#pragma unroll
+                for (int i = 0; i < 2; i++)
+#pragma unroll
+                    for (int j = 0; j < 2; j++) block[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(val[i], ph[j], block[i][j], 0, 0, 0);
+#pragma unroll
+                for (int i = 0; i < 2; i++)
+#pragma unroll
+                    for (int j = 0; j < 2; j++) acc[0][j][n + i] += block[i][j];
+            }
         }
     }
     // the two waves of 32 columns: each leaves the other's 16 and finishes its own (group j = part)

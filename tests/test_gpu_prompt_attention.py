@@ -76,3 +76,52 @@ def test_passes_store_activation_tiles(oracle, tmp_path, hd, heads, kv_heads):
         assert np.abs(got[0][f"logits{i}"] - o["logits"]).max() < 2e-3   # the bar of the forward pass over an fp16 pool
         apart = max(apart, float(np.abs(got[0][f"logits{i}"] - got[1][f"logits{i}"]).max()))
     assert 0 < apart < 2e-4   # (other sums, so some bit differs; the bar of the pass over an fp32 pool)
+
+
+ERROR_CHILD = """
+import sys
+from nvllm_amd import capi
+from tests import test_gpu_prompt_attention as T
+lib = capi.load_hip()
+lib.init_ops()
+print("error", T.error(lib, *map(int, sys.argv[1:])))
+"""
+
+
+def error(hip, hd, heads, kv_heads):
+    """2-norm of the results' distance from float64 over that of the results; queries of size 1, where the sums' roundings are most of it."""
+    parts, off, size = [(512, 300), (0, 300)], 0.0, 0.0
+    hip.nvllm_set_kv_elem_bytes(2)
+    for seed in range(3):
+        r = np.random.default_rng(seed)
+        pool = util.Pool(hip, 16, sum(-(-(a + n) // 16) for a, n in parts), 1, kv_heads, hd)
+        rows = [tuple(r.standard_normal((a + n, kv_heads * hd)).astype(np.float32) for _ in range(2)) for a, n in parts]
+        q = r.standard_normal((sum(n for _, n in parts), heads * hd)).astype(np.float32)
+        pos, seq = [], []
+        for i, (a, n) in enumerate(parts):
+            pool.new_table(-(-(a + n) // 16))
+            pool.grow(i, a + n)
+            util.op_kv_write_batch(hip, pool, rows[i][0], rows[i][1], 0, list(range(a + n)), [i] * (a + n), kv_heads, hd)
+            pos += list(range(a, a + n))
+            seq += [i] * n
+        got = util.op_paged_attention_batch(hip, pool, q, 0, pos, seq, max(pos) + 1, heads, kv_heads, hd)
+        pool.close()
+        at = 0
+        for i, (a, n) in enumerate(parts):
+            k, v = (x.astype(np.float16).astype(np.float64).reshape(-1, kv_heads, hd) for x in rows[i])
+            for h in range(heads):
+                w = want(q[at:at + n, h * hd:(h + 1) * hd], k[:, h * kv_heads // heads], v[:, h * kv_heads // heads], a)
+                off, size = off + ((got[at:at + n, h * hd:(h + 1) * hd] - w) ** 2).sum(), size + (w ** 2).sum()
+            at += n
+    return float(np.sqrt(off / size))
+
+
+@pytest.mark.parametrize("hd,heads,kv_heads", [(32, 8, 2), (64, 8, 2), (96, 8, 2), (128, 8, 2), (128, 8, 8)])
+def test_no_further_from_64_bits_than_sixteen_columns(hd, heads, kv_heads):
+    got = []
+    for items in ("1", "0"):
+        r = subprocess.run([sys.executable, "-c", ERROR_CHILD, str(hd), str(heads), str(kv_heads)], capture_output=True, text=True, timeout=110,
+                           env=dict(os.environ, PYTHONPATH=ROOT + os.pathsep + os.environ.get("PYTHONPATH", ""), NVLLM_ATTN_LONG=items))
+        assert r.returncode == 0, r.stderr[-2000:]
+        got.append(float(r.stdout.split()[-1]))
+    assert got[0] < got[1], got
