@@ -487,9 +487,9 @@ LongRuns attn_long_runs(const KvPoolView& pool, int H, int KVH, int hd) {
     const int ct = attn_tokens_per_item(H, KVH), ng = H / (16 / ct);
     // From nine sixteenths of a workgroup for each CU on: with fewer a workgroup's walk, 0.7 (1.1) us per 64 keys of heads of 64 (128), is longer
     // than the four times as many items that split theirs over four waves take.  us a layer, k_paged_attn16 and prompts, 32 heads on 4 of 64
-    // (16 on 4 of 128): three portions of 512 behind 512 60.4 and 27.6 (64.6 and 30.0), first portions 35.3 and 15.5 (43.2 and 18.7); one of
-    // 512 22.6 and 16.7 (128 items: 23.4 and 23.3), behind 1,500 38.5 and 28.6 (37.8 and 40.2); one of 256 there, 128 items, 21.5 and 25.0; three of
-    // 200, 300 items (152), 43.5 and 30.3 (51.0 and 35.6).  Portions of less than half a run's tokens stay as they were
+    // (16 on 4 of 128): three portions of 512 behind 512 61.3 and 28.1 (66.8 and 32.4), first portions 36.2 and 15.8 (44.2 and 19.3); one of
+    // 512 22.8 and 16.3 (128 items: 23.6 and 24.6), behind 1,500 38.7 and 27.9 (38.3 and 42.8); one of 256 there, 128 items, 21.1 and 24.6; three of
+    // 200, 300 items (156), 43.6 and 30.1 (52.4 and 38.1).  Portions of less than half a run's tokens stay as they were
     return {4 * ct, 2 * ct, cdiv(env > 0 ? env : rt().num_cus * 9 / 16, ng), std::max(1, rt().num_cus / ng)};
 }
 
@@ -498,7 +498,9 @@ LongRuns attn_long_runs(const KvPoolView& pool, int H, int KVH, int hd) {
 // where slices leave parts) and rows: 8 heads of 64 (two trips: 512 keys), 1 row of 220 and 500 9.0 and 4.5, 10.0 and 6.3, of 1,000, four trips, 10.0 and 12.6;
 // 16 rows 9.6 and 5.7, 12.6 and 8.2, 17.9 and 17.4; 32 rows (256 items) of 120, 220, 500, 1,000 7.6 and 6.3, 11.2 and 7.4, 16.7 and 12.8, 26.0 and 22.4; 64
 // 9.9 and 7.9 .. 43.5 and 40.7.  6 of 48, 120 and 240 keys 6.3 and 4.6, 8.6 and 5.0.  16 of 128, 1 and 8 rows of 100 7.6 and 5.4, 8.4 and 6.0, of 1,000
-// 11.7 and 22.9; 32 on 16 of 64, 100 and 300 6.4 and 5.6, 10.8 and 8.5.  More items: 64 of 32, 32 rows of 100 13.1 and 20.4
+// 11.7 and 22.9; 32 on 16 of 64, 100 and 300 6.4 and 5.6, 10.8 and 8.5.  More items: 64 of 32, 32 rows of 100 13.1 and 20.4.  Wide heads that fill the
+// CUs, up to eight trips, operators over rows that come from HBM: 16 of 128, 16 rows (256 items) of 200, 400, 700, 1,000 20.8 and 18.0, 29.8 and 26.5, 40.1
+// and 38.4, 52.1 and 53.0, 24 rows 31.6 and 22.6 .. 84.9 and 75.7, 32 29.0 and 26.4 .. 94.0 and 94.7; of 80 16 rows 18.6 and 17.0 .. 40.5 and 40.5
 static bool rows_alone(const AttnArgs& a, int pages) {
     static const int env = getenv("NVLLM_ATTN_ROWS") ? atoi(getenv("NVLLM_ATTN_ROWS")) : -1;   // 0: none; else up to that many pages
     const int group = a.H / a.KVH, cus = rt().num_cus;

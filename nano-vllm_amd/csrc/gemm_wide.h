@@ -204,7 +204,7 @@ __global__ __launch_bounds__(256 * WT, 1) void k_gemm_wide(GemmArgs p, int tiles
 
 // Feature tiles of a panel: those with which the tiles that an XCD works on at a time, a contiguous range of its CUs' number, bring the
 // fewest bytes into its L2 (`w` KiB a feature tile and step, `a` a token tile).  One, which is token tiles fastest, has all activations enter every
-// L2: TinyLlama-1.1B's w_down and wo, 200 tiles of 64 tokens, 55.9 us on average, in panels of four 53.9; its gate/up 123.8 and 122.4; with one plane of
+// L2: TinyLlama-1.1B's w_down and wo, 200 tiles of 64 tokens, 55.7 us on average, in panels of three (which this picks) 53.2, of four 52.9; its gate/up 125.5 and 124.1; with one plane of
 // activations no difference.
 inline int wide_panel(int tiles_n, int tiles_t, int w, int a) {
     const int range = std::min(cdiv(tiles_n * tiles_t, 8), rt().num_cus / 8);

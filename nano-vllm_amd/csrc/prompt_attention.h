@@ -5,7 +5,7 @@
 
 namespace nvllm {
 
-// `long_runs` int4 (first token, token count, last position, table offset), at most prompt_attn_tokens() tokens each, one launch with
+// `long_runs` int4 (first token, token count, last position, table offset), at most attn_long_runs().tokens tokens each, one launch with
 // the items of k.runs (one key slice each).
 struct PromptAttnArgs {
     AttnKArgs k;
