@@ -365,7 +365,7 @@ bool launch_gemm_f32(const F32Gemm& g, int prof_cls) {
     // per cycle of the mix of weights and activations) and to multiply (8 cycles per product and quad of k on four SIMDs):
     // larger tiles fetch less per product, smaller ones reach more CUs.  K = 512 at 301 tokens: 2 x 2 blocks of a 512-wide
     // output 8 us, 1 x 1 10 us; 2 x 4 of a 1,536-wide one 13.6 us against 17.0 in 2 x 2.  Three token blocks where two and four fill
-    // their last round worse: 2,816 features x 1,024 k at 80 tokens (176 tiles of 2 x 3; 440 of 1 x 2) 19.9 -> 15.5, 1,024 x 1,024 at
+    // their last round worse: 2,816 features x 1,024 k at 80 tokens (176 tiles of 2 x 3; 880 of 1 x 1) 19.9 -> 15.5, 1,024 x 1,024 at
     // 300 15.9 -> 14.4, 864 x 288 at 301 11.6 -> 7.9; pairs 2 x 768 x 288 at 200 10.9 -> 7.9, 2 x 2,816 x 1,024 at 170 38.0 -> 32.3.  (1 x 3 of a
     // plain one fetches as much per CU as 2 x 2: 13.6 -> 13.1 at best.)  With a short K in one round only: a second one has too few steps to hide its
     // start (K = 288, pairs of 768 at 690 tokens 18.1 -> 20.3, 864 features at 600 11.0 -> 12.7).

@@ -696,6 +696,8 @@ static void launch_attn_expand(const LatentKArgs& k, const ExpandArgs& e, int un
 }
 // Items of 32 columns (eight waves, as the forming has) on a quarter of the CUs at most, the forming on the others: five tokens at 1,050
 // beside 1,024 behind 1,024 positions, 32 heads of 512: 45 workgroups of 10.8 us and 256 of 14.4 one after the other, together 16.8 (253).
+// Up to 16 heads have items of 16 columns and four waves; rows of 11 to 17 tiles would take two more instances of the largest kernel, for widths
+// that no configuration has.  Neither was measured beside the forming: two launches, as without a rider.
 static bool attn_with_expand(const LatentKArgs& k, const LatentAttn& a, long units, int columns, ProfScope& ps) {
     if (!a.expand || columns != 32 || units * 4 > rt().num_cus) return false;
     const ExpandArgs e = latent_expand_args(*a.expand->prompt, *a.expand->plan, rt().num_cus - (int)units);
