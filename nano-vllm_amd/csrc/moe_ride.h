@@ -154,10 +154,10 @@ __device__ __forceinline__ void router_ride(const GemmArgs& p, int wave, int lan
 
 // Riders beside `tiles` workgroups, of which a CU holds one: on free CUs only, and only what is done about when the tiles are: up to two passes of the
 // router over a workgroup's blocks, of which a wave chooses for 16 tokens, and up to 4,096 choices to sort (256 threads; the launch of its own has 1,024).
-// us: a pass over the blocks, a step of four tokens' choices, the tiles at 900 TFLOP/s; and what the launches of router, choice and sorting take that are
-// saved.  Both ways, those launches and both products (Kb 64, 5,632 features, 31 and 32, 9): 2 of 16 experts, 400 and 1,029 tokens 31 and 50, 57 and 68;
-// 4 of 31 at 32 400, 1,029 (two trips of a rider), 1,500 33 and 41, 65 and 56, 54 and 63; 8 of 63 256, 700, 1,500 55 and 91, 71 and 68, 99 and 103; at 32
-// 46 and 85, 63 and 53, 80 and 76; of 1,536 features at 9 39 and 73, 50 and 35, 61 and 50.
+// In us: a pass over the blocks, a step of four tokens' choices, the tiles at 900 TFLOP/s; and what the launches of router, choice and sorting take that
+// are saved.  Those launches and both products together, riding and apart, pairs of 2,816 features over 2,048 k: 2 of 16 experts, 400 and 1,029 tokens 31
+// and 50, 57 and 68; 8 of 63, 256, 700, 1,500 tokens 55 and 91, 71 and 68, 99 and 103; over 1,024 k 4 of 31, 400, 1,029 (two trips of a rider), 1,500
+// tokens 33 and 41, 65 and 56, 54 and 63; 8 of 63 256, 700, 1,500 46 and 85, 63 and 53, 80 and 76; of 768 features over 288 k 39 and 73, 50 and 35, 61 and 50.
 inline int route_groups(const GemmArgs& a, int tiles) {
     const RoutePlan& r = a.route.plan;
     const int spare = rt().num_cus - tiles;

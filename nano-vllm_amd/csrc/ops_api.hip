@@ -490,6 +490,8 @@ void multi_head_attention(float* out, float* q, float* key_cache, float* value_c
     a.long_runs = s.d_long;
     a.n_long = s.n_long;
     a.kv_positions = s.kv_positions;
+    a.kv_rows = s.kv_rows;
+    a.qk_pairs = s.qk_pairs;
     launch_paged_attention(a);
 }
 
@@ -522,6 +524,8 @@ void paged_attention(float* out, float* q, KVCacheManager* mgr, BlockTable* bloc
     a.long_runs = s.d_long;
     a.n_long = s.n_long;
     a.kv_positions = s.kv_positions;
+    a.kv_rows = s.kv_rows;
+    a.qk_pairs = s.qk_pairs;
     launch_paged_attention(a);
 }
 
@@ -554,6 +558,8 @@ void paged_attention_batch(float* out, float* q, KVCacheManager* mgr, BlockTable
     a.long_runs = s.d_long;
     a.n_long = s.n_long;
     a.kv_positions = s.kv_positions;
+    a.kv_rows = s.kv_rows;
+    a.qk_pairs = s.qk_pairs;
     launch_paged_attention(a);
 }
 

@@ -3,10 +3,11 @@ and a choice and of the experts they can reach, not of the padding the launch ha
 beside that launch's own."""
 import ctypes as C
 
+import numpy as np
 import pytest
 
 from nvllm_amd import synth
-from tests import hybrid_util, latent_util
+from tests import hybrid_util, latent_util, util
 from tests.test_gpu_latent_ops import Dev, rng
 
 pytestmark = pytest.mark.gpu
@@ -85,3 +86,26 @@ def test_forming_beside_single_tokens(hip, tmp_path):
     assert "latent_expand" not in got[0] and got[1]["latent_expand"][0] == 2
     for i in (1, 2):
         assert got[0]["latent_attn_tok"][i] == got[1]["latent_attn_tok"][i] + got[1]["latent_expand"][i]
+
+
+@pytest.mark.parametrize("first,tokens", [(40, 1), (40, 30), (100, 700)])   # one row, a portion by 16 columns, one by 64
+def test_paged_attention_operator(hip, first, tokens):
+    heads, kv_heads, hd = 16, 4, 64
+    hip.nvllm_set_kv_elem_bytes(2)
+    try:
+        pool = util.Pool(hip, 16, -(-(first + tokens) // 16), 1, kv_heads, hd)
+        pool.new_table(-(-(first + tokens) // 16))
+        pool.grow(0, first + tokens)
+        rows = rng(1).standard_normal((first + tokens, kv_heads * hd)).astype(np.float32)
+        util.op_kv_write_batch(hip, pool, rows, rows, 0, list(range(first + tokens)), [0] * (first + tokens), kv_heads, hd)
+        hip.nvllm_prof_reset()
+        hip.nvllm_prof_enable(1)
+        util.op_paged_attention_batch(hip, pool, rng(2).standard_normal((tokens, heads * hd)).astype(np.float32), 0, list(range(first, first + tokens)), [0] * tokens,
+                                      first + tokens, heads, kv_heads, hd)
+    finally:
+        hip.nvllm_prof_enable(0)
+        hip.nvllm_set_kv_elem_bytes(4)
+    got = figures(hip)
+    pool.close()
+    pairs = sum(range(first + 1, first + tokens + 1))
+    assert got["attn"] == (1, (first + tokens) * 2.0 * kv_heads * hd * 2 + tokens * heads * hd * 8.0, 4.0 * pairs * heads * hd)
