@@ -12,7 +12,12 @@
 //
 // What bounds it: few tokens -- bytes of W, and below ~10 MB the launch itself; hundreds of tokens -- the fp32 matrix
 // rate (157 TFLOP/s).  These products occupy the vector unit: an addition of four registers between them costs half of one.
+// A launch of few tokens is a chain of trips to memory (a dependent launch that reads and writes one value: 1.6 us), so every trip
+// that depends on nothing starts at once: the arguments' lines, the tile's segment without a loop over them, and positions, cache rows,
+// angles and residual values with the first steps instead of behind the last.  us a pass before and with that: stories15M, one row
+// (34 launches) 213 -> 195; stories42M, 301 tokens 583 -> 571; Simivik-0.4B, 80 tokens (132 launches) 1,660 -> 1,603.
 #include <algorithm>
+#include <climits>
 
 #include "gemm_common.h"
 #include "gemm_f32_tail.h"
@@ -30,6 +35,7 @@ __global__ __launch_bounds__(KS * 64, f32_occupancy((PAIR ? 2 : 1) * NB * TB, NO
     constexpr int RING = NT * TB == 1 ? (NORM ? 3 : 4) : 2;
     constexpr int ITEMS = NB * TB * 64;   // results, four features of a token each
     constexpr int FPT = (ITEMS + KS * 64 - 1) / (KS * 64);
+    request_arguments<sizeof(F32Gemm)>();
     extern __shared__ __attribute__((aligned(16))) unsigned char lds_f32[];
     f4_t(*s_red)[NT * TB][64] = reinterpret_cast<f4_t(*)[NT * TB][64]>(lds_f32);                     // [wave]
     float(*s_ss)[TB * 16] = reinterpret_cast<float(*)[TB * 16]>(lds_f32 + KS * NT * TB * 1024);   // NORM: [wave]
@@ -43,9 +49,7 @@ __global__ __launch_bounds__(KS * 64, f32_occupancy((PAIR ? 2 : 1) * NB * TB, NO
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int x = lane & 15, g = lane >> 4;
     const int tile = (int)blockIdx.x;
-    int s = 0;
-    while (s + 1 < p.n_segs && tile >= p.seg[s + 1].first) s++;
-    const F32Segment& sg = p.seg[s];
+    const F32Segment& sg = p.seg[f32_segment(p, tile)];
     const int nb0 = (tile - sg.first) * NB, tb0 = (int)blockIdx.y * TB;
     const int K = p.K, T = p.T, N = sg.N;
     const float *W = sg.W, *W2 = sg.W2;
@@ -65,10 +69,43 @@ __global__ __launch_bounds__(KS * 64, f32_occupancy((PAIR ? 2 : 1) * NB * TB, NO
     const float* ap[TB];
 #pragma unroll
     for (int j = 0; j < TB; j++) {
-        const int t = min((tb0 + j) * 16 + x, T - 1);
-        ap[j] = p.in + (size_t)(p.in_rows ? p.in_rows[t] : t) * K + 4 * g;
+        int t = min((tb0 + j) * 16 + x, T - 1);
+        if (p.in_rows) {
+            t = p.in_rows[t];
+            asm volatile("" ::"v"(t));   // (waited for here, and not where launches without these rows meet)
+        }
+        ap[j] = p.in + (size_t)t * K + 4 * g;
     }
     const float* gp = NORM ? p.gain + 4 * g : nullptr;
+
+    // What the epilogue needs beside the sums travels with the first steps, and angles behind their positions; where the registers
+    // are full, with the last ones
+    constexpr bool EARLY = PAIR || NT * TB < 4 || f32_occupancy(NT * TB, NORM) < 4;
+    const bool turns = !PAIR && (sg.kind == F32Out::ROPE_Q || sg.kind == F32Out::ROPE_K), adds = !PAIR && sg.kind == F32Out::ADD;
+    int at[FPT], row[FPT];
+    f4_t side[FPT];   // angles, or what is added to
+    auto item = [&](int q, int& t, int& n) {
+        const int e = min((int)threadIdx.x + q * KS * 64, ITEMS - 1), l = e & 63;
+        t = min((tb0 + (e >> 6) % TB) * 16 + (l & 15), T - 1);
+        n = (nb0 + (e >> 6) / TB) * 16 + 4 * (l >> 4);
+    };
+#pragma unroll
+    for (int q = 0; q < FPT; q++) {
+        int t, n;
+        item(q, t, n);
+        at[q] = turns ? p.pos[t] : 0;
+    }
+    auto request_side = [&] {
+#pragma unroll
+        for (int q = 0; q < FPT; q++) {
+            int t, n;
+            item(q, t, n);
+            row[q] = PAIR ? -1 : f32_row(p, sg, t);
+            if (turns) side[q] = *reinterpret_cast<const f4_t*>(p.rope + (size_t)at[q] * (p.hd >> 1) + ((n % p.hd) >> 1));
+            else if (adds) side[q] = f32_old(sg, t, n);
+            else side[q] = f4_t{0.f, 0.f, 0.f, 0.f};
+        }
+    };
 
     f4_t w[RING][NT][2], a[RING][TB][2], gv[RING][NORM ? 2 : 1];
     const f4_t zero = {0.f, 0.f, 0.f, 0.f};
@@ -158,12 +195,14 @@ __global__ __launch_bounds__(KS * 64, f32_occupancy((PAIR ? 2 : 1) * NB * TB, NO
 #pragma unroll
         for (int r = 0; r + 1 < RING; r++)
             if (r < mine) load(r, r);
+        if constexpr (EARLY) request_side();
 #pragma unroll
         for (int r = 0; r + 1 < RING; r++)
             if (r < mine) multiply(r);
     } else {
 #pragma unroll
         for (int r = 0; r < RING; r++) load(r, r);
+        if constexpr (EARLY) request_side();
         int i0 = 0;
         for (; i0 + 2 * RING <= mine; i0 += RING) {
 #pragma unroll
@@ -181,6 +220,7 @@ __global__ __launch_bounds__(KS * 64, f32_occupancy((PAIR ? 2 : 1) * NB * TB, NO
         for (int r = 0; r < RING; r++)
             if (i0 + r + RING < mine) multiply(r);
     }
+    if constexpr (!EARLY) request_side();
     if (whole * F32_STEP < K && whole % KS == wave) {   // the rest of K (K % 4 == 0: a lane's four are in or out together)
         const int k = whole * F32_STEP;
 #pragma unroll
@@ -208,7 +248,7 @@ __global__ __launch_bounds__(KS * 64, f32_occupancy((PAIR ? 2 : 1) * NB * TB, NO
             ss[j] += __shfl_xor(ss[j], 32, 64);
         }
     }
-    auto finish = [&](int t, int n, f4_t y, f4_t u, float sum, f4_t old) {
+    auto finish = [&](int t, int n, f4_t y, f4_t u, float sum, f4_t side, int row) {
         if (t >= T || n >= N) return;
         float scale = NORM ? rinv_of(sum) : 1.f;
         if (p.row_weight) scale *= p.row_weight[t];
@@ -216,16 +256,8 @@ __global__ __launch_bounds__(KS * 64, f32_occupancy((PAIR ? 2 : 1) * NB * TB, NO
             y *= scale;
             if constexpr (PAIR) u *= scale;
         }
-        f32_finish<PAIR>(p, sg, t, n, y, u, old, PAIR ? zero : f32_turn(p, sg, t, n), PAIR ? -1 : f32_row(p, sg, t));
+        f32_finish<PAIR>(p, sg, t, n, y, u, side, side, row);
     };
-    const bool adds = !PAIR && sg.kind == F32Out::ADD;
-    // what the epilogue adds to is requested before the waves' sums meet
-    f4_t old[FPT];
-#pragma unroll
-    for (int q = 0; q < FPT; q++) {
-        const int e = min((int)threadIdx.x + q * KS * 64, ITEMS - 1), l = e & 63, j = (e >> 6) % TB, i = (e >> 6) / TB;
-        old[q] = adds ? f32_old(sg, min((tb0 + j) * 16 + (l & 15), T - 1), (nb0 + i) * 16 + 4 * (l >> 4)) : zero;
-    }
 #pragma unroll
     for (int n = 0; n < NT; n++)
 #pragma unroll
@@ -257,7 +289,7 @@ __global__ __launch_bounds__(KS * 64, f32_occupancy((PAIR ? 2 : 1) * NB * TB, NO
 #pragma unroll
             for (int v = 0; v < KS; v++) sum += s_ss[v][j * 16 + (l & 15)];
         }
-        finish((tb0 + j) * 16 + (l & 15), (nb0 + i) * 16 + 4 * (l >> 4), y, u, sum, old[q]);
+        finish((tb0 + j) * 16 + (l & 15), (nb0 + i) * 16 + 4 * (l >> 4), y, u, sum, side[q], row[q]);
     }
 }
 
@@ -279,9 +311,7 @@ template <bool PAIR>
 __global__ __launch_bounds__(256) void k_gemm_f32_any(F32Gemm p) {
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    int s = 0;
-    while (s + 1 < p.n_segs && (int)blockIdx.x >= p.seg[s + 1].first) s++;
-    const F32Segment& sg = p.seg[s];
+    const F32Segment& sg = p.seg[f32_segment(p, (int)blockIdx.x)];
     const int n = (((int)blockIdx.x - sg.first) * 4 + wave) * 4;
     int t0 = (int)blockIdx.y * 4;
     const int K = p.K, T = p.T, N = sg.N;
@@ -396,6 +426,7 @@ bool launch_gemm_f32(const F32Gemm& g, int prof_cls) {
         a.seg[s].first = tiles;
         tiles += cdiv(cdiv(a.seg[s].N, 16), NB);
     }
+    for (int s = a.n_segs; s < F32_SEGMENTS; s++) a.seg[s].first = INT_MAX;
     ProfScope ps(prof_cls, 4.0 * (weights * a.touched + (double)a.live * (a.K + outs)), 2.0 * a.live * weights);
     if (!rows16) {
         const dim3 grid(tiles, std::min(cdiv(a.T, 4), 32768));

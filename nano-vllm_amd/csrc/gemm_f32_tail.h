@@ -6,6 +6,14 @@
 
 namespace nvllm {
 
+// The segment of a feature tile (those that a launch has not begin past every tile).
+__device__ __forceinline__ int f32_segment(const F32Gemm& p, int tile) {
+    int s = 0;
+#pragma unroll
+    for (int i = 1; i < F32_SEGMENTS; i++) s += tile >= p.seg[i].first;
+    return s;
+}
+
 // What follows a token's complete sums of features n .. n+3 (n % 4 == 0; `old`: what ADD adds to).
 // `turn`: the angles of a quad that turns (f32_turn), `row`: its token's cache row.
 __device__ __forceinline__ f4_t f32_turn(const F32Gemm& p, const F32Segment& sg, int t, int n) {

@@ -13,7 +13,10 @@
 // 8 1,145 and 1,164.  So up to 6; passes of 6 and (tiles) 7 tokens at other widths: stories42M 303 and 352, four layers of
 // Llama-2-7B 522 and 551.
 // Eight rows to a workgroup instead of 16 (256 of them for wo and w_down) and six tiles in flight measured the same or
-// slower: it is the start of a launch, two dependent trips to memory, that is left.
+// slower: it is the start of a launch, two dependent trips to memory, that is left.  (With every trip that depends on nothing
+// started at once, as in gemm_f32.hip, a pass of one token 1,055 -> 1,035.)
+#include <climits>
+
 #include "gemm_f32_tail.h"
 #include "gemm_tile.h"
 
@@ -27,14 +30,13 @@ __global__ __launch_bounds__(KS * 64) void k_gemm_thin(F32Gemm p) {
     static_assert(!PAIR || NB == 1, "a pair is one block of either matrix");
     static_assert(NB <= KS, "a wave finishes a block");
     constexpr int NT = PAIR ? 2 : NB, RING = thin_ring(NT, NORM);
+    request_arguments<sizeof(F32Gemm)>();
     __shared__ f4_t s_red[KS][NT][64];
     __shared__ float s_ss[KS][16];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int x = lane & 15, g = lane >> 4;
-    int s = 0;
-    while (s + 1 < p.n_segs && (int)blockIdx.x >= p.seg[s + 1].first) s++;
-    const F32Segment& sg = p.seg[s];
+    const F32Segment& sg = p.seg[f32_segment(p, (int)blockIdx.x)];
     const int nb0 = ((int)blockIdx.x - sg.first) * NB;
     const int K = p.K, T = p.T, N = sg.N, blocks = (N + 15) >> 4;
     const h8_t* wp[NT];
@@ -44,16 +46,24 @@ __global__ __launch_bounds__(KS * 64) void k_gemm_thin(F32Gemm p) {
         wp[n] = reinterpret_cast<const h8_t*>(reinterpret_cast<const __half*>(W) + (size_t)(PAIR ? nb0 : min(nb0 + n, blocks - 1)) * sg.nb_stride) + lane;
     }
     const int tx = min(x, T - 1);   // columns past the last token compute it again and are not stored
-    const float* ap = p.in + (size_t)(p.in_rows ? p.in_rows[tx] : tx) * K + 8 * g;
-    const float* gp = NORM ? p.gain + 8 * g : nullptr;
-    // what the epilogue needs beside the sums travels from the start
-    const int nb = nb0 + (PAIR ? 0 : wave), n0 = nb * 16 + 4 * g;   // of the block this wave finishes
-    f4_t turn = {0.f, 0.f, 0.f, 0.f};
-    int row = -1;
-    if (!PAIR && wave < NB) {
-        turn = f32_turn(p, sg, tx, n0);
-        row = f32_row(p, sg, tx);
+    int from = tx;
+    if (p.in_rows) {
+        from = p.in_rows[tx];
+        asm volatile("" ::"v"(from));   // (waited for here, and not where launches without these rows meet)
     }
+    const float* ap = p.in + (size_t)from * K + 8 * g;
+    const float* gp = NORM ? p.gain + 8 * g : nullptr;
+    // what the epilogue needs beside the sums travels with the first tiles, and angles behind their positions
+    const int nb = nb0 + (PAIR ? 0 : wave), n0 = nb * 16 + 4 * g;   // of the block this wave finishes
+    const bool turns = !PAIR && wave < NB && (sg.kind == F32Out::ROPE_Q || sg.kind == F32Out::ROPE_K), adds = !PAIR && wave < NB && sg.kind == F32Out::ADD;
+    f4_t side = {0.f, 0.f, 0.f, 0.f};   // angles, or what is added to
+    int row = -1;
+    const int at = turns ? p.pos[tx] : 0;
+    auto request_side = [&] {
+        if (!PAIR && wave < NB) row = f32_row(p, sg, tx);
+        if (turns) side = *reinterpret_cast<const f4_t*>(p.rope + (size_t)at * (p.hd >> 1) + ((n0 % p.hd) >> 1));
+        else if (adds) side = f32_old(sg, tx, n0);
+    };
     h8_t w[RING][NT];
     f4_t a[RING][2], gv[RING][NORM ? 2 : 1];
     auto load = [&](int r, int i) {
@@ -104,12 +114,14 @@ __global__ __launch_bounds__(KS * 64) void k_gemm_thin(F32Gemm p) {
 #pragma unroll
         for (int r = 0; r + 1 < RING; r++)
             if (r < mine) load(r, r);
+        request_side();
 #pragma unroll
         for (int r = 0; r + 1 < RING; r++)
             if (r < mine) multiply(r);
     } else {
 #pragma unroll
         for (int r = 0; r < RING; r++) load(r, r);
+        request_side();
         int i0 = 0;
         for (; i0 + 2 * RING <= mine; i0 += RING) {
 #pragma unroll
@@ -127,7 +139,6 @@ __global__ __launch_bounds__(KS * 64) void k_gemm_thin(F32Gemm p) {
         for (int r = 0; r < RING; r++)
             if (i0 + r + RING < mine) multiply(r);
     }
-    const f4_t old = !PAIR && sg.kind == F32Out::ADD && wave < NB ? f32_old(sg, tx, n0) : zero;
 #pragma unroll
     for (int n = 0; n < NT; n++) s_red[wave][n][lane] = hi[n] + lo[n];
     if constexpr (NORM) {
@@ -153,7 +164,7 @@ __global__ __launch_bounds__(KS * 64) void k_gemm_thin(F32Gemm p) {
         y *= rinv;
         if constexpr (PAIR) u *= rinv;
     }
-    if (x < T && n0 < N) f32_finish<PAIR>(p, sg, x, n0, y, u, old, turn, row);
+    if (x < T && n0 < N) f32_finish<PAIR>(p, sg, x, n0, y, u, side, side, row);
     if (!PAIR && p.amax_pairs != nullptr) {
         // the block's first maximum per token, by the reference's scan (sampler.c:86-97): strict >, so a NaN never wins --
         // except at index 0, which nothing displaces: +inf there wins every comparison downstream
@@ -203,6 +214,7 @@ void launch_gemm_thin(const F32Gemm& g, int prof_cls) {
         a.seg[s].first = tiles;
         tiles += cdiv(cdiv(a.seg[s].N, 16), NB);
     }
+    for (int s = a.n_segs; s < F32_SEGMENTS; s++) a.seg[s].first = INT_MAX;
     ProfScope ps(prof_cls, 2.0 * weights + 4.0 * a.T * (a.K + outs), 2.0 * a.T * weights);
 #define NVLLM_GEMM_THIN(nb, ks, pair_)                                                                             \
     do {                                                                                                         \

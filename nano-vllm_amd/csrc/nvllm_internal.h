@@ -213,6 +213,19 @@ hipEvent_t prof_stop_event();
                               ::nvllm::prof_stop_event(), 0, __VA_ARGS__);                                   \
         HIP_CHECK(hipGetLastError());                                                                        \
     } while (0)
+// Requests every 64-byte line of the launch's first BYTES bytes of arguments at once (kernels call it first).  Their lines come from
+// memory in every launch, 0.2 us each, and a kernel that reads them as it needs them waits for one after the other.
+template <int BYTES>
+__device__ __forceinline__ void request_arguments() {
+    constexpr int LINES = (BYTES + 63) / 64;
+    static_assert(LINES <= 16, "one statement has them all");
+    const __attribute__((address_space(4))) int* at = (const __attribute__((address_space(4))) int*)__builtin_amdgcn_kernarg_segment_ptr();
+    int v[16];
+#pragma unroll
+    for (int i = 0; i < 16; i++) v[i] = at[(i < LINES ? i : 0) * 16];
+    asm volatile("" ::"s"(v[0]), "s"(v[1]), "s"(v[2]), "s"(v[3]), "s"(v[4]), "s"(v[5]), "s"(v[6]), "s"(v[7]), "s"(v[8]), "s"(v[9]), "s"(v[10]), "s"(v[11]),
+                 "s"(v[12]), "s"(v[13]), "s"(v[14]), "s"(v[15]));
+}
 // While one exists, ProfScope records nothing (and so creates no events): for entry points that
 // must not allocate.
 struct ProfSuppress {
