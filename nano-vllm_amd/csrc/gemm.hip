@@ -42,20 +42,14 @@
 
 namespace nvllm {
 
-#ifndef NVLLM_RW
-#define NVLLM_RW 4
-#endif
-#ifndef NVLLM_RA
-#define NVLLM_RA 2
-#endif
-
-// One workgroup = one tile (gemm_tile.h); weight ring of NVLLM_RW K-steps, activation ring of NVLLM_RA.
-template <int NBW, int TB, int NW, int EPI, typename KVT, int RW = NVLLM_RW>
+// One workgroup = one tile (gemm_tile.h); rings of RW K-steps of weights and activations.
+template <int NBW, int TB, int NW, int EPI, typename KVT, int RW = gemm_ring(NBW, TB, 2, EPI)>
 __global__ __launch_bounds__(NW * 64) void k_gemm(GemmArgs p) {
+    request_arguments<sizeof(GemmArgs)>();
     extern __shared__ __attribute__((aligned(16))) unsigned char lds_dyn[];
     h8_t w[RW][NBW];
     const TileIdx ix{(int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z, (int)gridDim.x};
-    gemm_tile<NBW, TB, NW, RW, NVLLM_RA, EPI, KVT, false, 0>(p, ix, lds_dyn, w, [](int) {}, (int)threadIdx.x);
+    gemm_tile<NBW, TB, NW, RW, gemm_ring_act(NBW, TB, RW), EPI, KVT, false, 0>(p, ix, lds_dyn, w, [](int) {}, (int)threadIdx.x);
 }
 
 // ------------------------------------------------------------------ launch
@@ -98,7 +92,7 @@ constexpr int MAX_COUNTERS = 1 << 16;
 
 // One instantiation: its dynamic LDS is the waves' partial tiles (1 KiB per wave, row block and
 // token block); sizes beyond the 64 KiB default are enabled once.
-template <int NBW, int TB, int NW, int EPI, typename KVT, int RW = NVLLM_RW>
+template <int NBW, int TB, int NW, int EPI, typename KVT, int RW = gemm_ring(NBW, TB, 2, EPI)>
 static void launch_k(const GemmArgs& a, dim3 grid) {
     constexpr int least = gemm_tile_lds<NBW, TB, NW>(), most = EPI == GemmEpilogue::F32 && TB > 1 ? std::max(least, GEMM_LDS_ALONE) : least;
     const int shmem = EPI == GemmEpilogue::F32 ? gemm_tile_lds<NBW, TB, NW>(a.e) : least;

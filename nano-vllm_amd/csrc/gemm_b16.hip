@@ -11,10 +11,11 @@ namespace nvllm {
 
 namespace {
 
-constexpr int NW = 8, RW = 4, RA = 2;
+constexpr int NW = 8;
 
 template <int NBW, int TB, int WAVES, int EPI, bool GRP, bool EXP = false>
 __global__ __launch_bounds__(WAVES * 64) void k_gemm_b16(GemmArgs p) {
+    request_arguments<sizeof(GemmArgs)>();
     extern __shared__ __attribute__((aligned(16))) unsigned char lds_dyn[];
     if constexpr (EPI == GemmEpilogue::LATENT_Q) {
         if ((int)blockIdx.x >= p.ride_from) {
@@ -22,9 +23,10 @@ __global__ __launch_bounds__(WAVES * 64) void k_gemm_b16(GemmArgs p) {
             return;
         }
     }
+    constexpr int RW = gemm_ring(NBW, TB, 1, EPI);
     h8_t w[RW][NBW];
     const TileIdx ix{(int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z, EPI == GemmEpilogue::LATENT_Q ? p.ride_from : (int)gridDim.x};
-    gemm_tile<NBW, TB, WAVES, RW, RA, EPI, float, false, 0, OpBf16, GRP, EXP>(p, ix, lds_dyn, w, [](int) {}, (int)threadIdx.x);
+    gemm_tile<NBW, TB, WAVES, RW, gemm_ring_act(NBW, TB, RW), EPI, float, false, 0, OpBf16, GRP, EXP>(p, ix, lds_dyn, w, [](int) {}, (int)threadIdx.x);
 }
 
 // The same with a mixture's router (SWIGLU_A16) or its choices (F32) in the workgroups from ride_from on (moe.h).  Each is a launch of
@@ -41,14 +43,16 @@ struct MoeRide {
 constexpr int ROUTER_NB = 2;   // 16-row blocks of the router and ...
 template <int NBW, int TB, int EPI>
 __global__ __launch_bounds__(NW * 64) void k_gemm_b16_moe(GemmArgs p, MoeRide r) {
+    request_arguments<sizeof(GemmArgs)>();
     extern __shared__ __attribute__((aligned(16))) unsigned char lds_dyn[];
     if ((int)blockIdx.x >= p.ride_from) {
         if (blockIdx.y != 0 || blockIdx.z != 0) return;
         if constexpr (EPI == GemmEpilogue::SWIGLU_A16) {   // ... 16 tokens each
             const int i = (int)blockIdx.x - p.ride_from;
             const TileIdx ix{i % r.router_tiles, 0, i / r.router_tiles, r.router_tiles};
+            constexpr int RW = gemm_ring(ROUTER_NB, 1, 1, GemmEpilogue::F32);
             h8_t w[RW][ROUTER_NB];
-            gemm_tile<ROUTER_NB, 1, NW, RW, RA, GemmEpilogue::F32, float, false, 0, OpBf16, false, false>(r.router, ix, lds_dyn, w, [](int) {}, (int)threadIdx.x);
+            gemm_tile<ROUTER_NB, 1, NW, RW, RW, GemmEpilogue::F32, float, false, 0, OpBf16, false, false>(r.router, ix, lds_dyn, w, [](int) {}, (int)threadIdx.x);
         } else if (r.chosen) {
             route_sort<false, NW * 64>(r.plan, nullptr, 0, reinterpret_cast<int*>(lds_dyn));
         } else {
@@ -56,9 +60,10 @@ __global__ __launch_bounds__(NW * 64) void k_gemm_b16_moe(GemmArgs p, MoeRide r)
         }
         return;
     }
+    constexpr int RW = gemm_ring(NBW, TB, 1, EPI);
     h8_t w[RW][NBW];
     const TileIdx ix{(int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z, p.ride_from};
-    gemm_tile<NBW, TB, NW, RW, RA, EPI, float, false, 0, OpBf16, false, false>(p, ix, lds_dyn, w, [](int) {}, (int)threadIdx.x);
+    gemm_tile<NBW, TB, NW, RW, gemm_ring_act(NBW, TB, RW), EPI, float, false, 0, OpBf16, false, false>(p, ix, lds_dyn, w, [](int) {}, (int)threadIdx.x);
 }
 template <int NBW, int TB, int EPI>
 void launch_stream_moe(const GemmArgs& a, const MoeRide& r, int riders, const GemmPlan& pl) {

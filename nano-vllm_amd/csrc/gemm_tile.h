@@ -35,6 +35,21 @@ struct TileIdx {
     int gx;        // feature tiles per token group (grid width, padding included)
 };
 
+// K-steps of weights and of activations in flight per wave.  Loads return in the order of their requests, so weights are in flight
+// no further ahead than the activations asked for behind them, and a CU takes no more in for more requests: what is in flight beyond the
+// trip's length queues.  us a launch of 64 rows at the widths of the 1.2B designs, rings of both of 2 / 3 / 4 / 5 / 7, and weights 4 with
+// activations 2: 64 x 32 tiles of a K split (w_down) 12.8 / 12.9 / 12.8 / 13.0 / 14.7 and 12.6 in fp16, 12.6 / 12.4 / 12.4 / 12.4 / 12.6 and 11.5 in
+// bf16; without one (the shared expert's) 12.0 / 12.6 / 13.3 / 13.1 / 13.6 and 13.4.  32 x 32 tiles with 4 and 8: 9.6 and 9.2 (LATENT_Q), 13.9 and
+// 15.5, 15.7 and 17.5; 32 x 16 tiles with 4 and 8: 7.2 and 6.6 (wo of Simivik).  64 x 16 tiles of experts 43.4 with 4 and 2 -> 39.3 with 4 of both; a
+// classifier of up to 16 rows has 3, so that two workgroups share a CU.  (Before, a wait for everything in flight stood in every step.)
+constexpr int gemm_ring(int NBW, int TB, int planes, int epi) {
+    if (NBW == 2) return TB == 1 ? 8 : 4;
+    if (NBW == 4 && TB == 2) return epi == GemmEpilogue::F32 || epi == GemmEpilogue::SWIGLU_A16 ? 2 : 4;
+    if (TB == 4) return planes == 2 ? 2 : 3;
+    return planes == 2 && NBW == 4 && TB == 1 && epi == GemmEpilogue::F32 ? 3 : 4;
+}
+constexpr int gemm_ring_act(int NBW, int TB, int ring) { return NBW == 4 && TB == 2 ? 2 : ring; }
+
 // bytes of dynamic LDS a tile needs: the waves' partial tiles, then four small arrays
 template <int NBW, int TB, int NW>
 constexpr int gemm_tile_lds() {
@@ -165,7 +180,8 @@ __device__ __forceinline__ bool gemm_tile(const GemmArgs& p, const TileIdx ix, u
     typedef f4_t RedTile[NBW][TB][64];
     RedTile* red = reinterpret_cast<RedTile*>(lds_dyn);
     float* s_rinv = reinterpret_cast<float*>(lds_dyn + NW * NBW * TB * 64 * 16);   // [TB * 16]
-    float (*s_part)[TB * 16] = reinterpret_cast<float (*)[TB * 16]>(s_rinv + TB * 16);   // [PARTS][TB * 16]
+    float (*s_part)[TB * 16 + 1] = reinterpret_cast<float (*)[TB * 16 + 1]>(s_rinv + TB * 16);   // [PARTS], rows of another bank each
+    static_assert(PARTS <= 2 * TB * 16, "the rows' pads fit what lies behind");
     unsigned* s_ticket = reinterpret_cast<unsigned*>(s_rinv + TB * 16 + NW * 64 + 2 * TB * 16);
 
     const int lane = tid & 63;
@@ -241,104 +257,175 @@ __device__ __forceinline__ bool gemm_tile(const GemmArgs& p, const TileIdx ix, u
 
     h8_t ah[RA][TB], al[RA][TB];
     auto kb_of = [&](int s) { return first + NW * s; };
-
-    // Loads are issued only for steps that exist (wave-uniform branches): a clamped
-    // re-load of the last tile would be real HBM traffic, since streamed weights are
-    // loaded non-temporally and do not stay in L2.
-    if (PRE == 0 || (PRE == 2 && !prefetched)) {
+    auto load_w = [&](int r, int s) {
 #pragma unroll
-        for (int s = 0; s < RW; s++)
-            if (s < nsteps) {
-                const int kb = kb_of(s);
+        for (int i = 0; i < NBW; i++) w[r][i] = NVLLM_WLOAD(wp[i] + (size_t)kb_of(s) * 64);
+    };
+    auto load_a = [&](int r, int s) {
 #pragma unroll
-                for (int i = 0; i < NBW; i++) w[s][i] = NVLLM_WLOAD(wp[i] + (size_t)kb * 64);
-            }
-    }
+        for (int j = 0; j < TB; j++) load_act(j, kb_of(s), ah[r][j], al[r][j]);
+    };
+    // requests stay in the order of their use: waits count what is younger
+    auto load = [&](int r, int s) {   // step s into entry r of rings of the same length
+        __builtin_amdgcn_sched_barrier(0);
+        load_w(r, s);
+        load_a(r % RA, s);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto multiply = [&](int r) {
 #pragma unroll
-    for (int s = 0; s < RA; s++)
-        if (s < nsteps) {
-            const int kb = kb_of(s);
+        for (int i = 0; i < NBW; i++)
 #pragma unroll
-            for (int j = 0; j < TB; j++) load_act(j, kb, ah[s][j], al[s][j]);
-        }
-    // 1/rms of this token group, from the producer's per-tile sums of squares: every
-    // thread sums a slice of one token's tiles (independent loads, issued while the
-    // first weight tiles are in flight); the slices meet in LDS before the epilogue.
-    if (p.e.ss_in != nullptr) {
-        const int tl = tid % (TB * 16), part = tid / (TB * 16);
-        const int t = min(tb0 * 16 + tl, p.T - 1);
-        const int src = p.e.ss_gather ? p.e.ss_gather[t] : t;
-        const float* sp = p.e.ss_in + (size_t)src * p.e.ss_tiles;
-        float ss = 0.f;
-        if constexpr (COH) {
-            for (int j = part; j < p.e.ss_tiles; j += PARTS)
-                ss += __builtin_bit_cast(float, __hip_atomic_load(reinterpret_cast<const unsigned*>(sp + j), __ATOMIC_RELAXED,
-                                                                  __HIP_MEMORY_SCOPE_AGENT));
-        } else {
-            for (int j = part; j < p.e.ss_tiles; j += PARTS) ss += sp[j];
-        }
-        s_part[part][tl] = ss;
-    }
-    NVLLM_TSTAMP(1, lane);
-    for (int s0 = 0; s0 < nsteps; s0 += RW) {
-#pragma unroll
-        for (int r = 0; r < RW; r++) {
-            const int s = s0 + r;
-            if (s < nsteps) {
-#pragma unroll
-                for (int i = 0; i < NBW; i++)
-#pragma unroll
-                    for (int j = 0; j < TB; j++) {
-                        acc[i][j] = OP::mfma(w[r][i], ah[r % RA][j], acc[i][j]);
+            for (int j = 0; j < TB; j++) {
+                acc[i][j] = OP::mfma(w[r][i], ah[r % RA][j], acc[i][j]);
 #ifndef NVLLM_ABLATE_LO
-                        if constexpr (OP::PLANES == 2) acc[i][j] = OP::mfma(w[r][i], al[r % RA][j], acc[i][j]);
+                if constexpr (OP::PLANES == 2) acc[i][j] = OP::mfma(w[r][i], al[r % RA][j], acc[i][j]);
 #endif
-                    }
-                if (s == 0) NVLLM_TSTAMP(2, acc[NBW - 1][TB - 1][0]);
-                if (s + RW < nsteps) {
-                    const int kbw = kb_of(s + RW);
-#pragma unroll
-                    for (int i = 0; i < NBW; i++) w[r][i] = NVLLM_WLOAD(wp[i] + (size_t)kbw * 64);
-                } else {
-                    slot_free(r);
-                }
-                if (s + RA < nsteps) {
-                    const int kba = kb_of(s + RA);
-#pragma unroll
-                    for (int j = 0; j < TB; j++) load_act(j, kba, ah[r % RA][j], al[r % RA][j]);
-                }
             }
-        }
-    }
-#pragma unroll
-    for (int r = 0; r < RW; r++)
-        if (r >= nsteps) slot_free(r);   // entries a short K slice never used
-    NVLLM_TSTAMP(3, acc[NBW - 1][TB - 1][0]);
-    // ---- 0. epilogue operands that do not depend on the sums: issue their loads now,
-    // so that they travel while the K split is being closed (every workgroup does it;
-    // only the one that ends up running the epilogue uses them).  Indices are clamped,
-    // not predicated: unconditional loads.
+    };
+
     const GemmEpilogue& ep = p.e;
+    // What the epilogue needs beside the sums is requested behind the first steps and waited for behind the last:
+    // 1/rms of this token group from the producer's per-tile sums of squares: every thread sums a slice of one token's tiles (up to
+    // SS_HELD of them held in registers over the K loop); the slices meet in LDS before the epilogue.  (Summed in front of the loop, each
+    // load waited for all before it: two to sixteen trips to memory before the first product.)
+    constexpr int SS_HELD = PARTS < 64 ? 64 / PARTS : 1;
+    float ss_held[SS_HELD];
+    const float* ss_row = nullptr;
+    const int ss_tl = tid / PARTS, ss_part = tid % PARTS;   // (lanes side by side read one token's sums: a line, and not one line each)
     float4 pf_x[FPT], pf_g[FPT];
     int pf_pos = 0, pf_row = -1;
+    f4_t pf_turn[FPT];
     __amdgpu_buffer_rsrc_t rs_x = gemm_rsrc(ep.x, (unsigned)p.T * (unsigned)p.N * 4u);
-    __amdgpu_buffer_rsrc_t rs_o = gemm_rsrc(ep.a16_out, (unsigned)p.Tb * (unsigned)ep.Kb_out * 2048u);
-    __amdgpu_buffer_rsrc_t rs_q = gemm_rsrc(ep.q_out, (unsigned)p.T * (unsigned)ep.QD * 4u);
-    if (EPI == GemmEpilogue::RESID_A16 || EPI == GemmEpilogue::RESID_B16) {
+    if (EPI == GemmEpilogue::ROPE_KV) {   // all items of a thread belong to one token (NW*64 is a multiple of TB*64)
+        const int e = min(tid, WITEMS - 1) & (ITEMS - 1);
+        const int t = min(tb0 * 16 + ((e >> 6) % TB) * 16 + (e & 15), p.T - 1);
+        pf_pos = ep.pos[t];
+        pf_row = ep.kv_row[t];
+    }
+    auto request_side = [&] {
+        if (ep.ss_in != nullptr) {
+            const int t = min(tb0 * 16 + ss_tl, p.T - 1);
+            int src = t;
+            if (ep.ss_gather) {
+                src = ep.ss_gather[t];
+                asm volatile("" ::"v"(src));
+            }
+            ss_row = ep.ss_in + (size_t)src * ep.ss_tiles;
+            if constexpr (!COH) {
+#pragma unroll
+                for (int q = 0; q < SS_HELD; q++) ss_held[q] = ss_row[min(ss_part + q * PARTS, ep.ss_tiles - 1)];
+            }
+        }
 #pragma unroll
         for (int s = 0; s < FPT; s++) {
             const int w_ = min(tid + s * NW * 64, WITEMS - 1);
             const int h = w_ >> ITEMS_SHIFT, e = w_ & (ITEMS - 1);
             const int l = e & 63, j = (e >> 6) % TB, i = (e >> 6) / TB;
-            const int t = min(tb0 * 16 + j * 16 + (l & 15), p.T - 1);
-            const int n = min((nb0 + 2 * h + i) * 16 + 4 * (l >> 4), p.N - 4);
-            if constexpr (COH)
-                pf_x[s] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rs_x, (t * p.N + n) * 4, 0, AUX_SC1));
-            else
-                pf_x[s] = *reinterpret_cast<const float4*>(ep.x + (size_t)t * p.N + n);
-            pf_g[s] = *reinterpret_cast<const float4*>(ep.gain_next + n);
+            const int n0 = (nb0 + 2 * h + i) * 16 + 4 * (l >> 4);
+            if (EPI == GemmEpilogue::RESID_A16 || EPI == GemmEpilogue::RESID_B16) {
+                const int t = min(tb0 * 16 + j * 16 + (l & 15), p.T - 1), n = min(n0, p.N - 4);
+                if constexpr (COH)
+                    pf_x[s] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rs_x, (t * p.N + n) * 4, 0, AUX_SC1));
+                else
+                    pf_x[s] = *reinterpret_cast<const float4*>(ep.x + (size_t)t * p.N + n);
+                pf_g[s] = *reinterpret_cast<const float4*>(ep.gain_next + n);
+            }
+            // (q and k begin at multiples of hd; values have an angle that nobody uses)
+            if (EPI == GemmEpilogue::ROPE_KV) pf_turn[s] = *reinterpret_cast<const f4_t*>(ep.rope + (size_t)pf_pos * (ep.hd >> 1) + ((n0 % ep.hd) >> 1));
         }
+    };
+
+    // Loads are issued only for steps that exist: a clamped re-load of the last tile would be real HBM traffic, since streamed
+    // weights are loaded non-temporally and do not stay in L2.  The steady loop requests without a condition: where paths with and
+    // without requests meet, the compiler waits for all of them.
+    const bool mine = PRE == 0 || (PRE == 2 && !prefetched);   // whether the first weights are requested here
+    if (nsteps < RW) {
+#pragma unroll
+        for (int s = 0; s + 1 < RW; s++)
+            if (s < nsteps) {
+                if (mine) load_w(s, s);
+                if (s < RA) load_a(s, s);
+            }
+        request_side();
+        NVLLM_TSTAMP(1, lane);
+#pragma unroll
+        for (int s = 0; s + 1 < RW; s++)
+            if (s < nsteps) {
+                multiply(s);
+                if (s == 0) NVLLM_TSTAMP(2, acc[NBW - 1][TB - 1][0]);
+                if (s + RA < nsteps) load_a(s % RA, s + RA);
+                slot_free(s);
+            }
+#pragma unroll
+        for (int r = 0; r < RW; r++)
+            if (r >= nsteps) slot_free(r);   // entries a short K slice never used
+    } else {
+        if constexpr (RA == RW && PRE == 0) {
+#pragma unroll
+            for (int r = 0; r < RW; r++) load(r, r);
+        } else {
+            if (mine) {
+#pragma unroll
+                for (int r = 0; r < RW; r++) load_w(r, r);
+            }
+#pragma unroll
+            for (int r = 0; r < RA; r++) load_a(r, r);
+        }
+        request_side();
+        NVLLM_TSTAMP(1, lane);
+        int i0 = 0;
+        for (; i0 + 2 * RW <= nsteps; i0 += RW) {
+#pragma unroll
+            for (int r = 0; r < RW; r++) {
+                multiply(r);
+                if (i0 + r == 0) NVLLM_TSTAMP(2, acc[NBW - 1][TB - 1][0]);
+                if constexpr (RA == RW) {
+                    load(r, i0 + r + RW);
+                } else {
+                    load_w(r, i0 + r + RW);
+                    load_a(r % RA, i0 + r + RA);
+                }
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < RW; r++) {
+            multiply(r);
+            if (i0 + r + RW < nsteps) load_w(r, i0 + r + RW);
+            else slot_free(r);
+            if (i0 + r + RA < nsteps) load_a(r % RA, i0 + r + RA);
+        }
+#pragma unroll
+        for (int r = 0; r < RW; r++)
+            if (i0 + RW + r < nsteps) {
+                multiply(r);
+                if (i0 + RW + r + RA < nsteps) load_a(r % RA, i0 + RW + r + RA);
+                slot_free(r);
+            }
     }
+    NVLLM_TSTAMP(3, acc[NBW - 1][TB - 1][0]);
+    if (ep.ss_in != nullptr) {
+        float ss = 0.f;
+        int j = ss_part;
+        if constexpr (COH) {
+            for (; j < ep.ss_tiles; j += PARTS)
+                ss += __builtin_bit_cast(float, __hip_atomic_load(reinterpret_cast<const unsigned*>(ss_row + j), __ATOMIC_RELAXED,
+                                                                  __HIP_MEMORY_SCOPE_AGENT));
+        } else {
+#pragma unroll
+            for (int q = 0; q < SS_HELD; q++)
+                if (ss_part + q * PARTS < ep.ss_tiles) ss += ss_held[q];
+#pragma unroll 4
+            for (j += SS_HELD * PARTS; j < ep.ss_tiles; j += PARTS) ss += ss_row[j];
+        }
+        s_part[ss_part][ss_tl] = ss;
+    }
+    // ---- 0. epilogue operands that do not depend on the sums and are too many to be held over the K loop: issue their loads now,
+    // so that they travel while the K split is being closed (every workgroup does it;
+    // only the one that ends up running the epilogue uses them).  Indices are clamped,
+    // not predicated: unconditional loads.
+    __amdgpu_buffer_rsrc_t rs_o = gemm_rsrc(ep.a16_out, (unsigned)p.Tb * (unsigned)ep.Kb_out * 2048u);
+    __amdgpu_buffer_rsrc_t rs_q = gemm_rsrc(ep.q_out, (unsigned)p.T * (unsigned)ep.QD * 4u);
     constexpr int HS = hyper_streams(EPI);
     HyperIn<HS ? HS : 1> pf_hyper[HS ? FPT : 1];
     HyperMix<HS ? HS : 1> hyper_c;
@@ -351,12 +438,6 @@ __device__ __forceinline__ bool gemm_tile(const GemmArgs& p, const TileIdx ix, u
             const int l = e & 63, j = (e >> 6) % TB, i = (e >> 6) / TB;
             hyper_load_4<HS>(pf_hyper[s], ep, p.N, min(tb0 * 16 + j * 16 + (l & 15), p.T - 1), min((nb0 + 2 * h + i) * 16 + 4 * (l >> 4), p.N - 4));
         }
-    }
-    if (EPI == GemmEpilogue::ROPE_KV) {   // all items of a thread belong to one token (NW*64 is a multiple of TB*64)
-        const int e = min(tid, WITEMS - 1) & (ITEMS - 1);
-        const int t = min(tb0 * 16 + ((e >> 6) % TB) * 16 + (e & 15), p.T - 1);
-        pf_pos = ep.pos[t];
-        pf_row = ep.kv_row[t];
     }
     // ---- 1. sum the waves' partial tiles through LDS: every wave stores all its tiles, ONE
     // barrier, then each thread collects its items w = (round h, e): the float4 for token t(e) and
@@ -572,9 +653,7 @@ __device__ __forceinline__ bool gemm_tile(const GemmArgs& p, const TileIdx ix, u
             } else {  // ROPE_KV
                 if (live) {
                     if (n < ep.QD + ep.KD) {   // q or k: rotate the two pairs of this float4 (layers.c:118-141)
-                        const int d = (n < ep.QD ? n : n - ep.QD) % ep.hd;
-                        const float2* tab = ep.rope + (size_t)pf_pos * (ep.hd >> 1) + (d >> 1);
-                        const float2 c0 = tab[0], c1 = tab[1];
+                        const float2 c0 = make_float2(pf_turn[s][0], pf_turn[s][1]), c1 = make_float2(pf_turn[s][2], pf_turn[s][3]);
                         const float a0 = y[0], b0 = y[1], a1 = y[2], b1 = y[3];
                         y[0] = __fsub_rn(__fmul_rn(a0, c0.x), __fmul_rn(b0, c0.y));
                         y[1] = __fadd_rn(__fmul_rn(a0, c0.y), __fmul_rn(b0, c0.x));
