@@ -399,58 +399,76 @@ __device__ __forceinline__ float of_quad(float v) {   // the value of thread Q o
     return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(i, i, Q * 0x55, 0xf, 0xf, false));
 }
 template <int TOKENS, int THREADS>
-__device__ __forceinline__ void tile_rinv(const GemmArgs& p, int tb0, float* s_rinv) {
-    constexpr int ROUNDS = (TOKENS * 4 + THREADS - 1) / THREADS;   // tokens of a thread
-    const int part = (int)threadIdx.x & 3, first = (int)threadIdx.x >> 2, cols = p.e.ss_tiles;
+struct TileRinv {
+    static constexpr int ROUNDS = (TOKENS * 4 + THREADS - 1) / THREADS;   // tokens of a thread
     const float* sp[ROUNDS];
-    float even[ROUNDS], odd[ROUNDS];
-#pragma unroll
-    for (int r = 0; r < ROUNDS; r++) {
-        const int t = min(tb0 * 16 + first + r * (THREADS / 4), p.T - 1);
-        sp[r] = p.e.ss_in + (size_t)(p.e.ss_gather ? p.e.ss_gather[t] : t) * cols;
-        even[r] = odd[r] = 0.f;
-    }
-    if ((cols & 3) == 0) {
-        for (int j0 = 0; j0 < cols; j0 += 64) {
-            f4_t v[ROUNDS][4];
-#pragma unroll
-            for (int r = 0; r < ROUNDS; r++)
-#pragma unroll
-                for (int i = 0; i < 4; i++) v[r][i] = *reinterpret_cast<const f4_t*>(sp[r] + min(j0 + 16 * i + 4 * part, cols - 4));
-#pragma unroll
-            for (int r = 0; r < ROUNDS; r++)
-#pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    if (j0 + 16 * i + 4 * part >= cols) v[r][i] = f4_t{0.f, 0.f, 0.f, 0.f};
-                    auto add = [&](auto q) {
-                        even[r] += of_quad<decltype(q)::value>(v[r][i][0]);
-                        odd[r] += of_quad<decltype(q)::value>(v[r][i][1]);
-                        even[r] += of_quad<decltype(q)::value>(v[r][i][2]);
-                        odd[r] += of_quad<decltype(q)::value>(v[r][i][3]);
-                    };
-                    add(std::integral_constant<int, 0>{});
-                    add(std::integral_constant<int, 1>{});
-                    add(std::integral_constant<int, 2>{});
-                    add(std::integral_constant<int, 3>{});
-                }
-        }
-    } else {
+    f4_t v[ROUNDS][4];   // the first 64 columns
+    __device__ __forceinline__ void load(int cols, int j0) {
 #pragma unroll
         for (int r = 0; r < ROUNDS; r++)
-            for (int j = 0; j < cols; j += 2) {
-                even[r] += sp[r][j];
-                if (j + 1 < cols) odd[r] += sp[r][j + 1];
-            }
-    }
 #pragma unroll
-    for (int r = 0; r < ROUNDS; r++) {
-        const int tl = first + r * (THREADS / 4);
-        if (part == 0 && tl < TOKENS) s_rinv[tl] = __fdiv_rn(1.0f, sqrtf(__fadd_rn(__fdiv_rn(even[r] + odd[r], (float)p.e.d_in), p.e.eps)));
+            for (int i = 0; i < 4; i++) v[r][i] = *reinterpret_cast<const f4_t*>(sp[r] + min(j0 + 16 * i + 4 * ((int)threadIdx.x & 3), cols - 4));
     }
+    // (columns in fours: 64 of them are asked for here)
+    __device__ __forceinline__ void request(const GemmArgs& p, int tb0) {
+        const int first = (int)threadIdx.x >> 2, cols = p.e.ss_tiles;
+#pragma unroll
+        for (int r = 0; r < ROUNDS; r++) {
+            const int t = min(tb0 * 16 + first + r * (THREADS / 4), p.T - 1);
+            sp[r] = p.e.ss_in + (size_t)(p.e.ss_gather ? p.e.ss_gather[t] : t) * cols;
+        }
+        if ((cols & 3) == 0) load(cols, 0);
+    }
+    __device__ __forceinline__ void finish(const GemmArgs& p, float* s_rinv) {
+        const int part = (int)threadIdx.x & 3, first = (int)threadIdx.x >> 2, cols = p.e.ss_tiles;
+        float even[ROUNDS], odd[ROUNDS];
+#pragma unroll
+        for (int r = 0; r < ROUNDS; r++) even[r] = odd[r] = 0.f;
+        if ((cols & 3) == 0) {
+            for (int j0 = 0; j0 < cols; j0 += 64) {
+                if (j0) load(cols, j0);
+#pragma unroll
+                for (int r = 0; r < ROUNDS; r++)
+#pragma unroll
+                    for (int i = 0; i < 4; i++) {
+                        if (j0 + 16 * i + 4 * part >= cols) v[r][i] = f4_t{0.f, 0.f, 0.f, 0.f};
+                        auto add = [&](auto q) {
+                            even[r] += of_quad<decltype(q)::value>(v[r][i][0]);
+                            odd[r] += of_quad<decltype(q)::value>(v[r][i][1]);
+                            even[r] += of_quad<decltype(q)::value>(v[r][i][2]);
+                            odd[r] += of_quad<decltype(q)::value>(v[r][i][3]);
+                        };
+                        add(std::integral_constant<int, 0>{});
+                        add(std::integral_constant<int, 1>{});
+                        add(std::integral_constant<int, 2>{});
+                        add(std::integral_constant<int, 3>{});
+                    }
+            }
+        } else {
+#pragma unroll
+            for (int r = 0; r < ROUNDS; r++)
+                for (int j = 0; j < cols; j += 2) {
+                    even[r] += sp[r][j];
+                    if (j + 1 < cols) odd[r] += sp[r][j + 1];
+                }
+        }
+#pragma unroll
+        for (int r = 0; r < ROUNDS; r++) {
+            const int tl = first + r * (THREADS / 4);
+            if (part == 0 && tl < TOKENS) s_rinv[tl] = __fdiv_rn(1.0f, sqrtf(__fadd_rn(__fdiv_rn(even[r] + odd[r], (float)p.e.d_in), p.e.eps)));
+        }
+    }
+};
+template <int TOKENS, int THREADS>
+__device__ __forceinline__ void tile_rinv(const GemmArgs& p, int tb0, float* s_rinv) {
+    TileRinv<TOKENS, THREADS> r;
+    r.request(p, tb0);
+    r.finish(p, s_rinv);
 }
 
 template <int FW, int KG, int EPI, typename KVT, int WR = 2, int TW = 4, typename OP = OpF16x2, bool GRP = false, bool EXP = false>
 __global__ __launch_bounds__(128 * WR * KG, 2) void k_gemm_prefill(GemmArgs p, int tiles_n, int tiles_t, int nbuf, int split_from) {
+    request_arguments<sizeof(GemmArgs)>();
     constexpr int PL = OP::PLANES;
     using G = PfGeom<FW, KG, WR, TW, PL>;
 #ifdef NVLLM_PF_ABLATE

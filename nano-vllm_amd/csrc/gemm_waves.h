@@ -36,6 +36,7 @@ constexpr bool waves_carry_route(int TBN, int EPI, int planes) {
 
 template <int TBN, int EPI, typename KVT, typename OP>
 __global__ __launch_bounds__(256, 1) void k_gemm_waves(GemmArgs p, int tiles_n, int tiles_t) {
+    request_arguments<sizeof(GemmArgs)>();
     constexpr int FB = WAVES_FB, PL = OP::PLANES, NA = PL * TBN, RING = waves_ring(PL, TBN);
     extern __shared__ __attribute__((aligned(16))) unsigned char lds_waves[];
     float* s_rinv = reinterpret_cast<float*>(lds_waves);
@@ -90,6 +91,9 @@ __global__ __launch_bounds__(256, 1) void k_gemm_waves(GemmArgs p, int tiles_n, 
     for (int f = 0; f < FB; f++)
 #pragma unroll
         for (int j = 0; j < TBN; j++) acc[f][j] = f4_t{0.f, 0.f, 0.f, 0.f};
+    // (in front of the first steps, which would be waited for with it; added up while they travel)
+    TileRinv<16 * TBN, 256> rinv;
+    if (p.e.ss_in != nullptr) rinv.request(p, tb0);
 #pragma unroll
     for (int r = 0; r < RING; r++) {
         const auto rw = operand(W, r < mine), ra = operand(A, r < mine);
@@ -101,7 +105,7 @@ __global__ __launch_bounds__(256, 1) void k_gemm_waves(GemmArgs p, int tiles_n, 
         __builtin_amdgcn_sched_barrier(0);
         next_step();
     }
-    if (p.e.ss_in != nullptr) tile_rinv<16 * TBN, 256>(p, tb0, s_rinv);
+    if (p.e.ss_in != nullptr) rinv.finish(p, s_rinv);
 
     // Step i out of registers r, each replaced by step i + RING's as soon as it has been multiplied.  The loop has one exit and
     // no condition around a request: where paths with and without requests meet, the compiler waits for all of them.

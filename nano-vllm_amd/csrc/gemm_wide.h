@@ -51,6 +51,7 @@ __device__ __forceinline__ void wide_wait() {
 // EXP: rows sorted by expert, every tile's of one (ExpertRows)
 template <int TBN, int WT, int EPI, typename KVT, typename OP, bool EXP = false>
 __global__ __launch_bounds__(256 * WT, 1) void k_gemm_wide(GemmArgs p, int tiles_n, int tiles_t, int panel) {
+    request_arguments<sizeof(GemmArgs)>();
     constexpr int PL = OP::PLANES;
     using G = WideGeom<TBN, PL, WT>;
     constexpr int RING = G::RING, CPW = G::CPW, WAVES = G::WAVES, TBW = TBN / WT;   // TBW: token blocks of a wave

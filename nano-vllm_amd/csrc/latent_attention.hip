@@ -572,6 +572,7 @@ struct LatentValueArgs {
 };
 template <int TW, int U>   // U: slices requested at once
 __global__ __launch_bounds__(VALUE_WAVES * 64) void k_latent_value(LatentValueArgs a) {
+    request_arguments<sizeof(LatentValueArgs)>();
     constexpr int LD = VALUE_KC * 32 + 8;   // halves of a row: 16 rows' pieces of 16 bytes meet every bank once
     constexpr int D = VALUE_KC * 32 / 256;  // pieces of four values a lane has
     __shared__ __attribute__((aligned(16))) __bf16 rows[16][LD];

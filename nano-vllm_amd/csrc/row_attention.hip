@@ -19,6 +19,7 @@ constexpr int ROW_WAVES = 8;
 
 template <int HD, int G>
 __global__ __launch_bounds__(64 * ROW_WAVES) void k_row_attn(AttnKArgs a) {
+    request_arguments<sizeof(AttnKArgs)>();
     constexpr int LPK = row_attn_lanes(HD), KEYS = 64 / LPK, AHEAD = 8;
     static_assert(KEYS * ROW_WAVES * AHEAD == row_attn_keys(HD));
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);

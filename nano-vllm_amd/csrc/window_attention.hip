@@ -210,6 +210,7 @@ __global__ __launch_bounds__(256) void k_conv_rope(ConvKArgs a) {
 // tokens and the rows of the state one after the other, 4.9 here.
 template <int KEEP>
 __global__ __launch_bounds__(256) void k_conv_rope_f32(ConvKArgs a) {
+    request_arguments<sizeof(ConvKArgs)>();
     const int item = blockIdx.y * 256 + threadIdx.x, t_mine = blockIdx.x;
     if (item >= a.items) return;
     const int4 span = a.spans[a.span_of[t_mine]];   // (first token, count, first position, sequence)
@@ -306,6 +307,7 @@ struct alignas(16) Piece {
 };
 template <int KEEP, int TOK>
 __global__ __launch_bounds__(256) void k_conv_rope_walk(ConvKArgs a, int T) {
+    request_arguments<sizeof(ConvKArgs)>();
     const int item = blockIdx.y * 256 + threadIdx.x, t0 = blockIdx.x * TOK;
     if (item >= a.items) return;
     int part, head, at, i = item;
