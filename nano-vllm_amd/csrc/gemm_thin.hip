@@ -25,6 +25,208 @@ namespace nvllm {
 // tiles in flight per wave, as many as 128 registers hold (16 waves per CU)
 constexpr int thin_ring(int NT, bool norm) { return NT == 1 ? 4 : NT == 2 ? (norm ? 3 : 4) : 2; }
 
+// What follows the complete sums of features n0 .. n0 + 3 of token x.
+template <bool PAIR>
+__device__ __forceinline__ void thin_finish(const F32Gemm& p, const F32Segment& sg, int x, int g, int nb, int n0, const f4_t& y, const f4_t& u, const f4_t& side, int row) {
+    const int T = p.T, N = sg.N;
+    if (x < T && n0 < N) f32_finish<PAIR>(p, sg, x, n0, y, u, side, side, row);
+    if (!PAIR && p.amax_pairs != nullptr) {
+        // the block's first maximum per token, by the reference's scan (sampler.c:86-97): strict >, so a NaN never wins --
+        // except at index 0, which nothing displaces: +inf there wins every comparison downstream
+        float bv = -INFINITY, bi = -1.0f;
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+            if (n0 + r < N && (y[r] > bv || (bi < 0.f && y[r] == bv))) {
+                bv = y[r];
+                bi = (float)(n0 + r);
+            }
+        if (n0 == 0 && y[0] != y[0]) {
+            bv = INFINITY;
+            bi = 0.f;
+        }
+#pragma unroll
+        for (int o = 16; o < 64; o <<= 1) {
+            const float ov = __shfl_xor(bv, o, 64), oi = __shfl_xor(bi, o, 64);
+            if (oi >= 0.f && (ov > bv || bi < 0.f || (ov == bv && oi < bi))) {
+                bv = ov;
+                bi = oi;
+            }
+        }
+        if (g == 0 && x < T) p.amax_pairs[(size_t)nb * p.amax_ld + x] = make_float2(bv, bi);
+    }
+}
+
+// The same with the activations in LDS, where every workgroup lays them out once, in operand order: [k tile][group of 8 k][token], the hi
+// plane and then the lo plane.  From memory a wave asks for 2 KiB of them beside each KiB of weights, and for 2 of gains where there is a
+// norm (every lane its operand, whichever of the 16 columns is alive).  The activations are asked for first (loads return in order), the ring of
+// weights behind them.  w_down of TinyLlama at one token: the products are done 5.9 us after the first workgroup's start instead of 7.8, the
+// launch after 8.0 instead of 8.9; what is left is its 23 MB, 4.6 us of them, behind a start of 1.1, the slowest wave's issue and layout, and two meetings.
+constexpr int thin_lds_ring(int NT) { return NT == 1 ? 8 : NT == 2 ? 6 : 3; }
+template <int NT, int KS>
+constexpr int thin_lds_bytes(int K, int T, bool norm) { return KS * NT * 1024 + K * T * 4 + (norm ? T * (K / 32) * 4 : 0); }
+template <int NB, int KS, bool PAIR, bool NORM>
+__global__ __launch_bounds__(KS * 64) void k_gemm_thin_lds(F32Gemm p) {
+    static_assert(!PAIR || NB == 1, "a pair is one block of either matrix");
+    static_assert(NB <= KS, "a wave finishes a block");
+    constexpr int NT = PAIR ? 2 : NB, RING = thin_lds_ring(NT), THREADS = KS * 64, LAP = 4;
+    request_arguments<sizeof(F32Gemm)>();
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds_thin[];
+    f4_t(*s_red)[NT][64] = reinterpret_cast<f4_t(*)[NT][64]>(lds_thin);   // [wave]
+    __half* s_act = reinterpret_cast<__half*>(lds_thin + KS * NT * 1024);
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int x = lane & 15, g = lane >> 4;
+    const F32Segment& sg = p.seg[f32_segment(p, (int)blockIdx.x)];
+    const int nb0 = ((int)blockIdx.x - sg.first) * NB;
+    const int K = p.K, T = p.T, N = sg.N, blocks = (N + 15) >> 4, Kb = K >> 5, K4 = K >> 2;
+    float* s_sq = reinterpret_cast<float*>(s_act + 2 * (size_t)K * T);   // NORM: [token][32 k]
+    const int tx = min(x, T - 1);   // columns past the last token compute it again and are not stored
+    const int nb = nb0 + (PAIR ? 0 : wave), n0 = nb * 16 + 4 * g;   // of the block this wave finishes
+    const bool turns = !PAIR && wave < NB && (sg.kind == F32Out::ROPE_Q || sg.kind == F32Out::ROPE_K), adds = !PAIR && wave < NB && sg.kind == F32Out::ADD;
+    const int at = turns ? p.pos[tx] : 0;
+
+    // activations: item i is four k of a token, LAP of a thread at a time
+    const int items = T * K4;
+    f4_t v[LAP], gn[NORM ? LAP : 1];
+    auto place = [&](int i, int& t, int& k4) {
+        t = 0;
+        k4 = min(i, items - 1);
+#pragma unroll
+        for (int u = 1; u < THIN_TOKENS; u++)
+            if (k4 >= K4) {
+                k4 -= K4;
+                t++;
+            }
+    };
+    auto request = [&](int i0) {
+#pragma unroll
+        for (int u = 0; u < LAP; u++) {
+            if (u * THREADS + i0 - (int)threadIdx.x >= items) continue;   // (uniform: nobody's)
+            int t, k4;
+            place(i0 + u * THREADS, t, k4);
+            if (p.in_rows) {
+                t = p.in_rows[t];
+                asm volatile("" ::"v"(t));
+            }
+            v[u] = *reinterpret_cast<const f4_t*>(p.in + (size_t)t * K + 4 * k4);
+            if constexpr (NORM) gn[u] = *reinterpret_cast<const f4_t*>(p.gain + 4 * k4);
+        }
+    };
+    auto lay_out = [&](int i0) {
+#pragma unroll
+        for (int u = 0; u < LAP; u++) {
+            const int i = i0 + u * THREADS;
+            if (i >= items) continue;
+            int t, k4;
+            place(i, t, k4);
+            f4_t a = v[u];
+            if constexpr (NORM) {
+                float sq = a[0] * a[0];
+#pragma unroll
+                for (int e = 1; e < 4; e++) sq = fmaf(a[e], a[e], sq);
+                // (K4 is a multiple of eight: eight lanes side by side have a token's 32 k)
+                sq += __shfl_xor(sq, 1, 64);
+                sq += __shfl_xor(sq, 2, 64);
+                sq += __shfl_xor(sq, 4, 64);
+                if ((k4 & 7) == 0) s_sq[t * Kb + (k4 >> 3)] = sq;
+                a *= gn[u];
+            }
+            alignas(8) _Float16 hi[4], lo[4];
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const float c = fminf(fmaxf(a[e], -65504.f), 65504.f);
+                hi[e] = (_Float16)c;
+                lo[e] = (_Float16)(c - (float)hi[e]);
+            }
+            __half* to = s_act + ((size_t)(k4 >> 1) * T + t) * 8 + 4 * (k4 & 1);
+            *reinterpret_cast<uint2*>(to) = *reinterpret_cast<uint2*>(hi);
+            *reinterpret_cast<uint2*>(to + (size_t)K * T) = *reinterpret_cast<uint2*>(lo);
+        }
+    };
+    request((int)threadIdx.x);
+
+    // weights: a step past the wave's last is requested through a descriptor of length zero: no traffic, and no branch around a request
+    const int mine = wave < Kb ? (Kb - wave + KS - 1) / KS : 0;
+    h8_t w[RING][NT];
+    const __half* W = reinterpret_cast<const __half*>(sg.W) + (size_t)nb0 * sg.nb_stride;
+    const __half* W2 = PAIR ? reinterpret_cast<const __half*>(sg.W2) + (size_t)nb0 * sg.nb_stride : nullptr;
+    unsigned of_w[NT];
+#pragma unroll
+    for (int n = 0; n < NT; n++) of_w[n] = PAIR ? 0u : (unsigned)min(n, blocks - 1 - nb0) * (unsigned)(sg.nb_stride * sizeof(__half));
+    auto load = [&](int r, int i) {
+        const int bytes = i < mine ? 0x7fffffff : 0;
+        const auto from = __builtin_amdgcn_make_buffer_rsrc(const_cast<__half*>(W), 0, bytes, 0x00020000);
+        const auto from2 = __builtin_amdgcn_make_buffer_rsrc(const_cast<__half*>(PAIR ? W2 : W), 0, bytes, 0x00020000);
+        const unsigned step = (unsigned)(wave + i * KS) * 1024u;
+        __builtin_amdgcn_sched_barrier(0);   // requests stay in the order of their use: waits count what is younger
+#pragma unroll
+        for (int n = 0; n < NT; n++)
+            w[r][n] = __builtin_bit_cast(h8_t, __builtin_amdgcn_raw_buffer_load_b128(PAIR && n == 1 ? from2 : from, lane * 16, step + of_w[n], /*nt*/ 2));
+        __builtin_amdgcn_sched_barrier(0);
+    };
+#pragma unroll
+    for (int r = 0; r < RING; r++) load(r, r);
+    lay_out((int)threadIdx.x);
+    for (int i0 = (int)threadIdx.x + LAP * THREADS; i0 - (int)threadIdx.x < items; i0 += LAP * THREADS) {
+        request(i0);
+        lay_out(i0);
+    }
+    // what the epilogue needs beside the sums travels with the first tiles
+    f4_t side = {0.f, 0.f, 0.f, 0.f};   // angles, or what is added to
+    int row = -1;
+    if (!PAIR && wave < NB) row = f32_row(p, sg, tx);
+    if (turns) side = *reinterpret_cast<const f4_t*>(p.rope + (size_t)at * (p.hd >> 1) + ((n0 % p.hd) >> 1));
+    else if (adds) side = f32_old(sg, tx, n0);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // (not for the weights in flight)
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+
+    const f4_t zero = {0.f, 0.f, 0.f, 0.f};
+    f4_t hi[NT], lo[NT];
+#pragma unroll
+    for (int n = 0; n < NT; n++) hi[n] = lo[n] = zero;
+    const h8_t* acts = reinterpret_cast<const h8_t*>(s_act) + (size_t)g * T + tx;
+    const int plane = K / 8 * T;
+    for (int i0 = 0; i0 < mine; i0 += RING) {
+#pragma unroll
+        for (int r = 0; r < RING; r++) {
+            if (i0 + r < mine) {
+                const h8_t* a = acts + (size_t)(wave + (i0 + r) * KS) * 4 * T;
+                const h8_t vh = a[0], vl = a[plane];
+#pragma unroll
+                for (int n = 0; n < NT; n++) {
+                    hi[n] = OpF16x2::mfma(w[r][n], vh, hi[n]);
+                    lo[n] = OpF16x2::mfma(w[r][n], vl, lo[n]);
+                }
+            }
+            load(r, i0 + r + RING);
+        }
+    }
+#pragma unroll
+    for (int n = 0; n < NT; n++) s_red[wave][n][lane] = hi[n] + lo[n];
+    __syncthreads();
+    if (wave >= NB || nb >= blocks) return;
+    f4_t y = s_red[0][PAIR ? 0 : wave][lane], u = zero;
+#pragma unroll
+    for (int q = 1; q < KS; q++) y += s_red[q][PAIR ? 0 : wave][lane];
+    if constexpr (PAIR) {
+        u = s_red[0][1][lane];
+#pragma unroll
+        for (int q = 1; q < KS; q++) u += s_red[q][1][lane];
+    }
+    if constexpr (NORM) {
+        float sum = 0.f;
+#pragma unroll 4
+        for (int j = g; j < Kb; j += 4) sum += s_sq[tx * Kb + j];
+        sum += __shfl_xor(sum, 16, 64);
+        sum += __shfl_xor(sum, 32, 64);
+        const float rinv = __fdiv_rn(1.0f, sqrtf(__fadd_rn(__fdiv_rn(sum, (float)K), p.eps)));
+        y *= rinv;
+        if constexpr (PAIR) u *= rinv;
+    }
+    thin_finish<PAIR>(p, sg, x, g, nb, n0, y, u, side, row);
+}
+
 template <int NB, int KS, bool PAIR, bool NORM>
 __global__ __launch_bounds__(KS * 64) void k_gemm_thin(F32Gemm p) {
     static_assert(!PAIR || NB == 1, "a pair is one block of either matrix");
@@ -164,31 +366,28 @@ __global__ __launch_bounds__(KS * 64) void k_gemm_thin(F32Gemm p) {
         y *= rinv;
         if constexpr (PAIR) u *= rinv;
     }
-    if (x < T && n0 < N) f32_finish<PAIR>(p, sg, x, n0, y, u, side, side, row);
-    if (!PAIR && p.amax_pairs != nullptr) {
-        // the block's first maximum per token, by the reference's scan (sampler.c:86-97): strict >, so a NaN never wins --
-        // except at index 0, which nothing displaces: +inf there wins every comparison downstream
-        float bv = -INFINITY, bi = -1.0f;
-#pragma unroll
-        for (int r = 0; r < 4; r++)
-            if (n0 + r < N && (y[r] > bv || (bi < 0.f && y[r] == bv))) {
-                bv = y[r];
-                bi = (float)(n0 + r);
-            }
-        if (n0 == 0 && y[0] != y[0]) {
-            bv = INFINITY;
-            bi = 0.f;
-        }
-#pragma unroll
-        for (int o = 16; o < 64; o <<= 1) {
-            const float ov = __shfl_xor(bv, o, 64), oi = __shfl_xor(bi, o, 64);
-            if (oi >= 0.f && (ov > bv || bi < 0.f || (ov == bv && oi < bi))) {
-                bv = ov;
-                bi = oi;
-            }
-        }
-        if (g == 0 && x < T) p.amax_pairs[(size_t)nb * p.amax_ld + x] = make_float2(bv, bi);
+    thin_finish<PAIR>(p, sg, x, g, nb, n0, y, u, side, row);
+}
+
+template <int NB, int KS, bool PAIR, bool NORM>
+static void launch_thin(const F32Gemm& a, int tiles) {
+    constexpr int NT = PAIR ? 2 : NB, MOST = 150 * 1024;
+    const long lds = thin_lds_bytes<NT, KS>(a.K, a.T, NORM);
+    // One or two tokens, and eight steps or more a wave: less hides the way over LDS, and more tokens are more to lay out than lanes read
+    // twice.  us a pass of TinyLlama, none and each of these this way: w_down (11 steps) 1, 2, 3, 6 tokens 1,043 -> 1,021, 1,058 -> 1,042, 1,063 -> 1,066,
+    // 1,145 -> 1,187; gate/up (8) 1,034, 1,055, 1,076, 1,194; classifier (8) 1,038, 1,056, 1,063, 1,152; q/k/v (4) 1,040, 1,054, 1,068, 1,164;
+    // wo (4) 1,069, 1,087, 1,089, 1,178; q/k/v of stories42M (1) 242 -> 254, wo and w_down 280.
+    const bool few = a.T <= 2 && a.K / 32 >= 8 * KS;
+    if (lds > MOST || !few) {
+        NVLLM_LAUNCH((k_gemm_thin<NB, KS, PAIR, NORM>), dim3(tiles), dim3(KS * 64), 0, a);
+        return;
     }
+    static bool enabled = false;
+    if (!enabled) {
+        HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_gemm_thin_lds<NB, KS, PAIR, NORM>), hipFuncAttributeMaxDynamicSharedMemorySize, MOST));
+        enabled = true;
+    }
+    NVLLM_LAUNCH((k_gemm_thin_lds<NB, KS, PAIR, NORM>), dim3(tiles), dim3(KS * 64), (int)lds, a);
 }
 
 void launch_gemm_thin(const F32Gemm& g, int prof_cls) {
@@ -218,8 +417,8 @@ void launch_gemm_thin(const F32Gemm& g, int prof_cls) {
     ProfScope ps(prof_cls, 2.0 * weights + 4.0 * a.T * (a.K + outs), 2.0 * a.T * weights);
 #define NVLLM_GEMM_THIN(nb, ks, pair_)                                                                             \
     do {                                                                                                         \
-        if (a.gain) NVLLM_LAUNCH((k_gemm_thin<nb, ks, pair_, true>), dim3(tiles), dim3((ks) * 64), 0, a);  \
-        else NVLLM_LAUNCH((k_gemm_thin<nb, ks, pair_, false>), dim3(tiles), dim3((ks) * 64), 0, a);        \
+        if (a.gain) launch_thin<nb, ks, pair_, true>(a, tiles);                                                 \
+        else launch_thin<nb, ks, pair_, false>(a, tiles);                                                       \
     } while (0)
     if (NB == 4) NVLLM_GEMM_THIN(4, 8, false);
     else if (pair) NVLLM_GEMM_THIN(1, 8, true);

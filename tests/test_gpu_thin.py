@@ -39,6 +39,16 @@ def test_few_rows(hip, oracle, tmp_path, n, kv_bytes, shape):
         assert np.abs(g["logits"] - o["logits"]).max() < (2e-4 if kv_bytes == 4 else 2e-3)
 
 
+@pytest.mark.parametrize("n", [1, 2, 3])
+@pytest.mark.parametrize("shape", [
+    dict(dim=2112, hidden_dim=4128, n_layers=1, n_heads=33, n_kv_heads=3, vocab_size=16500),   # 66 and 129 tiles of K: every wave's ring and one or two tiles more
+    dict(dim=2048, hidden_dim=4096, n_layers=1, n_heads=32, n_kv_heads=4, vocab_size=16400),   # the fewest tiles
+])
+def test_activations_laid_out_once(hip, oracle, tmp_path, n, shape):
+    """One and two rows at widths whose projections lay their activations out in LDS, and three rows, which do not."""
+    test_few_rows(hip, oracle, tmp_path, n, 4, shape)
+
+
 def batch(lib, path, kv_bytes, history, tokens, out):
     """Logits rows (and the library's token ids) of one pass of one sequence behind `history`."""
     w, cfg, st = capi.Weights(), capi.Config(), capi.RunState()
