@@ -45,9 +45,12 @@ struct F32Gemm {
     int live, touched = 1;   // for the figures of a profile: rows that are some token's, matrices they can be of
     // one STORE segment: its rows also go to this page-locked host array, laid out like its `out` (null: no)
     float* out_host = nullptr;
-    // fp16 weights, one STORE segment: (maximum, its first index) of each 16 outputs of a token -> [block][amax_ld]
+    // one STORE segment: (maximum, its first index) of each 16 outputs of a token -> [block][amax_ld] ...
     float2* amax_pairs = nullptr;
     int amax_ld = 0;
+    // ... and with them (launch_gemm_f32): every token's first index of its maximum, merged by a launch of its own; to a page-locked host array too
+    int* amax_out = nullptr;
+    int* amax_out_host = nullptr;
     // a mixture's choices and their sorting in one more workgroup, of pairs behind a norm (route.T 0: none)
     RoutePlan route{};
     const float* z = nullptr;   // router logits [T][ldz]

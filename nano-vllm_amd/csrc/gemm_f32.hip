@@ -29,7 +29,8 @@ constexpr int F32_STEP = 32;   // k per step: 128 bytes, a cache line, of every 
 // waves per SIMD the registers are dealt for: two workgroups of eight waves share a CU where the tiles allow it
 constexpr int f32_occupancy(int tiles, bool norm) { return tiles >= 6 ? 2 : tiles == 4 && norm ? 3 : 4; }
 
-template <int NB, int TB, int KS, bool PAIR, bool NORM>
+// AMAX: the classifier's, which leaves pairs (F32Gemm::amax_pairs)
+template <int NB, int TB, int KS, bool PAIR, bool NORM, bool AMAX = false>
 __global__ __launch_bounds__(KS * 64, f32_occupancy((PAIR ? 2 : 1) * NB * TB, NORM)) void k_gemm_f32(F32Gemm p) {
     constexpr int NT = PAIR ? 2 * NB : NB;   // weight blocks per step: all of the first matrix, then all of the second
     constexpr int RING = NT * TB == 1 ? (NORM ? 3 : 4) : 2;
@@ -81,7 +82,7 @@ __global__ __launch_bounds__(KS * 64, f32_occupancy((PAIR ? 2 : 1) * NB * TB, NO
     // What the epilogue needs beside the sums travels with the first steps, and angles behind their positions; where the registers
     // are full, with the last ones
     constexpr bool EARLY = PAIR || NT * TB < 4 || f32_occupancy(NT * TB, NORM) < 4;
-    const bool turns = !PAIR && (sg.kind == F32Out::ROPE_Q || sg.kind == F32Out::ROPE_K), adds = !PAIR && sg.kind == F32Out::ADD;
+    const bool turns = !PAIR && !AMAX && (sg.kind == F32Out::ROPE_Q || sg.kind == F32Out::ROPE_K), adds = !PAIR && sg.kind == F32Out::ADD;
     int at[FPT], row[FPT];
     f4_t side[FPT];   // angles, or what is added to
     auto item = [&](int q, int& t, int& n) {
@@ -96,6 +97,7 @@ __global__ __launch_bounds__(KS * 64, f32_occupancy((PAIR ? 2 : 1) * NB * TB, NO
         at[q] = turns ? p.pos[t] : 0;
     }
     auto request_side = [&] {
+        if constexpr (AMAX) return;   // (its rows are stored as they are)
 #pragma unroll
         for (int q = 0; q < FPT; q++) {
             int t, n;
@@ -249,14 +251,16 @@ __global__ __launch_bounds__(KS * 64, f32_occupancy((PAIR ? 2 : 1) * NB * TB, NO
         }
     }
     auto finish = [&](int t, int n, f4_t y, f4_t u, float sum, f4_t side, int row) {
-        if (t >= T || n >= N) return;
+        const bool live = t < T && n < N;
+        if (!AMAX && !live) return;
         float scale = NORM ? rinv_of(sum) : 1.f;
-        if (p.row_weight) scale *= p.row_weight[t];
+        if (p.row_weight) scale *= p.row_weight[AMAX ? min(t, T - 1) : t];
         if (NORM || p.row_weight) {
             y *= scale;
             if constexpr (PAIR) u *= scale;
         }
-        f32_finish<PAIR>(p, sg, t, n, y, u, side, side, row);
+        if (live) f32_finish<PAIR>(p, sg, t, n, y, u, side, side, row);
+        if constexpr (AMAX) f32_pairs(p, N, n >> 4, n, t, (n & 15) == 0 && live, y);
     };
 #pragma unroll
     for (int n = 0; n < NT; n++)
@@ -289,20 +293,20 @@ __global__ __launch_bounds__(KS * 64, f32_occupancy((PAIR ? 2 : 1) * NB * TB, NO
 #pragma unroll
             for (int v = 0; v < KS; v++) sum += s_ss[v][j * 16 + (l & 15)];
         }
-        finish((tb0 + j) * 16 + (l & 15), (nb0 + i) * 16 + 4 * (l >> 4), y, u, sum, side[q], row[q]);
+        finish((tb0 + j) * 16 + (l & 15), (nb0 + i) * 16 + 4 * (l >> 4), y, u, sum, AMAX ? zero : side[q], AMAX ? -1 : row[q]);
     }
 }
 
-template <int NB, int TB, int KS, bool PAIR, bool NORM>
+template <int NB, int TB, int KS, bool PAIR, bool NORM, bool AMAX = false>
 void launch_f32(const F32Gemm& a, dim3 grid) {
     constexpr int LDS = KS * ((PAIR ? 2 : 1) * NB * TB * 1024 + (NORM ? TB * 64 : 0));
     const int lds = (int)grid.x > a.route_from ? std::max(LDS, (int)route_sort_lds(a.route.T, a.route.E, a.route.top)) : LDS;
     static bool enabled = false;
     if (LDS > 64 * 1024 && !enabled) {
-        HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_gemm_f32<NB, TB, KS, PAIR, NORM>), hipFuncAttributeMaxDynamicSharedMemorySize, LDS));
+        HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_gemm_f32<NB, TB, KS, PAIR, NORM, AMAX>), hipFuncAttributeMaxDynamicSharedMemorySize, LDS));
         enabled = true;
     }
-    NVLLM_LAUNCH((k_gemm_f32<NB, TB, KS, PAIR, NORM>), grid, dim3(KS * 64), lds, a);
+    NVLLM_LAUNCH((k_gemm_f32<NB, TB, KS, PAIR, NORM, AMAX>), grid, dim3(KS * 64), lds, a);
 }
 
 // Rows that are no multiples of 16 bytes (K % 4 != 0, or a caller's odd pointer): a wave sums four features of four tokens,
@@ -374,8 +378,7 @@ __global__ __launch_bounds__(256) void k_gemm_f32_any(F32Gemm p) {
     }
 }
 
-bool launch_gemm_f32(const F32Gemm& g, int prof_cls) {
-    if (g.T <= 0 || g.n_segs == 0) return false;
+static bool launch_products(const F32Gemm& g, int prof_cls, bool* has_pairs) {
     F32Gemm a = g;
     const bool pair = a.seg[0].W2 != nullptr;
     double weights = 0, outs = 0;
@@ -428,10 +431,11 @@ bool launch_gemm_f32(const F32Gemm& g, int prof_cls) {
     }
     for (int s = a.n_segs; s < F32_SEGMENTS; s++) a.seg[s].first = INT_MAX;
     ProfScope ps(prof_cls, 4.0 * (weights * a.touched + (double)a.live * (a.K + outs)), 2.0 * a.live * weights);
-    if (!rows16) {
+    if (!rows16) {   // (its maxima are found in the rows)
         const dim3 grid(tiles, std::min(cdiv(a.T, 4), 32768));
         if (pair) NVLLM_LAUNCH(k_gemm_f32_any<true>, grid, dim3(256), 0, a);
         else NVLLM_LAUNCH(k_gemm_f32_any<false>, grid, dim3(256), 0, a);
+        *has_pairs = false;
         return false;
     }
     // Choices of few tokens and their sorting, by one workgroup more (route_rides)
@@ -441,7 +445,8 @@ bool launch_gemm_f32(const F32Gemm& g, int prof_cls) {
     const dim3 grid(tiles + rides, cdiv(Tb, TB));
 #define NVLLM_GEMM_F32(nb, tb, ks, pr)                                                                    \
     do {                                                                                                  \
-        if (a.gain) launch_f32<nb, tb, ks, pr, true>(a, grid);                                            \
+        if (!pr && a.gain && a.amax_out) launch_f32<nb, tb, ks, pr, true, !pr>(a, grid);                  \
+        else if (a.gain) launch_f32<nb, tb, ks, pr, true>(a, grid);                                       \
         else launch_f32<nb, tb, ks, pr, false>(a, grid);                                                  \
     } while (0)
 #define NVLLM_GEMM_F32_4_8(nb, tb, pr)                                                                    \
@@ -467,6 +472,17 @@ bool launch_gemm_f32(const F32Gemm& g, int prof_cls) {
     }
 #undef NVLLM_GEMM_F32_4_8
 #undef NVLLM_GEMM_F32
+    return rides;
+}
+
+bool launch_gemm_f32(const F32Gemm& g, int prof_cls) {
+    if (g.T <= 0 || g.n_segs == 0) return false;
+    if (g.amax_out && (!g.amax_pairs || g.amax_ld < g.T)) NVLLM_FATAL("fused arg-max needs a pair buffer of at least %d rows per block", g.T);
+    bool has_pairs = g.gain != nullptr && g.seg[0].W2 == nullptr;
+    const bool rides = launch_products(g, prof_cls, &has_pairs);
+    // one row of 32,000 scanned again 6.6 us, its 2,000 pairs merged 4.2
+    if (g.amax_out && has_pairs) launch_argmax_tiles(g.amax_out, g.amax_pairs, cdiv(g.seg[0].N, 16), g.T, g.amax_ld, g.amax_out_host);
+    else if (g.amax_out) launch_argmax_ld(g.amax_out, g.seg[0].out, g.T, g.seg[0].N, g.seg[0].ldo, g.amax_out_host);
     return rides;
 }
 

@@ -88,4 +88,30 @@ __device__ __forceinline__ f4_t f32_old(const F32Segment& sg, int t, int n) {   
     return v;
 }
 
+// The first maximum of a block's 16 features per token, by the reference's scan (sampler.c:86-97): strict >, so a NaN never wins --
+// except at index 0, which nothing displaces: +inf there wins every comparison downstream.  Lane (x, g): features n0 .. n0 + 3 of token x; the
+// whole wave comes here.
+__device__ __forceinline__ void f32_pairs(const F32Gemm& p, int N, int block, int n0, int t, bool writes, const f4_t& y) {
+    float bv = -INFINITY, bi = -1.0f;
+#pragma unroll
+    for (int r = 0; r < 4; r++)
+        if (n0 + r < N && (y[r] > bv || (bi < 0.f && y[r] == bv))) {
+            bv = y[r];
+            bi = (float)(n0 + r);
+        }
+    if (n0 == 0 && y[0] != y[0]) {
+        bv = INFINITY;
+        bi = 0.f;
+    }
+#pragma unroll
+    for (int o = 16; o < 64; o <<= 1) {
+        const float ov = __shfl_xor(bv, o, 64), oi = __shfl_xor(bi, o, 64);
+        if (oi >= 0.f && (ov > bv || bi < 0.f || (ov == bv && oi < bi))) {
+            bv = ov;
+            bi = oi;
+        }
+    }
+    if (writes) p.amax_pairs[(size_t)block * p.amax_ld + t] = make_float2(bv, bi);
+}
+
 }  // namespace nvllm

@@ -30,30 +30,7 @@ template <bool PAIR>
 __device__ __forceinline__ void thin_finish(const F32Gemm& p, const F32Segment& sg, int x, int g, int nb, int n0, const f4_t& y, const f4_t& u, const f4_t& side, int row) {
     const int T = p.T, N = sg.N;
     if (x < T && n0 < N) f32_finish<PAIR>(p, sg, x, n0, y, u, side, side, row);
-    if (!PAIR && p.amax_pairs != nullptr) {
-        // the block's first maximum per token, by the reference's scan (sampler.c:86-97): strict >, so a NaN never wins --
-        // except at index 0, which nothing displaces: +inf there wins every comparison downstream
-        float bv = -INFINITY, bi = -1.0f;
-#pragma unroll
-        for (int r = 0; r < 4; r++)
-            if (n0 + r < N && (y[r] > bv || (bi < 0.f && y[r] == bv))) {
-                bv = y[r];
-                bi = (float)(n0 + r);
-            }
-        if (n0 == 0 && y[0] != y[0]) {
-            bv = INFINITY;
-            bi = 0.f;
-        }
-#pragma unroll
-        for (int o = 16; o < 64; o <<= 1) {
-            const float ov = __shfl_xor(bv, o, 64), oi = __shfl_xor(bi, o, 64);
-            if (oi >= 0.f && (ov > bv || bi < 0.f || (ov == bv && oi < bi))) {
-                bv = ov;
-                bi = oi;
-            }
-        }
-        if (g == 0 && x < T) p.amax_pairs[(size_t)nb * p.amax_ld + x] = make_float2(bv, bi);
-    }
+    if (!PAIR && p.amax_pairs != nullptr) f32_pairs(p, N, nb, n0, x, g == 0 && x < T, y);
 }
 
 // The same with the activations in LDS, where every workgroup lays them out once, in operand order: [k tile][group of 8 k][token], the hi

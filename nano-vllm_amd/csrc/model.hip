@@ -377,7 +377,7 @@ static F32Gemm rows_qkv(const float* x, const StepArrays& st, int T, int D, cons
 // The reference's layer loop (model.c:352-418) on fp32 weights, five launches a layer: the norms, rotation, cache write,
 // SwiGLU and residual adds ride in the projections (gemm_f32.hip).  Leaves the logits of the output rows in d_logits.
 static void forward_f32(const StepArrays& st, int T, int B, Config* p, RunState* s, Weights* w, const KvPoolView& pool,
-                        const float2* rope, float* d_logits, float* logits_host) {
+                        const float2* rope, float* d_logits, float* logits_host, int* d_argmax, int* argmax_host) {
     const int D = p->dim, F = p->hidden_dim, hd = p->head_dim, H = p->n_heads, KVH = p->n_kv_heads;
     const int QD = H * hd, KD = KVH * hd, V = p->vocab_size;
     const float eps = 1e-5f;
@@ -396,6 +396,10 @@ static void forward_f32(const StepArrays& st, int T, int B, Config* p, RunState*
     F32Gemm head = F32Gemm(s->x, B, D).norm(w->rms_final_weight, eps);
     head.in_rows = st.d_out_idx;
     head.out_host = logits_host;
+    head.amax_out = d_argmax;
+    head.amax_out_host = argmax_host;
+    head.amax_ld = B;
+    head.amax_pairs = (float2*)ws_get(WS_AMAX_PAIRS, (size_t)cdiv(V, 16) * std::max(B, 1) * sizeof(float2));
     if (B > 0) launch_gemm_f32(head.add(w->lm_head, V, d_logits), PC_GEMM_HEAD);
 }
 
@@ -812,8 +816,7 @@ static long enqueue_pass(int* tokens, int num_tokens, int* pos_arr, int* seq_ids
         if (st.d_tok_src) launch_patch_tokens(st.d_tokens, st.d_tok_src, d_argmax, T);
         wait_for_row_copies();
         float* rows = direct_rows(s, B, V, waits);
-        forward_f32(st, T, B, p, s, w, pool, rope, d_logits, rows);
-        if (B > 0) launch_argmax_ld(d_argmax, d_logits, B, V, V, argmax_direct() ? next_slot(B).host : nullptr);
+        forward_f32(st, T, B, p, s, w, pool, rope, d_logits, rows, d_argmax, argmax_direct() && B > 0 ? next_slot(B).host : nullptr);
         return finish_pass(s, d_logits, d_argmax, B, V, PassView{}, waits, false, argmax_direct(), rows != nullptr);
     }
 
@@ -951,7 +954,7 @@ static long enqueue_pass(int* tokens, int num_tokens, int* pos_arr, int* seq_ids
         e5.amax_out = d_argmax;
         host_written = argmax_direct() && !chained;
         if (host_written) e5.amax_out_host = next_slot(B).host;
-        e5.amax_ld = (B + 63) & ~63;
+        e5.amax_ld = B;   // (few rows' pairs side by side: lanes that merge them read lines, not one line each)
         e5.amax_pairs = (float2*)ws_get(WS_AMAX_PAIRS, (size_t)cdiv(V, 16) * e5.amax_ld * sizeof(float2));
         if (thin_head) {
             F32Gemm head = F32Gemm(s->x, B, D).norm(m->rms_final, eps);
