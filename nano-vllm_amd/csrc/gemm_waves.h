@@ -91,7 +91,7 @@ __global__ __launch_bounds__(256, 1) void k_gemm_waves(GemmArgs p, int tiles_n, 
     for (int f = 0; f < FB; f++)
 #pragma unroll
         for (int j = 0; j < TBN; j++) acc[f][j] = f4_t{0.f, 0.f, 0.f, 0.f};
-    // (in front of the first steps, which would be waited for with it; added up while they travel)
+    // (in front of the first steps, which would be waited for with it; added up while they travel: q/k/v of Simivik at 1,029 tokens 23.5 -> 22.4 us)
     TileRinv<16 * TBN, 256> rinv;
     if (p.e.ss_in != nullptr) rinv.request(p, tb0);
 #pragma unroll
