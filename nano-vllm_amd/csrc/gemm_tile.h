@@ -285,38 +285,29 @@ __device__ __forceinline__ bool gemm_tile(const GemmArgs& p, const TileIdx ix, u
     };
 
     const GemmEpilogue& ep = p.e;
-    // What the epilogue needs beside the sums is requested behind the first steps and waited for behind the last:
-    // 1/rms of this token group from the producer's per-tile sums of squares: every thread sums a slice of one token's tiles (up to
-    // SS_HELD of them held in registers over the K loop); the slices meet in LDS before the epilogue.  (Summed in front of the loop, each
-    // load waited for all before it: two to sixteen trips to memory before the first product.)
+    // 1/rms of this token group comes from the producer's per-tile sums of squares: every thread sums a slice of one token's tiles; the slices
+    // meet in LDS before the epilogue.  Up to SS_HELD of them are requested behind the first steps and held in registers over the K loop.  (Summed in
+    // front of it, each load waited for all before it: two to sixteen trips to memory before the first product.)  The one-launch step, whose
+    // registers hold the next tile's weights, sums them beside the first steps.
     constexpr int SS_HELD = PARTS < 64 ? 64 / PARTS : 1;
     float ss_held[SS_HELD];
     const float* ss_row = nullptr;
     const int ss_tl = tid / PARTS, ss_part = tid % PARTS;   // (lanes side by side read one token's sums: a line, and not one line each)
+    // What the epilogue needs beside the sums: requested behind the first steps and waited for behind the last.  In the one-launch step behind the
+    // last: held over the loop they made it spill (64 tokens: 230 registers -> 256 and 58 more in scratch)
     float4 pf_x[FPT], pf_g[FPT];
     int pf_pos = 0, pf_row = -1;
     f4_t pf_turn[FPT];
     __amdgpu_buffer_rsrc_t rs_x = gemm_rsrc(ep.x, (unsigned)p.T * (unsigned)p.N * 4u);
-    if (EPI == GemmEpilogue::ROPE_KV) {   // all items of a thread belong to one token (NW*64 is a multiple of TB*64)
-        const int e = min(tid, WITEMS - 1) & (ITEMS - 1);
-        const int t = min(tb0 * 16 + ((e >> 6) % TB) * 16 + (e & 15), p.T - 1);
-        pf_pos = ep.pos[t];
-        pf_row = ep.kv_row[t];
-    }
-    auto request_side = [&] {
-        if (ep.ss_in != nullptr) {
-            const int t = min(tb0 * 16 + ss_tl, p.T - 1);
-            int src = t;
-            if (ep.ss_gather) {
-                src = ep.ss_gather[t];
-                asm volatile("" ::"v"(src));
-            }
-            ss_row = ep.ss_in + (size_t)src * ep.ss_tiles;
-            if constexpr (!COH) {
-#pragma unroll
-                for (int q = 0; q < SS_HELD; q++) ss_held[q] = ss_row[min(ss_part + q * PARTS, ep.ss_tiles - 1)];
-            }
+    auto request_positions = [&] {
+        if (EPI == GemmEpilogue::ROPE_KV) {   // all items of a thread belong to one token (NW*64 is a multiple of TB*64)
+            const int e = min(tid, WITEMS - 1) & (ITEMS - 1);
+            const int t = min(tb0 * 16 + ((e >> 6) % TB) * 16 + (e & 15), p.T - 1);
+            pf_pos = ep.pos[t];
+            pf_row = ep.kv_row[t];
         }
+    };
+    auto request_operands = [&] {
 #pragma unroll
         for (int s = 0; s < FPT; s++) {
             const int w_ = min(tid + s * NW * 64, WITEMS - 1);
@@ -335,16 +326,66 @@ __device__ __forceinline__ bool gemm_tile(const GemmArgs& p, const TileIdx ix, u
             if (EPI == GemmEpilogue::ROPE_KV) pf_turn[s] = *reinterpret_cast<const f4_t*>(ep.rope + (size_t)pf_pos * (ep.hd >> 1) + ((n0 % ep.hd) >> 1));
         }
     };
+    if constexpr (!COH) request_positions();
+    auto request_side = [&] {
+        if (ep.ss_in != nullptr) {
+            const int t = min(tb0 * 16 + ss_tl, p.T - 1);
+            int src = t;
+            if (ep.ss_gather) {
+                src = ep.ss_gather[t];
+                asm volatile("" ::"v"(src));
+            }
+            ss_row = ep.ss_in + (size_t)src * ep.ss_tiles;
+            if constexpr (COH) {
+                float ss = 0.f;
+                for (int j = ss_part; j < ep.ss_tiles; j += PARTS)
+                    ss += __builtin_bit_cast(float, __hip_atomic_load(reinterpret_cast<const unsigned*>(ss_row + j), __ATOMIC_RELAXED,
+                                                                      __HIP_MEMORY_SCOPE_AGENT));
+                s_part[ss_part][ss_tl] = ss;
+            } else {
+#pragma unroll
+                for (int q = 0; q < SS_HELD; q++) ss_held[q] = ss_row[min(ss_part + q * PARTS, ep.ss_tiles - 1)];
+            }
+        }
+        if constexpr (!COH) request_operands();
+    };
 
     // Loads are issued only for steps that exist: a clamped re-load of the last tile would be real HBM traffic, since streamed
-    // weights are loaded non-temporally and do not stay in L2.  The steady loop requests without a condition: where paths with and
-    // without requests meet, the compiler waits for all of them.
-    const bool mine = PRE == 0 || (PRE == 2 && !prefetched);   // whether the first weights are requested here
-    if (nsteps < RW) {
+    // weights are loaded non-temporally and do not stay in L2.
+    if constexpr (COH) {
+        // (requests under conditions, each waited for with all before it: with the loop below the one-launch step needs 26 to 56 registers more)
+        if (PRE == 0 || (PRE == 2 && !prefetched)) {
+#pragma unroll
+            for (int s = 0; s < RW; s++)
+                if (s < nsteps) load_w(s, s);
+        }
+#pragma unroll
+        for (int s = 0; s < RA; s++)
+            if (s < nsteps) load_a(s, s);
+        request_side();
+        NVLLM_TSTAMP(1, lane);
+        for (int s0 = 0; s0 < nsteps; s0 += RW) {
+#pragma unroll
+            for (int r = 0; r < RW; r++) {
+                const int s = s0 + r;
+                if (s < nsteps) {
+                    multiply(r);
+                    if (s == 0) NVLLM_TSTAMP(2, acc[NBW - 1][TB - 1][0]);
+                    if (s + RW < nsteps) load_w(r, s + RW);
+                    else slot_free(r);
+                    if (s + RA < nsteps) load_a(r % RA, s + RA);
+                }
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < RW; r++)
+            if (r >= nsteps) slot_free(r);   // entries a short K slice never used
+    } else if (nsteps < RW) {
+        static_assert(PRE == 0);
 #pragma unroll
         for (int s = 0; s + 1 < RW; s++)
             if (s < nsteps) {
-                if (mine) load_w(s, s);
+                load_w(s, s);
                 if (s < RA) load_a(s, s);
             }
         request_side();
@@ -359,16 +400,15 @@ __device__ __forceinline__ bool gemm_tile(const GemmArgs& p, const TileIdx ix, u
             }
 #pragma unroll
         for (int r = 0; r < RW; r++)
-            if (r >= nsteps) slot_free(r);   // entries a short K slice never used
+            if (r >= nsteps) slot_free(r);
     } else {
-        if constexpr (RA == RW && PRE == 0) {
+        // The steady loop requests without a condition: where paths with and without requests meet, the compiler waits for all of them.
+        if constexpr (RA == RW) {
 #pragma unroll
             for (int r = 0; r < RW; r++) load(r, r);
         } else {
-            if (mine) {
 #pragma unroll
-                for (int r = 0; r < RW; r++) load_w(r, r);
-            }
+            for (int r = 0; r < RW; r++) load_w(r, r);
 #pragma unroll
             for (int r = 0; r < RA; r++) load_a(r, r);
         }
@@ -404,20 +444,16 @@ __device__ __forceinline__ bool gemm_tile(const GemmArgs& p, const TileIdx ix, u
             }
     }
     NVLLM_TSTAMP(3, acc[NBW - 1][TB - 1][0]);
-    if (ep.ss_in != nullptr) {
+    if constexpr (COH) {
+        request_positions();
+        request_operands();
+    } else if (ep.ss_in != nullptr) {
         float ss = 0.f;
-        int j = ss_part;
-        if constexpr (COH) {
-            for (; j < ep.ss_tiles; j += PARTS)
-                ss += __builtin_bit_cast(float, __hip_atomic_load(reinterpret_cast<const unsigned*>(ss_row + j), __ATOMIC_RELAXED,
-                                                                  __HIP_MEMORY_SCOPE_AGENT));
-        } else {
 #pragma unroll
-            for (int q = 0; q < SS_HELD; q++)
-                if (ss_part + q * PARTS < ep.ss_tiles) ss += ss_held[q];
+        for (int q = 0; q < SS_HELD; q++)
+            if (ss_part + q * PARTS < ep.ss_tiles) ss += ss_held[q];
 #pragma unroll 4
-            for (j += SS_HELD * PARTS; j < ep.ss_tiles; j += PARTS) ss += ss_row[j];
-        }
+        for (int j = ss_part + SS_HELD * PARTS; j < ep.ss_tiles; j += PARTS) ss += ss_row[j];
         s_part[ss_part][ss_tl] = ss;
     }
     // ---- 0. epilogue operands that do not depend on the sums and are too many to be held over the K loop: issue their loads now,
@@ -449,7 +485,7 @@ __device__ __forceinline__ bool gemm_tile(const GemmArgs& p, const TileIdx ix, u
         for (int j = 0; j < TB; j++) red[wave][i][j][lane] = acc[i][j];
     __syncthreads();
     if (ep.ss_in != nullptr && tid < TB * 16) {
-        // 1/rms per token from the slices gathered at the top (s_part: visible since the barrier
+        // 1/rms per token from its slices' sums (s_part: visible since the barrier
         // above; s_rinv is read by the epilogue after at least one more barrier)
         float ss = 0.f;
 #pragma unroll
