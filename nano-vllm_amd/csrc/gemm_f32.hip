@@ -80,7 +80,7 @@ __global__ __launch_bounds__(KS * 64, f32_occupancy((PAIR ? 2 : 1) * NB * TB, NO
     const float* gp = NORM ? p.gain + 4 * g : nullptr;
 
     // What the epilogue needs beside the sums travels with the first steps, and angles behind their positions; where the registers
-    // are full, with the last ones
+    // are full (2 x 2 blocks at four waves a SIMD), behind the last
     constexpr bool EARLY = PAIR || NT * TB < 4 || f32_occupancy(NT * TB, NORM) < 4;
     const bool turns = !PAIR && !AMAX && (sg.kind == F32Out::ROPE_Q || sg.kind == F32Out::ROPE_K), adds = !PAIR && sg.kind == F32Out::ADD;
     int at[FPT], row[FPT];
@@ -90,14 +90,18 @@ __global__ __launch_bounds__(KS * 64, f32_occupancy((PAIR ? 2 : 1) * NB * TB, NO
         t = min((tb0 + (e >> 6) % TB) * 16 + (l & 15), T - 1);
         n = (nb0 + (e >> 6) / TB) * 16 + 4 * (l >> 4);
     };
+    auto request_positions = [&] {
 #pragma unroll
-    for (int q = 0; q < FPT; q++) {
-        int t, n;
-        item(q, t, n);
-        at[q] = turns ? p.pos[t] : 0;
-    }
+        for (int q = 0; q < FPT; q++) {
+            int t, n;
+            item(q, t, n);
+            at[q] = turns ? p.pos[t] : 0;
+        }
+    };
+    if constexpr (EARLY) request_positions();
     auto request_side = [&] {
         if constexpr (AMAX) return;   // (its rows are stored as they are)
+        if constexpr (!EARLY) request_positions();
 #pragma unroll
         for (int q = 0; q < FPT; q++) {
             int t, n;
@@ -222,7 +226,6 @@ __global__ __launch_bounds__(KS * 64, f32_occupancy((PAIR ? 2 : 1) * NB * TB, NO
         for (int r = 0; r < RING; r++)
             if (i0 + r + RING < mine) multiply(r);
     }
-    if constexpr (!EARLY) request_side();
     if (whole * F32_STEP < K && whole % KS == wave) {   // the rest of K (K % 4 == 0: a lane's four are in or out together)
         const int k = whole * F32_STEP;
 #pragma unroll
@@ -262,6 +265,7 @@ __global__ __launch_bounds__(KS * 64, f32_occupancy((PAIR ? 2 : 1) * NB * TB, NO
         if (live) f32_finish<PAIR>(p, sg, t, n, y, u, side, side, row);
         if constexpr (AMAX) f32_pairs(p, N, n >> 4, n, t, (n & 15) == 0 && live, y);
     };
+    if constexpr (!EARLY) request_side();
 #pragma unroll
     for (int n = 0; n < NT; n++)
 #pragma unroll

@@ -20,7 +20,6 @@ SPILLS = {
     "k_gemm_prefill<4, 1, 9, float, 2, 4, OpBf16, false, false>": 36,
     "k_window_attn<8, 16, 1, true, 2, false>": 14,
     "k_lightning_out<8>": 131,
-    "k_gemm_f32<2, 2, 4, false, false, false>": 2,
 }
 # and kernels whose next step's operands live in registers across this one's: at most these many registers
 REGISTERS = {
