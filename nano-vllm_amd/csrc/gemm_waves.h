@@ -92,8 +92,11 @@ __global__ __launch_bounds__(256, 1) void k_gemm_waves(GemmArgs p, int tiles_n, 
 #pragma unroll
         for (int j = 0; j < TBN; j++) acc[f][j] = f4_t{0.f, 0.f, 0.f, 0.f};
     // (in front of the first steps, which would be waited for with it; added up while they travel: q/k/v of Simivik at 1,029 tokens 23.5 -> 22.4 us)
+    // Hyper-connection updates follow products of activations that nothing scales: those tiles keep no registers for it (six blocks 16 spilled
+    // registers with them, 8 without).
+    constexpr bool SCALED = hyper_streams(EPI) == 0;
     TileRinv<16 * TBN, 256> rinv;
-    if (p.e.ss_in != nullptr) rinv.request(p, tb0);
+    if (SCALED && p.e.ss_in != nullptr) rinv.request(p, tb0);
 #pragma unroll
     for (int r = 0; r < RING; r++) {
         const auto rw = operand(W, r < mine), ra = operand(A, r < mine);
@@ -105,7 +108,7 @@ __global__ __launch_bounds__(256, 1) void k_gemm_waves(GemmArgs p, int tiles_n, 
         __builtin_amdgcn_sched_barrier(0);
         next_step();
     }
-    if (p.e.ss_in != nullptr) rinv.finish(p, s_rinv);
+    if (SCALED && p.e.ss_in != nullptr) rinv.finish(p, s_rinv);
 
     // Step i out of registers r, each replaced by step i + RING's as soon as it has been multiplied.  The loop has one exit and
     // no condition around a request: where paths with and without requests meet, the compiler waits for all of them.
@@ -170,6 +173,7 @@ template <int TBN, int EPI, typename KVT, typename OP>
 bool launch_waves(GemmArgs a, int tiles_n, int tiles_t) {   // whether a.route rode
     constexpr int NEED = 1024 + 16 * TBN * 1024, LDS = EPI == GemmEpilogue::SWIGLU_A16 && waves_carry_route(TBN, EPI, OP::PLANES) ? std::max(NEED, ROUTER_RIDE_LDS) : NEED;
     static_assert(LDS <= 160 * 1024, "the waves' sums must fit the CU's LDS");
+    if (hyper_streams(EPI) && a.e.ss_in) NVLLM_FATAL("hyper-connection updates take activations that are not scaled by token");
     static bool enabled = false;
     if (!enabled) {
         HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_gemm_waves<TBN, EPI, KVT, OP>), hipFuncAttributeMaxDynamicSharedMemorySize, LDS));

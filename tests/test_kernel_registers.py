@@ -15,8 +15,8 @@ MAGIC = b"__CLANG_OFFLOAD_BUNDLE__"
 
 # kernels that fill every register and spill some: at most these many of them
 SPILLS = {
-    "k_gemm_waves<6, 9, float, OpBf16>": 16,
-    "k_gemm_waves<7, 9, float, OpBf16>": 68,
+    "k_gemm_waves<6, 9, float, OpBf16>": 8,
+    "k_gemm_waves<7, 9, float, OpBf16>": 60,
     "k_gemm_prefill<4, 1, 9, float, 2, 4, OpBf16, false, false>": 36,
     "k_window_attn<8, 16, 1, true, 2, false>": 14,
     "k_lightning_out<8>": 131,
