@@ -42,14 +42,14 @@
 
 namespace nvllm {
 
-// One workgroup = one tile (gemm_tile.h); rings of RW K-steps of weights and activations.
+// One workgroup = one tile (gemm_tile.h); RW K-steps of weights in flight.
 template <int NBW, int TB, int NW, int EPI, typename KVT, int RW = gemm_ring(NBW, TB, 2, EPI)>
 __global__ __launch_bounds__(NW * 64) void k_gemm(GemmArgs p) {
     request_arguments<sizeof(GemmArgs)>();
     extern __shared__ __attribute__((aligned(16))) unsigned char lds_dyn[];
     h8_t w[RW][NBW];
     const TileIdx ix{(int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z, (int)gridDim.x};
-    gemm_tile<NBW, TB, NW, RW, gemm_ring_act(NBW, TB, RW), EPI, KVT, false, 0>(p, ix, lds_dyn, w, [](int) {}, (int)threadIdx.x);
+    gemm_tile<NBW, TB, NW, RW, gemm_ring_act(NBW, TB, 2, EPI), EPI, KVT, false, 0>(p, ix, lds_dyn, w, [](int) {}, (int)threadIdx.x);
 }
 
 // ------------------------------------------------------------------ launch

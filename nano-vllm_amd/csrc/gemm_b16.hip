@@ -23,10 +23,10 @@ __global__ __launch_bounds__(WAVES * 64) void k_gemm_b16(GemmArgs p) {
             return;
         }
     }
-    constexpr int RW = gemm_ring(NBW, TB, 1, EPI);
+    constexpr int RW = gemm_ring(NBW, TB, 1, EPI, GRP);
     h8_t w[RW][NBW];
     const TileIdx ix{(int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z, EPI == GemmEpilogue::LATENT_Q ? p.ride_from : (int)gridDim.x};
-    gemm_tile<NBW, TB, WAVES, RW, gemm_ring_act(NBW, TB, RW), EPI, float, false, 0, OpBf16, GRP, EXP>(p, ix, lds_dyn, w, [](int) {}, (int)threadIdx.x);
+    gemm_tile<NBW, TB, WAVES, RW, gemm_ring_act(NBW, TB, 1, EPI, GRP), EPI, float, false, 0, OpBf16, GRP, EXP>(p, ix, lds_dyn, w, [](int) {}, (int)threadIdx.x);
 }
 
 // The same with a mixture's router (SWIGLU_A16) or its choices (F32) in the workgroups from ride_from on (moe.h).  Each is a launch of
@@ -63,7 +63,7 @@ __global__ __launch_bounds__(NW * 64) void k_gemm_b16_moe(GemmArgs p, MoeRide r)
     constexpr int RW = gemm_ring(NBW, TB, 1, EPI);
     h8_t w[RW][NBW];
     const TileIdx ix{(int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z, p.ride_from};
-    gemm_tile<NBW, TB, NW, RW, gemm_ring_act(NBW, TB, RW), EPI, float, false, 0, OpBf16, false, false>(p, ix, lds_dyn, w, [](int) {}, (int)threadIdx.x);
+    gemm_tile<NBW, TB, NW, RW, gemm_ring_act(NBW, TB, 1, EPI), EPI, float, false, 0, OpBf16, false, false>(p, ix, lds_dyn, w, [](int) {}, (int)threadIdx.x);
 }
 template <int NBW, int TB, int EPI>
 void launch_stream_moe(const GemmArgs& a, const MoeRide& r, int riders, const GemmPlan& pl) {

@@ -35,20 +35,38 @@ struct TileIdx {
     int gx;        // feature tiles per token group (grid width, padding included)
 };
 
-// K-steps of weights and of activations in flight per wave.  Loads return in the order of their requests, so weights are in flight
-// no further ahead than the activations asked for behind them, and a CU takes no more in for more requests: what is in flight beyond the
-// trip's length queues.  us a launch of 64 rows at the widths of the 1.2B designs, rings of both of 2 / 3 / 4 / 5 / 7, and weights 4 with
-// activations 2: 64 x 32 tiles of a K split (w_down) 12.8 / 12.9 / 12.8 / 13.0 / 14.7 and 12.6 in fp16, 12.6 / 12.4 / 12.4 / 12.4 / 12.6 and 11.5 in
-// bf16; without one (the shared expert's) 12.0 / 12.6 / 13.3 / 13.1 / 13.6 and 13.4.  32 x 32 tiles with 4 and 8: 9.6 and 9.2 (LATENT_Q), 13.9 and
-// 15.5, 15.7 and 17.5; 32 x 16 tiles with 4 and 8: 7.2 and 6.6 (wo of Simivik).  64 x 16 tiles of experts 43.4 with 4 and 2 -> 39.3 with 4 of both; a
-// classifier of up to 16 rows has 3, so that two workgroups share a CU.  (Before, a wait for everything in flight stood in every step.)
-constexpr int gemm_ring(int NBW, int TB, int planes, int epi) {
-    if (NBW == 2) return TB == 1 ? 8 : 4;
+// K-steps of weights and of activations in flight per wave.  Loads return in the order of their requests, so weights are in flight no
+// further ahead than the activations asked for behind them, and a CU takes no more in for more requests: what is in flight beyond the trip's
+// length queues.  Most rings are of one length; four steps of weights and two of activations hold fewer registers, which is faster where
+// 64 features meet 32 tokens or the steps are few.  us a launch at the widths of TinyLlama and of the 1.2B designs, 64 rows unless said, with
+// a wait for everything in flight in every step (weights 4, activations 2) | weights 4, activations 2 | 3 of both | 4 of both | others:
+//   features x tokens                two planes                                   one plane
+//   32 x 16  wo                      7.6 | 7.5 | 7.6 | - | 6: 7.7, 8: 7.9         7.1 | 7.4 | 7.2 | - | 6: 6.7, 8: 6.7
+//            wo of stories42M, 32    5.2 | 4.9 | 5.2 | - | 6: 5.1, 8: 5.1
+//   32 x 32  q/k/v                   10.3 | 9.6 | 9.8 | 9.8                       13.7 | 13.1 | 12.8 | 12.6
+//   64 x 16  w_down, 9 rows          8.9 | 8.4 | 8.2 | 8.4                        experts' gate/up 43.3 | 40.8 | 40.6 | 39.4
+//            classifier, 9 rows      44.2 | 44.8 | 43.0 | 44.5
+//   64 x 32  w_down (RESID)          12.6 | 12.5 | 12.9 | 12.9                    11.7 | 11.5 | 12.2 | 12.0
+//            w_down (HYPER)                                                       12.1 | 12.4 | 12.4 | 12.0
+//            gate/up 32 rows, shared expert's w_down (F32)
+//                                    15.7 | 14.5 | 14.9 | 14.7 | 2: 14.5          12.3 | 13.7 | 13.2 | 13.2 | 2: 11.9
+//   96 x 32  gate/up                 17.2 | 16.8 | 16.9 | 16.3                    15.4 | 15.2 | 15.5 | 15.3
+//   64 x 64  classifier              177 | 176 | 175 | spills | 2: 174            175 | 175 | 173 | - | 2: 173
+//            gate/up                 9.7 | 10.1 | 9.9 | spills | 2: 9.3           14.4 | 12.9 | 12.7 | - | 2: 13.4
+//            products by head (K 64)                                              4.8 | 5.1 | 5.4 | - | 2: 5.3
+// (Two runs of one build differ by 0.1 to 0.3.  The products by head take 5.3 with the old wait too, behind the launch of 32 x 32 tiles that
+// ends 0.5 sooner now.)
+constexpr int gemm_ring(int NBW, int TB, int planes, int epi, bool groups = false) {
+    if (NBW == 2) return TB == 1 && planes == 1 ? 8 : 4;
     if (NBW == 4 && TB == 2) return epi == GemmEpilogue::F32 || epi == GemmEpilogue::SWIGLU_A16 ? 2 : 4;
-    if (TB == 4) return planes == 2 ? 2 : 3;
-    return planes == 2 && NBW == 4 && TB == 1 && epi == GemmEpilogue::F32 ? 3 : 4;
+    if (TB == 4) return planes == 2 ? 2 : groups ? 4 : 3;
+    return planes == 2 && NBW == 4 && TB == 1 && epi == GemmEpilogue::F32 ? 3 : 4;   // (a classifier of up to 16 rows: two workgroups share a CU)
 }
-constexpr int gemm_ring_act(int NBW, int TB, int ring) { return NBW == 4 && TB == 2 ? 2 : ring; }
+constexpr int gemm_ring_act(int NBW, int TB, int planes, int epi, bool groups = false) {
+    const int ring = gemm_ring(NBW, TB, planes, epi, groups);
+    const bool narrow = NBW == 2 && TB == 1 && planes == 2, wide = NBW == 4 && TB == 2 && hyper_streams(epi) == 0, by_group = TB == 4 && ring == 4;
+    return narrow || wide || by_group ? 2 : ring;
+}
 
 // bytes of dynamic LDS a tile needs: the waves' partial tiles, then four small arrays
 template <int NBW, int TB, int NW>

@@ -12,6 +12,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("T", [9, 20, 40, 59])   # one, two and four token blocks a tile, the last of them ragged
 @pytest.mark.parametrize("shape", [
     dict(dim=192, hidden_dim=480, n_heads=3, n_kv_heads=3),       # 6 and 15 tiles of K for eight waves
+    dict(dim=1056, hidden_dim=992, n_heads=33, n_kv_heads=3),     # four steps a wave and five, three and four
     dict(dim=2048, hidden_dim=2304, n_heads=32, n_kv_heads=4),    # eight steps a wave, nine
     dict(dim=2112, hidden_dim=2368, n_heads=33, n_kv_heads=3),    # eight or nine; 66 sums of squares
 ])
