@@ -38,14 +38,14 @@ __device__ __forceinline__ void thin_finish(const F32Gemm& p, const F32Segment& 
 // norm (every lane its operand, whichever of the 16 columns is alive).  The activations are asked for first (loads return in order), the ring of
 // weights behind them.  w_down of TinyLlama at one token: the products are done 5.9 us after the first workgroup's start instead of 7.8, the
 // launch after 8.0 instead of 8.9; what is left is its 23 MB, 4.6 us of them, behind a start of 1.1, the slowest wave's issue and layout, and two meetings.
-constexpr int thin_lds_ring(int NT) { return NT == 1 ? 8 : NT == 2 ? 6 : 3; }
+constexpr int thin_lds_ring(int NT) { return NT == 1 ? 8 : 6; }
 template <int NT, int KS>
 constexpr int thin_lds_bytes(int K, int T, bool norm) { return KS * NT * 1024 + K * T * 4 + (norm ? T * (K / 32) * 4 : 0); }
-template <int NB, int KS, bool PAIR, bool NORM>
-__global__ __launch_bounds__(KS * 64) void k_gemm_thin_lds(F32Gemm p) {
-    static_assert(!PAIR || NB == 1, "a pair is one block of either matrix");
-    static_assert(NB <= KS, "a wave finishes a block");
-    constexpr int NT = PAIR ? 2 : NB, RING = thin_lds_ring(NT), THREADS = KS * 64, LAP = 4;
+constexpr int THIN_LAP = 4;   // activations: items of four k of a token that a thread requests together
+constexpr int THIN_LDS_MOST = 84 * 1024;   // what launch_thin's rule comes to: 16 waves' sums, a lap of 16,384 values and their sums of squares
+template <int KS, bool PAIR, bool NORM>
+__global__ __launch_bounds__(KS * 64) void k_gemm_thin_lds(F32Gemm p) {   // a block, or one of either matrix, a workgroup
+    constexpr int NT = PAIR ? 2 : 1, RING = thin_lds_ring(NT), THREADS = KS * 64, LAP = THIN_LAP;
     request_arguments<sizeof(F32Gemm)>();
     extern __shared__ __attribute__((aligned(16))) unsigned char lds_thin[];
     f4_t(*s_red)[NT][64] = reinterpret_cast<f4_t(*)[NT][64]>(lds_thin);   // [wave]
@@ -54,12 +54,12 @@ __global__ __launch_bounds__(KS * 64) void k_gemm_thin_lds(F32Gemm p) {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int x = lane & 15, g = lane >> 4;
     const F32Segment& sg = p.seg[f32_segment(p, (int)blockIdx.x)];
-    const int nb0 = ((int)blockIdx.x - sg.first) * NB;
-    const int K = p.K, T = p.T, N = sg.N, blocks = (N + 15) >> 4, Kb = K >> 5, K4 = K >> 2;
+    const int nb = (int)blockIdx.x - sg.first;
+    const int K = p.K, T = p.T, Kb = K >> 5, K4 = K >> 2;
     float* s_sq = reinterpret_cast<float*>(s_act + 2 * (size_t)K * T);   // NORM: [token][32 k]
     const int tx = min(x, T - 1);   // columns past the last token compute it again and are not stored
-    const int nb = nb0 + (PAIR ? 0 : wave), n0 = nb * 16 + 4 * g;   // of the block this wave finishes
-    const bool turns = !PAIR && wave < NB && (sg.kind == F32Out::ROPE_Q || sg.kind == F32Out::ROPE_K), adds = !PAIR && wave < NB && sg.kind == F32Out::ADD;
+    const int n0 = nb * 16 + 4 * g;
+    const bool finishes = wave == 0, turns = !PAIR && finishes && (sg.kind == F32Out::ROPE_Q || sg.kind == F32Out::ROPE_K), adds = !PAIR && finishes && sg.kind == F32Out::ADD;
     const int at = turns ? p.pos[tx] : 0;
 
     // activations: item i is four k of a token, LAP of a thread at a time
@@ -125,11 +125,8 @@ __global__ __launch_bounds__(KS * 64) void k_gemm_thin_lds(F32Gemm p) {
     // weights: a step past the wave's last is requested through a descriptor of length zero: no traffic, and no branch around a request
     const int mine = wave < Kb ? (Kb - wave + KS - 1) / KS : 0;
     h8_t w[RING][NT];
-    const __half* W = reinterpret_cast<const __half*>(sg.W) + (size_t)nb0 * sg.nb_stride;
-    const __half* W2 = PAIR ? reinterpret_cast<const __half*>(sg.W2) + (size_t)nb0 * sg.nb_stride : nullptr;
-    unsigned of_w[NT];
-#pragma unroll
-    for (int n = 0; n < NT; n++) of_w[n] = PAIR ? 0u : (unsigned)min(n, blocks - 1 - nb0) * (unsigned)(sg.nb_stride * sizeof(__half));
+    const __half* W = reinterpret_cast<const __half*>(sg.W) + (size_t)nb * sg.nb_stride;
+    const __half* W2 = PAIR ? reinterpret_cast<const __half*>(sg.W2) + (size_t)nb * sg.nb_stride : nullptr;
     auto load = [&](int r, int i) {
         const int bytes = i < mine ? 0x7fffffff : 0;
         const auto from = __builtin_amdgcn_make_buffer_rsrc(const_cast<__half*>(W), 0, bytes, 0x00020000);
@@ -138,7 +135,7 @@ __global__ __launch_bounds__(KS * 64) void k_gemm_thin_lds(F32Gemm p) {
         __builtin_amdgcn_sched_barrier(0);   // requests stay in the order of their use: waits count what is younger
 #pragma unroll
         for (int n = 0; n < NT; n++)
-            w[r][n] = __builtin_bit_cast(h8_t, __builtin_amdgcn_raw_buffer_load_b128(PAIR && n == 1 ? from2 : from, lane * 16, step + of_w[n], /*nt*/ 2));
+            w[r][n] = __builtin_bit_cast(h8_t, __builtin_amdgcn_raw_buffer_load_b128(n == 1 ? from2 : from, lane * 16, step, /*nt*/ 2));
         __builtin_amdgcn_sched_barrier(0);
     };
 #pragma unroll
@@ -151,7 +148,7 @@ __global__ __launch_bounds__(KS * 64) void k_gemm_thin_lds(F32Gemm p) {
     // what the epilogue needs beside the sums travels with the first tiles
     f4_t side = {0.f, 0.f, 0.f, 0.f};   // angles, or what is added to
     int row = -1;
-    if (!PAIR && wave < NB) row = f32_row(p, sg, tx);
+    if (!PAIR && finishes) row = f32_row(p, sg, tx);
     if (turns) side = *reinterpret_cast<const f4_t*>(p.rope + (size_t)at * (p.hd >> 1) + ((n0 % p.hd) >> 1));
     else if (adds) side = f32_old(sg, tx, n0);
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // (not for the weights in flight)
@@ -182,10 +179,10 @@ __global__ __launch_bounds__(KS * 64) void k_gemm_thin_lds(F32Gemm p) {
 #pragma unroll
     for (int n = 0; n < NT; n++) s_red[wave][n][lane] = hi[n] + lo[n];
     __syncthreads();
-    if (wave >= NB || nb >= blocks) return;
-    f4_t y = s_red[0][PAIR ? 0 : wave][lane], u = zero;
+    if (!finishes) return;
+    f4_t y = s_red[0][0][lane], u = zero;
 #pragma unroll
-    for (int q = 1; q < KS; q++) y += s_red[q][PAIR ? 0 : wave][lane];
+    for (int q = 1; q < KS; q++) y += s_red[q][0][lane];
     if constexpr (PAIR) {
         u = s_red[0][1][lane];
 #pragma unroll
@@ -348,23 +345,33 @@ __global__ __launch_bounds__(KS * 64) void k_gemm_thin(F32Gemm p) {
 
 template <int NB, int KS, bool PAIR, bool NORM>
 static void launch_thin(const F32Gemm& a, int tiles) {
-    constexpr int NT = PAIR ? 2 : NB, MOST = 150 * 1024;
-    const long lds = thin_lds_bytes<NT, KS>(a.K, a.T, NORM);
-    // One or two tokens, and eight steps or more a wave: less hides the way over LDS, and more tokens are more to lay out than lanes read
-    // twice.  us a pass of TinyLlama, none and each of these this way: w_down (11 steps) 1, 2, 3, 6 tokens 1,043 -> 1,021, 1,058 -> 1,042, 1,063 -> 1,066,
-    // 1,145 -> 1,187; gate/up (8) 1,034, 1,055, 1,076, 1,194; classifier (8) 1,038, 1,056, 1,063, 1,152; q/k/v (4) 1,040, 1,054, 1,068, 1,164;
-    // wo (4) 1,069, 1,087, 1,089, 1,178; q/k/v of stories42M (1) 242 -> 254, wo and w_down 280.
-    const bool few = a.T <= 2 && a.K / 32 >= 8 * KS;
-    if (lds > MOST || !few) {
-        NVLLM_LAUNCH((k_gemm_thin<NB, KS, PAIR, NORM>), dim3(tiles), dim3(KS * 64), 0, a);
-        return;
+    if constexpr (NB == 1) {
+        constexpr int NT = PAIR ? 2 : 1;
+        const int lds = thin_lds_bytes<NT, KS>(a.K, a.T, NORM), Kb = a.K / 32;
+        // One or two tokens, and enough steps a wave to make up for the way over LDS.  With 8 waves (more workgroups than CUs) eight, as long as
+        // two workgroups share a CU; with 16 the more the fuller the chip, whose rate is the bound then, and activations in one lap (a
+        // second one returns behind the weights in flight).  us a launch as lanes read them and this way, one and two tokens:
+        //   8 waves, q/k/v        K 2,560 12.9 -> 10.9, 13.2 -> 11.3; 4,096 25.5 -> 21.7, 25.6 -> 22.5; 5,120 39.5 -> 28.1, 39.8 -> 29.3
+        //   8 waves, gate/up      K 2,048 13.9 -> 13.6, 14.0 -> 14.0; 3,584 28.9 -> 27.0, 29.0 -> 28.4; 4,096 (688 workgroups) 34.0 -> 33.8, 33.8 -> 34.2,
+        //                         (512) 24.9 -> 26.4 both, (352) 22.8 -> 21.4, 22.7 -> 22.4; 5,120 52.2 -> 47.5, 52.1 -> 49.6
+        //   8 waves, wo, w_down   K 5,120 14.8 -> 12.7, 14.8 -> 13.2; 13,824 35.5 -> 28.4, 35.6 -> 37.5 (118 KB)
+        //   16 waves, steps       64 workgroups, 16: 12.0 -> 9.4, 12.2 -> 10.4; 128, 8: 5.6 -> 5.6 (K 4,096: 7.5 -> 7.1, 7.5 -> 7.4), 9: 8.2 -> 8.5, 8.2 -> 8.8,
+        //                         10: 9.1 -> 8.3, 9.2 -> 8.7, 11: 9.9 -> 8.9, 10.0 -> 9.3; 192, 10: 9.4 -> 9.6, 9.3 -> 9.9, 16: 12.6 -> 11.9, 12.7 -> 12.6;
+        //                         224, 19: 15.7 -> 14.4, 15.8 -> 15.3; 256, 8: 8.2 -> 9.4, 8.2 -> 9.5, 16: 13.7 -> 13.9, 13.8 -> 14.3, 21: 17.7 -> 17.2, 17.8 -> 18.1
+        // Three tokens are more to lay out than lanes read twice (TinyLlama, all of its long projections: 1,063 -> 1,076 a pass), and the classifier's four
+        // blocks already share one reading (K 4,096 45.4 -> 47.1, 46.3 -> 47.8; 2,048 25.5 -> 25.3, 27.7 -> 27.4).
+        const bool pays = KS == 8 ? Kb >= 8 * KS && lds <= 80 * 1024 : Kb >= KS * (2 + tiles / 16) && (long)a.T * a.K <= 4L * THIN_LAP * KS * 64;
+        if (a.T <= 2 && pays) {
+            static bool enabled = false;
+            if (!enabled) {
+                HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_gemm_thin_lds<KS, PAIR, NORM>), hipFuncAttributeMaxDynamicSharedMemorySize, THIN_LDS_MOST));
+                enabled = true;
+            }
+            NVLLM_LAUNCH((k_gemm_thin_lds<KS, PAIR, NORM>), dim3(tiles), dim3(KS * 64), lds, a);
+            return;
+        }
     }
-    static bool enabled = false;
-    if (!enabled) {
-        HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_gemm_thin_lds<NB, KS, PAIR, NORM>), hipFuncAttributeMaxDynamicSharedMemorySize, MOST));
-        enabled = true;
-    }
-    NVLLM_LAUNCH((k_gemm_thin_lds<NB, KS, PAIR, NORM>), dim3(tiles), dim3(KS * 64), (int)lds, a);
+    NVLLM_LAUNCH((k_gemm_thin<NB, KS, PAIR, NORM>), dim3(tiles), dim3(KS * 64), 0, a);
 }
 
 void launch_gemm_thin(const F32Gemm& g, int prof_cls) {
