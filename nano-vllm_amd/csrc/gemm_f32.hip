@@ -482,10 +482,13 @@ static bool launch_products(const F32Gemm& g, int prof_cls, bool* has_pairs) {
 bool launch_gemm_f32(const F32Gemm& g, int prof_cls) {
     if (g.T <= 0 || g.n_segs == 0) return false;
     if (g.amax_out && (!g.amax_pairs || g.amax_ld < g.T)) NVLLM_FATAL("fused arg-max needs a pair buffer of at least %d rows per block", g.T);
-    bool has_pairs = g.gain != nullptr && g.seg[0].W2 == nullptr;
-    const bool rides = launch_products(g, prof_cls, &has_pairs);
-    // one row of 32,000 scanned again 6.6 us, its 2,000 pairs merged 4.2
-    if (g.amax_out && has_pairs) launch_argmax_tiles(g.amax_out, g.amax_pairs, cdiv(g.seg[0].N, 16), g.T, g.amax_ld, g.amax_out_host);
+    // Pairs from products behind a norm, of as many outputs as fp32 has whole numbers for (a pair's index is one); else the rows are scanned
+    bool has_pairs = g.amax_out && g.gain && !g.seg[0].W2 && g.seg[0].N <= 1 << 24;
+    F32Gemm a = g;
+    if (!has_pairs) a.amax_out = nullptr;
+    const bool rides = launch_products(a, prof_cls, &has_pairs);
+    // us a launch for one row of 32,000, 64 and 128 of them: scanned 7.2, 8.1, 8.9, pairs merged 6.0, 7.5, 9.0 (and the classifier no slower for leaving them)
+    if (has_pairs) launch_argmax_tiles(g.amax_out, g.amax_pairs, cdiv(g.seg[0].N, 16), g.T, g.amax_ld, g.amax_out_host);
     else if (g.amax_out) launch_argmax_ld(g.amax_out, g.seg[0].out, g.T, g.seg[0].N, g.seg[0].ldo, g.amax_out_host);
     return rides;
 }
