@@ -546,7 +546,7 @@ void LatentHyperModel::forward_b16(const PassArgs& a, const StepArrays& st, cons
     e.amax_out_host = a.argmax_host;
     e.out_host = a.logits_host;
     e.amax_ld = B;
-    e.amax_pairs = (float2*)ws_get(WS_AMAX_PAIRS, (size_t)cdiv(V_, 32) * e.amax_ld * sizeof(float2));
+    e.amax_pairs = (float2*)ws_get(WS_AMAX_PAIRS, amax_pair_bytes(cdiv(V_, 32), B));
     launch_gemm_b16(head_, rows, B, e, PC_GEMM_HEAD);
 }
 

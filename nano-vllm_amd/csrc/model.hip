@@ -399,7 +399,7 @@ static void forward_f32(const StepArrays& st, int T, int B, Config* p, RunState*
     head.amax_out = d_argmax;
     head.amax_out_host = argmax_host;
     head.amax_ld = B;
-    head.amax_pairs = (float2*)ws_get(WS_AMAX_PAIRS, (size_t)cdiv(V, 16) * std::max(B, 1) * sizeof(float2));
+    head.amax_pairs = (float2*)ws_get(WS_AMAX_PAIRS, amax_pair_bytes(cdiv(V, 16), B));
     if (B > 0) launch_gemm_f32(head.add(w->lm_head, V, d_logits), PC_GEMM_HEAD);
 }
 
@@ -955,7 +955,7 @@ static long enqueue_pass(int* tokens, int num_tokens, int* pos_arr, int* seq_ids
         host_written = argmax_direct() && !chained;
         if (host_written) e5.amax_out_host = next_slot(B).host;
         e5.amax_ld = B;   // (few rows' pairs side by side: lanes that merge them read lines, not one line each)
-        e5.amax_pairs = (float2*)ws_get(WS_AMAX_PAIRS, (size_t)cdiv(V, 16) * e5.amax_ld * sizeof(float2));
+        e5.amax_pairs = (float2*)ws_get(WS_AMAX_PAIRS, amax_pair_bytes(cdiv(V, 16), B));
         if (thin_head) {
             F32Gemm head = F32Gemm(s->x, B, D).norm(m->rms_final, eps);
             head.in_rows = st.d_out_idx;

@@ -145,6 +145,9 @@ enum WsSlot {
     WS_COUNT
 };
 void* ws_get(WsSlot slot, size_t bytes);
+// Bytes of WS_AMAX_PAIRS for `rows` rows of pairs of `blocks` blocks: room for 64 rows at a time, so that a batch which grows row by row does
+// not free and allocate it (and wait for the passes in flight) at every fourth size.
+inline size_t amax_pair_bytes(int blocks, int rows) { return (size_t)blocks * ((rows + 63) & ~63) * sizeof(float2); }
 void* ws_try(WsSlot slot, size_t bytes);   // null: no memory
 
 // Pinned host staging for the integer arrays of one call.

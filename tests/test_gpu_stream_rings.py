@@ -1,9 +1,14 @@
 """Streaming projections where a wave's K-steps are fewer than, as many as and a few more than it has in flight, and where a token has
 more sums of squares than are held over the K loop; and the token ids that the classifier's blocks of fp32 models leave."""
+import ctypes as C
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 
-from nvllm_amd import synth
+from nvllm_amd import capi, synth
 from tests import test_gpu_thin
 
 pytestmark = pytest.mark.gpu
@@ -89,3 +94,26 @@ def test_ids_beyond_what_fp32_holds(hip, tmp_path):
     want = got.argmax(1)
     assert (want >= 1 << 24).all() and (want % 2 == 1).any()
     assert picked == want.tolist()
+
+
+def pair_room_of_one_row(folder):
+    """Bytes that the first pass of one row takes on the GPU and keeps (run in a process of its own: what a pass keeps only grows)."""
+    hip, vocab = capi.load_hip(), 1 << 20
+    hip.init_ops()
+    free, total = C.c_size_t(), C.c_size_t()
+    seen = []
+    for words in (500, vocab):
+        path = os.path.join(folder, "m%d.bin" % words)
+        fp32_model(path, 1, 32, words)
+        test_gpu_thin.batch(hip, path, 4, [5], [6], [0])
+        assert C.CDLL("libamdhip64.so").hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+        seen.append(free.value)
+    return seen[0] - seen[1]
+
+
+def test_pairs_have_room_for_64_rows_from_the_first_row_on(hip, tmp_path):
+    """A batch that grows row by row does not allocate them again and again."""
+    code = "from tests import test_gpu_stream_rings as t; print('ROOM', t.pair_room_of_one_row(%r))" % str(tmp_path)
+    out = subprocess.run([sys.executable, "-c", code], cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))), capture_output=True, text=True, timeout=100)
+    assert out.returncode == 0, out.stderr[-2000:]
+    assert int(out.stdout.split("ROOM")[1]) >= 64 * (1 << 16) * 8
