@@ -82,7 +82,7 @@ __global__ __launch_bounds__(KS * 64, f32_occupancy((PAIR ? 2 : 1) * NB * TB, NO
     // What the epilogue needs beside the sums travels with the first steps, and angles behind their positions; where the registers
     // are full (2 x 2 blocks at four waves a SIMD), behind the last
     constexpr bool EARLY = PAIR || NT * TB < 4 || f32_occupancy(NT * TB, NORM) < 4;
-    const bool turns = !PAIR && !AMAX && (sg.kind == F32Out::ROPE_Q || sg.kind == F32Out::ROPE_K), adds = !PAIR && sg.kind == F32Out::ADD;
+    const bool turns = !PAIR && !AMAX && f32_turns(sg), adds = !PAIR && sg.kind == F32Out::ADD;
     int at[FPT], row[FPT];
     f4_t side[FPT];   // angles, or what is added to
     auto item = [&](int q, int& t, int& n) {
@@ -107,7 +107,7 @@ __global__ __launch_bounds__(KS * 64, f32_occupancy((PAIR ? 2 : 1) * NB * TB, NO
             int t, n;
             item(q, t, n);
             row[q] = PAIR ? -1 : f32_row(p, sg, t);
-            if (turns) side[q] = *reinterpret_cast<const f4_t*>(p.rope + (size_t)at[q] * (p.hd >> 1) + ((n % p.hd) >> 1));
+            if (turns) side[q] = f32_angles(p, at[q], n);
             else if (adds) side[q] = f32_old(sg, t, n);
             else side[q] = f4_t{0.f, 0.f, 0.f, 0.f};
         }
@@ -262,7 +262,7 @@ __global__ __launch_bounds__(KS * 64, f32_occupancy((PAIR ? 2 : 1) * NB * TB, NO
             y *= scale;
             if constexpr (PAIR) u *= scale;
         }
-        if (live) f32_finish<PAIR>(p, sg, t, n, y, u, side, side, row);
+        if (live) f32_finish<PAIR>(p, sg, t, n, y, u, side, row);
         if constexpr (AMAX) f32_pairs(p, N, n >> 4, n, t, (n & 15) == 0 && live, y);
     };
     if constexpr (!EARLY) request_side();
@@ -376,8 +376,11 @@ __global__ __launch_bounds__(256) void k_gemm_f32_any(F32Gemm p) {
                 y[i] = total(acc[j][i]) * scale;
                 if (PAIR) u[i] = total(acc2[j][i]) * scale;
             }
-            if (lane == 0 && t0 + j < T)
-                f32_finish<PAIR>(p, sg, t0 + j, n, y, u, !PAIR && sg.kind == F32Out::ADD ? f32_old(sg, t0 + j, n) : u, f32_turn(p, sg, t0 + j, n), f32_row(p, sg, t0 + j));
+            const int t = t0 + j;
+            if (lane == 0 && t < T) {
+                const f4_t side = PAIR ? u : sg.kind == F32Out::ADD ? f32_old(sg, t, n) : f32_turns(sg) ? f32_angles(p, p.pos[t], n) : u;
+                f32_finish<PAIR>(p, sg, t, n, y, u, side, f32_row(p, sg, t));
+            }
         }
     }
 }

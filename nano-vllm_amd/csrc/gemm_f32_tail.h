@@ -14,17 +14,18 @@ __device__ __forceinline__ int f32_segment(const F32Gemm& p, int tile) {
     return s;
 }
 
-// What follows a token's complete sums of features n .. n+3 (n % 4 == 0; `old`: what ADD adds to).
-// `turn`: the angles of a quad that turns (f32_turn), `row`: its token's cache row.
-__device__ __forceinline__ f4_t f32_turn(const F32Gemm& p, const F32Segment& sg, int t, int n) {
-    if (sg.kind != F32Out::ROPE_Q && sg.kind != F32Out::ROPE_K) return f4_t{0.f, 0.f, 0.f, 0.f};
-    return *reinterpret_cast<const f4_t*>(p.rope + (size_t)p.pos[t] * (p.hd >> 1) + ((n % p.hd) >> 1));   // (hd is a multiple of 8)
+// The angles of features n .. n+3 of a head (n % 4 == 0) at position `pos`.
+__device__ __forceinline__ bool f32_turns(const F32Segment& sg) { return sg.kind == F32Out::ROPE_Q || sg.kind == F32Out::ROPE_K; }
+__device__ __forceinline__ f4_t f32_angles(const F32Gemm& p, int pos, int n) {
+    return *reinterpret_cast<const f4_t*>(p.rope + (size_t)pos * (p.hd >> 1) + ((n % p.hd) >> 1));   // (hd is a multiple of 8)
 }
 __device__ __forceinline__ int f32_row(const F32Gemm& p, const F32Segment& sg, int t) {
     return sg.kind == F32Out::ROPE_K || sg.kind == F32Out::KV_V ? p.kv_row[t] : -1;
 }
+// What follows a token's complete sums of features n .. n+3 (n % 4 == 0).  `side`: what ADD adds to, or the angles of a quad that turns;
+// `row`: its token's cache row.
 template <bool PAIR>
-__device__ __forceinline__ void f32_finish(const F32Gemm& p, const F32Segment& sg, int t, int n, f4_t y, const f4_t u, const f4_t old, const f4_t turn, int row) {
+__device__ __forceinline__ void f32_finish(const F32Gemm& p, const F32Segment& sg, int t, int n, f4_t y, const f4_t u, const f4_t side, int row) {
     if constexpr (PAIR) {
 #pragma unroll
         for (int r = 0; r < 4; r++) {
@@ -35,7 +36,7 @@ __device__ __forceinline__ void f32_finish(const F32Gemm& p, const F32Segment& s
         switch (sg.kind) {
             case F32Out::ADD:
 #pragma unroll
-                for (int r = 0; r < 4; r++) y[r] = __fadd_rn(old[r], y[r]);
+                for (int r = 0; r < 4; r++) y[r] = __fadd_rn(side[r], y[r]);
                 break;
             case F32Out::SILU:
 #pragma unroll
@@ -47,7 +48,7 @@ __device__ __forceinline__ void f32_finish(const F32Gemm& p, const F32Segment& s
                 break;
             case F32Out::ROPE_Q:
             case F32Out::ROPE_K: {   // the two pairs of this quad turn (layers.c:118-141)
-                const float2 c0 = make_float2(turn[0], turn[1]), c1 = make_float2(turn[2], turn[3]);
+                const float2 c0 = make_float2(side[0], side[1]), c1 = make_float2(side[2], side[3]);
                 y = f4_t{__fsub_rn(__fmul_rn(y[0], c0.x), __fmul_rn(y[1], c0.y)), __fadd_rn(__fmul_rn(y[0], c0.y), __fmul_rn(y[1], c0.x)),
                          __fsub_rn(__fmul_rn(y[2], c1.x), __fmul_rn(y[3], c1.y)), __fadd_rn(__fmul_rn(y[2], c1.y), __fmul_rn(y[3], c1.x))};
                 break;

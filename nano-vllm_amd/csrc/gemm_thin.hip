@@ -29,7 +29,7 @@ constexpr int thin_ring(int NT, bool norm) { return NT == 1 ? 4 : NT == 2 ? (nor
 template <bool PAIR>
 __device__ __forceinline__ void thin_finish(const F32Gemm& p, const F32Segment& sg, int x, int g, int nb, int n0, const f4_t& y, const f4_t& u, const f4_t& side, int row) {
     const int T = p.T, N = sg.N;
-    if (x < T && n0 < N) f32_finish<PAIR>(p, sg, x, n0, y, u, side, side, row);
+    if (x < T && n0 < N) f32_finish<PAIR>(p, sg, x, n0, y, u, side, row);
     if (!PAIR && p.amax_pairs != nullptr) f32_pairs(p, N, nb, n0, x, g == 0 && x < T, y);
 }
 
@@ -59,7 +59,7 @@ __global__ __launch_bounds__(KS * 64) void k_gemm_thin_lds(F32Gemm p) {   // a b
     float* s_sq = reinterpret_cast<float*>(s_act + 2 * (size_t)K * T);   // NORM: [token][32 k]
     const int tx = min(x, T - 1);   // columns past the last token compute it again and are not stored
     const int n0 = nb * 16 + 4 * g;
-    const bool finishes = wave == 0, turns = !PAIR && finishes && (sg.kind == F32Out::ROPE_Q || sg.kind == F32Out::ROPE_K), adds = !PAIR && finishes && sg.kind == F32Out::ADD;
+    const bool finishes = wave == 0, turns = !PAIR && finishes && f32_turns(sg), adds = !PAIR && finishes && sg.kind == F32Out::ADD;
     const int at = turns ? p.pos[tx] : 0;
 
     // activations: item i is four k of a token, LAP of a thread at a time
@@ -149,7 +149,7 @@ __global__ __launch_bounds__(KS * 64) void k_gemm_thin_lds(F32Gemm p) {   // a b
     f4_t side = {0.f, 0.f, 0.f, 0.f};   // angles, or what is added to
     int row = -1;
     if (!PAIR && finishes) row = f32_row(p, sg, tx);
-    if (turns) side = *reinterpret_cast<const f4_t*>(p.rope + (size_t)at * (p.hd >> 1) + ((n0 % p.hd) >> 1));
+    if (turns) side = f32_angles(p, at, n0);
     else if (adds) side = f32_old(sg, tx, n0);
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // (not for the weights in flight)
     __builtin_amdgcn_s_barrier();
@@ -231,13 +231,13 @@ __global__ __launch_bounds__(KS * 64) void k_gemm_thin(F32Gemm p) {
     const float* gp = NORM ? p.gain + 8 * g : nullptr;
     // what the epilogue needs beside the sums travels with the first tiles, and angles behind their positions
     const int nb = nb0 + (PAIR ? 0 : wave), n0 = nb * 16 + 4 * g;   // of the block this wave finishes
-    const bool turns = !PAIR && wave < NB && (sg.kind == F32Out::ROPE_Q || sg.kind == F32Out::ROPE_K), adds = !PAIR && wave < NB && sg.kind == F32Out::ADD;
+    const bool turns = !PAIR && wave < NB && f32_turns(sg), adds = !PAIR && wave < NB && sg.kind == F32Out::ADD;
     f4_t side = {0.f, 0.f, 0.f, 0.f};   // angles, or what is added to
     int row = -1;
     const int at = turns ? p.pos[tx] : 0;
     auto request_side = [&] {
         if (!PAIR && wave < NB) row = f32_row(p, sg, tx);
-        if (turns) side = *reinterpret_cast<const f4_t*>(p.rope + (size_t)at * (p.hd >> 1) + ((n0 % p.hd) >> 1));
+        if (turns) side = f32_angles(p, at, n0);
         else if (adds) side = f32_old(sg, tx, n0);
     };
     h8_t w[RING][NT];
