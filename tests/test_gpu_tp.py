@@ -4,8 +4,6 @@ whole model."""
 import ctypes as C
 import json
 import os
-import subprocess
-import sys
 
 import numpy as np
 import pytest
@@ -15,7 +13,7 @@ from tests import util
 
 pytestmark = pytest.mark.gpu
 
-ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+WORKER = os.path.join(os.path.dirname(os.path.abspath(__file__)), "tp_worker.py")
 TIGHT_TOL = 2e-4     # as for the single-process forward pass
 LOGITS_TOL = 2e-2
 
@@ -181,11 +179,8 @@ def test_ranks_sharing_one_gpu_match_the_oracle(tmp_path, tmp_models, world, kv_
         spec["probe_counts"] = [4, 1000, 128 * 4096]
     env = dict(os.environ, MASTER_ADDR="127.0.0.1", OMP_NUM_THREADS="8" if big else ("1" if world > 4 else "2"), HSA_ENABLE_IPC_MODE_LEGACY="0")
     port = 29620 + world + kv_bytes + (40 if big else 0) + (100 if exchange == "peer" else 0)
-    out = subprocess.run([sys.executable, "-m", "torch.distributed.run", "--nnodes=1", "--nproc-per-node", str(world),
-                          "--master-addr", "127.0.0.1", "--master-port", str(port),
-                          os.path.join(ROOT, "tests", "tp_worker.py"), json.dumps(spec)],
-                         env=env, capture_output=True, text=True, timeout=500)
-    assert out.returncode == 0, (out.stdout[-2000:], out.stderr[-4000:])
+    out = util.run_ranks(world, port, [WORKER, json.dumps(spec)], tmp_path / "ranks", env, 500)
+    assert out.returncode == 0, out.said
     for rank in range(world):
         r = json.load(open(tmp_path / f"rank{rank}.json"))
         assert r["same_trace"] and r["same_tokens"], r
@@ -207,16 +202,12 @@ def test_a_rank_left_alone_by_its_peers_stops_with_a_message(tmp_path, tmp_model
     spec = dict(name="tiny", over=GQA, model_path=path, n_seqs=1, seed=23, n_new=1, chunk=12, kv_bytes=2, out_dir=str(tmp_path),
                 exchange="peer", lonely_call=True)
     env = dict(os.environ, MASTER_ADDR="127.0.0.1", OMP_NUM_THREADS="2", HSA_ENABLE_IPC_MODE_LEGACY="0", NVLLM_TP_PEER_WAIT_S="2")
-    out = subprocess.run([sys.executable, "-m", "torch.distributed.run", "--nnodes=1", "--nproc-per-node", "2",
-                          "--master-addr", "127.0.0.1", "--master-port", "29791",
-                          os.path.join(ROOT, "tests", "tp_worker.py"), json.dumps(spec)],
-                         env=env, capture_output=True, text=True, timeout=300)
+    out = util.run_ranks(2, 29791, [WORKER, json.dumps(spec)], tmp_path / "ranks", env, 300)
     assert out.returncode != 0
-    text = out.stdout + out.stderr
-    assert "LONELY waited" in text and "LONELY still alive" not in text, text[-3000:]
-    waited = float(text.split("LONELY waited")[1].split()[0])
+    assert "LONELY waited" in out.stdout and "LONELY still alive" not in out.stdout, out.said
+    waited = float(out.stdout.split("LONELY waited")[1].split()[0])
     assert 1.5 < waited < 5.5, waited          # one wait of 2 s (phase A); three calls x two phases sat out in full would be 12 s
-    assert "waited 2 s for a flag" in text, text[-3000:]
+    assert out.said.startswith("rank 0: nvllm: ") and "waited 2 s for a flag" in out.said.splitlines()[0], out.said
 
 
 def test_residual_tail_inside_the_peer_exchange_gives_the_same_bits(tmp_path, tmp_models):
@@ -231,11 +222,8 @@ def test_residual_tail_inside_the_peer_exchange_gives_the_same_bits(tmp_path, tm
         spec = dict(name="tiny", over=GQA, model_path=path, n_seqs=4, seed=23, n_new=12, chunk=12, kv_bytes=2, out_dir=str(out_dir),
                     exchange="peer", probe_counts=[1000])
         env = dict(os.environ, MASTER_ADDR="127.0.0.1", OMP_NUM_THREADS="2", HSA_ENABLE_IPC_MODE_LEGACY="0", NVLLM_TP_PEER_FUSED=fused)
-        out = subprocess.run([sys.executable, "-m", "torch.distributed.run", "--nnodes=1", "--nproc-per-node", "2",
-                              "--master-addr", "127.0.0.1", "--master-port", str(29795 + int(fused)),
-                              os.path.join(ROOT, "tests", "tp_worker.py"), json.dumps(spec)],
-                             env=env, capture_output=True, text=True, timeout=300)
-        assert out.returncode == 0, (out.stdout[-2000:], out.stderr[-4000:])
+        out = util.run_ranks(2, 29795 + int(fused), [WORKER, json.dumps(spec)], out_dir / "ranks", env, 300)
+        assert out.returncode == 0, out.said
         rs = [json.load(open(out_dir / f"rank{rank}.json")) for rank in range(2)]
         assert all(r["same_tokens"] and r["same_trace"] for r in rs), rs
         assert rs[0]["logits_crc"] == rs[1]["logits_crc"]          # the ranks hold the same logits

@@ -10,6 +10,7 @@ import sys
 import pytest
 
 from nvllm_amd import capi
+from tests import util
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
@@ -77,3 +78,18 @@ def test_two_gloo_ranks_reproduce_the_unsharded_projections(tmp_path):
         assert r["heads"] == [4 * rank, 4] and r["kv"] == [2 * rank, 2] and r["hidden"] == [160 * rank, 160]
         # same terms, summed in a different order (slice by slice): fp32 rounding only
         assert r["err_o"] < 1e-5 and r["err_m"] < 1e-5, r
+
+
+def test_a_failed_run_of_ranks_shows_what_the_library_said_first(tmp_path):
+    """A rank says why and aborts; a long traceback of another and the launcher's report follow."""
+    script = tmp_path / "rank.py"
+    script.write_text("import os, sys\n"
+                      "if os.environ['RANK'] == '1':\n"
+                      "    os.write(2, b'nvllm: the reason (file:1)\\n')\n"
+                      "    os.write(2, b'and more\\n' * 1000)\n"
+                      "    os.abort()\n"
+                      "sys.stdin.read()\n")
+    out = util.run_ranks(2, 29801, [str(script)], tmp_path / "ranks", dict(os.environ, OMP_NUM_THREADS="1"), 100)
+    assert out.returncode != 0
+    assert out.said.splitlines()[0] == "rank 1: nvllm: the reason (file:1)"
+    assert "and more" in out.said and "SIGABRT" in out.said

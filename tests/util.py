@@ -1,6 +1,10 @@
 """Helpers shared by the tests: call the operators of include/ops.h on numpy data
 through any of the three libraries (HIP product, CPU oracle, reference build)."""
 import ctypes as C
+import glob
+import os
+import subprocess
+import sys
 
 import numpy as np
 
@@ -9,6 +13,23 @@ from nvllm_amd import capi
 
 def f32(a):
     return np.ascontiguousarray(a, dtype=np.float32)
+
+
+def run_ranks(world, port, argv, log_dir, env, timeout):
+    """`world` processes of a script under torch's launcher.  Returns its result, with `said`: what to show of a failure.  First every
+    line that the library printed before it stopped a rank ("nvllm: ..."; a traceback and the launcher's report would push it out of
+    sight), then the end of each rank's stderr and of the launcher's."""
+    out = subprocess.run([sys.executable, "-m", "torch.distributed.run", "--nnodes=1", "--nproc-per-node", str(world), "--master-addr", "127.0.0.1",
+                          "--master-port", str(port), "--log-dir", str(log_dir), "--tee", "3", *argv], env=env, capture_output=True, text=True, timeout=timeout)
+    reasons, ends = [], []
+    for path in sorted(glob.glob(os.path.join(str(log_dir), "**", "stderr.log"), recursive=True)):
+        rank = os.path.basename(os.path.dirname(path))
+        with open(path, errors="replace") as f:
+            text = f.read()
+        reasons += ["rank %s: %s" % (rank, line) for line in text.splitlines() if line.startswith("nvllm:")]
+        ends.append("rank %s ... %s" % (rank, text[-1500:]))
+    out.said = "\n".join(reasons + ends + [out.stdout[-1000:], out.stderr[-2000:]])
+    return out
 
 
 class Pool:
