@@ -45,7 +45,8 @@ struct TileIdx {
 //            wo of stories42M, 32    5.2 | 4.9 | 5.2 | - | 6: 5.1, 8: 5.1
 //   32 x 32  q/k/v                   10.3 | 9.6 | 9.8 | 9.8                       13.7 | 13.1 | 12.8 | 12.6
 //   64 x 16  w_down, 9 rows          8.9 | 8.4 | 8.2 | 8.4                        experts' gate/up 43.3 | 40.8 | 40.6 | 39.4
-//            classifier, 9 rows      44.2 | 44.8 | 43.0 | 44.5
+//            classifier, 9 rows      44.2 | 44.8 | 43.0 | 44.5                     44.9 | 44.2 | 43.4 | 44.1
+//            classifier, one row                                                  27.8 | 29.5 | 27.7 | 28.3 (experts' w_down 17.9 | 19.3 | 17.1 | 17.1)
 //   64 x 32  w_down (RESID)          12.6 | 12.5 | 12.9 | 12.9                    11.7 | 11.5 | 12.2 | 12.0
 //            w_down (HYPER)                                                       12.1 | 12.4 | 12.4 | 12.0
 //            gate/up 32 rows, shared expert's w_down (F32)
@@ -56,16 +57,19 @@ struct TileIdx {
 //            products by head (K 64)                                              4.8 | 5.1 | 5.4 | - | 2: 5.3
 // (Two runs of one build differ by 0.1 to 0.3.  The products by head take 5.3 with the old wait too, behind the launch of 32 x 32 tiles that
 // ends 0.5 sooner now.)
+// Tiles of 64 x 64 whose epilogue adds to rows: a loop that waits for everything in flight in every step, and holds nothing over it for the
+// epilogue (w_down of TinyLlama, 160 and 200 tokens 22.5 and 23.2 us against 23.2 and 24.0 without those waits, of Suselorn-1.2B, 101 tokens 14.7 against 15.1).
+constexpr bool gemm_step_waits(int TB, int epi) { return TB == 4 && (epi == GemmEpilogue::RESID_A16 || hyper_streams(epi) > 0); }
 constexpr int gemm_ring(int NBW, int TB, int planes, int epi, bool groups = false) {
     if (NBW == 2) return TB == 1 && planes == 1 ? 8 : 4;
     if (NBW == 4 && TB == 2) return epi == GemmEpilogue::F32 || epi == GemmEpilogue::SWIGLU_A16 ? 2 : 4;
-    if (TB == 4) return planes == 2 ? 2 : groups ? 4 : 3;
-    return planes == 2 && NBW == 4 && TB == 1 && epi == GemmEpilogue::F32 ? 3 : 4;   // (a classifier of up to 16 rows: two workgroups share a CU)
+    if (TB == 4) return gemm_step_waits(TB, epi) || groups ? 4 : planes == 2 ? 2 : 3;
+    return NBW == 4 && TB == 1 && epi == GemmEpilogue::F32 ? 3 : 4;   // (a classifier of up to 16 rows: two workgroups share a CU)
 }
 constexpr int gemm_ring_act(int NBW, int TB, int planes, int epi, bool groups = false) {
     const int ring = gemm_ring(NBW, TB, planes, epi, groups);
-    const bool narrow = NBW == 2 && TB == 1 && planes == 2, wide = NBW == 4 && TB == 2 && hyper_streams(epi) == 0, by_group = TB == 4 && ring == 4;
-    return narrow || wide || by_group ? 2 : ring;
+    const bool narrow = NBW == 2 && TB == 1 && planes == 2, wide = NBW == 4 && TB == 2 && hyper_streams(epi) == 0, tall = TB == 4 && ring == 4;
+    return narrow || wide || tall ? 2 : ring;
 }
 
 // bytes of dynamic LDS a tile needs: the waves' partial tiles, then four small arrays
@@ -303,6 +307,7 @@ __device__ __forceinline__ bool gemm_tile(const GemmArgs& p, const TileIdx ix, u
     };
 
     const GemmEpilogue& ep = p.e;
+    constexpr bool STEP_WAITS = COH || gemm_step_waits(TB, EPI);
     // 1/rms of this token group comes from the producer's per-tile sums of squares: every thread sums a slice of one token's tiles; the slices
     // meet in LDS before the epilogue.  Up to SS_HELD of them are requested behind the first steps and held in registers over the K loop.  (Summed in
     // front of it, each load waited for all before it: two to sixteen trips to memory before the first product.)  The one-launch step, whose
@@ -311,8 +316,8 @@ __device__ __forceinline__ bool gemm_tile(const GemmArgs& p, const TileIdx ix, u
     float ss_held[SS_HELD];
     const float* ss_row = nullptr;
     const int ss_tl = tid / PARTS, ss_part = tid % PARTS;   // (lanes side by side read one token's sums: a line, and not one line each)
-    // What the epilogue needs beside the sums: requested behind the first steps and waited for behind the last.  In the one-launch step behind the
-    // last: held over the loop they made it spill (64 tokens: 230 registers -> 256 and 58 more in scratch)
+    // What the epilogue needs beside the sums: requested behind the first steps and waited for behind the last.  With STEP_WAITS requested behind the
+    // last: held over the loop they made the one-launch step spill (64 tokens: 230 registers -> 256 and 58 more in scratch)
     float4 pf_x[FPT], pf_g[FPT];
     int pf_pos = 0, pf_row = -1;
     f4_t pf_turn[FPT];
@@ -365,12 +370,12 @@ __device__ __forceinline__ bool gemm_tile(const GemmArgs& p, const TileIdx ix, u
                 for (int q = 0; q < SS_HELD; q++) ss_held[q] = ss_row[min(ss_part + q * PARTS, ep.ss_tiles - 1)];
             }
         }
-        if constexpr (!COH) request_operands();
+        if constexpr (!STEP_WAITS) request_operands();
     };
 
     // Loads are issued only for steps that exist: a clamped re-load of the last tile would be real HBM traffic, since streamed
     // weights are loaded non-temporally and do not stay in L2.
-    if constexpr (COH) {
+    if constexpr (STEP_WAITS) {
         // (requests under conditions, each waited for with all before it: with the loop below the one-launch step needs 26 to 56 registers more)
         if (PRE == 0 || (PRE == 2 && !prefetched)) {
 #pragma unroll
@@ -462,10 +467,9 @@ __device__ __forceinline__ bool gemm_tile(const GemmArgs& p, const TileIdx ix, u
             }
     }
     NVLLM_TSTAMP(3, acc[NBW - 1][TB - 1][0]);
-    if constexpr (COH) {
-        request_positions();
-        request_operands();
-    } else if (ep.ss_in != nullptr) {
+    if constexpr (COH) request_positions();
+    if constexpr (STEP_WAITS) request_operands();
+    if (!COH && ep.ss_in != nullptr) {
         float ss = 0.f;
 #pragma unroll
         for (int q = 0; q < SS_HELD; q++)
