@@ -233,7 +233,7 @@ int nvllm_tp_init_custom(int rank, int world, nvllm_allreduce_fn fn, void* ctx);
  * one rank in rank order, so all ranks hold the same bits).  No counterpart in the reference, whose
  * forward pass runs in one process (the sums it replaces: src/model.c:385,392).
  *   every rank:  nvllm_tp_peer_handle(mine);            then all-gather the handles in rank order
- *   every rank:  nvllm_tp_init_peer(rank, world, all);  (world <= 8)
+ *   every rank:  nvllm_tp_init_peer(rank, world, all);  (world <= 8; four ranks that share one GPU are refused)
  * Every rank must make the same sequence of forward calls.  A rank that waits 30 s for a peer stops
  * the process with a message at its next call.  Both return 0, or -1 with a message. */
 #define NVLLM_TP_PEER_HANDLE_BYTES 64

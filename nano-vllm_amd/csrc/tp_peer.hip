@@ -53,7 +53,8 @@ constexpr size_t FLAG_LINE = 128;
 constexpr size_t FLAGS_BYTES = 2 /*phase*/ * 2 /*parity*/ * PEER_MAX_WORLD * FLAG_LINE;
 constexpr size_t STAGE_FLOATS = PEER_MAX_FLOATS + 4 * PEER_MAX_WORLD;   // world slices of ceil(count / world) rounded to 4
 constexpr size_t RED_FLOATS = PEER_MAX_FLOATS / 2 + 4;                  // one slice at world >= 2
-constexpr size_t STAGE_OFF = FLAGS_BYTES;
+constexpr size_t PLACE_OFF = FLAGS_BYTES;   // which GPU the segment lies on
+constexpr size_t STAGE_OFF = FLAGS_BYTES + FLAG_LINE;
 constexpr size_t RED_OFF = STAGE_OFF + 2 * STAGE_FLOATS * sizeof(float);
 constexpr size_t SEG_BYTES = RED_OFF + 2 * RED_FLOATS * sizeof(float);
 
@@ -215,6 +216,25 @@ __global__ __launch_bounds__(PEER_THREADS) void k_peer_allreduce(PeerArgs a) {
     }
 }
 
+// Which GPU: what its driver says of it and where it sits.
+struct PeerPlace {
+    char bus[48];
+    hipUUID id;
+};
+static_assert(sizeof(PeerPlace) <= FLAG_LINE, "a line of the segment holds it");
+bool peer_place(PeerPlace* at) {
+    int ordinal = 0;
+    hipDevice_t dev;
+    memset(at, 0, sizeof *at);
+    const bool known = hipGetDevice(&ordinal) == hipSuccess && hipDeviceGet(&dev, ordinal) == hipSuccess &&
+                       hipDeviceGetPCIBusId(at->bus, (int)sizeof at->bus, ordinal) == hipSuccess && hipDeviceGetUuid(&at->id, dev) == hipSuccess;
+    if (!known) (void)hipGetLastError();
+    return known;
+}
+// Ranks on one GPU that a session refuses.  Ranks that share a GPU are rehearsals (nothing promises that kernels of several processes run at
+// once, and the exchange waits for it); a rank of four has stopped there for a reason that is not known, two and eight pass their tests.
+constexpr int PEER_REFUSED_ON_ONE_GPU = 4;
+
 struct PeerState {
     unsigned char* own = nullptr;        // this rank's segment (exported)
     bool own_in_use = false;             // handed to a session; the next handle request makes a fresh one
@@ -337,6 +357,9 @@ int nvllm_tp_peer_handle(void* handle) {
             return -1;
         }
         HIP_CHECK(hipMemset(s.own, 0, FLAGS_BYTES));   // serial numbers start at 1: no flag is up
+        PeerPlace here;
+        (void)peer_place(&here);
+        HIP_CHECK(hipMemcpy(s.own + PLACE_OFF, &here, sizeof here, hipMemcpyHostToDevice));
         HIP_CHECK(hipDeviceSynchronize());
         s.own_in_use = false;
     }
@@ -360,6 +383,16 @@ int nvllm_tp_init_peer(int rank, int world, const void* handles) {
     }
     ensure_init();
     const unsigned char* hs = static_cast<const unsigned char*>(handles);
+    auto unmap = [&](int n) {
+        for (int i = 0; i < n; i++)
+            if (s.opened[i]) {
+                (void)hipIpcCloseMemHandle(s.seg[i]);
+                s.opened[i] = false;
+            }
+    };
+    PeerPlace here;
+    const bool placed = peer_place(&here);
+    int together = 1;   // ranks on this GPU
     for (int j = 0; j < world; j++) {
         s.opened[j] = false;
         if (j == rank) {
@@ -372,15 +405,19 @@ int nvllm_tp_init_peer(int rank, int world, const void* handles) {
         if (hipIpcOpenMemHandle(&p, h, hipIpcMemLazyEnablePeerAccess) != hipSuccess) {
             (void)hipGetLastError();
             fprintf(stderr, "nvllm: hipIpcOpenMemHandle failed for rank %d's exchange segment\n", j);
-            for (int i = 0; i < j; i++)
-                if (s.opened[i]) {
-                    (void)hipIpcCloseMemHandle(s.seg[i]);
-                    s.opened[i] = false;
-                }
+            unmap(j);
             return -1;
         }
         s.seg[j] = static_cast<unsigned char*>(p);
         s.opened[j] = true;
+        PeerPlace there;
+        if (hipMemcpy(&there, s.seg[j] + PLACE_OFF, sizeof there, hipMemcpyDeviceToHost) != hipSuccess) (void)hipGetLastError();
+        else if (placed && memcmp(&there, &here, sizeof here) == 0) together++;
+    }
+    if (together == PEER_REFUSED_ON_ONE_GPU) {
+        fprintf(stderr, "nvllm: nvllm_tp_init_peer(%d, %d): %d ranks share this GPU, which the peer exchange does not take\n", rank, world, together);
+        unmap(world);
+        return -1;
     }
     if (!s.tickets) {
         HIP_CHECK(hipMalloc(reinterpret_cast<void**>(&s.tickets), 3 * sizeof(unsigned)));
@@ -405,11 +442,7 @@ int nvllm_tp_init_peer(int rank, int world, const void* handles) {
     s.world = world;
     s.calls = s.floats = 0;
     if (nvllm_tp_init_custom(rank, world, peer_allreduce, nullptr) != 0) {
-        for (int j = 0; j < world; j++)
-            if (s.opened[j]) {
-                (void)hipIpcCloseMemHandle(s.seg[j]);
-                s.opened[j] = false;
-            }
+        unmap(world);
         return -1;
     }
     s.own_in_use = true;

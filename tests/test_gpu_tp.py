@@ -160,7 +160,7 @@ def test_setup_is_refused_twice_and_for_bad_placements(hip):
                                            # comparison draws from probabilities that must agree to ~1e-6)
     (2, 2, GQA, "peer"),                   # the library's own exchange: kernels that store into each other's segments
     pytest.param(4, 4, GQA, "peer",        # one kv head (two query heads) per rank
-                 marks=pytest.mark.skip(reason="a rank ended by SIGABRT once in a run of all tests; its message was not kept and the cause is not known")),
+                 marks=pytest.mark.skip(reason="refused: a rank of four on one GPU ended by SIGABRT once in a run of all tests; its message was not kept and the cause is not known")),
     (2, 4, LLAMA7B_LAYER, "peer"),
     (8, 4, dict(dim=512, hidden_dim=512, n_layers=2, n_heads=8, n_kv_heads=8, vocab_size=600, max_seq_len=160), "peer"),
                                            # BASELINE.json configs[4]'s degree: eight ranks, one head of 64 and 64 hidden columns each
