@@ -79,9 +79,12 @@ __global__ __launch_bounds__(KS * 64, f32_occupancy((PAIR ? 2 : 1) * NB * TB, NO
     }
     const float* gp = NORM ? p.gain + 4 * g : nullptr;
 
-    // What the epilogue needs beside the sums travels with the first steps, and angles behind their positions; where the registers
-    // are full (2 x 2 blocks at four waves a SIMD), behind the last
-    constexpr bool EARLY = PAIR || NT * TB < 4 || f32_occupancy(NT * TB, NORM) < 4;
+    // What the epilogue needs beside the sums travels with the first steps, and angles behind their positions; with four blocks or more it is
+    // asked for behind the last: their products hide less of a wait for it in front of them than the meeting of the waves' sums hides behind, and
+    // 2 x 2 blocks at four waves a SIMD have no registers for it.  us a launch with the first steps -> behind the last, q/k/v: 2 x 2 blocks of
+    // stories42M, 150 tokens 9.6 -> 8.7, of stories15M, 240 tokens 7.3 -> 6.6; 2 x 3 of stories42M, 480 tokens 17.1 -> 16.7; 2 x 4, 301 tokens 13.1 -> 12.0,
+    // 900 tokens 29.4 -> 28.4 (w_down 12.3 -> 11.6); the other way 1 x 1 blocks of stories15M, one row 4.6 against 5.1.
+    constexpr bool EARLY = PAIR || NT * TB < 4;
     const bool turns = !PAIR && !AMAX && f32_turns(sg), adds = !PAIR && sg.kind == F32Out::ADD;
     int at[FPT], row[FPT];
     f4_t side[FPT];   // angles, or what is added to
