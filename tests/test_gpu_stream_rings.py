@@ -49,13 +49,24 @@ def scan(row):
 
 
 @pytest.mark.parametrize("T,rows", [(1, 1), (9, 9), (40, 3), (59, 59)])
-@pytest.mark.parametrize("dim,vocab", [(96, 1003), (288, 16385)])   # 63 blocks, and 1,025: one more than full tiles of two have
+@pytest.mark.parametrize("dim,vocab", [(96, 1003), (288, 16401)])   # one block more than full tiles have
 def test_ids_of_fp32_models(hip, tmp_path, T, rows, dim, vocab):
+    s = synth.ModelShape(dim=dim, hidden_dim=2 * dim, n_layers=1, n_heads=6, n_kv_heads=6, vocab_size=vocab, max_seq_len=64)
     path = str(tmp_path / "m.bin")
-    fp32_model(path, T, dim, vocab)
+    synth.write_model(path, s, seed=T, dtype="f32", shared=True, exact16=False)
     ids = np.random.default_rng(T).integers(3, vocab, 5 + T).tolist()
     out = [(7 * k) % T for k in range(rows)]
     got, picked = test_gpu_thin.batch(hip, path, 4, ids[:5], ids[5:], out)
+    assert picked == got.argmax(1).tolist()
+
+
+@pytest.mark.parametrize("T,rows", [(1, 1), (9, 9), (40, 3), (59, 59)])
+@pytest.mark.parametrize("dim,vocab", [(96, 1003), (288, 16385)])   # 63 blocks; 1,025, whose last tile of two is half empty (16,401 words have 1,026)
+def test_ids_where_the_last_tile_is_half_empty(hip, tmp_path, T, rows, dim, vocab):
+    path = str(tmp_path / "m.bin")
+    fp32_model(path, T, dim, vocab)
+    ids = np.random.default_rng(T).integers(3, vocab, 5 + T).tolist()
+    got, picked = test_gpu_thin.batch(hip, path, 4, ids[:5], ids[5:], [(7 * k) % T for k in range(rows)])
     assert picked == got.argmax(1).tolist()
 
 

@@ -40,9 +40,18 @@ def test_few_rows(hip, oracle, tmp_path, n, kv_bytes, shape):
 
 
 @pytest.mark.parametrize("n", [1, 2, 3])
+@pytest.mark.parametrize("shape", [
+    dict(dim=2112, hidden_dim=4128, n_layers=1, n_heads=33, n_kv_heads=3, vocab_size=16500),   # 66 and 129 tiles of K: every wave's ring and one or two tiles more
+    dict(dim=2048, hidden_dim=4096, n_layers=1, n_heads=32, n_kv_heads=4, vocab_size=16400),   # the fewest tiles
+])
+def test_activations_laid_out_once(hip, oracle, tmp_path, n, shape):
+    """One and two rows at widths whose projections lay their activations out in LDS, and three rows, which do not."""
+    test_few_rows(hip, oracle, tmp_path, n, 4, shape)
+
+
+@pytest.mark.parametrize("n", [1, 2, 3])
 @pytest.mark.parametrize("kv_bytes", [4, 2])
 @pytest.mark.parametrize("shape", [
-    dict(dim=2112, hidden_dim=4128, n_layers=1, n_heads=33, n_kv_heads=3, vocab_size=16500),   # gate/up: 66 tiles of K, every wave's ring and one or two more
     dict(dim=2048, hidden_dim=4096, n_layers=1, n_heads=32, n_kv_heads=32, vocab_size=16400),  # q/k/v and gate/up: the fewest tiles
     dict(dim=1024, hidden_dim=3104, n_layers=1, n_heads=16, n_kv_heads=4, vocab_size=500),     # w_down on 16 waves: a tile more than the fewest
     dict(dim=512, hidden_dim=8192, n_layers=1, n_heads=8, n_kv_heads=4, vocab_size=500),       # two tokens: a lap to the last value; 8,224 are one value of every thread too many
@@ -50,8 +59,7 @@ def test_few_rows(hip, oracle, tmp_path, n, kv_bytes, shape):
     dict(dim=1024, hidden_dim=512, n_layers=1, n_heads=16, n_kv_heads=4, vocab_size=16),       # the classifier on 16 waves, with the norm: one block, two tiles of K a wave
     dict(dim=5120, hidden_dim=480, n_layers=1, n_heads=40, n_kv_heads=8, vocab_size=500),      # q/k/v and wo on 8 waves: two laps, the second one ragged
 ])
-def test_activations_laid_out_once(hip, oracle, tmp_path, n, kv_bytes, shape):
-    """One and two rows at widths whose projections lay their activations out in LDS, and three rows, which do not."""
+def test_lines_of_the_rule_for_activations_laid_out_once(hip, oracle, tmp_path, n, kv_bytes, shape):
     test_few_rows(hip, oracle, tmp_path, n, kv_bytes, shape)
 
 
