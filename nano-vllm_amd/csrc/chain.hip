@@ -15,8 +15,8 @@
 // has drained its stores -- but a hand-off through memory costs what a kernel boundary costs: the
 // phase ends when its SLOWEST workgroup has stored (3 to 5 us behind the median), detecting that
 // takes another 1 to 2 us, and issuing a ring holds a wave for its bytes / ~50 GB/s.  TinyLlama-1.1B
-// at 64 rows: 70 us per layer here against 65 us as five kernels; the 42M shape at 32 rows: 0.28 ms
-// per step against 0.27.  The switch is therefore OFF unless asked for (NVLLM_DECODE_CHAIN=1 or
+// at 64 rows of 1,088 cached: 1,695 us a pass against 1,600 as five kernels a layer; the 42M shape at
+// 32 rows: 371 against 373.  The switch is therefore OFF unless asked for (NVLLM_DECODE_CHAIN=1 or
 // nvllm_set_decode_chain); the results are the same bits either way.
 //
 // How.  A grid of one 512-thread workgroup per CU runs, per layer, five phases with the work
