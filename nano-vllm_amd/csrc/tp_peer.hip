@@ -233,7 +233,10 @@ bool peer_place(PeerPlace* at) {
 }
 // Ranks on one GPU that a session refuses.  Ranks that share a GPU are rehearsals (nothing promises that kernels of several processes run at
 // once, and the exchange waits for it); a rank of four has stopped there for a reason that is not known, two and eight pass their tests.
-constexpr int PEER_REFUSED_ON_ONE_GPU = 4;
+int peer_refused_on_one_gpu() {
+    const char* e = getenv("NVLLM_TP_PEER_REFUSED");   // (another number, for a test that has two)
+    return e ? atoi(e) : 4;
+}
 
 struct PeerState {
     unsigned char* own = nullptr;        // this rank's segment (exported)
@@ -414,7 +417,7 @@ int nvllm_tp_init_peer(int rank, int world, const void* handles) {
         if (hipMemcpy(&there, s.seg[j] + PLACE_OFF, sizeof there, hipMemcpyDeviceToHost) != hipSuccess) (void)hipGetLastError();
         else if (placed && memcmp(&there, &here, sizeof here) == 0) together++;
     }
-    if (together == PEER_REFUSED_ON_ONE_GPU) {
+    if (together == peer_refused_on_one_gpu()) {
         fprintf(stderr, "nvllm: nvllm_tp_init_peer(%d, %d): %d ranks share this GPU, which the peer exchange does not take\n", rank, world, together);
         unmap(world);
         return -1;

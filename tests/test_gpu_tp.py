@@ -195,6 +195,16 @@ def test_ranks_sharing_one_gpu_match_the_oracle(tmp_path, tmp_models, world, kv_
             print(f"peer all-reduce of 128 x 4096 floats, {world} ranks on one GPU: {r['allreduce_us_128x4096']:.1f} us (rank {rank})")
 
 
+def test_ranks_that_may_not_share_a_gpu_are_refused(tmp_path, tmp_models):
+    """Every rank finds the others' segments on its own GPU and says so before any of them is used (two ranks in the place of four)."""
+    path, shape = tmp_models("tiny", seed=5, **GQA)
+    spec = dict(name="tiny", over=GQA, model_path=path, n_seqs=1, seed=23, n_new=1, chunk=12, kv_bytes=2, out_dir=str(tmp_path), exchange="peer")
+    env = dict(os.environ, MASTER_ADDR="127.0.0.1", OMP_NUM_THREADS="2", HSA_ENABLE_IPC_MODE_LEGACY="0", NVLLM_TP_PEER_REFUSED="2")
+    out = util.run_ranks(2, 29793, [WORKER, json.dumps(spec)], tmp_path / "ranks", env, 300)
+    assert out.returncode != 0
+    assert "2 ranks share this GPU" in out.said.splitlines()[0], out.said
+
+
 def test_a_rank_left_alone_by_its_peers_stops_with_a_message(tmp_path, tmp_models):
     """Rank 0 makes three all-reduce calls that rank 1 never makes.  The kernels' waits are bounded (2 s here, 30 s
     by default) and only the first one is sat out; the launches end, and the next call stops the process with a message."""

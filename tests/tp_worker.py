@@ -61,7 +61,9 @@ def main():
         gathered = [torch.zeros(capi.TP_PEER_HANDLE_BYTES, dtype=torch.uint8) for _ in range(world)]
         dist.all_gather(gathered, torch.tensor(list(mine), dtype=torch.uint8))
         handles = (C.c_ubyte * (capi.TP_PEER_HANDLE_BYTES * world))(*[int(b) for t in gathered for b in t])
-        assert hip.nvllm_tp_init_peer(rank, world, handles) == 0
+        joined = hip.nvllm_tp_init_peer(rank, world, handles)
+        dist.barrier()   # (a rank that is refused keeps its segment until all have looked at it)
+        assert joined == 0
         if spec.get("lonely_call"):
             # rank 0 all-reduces alone: its kernel must give up after NVLLM_TP_PEER_WAIT_S, the launch must end,
             # and the next call on the host must stop the process with a message (the test reads stderr)
